@@ -1,0 +1,85 @@
+// Products summed over the batch:  out[g, j, i] = sum over the entries e of group g of  P[e, j, :] . Q[e, i, :]
+// -- the gradient of an operand that the forward product broadcast over the batch (a weight), which the reference forms
+// as one product per entry followed by a sum over them (cpm_kernels/torch/gemm.py:115-186, 219-239).
+#include "gemm_tile.h"
+
+namespace cpmk {
+
+// ---------------------------------------------------------------------------------------
+// Products summed over the batch
+// ---------------------------------------------------------------------------------------
+// Partial sums a product of (n, m) outputs over `batch` entries is formed in: as few as give most compute units a tile,
+// a divisor of the batch, and at most kSumMax entries each (the int8 form keeps their scales in a 4 KB strip).
+constexpr int kSumMax = 16;
+static int32_t sum_groups(int32_t m, int32_t n, int32_t batch) {
+    const int64_t cus = compute_units(), tiles = ceil_div(n, 128) * ceil_div(m, 128);
+    for (int32_t g = 1; g < batch; ++g)
+        if (batch % g == 0 && batch / g <= kSumMax && tiles * g * 4 >= cus * 3) return g;
+    return batch;
+}
+
+static int gemm_sum_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
+                             const void* srow, void* out, hipStream_t st) {
+    if (m < 0 || n < 0 || k <= 0 || batch < 1 || groups < 1 || batch % groups || batch / groups > kSumMax || groups > 65535) return CPMK_EBADARG;
+    if (m % 4 || n % 4) return CPMK_EALIGN;
+    if (m == 0 || n == 0) return 0;
+    if (any_null(A, B, out) || (!f16 && srow == nullptr)) return CPMK_EBADARG;
+    const int32_t kb = f16 ? 2 * k : k;        // bytes per row
+    if (k > (1 << 29) || (int64_t)n * kb >= (1ll << 32) || (int64_t)m * kb >= (1ll << 32)) return CPMK_ETOOBIG;
+    if (!aligned16(out) || (f16 ? (kb <= 64 || kb % 4 != 0) : kb % 128 != 0)) return CPMK_EALIGN;
+    const bool whole = kb % 16 == 0 && aligned16(A) && aligned16(B);
+    if (!whole && (!f16 || ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 3u))) return CPMK_EALIGN;
+    GemmArgs a;
+    a.P = (const int8_t*)B; a.Q = (const int8_t*)A; a.out = out;
+    a.srow = (const half_t*)srow; a.scol = nullptr;
+    a.strideP = (int64_t)n * kb;
+    a.strideQ = (int64_t)m * kb;
+    a.n = n; a.m = m; a.k = kb; a.bc_row = 0; a.bc_col = 0;
+    a.tiles_r = a.tiles_c = 0;
+    a.edge_in = 0;
+    a.nsum = batch / groups;
+    const uint32_t nkb = (uint32_t)(kb / (kb % 128 == 0 ? 128 : 64));
+    if ((uint64_t)nkb * a.nsum >= 65536) return CPMK_ETOOBIG;
+    a.kmagic = (uint32_t)(((1ull << 32) + nkb - 1) / nkb);
+    const int64_t cus = compute_units();
+    if (!f16) {
+        // Bound by the LDS reads of the K loop.  Beside the int32 accumulators a wave holds as many fp32 sums, so its share of
+        // the tile is 64 x 64 where the plain product's is 128 x 64: 256x128 tiles of eight waves.  10240 x 4096 outputs over
+        // 8 entries of 512: 196 us, against 287 us for the products one by one and 149 us for adding them up; waves of
+        // 128 x 64, one per SIMD, 316 us (their accumulators have to be carried between the two register files to be folded).
+        if (ceil_div(n, 256) * ceil_div(m, 128) * groups * 4 >= cus * 3) return launch_dma<4, 2, 2, 2, 128, kEpiSumI8, 2, 0, 16>(a, groups, st);
+        // too few of them for most compute units: 128x128 tiles, two workgroups a compute unit when there are more than compute
+        // units (1024 x 2560 over 4 x 256: 12.0 us; 15.2 as 256x128), else the deeper ring (2048 x 2048 over 8 x 512: 29.8 us; two stages 31.3)
+        const int64_t mid = ceil_div(n, 128) * ceil_div(m, 128) * groups;
+        if (mid > cus) return launch_dma<2, 2, 2, 2, 128, kEpiSumI8, 2, 0, 16>(a, groups, st, 2);
+        return launch_dma<2, 2, 2, 2, 128, kEpiSumI8, kRingSmall, 0, 16>(a, groups, st);
+    }
+    const bool large = ceil_div(n, 256) * ceil_div(m, 256) * groups * 4 >= cus * 3;
+    if (kb % 128 == 0) return large ? launch_dma<2, 4, 4, 2, 128, kEpiSumF16, 2, 0, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 128, kEpiSumF16, kRingSmall, 0, 16>(a, groups, st);
+    if (whole) return large ? launch_dma<2, 4, 4, 2, 64, kEpiSumF16, 4, 4, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 64, kEpiSumF16, kRingSmall, 4, 16>(a, groups, st);
+    return large ? launch_dma<2, 4, 4, 2, 64, kEpiSumF16, 4, 12, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 64, kEpiSumF16, kRingSmall, 12, 16>(a, groups, st);
+}
+
+}  // namespace cpmk
+
+using namespace cpmk;
+
+extern "C" {
+
+int cpmk_gemm_sum_groups(int32_t m, int32_t n, int32_t batch) {
+    return m < 0 || n < 0 || batch < 1 ? 1 : sum_groups(m, n, batch);
+}
+
+int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
+                             const void* scale_row, void* out, void* stream) {
+    clear_stale_error();
+    return gemm_sum_dispatch(false, m, k, n, batch, groups, A, B, scale_row, out, (hipStream_t)stream);
+}
+
+int cpmk_gemm_fp16_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
+                       void* out, void* stream) {
+    clear_stale_error();
+    return gemm_sum_dispatch(true, m, k, n, batch, groups, A, B, nullptr, out, (hipStream_t)stream);
+}
+
+}  // extern "C"

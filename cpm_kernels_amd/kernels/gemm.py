@@ -129,6 +129,34 @@ def gemm_scale_y(batch: int, n: int, m: int,
     cpmk.gemm_scale_y(batch, n, m, mat, scale_y, out, _stream(stream))
 
 
+def gemm_sum_groups(m: int, n: int, batch: int) -> int:
+    """Partial sums that gemm_int8_scale_sum / gemm_fp16_sum form for (n, m) outputs over `batch` entries: as few as
+    keep the device busy (a divisor of the batch)."""
+    return cpmk.gemm_sum_groups(m, n, batch)
+
+
+def gemm_int8_scale_sum(m: int, k: int, n: int, batch: int, groups: int,
+                        A: DevicePointer,           # (batch, m, k)     int8
+                        B: DevicePointer,           # (batch, n, k)     int8
+                        scale_row: DevicePointer,   # (batch, n)        fp16
+                        out: DevicePointer,         # (groups, n, m)    fp16
+                        stream: CUDAStream):
+    """out[g] = sum over the entries of group g of scale_row * (B x A^T): the reference's gemm_int8 + gemm_scale_x +
+    sum over the batch (torch/gemm.py:115-186), each sum in fp32 and rounded once.  k is a multiple of 128."""
+    assert m % 4 == 0 and n % 4 == 0 and k % 128 == 0
+    cpmk.gemm_int8_scale_sum(m, k, n, batch, groups, A, B, scale_row, out, _stream(stream))
+
+
+def gemm_fp16_sum(m: int, k: int, n: int, batch: int, groups: int,
+                  A: DevicePointer,         # (batch, m, k)     fp16
+                  B: DevicePointer,         # (batch, n, k)     fp16
+                  out: DevicePointer,       # (groups, n, m)    fp16
+                  stream: CUDAStream):
+    """out[g] = sum over the entries of group g of B x A^T: gemm_fp16 + sum over the batch (torch/gemm.py:219-239)."""
+    assert m % 4 == 0 and n % 4 == 0 and k % 2 == 0 and k > 32
+    cpmk.gemm_fp16_sum(m, k, n, batch, groups, A, B, out, _stream(stream))
+
+
 def gemm_fp16(m: int, k: int, n: int,
               batchA: int, batchB: int,
               aT: bool, bT: bool,

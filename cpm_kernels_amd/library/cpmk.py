@@ -25,6 +25,8 @@ _LAUNCHERS = {
     "cpmk_gemm_quantize_pair": [ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p],
     "cpmk_gemm_quantize_cols": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
     "cpmk_gemm_fp16": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
+    "cpmk_gemm_int8_scale_sum": [ctypes.c_int32] * 5 + [ctypes.c_void_p] * 5,
+    "cpmk_gemm_fp16_sum": [ctypes.c_int32] * 5 + [ctypes.c_void_p] * 4,
     "cpmk_gemv_fp16": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
     "cpmk_gemv_fp16_transpose": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
     "cpmk_gemv_broadcast_mat_fp16": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
@@ -83,7 +85,7 @@ _LAUNCHERS = {
 
 EXPORTED_SYMBOLS = sorted(list(_LAUNCHERS) + [
     "cpmk_version", "cpmk_error_string", "cpmk_device_count", "cpmk_get_device",
-    "cpmk_set_device", "cpmk_device_props", "cpmk_exchange_capture_slots_left",
+    "cpmk_set_device", "cpmk_device_props", "cpmk_exchange_capture_slots_left", "cpmk_gemm_sum_groups",
 ])
 
 
@@ -130,6 +132,11 @@ def exchange_capture_slots_left() -> int:
     n = ctypes.c_int32(0)
     checkStatus(lib.cpmk_exchange_capture_slots_left(ctypes.byref(n)))
     return n.value
+
+
+@lib.bind("cpmk_gemm_sum_groups", [ctypes.c_int32] * 3, ctypes.c_int32)
+def gemm_sum_groups(m: int, n: int, batch: int) -> int:
+    return lib.cpmk_gemm_sum_groups(m, n, batch)
 
 
 @lib.bind("cpmk_device_count", [ctypes.POINTER(ctypes.c_int)], ctypes.c_int)

@@ -9,7 +9,7 @@ the six-launch sequence, which ``fused=False`` still runs through the kernel-lev
 import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale, gemm_quantize, gemm_quantize_cols, \
-    gemm_quantize_pair, gemm_fp16, gemm_backward_round_scale, gemm_backward_scale_round, transpose, transpose_i8
+    gemm_quantize_pair, gemm_fp16, gemm_sum_groups, gemm_int8_scale_sum, gemm_fp16_sum, arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_scale_round, transpose, transpose_i8
 from ._common import cur_stream
 
 
@@ -106,6 +106,30 @@ def gemm_and_scale(quantA, scaleA, quantB, scaleB, aT, bT, fused=True) -> torch.
     return result_fp
 
 
+def _sum_entries(parts: torch.Tensor) -> torch.Tensor:
+    """(g, r, c) -> (1, r, c), fp32 sums rounded once"""
+    if parts.size(0) == 1:
+        return parts
+    out = torch.empty((1,) + parts.shape[1:], dtype=torch.half, device=parts.device)
+    arith_batch_add_backward(parts.size(0), parts.stride(0), parts.data_ptr(), out.data_ptr(), cur_stream())
+    return out
+
+
+def gemm_and_scale_sum(quantA, scaleA, quantB) -> torch.Tensor:
+    """(1, M, N): the sum over the batch of scaleA * (quantA x quantB^T), quantA (b, M, K) and quantB (b, N, K)."""
+    batch, M, K = quantA.size()
+    N = quantB.size(1)
+    groups = gemm_sum_groups(N, M, batch)
+    if groups == batch or quantB.size(0) != batch or max(M, N) * K >= 2 ** 31 or batch * K >= 2 ** 22:
+        return _sum_entries(gemm_and_scale(quantA, scaleA, quantB, None, False, True))
+    if K % 128 != 0:
+        quantA, quantB = _zero_padded_i8(quantA), _zero_padded_i8(quantB)
+    parts = torch.empty((groups, M, N), dtype=torch.half, device=quantA.device)
+    gemm_int8_scale_sum(N, quantA.size(2), M, batch, groups, quantB.data_ptr(), quantA.data_ptr(), scaleA.data_ptr(),
+                        parts.data_ptr(), cur_stream())
+    return _sum_entries(parts)
+
+
 class GEMMInt8(torch.autograd.Function):
     @staticmethod
     def forward(ctx, A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool, fused: bool = True):
@@ -165,6 +189,8 @@ class GEMMInt8(torch.autograd.Function):
             quant_G_a = _rows_padded_i8(quant_G_a)                      # both contracted over N
             if in_aT:       # grad_A (b, K, M) = qB_t x quant_G_a^T, scaled per column m
                 grad_A = gemm_and_scale(qB_t, None, quant_G_a, scale_G_a, False, True)
+            elif scale_A.size(0) == 1:      # ... summed over the batch that A was broadcast over
+                grad_A = gemm_and_scale_sum(quant_G_a, scale_G_a, qB_t)
             else:           # grad_A (b, M, K) = quant_G_a x qB_t^T, scaled per row m
                 grad_A = gemm_and_scale(quant_G_a, scale_G_a, qB_t, None, False, True)
             del scale_G_a, quant_G_a, qB_t
@@ -175,7 +201,9 @@ class GEMMInt8(torch.autograd.Function):
             qG_t = _rows_padded_i8(_transposed_copy_i8(quant_G_b))      # (b, N, M)
             del quant_G_b
             qA_t = _rows_padded_i8(_transposed_copy_i8(quantized_A))    # (bA, K, M); both contracted over M
-            if in_bT:       # grad_B (b, N, K) = qG_t x qA_t^T, scaled per row n
+            if in_bT and scale_B.size(0) == 1:      # summed over the batch that B was broadcast over
+                grad_B = gemm_and_scale_sum(qG_t, scale_G_b, qA_t)
+            elif in_bT:     # grad_B (b, N, K) = qG_t x qA_t^T, scaled per row n
                 grad_B = gemm_and_scale(qG_t, scale_G_b, qA_t, None, False, True)
             else:           # grad_B (b, K, N) = qA_t x qG_t^T, scaled per column n
                 grad_B = gemm_and_scale(qA_t, None, qG_t, scale_G_b, False, True)
@@ -223,8 +251,11 @@ def _rows_padded_i8(x: torch.Tensor) -> torch.Tensor:
     tile kernel's whole-slab path applies whatever k is (at k = 500 it is several times faster than the kernels
     for ragged rows, and the copy costs two passes over the operand)."""
     k = x.size(2)
-    if k % 64 == 0 or k < 128:
-        return x
+    return x if k % 64 == 0 or k < 128 else _zero_padded_i8(x)
+
+
+def _zero_padded_i8(x: torch.Tensor) -> torch.Tensor:
+    k = x.size(2)
     padded = torch.zeros((x.size(0), x.size(1), (k + 127) // 128 * 128), dtype=torch.int8, device=x.device)
     padded[:, :, :k].copy_(x)
     return padded
@@ -254,6 +285,24 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
     return out
 
 
+def gemm_pth_fp16_sum(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch.Tensor:
+    """The same product summed over the batch, (1, M, N)."""
+    M, K, N = _dims(A, B, aT, bT)
+    batch = A.size(0)
+    if batch == B.size(0) and batch > 1:
+        groups = gemm_sum_groups(N, M, batch)
+        per = batch // groups
+        if groups < batch and aT and not bT:
+            # both operands stored (K, rows): the entries of a group are one longer contraction as they lie
+            return _sum_entries(gemm_pth_fp16(A.view(groups, per * K, M), True, B.view(groups, per * K, N), False))
+        if groups < batch and not aT and bT and M % 4 == 0 and N % 4 == 0 and K > 32 and max(M, N) * K < 2 ** 31 and \
+                batch * K < 2 ** 21 and (A.data_ptr() | B.data_ptr()) % 4 == 0:
+            parts = torch.empty((groups, M, N), dtype=torch.half, device=A.device)
+            gemm_fp16_sum(N, K, M, batch, groups, B.data_ptr(), A.data_ptr(), parts.data_ptr(), cur_stream())
+            return _sum_entries(parts)
+    return _sum_entries(gemm_pth_fp16(A, aT, B, bT))
+
+
 class GEMMFloat(torch.autograd.Function):
     @staticmethod
     def forward(ctx, A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool):
@@ -272,12 +321,10 @@ class GEMMFloat(torch.autograd.Function):
         assert grad_f.is_cuda and grad_f.is_contiguous() and grad_f.dtype == torch.float16
         aT, bT = ctx.aT, ctx.bT
         A, B = ctx.saved_tensors
-        grad_A = gemm_pth_fp16(B, bT, grad_f, True) if aT else gemm_pth_fp16(grad_f, False, B, not bT)
-        grad_B = gemm_pth_fp16(grad_f, True, A, aT) if bT else gemm_pth_fp16(A, not aT, grad_f, False)
-        if A.size(0) == 1 and grad_A.size(0) > 1:
-            grad_A = grad_A.sum(dim=0, keepdim=True)
-        if B.size(0) == 1 and grad_B.size(0) > 1:
-            grad_B = grad_B.sum(dim=0, keepdim=True)
+        product_A = gemm_pth_fp16_sum if A.size(0) == 1 else gemm_pth_fp16
+        product_B = gemm_pth_fp16_sum if B.size(0) == 1 else gemm_pth_fp16
+        grad_A = product_A(B, bT, grad_f, True) if aT else product_A(grad_f, False, B, not bT)
+        grad_B = product_B(grad_f, True, A, aT) if bT else product_B(A, not aT, grad_f, False)
         return grad_A, None, grad_B, None
 
 

@@ -169,6 +169,19 @@ int cpmk_gemm_quantize_cols(int32_t batch, int32_t n, int32_t m, const void* mat
  * Requires m, n, k even as the reference asserts.        kernels/gemm.py:188-256 (cuBLASLt) */
 int cpmk_gemm_fp16(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB,
                    int aT, int bT, const void* A, const void* B, void* out, void* stream);
+
+/* Products summed over the batch: the gradient of an operand that the forward product broadcast over the batch
+ * (cpm_kernels/torch/gemm.py:115-186, 219-239 form one product per entry and add them up).  Both operands K-major, A (batch, m, k)
+ * and B (batch, n, k); out (groups, n, m) fp16 with out[g] the sum over the batch / groups consecutive entries of group g
+ * (groups divides batch, at most 16 entries a group), accumulated in fp32 and rounded once.
+ * int8: each entry's int32 product is scaled by scale_row (batch, n) first; k a multiple of 128, buffers on 16-byte boundaries.
+ * fp16: k > 32, buffers on 4-byte boundaries.  m and n multiples of 4.
+ * cpmk_gemm_sum_groups: as few groups as keep the device busy. */
+int cpmk_gemm_sum_groups(int32_t m, int32_t n, int32_t batch);
+int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
+                             const void* scale_row, void* out, void* stream);
+int cpmk_gemm_fp16_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
+                       void* out, void* stream);
 /* out[b,o] = sum_k mat[b,o,k] vec[b,k]      kernels/gemv.py:82-149 / cuda/gemv.cu:78-107 */
 int cpmk_gemv_fp16(int32_t batch, int32_t dim_out, int32_t dim_in, const void* mat,
                    const void* vec, void* out, void* stream);

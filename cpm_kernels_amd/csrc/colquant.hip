@@ -4,7 +4,13 @@
 // 79-98), with q written either in place (b, n, m) or transposed (b, m, n).  The transposed form
 // is what lets torch-level bmm feed operands given as (batch, K, N) to the K-major int8 GEMM
 // (the reference's GEMMInt8.forward, torch/gemm.py:84-113, quantises such an operand along
-// dim 1 and leaves the transposition to cuBLASLt).
+// dim 1 and leaves the transposition to cuBLASLt).  Or both: a product that will be differentiated
+// needs the transposed form now and the other one for its backward pass.
+// With row scales the values are mat[b,i,j] * row_scale[b,i] and the divisor is the fp32 absmax / 127
+// (cu_gemm_backward_scale_round, cuda/gemm.cu:139-172): the gradient on its way to the product with
+// the other operand.
+// Either output may have rows longer than the matrix's, filled up with zeros: a product contracts over
+// whole slabs then, whatever the number of rows or columns is.
 #include "dim1.h"
 #include "exchange.h"
 
@@ -20,10 +26,26 @@ namespace cpmk {
 // UA: any m and alignment: a piece inside its row still moves whole, at whatever address it lies (global accesses need
 // no alignment); the piece across a row's end is read (and its scales and, not transposed, its int8 values are
 // written) in at most three narrower accesses.
-template <int NT, bool TRANSPOSED, bool NTH, bool UA = false>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_col_quantize_team(int32_t n, int32_t m, int32_t tiles_per_batch, int32_t parts,
-                                                          const half_t* __restrict__ mat, half_t* __restrict__ scale,
-                                                          int8_t* __restrict__ out, uint32_t nteams, XchLaunch xl) {
+// OUT: bit 0 the transposed output, bit 1 the one in place.
+struct ColQuantArgs {
+    int32_t n, m;
+    const half_t* mat;
+    const half_t* row_scale;      // SCALED: (batch, n), or (n) shared by the batch
+    int bc;
+    half_t* scale;                // (batch, m)
+    int8_t* out_t;                // (batch, m, ld_t)
+    int8_t* out_n;                // (batch, n, ld_n)
+    int32_t ld_t, ld_n;
+};
+constexpr int kOutT = 1, kOutN = 2;
+
+template <int NT, int OUT, bool NTH, bool UA, bool SCALED>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_col_quantize_team(ColQuantArgs a, int32_t tiles_per_batch, int32_t parts,
+                                                          uint32_t nteams, XchLaunch xl) {
+    constexpr bool TRANSPOSED = (OUT & kOutT) != 0, NATURAL = (OUT & kOutN) != 0;
+    const int32_t n = a.n, m = a.m;
+    const half_t* const mat = a.mat;
+    half_t* const scale = a.scale;
     constexpr int LPR = 8, R = 8, COLS = 64, ROWS = NT / LPR * R;
     uint64_t* const xch = xl.region;
     const uint32_t tag = xl.tag;
@@ -39,6 +61,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     const int32_t row0 = part * ROWS + rg * 8;           // this lane's first row
     const int64_t boff = (int64_t)b * n * m;
 
+    float sx[R];        // SCALED: the lane's rows' scales, requested ahead of the tile
+    if constexpr (SCALED) {
+        const half_t* rs = a.row_scale + (a.bc ? 0 : (int64_t)b * n);
+#pragma unroll
+        for (int p = 0; p < R; ++p) sx[p] = row0 + p < n ? (float)rs[row0 + p] : 0.0f;
+    }
     half8_t v[R];
 #pragma unroll
     for (int p = 0; p < R; ++p) {
@@ -58,20 +86,29 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
             v[p] = NTH ? __builtin_nontemporal_load(src) : *src;        // read once; the int8 output below is what the next kernel wants in cache
         }
     }
-    // |x| maxima of the lane's 8 columns as integers; a NaN among them (rare) repeats the maximum in
-    // floating point, which skips NaN elements
-    ushort8_t um = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int p = 0; p < R; ++p) um = absbits_max(um, v[p]);
-    half8_t hm = __builtin_bit_cast(half8_t, um);
-    if (absbits_max_of(um) > 0x7c00u) {
-        hm = __builtin_elementwise_abs(v[0]);
-#pragma unroll
-        for (int p = 1; p < R; ++p) hm = __builtin_elementwise_max(hm, __builtin_elementwise_abs(v[p]));
-    }
     float mx[8];
+    if constexpr (SCALED) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) mx[e] = (float)hm[e];
+        for (int e = 0; e < 8; ++e) mx[e] = 0.0f;
+#pragma unroll
+        for (int p = 0; p < R; ++p)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mx[e] = fmaxf(mx[e], fabsf((float)v[p][e] * sx[p]));       // (skips NaN products, as the reference's fmaxf does)
+    } else {
+        // |x| maxima of the lane's 8 columns as integers; a NaN among them (rare) repeats the maximum in
+        // floating point, which skips NaN elements
+        ushort8_t um = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int p = 0; p < R; ++p) um = absbits_max(um, v[p]);
+        half8_t hm = __builtin_bit_cast(half8_t, um);
+        if (absbits_max_of(um) > 0x7c00u) {
+            hm = __builtin_elementwise_abs(v[0]);
+#pragma unroll
+            for (int p = 1; p < R; ++p) hm = __builtin_elementwise_max(hm, __builtin_elementwise_abs(v[p]));
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mx[e] = (float)hm[e];
+    }
     if (parts == 1) {
         coltile_reduce<NT, LPR, 1, true>(mx, lds);       // every lane: the maxima of its 8 columns
     } else {
@@ -100,8 +137,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     float s[8], y[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        sh[e] = scale_from_absmax(mx[e]);
-        s[e] = (float)sh[e];
+        if constexpr (SCALED) {
+            s[e] = (float)((double)mx[e] / 127.0);       // float / double constant, as the reference writes it
+            sh[e] = (half_t)s[e];
+        } else {
+            sh[e] = scale_from_absmax(mx[e]);
+            s[e] = (float)sh[e];
+        }
         y[e] = 1.0f / s[e];
     }
     if (part == 0 && rg == 0) {
@@ -119,7 +161,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     uint32_t q[R][2];       // [row p][columns 0-3 | 4-7], one byte each
     bool normal = true;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) normal = normal && scale_is_normal(sh[e]);
+    for (int e = 0; e < 8; ++e) normal = normal && (SCALED ? own_scale_in_range(s[e]) : scale_is_normal(sh[e]));
     if (__builtin_amdgcn_ballot_w64(!normal) == 0) {    // every scale of the wave's columns is a normal number: the short rounding sequence
 #pragma unroll
         for (int p = 0; p < R; ++p) {
@@ -128,7 +170,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
             asm volatile("" : "+v"(vp));             // keeps the fp32 conversions of the two paths apart (hoisted above the branch they hold 64 registers)
             const half8_t vh = __builtin_bit_cast(half8_t, vp);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) t[e] = quant_i8_own_scale_bits((float)vh[e], s[e], y[e]);
+            for (int e = 0; e < 8; ++e)
+                t[e] = SCALED ? quant_i8_own_fp32_scale_bits((float)vh[e] * sx[p], s[e], y[e]) : quant_i8_own_scale_bits((float)vh[e], s[e], y[e]);
             q[p][0] = pack4_i8((int32_t)t[0], (int32_t)t[1], (int32_t)t[2], (int32_t)t[3]);
             q[p][1] = pack4_i8((int32_t)t[4], (int32_t)t[5], (int32_t)t[6], (int32_t)t[7]);
             __builtin_amdgcn_sched_barrier(0);      // one row at a time: interleaving all 64 elements costs registers
@@ -137,24 +180,26 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 #pragma unroll
         for (int p = 0; p < R; ++p) {
             int32_t t[8];
+            int4_t vp = __builtin_bit_cast(int4_t, v[p]);
+            if constexpr (SCALED) asm volatile("" : "+v"(vp));             // (the products of the maxima are not to be kept for here)
+            const half8_t vh = __builtin_bit_cast(half8_t, vp);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) t[e] = quant_i8_rcp((float)v[p][e], s[e], y[e]);
+            for (int e = 0; e < 8; ++e) t[e] = SCALED ? quant_i8((float)vh[e] * sx[p], s[e]) : quant_i8_rcp((float)vh[e], s[e], y[e]);
             q[p][0] = pack4_i8(t[0], t[1], t[2], t[3]);
             q[p][1] = pack4_i8(t[4], t[5], t[6], t[7]);
+            if constexpr (SCALED) __builtin_amdgcn_sched_barrier(0);
         }
     }
-    if (col0 < m) {
-        if constexpr (!TRANSPOSED) {
+    if constexpr (NATURAL) {
+        if (col0 < a.ld_n) {
+            int8_t* const obase = a.out_n + (int64_t)b * n * a.ld_n;
 #pragma unroll
             for (int p = 0; p < R; ++p)
                 if (row0 + p < n) {
-                    int8_t* dst = out + boff + ((uint32_t)(row0 + p) * (uint32_t)m + (uint32_t)col0);
-                    if constexpr (UA) {
-                        if (col0 + 8 <= m) {
-                            store_byte8_any(dst, q[p][0], q[p][1]);
-                        } else {
-                            store_byte8_head_any(dst, m & 7, q[p][0], q[p][1]);
-                        }
+                    int8_t* dst = obase + ((uint32_t)(row0 + p) * (uint32_t)a.ld_n + (uint32_t)col0);
+                    if constexpr (UA) {       // (ld_n is m, or a multiple of 16 beyond it: the piece across the matrix's edge ends in zeros then)
+                        if (col0 + 8 <= a.ld_n) store_byte8_any(dst, q[p][0], q[p][1]);
+                        else store_byte8_head_any(dst, a.ld_n & 7, q[p][0], q[p][1]);
                     } else {
                         *reinterpret_cast<uint2_t*>(dst) = uint2_t{q[p][0], q[p][1]};
                     }
@@ -194,14 +239,44 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
             const int c = ps * (NT / 32) + (tid >> 5);
             const int32_t col = ct * COLS + c;
             const int4_t w = *reinterpret_cast<const int4_t*>(tbuf + c * ROWS + (((piece * 2) ^ ((c >> 3) << 3)) << 3));
-            int8_t* dst = out + boff + ((uint32_t)col * (uint32_t)n + (uint32_t)prow);
-            if (col < m) {             // n % 8 == 0: a piece is whole, half or not there
-                if (prow + 16 <= n) *reinterpret_cast<int4_t*>(dst) = w;
-                else if (prow + 8 <= n) *reinterpret_cast<uint2_t*>(dst) = uint2_t{(uint32_t)w.x, (uint32_t)w.y};
+            int8_t* dst = a.out_t + (int64_t)b * m * a.ld_t + ((uint32_t)col * (uint32_t)a.ld_t + (uint32_t)prow);
+            if (col < m) {             // ld_t % 8 == 0: a piece is whole, half or not there
+                if (prow + 16 <= a.ld_t) *reinterpret_cast<int4_t*>(dst) = w;
+                else if (prow + 8 <= a.ld_t) *reinterpret_cast<uint2_t*>(dst) = uint2_t{(uint32_t)w.x, (uint32_t)w.y};
             }
         }
     }
     if (parts > 1 && tid < 64) xch_retire(xl, team, parts);
+}
+
+// Any shape, both passes through memory: columns taller than a team holds, or launches recorded when no packets are left.
+// 64 columns x 4 row groups per workgroup.
+__global__ __launch_bounds__(256) void k_col_quantize_any(ColQuantArgs a) {
+    __shared__ float red[4][64];
+    const int c = threadIdx.x & 63, rg = threadIdx.x >> 6;
+    const int32_t n = a.n, m = a.m, col = blockIdx.x * 64 + c;
+    const int64_t b = blockIdx.y;
+    const half_t* mat = a.mat + b * n * m;
+    const half_t* rs = a.row_scale ? a.row_scale + (a.bc ? 0 : b * n) : nullptr;
+    auto value = [&](int32_t i) __attribute__((always_inline)) {
+        const float x = (float)mat[(int64_t)i * m + col];
+        return rs ? x * (float)rs[i] : x;
+    };
+    float mx = 0.0f;
+    if (col < m)
+        for (int32_t i = rg; i < n; i += 4) mx = fmaxf(mx, fabsf(value(i)));
+    red[rg][c] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0][c], red[1][c]), fmaxf(red[2][c], red[3][c]));
+    const float sf = (float)((double)mx / 127.0);
+    const half_t sh = rs ? (half_t)sf : scale_from_absmax(mx);
+    const float s = rs ? sf : (float)sh;
+    if (rg == 0 && col < m) a.scale[b * m + col] = sh;
+    for (int32_t i = rg; i < max(n, a.ld_t); i += 4) {
+        const int8_t q = col < m && i < n ? (int8_t)quant_i8(value(i), s) : 0;
+        if (a.out_t && col < m && i < a.ld_t) a.out_t[(b * m + col) * a.ld_t + i] = q;
+        if (a.out_n && col < a.ld_n && i < n) a.out_n[(b * n + i) * a.ld_n + col] = q;
+    }
 }
 
 // Any shape: rounding with per-column scales into the transposed layout, one element per thread.
@@ -227,6 +302,74 @@ extern "C" {
 int cpmk_gemm_calc_scale_transpose(int32_t, int32_t, int32_t, const void*, void*, void*);
 int cpmk_gemm_round_transpose(int32_t, int32_t, int32_t, const void*, const void*, void*, void*);
 
+}  // extern "C"
+
+// The team kernel on (batch, n, m): 0, an error code, or -1 when the shape is not one it takes.
+template <bool SCALED>
+static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st) {
+    const int32_t n = p.n, m = p.m;
+    // a team here only exchanges one maximum per column and gathers it in a loop over the parts, so
+    // it may be larger than the teams of the kernels that keep per-part values in registers
+    // (16384 rows; far fewer workgroups than are resident at once, which is what progress needs)
+    constexpr int64_t kColMaxParts = 32;
+    const int64_t tiles = ceil_div(p.out_n ? p.ld_n : m, 64), parts = ceil_div(n, 512);
+    // rows of whole 16-byte pieces in aligned buffers: 16-byte accesses; any other width or alignment: the same kernel moving
+    // its columns one by one (the transposed output runs along n either way)
+    const bool wide = (m % 8 == 0) && aligned16(p.mat) && aligned16(p.scale) && ((reinterpret_cast<uintptr_t>(p.out_n) & 7u) == 0);
+    const bool team_ok = (!p.out_t || (p.ld_t % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out_t) & 7u) == 0)) &&
+                         (int64_t)n * (p.out_n ? p.ld_n : m) < (1ll << 31) && (int64_t)m * p.ld_t < (1ll << 31) && p.ld_t <= parts * 512 &&
+                         parts <= kColMaxParts && tiles * parts <= kXchSlots;
+    if (!team_ok) return -1;
+    // teams use one packet slot per (team, part): batches beyond the pool go out in several launches
+    const int64_t per_launch = parts > 1 ? kXchSlots / (tiles * parts) : ((1ll << 31) - 8) / (tiles * parts);
+    for (int64_t b0 = 0; b0 < batch; b0 += per_launch) {
+        const int64_t nb = batch - b0 < per_launch ? batch - b0 : per_launch;
+        XchScope xs;
+        if (parts > 1) {
+            const int rc = xs.begin(tiles * nb * parts, st);
+            if (rc == kXchFull && b0 == 0) return -1;       // recorded into a graph and the capture reserve is used up: the separate kernels
+            if (rc != 0) return rc == kXchFull ? CPMK_ETOOBIG : rc;
+        }
+        const bool lines = m % 64 == 0 && (reinterpret_cast<uintptr_t>(p.mat) & 127u) == 0;
+        ColQuantArgs q = p;
+        q.mat += b0 * n * m;
+        if (p.row_scale && !p.bc) q.row_scale += b0 * n;
+        q.scale += b0 * m;
+        if (p.out_t) q.out_t += b0 * m * p.ld_t;
+        if (p.out_n) q.out_n += b0 * n * p.ld_n;
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)xch_team_grid(tiles * nb, parts)), dim3(512), 0, st, q, (int32_t)tiles, (int32_t)parts,
+                               (uint32_t)(tiles * nb), xs.xl);
+        };
+        auto pick = [&](auto oc) {
+            constexpr int OUT = decltype(oc)::value;
+            if (!wide) go(k_col_quantize_team<512, OUT, false, true, SCALED>);
+            else if (lines) go(k_col_quantize_team<512, OUT, true, false, SCALED>);
+            else go(k_col_quantize_team<512, OUT, false, false, SCALED>);
+        };
+        if (p.out_t && p.out_n) {
+            if constexpr (!SCALED) pick(std::integral_constant<int, kOutT | kOutN>{});
+        } else if (p.out_t) {
+            pick(std::integral_constant<int, kOutT>{});
+        } else {
+            pick(std::integral_constant<int, kOutN>{});
+        }
+        const int e = launch_status();
+        const int rc2 = xs.end();
+        if (e != 0 || rc2 != 0) return e ? e : rc2;
+    }
+    return 0;
+}
+
+namespace cpmk {
+int col_scale_round_team(int32_t batch, int32_t n, int32_t m, const void* mat, const void* row_scale, int bc, void* scale, void* out, void* stream) {
+    const ColQuantArgs p = {n, m, (const half_t*)mat, (const half_t*)row_scale, bc, (half_t*)scale, nullptr, (int8_t*)out, 0, m};
+    return col_quantize<true>(batch, p, (hipStream_t)stream);
+}
+}  // namespace cpmk
+
+extern "C" {
+
 int cpmk_gemm_quantize_cols(int32_t batch, int32_t n, int32_t m, const void* mat, void* scale, void* out,
                             int out_transposed, void* stream) {
     clear_stale_error();
@@ -235,57 +378,41 @@ int cpmk_gemm_quantize_cols(int32_t batch, int32_t n, int32_t m, const void* mat
     if (n == 0) return cpmk_gemm_calc_scale_transpose(batch, n, m, mat, scale, stream);       // (columns of no elements: scale 0, nothing to round)
     if (any_null(mat, scale, out)) return CPMK_EBADARG;
     hipStream_t st = (hipStream_t)stream;
-    // a team here only exchanges one maximum per column and gathers it in a loop over the parts, so
-    // it may be larger than the teams of the kernels that keep per-part values in registers
-    // (16384 rows; far fewer workgroups than are resident at once, which is what progress needs)
-    constexpr int64_t kColMaxParts = 32;
-    const int64_t tiles = ceil_div(m, 64), parts = ceil_div(n, 512);
-    // rows of whole 16-byte pieces in aligned buffers: 16-byte accesses; any other width or alignment: the same kernel moving
-    // its columns one by one (the transposed output runs along n either way)
-    const bool wide = (m % 8 == 0) && aligned16(mat) && aligned16(scale) && ((reinterpret_cast<uintptr_t>(out) & 7u) == 0);
-    const bool team_ok = (!out_transposed || (n % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 7u) == 0)) && (int64_t)n * m < (1ll << 31) &&
-                         parts <= kColMaxParts && tiles * parts <= kXchSlots;
-    if (team_ok) {
-        // teams use one packet slot per (team, part): batches beyond the pool go out in several launches
-        const int64_t per_launch = parts > 1 ? kXchSlots / (tiles * parts) : ((1ll << 31) - 8) / (tiles * parts);
-        bool no_slots = false;
-        for (int64_t b0 = 0; b0 < batch; b0 += per_launch) {
-            const int64_t nb = batch - b0 < per_launch ? batch - b0 : per_launch;
-            XchScope xs;
-            if (parts > 1) {
-                const int rc = xs.begin(tiles * nb * parts, st);
-                if (rc == kXchFull && b0 == 0) {
-                    no_slots = true;       // recorded into a graph and the capture reserve is used up: the separate kernels below
-                    break;
-                }
-                if (rc != 0) return rc == kXchFull ? CPMK_ETOOBIG : rc;
-            }
-            const bool lines = m % 64 == 0 && (reinterpret_cast<uintptr_t>(mat) & 127u) == 0;
-            auto go = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3((unsigned)xch_team_grid(tiles * nb, parts)), dim3(512), 0, st, n, m, (int32_t)tiles, (int32_t)parts,
-                                   (const half_t*)mat + b0 * n * m, (half_t*)scale + b0 * m, (int8_t*)out + b0 * n * m, (uint32_t)(tiles * nb), xs.xl);
-            };
-            if (out_transposed) {
-                if (!wide) go(k_col_quantize_team<512, true, false, true>);
-                else if (lines) go(k_col_quantize_team<512, true, true>);
-                else go(k_col_quantize_team<512, true, false>);
-            } else {
-                if (!wide) go(k_col_quantize_team<512, false, false, true>);
-                else if (lines) go(k_col_quantize_team<512, false, true>);
-                else go(k_col_quantize_team<512, false, false>);
-            }
-            const int e = launch_status();
-            const int rc2 = xs.end();
-            if (e != 0 || rc2 != 0) return e ? e : rc2;
-        }
-        if (!no_slots) return 0;
-    }
+    const ColQuantArgs p = {n, m, (const half_t*)mat, nullptr, 0, (half_t*)scale, out_transposed ? (int8_t*)out : nullptr,
+                            out_transposed ? nullptr : (int8_t*)out, out_transposed ? n : 0, out_transposed ? 0 : m};
+    const int rc = col_quantize<false>(batch, p, st);
+    if (rc >= 0) return rc;
     if (int e = cpmk_gemm_calc_scale_transpose(batch, n, m, mat, scale, stream)) return e;
     if (!out_transposed) return cpmk_gemm_round_transpose(batch, n, m, mat, scale, out, stream);
     const int64_t total = (int64_t)batch * n * m;
     hipLaunchKernelGGL(k_round_cols_transposed, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, total, n, m,
                        (const half_t*)mat, (const half_t*)scale, (int8_t*)out);
     return launch_status();
+}
+
+int cpmk_gemm_quantize_cols_ld(int32_t batch, int32_t n, int32_t m, const void* mat, const void* row_scale, int broad_cast_row,
+                               void* scale, void* out_t, int32_t ld_t, void* out_n, int32_t ld_n, void* stream) {
+    clear_stale_error();
+    if (batch < 0 || n < 1 || m < 0 || (out_t && (ld_t < n || ld_t % 16)) || (out_n && (ld_n < m || (ld_n != m && ld_n % 16)))) return CPMK_EBADARG;
+    if ((out_t == nullptr) == (out_n == nullptr) && (row_scale || out_t == nullptr)) return CPMK_EBADARG;       // (both outputs: without row scales only)
+    if ((int64_t)batch * m == 0) return 0;
+    if (any_null(mat, scale)) return CPMK_EBADARG;
+    const ColQuantArgs p = {n, m, (const half_t*)mat, (const half_t*)row_scale, broad_cast_row, (half_t*)scale, (int8_t*)out_t, (int8_t*)out_n,
+                            out_t ? ld_t : 0, out_n ? ld_n : 0};
+    const int rc = row_scale ? col_quantize<true>(batch, p, (hipStream_t)stream) : col_quantize<false>(batch, p, (hipStream_t)stream);
+    if (rc >= 0) return rc;
+    for (int64_t b0 = 0; b0 < batch; b0 += 65535) {       // (grid y: at most 65535 batch entries per launch)
+        const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
+        ColQuantArgs q = p;
+        q.mat += b0 * n * m;
+        if (q.row_scale && !q.bc) q.row_scale += b0 * n;
+        q.scale += b0 * m;
+        if (q.out_t) q.out_t += b0 * m * q.ld_t;
+        if (q.out_n) q.out_n += b0 * n * q.ld_n;
+        hipLaunchKernelGGL(k_col_quantize_any, dim3((unsigned)ceil_div(q.out_n ? q.ld_n : m, 64), (unsigned)nb), dim3(256), 0, (hipStream_t)stream, q);
+        if (int e = launch_status()) return e;
+    }
+    return 0;
 }
 
 }  // extern "C"

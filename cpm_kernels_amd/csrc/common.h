@@ -232,6 +232,23 @@ __device__ inline uint32_t quant_i8_own_scale_bits(float x, float s, float y) {
     return __builtin_bit_cast(uint32_t, t);
 }
 
+// The same for a divisor s = fp32(max|x| / 127) of the data's own that is no fp16 number (the backward quantisers, whose
+// x are products of two fp16 numbers, exact in fp32).  y = 1/s correctly rounded leaves q0 = x * y within two units in the
+// last place of x / s and one residual step q1 within one; a residual step from such a q1 with such a y gives the correctly
+// rounded quotient (Markstein, IBM J. Res. Dev. 34, 1990, theorem on the division by fused multiply-adds), so the rint() below
+// sees what the IEEE division gives.  The residuals are exact: with s in [2^-60, 2^60] and |x / s| <= 127.1 no product of
+// the steps comes near the subnormal range except for quotients far below one half, which round to 0 either way.
+// Two operations more than the fp16 form, half of the division's.
+__device__ inline bool own_scale_in_range(float s) { return s >= 0x1p-60f && s <= 0x1p60f; }
+__device__ inline uint32_t quant_i8_own_fp32_scale_bits(float x, float s, float y) {
+    const float q0 = x * y;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-s, q0, x), y, q0);
+    const float q2 = __builtin_fmaf(__builtin_fmaf(-s, q1, x), y, q1);
+    float t = q2 + 12582912.0f;
+    asm("" : "+v"(t));          // the sum must exist as a rounded fp32 number
+    return __builtin_bit_cast(uint32_t, t);
+}
+
 // Low bytes of four integers (each already within int8 range) into one dword: three byte
 // permutes.  v_perm_b32 selector bytes 0-3 pick from the second operand, 4-7 from the first, 0x0c is zero.
 __device__ inline uint32_t pack4_i8(int32_t a, int32_t b, int32_t c, int32_t d) {
@@ -307,6 +324,8 @@ int gemv_f16_mfma(int32_t batch, int32_t dim_out, int32_t dim_in, const void* ma
 
 // Column scales (cu_gemm_calc_scale_transpose) on the register-tile team kernel of train.hip: 0, an error code, or -1 (shape not taken)
 int col_absmax_team(int32_t batch, int32_t n, int32_t m, const void* mat, void* out, void* stream);
+// cu_gemm_backward_scale_round on the column quantiser of colquant.hip: 0, an error code, or -1 (shape not taken)
+int col_scale_round_team(int32_t batch, int32_t n, int32_t m, const void* mat, const void* row_scale, int bc, void* scale, void* out, void* stream);
 
 // Compute units of the current device (cached per device ordinal; 256 if the query fails).  The cache
 // is atomic: host threads that make their first call together each ask the runtime and store the

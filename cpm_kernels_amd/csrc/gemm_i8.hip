@@ -163,14 +163,14 @@ __global__ __launch_bounds__(WAVES_R* WAVES_C * 64) void k_gemm_kmajor(GemmArgs 
         for (int j = 0; j < TC; ++j) {
             const int32_t col = i0 + wc * TC * 32 + j * 32 + lrow;
             float sy = 0.0f;
-            if (FUSED && col < a.m) sy = (float)a.scol[(a.bc_col ? 0 : (int64_t)b * a.m) + col];
+            if (FUSED && col < a.m) sy = a.scol ? (float)a.scol[(a.bc_col ? 0 : (int64_t)b * a.m) + col] : 1.0f;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int32_t row = j0 + wr * TR * 32 + i * 32 + (e >> 2) * 8 + lk * 4 + (e & 3);
                 if (row < a.n && col < a.m) {
                     const int64_t o = obase + (int64_t)row * a.m + col;
                     if (FUSED) {
-                        const float sx = (float)a.srow[a.bc_row ? row : (int64_t)b * a.n + row];
+                        const float sx = a.srow ? (float)a.srow[a.bc_row ? row : (int64_t)b * a.n + row] : 1.0f;
                         reinterpret_cast<half_t*>(a.out)[o] = dequant(acc[i][j][e], sx, sy);
                     } else {
                         reinterpret_cast<int32_t*>(a.out)[o] = acc[i][j][e];
@@ -238,14 +238,14 @@ __global__ __launch_bounds__(256) void k_gemm_generic(GemmArgs a, int p_kmajor, 
         const int32_t row = j0 + ty * 4 + r;
         if (row >= a.n) continue;
         float sx = 0.0f;
-        if (FUSED) sx = (float)a.srow[a.bc_row ? row : (int64_t)b * a.n + row];
+        if (FUSED) sx = a.srow ? (float)a.srow[a.bc_row ? row : (int64_t)b * a.n + row] : 1.0f;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const int32_t col = i0 + tx + c * 16;
             if (col >= a.m) continue;
             const int64_t o = obase + (int64_t)row * a.m + col;
             if (FUSED) {
-                const float sy = (float)a.scol[(a.bc_col ? 0 : (int64_t)b * a.m) + col];
+                const float sy = a.scol ? (float)a.scol[(a.bc_col ? 0 : (int64_t)b * a.m) + col] : 1.0f;
                 reinterpret_cast<half_t*>(a.out)[o] = dequant(acc[r][c], sx, sy);
             } else {
                 reinterpret_cast<int32_t*>(a.out)[o] = acc[r][c];
@@ -278,7 +278,7 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
     if (!(batchA == batchB || batchA == 1 || batchB == 1)) return CPMK_EBADARG;   // :140
     const int batch = batchA > batchB ? batchA : batchB;
     if (m == 0 || n == 0) return 0;
-    if (out == nullptr || (k > 0 && any_null(A, B)) || (FUSED && any_null(srow, scol))) return CPMK_EBADARG;
+    if (out == nullptr || (k > 0 && any_null(A, B)) || (FUSED && srow == nullptr && scol == nullptr)) return CPMK_EBADARG;
     if (batch > 65535) {      // some kernels index the batch with the grid's z dimension: at most 65535 entries per call
         constexpr int64_t ESZ_OUT = FUSED ? 2 : 4;
         for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
@@ -611,6 +611,15 @@ int cpmk_gemm_int8(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batc
 int cpmk_gemm_int8_scale(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT,
                          const void* A, const void* B, const void* scale_row, const void* scale_col,
                          int broad_cast_row, int broad_cast_col, void* out, void* stream) {
+    clear_stale_error();
+    if ((int64_t)n * m > 0 && any_null(scale_row, scale_col)) return CPMK_EBADARG;
+    return gemm_dispatch<true>(m, k, n, batchA, batchB, aT, bT, A, B, scale_row, scale_col, broad_cast_row,
+                               broad_cast_col, out, (hipStream_t)stream);
+}
+
+int cpmk_gemm_int8_scale_one(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT,
+                             const void* A, const void* B, const void* scale_row, const void* scale_col,
+                             int broad_cast_row, int broad_cast_col, void* out, void* stream) {
     clear_stale_error();
     return gemm_dispatch<true>(m, k, n, batchA, batchB, aT, bT, A, B, scale_row, scale_col, broad_cast_row,
                                broad_cast_col, out, (hipStream_t)stream);

@@ -10,8 +10,8 @@ struct GemmArgs {
     const int8_t* P;      // row operand
     const int8_t* Q;      // column operand
     void* out;            // int32 or fp16, (batch, n, m)
-    const half_t* srow;   // fused epilogue: scale per output row j
-    const half_t* scol;   // fused epilogue: scale per output column i
+    const half_t* srow;   // fused epilogue: scale per output row j (null: one)
+    const half_t* scol;   // fused epilogue: scale per output column i (null: one)
     int64_t strideP, strideQ;   // batch strides in bytes (0 = broadcast)
     int32_t n, m, k;
     int32_t bc_row, bc_col;
@@ -348,12 +348,12 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
 #pragma unroll
         for (int i = 0; i < AR; ++i) {
             const int32_t row = min(j0 + wr * TR * 32 + i * 16 + r16, a.n - 1);
-            sxh[i] = a.srow[a.bc_row ? row : (int64_t)b * a.n + row];
+            sxh[i] = a.srow ? a.srow[a.bc_row ? row : (int64_t)b * a.n + row] : (half_t)1.0f;
         }
 #pragma unroll
         for (int j = 0; j < AC; ++j) {
             const int32_t col = min(i0 + wc * TC * 32 + j * 16 + q * 4, a.m - 4);   // m % 4 == 0
-            syh[j] = *reinterpret_cast<const half4_t*>(a.scol + (a.bc_col ? 0 : (int64_t)b * a.m) + col);
+            syh[j] = a.scol ? *reinterpret_cast<const half4_t*>(a.scol + (a.bc_col ? 0 : (int64_t)b * a.m) + col) : half4_t{1, 1, 1, 1};
         }
     }
 
@@ -688,14 +688,14 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
 #pragma unroll
         for (int i = 0; i < TR; ++i) {
             const int32_t row = min(j0 + wr * TR * 32 + i * 32 + lrow, a.n - 1);
-            sxh[i] = a.srow[a.bc_row ? row : (int64_t)b * a.n + row];
+            sxh[i] = a.srow ? a.srow[a.bc_row ? row : (int64_t)b * a.n + row] : (half_t)1.0f;
         }
 #pragma unroll
         for (int j = 0; j < TC; ++j)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 const int32_t col = min(i0 + wc * TC * 32 + j * 32 + g4 * 8 + lk * 4, a.m - 4);   // m % 4 == 0
-                syh[j][g4] = *reinterpret_cast<const half4_t*>(a.scol + (a.bc_col ? 0 : (int64_t)b * a.m) + col);
+                syh[j][g4] = a.scol ? *reinterpret_cast<const half4_t*>(a.scol + (a.bc_col ? 0 : (int64_t)b * a.m) + col) : half4_t{1, 1, 1, 1};
             }
     }
 
@@ -996,7 +996,7 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
 // products of the other)
 template <int WR, int WC, int TR, int TC, int BKB, int EPI, bool HALVES, int NST, int LAY, int MF>
 __global__ __launch_bounds__(WR* WC * 64, EPI == kEpiSumI8 ? 2 : 1) void k_gemm_dma(DmaArgs da) {
-    static_assert(!(HALVES && LAY != 0), "half tiles only with K-major operands");
+    static_assert(!(HALVES && (LAY & 4) != 0), "half tiles only where the depth is whole slabs");
     static_assert(MF == 16 || MF == 32, "MFMA tile");
     constexpr int BR = WR * TR * 32, BC = WC * TC * 32;
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
@@ -1013,8 +1013,8 @@ __global__ __launch_bounds__(WR* WC * 64, EPI == kEpiSumI8 ? 2 : 1) void k_gemm_
         const GemmItem nxt = gemm_item<BR, BC>(L + G, da);
         if (HALVES && cur.half) {
             if constexpr (HALVES) {
-                if constexpr (MF == 16) have_slabs = gemm_dma_tile<WR, WC, TR / 2, TC, BKB, EPI, NST>(da.g, smem, stg, lds_base, cur, nxt, have_slabs, ring);
-                else have_slabs = gemm_dma_tile32<WR, WC, TR / 2, TC, BKB, EPI, NST>(da.g, smem, stg, lds_base, cur, nxt, have_slabs, ring);
+                if constexpr (MF == 16) have_slabs = gemm_dma_tile<WR, WC, TR / 2, TC, BKB, EPI, NST, LAY>(da.g, smem, stg, lds_base, cur, nxt, have_slabs, ring);
+                else have_slabs = gemm_dma_tile32<WR, WC, TR / 2, TC, BKB, EPI, NST, LAY>(da.g, smem, stg, lds_base, cur, nxt, have_slabs, ring);
             }
         } else {
             if constexpr (MF == 16) have_slabs = gemm_dma_tile<WR, WC, TR, TC, BKB, EPI, NST, LAY>(da.g, smem, stg, lds_base, cur, nxt, have_slabs, ring);
@@ -1060,11 +1060,14 @@ static int launch_dma(GemmArgs& a, int batch, hipStream_t st, int per_cu = 1) {
     const int64_t r = total % grid;
     da.nfull = (uint32_t)total;
     da.nhalf = 0;
-    if constexpr (TR % 2 == 0 && LAY == 0 && ((BR / 2 + BC) / (1024 / BKB)) % (WR * WC) == 0) {      // (a half tile's slab must split evenly over the waves too)
-        if (r > 0 && 2 * r <= grid) {
+    // (a half tile's slab must split evenly over the waves too, and rows of K of half a tile be whole 128-byte groups;
+    // a tile moved inside the matrix has no half of its own)
+    constexpr bool F16 = EPI == kEpiF16 || EPI == kEpiSumF16;
+    if constexpr (TR % 2 == 0 && (LAY & 4) == 0 && ((BR / 2 + BC) / (1024 / BKB)) % (WR * WC) == 0 && (BR / 2) * (F16 ? 2 : 1) % 128 == 0) {
+        if (r > 0 && 2 * r <= grid && (a.edge_in & 1) == 0) {
             da.nfull = (uint32_t)(total - r);
             da.nhalf = (uint32_t)(2 * r);
-            return launch_dma_kernel<WR, WC, TR, TC, BKB, EPI, true, NST, 0, MF>(da, (unsigned)grid, st);
+            return launch_dma_kernel<WR, WC, TR, TC, BKB, EPI, true, NST, LAY, MF>(da, (unsigned)grid, st);
         }
     }
     return launch_dma_kernel<WR, WC, TR, TC, BKB, EPI, false, NST, LAY, MF>(da, (unsigned)grid, st);

@@ -233,6 +233,7 @@ struct RowsArgs {
     const half_t* mat0; half_t* scale0; int8_t* out0; int64_t rows0;
     const half_t* mat1; half_t* scale1; int8_t* out1; int64_t rows1;
     int32_t m;
+    int32_t ld;       // bytes from one output row to the next: m, or a multiple of 16 beyond it whose surplus is zeros
 };
 
 // (the launcher counts on 8 resident workgroups per compute unit up to NV = 8, 4 beyond)
@@ -240,14 +241,15 @@ struct RowsArgs {
 // 16-byte load and leaves in one 8-byte store (global accesses need no alignment), the piece across a row's end in at
 // most three narrower accesses each way.
 template <int NV, bool QUANT, bool UA = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA ? (NV <= 4 ? 8 : NV <= 8 ? 4 : 2) : (NV <= 8 ? 8 : 4)))) void k_rows(RowsArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA && NV > 4 ? 4 : 8))) void k_rows(RowsArgs a) {
     const int lane = threadIdx.x & 63;
     const int64_t nw = (int64_t)gridDim.x * 4;
     const int64_t rows = a.rows0 + a.rows1;
     const int32_t m = a.m;
     int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
-    const int m8 = UA ? (m + 7) >> 3 : m >> 3;
+    const int m8 = m >> 3;
+    const int l8 = (a.ld + 7) >> 3;      // pieces of an output row
     half8_t cur[NV];
     auto load = [&](half8_t (&v)[NV], int64_t r) __attribute__((always_inline)) {
         const half_t* mat = r < a.rows0 ? a.mat0 + r * m : a.mat1 + (r - a.rows0) * m;
@@ -275,10 +277,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA ? (NV <=
     auto store = [&](int8_t* orow, int j, uint2_t w) __attribute__((always_inline)) {
         if constexpr (!UA) {
             reinterpret_cast<uint2_t*>(orow)[j] = w;
-        } else if (j * 8 + 8 <= m) {
+        } else if (j * 8 + 8 <= a.ld) {
             store_byte8_any(orow + j * 8, w.x, w.y);
         } else {
-            store_byte8_head_any(orow + j * 8, m & 7, w.x, w.y);       // (callers pass j < ceil(m / 8))
+            store_byte8_head_any(orow + j * 8, a.ld & 7, w.x, w.y);       // (callers pass j < ceil(ld / 8))
         }
     };
     load(cur, row);
@@ -311,7 +313,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA ? (NV <=
         if (lane == 0) (second ? a.scale1 : a.scale0)[lrow] = sh;
         if (QUANT) {
             const float s = (float)sh, y = 1.0f / s;
-            int8_t* const orow = (second ? a.out1 : a.out0) + lrow * m;
+            int8_t* const orow = (second ? a.out1 : a.out0) + lrow * a.ld;
             if (scale_is_normal(sh)) {       // (the same for the whole wave) the short rounding sequence
 #pragma unroll
                 for (int i = 0; i < NV; ++i) {
@@ -325,13 +327,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA ? (NV <=
                     uint2_t w;
                     w.x = pack4_i8((int32_t)q[0], (int32_t)q[1], (int32_t)q[2], (int32_t)q[3]);
                     w.y = pack4_i8((int32_t)q[4], (int32_t)q[5], (int32_t)q[6], (int32_t)q[7]);
-                    if (j < m8) store(orow, j, w);
+                    if (j < l8) store(orow, j, w);
                 }
             } else {
 #pragma unroll
                 for (int i = 0; i < NV; ++i) {
                     const int j = lane + i * 64;
-                    if (j < m8) {
+                    if (j < l8) {
                         int32_t q[8];
 #pragma unroll
                         for (int e = 0; e < 8; ++e) q[e] = quant_i8_rcp((float)cur[i][e], s, y);
@@ -349,11 +351,88 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA ? (NV <=
     }
 }
 
+// The same for rows of more than 4096 columns: a workgroup per row, NV 16-byte pieces a thread (up to 16384 columns), the
+// maxima of its four waves exchanged through LDS.  Bound by memory: several workgroups share a compute unit and one's
+// loads pass under another's rounding.  A wave per row held such rows in 64 to 128 registers, and those past 8192
+// columns went through memory twice (scales, then rounding): [4096, 10240] 41 us; 24 us here.
+template <int NV, bool QUANT, bool UA>
+__global__ __launch_bounds__(256) void k_rows_wg(RowsArgs a) {
+    __shared__ uint32_t red[4];
+    __shared__ float redf[4];
+    const int tid = threadIdx.x;
+    const int32_t m = a.m;
+    const int64_t row = blockIdx.x;
+    const bool second = row >= a.rows0;
+    const int64_t lrow = second ? row - a.rows0 : row;
+    const half_t* mat = (second ? a.mat1 : a.mat0) + lrow * m;
+    half8_t v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int j = (tid + i * 256) * 8;
+        half8_t x = {0, 0, 0, 0, 0, 0, 0, 0};
+        if constexpr (!UA) {
+            if (j < m) x = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(mat + j));
+        } else {
+            if (j + 8 <= m) x = load_half8_any(mat + j);
+            else if (j < m) x = load_half8_head_any(mat + j, m & 7, x);
+        }
+        v[i] = x;
+    }
+    ushort8_t um = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < NV; ++i) um = absbits_max(um, v[i]);
+    const uint32_t wb = wave_max_u32_uniform(absbits_max_of(um));
+    if ((tid & 63) == 0) red[tid >> 6] = wb;
+    __syncthreads();
+    const uint32_t ub = max(max(red[0], red[1]), max(red[2], red[3]));
+    float mx = (float)__builtin_bit_cast(half_t, (uint16_t)ub);
+    if (ub > 0x7c00u) {      // (the same for the whole workgroup) a NaN in the row: the maximum that skips NaN elements
+        mx = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            int4_t ci = __builtin_bit_cast(int4_t, v[i]);
+            asm volatile("" : "+v"(ci));         // nothing of this rare path is to be computed ahead of the branch
+            const half8_t h = __builtin_bit_cast(half8_t, ci);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mx = fmaxf(fabsf((float)h[e]), mx);
+        }
+        mx = block_max<4>(mx, redf);
+    }
+    const half_t sh = scale_from_absmax(mx);
+    if (tid == 0) (second ? a.scale1 : a.scale0)[lrow] = sh;
+    if constexpr (QUANT) {
+        const float s = (float)sh, y = 1.0f / s;
+        int8_t* const orow = (second ? a.out1 : a.out0) + lrow * a.ld;
+        const bool normal = scale_is_normal(sh);       // (the same for the whole workgroup)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int j = (tid + i * 256) * 8;
+            int4_t ci = __builtin_bit_cast(int4_t, v[i]);
+            asm volatile("" : "+v"(ci));     // (a piece's fp32 conversions are made where they are used)
+            const half8_t h = __builtin_bit_cast(half8_t, ci);
+            int32_t q[8];
+            if (normal) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) q[e] = (int32_t)quant_i8_own_scale_bits((float)h[e], s, y);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) q[e] = quant_i8_rcp((float)h[e], s, y);
+            }
+            const uint2_t w = {pack4_i8(q[0], q[1], q[2], q[3]), pack4_i8(q[4], q[5], q[6], q[7])};
+            if (j < a.ld) {
+                if constexpr (!UA) *reinterpret_cast<uint2_t*>(orow + j) = w;
+                else if (j + 8 <= a.ld) store_byte8_any(orow + j, w.x, w.y);
+                else store_byte8_head_any(orow + j, a.ld & 7, w.x, w.y);
+            }
+        }
+    }
+}
+
 // Workgroups (4 waves each) for k_rows: between 1 and max_k per compute unit (what the register
 // budget lets be resident at once), the count that wastes the fewest wave-rows; more workgroups
 // on a tie.
-static unsigned rows_grid(int64_t rows, int cus, int nv) {
-    const int max_k = nv <= 8 ? 8 : 4;
+static unsigned rows_grid(int64_t rows, int cus) {
+    constexpr int max_k = 8;
     const int64_t need = ceil_div(rows, 4);
     if (need <= (int64_t)cus) return (unsigned)need;
     int64_t best = cus;
@@ -369,14 +448,30 @@ static unsigned rows_grid(int64_t rows, int cus, int nv) {
     return (unsigned)best;
 }
 
+constexpr int32_t kRowsMax = 16384;      // columns of the longest row that is held in registers
+constexpr int32_t kRowsWave = 4096;      // ... by one wave
+
 template <bool QUANT, bool UA = false>
-static void launch_rows(const RowsArgs& ra, int nv, hipStream_t st) {
-    const dim3 g(rows_grid(ra.rows0 + ra.rows1, compute_units(), nv));
+static int launch_rows(const RowsArgs& ra, hipStream_t st) {
+    const int64_t rows = ra.rows0 + ra.rows1;
+    const int32_t len = ra.ld > ra.m ? ra.ld : ra.m;
+    if (ra.m > kRowsWave) {
+        if (!grid_fits(rows)) return CPMK_ETOOBIG;
+        const dim3 g((unsigned)rows);
+        const int nv = (int)ceil_div(len, 2048);
+        if (nv <= 3) hipLaunchKernelGGL((k_rows_wg<3, QUANT, UA>), g, dim3(256), 0, st, ra);
+        else if (nv <= 4) hipLaunchKernelGGL((k_rows_wg<4, QUANT, UA>), g, dim3(256), 0, st, ra);
+        else if (nv <= 5) hipLaunchKernelGGL((k_rows_wg<5, QUANT, UA>), g, dim3(256), 0, st, ra);
+        else hipLaunchKernelGGL((k_rows_wg<8, QUANT, UA>), g, dim3(256), 0, st, ra);
+        return launch_status();
+    }
+    const int nv = (int)ceil_div(len, 512);
+    const dim3 g(rows_grid(rows, compute_units()));
     if (nv <= 1) hipLaunchKernelGGL((k_rows<1, QUANT, UA>), g, dim3(256), 0, st, ra);
     else if (nv <= 2) hipLaunchKernelGGL((k_rows<2, QUANT, UA>), g, dim3(256), 0, st, ra);
     else if (nv <= 4) hipLaunchKernelGGL((k_rows<4, QUANT, UA>), g, dim3(256), 0, st, ra);
-    else if (nv <= 8) hipLaunchKernelGGL((k_rows<8, QUANT, UA>), g, dim3(256), 0, st, ra);
-    else hipLaunchKernelGGL((k_rows<16, QUANT, UA>), g, dim3(256), 0, st, ra);
+    else hipLaunchKernelGGL((k_rows<8, QUANT, UA>), g, dim3(256), 0, st, ra);
+    return launch_status();
 }
 
 static int check3(int32_t batch, int32_t n, int32_t m) {
@@ -396,12 +491,9 @@ static int row_absmax(int64_t rows, int32_t m, const void* mat, void* out, hipSt
         if (vec) hipLaunchKernelGGL((k_row_absmax<256, true>), dim3((unsigned)rows), dim3(256), 0, st, rows, m, p, o);
         else hipLaunchKernelGGL((k_row_absmax<256, false>), dim3((unsigned)rows), dim3(256), 0, st, rows, m, p, o);
     } else {
-        const int nv = (int)ceil_div(m, 512);
-        if (nv <= 16) {
-            const RowsArgs ra = {p, o, nullptr, rows, nullptr, nullptr, nullptr, 0, m};
-            if (vec) launch_rows<false>(ra, nv, st);
-            else launch_rows<false, true>(ra, nv, st);
-            return launch_status();
+        if (m <= kRowsMax) {
+            const RowsArgs ra = {p, o, nullptr, rows, nullptr, nullptr, nullptr, 0, m, m};
+            return vec ? launch_rows<false>(ra, st) : launch_rows<false, true>(ra, st);
         }
         if (!grid_fits(ceil_div(rows, 4))) return CPMK_ETOOBIG;
         const unsigned g = (unsigned)ceil_div(rows, 4);
@@ -453,6 +545,14 @@ static int dequant_launch(int32_t batch, int32_t n, int32_t m, const void* mat, 
     else if (quads) go(k_dequant<MODE, 4>, 4);
     else go(k_dequant<MODE, 1>, 1);
     return launch_status();
+}
+
+static int quantize_pair(int64_t rows0, const void* mat0, void* scale0, void* out0, int64_t rows1, const void* mat1, void* scale1,
+                         void* out1, int32_t m, int32_t ld, hipStream_t st) {
+    const bool vec = (m % 8 == 0) && (ld % 8 == 0) && (rows0 == 0 || (aligned16(mat0) && (reinterpret_cast<uintptr_t>(out0) & 7u) == 0)) &&
+                     (rows1 == 0 || (aligned16(mat1) && (reinterpret_cast<uintptr_t>(out1) & 7u) == 0));
+    const RowsArgs ra = {(const half_t*)mat0, (half_t*)scale0, (int8_t*)out0, rows0, (const half_t*)mat1, (half_t*)scale1, (int8_t*)out1, rows1, m, ld};
+    return vec ? launch_rows<true>(ra, st) : launch_rows<true, true>(ra, st);
 }
 
 }  // namespace cpmk
@@ -548,13 +648,7 @@ int cpmk_gemm_quantize(int32_t batch, int32_t n, int32_t m, const void* mat, voi
         const int64_t rows = (int64_t)batch * n;
         if (rows == 0) return 0;
         if (any_null(scale) || (m > 0 && any_null(mat, out))) return CPMK_EBADARG;
-        const bool vec = (m % 8 == 0) && aligned16(mat) && ((reinterpret_cast<uintptr_t>(out) & 7u) == 0);
-        if (m > 0 && m <= 64 * 8 * 16) {
-            const RowsArgs ra = {(const half_t*)mat, (half_t*)scale, (int8_t*)out, rows, nullptr, nullptr, nullptr, 0, m};
-            if (vec) launch_rows<true>(ra, (int)ceil_div(m, 512), st);
-            else launch_rows<true, true>(ra, (int)ceil_div(m, 512), st);
-            return launch_status();
-        }
+        if (m > 0 && m <= kRowsMax) return quantize_pair(rows, mat, scale, out, 0, nullptr, nullptr, nullptr, m, m, st);
         if (int e = cpmk_gemm_calc_scale(batch, n, m, mat, scale, stream)) return e;
         return cpmk_gemm_round(batch, n, m, mat, scale, out, stream);
     }
@@ -567,19 +661,22 @@ int cpmk_gemm_quantize_pair(int64_t rows0, const void* mat0, void* scale0, void*
     if (rows0 < 0 || rows1 < 0 || m < 0 || rows0 > 0x7fffffff || rows1 > 0x7fffffff) return CPMK_EBADARG;
     if (m == 0 || rows0 + rows1 == 0) return 0;
     if ((rows0 > 0 && any_null(mat0, scale0, out0)) || (rows1 > 0 && any_null(mat1, scale1, out1))) return CPMK_EBADARG;
-    const bool vec = (m % 8 == 0) && (rows0 == 0 || (aligned16(mat0) && (reinterpret_cast<uintptr_t>(out0) & 7u) == 0)) &&
-                     (rows1 == 0 || (aligned16(mat1) && (reinterpret_cast<uintptr_t>(out1) & 7u) == 0));
-    if (m <= 64 * 8 * 16) {
-        const RowsArgs ra = {(const half_t*)mat0, (half_t*)scale0, (int8_t*)out0, rows0,
-                             (const half_t*)mat1, (half_t*)scale1, (int8_t*)out1, rows1, m};
-        if (vec) launch_rows<true>(ra, (int)ceil_div(m, 512), (hipStream_t)stream);
-        else launch_rows<true, true>(ra, (int)ceil_div(m, 512), (hipStream_t)stream);
-        return launch_status();
-    }
+    if (m <= kRowsMax) return quantize_pair(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, m, (hipStream_t)stream);
     if (rows0 > 0)
         if (int e = cpmk_gemm_quantize(1, (int32_t)rows0, m, mat0, scale0, out0, 0, stream)) return e;
     if (rows1 > 0) return cpmk_gemm_quantize(1, (int32_t)rows1, m, mat1, scale1, out1, 0, stream);
     return 0;
+}
+
+int cpmk_gemm_quantize_pair_ld(int64_t rows0, const void* mat0, void* scale0, void* out0, int64_t rows1, const void* mat1,
+                               void* scale1, void* out1, int32_t m, int32_t ld, void* stream) {
+    clear_stale_error();
+    if (rows0 < 0 || rows1 < 0 || m < 1 || rows0 > 0x7fffffff || rows1 > 0x7fffffff || ld < m) return CPMK_EBADARG;
+    if (ld != m && (ld % 16 || ld > ceil_div(m, 128) * 128)) return CPMK_EBADARG;
+    if (m > kRowsMax) return CPMK_ETOOBIG;
+    if (rows0 + rows1 == 0) return 0;
+    if ((rows0 > 0 && any_null(mat0, scale0, out0)) || (rows1 > 0 && any_null(mat1, scale1, out1))) return CPMK_EBADARG;
+    return quantize_pair(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, ld, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -321,8 +321,9 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     const uint32_t tag = xl.tag;
     constexpr int NT = 512, LPR = 8, R = 8;
     using T = ColTile<NT, LPR, R>;
-    constexpr bool TWO = KIND != kLnFwdV && KIND != kLnFwdMV && KIND != kScaleRound && KIND != kColAbsmax;     // reads grad_in too
-    constexpr bool IS_MAX = KIND == kScaleRound || KIND == kColAbsmax;
+    static_assert(KIND != kScaleRound, "colquant.hip");
+    constexpr bool TWO = KIND != kLnFwdV && KIND != kLnFwdMV && KIND != kColAbsmax;     // reads grad_in too
+    constexpr bool IS_MAX = KIND == kColAbsmax;
     constexpr int NV = (KIND == kLnFwdMV || KIND == kLnBwdMV) ? 2 : 1;      // statistics per column
     __shared__ float lds[(T::NW + 1) * T::COLS * NV];
     __shared__ float tot[T::COLS * 2];
@@ -340,7 +341,6 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     // The per-column and per-row operands of the sums are requested ahead of the tiles: loads return in
     // order, and behind the tiles they would hold the sums back until the last piece had arrived.
     half8_t hv = {0, 0, 0, 0, 0, 0, 0, 0}, hm = {0, 0, 0, 0, 0, 0, 0, 0};
-    half_t sxh[R];
     constexpr bool NTH = MODE == 0, UA = MODE == 2;
     auto load8 = [&](const half_t* src) __attribute__((always_inline)) {       // eight per-column values of this lane's columns
         half8_t r = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -362,29 +362,19 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     };
     if (live && (KIND == kLnBwdV || KIND == kLnBwdMV)) hv = load8(p.var + (int64_t)b * p.m + col0);
     if (live && KIND == kLnBwdMV) hm = load8(p.mean + (int64_t)b * p.m + col0);
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-        sxh[q] = (half_t)0.0f;
-        if (KIND == kScaleRound) {
-            const int32_t row = own0 + q * T::RPP + rg;
-            if (row < p.n) sxh[q] = p.sx[(p.bc ? 0 : (int64_t)b * p.n) + row];
-        }
-    }
     half8_t va[R], vg[TWO ? R : 1];
     // every input byte is read once: non-temporal loads; non-temporal stores too, except for the softmax
     // gradient, where they measured 1-2 % slower
     constexpr bool NTS = NTH && KIND != kSoftmaxBwd;
     coltile_load<NT, LPR, R, NTH, UA>(va, p.a + boff, own_n, p.m, col0, (half_t)0.0f);
     if constexpr (TWO) coltile_load<NT, LPR, R, NTH, UA>(vg, p.g + boff, own_n, p.m, col0, (half_t)0.0f);
-    float mean[8], var[8], c3[8], sxv[R];
+    float mean[8], var[8], c3[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         var[e] = (float)hv[e];
         c3[e] = -0.5f * var[e] * var[e] * var[e];
         mean[e] = (float)hm[e];
     }
-#pragma unroll
-    for (int q = 0; q < R; ++q) sxv[q] = (float)sxh[q];
 
     float s[NV * 8];
 #pragma unroll
@@ -400,8 +390,7 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
             else if constexpr (KIND == kLnBwdV) s[e] += gi * c3[e] * x;
             else if constexpr (KIND == kLnBwdMV) { s[e] += gi * c3[e] * (x - mean[e]); s[8 + e] += -gi * var[e]; }
             else if constexpr (KIND == kSoftmaxBwd) s[e] += x * gi;
-            else if constexpr (KIND == kColAbsmax) s[e] = fmaxf(s[e], fabsf(x));
-            else s[e] = fmaxf(s[e], fabsf(x * sxv[q]));
+            else s[e] = fmaxf(s[e], fabsf(x));
         }
     if (parts == 1) {
         coltile_reduce<NT, LPR, NV, IS_MAX>(s, lds);      // every lane: the statistics of its 8 columns
@@ -437,7 +426,6 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
         if constexpr (KIND == kLnFwdV) k1[e] = rsqrtf(s[e] / fn + p.eps);
         else if constexpr (KIND == kLnFwdMV) { k0[e] = s[e] / fn; k1[e] = rsqrtf(s[8 + e] / fn - k0[e] * k0[e] + p.eps); }
         else if constexpr (KIND == kLnBwdMV) s[8 + e] -= 2.0f * s[e] * mean[e];        // local_grad_mean -= 2 * local_grad_var * local_mean
-        else if constexpr (KIND == kScaleRound) k0[e] = (float)((double)s[e] / 127.0);     // float / double constant, as the reference writes it
     }
     if (live && part == 0 && rg == 0) {
         half8_t h0, h1;
@@ -445,7 +433,6 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
         for (int e = 0; e < 8; ++e) { h0[e] = (half_t)k0[e]; h1[e] = (half_t)k1[e]; }
         if (KIND == kLnFwdV || KIND == kLnFwdMV) store8(p.out_var + (int64_t)b * p.m + col0, h1);
         if (KIND == kLnFwdMV) store8(p.out_mean + (int64_t)b * p.m + col0, h0);
-        if (KIND == kScaleRound) store8(p.out_var + (int64_t)b * p.m + col0, h0);
         if constexpr (KIND == kColAbsmax) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) h0[e] = scale_from_absmax(s[e]);
@@ -454,28 +441,6 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     }
     if constexpr (KIND == kColAbsmax) {
         // the scales are all there is to write
-    } else if constexpr (KIND == kScaleRound) {
-        if (live) {
-#pragma unroll
-            for (int q = 0; q < R; ++q) {
-                const int32_t lrow = q * T::RPP + rg;
-                if (lrow < own_n) {
-                    int32_t t[8];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) t[e] = quant_i8((float)va[q][e] * sxv[q], k0[e]);
-                    int8_t* dst = p.out_i8 + boff + ((uint32_t)lrow * (uint32_t)p.m + (uint32_t)col0);
-                    if constexpr (UA) {
-                        if (col0 + 8 <= p.m) {
-                            store_byte8_any(dst, pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7]));
-                        } else {
-                            store_byte8_head_any(dst, p.m & 7, pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7]));
-                        }
-                    } else {
-                        *reinterpret_cast<uint2_t*>(dst) = uint2_t{pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7])};
-                    }
-                }
-            }
-        }
     } else {
 #pragma unroll
         for (int q = 0; q < R; ++q)
@@ -496,10 +461,24 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     if (parts > 1 && tid < 64) xch_retire(xl, team, parts);
 }
 
+// eight products x * sy rounded to multiples of s (own: s is the data's own and in the range of the short sequence)
+__device__ __forceinline__ uint2_t round8_own_scale(half8_t x, half8_t sy, float s, float y, bool own) {
+    int32_t t[8];
+    if (own) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] = (int32_t)quant_i8_own_fp32_scale_bits((float)x[e] * (float)sy[e], s, y);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] = quant_i8((float)x[e] * (float)sy[e], s);
+    }
+    return uint2_t{pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7])};
+}
+
 // cu_gemm_backward_round_scale: per-row absmax of mat * scale_y[col] -> scale_x, then rounding.
+// (ld: bytes from one row of the output to the next; past the matrix's columns they are zeros)
 __global__ __launch_bounds__(256) void k_round_scale_rows(int32_t n, int32_t m, const half_t* __restrict__ mat,
                                                           const half_t* __restrict__ scale_y, int8_t* __restrict__ out,
-                                                          half_t* __restrict__ scale_x, int bc) {
+                                                          half_t* __restrict__ scale_x, int bc, int32_t ld) {
     __shared__ float red[4];
     const int64_t row = blockIdx.x;                    // b*n + i
     const int64_t b = row / n;
@@ -510,14 +489,14 @@ __global__ __launch_bounds__(256) void k_round_scale_rows(int32_t n, int32_t m, 
     mx = block_max<4>(mx, red);
     const float s = (float)((double)mx / 127.0);
     if (threadIdx.x == 0) scale_x[row] = (half_t)s;
-    for (int32_t j = threadIdx.x; j < m; j += 256) out[row * m + j] = (int8_t)quant_i8((float)x[j] * (float)sy[j], s);
+    for (int32_t j = threadIdx.x; j < ld; j += 256) out[row * ld + j] = j < m ? (int8_t)quant_i8((float)x[j] * (float)sy[j], s) : 0;
 }
 
 // The same with a wave per row and 16-byte accesses (m % 8 == 0, aligned pointers); the second pass
 // over the row finds it in the cache.
 __global__ __launch_bounds__(256) void k_round_scale_rows_wide(int64_t rows, int32_t n, int32_t m, const half_t* __restrict__ mat,
                                                                const half_t* __restrict__ scale_y, int8_t* __restrict__ out,
-                                                               half_t* __restrict__ scale_x, int bc) {
+                                                               half_t* __restrict__ scale_x, int bc, int32_t ld) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
@@ -533,12 +512,15 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_wide(int64_t rows, int
     mx = wave_max(mx);
     const float s = (float)((double)mx / 127.0);
     if (lane == 0) scale_x[row] = (half_t)s;
-    for (int32_t j = lane * 8; j < m; j += 512) {
-        const half8_t xv = *reinterpret_cast<const half8_t*>(x + j), sv = *reinterpret_cast<const half8_t*>(sy + j);
-        int32_t t[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) t[e] = quant_i8((float)xv[e] * (float)sv[e], s);
-        *reinterpret_cast<uint2_t*>(out + row * m + j) = uint2_t{pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7])};
+    const float y = 1.0f / s;
+    const bool own = own_scale_in_range(s);       // (the same for the whole wave)
+    for (int32_t j = lane * 8; j < ld; j += 512) {
+        uint2_t w = {0u, 0u};
+        if (j < m) {
+            const half8_t xv = *reinterpret_cast<const half8_t*>(x + j), sv = *reinterpret_cast<const half8_t*>(sy + j);
+            w = round8_own_scale(xv, sv, s, y, own);
+        }
+        *reinterpret_cast<uint2_t*>(out + row * ld + j) = w;
     }
 }
 
@@ -551,7 +533,7 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_wide(int64_t rows, int
 template <int P, int U, bool UA>
 __global__ __launch_bounds__(256) void k_round_scale_rows_reg(int64_t rows, int32_t n, int32_t m, const half_t* __restrict__ mat,
                                                               const half_t* __restrict__ scale_y, int8_t* __restrict__ out,
-                                                              half_t* __restrict__ scale_x, int bc) {
+                                                              half_t* __restrict__ scale_x, int bc, int32_t ld) {
     const int lane = threadIdx.x & 63;
     const int64_t row0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * U;
     if (row0 >= rows) return;
@@ -593,21 +575,21 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_reg(int64_t rows, int3
         const float s = (float)((double)mx / 127.0);
         const int64_t row = row0 + u;
         if (row < rows) {
+            const float y = 1.0f / s;
+            const bool own = own_scale_in_range(s);       // (the same for the whole wave)
             if (lane == 0) scale_x[row] = (half_t)s;
 #pragma unroll
             for (int p = 0; p < P; ++p) {
                 const int32_t j = lane * 8 + p * 512;
-                if (j < m) {
-                    int32_t t[8];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) t[e] = quant_i8((float)xv[u][p][e] * (float)sv[u][p][e], s);
-                    int8_t* dst = out + row * m + j;
+                if (j < ld) {        // (past the end of the row: zeros)
+                    const uint2_t w = round8_own_scale(xv[u][p], sv[u][p], s, y, own);
+                    int8_t* dst = out + row * ld + j;
                     if constexpr (!UA) {
-                        *reinterpret_cast<uint2_t*>(dst) = uint2_t{pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7])};
-                    } else if (j + 8 <= m) {
-                        store_byte8_any(dst, pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7]));
+                        *reinterpret_cast<uint2_t*>(dst) = w;
+                    } else if (j + 8 <= ld) {
+                        store_byte8_any(dst, w.x, w.y);
                     } else {
-                        store_byte8_head_any(dst, m & 7, pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7]));
+                        store_byte8_head_any(dst, ld & 7, w.x, w.y);
                     }
                 }
             }
@@ -911,7 +893,7 @@ static int launch_col(int32_t batch, const ColArgs& p, void* stream, bool missin
     const bool wide = (int64_t)p.n * p.m < (1ll << 31) && parts <= kColTeamMaxParts && tiles * parts <= kXchSlots;
     auto on_line = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 127u) == 0; };
     const bool lines = p.m % 64 == 0 && on_line(p.a) && on_line(p.g) && on_line(p.out);      // (a null pointer counts as aligned)
-    if (wide) {
+    if constexpr (KIND != kScaleRound) if (wide) {
         // teams use one packet slot per (team, part): batches beyond the pool go out in several launches
         const int64_t per_launch = parts > 1 ? kXchSlots / (tiles * parts) : ((1ll << 31) - 8) / (tiles * parts);
         bool no_slots = false;
@@ -1101,12 +1083,22 @@ int cpmk_gemm_backward_scale_round(int32_t batch, int32_t n, int32_t m, const vo
     clear_stale_error();
     ColArgs p = {n, m, (const half_t*)mat, nullptr, nullptr, nullptr, (const half_t*)scale_x, nullptr, (int8_t*)out, nullptr,
                  (half_t*)scale_y, 0.0f, broad_cast_x};
-    return launch_col<kScaleRound>(batch, p, stream, any_null(mat, scale_x, out, scale_y));
+    const bool missing = any_null(mat, scale_x, out, scale_y);
+    if (batch > 0 && n > 0 && m > 0 && !missing) {
+        const int rc = col_scale_round_team(batch, n, m, mat, scale_x, broad_cast_x, scale_y, out, stream);
+        if (rc >= 0) return rc;
+    }
+    return launch_col<kScaleRound>(batch, p, stream, missing);
 }
 int cpmk_gemm_backward_round_scale(int32_t batch, int32_t n, int32_t m, const void* mat, const void* scale_y, void* out, void* scale_x,
                                    int broad_cast_y, void* stream) {
+    return cpmk_gemm_backward_round_scale_ld(batch, n, m, mat, scale_y, out, m, scale_x, broad_cast_y, stream);
+}
+
+int cpmk_gemm_backward_round_scale_ld(int32_t batch, int32_t n, int32_t m, const void* mat, const void* scale_y, void* out, int32_t ld,
+                                      void* scale_x, int broad_cast_y, void* stream) {
     clear_stale_error();
-    if (batch < 0 || n < 0 || m < 0) return CPMK_EBADARG;
+    if (batch < 0 || n < 0 || m < 0 || ld < m || (ld != m && (ld % 16 || ld > (m + 127) / 128 * 128))) return CPMK_EBADARG;
     const int64_t rows = (int64_t)batch * n;
     if (rows == 0) return 0;
     if (rows > 0x7fffffff) return CPMK_ETOOBIG;
@@ -1117,7 +1109,7 @@ int cpmk_gemm_backward_round_scale(int32_t batch, int32_t n, int32_t m, const vo
             constexpr int P = decltype(pc)::value, U = decltype(uc)::value;
             auto run = [&](auto kern) {
                 hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(rows, 4 * U)), dim3(256), 0, (hipStream_t)stream, rows, n, m, (const half_t*)mat,
-                                   (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, broad_cast_y);
+                                   (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, broad_cast_y, ld);
             };
             if (vec16) run(k_round_scale_rows_reg<P, U, false>);
             else run(k_round_scale_rows_reg<P, U, true>);
@@ -1129,11 +1121,11 @@ int cpmk_gemm_backward_round_scale(int32_t batch, int32_t n, int32_t m, const vo
     }
     if (vec16) {
         hipLaunchKernelGGL(k_round_scale_rows_wide, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, (hipStream_t)stream, rows, n, m,
-                           (const half_t*)mat, (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, broad_cast_y);
+                           (const half_t*)mat, (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, broad_cast_y, ld);
         return launch_status();
     }
     hipLaunchKernelGGL(k_round_scale_rows, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, n, m, (const half_t*)mat,
-                       (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, broad_cast_y);
+                       (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, broad_cast_y, ld);
     return launch_status();
 }
 

@@ -59,16 +59,17 @@ __global__ __launch_bounds__(256) void k_transpose(int32_t n, int32_t m, const h
 struct __attribute__((packed, aligned(1))) Byte16Any { uint32_t x, y, z, w; };
 
 template <bool IN, bool OUT>
-__global__ __launch_bounds__(256) void k_transpose_i8(int32_t n, int32_t m, const int8_t* __restrict__ in, int8_t* __restrict__ out) {
+__global__ __launch_bounds__(256) void k_transpose_i8(int32_t n, int32_t m, int32_t ldi, int32_t ldo, const int8_t* __restrict__ in, int8_t* __restrict__ out) {
     __shared__ __attribute__((aligned(16))) int8_t tile[64][68];        // pitch 68: dword-aligned rows, 17 banks apart
-    const int64_t boff = (int64_t)blockIdx.z * n * m;
+    in += (int64_t)blockIdx.z * n * ldi;
+    out += (int64_t)blockIdx.z * m * ldo;
     const int32_t r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
     const int pc = threadIdx.x & 3, rr = threadIdx.x >> 2;          // 4 pieces of 16 bytes x 64 rows
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     if constexpr (IN) {
         const int32_t c = c0 + pc * 16;
         if (r0 + rr < n && c < m) {
-            const int8_t* src = in + boff + (int64_t)(r0 + rr) * m + c;
+            const int8_t* src = in + (int64_t)(r0 + rr) * ldi + c;
             if (c + 16 <= m) {
                 const Byte16Any v = *reinterpret_cast<const Byte16Any*>(src);
                 uint32_t* dst = reinterpret_cast<uint32_t*>(&tile[rr][pc * 16]);
@@ -79,31 +80,33 @@ __global__ __launch_bounds__(256) void k_transpose_i8(int32_t n, int32_t m, cons
         }
     } else {
         for (int r = ty; r < 64; r += 4)
-            if (r0 + r < n && c0 + tx < m) tile[r][tx] = in[boff + (int64_t)(r0 + r) * m + c0 + tx];
+            if (r0 + r < n && c0 + tx < m) tile[r][tx] = in[(int64_t)(r0 + r) * ldi + c0 + tx];
     }
     __syncthreads();
     if constexpr (OUT) {
         // row rr of the transposed tile = column rr of the tile; this thread's 16 bytes are its rows pc*16 .. pc*16+15
         const int32_t r = r0 + pc * 16;
-        if (c0 + rr < m && r < n) {
-            int8_t* dst = out + boff + (int64_t)(c0 + rr) * n + r;
-            if (r + 16 <= n) {
+        if (c0 + rr < m && r < ldo) {
+            int8_t* dst = out + (int64_t)(c0 + rr) * ldo + r;
+            if (r >= n) {                            // (ldo > n is a multiple of 16)
+                *reinterpret_cast<Byte16Any*>(dst) = Byte16Any{0, 0, 0, 0};
+            } else if (r + 16 <= ldo) {
                 uint32_t w[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     uint32_t x = 0;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) x |= (uint32_t)(uint8_t)tile[pc * 16 + q * 4 + e][rr] << (8 * e);
+                    for (int e = 0; e < 4; ++e) x |= (r + q * 4 + e < n ? (uint32_t)(uint8_t)tile[pc * 16 + q * 4 + e][rr] : 0u) << (8 * e);
                     w[q] = x;
                 }
                 *reinterpret_cast<Byte16Any*>(dst) = Byte16Any{w[0], w[1], w[2], w[3]};
             } else {
-                for (int e = 0; e < n - r; ++e) dst[e] = tile[pc * 16 + e][rr];
+                for (int e = 0; e < ldo - r; ++e) dst[e] = tile[pc * 16 + e][rr];
             }
         }
     } else {
         for (int c = ty; c < 64; c += 4)
-            if (c0 + c < m && r0 + tx < n) out[boff + (int64_t)(c0 + c) * n + r0 + tx] = tile[tx][c];
+            if (c0 + c < m && r0 + tx < ldo) out[(int64_t)(c0 + c) * ldo + r0 + tx] = r0 + tx < n ? tile[tx][c] : 0;
     }
 }
 
@@ -181,18 +184,22 @@ int cpmk_transpose(int32_t batch, int32_t n, int32_t m, const void* inp, void* o
 }
 
 int cpmk_transpose_i8(int32_t batch, int32_t n, int32_t m, const void* inp, void* out, void* stream) {
+    return cpmk_transpose_i8_ld(batch, n, m, inp, m, out, n, stream);
+}
+
+int cpmk_transpose_i8_ld(int32_t batch, int32_t n, int32_t m, const void* inp, int32_t ld_in, void* out, int32_t ld_out, void* stream) {
     clear_stale_error();
-    if (batch < 0 || n < 0 || m < 0) return CPMK_EBADARG;
+    if (batch < 0 || n < 0 || m < 0 || ld_in < m || ld_out < n || (ld_out != n && ld_out % 16)) return CPMK_EBADARG;
     if ((int64_t)batch * n * m == 0) return 0;
     if (any_null(inp, out)) return CPMK_EBADARG;
-    if (ceil_div(n, 64) > 65535) return CPMK_ETOOBIG;
-    const bool win = m >= 16, wout = n >= 16;       // pieces of sixteen on a side whose rows hold at least one
+    if (ceil_div(ld_out, 64) > 65535) return CPMK_ETOOBIG;
+    const bool win = m >= 16, wout = ld_out >= 16;       // pieces of sixteen on a side whose rows hold at least one
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {       // (grid z: at most 65535 batch entries per launch)
         const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
-        const dim3 grid((unsigned)ceil_div(m, 64), (unsigned)ceil_div(n, 64), (unsigned)nb);
-        const int8_t* src = (const int8_t*)inp + b0 * n * m;
-        int8_t* dst = (int8_t*)out + b0 * n * m;
-        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, n, m, src, dst); };
+        const dim3 grid((unsigned)ceil_div(m, 64), (unsigned)ceil_div(ld_out, 64), (unsigned)nb);
+        const int8_t* src = (const int8_t*)inp + b0 * n * ld_in;
+        int8_t* dst = (int8_t*)out + b0 * m * ld_out;
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, n, m, ld_in, ld_out, src, dst); };
         if (win) { if (wout) go(k_transpose_i8<true, true>); else go(k_transpose_i8<true, false>); }
         else { if (wout) go(k_transpose_i8<false, true>); else go(k_transpose_i8<false, false>); }
         if (int e = launch_status()) return e;

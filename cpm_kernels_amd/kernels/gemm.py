@@ -129,6 +129,50 @@ def gemm_scale_y(batch: int, n: int, m: int,
     cpmk.gemm_scale_y(batch, n, m, mat, scale_y, out, _stream(stream))
 
 
+def gemm_int8_scale_one(m: int, k: int, n: int, batchA: int, batchB: int, aT: bool, bT: bool,
+                        A: DevicePointer, B: DevicePointer,
+                        scale_row: DevicePointer,   # as in gemm_int8_scale; one of the two may be None
+                        scale_col: DevicePointer,
+                        broad_cast_row: bool, broad_cast_col: bool,
+                        out: DevicePointer,         # (batch, n, m)  fp16
+                        stream: CUDAStream):
+    """gemm_int8 + gemm_scale_x / gemm_scale_y (kernels/gemm.py:309-347) in one launch."""
+    assert m % 4 == 0 and n % 4 == 0 and k % 4 == 0
+    assert batchA == batchB or batchA == 1 or batchB == 1
+    cpmk.gemm_int8_scale_one(m, k, n, batchA, batchB, 1 if aT else 0, 1 if bT else 0, A, B, scale_row, scale_col,
+                             1 if broad_cast_row else 0, 1 if broad_cast_col else 0, out, _stream(stream))
+
+
+def gemm_quantize_cols_ld(batch: int, n: int, m: int, mat: DevicePointer,
+                          row_scale: DevicePointer,   # (batch, n) fp16, (n) if broad_cast_row, or None
+                          broad_cast_row: bool,
+                          scale: DevicePointer,       # (batch, m)        fp16
+                          out_t: DevicePointer,       # (batch, m, ld_t)  int8, or None
+                          ld_t: int,
+                          out_n: DevicePointer,       # (batch, n, ld_n)  int8, or None
+                          ld_n: int,
+                          stream: CUDAStream):
+    """Per-column quantisation of mat (times row_scale: gemm_backward_scale_round) in the transposed and / or the matrix's
+    own layout, rows filled up with zeros to ld_t / ld_n bytes."""
+    cpmk.gemm_quantize_cols_ld(batch, n, m, mat, row_scale, 1 if broad_cast_row else 0, scale, out_t, ld_t, out_n, ld_n, _stream(stream))
+
+
+def gemm_quantize_pair_ld(rows0: int, mat0: DevicePointer, scale0: DevicePointer, out0: DevicePointer,
+                          rows1: int, mat1: DevicePointer, scale1: DevicePointer, out1: DevicePointer,
+                          m: int, ld: int, stream: CUDAStream):
+    """gemm_quantize_pair with int8 rows filled up with zeros to ld bytes; m <= 16384."""
+    cpmk.gemm_quantize_pair_ld(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, ld, _stream(stream))
+
+
+def gemm_backward_round_scale_ld(batch: int, n: int, m: int, mat: DevicePointer, scale_y: DevicePointer,
+                                 out: DevicePointer,        # (batch, n, ld)  int8
+                                 ld: int,
+                                 scale_x: DevicePointer,    # (batch, n)      fp16
+                                 broad_cast_y: bool, stream: CUDAStream):
+    """gemm_backward_round_scale with rows filled up with zeros to ld bytes."""
+    cpmk.gemm_backward_round_scale_ld(batch, n, m, mat, scale_y, out, ld, scale_x, 1 if broad_cast_y else 0, _stream(stream))
+
+
 def gemm_sum_groups(m: int, n: int, batch: int) -> int:
     """Partial sums that gemm_int8_scale_sum / gemm_fp16_sum form for (n, m) outputs over `batch` entries: as few as
     keep the device busy (a divisor of the batch)."""

@@ -18,3 +18,13 @@ def transpose_i8(batch: int, n: int, m: int,
     """The same for int8 tensors (no counterpart in the reference: its cuBLASLt product reads int8
     operands in either layout, kernels/gemm.py:127-186)."""
     cpmk.transpose_i8(batch, n, m, inp, out, _stream(stream))
+
+
+def transpose_i8_ld(batch: int, n: int, m: int,
+                    inp: DevicePointer,    # (batch, n, ld_in) int8, m columns of it
+                    ld_in: int,
+                    out: DevicePointer,    # (batch, m, ld_out) int8
+                    ld_out: int,
+                    stream: CUDAStream):
+    """transpose_i8 between rows of ld_in and ld_out bytes, the latter filled up with zeros."""
+    cpmk.transpose_i8_ld(batch, n, m, inp, ld_in, out, ld_out, _stream(stream))

@@ -8,8 +8,10 @@ the six-launch sequence, which ``fused=False`` still runs through the kernel-lev
 """
 import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
-    gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale, gemm_quantize, gemm_quantize_cols, \
-    gemm_quantize_pair, gemm_fp16, gemm_sum_groups, gemm_int8_scale_sum, gemm_fp16_sum, arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_scale_round, transpose, transpose_i8
+    gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
+    gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups, gemm_int8_scale_sum, gemm_fp16_sum, \
+    arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
+    transpose_i8, transpose_i8_ld
 from ._common import cur_stream
 
 
@@ -44,19 +46,42 @@ def quantize(mat: torch.Tensor, transpose: bool):
     return scale, out
 
 
-def quantize_k_major(mat: torch.Tensor, k_is_dim1: bool):
-    """Quantise along K and return (scale, int8 tensor with K as the last, contiguous dim):
-    for an operand stored (b, rows, K) that is `quantize(mat, False)`; for one stored (b, K, cols)
-    the per-column quantisation of `quantize(mat, True)` with the result written transposed,
-    (b, cols, K).  Same scales and int8 values either way."""
-    if not k_is_dim1:
-        return quantize(mat, False)
-    assert mat.is_contiguous() and mat.is_cuda and mat.dtype == torch.half
-    b, k, cols = mat.size()
-    scale = torch.empty((b, cols), dtype=torch.half, device=mat.device)
-    out = torch.empty((b, cols, k), dtype=torch.int8, device=mat.device)
-    gemm_quantize_cols(b, k, cols, mat.data_ptr(), scale.data_ptr(), out.data_ptr(), True, cur_stream())
-    return scale, out
+def _row_bytes(k: int) -> int:
+    """Bytes from one row of a quantised operand to the next when it is contracted over its k columns: whole 128-byte slabs
+    of the tile kernel, the surplus zeros, which add nothing (NS shape with K = 4100: 150 us, 233-250 with the rest of each
+    row taken on its own; K = 4032 also ran 5-10 % behind on 64-byte slabs).  Short rows of whole 64-byte slabs stay as they are."""
+    return k if k % 128 == 0 or k > 16384 or (k % 64 == 0 and k < 1024) else (k + 127) // 128 * 128
+
+
+def _quantize_rows(*mats):
+    """One or two (b, rows, K) operands quantised along K in one launch: [(scale (b, rows), int8 (b, rows, _row_bytes(K)))]"""
+    K = mats[0].size(2)
+    ld = _row_bytes(K)
+    if K > 16384:
+        return [quantize(x, False) for x in mats]
+    out = [(torch.empty(x.shape[:2], dtype=torch.half, device=x.device),
+            torch.empty((x.size(0), x.size(1), ld), dtype=torch.int8, device=x.device)) for x in mats]
+    args = []
+    for x, (s, q) in zip(mats, out):
+        args += [x.size(0) * x.size(1), x.data_ptr(), s.data_ptr(), q.data_ptr()]
+    if len(mats) == 1:
+        args += [0, 0, 0, 0]
+    gemm_quantize_pair_ld(*args, K, ld, cur_stream())
+    return out
+
+
+def _quantize_cols(x, both: bool, row_scale=None):
+    """A (b, n, m) operand quantised along n: scale (b, m), int8 (b, m, _row_bytes(n)) and, with `both`, the same values
+    where they were, (b, n, _row_bytes(m)) (else None).  row_scale: of the values multiplied by it, see gemm_backward_scale_round."""
+    b, n, m = x.size()
+    scale = torch.empty((b, m), dtype=torch.half, device=x.device)
+    ld_t, ld_n = (n + 15) // 16 * 16 if n > 16384 else _row_bytes(n), _row_bytes(m) if both else 0
+    out_t = torch.empty((b, m, ld_t), dtype=torch.int8, device=x.device)
+    out_n = torch.empty((b, n, ld_n), dtype=torch.int8, device=x.device) if both else None
+    gemm_quantize_cols_ld(b, n, m, x.data_ptr(), None if row_scale is None else row_scale.data_ptr(),
+                          row_scale is not None and row_scale.size(0) == 1, scale.data_ptr(), out_t.data_ptr(), ld_t,
+                          out_n.data_ptr() if both else None, ld_n, cur_stream())
+    return scale, out_t, out_n
 
 
 def _dims(quantA, quantB, aT, bT):
@@ -74,23 +99,11 @@ def gemm_and_scale(quantA, scaleA, quantB, scaleB, aT, bT, fused=True) -> torch.
     batch = max(quantA.size(0), quantB.size(0))
     result_fp = torch.empty((batch, M, N), dtype=torch.float16, device=quantA.device)
     if fused:
-        # The MFMA tile kernel reads both operands with K contiguous; an int8 operand given the other
-        # way round (the backward products) costs one transposed copy, far less than the general kernel.
-        if aT:
-            quantA, aT = _transposed_copy_i8(quantA), False
-        if not bT:
-            quantB, bT = _transposed_copy_i8(quantB), True
-        # A missing scale is a vector of ones: (acc * s) * 1 rounds exactly as gemm_scale_x / gemm_scale_y
-        # do, and the int32 accumulators never travel through memory.
-        if scaleA is None:
-            scaleA = torch.ones((1, M), dtype=torch.half, device=quantA.device)
-        if scaleB is None:
-            scaleB = torch.ones((1, N), dtype=torch.half, device=quantA.device)
-        gemm_int8_scale(N, K, M, quantB.size(0), quantA.size(0), bT, aT,
-                        quantB.data_ptr(), quantA.data_ptr(),
-                        scaleA.data_ptr(), scaleB.data_ptr(),
-                        scaleA.size(0) == 1, scaleB.size(0) == 1,
-                        result_fp.data_ptr(), cur_stream())
+        gemm_int8_scale_one(N, K, M, quantB.size(0), quantA.size(0), bT, aT,
+                            quantB.data_ptr(), quantA.data_ptr(),
+                            None if scaleA is None else scaleA.data_ptr(), None if scaleB is None else scaleB.data_ptr(),
+                            scaleA is None or scaleA.size(0) == 1, scaleB is None or scaleB.size(0) == 1,
+                            result_fp.data_ptr(), cur_stream())
         return result_fp
     result_i32 = torch.empty((batch, M, N), dtype=torch.int32, device=quantA.device)
     gemm_int8(N, K, M, quantB.size(0), quantA.size(0), bT, aT,
@@ -120,10 +133,8 @@ def gemm_and_scale_sum(quantA, scaleA, quantB) -> torch.Tensor:
     batch, M, K = quantA.size()
     N = quantB.size(1)
     groups = gemm_sum_groups(N, M, batch)
-    if groups == batch or quantB.size(0) != batch or max(M, N) * K >= 2 ** 31 or batch * K >= 2 ** 22:
+    if groups == batch or quantB.size(0) != batch or K % 128 != 0 or max(M, N) * K >= 2 ** 31 or batch * K >= 2 ** 22:
         return _sum_entries(gemm_and_scale(quantA, scaleA, quantB, None, False, True))
-    if K % 128 != 0:
-        quantA, quantB = _zero_padded_i8(quantA), _zero_padded_i8(quantB)
     parts = torch.empty((groups, M, N), dtype=torch.half, device=quantA.device)
     gemm_int8_scale_sum(N, quantA.size(2), M, batch, groups, quantB.data_ptr(), quantA.data_ptr(), scaleA.data_ptr(),
                         parts.data_ptr(), cur_stream())
@@ -132,38 +143,46 @@ def gemm_and_scale_sum(quantA, scaleA, quantB) -> torch.Tensor:
 
 class GEMMInt8(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool, fused: bool = True):
+    def forward(ctx, A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool, fused: bool = True, train: bool = True):
         """A: (batchA, M, K) [(batchA, K, M) if aT], B: (batchB, K, N) [(batchB, N, K) if bT]
         -> (batch, M, N) fp16.  reference: torch/gemm.py:84-113"""
         assert A.is_cuda and B.is_cuda and A.device == B.device
         assert A.is_contiguous() and B.is_contiguous()
         assert A.dtype == torch.half and B.dtype == torch.half
-        if fused:
-            # both operands are brought to K-major int8 while they are quantised, so every
-            # layout runs on the fast GEMM kernel: A (bA, M, K) and B (bB, N, K)
-            if not aT and bT and A.size(2) == B.size(2):
-                # both already K-major: one launch quantises the two of them
-                scale_A = torch.empty(A.shape[:2], dtype=torch.half, device=A.device)
-                scale_B = torch.empty(B.shape[:2], dtype=torch.half, device=A.device)
-                quantized_A = torch.empty(A.shape, dtype=torch.int8, device=A.device)
-                quantized_B = torch.empty(B.shape, dtype=torch.int8, device=A.device)
-                gemm_quantize_pair(A.size(0) * A.size(1), A.data_ptr(), scale_A.data_ptr(), quantized_A.data_ptr(),
-                                   B.size(0) * B.size(1), B.data_ptr(), scale_B.data_ptr(), quantized_B.data_ptr(),
-                                   A.size(2), cur_stream())
-            else:
-                scale_A, quantized_A = quantize_k_major(A, aT)
-                scale_B, quantized_B = quantize_k_major(B, not bT)
-            # the int8 tensors are held as (bA, M, K) and (bB, N, K) whatever the operand layout was
-            ctx.stored = (False, True)
-        else:
+        ctx.layout = (aT, bT)
+        ctx.fused = fused
+        if not fused:
             scale_A = calc_scale(A, aT)
             scale_B = calc_scale(B, not bT)
             quantized_A = round_i8(A, scale_A, aT)
             quantized_B = round_i8(B, scale_B, not bT)
-            ctx.stored = (aT, bT)
-        ctx.save_for_backward(scale_A, quantized_A, scale_B, quantized_B)
-        ctx.layout = (aT, bT)
-        return gemm_and_scale(quantized_A, scale_A, quantized_B, scale_B, ctx.stored[0], ctx.stored[1], fused)
+            ctx.save_for_backward(scale_A, quantized_A, scale_B, quantized_B)
+            return gemm_and_scale(quantized_A, scale_A, quantized_B, scale_B, aT, bT, False)
+        # Both operands are brought to K-major int8 while they are quantised, so every layout runs on the fast GEMM kernel:
+        # A (bA, M, ld) and B (bB, N, ld).  An operand that is quantised along its columns and whose partner wants a gradient
+        # also leaves its int8 values where they were: that product is contracted over its other dimension.
+        M, K, N = _dims(A, B, aT, bT)
+        assert M % 4 == 0 and K % 4 == 0 and N % 4 == 0
+        want_A, want_B = train and ctx.needs_input_grad[0], train and ctx.needs_input_grad[2]
+        own_A = own_B = None
+        if not aT and bT:
+            (scale_A, quant_A), (scale_B, quant_B) = _quantize_rows(A, B)
+        else:
+            if aT:
+                scale_A, quant_A, own_A = _quantize_cols(A, want_B)
+            else:
+                (scale_A, quant_A), = _quantize_rows(A)
+            if bT:
+                (scale_B, quant_B), = _quantize_rows(B)
+            else:
+                scale_B, quant_B, own_B = _quantize_cols(B, want_A)
+        if quant_A.size(2) != quant_B.size(2):      # (contractions beyond what the row quantiser holds in registers)
+            quant_A, quant_B = (x[:, :, :K].contiguous() for x in (quant_A, quant_B))
+        if train:
+            ctx.dims = (M, K, N)
+            ctx.own = (own_A is not None, own_B is not None)
+            ctx.save_for_backward(scale_A, quant_A if own_A is None else own_A, scale_B, quant_B if own_B is None else own_B)
+        return gemm_and_scale(quant_A, scale_A, quant_B, scale_B, False, True)
 
     @staticmethod
     def backward(ctx, grad_f: torch.Tensor):
@@ -172,46 +191,49 @@ class GEMMInt8(torch.autograd.Function):
         scales only (the other operand's scales went into the gradient before rounding)."""
         assert grad_f.is_contiguous() and grad_f.is_cuda and grad_f.dtype == torch.float16
         scale_A, quantized_A, scale_B, quantized_B = ctx.saved_tensors
-        aT, bT = ctx.stored
+        aT, bT = ctx.layout
         batch, m, n = grad_f.size()
         st = cur_stream()
-
+        if ctx.fused:
+            # Each gradient is formed directly in the layout its operand came in, summed inside the product where the operand was
+            # broadcast over the batch.
+            M, K, N = ctx.dims
+            own_A, own_B = ctx.own
+            grad_A = grad_B = None
+            if ctx.needs_input_grad[0]:                                     # contracted over N
+                ld = _row_bytes(N)
+                scale_G = torch.empty((batch, M), dtype=torch.half, device=grad_f.device)
+                quant_G = torch.empty((batch, M, ld), dtype=torch.int8, device=grad_f.device)
+                gemm_backward_round_scale_ld(batch, M, N, grad_f.data_ptr(), scale_B.data_ptr(), quant_G.data_ptr(), ld,
+                                             scale_G.data_ptr(), scale_B.size(0) == 1, st)
+                summed = scale_A.size(0) == 1 and batch > 1 and not aT
+                other, lies = _contracted(quantized_B, K, N, ld, own_B, summed)
+                if aT:              # grad_A (b, K, M), scaled per column m
+                    grad_A = gemm_and_scale(other, None, quant_G, scale_G, lies, True)
+                elif summed:
+                    grad_A = gemm_and_scale_sum(quant_G, scale_G, other)
+                else:               # grad_A (b, M, K), scaled per row m
+                    grad_A = gemm_and_scale(quant_G, scale_G, other, None, False, not lies)
+                del quant_G, other
+                if scale_A.size(0) == 1 and grad_A.size(0) > 1:
+                    grad_A = grad_A.sum(dim=0, keepdim=True)
+            if ctx.needs_input_grad[2]:                                     # contracted over M
+                scale_G, quant_G, _ = _quantize_cols(grad_f, False, scale_A)
+                summed = scale_B.size(0) == 1 and batch > 1 and bT
+                other, lies = _contracted(quantized_A, K, M, quant_G.size(2), own_A, summed)
+                if summed:
+                    grad_B = gemm_and_scale_sum(quant_G, scale_G, other)
+                elif bT:            # grad_B (b, N, K), scaled per row n
+                    grad_B = gemm_and_scale(quant_G, scale_G, other, None, False, not lies)
+                else:               # grad_B (b, K, N), scaled per column n
+                    grad_B = gemm_and_scale(other, None, quant_G, scale_G, lies, True)
+                if scale_B.size(0) == 1 and grad_B.size(0) > 1:
+                    grad_B = grad_B.sum(dim=0, keepdim=True)
+            return grad_A, None, grad_B, None, None, None
         scale_G_a = torch.empty((batch, m), dtype=torch.half, device=grad_f.device)
         quant_G_a = torch.empty((batch, m, n), dtype=torch.int8, device=grad_f.device)
         gemm_backward_round_scale(batch, m, n, grad_f.data_ptr(), scale_B.data_ptr(), quant_G_a.data_ptr(),
                                   scale_G_a.data_ptr(), scale_B.size(0) == 1, st)
-        if ctx.stored == (False, True):
-            # The fused forward holds quantized_A as (bA, M, K) and quantized_B as (bB, N, K).  Each gradient is
-            # formed directly in the layout its operand came in, from operands with the contraction index
-            # contiguous: no product on the general kernel and no transposition of a result.
-            in_aT, in_bT = ctx.layout
-            qB_t = _rows_padded_i8(_transposed_copy_i8(quantized_B))    # (bB, K, N)
-            quant_G_a = _rows_padded_i8(quant_G_a)                      # both contracted over N
-            if in_aT:       # grad_A (b, K, M) = qB_t x quant_G_a^T, scaled per column m
-                grad_A = gemm_and_scale(qB_t, None, quant_G_a, scale_G_a, False, True)
-            elif scale_A.size(0) == 1:      # ... summed over the batch that A was broadcast over
-                grad_A = gemm_and_scale_sum(quant_G_a, scale_G_a, qB_t)
-            else:           # grad_A (b, M, K) = quant_G_a x qB_t^T, scaled per row m
-                grad_A = gemm_and_scale(quant_G_a, scale_G_a, qB_t, None, False, True)
-            del scale_G_a, quant_G_a, qB_t
-            scale_G_b = torch.empty((batch, n), dtype=torch.half, device=grad_f.device)
-            quant_G_b = torch.empty((batch, m, n), dtype=torch.int8, device=grad_f.device)
-            gemm_backward_scale_round(batch, m, n, grad_f.data_ptr(), scale_A.data_ptr(), quant_G_b.data_ptr(),
-                                      scale_G_b.data_ptr(), scale_A.size(0) == 1, st)
-            qG_t = _rows_padded_i8(_transposed_copy_i8(quant_G_b))      # (b, N, M)
-            del quant_G_b
-            qA_t = _rows_padded_i8(_transposed_copy_i8(quantized_A))    # (bA, K, M); both contracted over M
-            if in_bT and scale_B.size(0) == 1:      # summed over the batch that B was broadcast over
-                grad_B = gemm_and_scale_sum(qG_t, scale_G_b, qA_t)
-            elif in_bT:     # grad_B (b, N, K) = qG_t x qA_t^T, scaled per row n
-                grad_B = gemm_and_scale(qG_t, scale_G_b, qA_t, None, False, True)
-            else:           # grad_B (b, K, N) = qA_t x qG_t^T, scaled per column n
-                grad_B = gemm_and_scale(qA_t, None, qG_t, scale_G_b, False, True)
-            if scale_A.size(0) == 1 and grad_A.size(0) > 1:
-                grad_A = grad_A.sum(dim=0, keepdim=True)
-            if scale_B.size(0) == 1 and grad_B.size(0) > 1:
-                grad_B = grad_B.sum(dim=0, keepdim=True)
-            return grad_A, None, grad_B, None, None
         if aT:
             grad_A = gemm_and_scale(quantized_B, None, quant_G_a, scale_G_a, bT, True)
         else:
@@ -231,34 +253,22 @@ class GEMMInt8(torch.autograd.Function):
             grad_A = grad_A.sum(dim=0, keepdim=True)
         if scale_B.size(0) == 1 and grad_B.size(0) > 1:
             grad_B = grad_B.sum(dim=0, keepdim=True)
-        # back to the layout the operands came in
-        if ctx.layout[0] != aT:
-            grad_A = grad_A.transpose(1, 2).contiguous()
-        if ctx.layout[1] != bT:
-            grad_B = grad_B.transpose(1, 2).contiguous()
-        return grad_A, None, grad_B, None, None
+        return grad_A, None, grad_B, None, None, None
 
 
-def _transposed_copy_i8(x: torch.Tensor) -> torch.Tensor:
-    out = torch.empty((x.size(0), x.size(2), x.size(1)), dtype=torch.int8, device=x.device)
-    transpose_i8(x.size(0), x.size(1), x.size(2), x.data_ptr(), out.data_ptr(), cur_stream())
-    return out
-
-
-def _rows_padded_i8(x: torch.Tensor) -> torch.Tensor:
-    """A (b, r, k) operand that is contracted over k, with its rows lengthened by zeros to a multiple of 128
-    bytes when k is not a multiple of 64: padded on both operands of a product the zeros add nothing, and the
-    tile kernel's whole-slab path applies whatever k is (at k = 500 it is several times faster than the kernels
-    for ragged rows, and the copy costs two passes over the operand)."""
-    k = x.size(2)
-    return x if k % 64 == 0 or k < 128 else _zero_padded_i8(x)
-
-
-def _zero_padded_i8(x: torch.Tensor) -> torch.Tensor:
-    k = x.size(2)
-    padded = torch.zeros((x.size(0), x.size(1), (k + 127) // 128 * 128), dtype=torch.int8, device=x.device)
-    padded[:, :, :k].copy_(x)
-    return padded
+def _contracted(q, K, length, ld, own, must_copy):
+    """The saved int8 values of an operand -- (b, length, K-major rows), or with `own` (b, K, length padded) -- for a product
+    contracted over `length`: (operand, whether it lies as (b, length, K)).  The tile kernel reads it as it lies where rows and
+    length are whole pieces and slabs, 8 % slower than from (b, K, ld), which is less than the transposition costs."""
+    if own and q.size(2) == ld:
+        return q, False
+    if own:
+        q, own = q[:, :, :length].transpose(1, 2).contiguous(), False       # (a padding of another length: only past 16384)
+    if not must_copy and q.size(2) == K and length == ld and length % 128 == 0 and K % 16 == 0:
+        return q, True
+    out = torch.empty((q.size(0), K, ld), dtype=torch.int8, device=q.device)
+    transpose_i8_ld(q.size(0), length, K, q.data_ptr(), q.size(2), out.data_ptr(), ld, cur_stream())
+    return out, False
 
 
 def _transposed_copy(x: torch.Tensor) -> torch.Tensor:
@@ -269,16 +279,16 @@ def _transposed_copy(x: torch.Tensor) -> torch.Tensor:
 
 def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch.Tensor:
     """reference: torch/gemm.py:189-203; operands are passed swapped to the kernel so that the
-    (M, N) result comes out row-major.  The MFMA tile kernel is fastest with K as the contiguous
-    dimension of both operands (A as (b, M, K), B as (b, N, K)).  An operand given the other way
-    round is read as it lies (2-byte LDS reads build the MFMA fragments, 20-60 % more time in
-    the product) unless the product is so large next to the operand that one transposed copy of it
-    is cheaper: measured break-even at about 2048 rows of the other operand for B, 512 for A."""
+    (M, N) result comes out row-major.  The MFMA tile kernel reads an operand stored (K, rows) as it lies, at 2-8 % more time
+    than K-major ones: a transposed copy pays only for products very large next to the operand.  Measured (direct / with a copy):
+    8 x 4096 x 4096 x 512, B transposed 108 / 121 us, A 109 / 118; 4 x 1024 x 4096 x 512 34 / 40-44; 8192 x 4096 x 4096 204 / 208;
+    8 x 10240 x 4096 x 512, B transposed 298 / 279; 4096 x 4096 x 10240, A transposed 298 / 275.  Rows of A that are
+    not whole 16-byte pieces are copied always."""
     M, K, N = _dims(A, B, aT, bT)
     if K % 64 == 0 and N % 8 == 0 and M * K < 2 ** 31 and N * K < 2 ** 31:
-        if aT and ((N > 512 and K > 128) or M % 8 != 0):     # (short K: the product is bound by writing its output)
+        if aT and ((N * (B.size(0) // A.size(0)) > 8192 and K > 128) or M % 8 != 0):     # (short K: the product is bound by writing its output)
             A, aT = _transposed_copy(A), False
-        if not bT and M > 2048 and K > 128:
+        if not bT and M > 8192 and K > 128:
             B, bT = _transposed_copy(B), True
     out = torch.empty((max(A.size(0), B.size(0)), M, N), dtype=torch.half, device=A.device)
     gemm_fp16(N, K, M, B.size(0), A.size(0), bT, aT, B.data_ptr(), A.data_ptr(), out.data_ptr(), cur_stream())
@@ -332,5 +342,5 @@ def bmm(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool, int8: bool = False
     assert A.ndim == 3
     assert B.ndim == 3
     if int8:
-        return GEMMInt8.apply(A, aT, B, bT, fused)
+        return GEMMInt8.apply(A, aT, B, bT, fused, torch.is_grad_enabled())
     return GEMMFloat.apply(A, aT, B, bT)

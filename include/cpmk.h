@@ -138,6 +138,11 @@ int cpmk_gemm_int8_scale(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
                          const void* scale_col /* fp16, per out col i */,
                          int broad_cast_row, int broad_cast_col,
                          void* out /* fp16 */, void* stream);
+/* ... where one of the scales may be null: the accumulator is then scaled along the other side only (gemm_scale_x / gemm_scale_y
+ * of the backward products). */
+int cpmk_gemm_int8_scale_one(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT,
+                             const void* A, const void* B, const void* scale_row, const void* scale_col,
+                             int broad_cast_row, int broad_cast_col, void* out, void* stream);
 
 /* Fused absmax + round of cpm_kernels/torch/gemm.py:5-38 (calc_scale then round_i8 on the
  * same tensor): one read of mat, writes scale and the int8 tensor.  transpose = 0 uses
@@ -153,6 +158,10 @@ int cpmk_gemm_quantize(int32_t batch, int32_t n, int32_t m, const void* mat,
 int cpmk_gemm_quantize_pair(int64_t rows0, const void* mat0, void* scale0, void* out0,
                             int64_t rows1, const void* mat1, void* scale1, void* out1,
                             int32_t m, void* stream);
+/* ... with the int8 rows filled up with zeros to ld bytes (m, or a multiple of 16 up to the next multiple of 128), so that a product
+ * contracts over whole slabs whatever m is.  m <= 16384. */
+int cpmk_gemm_quantize_pair_ld(int64_t rows0, const void* mat0, void* scale0, void* out0, int64_t rows1, const void* mat1,
+                               void* scale1, void* out1, int32_t m, int32_t ld, void* stream);
 
 /* Per-column scales (b,m) and rounding in one pass, as cpmk_gemm_quantize with transpose = 1
  * (cpm_kernels/torch/gemm.py:98-102 for an operand given as (b, K, N)), with the int8 result
@@ -162,6 +171,12 @@ int cpmk_gemm_quantize_pair(int64_t rows0, const void* mat0, void* scale0, void*
  * bit-identical to calc_scale_transpose + round_transpose. */
 int cpmk_gemm_quantize_cols(int32_t batch, int32_t n, int32_t m, const void* mat,
                             void* scale, void* out, int out_transposed, void* stream);
+/* The same with everything a product that is differentiated needs: values optionally multiplied by row_scale (batch, n) -- (n) with
+ * broad_cast_row -- as cpmk_gemm_backward_scale_round does; out_t (batch, m, ld_t) the transposed and out_n (batch, n, ld_n) the untransposed
+ * int8 values (null: not wanted; both only without row scales).  Rows are filled up with zeros to ld_t resp. ld_n bytes
+ * (a multiple of 16; ld_n may be m). */
+int cpmk_gemm_quantize_cols_ld(int32_t batch, int32_t n, int32_t m, const void* mat, const void* row_scale, int broad_cast_row,
+                               void* scale, void* out_t, int32_t ld_t, void* out_n, int32_t ld_n, void* stream);
 
 /* ---- fp16 products next to the path (attention scores, fp16 decode) ---------------- */
 /* Same operand convention as cpmk_gemm_int8 with fp16 operands and fp16 output, fp32
@@ -356,6 +371,9 @@ int cpmk_layernorm_backward_mv(int32_t batch, int32_t n, int32_t m, const void* 
  *                                                     kernels/gemm.py:261-283 / gemm.cu:102-133 */
 int cpmk_gemm_backward_round_scale(int32_t batch, int32_t n, int32_t m, const void* mat, const void* scale_y,
                                    void* out, void* scale_x, int broad_cast_y, void* stream);
+/* ... with rows of the output filled up with zeros to ld bytes (m, or a multiple of 16 up to the next multiple of 128) */
+int cpmk_gemm_backward_round_scale_ld(int32_t batch, int32_t n, int32_t m, const void* mat, const void* scale_y, void* out, int32_t ld,
+                                      void* scale_x, int broad_cast_y, void* stream);
 /* The same along dim 1: scale_y[b,j] from max_i |mat*scale_x|.   kernels/gemm.py:285-307 / gemm.cu:136-172 */
 int cpmk_gemm_backward_scale_round(int32_t batch, int32_t n, int32_t m, const void* mat, const void* scale_x,
                                    void* out, void* scale_y, int broad_cast_x, void* stream);
@@ -382,6 +400,8 @@ int cpmk_transpose(int32_t batch, int32_t n, int32_t m, const void* inp, void* o
  * int8 operands in either layout (kernels/gemm.py:127-186): the backward products of
  * torch/gemm.py:115-186 use this to bring their operands to the layout of the MFMA tile kernel. */
 int cpmk_transpose_i8(int32_t batch, int32_t n, int32_t m, const void* inp, void* out, void* stream);
+/* ... between rows of ld_in and ld_out bytes (ld_in >= m; ld_out >= n, the surplus filled with zeros) */
+int cpmk_transpose_i8_ld(int32_t batch, int32_t n, int32_t m, const void* inp, int32_t ld_in, void* out, int32_t ld_out, void* stream);
 /* array[pos] += val (int32).                          kernels/utils.py:39-53 / utils.cu:31-35 */
 int cpmk_array_add(void* array, int32_t pos, int32_t val, void* stream);
 /* logits = logits / temperature - frequency_penalty*freq - presence_penalty*(freq > 0), in place.

@@ -1,6 +1,7 @@
 // Normalisation over dim 1 of (batch, n, m) fp16 and over contiguous rows (decode step):
 //   mean = rd_mean ? sum x / n : 0;  var = sum x^2 / n - mean^2;
 //   y = fp16( (x - mean) * rsqrt(var + eps) )            (cuda/layernorm.cu:6-71, :343-381)
+// (mean and the reciprocal deviation of every column optionally kept for the backward pass, fp32)
 // optionally followed, on the fp16-rounded y, by the affine of cu_arith_ln_mul_add /
 // cu_arith_ln_mul (cuda/arith.cu:97-127): fp16 fma(y, alpha[i], beta[i]) or y * alpha[i].
 #include "dim1.h"
@@ -32,7 +33,7 @@ __global__ __launch_bounds__(NT) void k_layernorm_tile(int32_t n, int32_t m, int
                                                        const half_t* mat, half_t* out,
                                                        const half_t* __restrict__ alpha,
                                                        const half_t* __restrict__ beta, float eps,
-                                                       int rd_mean) {
+                                                       int rd_mean, float* __restrict__ stats) {
     using T = ColTile<NT, LPR, R>;
     __shared__ float lds[(T::NW + 1) * T::COLS * 2];
     __shared__ half_t coef[2][T::ROWS];   // alpha and beta of the tile's rows
@@ -93,6 +94,16 @@ __global__ __launch_bounds__(NT) void k_layernorm_tile(int32_t n, int32_t m, int
         rstd[e] = rsqrtf(var + eps);
     }
     const int rg = threadIdx.x / LPR;
+    if constexpr (AFF) {
+        if (stats != nullptr && rg == 0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (col0 + e < m) {
+                    stats[(int64_t)b * 2 * m + col0 + e] = mean[e];
+                    stats[((int64_t)b * 2 + 1) * m + col0 + e] = rstd[e];
+                }
+        }
+    }
 #pragma unroll
     for (int p = 0; p < R; ++p) {
         half8_t y;
@@ -115,7 +126,7 @@ __global__ __launch_bounds__(NT) void k_layernorm_team(int32_t n, int32_t m, int
                                                        const half_t* mat, half_t* out,
                                                        const half_t* __restrict__ alpha,
                                                        const half_t* __restrict__ beta, float eps, int rd_mean,
-                                                       uint32_t nteams, XchLaunch xl) {
+                                                       float* __restrict__ stats, uint32_t nteams, XchLaunch xl) {
     constexpr int LPR = 8;
     using T = ColTile<NT, LPR, R>;
     static_assert(T::COLS * 2 == kXchVals, "slot layout");
@@ -190,8 +201,16 @@ __global__ __launch_bounds__(NT) void k_layernorm_team(int32_t n, int32_t m, int
             mu = sum / fn;
             var -= mu * mu;
         }
+        const float rs = ok ? rsqrtf(var + eps) : __builtin_nanf("");
         tot[tid] = mu;
-        tot[T::COLS + tid] = ok ? rsqrtf(var + eps) : __builtin_nanf("");
+        tot[T::COLS + tid] = rs;
+        if constexpr (AFF) {
+            const int32_t c = (int32_t)(ct * T::COLS) + tid;
+            if (stats != nullptr && part == 0 && c < m) {
+                stats[(int64_t)b * 2 * m + c] = mu;
+                stats[((int64_t)b * 2 + 1) * m + c] = rs;
+            }
+        }
         if (!ok) xch_flag(xl, kXchStatusTimeout);
     }
     __syncthreads();
@@ -220,7 +239,7 @@ __global__ __launch_bounds__(NT) void k_layernorm_team(int32_t n, int32_t m, int
 __global__ __launch_bounds__(256) void k_layernorm_generic(int32_t n, int32_t m, const half_t* mat, half_t* out,
                                                            const half_t* __restrict__ alpha,
                                                            const half_t* __restrict__ beta, float eps,
-                                                           int rd_mean) {
+                                                           int rd_mean, float* __restrict__ stats) {
     __shared__ float red[2][4][64];
     const int c = threadIdx.x & 63, rg = threadIdx.x >> 6;
     const int32_t col = blockIdx.x * 64 + c;
@@ -245,6 +264,10 @@ __global__ __launch_bounds__(256) void k_layernorm_generic(int32_t n, int32_t m,
         var -= mean * mean;
     }
     const float rstd = rsqrtf(var + eps);
+    if (stats != nullptr && rg == 0 && col < m) {
+        stats[(int64_t)blockIdx.y * 2 * m + col] = mean;
+        stats[((int64_t)blockIdx.y * 2 + 1) * m + col] = rstd;
+    }
     if (col < m) {
         for (int32_t i = rg; i < n; i += 4) {
             const int64_t o = boff + (int64_t)i * m + col;
@@ -281,24 +304,24 @@ __global__ __launch_bounds__(256) void k_layernorm_rows(int32_t n, const half_t*
 
 template <int LPR, int R, int MODE = 0>
 static void launch_tile(int32_t batch, int32_t n, int32_t m, const half_t* mat, half_t* out, const half_t* alpha,
-                        const half_t* beta, float eps, int rd_mean, hipStream_t st) {
+                        const half_t* beta, float eps, int rd_mean, float* stats, hipStream_t st) {
     constexpr int NT = 1024;
     const int32_t tiles = (int32_t)ceil_div(m, LPR * 8);
     if (alpha != nullptr)
         hipLaunchKernelGGL((k_layernorm_tile<NT, LPR, R, true, MODE>), dim3((unsigned)((int64_t)tiles * batch)), dim3(NT), 0, st, n,
-                           m, tiles, mat, out, alpha, beta, eps, rd_mean);
+                           m, tiles, mat, out, alpha, beta, eps, rd_mean, stats);
     else
         hipLaunchKernelGGL((k_layernorm_tile<NT, LPR, R, false, MODE>), dim3((unsigned)((int64_t)tiles * batch)), dim3(NT), 0, st, n,
-                           m, tiles, mat, out, alpha, beta, eps, rd_mean);
+                           m, tiles, mat, out, alpha, beta, eps, rd_mean, stats);
 }
 
 template <int LPR, int MODE = 0>
 static bool launch_tile_r(int r, int32_t batch, int32_t n, int32_t m, const half_t* mat, half_t* out,
-                          const half_t* alpha, const half_t* beta, float eps, int rd_mean, hipStream_t st) {
-    if (r <= 1) launch_tile<LPR, 1, MODE>(batch, n, m, mat, out, alpha, beta, eps, rd_mean, st);
-    else if (r <= 2) launch_tile<LPR, 2, MODE>(batch, n, m, mat, out, alpha, beta, eps, rd_mean, st);
-    else if (r <= 4) launch_tile<LPR, 4, MODE>(batch, n, m, mat, out, alpha, beta, eps, rd_mean, st);
-    else if (r <= 8) launch_tile<LPR, 8, MODE>(batch, n, m, mat, out, alpha, beta, eps, rd_mean, st);
+                          const half_t* alpha, const half_t* beta, float eps, int rd_mean, float* stats, hipStream_t st) {
+    if (r <= 1) launch_tile<LPR, 1, MODE>(batch, n, m, mat, out, alpha, beta, eps, rd_mean, stats, st);
+    else if (r <= 2) launch_tile<LPR, 2, MODE>(batch, n, m, mat, out, alpha, beta, eps, rd_mean, stats, st);
+    else if (r <= 4) launch_tile<LPR, 4, MODE>(batch, n, m, mat, out, alpha, beta, eps, rd_mean, stats, st);
+    else if (r <= 8) launch_tile<LPR, 8, MODE>(batch, n, m, mat, out, alpha, beta, eps, rd_mean, stats, st);
     else return false;
     return true;
 }
@@ -308,7 +331,7 @@ static bool launch_tile_r(int r, int32_t batch, int32_t n, int32_t m, const half
 // names (fixed_slots of them) and a shape that needs more is refused with CPMK_ETOOBIG.
 static int layernorm_dispatch(int32_t batch, int32_t n, int32_t m, const void* mat, void* out, const void* alpha,
                               const void* beta, float eps, int rd_mean, hipStream_t st, const XchLaunch* fixed = nullptr,
-                              int64_t fixed_slots = 0) {
+                              int64_t fixed_slots = 0, float* stats = nullptr) {
     if (batch < 0 || n < 0 || m < 0) return CPMK_EBADARG;
     if ((int64_t)batch * n * m == 0) return 0;
     if (any_null(mat, out)) return CPMK_EBADARG;
@@ -361,7 +384,7 @@ static int layernorm_dispatch(int32_t batch, int32_t n, int32_t m, const void* m
                     half_t* yb = y + b0 * n * m;
                     auto go = [&](auto kern, int threads) {
                         hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, n, m, (int32_t)tiles, (int32_t)parts, xb, yb, al, be, eps,
-                                           rd_mean, (uint32_t)(tiles * nb), xl);
+                                           rd_mean, stats ? stats + b0 * 2 * m : nullptr, (uint32_t)(tiles * nb), xl);
                     };
                     auto pick = [&](auto modec) {
                         constexpr int MODE = decltype(modec)::value;
@@ -383,18 +406,18 @@ static int layernorm_dispatch(int32_t batch, int32_t n, int32_t m, const void* m
                 if (!no_slots) return 0;
             }
         }
-        if (!wide) ok = n <= 128 * 8 && launch_tile_r<8, 2>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, st);
-        else if (n <= 128 * 8 && m >= 64 && !lines) ok = launch_tile_r<8, 1>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, st);
-        else if (n <= 128 * 8 && m >= 64) ok = launch_tile_r<8>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, st);
-        else if (n <= 256 * 8 && m >= 32) ok = launch_tile_r<4>((int)ceil_div(n, 256), batch, n, m, x, y, al, be, eps, rd_mean, st);
-        else ok = launch_tile_r<2>((int)ceil_div(n, 512), batch, n, m, x, y, al, be, eps, rd_mean, st);
+        if (!wide) ok = n <= 128 * 8 && launch_tile_r<8, 2>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
+        else if (n <= 128 * 8 && m >= 64 && !lines) ok = launch_tile_r<8, 1>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
+        else if (n <= 128 * 8 && m >= 64) ok = launch_tile_r<8>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
+        else if (n <= 256 * 8 && m >= 32) ok = launch_tile_r<4>((int)ceil_div(n, 256), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
+        else ok = launch_tile_r<2>((int)ceil_div(n, 512), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
         if (ok) return launch_status();
     }
     // the batch is the grid's y dimension (at most 65535): larger batches go out in several launches
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
         const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;
         hipLaunchKernelGGL(k_layernorm_generic, dim3((unsigned)ceil_div(m, 64), (unsigned)nb), dim3(256), 0, st, n, m,
-                           x + b0 * n * m, y + b0 * n * m, al, be, eps, rd_mean);
+                           x + b0 * n * m, y + b0 * n * m, al, be, eps, rd_mean, stats ? stats + b0 * 2 * m : nullptr);
         if (int e = launch_status()) return e;
     }
     return 0;
@@ -460,6 +483,13 @@ int cpmk_layernorm_affine_forward(int32_t batch, int32_t n, int32_t m, const voi
     clear_stale_error();
     if (alpha == nullptr) return CPMK_EBADARG;
     return layernorm_dispatch(batch, n, m, mat, out, alpha, beta, eps, rd_mean, (hipStream_t)stream);
+}
+
+int cpmk_layernorm_affine_forward_stats(int32_t batch, int32_t n, int32_t m, const void* mat, const void* alpha,
+                                        const void* beta, void* out, void* stats, float eps, int rd_mean, void* stream) {
+    clear_stale_error();
+    if (alpha == nullptr || stats == nullptr) return CPMK_EBADARG;
+    return layernorm_dispatch(batch, n, m, mat, out, alpha, beta, eps, rd_mean, (hipStream_t)stream, nullptr, 0, (float*)stats);
 }
 
 int cpmk_layernorm_step(int32_t batch, int32_t n, const void* mat, void* out, float eps, int rd_mean,

@@ -33,6 +33,27 @@ def layernorm_affine_forward(batch: int, n: int, m: int,
                                   _stream(stream))
 
 
+def layernorm_affine_forward_stats(batch: int, n: int, m: int, mat: DevicePointer, alpha: DevicePointer, beta, out: DevicePointer,
+                                   stats: DevicePointer,    # (batch, 2, m) fp32
+                                   eps: float, rd_mean: bool, stream: CUDAStream):
+    """layernorm_affine_forward that also leaves every column's mean and reciprocal deviation for the backward pass."""
+    cpmk.layernorm_affine_forward_stats(batch, n, m, mat, alpha, beta or None, out, stats, eps, 1 if rd_mean else 0, _stream(stream))
+
+
+def layernorm_affine_backward(batch: int, n: int, m: int,
+                              mat: DevicePointer,         # (batch, n, m)
+                              grad_out: DevicePointer,    # (batch, n, m)
+                              alpha: DevicePointer,       # (n)
+                              stats: DevicePointer,       # (batch, 2, m) fp32
+                              grad: DevicePointer,        # (batch, n, m)
+                              grad_alpha: DevicePointer,  # (n)
+                              grad_beta,                  # (n), or None: the norm without a mean
+                              partials: DevicePointer,    # batch * ceil(m / 64) * 2 * n fp32
+                              stream: CUDAStream):
+    """The whole backward pass of layernorm_affine_forward (torch/layernorm.py:31-86, 113-156)."""
+    cpmk.layernorm_affine_backward(batch, n, m, mat, grad_out, alpha, stats, grad, grad_alpha, grad_beta, partials, _stream(stream))
+
+
 def layernorm_step(batch: int, n: int,
                    mat: DevicePointer,    # (batch, n)  fp16
                    out: DevicePointer,    # (batch, n)  fp16

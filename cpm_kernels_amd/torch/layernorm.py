@@ -2,14 +2,14 @@
 cpm_kernels/torch/layernorm.py."""
 import torch
 from ..kernels import layernorm_forward, layernorm_inplace_forward, layernorm_affine_forward, \
-    layernorm_forward_v, layernorm_forward_mv, layernorm_backward_v, layernorm_backward_mv, \
+    layernorm_affine_forward_stats, layernorm_affine_backward, layernorm_forward_v, layernorm_forward_mv, layernorm_backward_v, layernorm_backward_mv, \
     arith_ln_mul_add, arith_ln_mul, arith_ln_add_backward, arith_ln_mul_backward
 from ._common import cur_stream, check_half
 
 
 class OpLayerNorm(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x: torch.Tensor, eps: float, weight: torch.Tensor, bias, fused: bool = True):
+    def forward(ctx, x: torch.Tensor, eps: float, weight: torch.Tensor, bias, fused: bool = True, train: bool = True):
         """bias given: mean-subtracting norm then y*weight+bias (OpLayerNormMean,
         torch/layernorm.py:7-29); bias None: RMS norm then y*weight (OpLayerNormNoMean, :88-111)."""
         check_half(x, 3)
@@ -17,9 +17,15 @@ class OpLayerNorm(torch.autograd.Function):
         b, n, m = x.size()
         out = torch.empty((b, n, m), device=x.device, dtype=torch.float16)
         rd_mean = bias is not None
-        ctx.save_for_backward(x, weight)
         ctx.eps = eps
         ctx.rd_mean = rd_mean
+        if fused and train:     # the statistics are kept for the backward pass
+            stats = torch.empty((b, 2, m), device=x.device, dtype=torch.float32)
+            layernorm_affine_forward_stats(b, n, m, x.data_ptr(), weight.data_ptr(), bias.data_ptr() if rd_mean else None,
+                                           out.data_ptr(), stats.data_ptr(), eps, rd_mean, cur_stream())
+            ctx.save_for_backward(x, weight, stats)
+            return out
+        ctx.save_for_backward(x, weight, None)
         if fused:
             layernorm_affine_forward(b, n, m, x.data_ptr(), weight.data_ptr(),
                                      bias.data_ptr() if rd_mean else None, out.data_ptr(), eps, rd_mean,
@@ -34,14 +40,23 @@ class OpLayerNorm(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output: torch.Tensor):
-        """The reference's sequence (torch/layernorm.py:31-86, 113-156): the normalised tensor and its
+        """One pass over the input and the gradient from the statistics of the fused forward pass.  Without them the
+        reference's sequence (torch/layernorm.py:31-86, 113-156): the normalised tensor and its
         statistics are recomputed, the affine gradients are two channel sums, and the input
         gradient is the norm's backward kernel applied to grad_output * weight."""
         check_half(grad_output, 3)
-        x, weight = ctx.saved_tensors
+        x, weight, stats = ctx.saved_tensors
         b, n, m = x.size()
         st = cur_stream()
         half = dict(device=x.device, dtype=torch.float16)
+        if stats is not None and x.numel() > 0:
+            grad = torch.empty_like(x)
+            grad_weight = torch.empty((n,), **half)
+            grad_bias = torch.empty((n,), **half) if ctx.rd_mean else None
+            partials = torch.empty((b * ((m + 63) // 64), 2, n), device=x.device, dtype=torch.float32)
+            layernorm_affine_backward(b, n, m, x.data_ptr(), grad_output.data_ptr(), weight.data_ptr(), stats.data_ptr(), grad.data_ptr(),
+                                      grad_weight.data_ptr(), grad_bias.data_ptr() if ctx.rd_mean else None, partials.data_ptr(), st)
+            return grad, None, grad_weight, grad_bias, None, None
         layer_out = torch.empty((b, n, m), **half)
         var = torch.empty((b, m), **half)
         mean = torch.empty((b, m), **half) if ctx.rd_mean else None
@@ -62,7 +77,7 @@ class OpLayerNorm(torch.autograd.Function):
             layernorm_backward_mv(b, n, m, x.data_ptr(), grad_x.data_ptr(), mean.data_ptr(), var.data_ptr(), grad.data_ptr(), st)
         else:
             layernorm_backward_v(b, n, m, x.data_ptr(), grad_x.data_ptr(), var.data_ptr(), grad.data_ptr(), st)
-        return grad, None, grad_weight, grad_bias, None
+        return grad, None, grad_weight, grad_bias, None, None
 
 
 class OpLayerNormMean(OpLayerNorm):
@@ -105,7 +120,7 @@ class LayerNorm(torch.nn.Module):
     def forward(self, x: torch.Tensor):
         check_half(x, 3)
         assert x.size(1) == self.weight.size(0)
-        return OpLayerNorm.apply(x, self.eps, self.weight, self.bias, self.fused)
+        return OpLayerNorm.apply(x, self.eps, self.weight, self.bias, self.fused, torch.is_grad_enabled())
 
 
 class LayerNormTH(torch.nn.Module):

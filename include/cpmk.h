@@ -266,6 +266,14 @@ int cpmk_layernorm_affine_forward(int32_t batch, int32_t n, int32_t m, const voi
                                   const void* alpha /* (n) fp16 */,
                                   const void* beta /* (n) fp16 or NULL */, void* out,
                                   float eps, int rd_mean, void* stream);
+/* ... which also leaves stats (batch, 2, m) fp32: the mean (0 without rd_mean) and the reciprocal deviation of every column */
+int cpmk_layernorm_affine_forward_stats(int32_t batch, int32_t n, int32_t m, const void* mat, const void* alpha,
+                                        const void* beta, void* out, void* stats, float eps, int rd_mean, void* stream);
+/* Its backward pass: grad (batch, n, m), grad_alpha (n) and grad_beta (n; null for the norm without a mean) from the input, the
+ * output's gradient and the statistics.  partials: scratch of batch * ceil(m / 64) * 2 * n floats.
+ *                                                                   cpm_kernels/torch/layernorm.py:31-86, 113-156 */
+int cpmk_layernorm_affine_backward(int32_t batch, int32_t n, int32_t m, const void* mat, const void* grad_out, const void* alpha,
+                                   const void* stats, void* grad, void* grad_alpha, void* grad_beta, void* partials, void* stream);
 
 /* ---- softmax over dim 1 of (batch,n,m) (kernels/softmax.py, cuda/softmax.cu) ------
  * M = max(max_i x, -1e6); S = sum_i exp(x-M) + 1e-10; out = fp16(exp(x-M)/S).

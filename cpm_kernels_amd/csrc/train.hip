@@ -72,6 +72,45 @@ __global__ __launch_bounds__(256) void k_ew(int64_t cols, uint32_t chunks, int64
     else store_half8_head_any(out + i, t, r);
 }
 
+// BC 1 over many rows: a thread takes the same eight columns of U rows, so a and b are fetched once for U rows and U loads are in
+// flight; every element of x and out is touched once, which the non-temporal hint says.
+// Bound by memory.  16 x (64 x s x s), in place: s = 1024 718 us (6.2 TB/s of x, a and out; 822 with one row a thread),
+// s = 512 190 (194), s = 500 176 (190); 4 x (64 x 512 x 512) 52 (65).  Two rows a thread 726, 186, 177, 51; the groups of
+// rows one after the other instead of side by side 759, 220, 167, 53 (at s = 512 the four rows of a thread lie 2^25 bytes apart).
+template <int OP, int U, bool ANY>
+__global__ __launch_bounds__(256) void k_ew_rows(int64_t cols, uint32_t chunks, int64_t rows, const half_t* x, const half_t* __restrict__ a,
+                                                 const half_t* __restrict__ b, half_t* out) {
+    const uint32_t groups = gridDim.x / chunks;
+    const int64_t r0 = (int64_t)(blockIdx.x % groups) * U;
+    const int64_t c = ((int64_t)(blockIdx.x / groups) * 256 + threadIdx.x) * 8;
+    if (c >= cols) return;
+    const int t = !ANY || cols - c >= 8 ? 8 : (int)(cols - c);        // elements of this piece inside the row
+    const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    auto get = [&](const half_t* p) __attribute__((always_inline)) {
+        if constexpr (!ANY) return *reinterpret_cast<const half8_t*>(p);
+        else return t == 8 ? load_half8_any(p) : load_half8_head_any(p, t, zero);
+    };
+    half8_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const half_t* p = x + min(r0 + u, rows - 1) * cols + c;
+        if constexpr (!ANY) v[u] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(p));
+        else v[u] = get(p);
+    }
+    const half8_t av = get(a + c), bv = b ? get(b + c) : zero;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (r0 + u >= rows) break;
+        half8_t r;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[e] = ew_apply(OP, v[u][e], av[e], bv[e]);
+        half_t* o = out + (r0 + u) * cols + c;
+        if constexpr (!ANY) __builtin_nontemporal_store(r, reinterpret_cast<half8_t*>(o));
+        else if (t == 8) store_half8_any(o, r);
+        else store_half8_head_any(o, t, r);
+    }
+}
+
 template <int V>
 __global__ __launch_bounds__(256) void k_global_scale(int64_t n, const half_t* inp, float scale, half_t* out) {
     typedef half_t vec_t __attribute__((ext_vector_type(V)));
@@ -853,6 +892,18 @@ static int launch_ew(int64_t rows, int64_t cols, int64_t n, const void* x, const
     const bool wide = cols % 8 == 0 && aligned16(x) && aligned16(out) && (BC == 2 || (aligned16(a) && (!b || aligned16(b))));
     const int64_t chunks = ceil_div(cols, 256 * 8);
     if (rows * chunks > 0x7fffffffll) return CPMK_ETOOBIG;
+    if constexpr (BC == 1) {
+        // enough pieces to keep the device busy with four rows each
+        if (rows >= 2 && rows * chunks >= 4 * 8 * (int64_t)compute_units()) {
+            auto go = [&](auto kern, int u) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)(ceil_div(rows, u) * chunks)), dim3(256), 0, (hipStream_t)stream, cols, (uint32_t)chunks, rows,
+                                   (const half_t*)x, (const half_t*)a, (const half_t*)b, (half_t*)out);
+            };
+            if (rows == 2) { if (wide) go(k_ew_rows<OP, 2, false>, 2); else go(k_ew_rows<OP, 2, true>, 2); }
+            else { if (wide) go(k_ew_rows<OP, 4, false>, 4); else go(k_ew_rows<OP, 4, true>, 4); }
+            return launch_status();
+        }
+    }
     const dim3 grid((unsigned)(rows * chunks));
     if (wide)
         hipLaunchKernelGGL((k_ew<OP, BC, false>), grid, dim3(256), 0, (hipStream_t)stream, cols, (uint32_t)chunks, n, (const half_t*)x,

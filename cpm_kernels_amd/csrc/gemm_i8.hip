@@ -514,13 +514,18 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     a.edge_in = 0;
     a.nsum = 1;
     a.kmagic = 0;
-    const bool wide = aligned16(out) && m % 4 == 0;       // the tile kernel stores 16-byte pieces of output rows (8-byte halves where m % 8 == 4)
+    // The tile kernel stores 16-byte pieces of output rows that start on dwords, and 8-byte halves at a row's end.  Rows of 4j + 2
+    // elements end in neither: their last column tile lies inside the matrix (edge_in), which takes a matrix of at least one tile.
+    const bool odd = m % 4 != 0;
+    // (Tiles of the general kernel waste less of narrow ones: 80 heads of 150 x 150 6.7 us there, 9.0 here; 228 of 402 x 402, 58 and 33.)
+    const bool wide = (reinterpret_cast<uintptr_t>(out) & 3u) == 0 && (!odd || m >= 192);
     const bool p_kmajor = !bT, q_kmajor = aT != 0;
     if (p_kmajor && q_kmajor && wide && k > 0 && (k % 32 == 0) && aligned16(A) && aligned16(B) &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
         const bool whole128 = k % 64 == 0;       // the depth is whole 128-byte slabs (else whole 64-byte ones: 96, 160 ...)
-        if (big * 4 >= compute_units() * 3 && n > 128 && m > 128) {
+        a.edge_in = odd ? 2 : 0;
+        if (big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!odd || m >= 256)) {
             if (whole128 && k >= 256) return launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 0, 16>(a, batch, st);
             // Products of a few slabs -- attention scores, K = 64 -- are all prologue and epilogue, bound by the stores (and
             // depths of whole 64-byte slabs only need this form anyway):
@@ -539,24 +544,26 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     if (p_kmajor && q_kmajor && wide && k > 32 && (reinterpret_cast<uintptr_t>(A) & 3u) == 0 && (reinterpret_cast<uintptr_t>(B) & 3u) == 0 &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
-        const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128;
+        const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!odd || m >= 256);
+        a.edge_in = odd ? 2 : 0;
         if (k % 8 == 0 && aligned16(A) && aligned16(B))       // whole, aligned 16-byte pieces
             return large ? launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, 4, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, 4, 32>(a, batch, st);
         return large ? launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, 12, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, 12, 32>(a, batch, st);
     }
     // an operand stored (K, rows): the tile kernel reads it as it lies, with transposing LDS reads for the fragments
-    // (rows of such an operand that are not whole 16-byte pieces, but whole 8-byte ones: tiles that stay inside the matrix,
-    // which takes a matrix of at least one tile)
+    // (rows of such an operand that are not whole 16-byte pieces: tiles that stay inside the matrix, which takes a matrix of at
+    // least one tile)
     const bool in_p = !p_kmajor && n % 8 != 0, in_q = !q_kmajor && m % 8 != 0;
-    const bool low = n <= 64;                // 64 x 256 tiles for few output rows (attention: probabilities x values)
+    // 64 x 256 tiles for few output rows (attention: probabilities x values)
+    const bool low = n <= 64 && !((in_q || odd) && m < 256);
     if (!(p_kmajor && q_kmajor) && wide && k > 0 && (k % 64 == 0) && aligned16(A) && aligned16(B) &&
-        (!in_p || (n % 4 == 0 && n >= 128)) && (!in_q || (m % 4 == 0 && m >= (low ? 256 : 128))) &&
+        (!in_p || n >= 128) && (!in_q || m >= (low ? 256 : 128)) &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
         const int lay = (p_kmajor ? 0 : 1) | (q_kmajor ? 0 : 2);
         // else 256x256 tiles when they give most compute units a tile, else 128x128 (as for K-major operands)
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
-        const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!in_q || m >= 256);
-        a.edge_in = (in_p ? 1 : 0) | (in_q ? 2 : 0);
+        const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!(in_q || odd) || m >= 256);
+        a.edge_in = (in_p ? 1 : 0) | (in_q || odd ? 2 : 0);
         switch (lay) {
             case 1:
                 if (low) return launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 1, 32>(a, batch, st);
@@ -569,12 +576,13 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
                 return large ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 3, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 3, 32>(a, batch, st);
         }
     }
-    // one operand stored (K, rows) and a depth that is not whole slabs (attention: probabilities x values over 500 keys):
-    // the 32x32 form of the tile kernel, the rest of the depth straight from memory into the fragments
-    if (p_kmajor != q_kmajor && wide && k > 64 && (k % 64 != 0) && aligned16(A) && aligned16(B) &&
-        (!in_p || (n % 4 == 0 && n >= 128)) && (!in_q || (m % 4 == 0 && m >= (low ? 256 : 128))) &&
+    // an operand stored (K, rows) and a depth that is not whole slabs (attention: probabilities x values over 500 keys, scores
+    // over heads of 80): the 32x32 form of the tile kernel, the rest of the depth straight from memory into the fragments
+    if (!(p_kmajor && q_kmajor) && wide && k > 64 && (k % 64 != 0) && aligned16(A) && aligned16(B) &&
+        (!in_p || n >= 128) && (!in_q || m >= (low ? 256 : 128)) &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
-        a.edge_in = (in_p ? 1 : 0) | (in_q ? 2 : 0);
+        a.edge_in = (in_p ? 1 : 0) | (in_q || odd ? 2 : 0);
+        if (!p_kmajor && !q_kmajor) return launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 15, 32>(a, batch, st, 2);
         if (!p_kmajor) return low ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 13, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 13, 32>(a, batch, st);
         return low ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 14, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 14, 32>(a, batch, st);
     }

@@ -77,15 +77,15 @@ __device__ __forceinline__ GemmItem gemm_item(uint32_t L, const DmaArgs& da) {
     it.j0 = (int32_t)((g * GRP + tin % rows_in_group) * BR + (h & 1) * (BR / 2));
     it.i0 = (int32_t)((tin / rows_in_group) * BC);
     // An operand stored (K, rows) whose rows are not whole 16-byte pieces cannot be read past the matrix's edge piece by
-    // piece: its last tile then lies inside the matrix and overlaps its neighbour, whose outputs it computes again
-    // (the same bits, stored twice).
+    // piece, and output rows of 4j + 2 elements end in less than half a piece: the last tile then lies inside the matrix and
+    // overlaps its neighbour, whose outputs it computes again (the same bits, stored twice).
     if (da.g.edge_in & 1) it.j0 = min(it.j0, da.g.n - BR);
     if (da.g.edge_in & 2) it.i0 = min(it.i0, da.g.m - BC);
     return it;
 }
 
 // A 16-byte piece of an output row on its way to memory; `left` = elements from the piece's first to the end of
-// the row (a multiple of 4, at least 4).  fp16 rows of 8j + 4 elements start on 8-byte boundaries and end in half a piece:
+// the row (a multiple of 4, at least 4; at least 8 in a tile that lies inside the matrix, see edge_in).  fp16 rows of 8j + 4 elements start on 8-byte boundaries and end in half a piece:
 // whole pieces leave as 16 bytes wherever they lie (global stores need no alignment; as two 8-byte halves the scores of 1024 heads
 // of 500 x 500 took 175 us instead of 163, 128 heads of 588 x 588 52 instead of 46).
 template <int ESZ>

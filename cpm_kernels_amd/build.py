@@ -13,6 +13,7 @@ from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
+NATIVE_SRC = os.path.join(HERE, "native")     # Python extension modules (host C++)
 BENCH_SRC = os.path.join(HERE, "bench")       # yardstick kernels for bench.py; a library of their own
 LIBDIR = os.path.join(HERE, "lib")
 LIBNAME = "libcpmk_hip.so"
@@ -78,8 +79,22 @@ def build_library(verbose=True, jobs=None):
     os.replace(tmp, library_path())
     if verbose:
         print("[cpmk build] linked %s" % library_path(), flush=True)
+    build_native(verbose)
     build_bench_library(verbose)
     return library_path()
+
+
+def build_native(verbose=True):
+    """The extension modules that call the library from Python (host code only)."""
+    import sysconfig
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    os.makedirs(LIBDIR, exist_ok=True)
+    base = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-I" + sysconfig.get_paths()["include"]]
+    out = os.path.join(LIBDIR, "_cpmk_call.so")
+    _run(base + [os.path.join(NATIVE_SRC, "call.cpp"), "-o", out + ".tmp"])
+    os.replace(out + ".tmp", out)
+    if verbose:
+        print("[cpmk build] linked %s" % out, flush=True)
 
 
 def build_bench_library(verbose=True):

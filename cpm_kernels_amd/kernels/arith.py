@@ -1,6 +1,6 @@
 """Elementwise helpers the path's callers use, with the signatures of cpm_kernels/kernels/arith.py."""
 from ..library import cpmk
-from .base import DevicePointer, CUDAStream, _stream
+from .base import DevicePointer, CUDAStream
 
 
 def arith_element_add(batch: int, n: int,
@@ -10,7 +10,7 @@ def arith_element_add(batch: int, n: int,
                       stream: CUDAStream):
     """out = x + y.  reference: kernels/arith.py:43-66"""
     assert n % 2 == 0
-    cpmk.arith_element_add(batch, n, x, y, out, _stream(stream))
+    cpmk.arith_element_add(batch, n, x, y, out, stream)
 
 
 def arith_ln_mul_add(batch: int, n: int, m: int,
@@ -22,7 +22,7 @@ def arith_ln_mul_add(batch: int, n: int, m: int,
     """out = x * alpha[None, :, None] + beta[None, :, None] (fp16 fma).
     reference: kernels/arith.py:135-161"""
     assert m % 2 == 0
-    cpmk.arith_ln_mul_add(batch, n, m, inp, alpha, beta, out, _stream(stream))
+    cpmk.arith_ln_mul_add(batch, n, m, inp, alpha, beta, out, stream)
 
 
 def arith_ln_mul(batch: int, n: int, m: int,
@@ -32,7 +32,7 @@ def arith_ln_mul(batch: int, n: int, m: int,
                  stream: CUDAStream):
     """out = x * alpha[None, :, None].  reference: kernels/arith.py:190-214"""
     assert m % 2 == 0
-    cpmk.arith_ln_mul(batch, n, m, inp, alpha, out, _stream(stream))
+    cpmk.arith_ln_mul(batch, n, m, inp, alpha, out, stream)
 
 
 def arith_global_scale(n: int,
@@ -41,7 +41,7 @@ def arith_global_scale(n: int,
                        out: DevicePointer,    # (n,) fp16
                        stream: CUDAStream):
     """out = fp16(float(x) * scale).  reference: kernels/arith.py:24-41"""
-    cpmk.arith_global_scale(n, inp, scale, out, _stream(stream))
+    cpmk.arith_global_scale(n, inp, scale, out, stream)
 
 
 def arith_element_mul(batch: int, n: int,
@@ -51,7 +51,7 @@ def arith_element_mul(batch: int, n: int,
                       stream: CUDAStream):
     """out = x * y.  reference: kernels/arith.py:68-91"""
     assert n % 2 == 0
-    cpmk.arith_element_mul(batch, n, x, y, out, _stream(stream))
+    cpmk.arith_element_mul(batch, n, x, y, out, stream)
 
 
 def arith_batch_add_forward(batch: int, n: int,
@@ -61,7 +61,7 @@ def arith_batch_add_forward(batch: int, n: int,
                             stream: CUDAStream):
     """out = x + y[None, :].  reference: kernels/arith.py:93-116"""
     assert n % 2 == 0
-    cpmk.arith_batch_add_forward(batch, n, x, y, out, _stream(stream))
+    cpmk.arith_batch_add_forward(batch, n, x, y, out, stream)
 
 
 def arith_batch_add_backward(batch: int, n: int,
@@ -69,7 +69,7 @@ def arith_batch_add_backward(batch: int, n: int,
                              grad: DevicePointer,        # (n)         fp16
                              stream: CUDAStream):
     """grad = grad_out.sum(0).  reference: kernels/arith.py:118-133"""
-    cpmk.arith_batch_add_backward(batch, n, grad_out, grad, _stream(stream))
+    cpmk.arith_batch_add_backward(batch, n, grad_out, grad, stream)
 
 
 def arith_ln_add(batch: int, n: int, m: int,
@@ -79,7 +79,7 @@ def arith_ln_add(batch: int, n: int, m: int,
                  stream: CUDAStream):
     """out = x + beta[None, :, None].  reference: kernels/arith.py:163-188"""
     assert m % 2 == 0
-    cpmk.arith_ln_add(batch, n, m, inp, beta, out, _stream(stream))
+    cpmk.arith_ln_add(batch, n, m, inp, beta, out, stream)
 
 
 def arith_ln_div(batch: int, n: int, m: int,
@@ -90,7 +90,7 @@ def arith_ln_div(batch: int, n: int, m: int,
     """out = x * (1 / alpha)[None, :, None] with the reciprocal rounded to fp16 first.
     reference: kernels/arith.py:216-240"""
     assert m % 2 == 0
-    cpmk.arith_ln_div(batch, n, m, inp, alpha, out, _stream(stream))
+    cpmk.arith_ln_div(batch, n, m, inp, alpha, out, stream)
 
 
 def arith_ln_sub_div(batch: int, n: int, m: int,
@@ -102,7 +102,7 @@ def arith_ln_sub_div(batch: int, n: int, m: int,
     """out = (x - beta) / alpha evaluated as one fp16 fma with fp16(1/alpha) and fp16(-beta/alpha).
     reference: kernels/arith.py:242-269"""
     assert m % 2 == 0
-    cpmk.arith_ln_sub_div(batch, n, m, inp, alpha, beta, out, _stream(stream))
+    cpmk.arith_ln_sub_div(batch, n, m, inp, alpha, beta, out, stream)
 
 
 def arith_ln_mul_backward(batch: int, n: int, m: int,
@@ -111,7 +111,7 @@ def arith_ln_mul_backward(batch: int, n: int, m: int,
                           grad: DevicePointer,        # (n)            fp16
                           stream: CUDAStream):
     """grad = (x * grad_out).sum((0, 2)).  reference: kernels/arith.py:271-289"""
-    cpmk.arith_ln_mul_backward(batch, n, m, inp, grad_out, grad, _stream(stream))
+    cpmk.arith_ln_mul_backward(batch, n, m, inp, grad_out, grad, stream)
 
 
 def arith_ln_add_backward(batch: int, n: int, m: int,
@@ -119,7 +119,7 @@ def arith_ln_add_backward(batch: int, n: int, m: int,
                           grad: DevicePointer,        # (n)            fp16
                           stream: CUDAStream):
     """grad = grad_out.sum((0, 2)).  reference: kernels/arith.py:291-307"""
-    cpmk.arith_ln_add_backward(batch, n, m, grad_out, grad, _stream(stream))
+    cpmk.arith_ln_add_backward(batch, n, m, grad_out, grad, stream)
 
 
 def arith_batch_mul_add(batch: int, n: int,
@@ -130,7 +130,7 @@ def arith_batch_mul_add(batch: int, n: int,
                         stream: CUDAStream):
     """out = x * alpha[None, :] + beta[None, :] (fp16 fma).  reference: kernels/arith.py:309-331"""
     assert n % 2 == 0
-    cpmk.arith_batch_mul_add(batch, n, x, alpha, beta, out, _stream(stream))
+    cpmk.arith_batch_mul_add(batch, n, x, alpha, beta, out, stream)
 
 
 def arith_batch_mul(batch: int, n: int,
@@ -140,4 +140,4 @@ def arith_batch_mul(batch: int, n: int,
                     stream: CUDAStream):
     """out = x * alpha[None, :].  reference: kernels/arith.py:333-354"""
     assert n % 2 == 0
-    cpmk.arith_batch_mul(batch, n, x, alpha, out, _stream(stream))
+    cpmk.arith_batch_mul(batch, n, x, alpha, out, stream)

@@ -12,10 +12,3 @@ CUDAStream = ctypes.c_void_p     # name kept; on ROCm torch's ``.cuda_stream`` i
 
 def round_up(x: int, m: int) -> int:
     return (x + m - 1) // m * m
-
-
-def _stream(stream):
-    """Accept an int, None or a ctypes.c_void_p like the reference's launch path does."""
-    if isinstance(stream, ctypes.c_void_p):
-        return stream
-    return ctypes.c_void_p(stream)

@@ -1,6 +1,6 @@
 """Token-embedding gathers with the signatures of cpm_kernels/kernels/embedding.py ."""
 from ..library import cpmk
-from .base import DevicePointer, CUDAStream, _stream
+from .base import DevicePointer, CUDAStream
 
 
 def embedding_forward(batch: int,
@@ -11,7 +11,7 @@ def embedding_forward(batch: int,
                       out: DevicePointer,        # (batch, hidden_size, seq_len) fp16
                       stream: CUDAStream):
     """reference: kernels/embedding.py:14-34"""
-    cpmk.embedding_forward(batch, hidden_size, seq_len, ids, weights, out, _stream(stream))
+    cpmk.embedding_forward(batch, hidden_size, seq_len, ids, weights, out, stream)
 
 
 def embedding_step(batch: int, embedding_size: int,
@@ -20,7 +20,7 @@ def embedding_step(batch: int, embedding_size: int,
                    out: DevicePointer,            # (batch, embedding_size) fp16
                    stream: CUDAStream):
     """reference: kernels/embedding.py:88-105"""
-    cpmk.embedding_step(batch, embedding_size, ids, weights, out, _stream(stream))
+    cpmk.embedding_step(batch, embedding_size, ids, weights, out, stream)
 
 
 def embedding_backward_stage1(batch: int, seq_len: int, hidden_size: int,
@@ -33,7 +33,7 @@ def embedding_backward_stage1(batch: int, seq_len: int, hidden_size: int,
                               stream: CUDAStream):
     """Sums runs of equal sorted ids inside each batch entry.  reference: kernels/embedding.py:36-65"""
     cpmk.embedding_backward_stage1(batch, seq_len, hidden_size, grad_out, argsort_ids, sorted_ids, grad, aux_grad,
-                                   aux_grad_idx, _stream(stream))
+                                   aux_grad_idx, stream)
 
 
 def embedding_backward_stage2(batch: int, hidden_size: int,
@@ -42,4 +42,4 @@ def embedding_backward_stage2(batch: int, hidden_size: int,
                               grad: DevicePointer,            # (vocab_size, m)
                               stream: CUDAStream):
     """Adds the per-entry tail runs into grad.  reference: kernels/embedding.py:67-86"""
-    cpmk.embedding_backward_stage2(batch, hidden_size, aux_grad, aux_grad_idx, grad, _stream(stream))
+    cpmk.embedding_backward_stage2(batch, hidden_size, aux_grad, aux_grad_idx, grad, stream)

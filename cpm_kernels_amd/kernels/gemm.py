@@ -1,7 +1,7 @@
 """Quantisation, int8 GEMM and dequantisation launchers with the signatures of
 cpm_kernels/kernels/gemm.py.  Arithmetic contracts are stated in include/cpmk.h."""
 from ..library import cpmk
-from .base import DevicePointer, CUDAStream, _stream
+from .base import DevicePointer, CUDAStream
 
 
 def gemm_round(batch: int, n: int, m: int,
@@ -10,7 +10,7 @@ def gemm_round(batch: int, n: int, m: int,
                out: DevicePointer,      # (b, n, m)  int8
                stream: CUDAStream):
     """reference: kernels/gemm.py:21-41"""
-    cpmk.gemm_round(batch, n, m, mat, scale, out, _stream(stream))
+    cpmk.gemm_round(batch, n, m, mat, scale, out, stream)
 
 
 def gemm_round_transpose(batch: int, n: int, m: int,
@@ -19,7 +19,7 @@ def gemm_round_transpose(batch: int, n: int, m: int,
                          out: DevicePointer,    # (b, n, m)  int8
                          stream: CUDAStream):
     """reference: kernels/gemm.py:43-63"""
-    cpmk.gemm_round_transpose(batch, n, m, mat, scale, out, _stream(stream))
+    cpmk.gemm_round_transpose(batch, n, m, mat, scale, out, stream)
 
 
 def gemm_scale(batch: int, n: int, m: int,
@@ -31,7 +31,7 @@ def gemm_scale(batch: int, n: int, m: int,
                stream: CUDAStream):
     """reference: kernels/gemm.py:65-89"""
     cpmk.gemm_scale(batch, n, m, mat, scale_x, scale_y, out, int(bool(broad_cast_x)),
-                    int(bool(broad_cast_y)), _stream(stream))
+                    int(bool(broad_cast_y)), stream)
 
 
 def gemm_calc_scale(batch: int, n: int, m: int,
@@ -39,7 +39,7 @@ def gemm_calc_scale(batch: int, n: int, m: int,
                     out: DevicePointer,    # (b, n)    fp16
                     stream: CUDAStream):
     """reference: kernels/gemm.py:91-107"""
-    cpmk.gemm_calc_scale(batch, n, m, mat, out, _stream(stream))
+    cpmk.gemm_calc_scale(batch, n, m, mat, out, stream)
 
 
 def gemm_calc_scale_transpose(batch: int, n: int, m: int,
@@ -47,7 +47,7 @@ def gemm_calc_scale_transpose(batch: int, n: int, m: int,
                               out: DevicePointer,    # (b, m)    fp16
                               stream: CUDAStream):
     """reference: kernels/gemm.py:109-125"""
-    cpmk.gemm_calc_scale_transpose(batch, n, m, inp, out, _stream(stream))
+    cpmk.gemm_calc_scale_transpose(batch, n, m, inp, out, stream)
 
 
 def gemm_int8(m: int, k: int, n: int,
@@ -60,7 +60,7 @@ def gemm_int8(m: int, k: int, n: int,
     """reference: kernels/gemm.py:127-186 (cuBLASLt); same asserts (:139-140)."""
     assert m % 4 == 0 and n % 4 == 0 and k % 4 == 0
     assert batchA == batchB or batchA == 1 or batchB == 1
-    cpmk.gemm_int8(m, k, n, batchA, batchB, int(bool(aT)), int(bool(bT)), A, B, out, _stream(stream))
+    cpmk.gemm_int8(m, k, n, batchA, batchB, int(bool(aT)), int(bool(bT)), A, B, out, stream)
 
 
 def gemm_int8_scale(m: int, k: int, n: int,
@@ -77,7 +77,7 @@ def gemm_int8_scale(m: int, k: int, n: int,
     assert m % 4 == 0 and n % 4 == 0 and k % 4 == 0
     assert batchA == batchB or batchA == 1 or batchB == 1
     cpmk.gemm_int8_scale(m, k, n, batchA, batchB, int(bool(aT)), int(bool(bT)), A, B, scale_row, scale_col,
-                         int(bool(broad_cast_row)), int(bool(broad_cast_col)), out, _stream(stream))
+                         int(bool(broad_cast_row)), int(bool(broad_cast_col)), out, stream)
 
 
 def gemm_quantize(batch: int, n: int, m: int,
@@ -88,7 +88,7 @@ def gemm_quantize(batch: int, n: int, m: int,
                   stream: CUDAStream):
     """gemm_calc_scale[_transpose] + gemm_round[_transpose] in one call (fuses
     torch/gemm.py:5-38)."""
-    cpmk.gemm_quantize(batch, n, m, mat, scale, out, int(bool(transpose)), _stream(stream))
+    cpmk.gemm_quantize(batch, n, m, mat, scale, out, int(bool(transpose)), stream)
 
 
 def gemm_quantize_pair(rows0: int, mat0: DevicePointer, scale0: DevicePointer, out0: DevicePointer,
@@ -96,7 +96,7 @@ def gemm_quantize_pair(rows0: int, mat0: DevicePointer, scale0: DevicePointer, o
                        m: int, stream: CUDAStream):
     """gemm_quantize(transpose=False) of two tensors with rows of length m (rows0 x m fp16 at
     mat0, rows1 x m at mat1) in one launch."""
-    cpmk.gemm_quantize_pair(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, _stream(stream))
+    cpmk.gemm_quantize_pair(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, stream)
 
 
 def gemm_quantize_cols(batch: int, n: int, m: int,
@@ -108,7 +108,7 @@ def gemm_quantize_cols(batch: int, n: int, m: int,
     """gemm_calc_scale_transpose + gemm_round_transpose in one pass (fuses torch/gemm.py:5-38 for
     an operand quantised along dim 1), optionally writing the int8 tensor transposed so that it
     is K-major for gemm_int8."""
-    cpmk.gemm_quantize_cols(batch, n, m, mat, scale, out, int(bool(out_transposed)), _stream(stream))
+    cpmk.gemm_quantize_cols(batch, n, m, mat, scale, out, int(bool(out_transposed)), stream)
 
 
 def gemm_scale_x(batch: int, n: int, m: int,
@@ -117,7 +117,7 @@ def gemm_scale_x(batch: int, n: int, m: int,
                  out: DevicePointer,        # (b, n, m)  fp16
                  stream: CUDAStream):
     """reference: kernels/gemm.py:309-327"""
-    cpmk.gemm_scale_x(batch, n, m, mat, scale_x, out, _stream(stream))
+    cpmk.gemm_scale_x(batch, n, m, mat, scale_x, out, stream)
 
 
 def gemm_scale_y(batch: int, n: int, m: int,
@@ -126,7 +126,7 @@ def gemm_scale_y(batch: int, n: int, m: int,
                  out: DevicePointer,        # (b, n, m)  fp16
                  stream: CUDAStream):
     """reference: kernels/gemm.py:329-347"""
-    cpmk.gemm_scale_y(batch, n, m, mat, scale_y, out, _stream(stream))
+    cpmk.gemm_scale_y(batch, n, m, mat, scale_y, out, stream)
 
 
 def gemm_int8_scale_one(m: int, k: int, n: int, batchA: int, batchB: int, aT: bool, bT: bool,
@@ -140,7 +140,7 @@ def gemm_int8_scale_one(m: int, k: int, n: int, batchA: int, batchB: int, aT: bo
     assert m % 4 == 0 and n % 4 == 0 and k % 4 == 0
     assert batchA == batchB or batchA == 1 or batchB == 1
     cpmk.gemm_int8_scale_one(m, k, n, batchA, batchB, 1 if aT else 0, 1 if bT else 0, A, B, scale_row, scale_col,
-                             1 if broad_cast_row else 0, 1 if broad_cast_col else 0, out, _stream(stream))
+                             1 if broad_cast_row else 0, 1 if broad_cast_col else 0, out, stream)
 
 
 def gemm_quantize_cols_ld(batch: int, n: int, m: int, mat: DevicePointer,
@@ -154,14 +154,14 @@ def gemm_quantize_cols_ld(batch: int, n: int, m: int, mat: DevicePointer,
                           stream: CUDAStream):
     """Per-column quantisation of mat (times row_scale: gemm_backward_scale_round) in the transposed and / or the matrix's
     own layout, rows filled up with zeros to ld_t / ld_n bytes."""
-    cpmk.gemm_quantize_cols_ld(batch, n, m, mat, row_scale, 1 if broad_cast_row else 0, scale, out_t, ld_t, out_n, ld_n, _stream(stream))
+    cpmk.gemm_quantize_cols_ld(batch, n, m, mat, row_scale, 1 if broad_cast_row else 0, scale, out_t, ld_t, out_n, ld_n, stream)
 
 
 def gemm_quantize_pair_ld(rows0: int, mat0: DevicePointer, scale0: DevicePointer, out0: DevicePointer,
                           rows1: int, mat1: DevicePointer, scale1: DevicePointer, out1: DevicePointer,
                           m: int, ld: int, stream: CUDAStream):
     """gemm_quantize_pair with int8 rows filled up with zeros to ld bytes; m <= 16384."""
-    cpmk.gemm_quantize_pair_ld(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, ld, _stream(stream))
+    cpmk.gemm_quantize_pair_ld(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, ld, stream)
 
 
 def gemm_backward_round_scale_ld(batch: int, n: int, m: int, mat: DevicePointer, scale_y: DevicePointer,
@@ -170,7 +170,7 @@ def gemm_backward_round_scale_ld(batch: int, n: int, m: int, mat: DevicePointer,
                                  scale_x: DevicePointer,    # (batch, n)      fp16
                                  broad_cast_y: bool, stream: CUDAStream):
     """gemm_backward_round_scale with rows filled up with zeros to ld bytes."""
-    cpmk.gemm_backward_round_scale_ld(batch, n, m, mat, scale_y, out, ld, scale_x, 1 if broad_cast_y else 0, _stream(stream))
+    cpmk.gemm_backward_round_scale_ld(batch, n, m, mat, scale_y, out, ld, scale_x, 1 if broad_cast_y else 0, stream)
 
 
 def gemm_sum_groups(m: int, n: int, batch: int) -> int:
@@ -188,7 +188,7 @@ def gemm_int8_scale_sum(m: int, k: int, n: int, batch: int, groups: int,
     """out[g] = sum over the entries of group g of scale_row * (B x A^T): the reference's gemm_int8 + gemm_scale_x +
     sum over the batch (torch/gemm.py:115-186), each sum in fp32 and rounded once.  k is a multiple of 128."""
     assert m % 4 == 0 and n % 4 == 0 and k % 128 == 0
-    cpmk.gemm_int8_scale_sum(m, k, n, batch, groups, A, B, scale_row, out, _stream(stream))
+    cpmk.gemm_int8_scale_sum(m, k, n, batch, groups, A, B, scale_row, out, stream)
 
 
 def gemm_fp16_sum(m: int, k: int, n: int, batch: int, groups: int,
@@ -198,7 +198,7 @@ def gemm_fp16_sum(m: int, k: int, n: int, batch: int, groups: int,
                   stream: CUDAStream):
     """out[g] = sum over the entries of group g of B x A^T: gemm_fp16 + sum over the batch (torch/gemm.py:219-239)."""
     assert m % 4 == 0 and n % 4 == 0 and k % 2 == 0 and k > 32
-    cpmk.gemm_fp16_sum(m, k, n, batch, groups, A, B, out, _stream(stream))
+    cpmk.gemm_fp16_sum(m, k, n, batch, groups, A, B, out, stream)
 
 
 def gemm_fp16(m: int, k: int, n: int,
@@ -211,7 +211,7 @@ def gemm_fp16(m: int, k: int, n: int,
     """reference: kernels/gemm.py:188-256 (cuBLASLt); same asserts (:200-201).  fp32 accumulation."""
     assert m % 2 == 0 and n % 2 == 0 and k % 2 == 0
     assert batchA == batchB or batchA == 1 or batchB == 1
-    cpmk.gemm_fp16(m, k, n, batchA, batchB, int(bool(aT)), int(bool(bT)), A, B, out, _stream(stream))
+    cpmk.gemm_fp16(m, k, n, batchA, batchB, int(bool(aT)), int(bool(bT)), A, B, out, stream)
 
 
 def gemm_backward_round_scale(batch: int, n: int, m: int,
@@ -222,7 +222,7 @@ def gemm_backward_round_scale(batch: int, n: int, m: int,
                               broad_cast_y: bool,
                               stream: CUDAStream):
     """Row scales and int8 rounding of mat * scale_y.  reference: kernels/gemm.py:261-283"""
-    cpmk.gemm_backward_round_scale(batch, n, m, mat, scale_y, out, scale_x, int(bool(broad_cast_y)), _stream(stream))
+    cpmk.gemm_backward_round_scale(batch, n, m, mat, scale_y, out, scale_x, int(bool(broad_cast_y)), stream)
 
 
 def gemm_backward_scale_round(batch: int, n: int, m: int,
@@ -233,4 +233,4 @@ def gemm_backward_scale_round(batch: int, n: int, m: int,
                               broad_cast_x: bool,
                               stream: CUDAStream):
     """Column scales and int8 rounding of mat * scale_x.  reference: kernels/gemm.py:285-307"""
-    cpmk.gemm_backward_scale_round(batch, n, m, mat, scale_x, out, scale_y, int(bool(broad_cast_x)), _stream(stream))
+    cpmk.gemm_backward_scale_round(batch, n, m, mat, scale_x, out, scale_y, int(bool(broad_cast_x)), stream)

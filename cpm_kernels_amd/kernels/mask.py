@@ -1,6 +1,6 @@
 """Padding mask launcher with the signature of cpm_kernels/kernels/mask.py."""
 from ..library import cpmk
-from .base import DevicePointer, CUDAStream, _stream
+from .base import DevicePointer, CUDAStream
 
 
 def mask(batch: int, n: int, m: int,
@@ -10,4 +10,4 @@ def mask(batch: int, n: int, m: int,
          out: DevicePointer,     # (batch, n, m)  fp16
          stream: CUDAStream):
     """out[b,i,j] = mask[b,j] ? inp[b,i,j] : value.  reference: kernels/mask.py:12-35"""
-    cpmk.mask(batch, n, m, inp, mask, value, out, _stream(stream))
+    cpmk.mask(batch, n, m, inp, mask, value, out, stream)

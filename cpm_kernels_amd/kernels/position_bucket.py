@@ -1,6 +1,6 @@
 """Relative position bias launchers with the signatures of cpm_kernels/kernels/position_bucket.py."""
 from ..library import cpmk
-from .base import DevicePointer, CUDAStream, _stream
+from .base import DevicePointer, CUDAStream
 
 
 def position_embedding_init(num_buckets: int, max_distance: int,
@@ -8,7 +8,7 @@ def position_embedding_init(num_buckets: int, max_distance: int,
                             bidirectional: bool,
                             stream: CUDAStream):
     """reference: kernels/position_bucket.py:14-30"""
-    cpmk.position_embedding_init(num_buckets, max_distance, out, int(bool(bidirectional)), _stream(stream))
+    cpmk.position_embedding_init(num_buckets, max_distance, out, int(bool(bidirectional)), stream)
 
 
 def position_embedding_forward(query_len: int, key_len: int, num_buckets: int, max_distance: int,
@@ -20,7 +20,7 @@ def position_embedding_forward(query_len: int, key_len: int, num_buckets: int, m
                                stream: CUDAStream):
     """reference: kernels/position_bucket.py:32-58"""
     cpmk.position_embedding_forward(query_len, key_len, num_buckets, max_distance, num_heads, position_mapping,
-                                    weight, out, int(bool(bidirectional)), _stream(stream))
+                                    weight, out, int(bool(bidirectional)), stream)
 
 
 def position_embedding_step(query_pos: int, key_len: int, num_buckets: int, max_distance: int,
@@ -32,7 +32,7 @@ def position_embedding_step(query_pos: int, key_len: int, num_buckets: int, max_
                             stream: CUDAStream):
     """reference: kernels/position_bucket.py:88-113"""
     cpmk.position_embedding_step(query_pos, key_len, num_buckets, max_distance, num_heads, position_mapping,
-                                 weight, out, int(bool(bidirectional)), _stream(stream))
+                                 weight, out, int(bool(bidirectional)), stream)
 
 
 def position_embedding_backward(query_len: int, key_len: int, num_buckets: int, max_distance: int,
@@ -44,4 +44,4 @@ def position_embedding_backward(query_len: int, key_len: int, num_buckets: int, 
                                 stream: CUDAStream):
     """reference: kernels/position_bucket.py:60-86"""
     cpmk.position_embedding_backward(query_len, key_len, num_buckets, max_distance, num_heads, position_mapping,
-                                     grad_out, grad, int(bool(bidirectional)), _stream(stream))
+                                     grad_out, grad, int(bool(bidirectional)), stream)

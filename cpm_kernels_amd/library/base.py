@@ -69,6 +69,24 @@ def find_lib(name: str):
     return ctypes.util.find_library(name)
 
 
+def load_native(name: str):
+    """The in-tree extension module lib/<name>.so (cpm_kernels_amd/build.py), None if it is not there."""
+    import importlib.machinery
+    import importlib.util
+    path = os.path.join(_PKG_DIR, "lib", name + ".so")
+    if not os.path.exists(path):
+        logger.warning("%s is not built", path)
+        return None
+    try:
+        loader = importlib.machinery.ExtensionFileLoader(name, path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location(name, path, loader=loader))
+        loader.exec_module(module)
+        return module
+    except ImportError as e:
+        logger.warning("Could not load %s: %s", path, e)
+        return None
+
+
 class Lib:
     def __init__(self, name: str, path=None):
         self._name = name
@@ -90,6 +108,16 @@ class Lib:
     @property
     def loaded(self) -> bool:
         return self._lib is not None
+
+    def address(self, name):
+        """The address of a symbol, None if the library or the symbol is missing."""
+        if self._lib is None:
+            return None
+        try:
+            return ctypes.cast(getattr(self._lib, name), ctypes.c_void_p).value
+        except AttributeError:
+            logger.warning("Symbol %s not found in %s", name, self._path)
+            return None
 
     def bind(self, name, arg_types, ret_type) -> Callable[[LibCall], LibCall]:
         if self._lib is None:

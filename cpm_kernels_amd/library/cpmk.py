@@ -1,4 +1,4 @@
-"""ctypes binding of libcpmk_hip.so (include/cpmk.h).
+"""Binding of libcpmk_hip.so (include/cpmk.h): the launchers through native/call.cpp, the rest through ctypes.
 
 Replaces cpm_kernels/library/{cuda,cudart,cublaslt}.py of the reference: instead of a CUDA
 driver launch (library/cuda.py:249-267) or a cuBLASLt call (library/cublaslt.py:113-150)
@@ -6,91 +6,31 @@ per kernel, every kernel has one ``extern "C"`` launcher.  A non-zero status rai
 ``RuntimeError`` like the reference's check*Status helpers (library/cudart.py:325-327).
 """
 import ctypes
-from .base import Lib
+from .base import Lib, load_native
 
 lib = Lib("cpmk_hip")
 
-# launchers: name -> argument ctypes (all return int status)
-_LAUNCHERS = {
-    "cpmk_gemm_calc_scale": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_calc_scale_transpose": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_round": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_round_transpose": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_scale": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_gemm_scale_x": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_scale_y": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_int8": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_int8_scale": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_quantize": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_gemm_quantize_pair": [ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p],
-    "cpmk_gemm_quantize_cols": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_gemm_fp16": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_quantize_cols_ld": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p],
-    "cpmk_gemm_quantize_pair_ld": [ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p],
-    "cpmk_gemm_backward_round_scale_ld": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_gemm_int8_scale_one": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_transpose_i8_ld": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p],
-    "cpmk_gemm_int8_scale_sum": [ctypes.c_int32] * 5 + [ctypes.c_void_p] * 5,
-    "cpmk_gemm_fp16_sum": [ctypes.c_int32] * 5 + [ctypes.c_void_p] * 4,
-    "cpmk_gemv_fp16": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemv_fp16_transpose": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemv_broadcast_mat_fp16": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_embedding_forward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_embedding_step": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_copy_data_to_kv": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p],
-    "cpmk_gemv_calc_scale": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemv_round": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemv_broadcast_mat_int8": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_layernorm_forward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_layernorm_forward_noalloc": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_layernorm_step": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_layernorm_affine_forward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_layernorm_affine_forward_stats": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_layernorm_affine_backward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32] + [ctypes.c_void_p] * 9,
-    "cpmk_softmax_forward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_softmax_step_inplace": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gelu_forward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_position_embedding_init": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_position_embedding_forward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_position_embedding_step": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_arith_ln_mul_add": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_ln_mul": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_element_add": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_mask": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_global_scale": [ctypes.c_int64, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_element_mul": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_batch_add_forward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_batch_add_backward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_ln_add": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_ln_div": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_ln_sub_div": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_ln_mul_backward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_ln_add_backward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_batch_mul_add": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_arith_batch_mul": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gelu_backward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_softmax_backward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_layernorm_forward_v": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p],
-    "cpmk_layernorm_forward_mv": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p],
-    "cpmk_layernorm_backward_v": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_layernorm_backward_mv": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_gemm_backward_round_scale": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_gemm_backward_scale_round": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_position_embedding_backward": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "cpmk_embedding_backward_stage1": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_embedding_backward_stage2": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_transpose": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_transpose_i8": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_array_add": [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p],
-    "cpmk_adjustify_logits": [ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_float, ctypes.c_float, ctypes.c_float, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_copy_extend_buffer": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_has_nan_inf": [ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_copy_pos_hidden": [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
-    "cpmk_async_status": [],
-    "cpmk_selftest_exchange_timeout": [ctypes.c_int32, ctypes.c_void_p],
-}
+# the launchers (all return an int status), without their prefix; native/call.cpp takes their argument types from include/cpmk.h
+_LAUNCHERS = (
+    "gemm_calc_scale", "gemm_calc_scale_transpose", "gemm_round", "gemm_round_transpose", "gemm_scale",
+    "gemm_scale_x", "gemm_scale_y", "gemm_int8", "gemm_int8_scale", "gemm_quantize", "gemm_quantize_pair",
+    "gemm_quantize_cols", "gemm_fp16", "gemm_quantize_cols_ld", "gemm_quantize_pair_ld",
+    "gemm_backward_round_scale_ld", "gemm_int8_scale_one", "transpose_i8_ld", "gemm_int8_scale_sum", "gemm_fp16_sum",
+    "gemv_fp16", "gemv_fp16_transpose", "gemv_broadcast_mat_fp16", "embedding_forward", "embedding_step",
+    "copy_data_to_kv", "gemv_calc_scale", "gemv_round", "gemv_broadcast_mat_int8", "layernorm_forward",
+    "layernorm_forward_noalloc", "layernorm_step", "layernorm_affine_forward", "layernorm_affine_forward_stats",
+    "layernorm_affine_backward", "softmax_forward", "softmax_step_inplace", "gelu_forward", "position_embedding_init",
+    "position_embedding_forward", "position_embedding_step", "arith_ln_mul_add", "arith_ln_mul", "arith_element_add",
+    "mask", "arith_global_scale", "arith_element_mul", "arith_batch_add_forward", "arith_batch_add_backward",
+    "arith_ln_add", "arith_ln_div", "arith_ln_sub_div", "arith_ln_mul_backward", "arith_ln_add_backward",
+    "arith_batch_mul_add", "arith_batch_mul", "gelu_backward", "softmax_backward", "layernorm_forward_v",
+    "layernorm_forward_mv", "layernorm_backward_v", "layernorm_backward_mv", "gemm_backward_round_scale",
+    "gemm_backward_scale_round", "position_embedding_backward", "embedding_backward_stage1",
+    "embedding_backward_stage2", "transpose", "transpose_i8", "array_add", "adjustify_logits", "copy_extend_buffer",
+    "has_nan_inf", "copy_pos_hidden", "async_status", "selftest_exchange_timeout",
+)
 
-EXPORTED_SYMBOLS = sorted(list(_LAUNCHERS) + [
+EXPORTED_SYMBOLS = sorted(["cpmk_" + n for n in _LAUNCHERS] + [
     "cpmk_version", "cpmk_error_string", "cpmk_device_count", "cpmk_get_device",
     "cpmk_set_device", "cpmk_device_props", "cpmk_exchange_capture_slots_left", "cpmk_gemm_sum_groups",
 ])
@@ -111,17 +51,31 @@ def checkStatus(status: int) -> None:
         raise RuntimeError("HIP Error: %s" % error_string(status))
 
 
-def _make(name, argtypes):
-    @lib.bind(name, argtypes, ctypes.c_int)
+def _address(obj):
+    """The address a pointer argument that is neither an int nor None stands for (ctypes.c_void_p and what ctypes casts to it)."""
+    return obj.value if isinstance(obj, ctypes.c_void_p) else ctypes.cast(obj, ctypes.c_void_p).value
+
+
+_native = load_native("_cpmk_call") if lib.loaded else None
+if _native is not None:
+    _native.init(lib.address("cpmk_error_string"), _address)
+
+
+def _make(name):
+    address = lib.address(name)
+    if address is not None and _native is not None:
+        return _native.bind(name, address)
+
     def call(*args):
-        checkStatus(getattr(lib, name)(*args))
+        if lib.loaded and _native is not None:
+            raise AttributeError("%s: undefined symbol: %s" % (lib.path, name))
+        raise RuntimeError("Library %s is not initialized" % ("_cpmk_call" if lib.loaded else "cpmk_hip"))
     call.__name__ = name[len("cpmk_"):]
-    call.__doc__ = "Launch %s (see include/cpmk.h)." % name
     return call
 
 
-for _name, _argtypes in _LAUNCHERS.items():
-    globals()[_name[len("cpmk_"):]] = _make(_name, _argtypes)
+for _name in _LAUNCHERS:
+    globals()[_name] = _make("cpmk_" + _name)
 
 
 def check() -> None:

@@ -30,6 +30,21 @@ __device__ __forceinline__ half8_t load_half8_any(const half_t* p) { return __bu
 __device__ __forceinline__ void store_half8_any(half_t* p, half8_t v) { *reinterpret_cast<Half8Any*>(p) = __builtin_bit_cast(Half8Any, v); }
 __device__ __forceinline__ void store_byte8_any(int8_t* p, uint32_t lo, uint32_t hi) { *reinterpret_cast<Byte8Any*>(p) = Byte8Any{lo, hi}; }
 
+// An 8 x 8 block of halves, one row per vector, transposed in registers: 32 v_perm_b32 (selector bytes 0-3 pick from the
+// second operand, 4-7 from the first).
+__device__ __forceinline__ void transpose_half8x8(half8_t (&v)[8]) {
+    uint4_t r[8];
+#pragma unroll
+    for (int p = 0; p < 8; ++p) r[p] = __builtin_bit_cast(uint4_t, v[p]);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        uint4_t t;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t[k] = __builtin_amdgcn_perm(r[2 * k + 1][c >> 1], r[2 * k][c >> 1], (c & 1) ? 0x07060302u : 0x05040100u);
+        v[c] = __builtin_bit_cast(half8_t, t);
+    }
+}
+
 // The first t (1..7, the same for the whole wave) of eight halves at p, at any address, in at most three accesses
 // (8, 4 and 2 bytes); the other elements of the result keep `r`'s values.
 struct __attribute__((packed, aligned(2))) Half4Any { uint32_t x, y; };

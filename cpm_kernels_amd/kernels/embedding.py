@@ -43,3 +43,23 @@ def embedding_backward_stage2(batch: int, hidden_size: int,
                               stream: CUDAStream):
     """Adds the per-entry tail runs into grad.  reference: kernels/embedding.py:67-86"""
     cpmk.embedding_backward_stage2(batch, hidden_size, aux_grad, aux_grad_idx, grad, stream)
+
+
+def embedding_order_ids(tokens: int,
+                        ids: DevicePointer,             # (tokens) int32
+                        order: DevicePointer,           # (tokens) int32
+                        sorted_ids: DevicePointer,      # (tokens) int32
+                        stream: CUDAStream):
+    """The tokens in the order of their ids, equal ids in the order of the tokens (quadratic in the number of tokens)."""
+    cpmk.embedding_order_ids(tokens, ids, order, sorted_ids, stream)
+
+
+def embedding_backward_rows(tokens: int, hidden_size: int,
+                            grad_rows: DevicePointer,   # (tokens, hidden_size) fp16
+                            order: DevicePointer,       # (tokens) int32: tokens sorted by their ids
+                            sorted_ids: DevicePointer,  # (tokens) int32
+                            grad: DevicePointer,        # (vocab_size, hidden_size) fp16, rows of absent ids are left alone
+                            partials: DevicePointer,    # 2 * ceil(tokens / 32) * hidden_size fp32
+                            stream: CUDAStream):
+    """What embedding_backward_stage1 and _stage2 compute together, summed in fp32 and rounded once."""
+    cpmk.embedding_backward_rows(tokens, hidden_size, grad_rows, order, sorted_ids, grad, partials, stream)

@@ -26,8 +26,8 @@ _LAUNCHERS = (
     "arith_batch_mul_add", "arith_batch_mul", "gelu_backward", "softmax_backward", "layernorm_forward_v",
     "layernorm_forward_mv", "layernorm_backward_v", "layernorm_backward_mv", "gemm_backward_round_scale",
     "gemm_backward_scale_round", "position_embedding_backward", "embedding_backward_stage1",
-    "embedding_backward_stage2", "transpose", "transpose_i8", "array_add", "adjustify_logits", "copy_extend_buffer",
-    "has_nan_inf", "copy_pos_hidden", "async_status", "selftest_exchange_timeout",
+    "embedding_backward_stage2", "embedding_order_ids", "embedding_backward_rows", "transpose", "transpose_i8", "array_add",
+    "adjustify_logits", "copy_extend_buffer", "has_nan_inf", "copy_pos_hidden", "async_status", "selftest_exchange_timeout",
 )
 
 EXPORTED_SYMBOLS = sorted(["cpmk_" + n for n in _LAUNCHERS] + [

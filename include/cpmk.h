@@ -401,6 +401,14 @@ int cpmk_embedding_backward_stage1(int32_t batch, int32_t seq_len, int32_t hidde
 int cpmk_embedding_backward_stage2(int32_t batch, int32_t hidden_size, const void* aux_grad, const void* aux_grad_idx,
                                    void* grad, void* stream);
 
+/* The tokens in the order of their ids (equal ids in the order of the tokens): order[r] = token, sorted_ids[r] = its id.
+ * Quadratic in the number of tokens: meant for up to some tens of thousands. */
+int cpmk_embedding_order_ids(int32_t tokens, const void* ids, void* order, void* sorted_ids, void* stream);
+/* The whole gradient of a table from gradient rows (tokens, hidden) and the order of the ids: the fp32 sum of the rows of
+ * every id that occurs, rounded once; other rows of grad are left alone.  partials: 2 * ceil(tokens / 32) * hidden fp32. */
+int cpmk_embedding_backward_rows(int32_t tokens, int32_t hidden_size, const void* grad_rows, const void* order,
+                                 const void* sorted_ids, void* grad, void* partials, void* stream);
+
 /* (batch, n, m) -> (batch, m, n), fp16.               kernels/transpose.py:11-29 / transpose.cu:6-24 */
 int cpmk_transpose(int32_t batch, int32_t n, int32_t m, const void* inp, void* out, void* stream);
 

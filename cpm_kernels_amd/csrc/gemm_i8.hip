@@ -361,7 +361,7 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
         }
     }
     // one operand stored (K, rows) and a depth beyond one slab that is not whole slabs: the 32x32 form of the tile kernel,
-    // the rest of the depth straight from memory into the fragments
+    // the rest of the depth as a slab filled up with zeros
     if (p_kmajor != q_kmajor && wide && k > 128 && (k % 4 == 0) && aligned16(A) && aligned16(B) && (!in_p || n >= 128) &&
         (!in_q || m >= 128) && (int64_t)n * k < (1ll << 32) && (int64_t)m * k < (1ll << 32)) {
         constexpr int EPI = FUSED ? kEpiDequant : kEpiInt32;
@@ -540,7 +540,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         return launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 0, 32>(a, batch, st);
     }
     // a depth that is not whole 64-byte slabs (K = 40, 72, 500, 1000 ...): the same kernels, the rest of the depth straight
-    // from memory into the fragments
+    // from memory into the fragments (large tiles) or as a slab filled up with zeros
     if (p_kmajor && q_kmajor && wide && k > 32 && (reinterpret_cast<uintptr_t>(A) & 3u) == 0 && (reinterpret_cast<uintptr_t>(B) & 3u) == 0 &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
@@ -577,7 +577,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         }
     }
     // an operand stored (K, rows) and a depth that is not whole slabs (attention: probabilities x values over 500 keys, scores
-    // over heads of 80): the 32x32 form of the tile kernel, the rest of the depth straight from memory into the fragments
+    // over heads of 80): the 32x32 form of the tile kernel, the rest of the depth as a slab filled up with zeros
     if (!(p_kmajor && q_kmajor) && wide && k > 64 && (k % 64 != 0) && aligned16(A) && aligned16(B) &&
         (!in_p || n >= 128) && (!in_q || m >= (low ? 256 : 128)) &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {

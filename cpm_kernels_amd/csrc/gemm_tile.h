@@ -106,8 +106,13 @@ __device__ __forceinline__ void store_piece(int8_t* dst, int4_t v, int32_t left)
 // fragment reads free of bank conflicts.  The DMA writes LDS in lane order, so the exchange happens in the choice of
 // what a lane fetches.
 // SUM: slab kt of a tile is slab kt % nkb of batch entry kt / nkb (counted from the tile's first entry).
-template <int BR, int BC, int BKB, int NW, int NST, int LAY, bool F16, bool TSW = false, bool SUM = false>
+// REST: a depth that is not whole slabs has the rest of it (`rem` bytes of a K-major row, any number of dwords) as slab 0
+// and its whole slabs behind that one.  What the DMA fetches past the end of K -- the last 16 bytes of a K-major row, the
+// last row of a (K, L) operand, again and again -- each lane puts right in LDS once slab 0 has landed (finish_rest): dwords
+// moved down to their places, zeros beyond K.
+template <int BR, int BC, int BKB, int NW, int NST, int LAY, bool F16, bool TSW = false, bool SUM = false, bool REST = false>
 struct SlabDma {
+    static_assert(!(REST && SUM), "sums over the batch take the rest of the depth from memory");
     static constexpr bool PT = (LAY & 1) != 0, QT = (LAY & 2) != 0;
     static constexpr int ESZ_IN = F16 ? 2 : 1;            // bytes per operand element
     static constexpr int EPP = 16 / ESZ_IN;               // elements per 16-byte piece
@@ -124,6 +129,8 @@ struct SlabDma {
     const int wave, lane;
     int nk;                     // slabs per tile
     int nkb;                    // ... and per batch entry
+    int rem;                    // REST: bytes of K in slab 0, or 0: whole slabs only
+    int32_t oj0, oi0;           // first row / column of the tile
     bool ahead;                 // the next tile is fetched ahead (only if its LDS layout is this one's)
     bool deep;                  // at least as many slabs as stages
     int LD;                     // slabs in flight: the slab requested at iteration `it` is number it + LD of this tile
@@ -158,11 +165,42 @@ struct SlabDma {
         return (uint32_t)grow * (uint32_t)a.k + c * 16;
     }
 
+    // REST: the same for slab 0, relative to the end of the whole slabs; 16 bytes further on for a K-major operand (kofs takes
+    // them off again), whose last 16 bytes of K may begin before that
+    __device__ __forceinline__ uint32_t rest_voff(int d, int32_t oj, int32_t oi) const {
+        const int dd = wave + d * NW;
+        const bool q = dd * RPI >= BR;
+        if ((PT && !q) || (QT && q)) {
+            const int ppr = (q ? BC : BR) / EPP;
+            const int kr = (q ? dd - BR / RPI : dd) * (64 / ppr) + lane / ppr;
+            const int32_t L = q ? a.m : a.n;
+            return calc_voff(d, oj, oi) - (uint32_t)(kr - min(kr, rem / ESZ_IN - 1)) * (uint32_t)L * (uint32_t)ESZ_IN;
+        }
+        const int r = dd * RPI + lane / CPR;
+        const int c = (lane % CPR) ^ swz(r);
+        const int32_t grow = q ? min(oi + (r - BR), a.m - 1) : min(oj + r, a.n - 1);
+        return (uint32_t)grow * (uint32_t)a.k + (uint32_t)(16 + min(c * 16, rem - 16));
+    }
+    // bytes from an operand's start to slab kt
+    __device__ __forceinline__ int64_t kofs(bool q, int kt) const {
+        const int64_t kstep = q ? kstepQ : kstepP;
+        if constexpr (REST) {
+            if (rem != 0) {
+                const bool kmajor = q ? !QT : !PT;
+                return (kt == 0 ? nk - 1 : kt - 1) * kstep - (kt == 0 && kmajor ? 16 : 0);
+            }
+        }
+        return kt * kstep;
+    }
+
     __device__ __forceinline__ SlabDma(const GemmArgs& a_, uint32_t lds_base, const GemmItem& cur_item, const GemmItem& nxt_item,
                                        int wave_, int lane_, int ring)
         : a(a_), wave(wave_), lane(lane_) {
         nkb = a.k / BKB;
-        nk = SUM ? nkb * a.nsum : nkb;
+        rem = REST ? a.k - nkb * BKB : 0;
+        nk = SUM ? nkb * a.nsum : REST && rem != 0 ? nkb + 1 : nkb;
+        oj0 = cur_item.j0;
+        oi0 = cur_item.i0;
         const uint32_t b = SUM ? cur_item.b * (uint32_t)a.nsum : cur_item.b;
         Pb = a.P + (int64_t)b * a.strideP;
         Qb = a.Q + (int64_t)b * a.strideQ;
@@ -203,7 +241,7 @@ struct SlabDma {
             const uint32_t e = nkb == 1 ? (uint32_t)kt : __umulhi((uint32_t)kt, a.kmagic);       // kt / nkb (exact for kt * nkb < 2^32)
             lds_dma16(v, (q ? qb : pb) + (int64_t)e * (q ? a.strideQ : a.strideP) + (kt - (int)e * nkb) * BKB, ldst[d] + stage * STAGE);
         } else {
-            lds_dma16(v, (q ? qb : pb) + kt * (q ? kstepQ : kstepP), ldst[d] + stage * STAGE);
+            lds_dma16(v, (q ? qb : pb) + kofs(q, kt), ldst[d] + stage * STAGE);
         }
     }
 
@@ -211,6 +249,44 @@ struct SlabDma {
     __device__ __forceinline__ void retarget() {
 #pragma unroll
         for (int d = 0; d < CNT; ++d) voff[d] = calc_voff(d, tj0, ti0);
+    }
+    // ... and those of their slab 0, where that is the rest of the depth
+    __device__ __forceinline__ void retarget_rest() {
+#pragma unroll
+        for (int d = 0; d < CNT; ++d) voff[d] = rest_voff(d, tj0, ti0);
+    }
+
+    // Slab 0 as the DMA left it -> the rest of the depth followed by zeros.  Every lane works on the 16 bytes it fetched itself, so
+    // its own wave's wait before and the workgroup's barrier after are all it takes.
+    __device__ __forceinline__ void finish_rest() const {
+        if (rem == 0) return;
+        typedef __attribute__((address_space(3))) int4_t* lds_ptr;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < CNT; ++d) {
+            const int dd = wave + d * NW;
+            const bool q = isq[d];
+            lds_ptr p = (lds_ptr)(uintptr_t)(ldst[d] + (uint32_t)(ring0 * STAGE + lane * 16));
+            if ((PT && !q) || (QT && q)) {
+                const int ppr = (q ? BC : BR) / EPP;
+                const int kr = (q ? dd - BR / RPI : dd) * (64 / ppr) + lane / ppr;
+                if (kr * ESZ_IN >= rem) *p = int4_t{0, 0, 0, 0};
+            } else {
+                const int c = (lane % CPR) ^ swz(dd * RPI + lane / CPR);
+                const int over = min(c * 16 + 16 - rem, 16);       // bytes of the piece beyond K: 4 ... 16 (or none)
+                if (over > 0) {
+                    const int4_t t = *p;
+                    const int32_t w[8] = {t.x, t.y, t.z, t.w, 0, 0, 0, 0};
+                    const int sh = over >> 2;
+                    int4_t v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = sh == 1 ? w[e + 1] : sh == 2 ? w[e + 2] : sh == 3 ? w[e + 3] : 0;
+                    *p = v;
+                }
+            }
+        }
+        asm volatile("" ::: "memory");
     }
 
     // A tile's start.  Without slabs on their way: request the first NST, wait for slab 0.  Otherwise the first LD
@@ -221,14 +297,23 @@ struct SlabDma {
             static_for<0, NST>([&](auto sc) __attribute__((always_inline)) {
                 constexpr int st = decltype(sc)::value;
                 static_for<0, CNT>([&](auto dc) __attribute__((always_inline)) {
-                    issue<decltype(dc)::value, false>(min(st, nk - 1), (ring0 + st) % NST);
+                    constexpr int d = decltype(dc)::value;
+                    if constexpr (REST && st == 0) {
+                        if (rem != 0) {
+                            lds_dma16(rest_voff(d, oj0, oi0), (isq[d] ? Qb : Pb) + kofs(isq[d], 0), ldst[d] + ring0 * STAGE);
+                            return;
+                        }
+                    }
+                    issue<d, false>(min(st, nk - 1), (ring0 + st) % NST);
                 });
             });
             if (deep) wait_vmcnt<(NST - 1) * CNT>();   // slab 0 (and the scale loads issued before it) has landed
             else wait_vmcnt<0>();
+            if constexpr (REST) finish_rest();
             __syncthreads();
         } else {
             wait_vmcnt<0>();
+            if constexpr (REST) finish_rest();
             __syncthreads();
         }
     }
@@ -286,10 +371,10 @@ struct StripOut {
 // lets the compiler keep the accumulators in place and the MFMA/memory interleave as written.
 // Returns true if the next tile's first slabs are on their way.
 //
-// LAY bit 2: the depth is not whole slabs (any multiple of 4 bytes).  The slabs of the ring cover the whole ones; the
+// LAY bit 2: the depth is not whole slabs (any multiple of 4 bytes).  Here the slabs of the ring cover the whole ones; the
 // rest of the depth (less than a slab) goes from memory straight into the fragment registers before the K loop starts
-// -- a lane's 16 bytes of a k-step are the same bytes in memory as in the stage -- with zeros past the end of K.  (An
-// operand stored (K, rows) beside it: the 32x32 form only, which gathers such a fragment element by element.)
+// -- a lane's 16 bytes of a k-step are the same bytes in memory as in the stage -- with zeros past the end of K.  (Beside an
+// operand stored (K, rows): the 32x32 form only, where the rest is a slab of the ring, SlabDma's REST.)
 // LAY bit 3, with bit 2: the rest of a row may start off a 16-byte boundary and end inside a piece (depths and rows of
 // whole dwords only); without it every piece of the rest is whole and aligned.
 // LAY marks operands whose rows are K instead: bit 0 = the row operand is stored (K, n), bit 1 =
@@ -646,7 +731,12 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
     constexpr int KS = BKB / 32, CPR = BKB / 16;
     constexpr int NW = WR * WC, BR = WR * TR * 32, BC = WC * TC * 32;
     constexpr bool TRP = PT, TRQ = QT;             // fragments of a (K, L) operand: transposing LDS reads
-    using Dma = SlabDma<BR, BC, BKB, NW, NST, LAY, F16, TRP || TRQ>;
+    // The rest of a depth that is not whole slabs is a slab of its own: beside an operand stored (K, rows), whose fragments would
+    // have to be gathered two bytes at a time (64 x 500 x 500 over 1024 heads: 161 -> 132 us, 500 x 80 x 500 289 -> 243 us), and in the
+    // small tiles (500 x 500 x 64 over 512 heads 105 -> 93 us).  256 x 256 tiles of K-major operands are bound by their products and
+    // multiply no slab that is mostly zeros: 16 x 1000^3 60.4 us, 62.1 us so.
+    constexpr bool REST = (LAY & 4) != 0 && (PT || QT || BR * BC < 256 * 256);
+    using Dma = SlabDma<BR, BC, BKB, NW, NST, LAY, F16, TRP || TRQ, false, REST>;
     constexpr int STAGE = Dma::STAGE, CNT = Dma::CNT;      // bytes per ring stage; DMA instructions per wave and slab
     constexpr int NM = TR * TC;
     constexpr int RPW = 256 / BKB;                 // rows per 256-byte bank wrap
@@ -655,7 +745,6 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
     const int wr = wave / WC, wc = wave % WC;
     const int lrow = lane & 31, lk = lane >> 5;
     const int32_t K = a.k;
-    const int nk = K / BKB;
     auto swz = [](int r) __attribute__((always_inline)) { return (r / RPW) & (CPR - 1); };
     // fragment offsets for k-step 0; step s reads logical chunk 2s + lk: xor (2s << 4) commutes with the swizzle
     int offP[TR], offQ[TC];
@@ -675,7 +764,7 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
     const uint32_t b = cur_item.b;
     const int32_t j0 = cur_item.j0, i0 = cur_item.i0;
     const bool ahead = dma.ahead;
-    const int LD = dma.LD, ring0 = dma.ring0;
+    const int nk = dma.nk, LD = dma.LD, ring0 = dma.ring0;
     auto dma1 = [&](auto dc, int kt, auto tailc, int stage) __attribute__((always_inline)) {
         dma.template issue<decltype(dc)::value, decltype(tailc)::value>(kt, stage);
     };
@@ -706,19 +795,16 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
         for (int j = 0; j < TC; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
-    if constexpr ((LAY & 4) != 0) {
-        // The depth beyond the last whole slab, as in the 16x16 form.  Here either operand may also be stored (K, rows): its
-        // fragment -- a lane's 8 (fp16) or 16 (int8) consecutive values of K for its own row -- is then gathered element
-        // by element, adjacent lanes reading adjacent elements of a row of K.  K-major pieces may start at any address
-        // and end inside the piece (rows of K that are whole dwords, not whole 16-byte pieces).
+    if constexpr ((LAY & 4) != 0 && !REST) {
+        // The depth beyond the last whole slab, as in the 16x16 form.  Pieces may start at any address and end inside (rows of K
+        // that are whole dwords, not whole 16-byte pieces).
         const int32_t K1 = nk * BKB, rem = K - K1;           // bytes
         if (rem > 0) {
-            constexpr int EPP = 16 / ESZ_IN;
             struct __attribute__((packed, aligned(1))) Piece16 { uint32_t x, y, z, w; };
             const int8_t* Pr = a.P + (int64_t)b * a.strideP;
             const int8_t* Qr = a.Q + (int64_t)b * a.strideQ;
             // a K-major operand's piece: bytes [kc, kc + 16) of the rest of row `row`, zeros from byte `rem` on
-            // (both without branches -- a load under a condition would be waited for before the next one is issued.  The
+            // (without branches -- a load under a condition would be waited for before the next one is issued.  The
             // piece: the 16 bytes that end where the piece or K ends, moved down by the dwords that lie beyond K.)
             auto piece = [&](const int8_t* base, int32_t row, int32_t kc) __attribute__((always_inline)) {
                 if constexpr ((LAY & 8) == 0) {      // whole pieces only: one load under one condition (15 % quicker than the form below where it applies)
@@ -738,46 +824,19 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
                 for (int d = 0; d < 4; ++d) v[d] = sh == 0 ? w[d] : sh == 1 ? w[d + 1] : sh == 2 ? w[d + 2] : sh == 3 ? w[d + 3] : 0;
                 return v;
             };
-            // a (K, L) operand's piece: elements [ke, ke + EPP) of the rest of K for element `row` of the rows of K
-            auto gather = [&](const int8_t* base, int32_t L, int32_t row, int32_t ke) __attribute__((always_inline)) {
-                const int32_t kel0 = K1 / ESZ_IN, krem = rem / ESZ_IN;
-                if constexpr (F16) {
-                    half8_t h;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const half_t x = reinterpret_cast<const half_t*>(base)[(int64_t)(kel0 + min(ke + e, krem - 1)) * L + row];
-                        h[e] = ke + e < krem ? x : (half_t)0.0f;
-                    }
-                    return __builtin_bit_cast(int4_t, h);
-                } else {
-                    int4_t v = {0, 0, 0, 0};
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const uint32_t x = (uint8_t)base[(int64_t)(kel0 + min(ke + e, krem - 1)) * L + row];
-                        v[e >> 2] |= (int32_t)((ke + e < krem ? x : 0u) << (8 * (e & 3)));
-                    }
-                    return v;
-                }
-            };
             auto load_ks = [&](int4_t (&rp)[TR], int4_t (&rq)[TC], int ks) __attribute__((always_inline)) {
                 const int32_t kc = ks * 32 + lk * 16;
 #pragma unroll
                 for (int i = 0; i < TR; ++i) {
                     const int32_t row = min(j0 + wr * TR * 32 + i * 32 + lrow, a.n - 1);
                     rp[i] = int4_t{0, 0, 0, 0};
-                    if (ks * 32 < rem) {
-                        if constexpr (PT) rp[i] = gather(Pr, a.n, row, kc / ESZ_IN);
-                        else rp[i] = piece(Pr, row, kc);
-                    }
+                    if (ks * 32 < rem) rp[i] = piece(Pr, row, kc);
                 }
 #pragma unroll
                 for (int j = 0; j < TC; ++j) {
                     const int32_t col = min(i0 + wc * TC * 32 + j * 32 + lrow, a.m - 1);
                     rq[j] = int4_t{0, 0, 0, 0};
-                    if (ks * 32 < rem) {
-                        if constexpr (QT) rq[j] = gather(Qr, a.m, col, kc / ESZ_IN);
-                        else rq[j] = piece(Qr, col, kc);
-                    }
+                    if (ks * 32 < rem) rq[j] = piece(Qr, col, kc);
                 }
             };
             auto mac_ks = [&](const int4_t (&rp)[TR], const int4_t (&rq)[TC], int ks) __attribute__((always_inline)) {
@@ -793,22 +852,12 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
                         }
                 }
             };
-            if constexpr (PT || QT) {
-                // gathered fragments are many small loads: every k-step's are requested before the first product -- one trip
-                // to memory, not one per k-step
-                int4_t rp[KS][TR], rq[KS][TC];
+            // a k-step at a time, which keeps the wide accumulator tiles of this form in registers
 #pragma unroll
-                for (int ks = 0; ks < KS; ++ks) load_ks(rp[ks], rq[ks], ks);
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) mac_ks(rp[ks], rq[ks], ks);
-            } else {
-                // (K-major operands only: a k-step at a time, which keeps the wide accumulator tiles of this form in registers)
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) {
-                    int4_t rp[TR], rq[TC];
-                    load_ks(rp, rq, ks);
-                    mac_ks(rp, rq, ks);
-                }
+            for (int ks = 0; ks < KS; ++ks) {
+                int4_t rp[TR], rq[TC];
+                load_ks(rp, rq, ks);
+                mac_ks(rp, rq, ks);
             }
         }
     }
@@ -924,8 +973,17 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
     };
     int it = 0;
     for (; it < nk - LD; ++it) slab(it, std::false_type{});       // slabs LD .. nk-1 of this tile follow
-    dma.retarget();
-    for (; it < nk; ++it) slab(it, std::true_type{});             // then the tail's
+    if constexpr (REST) {
+        for (; it < nk; ++it) {                                   // then the tail's, slab 0 of the next tile first
+            const int s = it - (nk - LD);
+            if (s == 0 && ahead && dma.rem != 0) dma.retarget_rest();
+            else if (s <= 1) dma.retarget();
+            slab(it, std::true_type{});
+        }
+    } else {
+        dma.retarget();
+        for (; it < nk; ++it) slab(it, std::true_type{});         // then the tail's
+    }
     if (!ahead) wait_vmcnt<0>();         // drain the clamped loads before the ring is reused
     ring = cur;                          // (ring0 + nk) % NST: where the next tile's slab 0 is, or will be put
 

@@ -556,35 +556,35 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     const bool in_p = !p_kmajor && n % 8 != 0, in_q = !q_kmajor && m % 8 != 0;
     // 64 x 256 tiles for few output rows (attention: probabilities x values)
     const bool low = n <= 64 && !((in_q || odd) && m < 256);
-    if (!(p_kmajor && q_kmajor) && wide && k > 0 && (k % 64 == 0) && aligned16(A) && aligned16(B) &&
+    if (!(p_kmajor && q_kmajor) && wide && k >= 64 && aligned16(A) && aligned16(B) &&
         (!in_p || n >= 128) && (!in_q || m >= (low ? 256 : 128)) &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
         const int lay = (p_kmajor ? 0 : 1) | (q_kmajor ? 0 : 2);
-        // else 256x256 tiles when they give most compute units a tile, else 128x128 (as for K-major operands)
-        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
-        const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!(in_q || odd) || m >= 256);
+        // 256x256 tiles when they give most compute units a tile, else 128x128 (as for K-major operands) -- and when the
+        // larger ones cover over half as much again as the smaller ones do, where that costs more than their better ratio of products to reads
+        // saves: 300 x 300 over 400 heads, K = 512 152 us with large tiles, 125 us with small ones, K = 80 both stored (K, rows) 66 and 48 us;
+        // 580 x 580 (1.44 times the area) alike; with one operand K-major and K = 80 70 us with large tiles, 74 us with small ones.
+        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256), mid = ceil_div(n, 128) * ceil_div(m, 128);
+        const bool waste = big * 8 > mid * 3 && (lay == 3 || k >= 256);
+        const bool large = !waste && big * batch * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!(in_q || odd) || m >= 256);
         a.edge_in = (in_p ? 1 : 0) | (in_q || odd ? 2 : 0);
+        // a depth that is not whole slabs (probabilities x values over 500 keys, scores over heads of 80): its rest is a slab
+        // filled up with zeros
+        const bool rest = k % 64 != 0;
         switch (lay) {
             case 1:
-                if (low) return launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 1, 32>(a, batch, st);
-                return large ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 1, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 1, 32>(a, batch, st);
+                if (low) return rest ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 13, 32>(a, batch, st) : launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 1, 32>(a, batch, st);
+                if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 13, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 1, 16>(a, batch, st);
+                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 13, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 1, 32>(a, batch, st);
             case 2:
-                if (low) return launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 2, 32>(a, batch, st);
-                return large ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 2, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 2, 32>(a, batch, st);
+                if (low) return rest ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 14, 32>(a, batch, st) : launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 2, 32>(a, batch, st);
+                if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 14, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 2, 16>(a, batch, st);
+                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 14, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 2, 32>(a, batch, st);
             default:
-                if (low) return launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 3, 32>(a, batch, st);
-                return large ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 3, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 3, 32>(a, batch, st);
+                if (low && !rest) return launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 3, 32>(a, batch, st);
+                if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 15, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 3, 16>(a, batch, st);
+                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 15, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 3, 32>(a, batch, st);
         }
-    }
-    // an operand stored (K, rows) and a depth that is not whole slabs (attention: probabilities x values over 500 keys, scores
-    // over heads of 80): the 32x32 form of the tile kernel, the rest of the depth as a slab filled up with zeros
-    if (!(p_kmajor && q_kmajor) && wide && k > 64 && (k % 64 != 0) && aligned16(A) && aligned16(B) &&
-        (!in_p || n >= 128) && (!in_q || m >= (low ? 256 : 128)) &&
-        (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
-        a.edge_in = (in_p ? 1 : 0) | (in_q || odd ? 2 : 0);
-        if (!p_kmajor && !q_kmajor) return launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 15, 32>(a, batch, st, 2);
-        if (!p_kmajor) return low ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 13, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 13, 32>(a, batch, st);
-        return low ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 14, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 14, 32>(a, batch, st);
     }
     for (int64_t r0 = 0; r0 < n; r0 += 65535ll * 64) {        // (rows beyond the grid's y dimension: several launches)
         const int64_t nr = n - r0 < 65535ll * 64 ? n - r0 : 65535ll * 64;

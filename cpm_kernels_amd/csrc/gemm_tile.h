@@ -319,6 +319,23 @@ struct SlabDma {
     }
 };
 
+// The last iterations of a tile, from `it` on: the next tile's slab 0 first, which has offsets of its own where it is the rest of
+// the depth.
+template <bool REST, class Dma, class F>
+__device__ __forceinline__ void tail_slabs(Dma& dma, int it, F&& slab) {
+    if constexpr (REST) {
+        const int first = it;
+        for (; it < dma.nk; ++it) {
+            if (it == first && dma.ahead && dma.rem != 0) dma.retarget_rest();
+            else if (it <= first + 1) dma.retarget();
+            slab(it, std::true_type{});
+        }
+    } else {
+        dma.retarget();
+        for (; it < dma.nk; ++it) slab(it, std::true_type{});
+    }
+}
+
 // The way out of a tile, shared by the two forms of the tile function.  Results leave through a 4 KB strip of
 // LDS per wave: a lane holds 4-column pieces of ONE output row, so storing straight from the accumulators
 // would touch 32 different rows with 8 or 16 bytes each per instruction.  Written to the strip as 32 rows x RB
@@ -374,7 +391,7 @@ struct StripOut {
 // LAY bit 2: the depth is not whole slabs (any multiple of 4 bytes).  Here the slabs of the ring cover the whole ones; the
 // rest of the depth (less than a slab) goes from memory straight into the fragment registers before the K loop starts
 // -- a lane's 16 bytes of a k-step are the same bytes in memory as in the stage -- with zeros past the end of K.  (Beside an
-// operand stored (K, rows): the 32x32 form only, where the rest is a slab of the ring, SlabDma's REST.)
+// operand stored (K, rows) the rest is a slab of the ring: SlabDma's REST.)
 // LAY bit 3, with bit 2: the rest of a row may start off a 16-byte boundary and end inside a piece (depths and rows of
 // whole dwords only); without it every piece of the rest is whole and aligned.
 // LAY marks operands whose rows are K instead: bit 0 = the row operand is stored (K, n), bit 1 =
@@ -397,7 +414,8 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
     constexpr int AR = TR * 2, AC = TC * 2;        // 16x16 MFMA tiles of a wave
     constexpr int NW = WR * WC, BR = WR * TR * 32, BC = WC * TC * 32;
     constexpr bool TRP = PT, TRQ = QT;             // fragments of a (K, L) operand: transposing LDS reads
-    using Dma = SlabDma<BR, BC, BKB, NW, NST, LAY, F16, TRP || TRQ, SUM>;
+    constexpr bool REST = (LAY & 4) != 0 && (PT || QT);       // the rest of the depth is a slab of the ring
+    using Dma = SlabDma<BR, BC, BKB, NW, NST, LAY, F16, TRP || TRQ, SUM, REST>;
     constexpr int STAGE = Dma::STAGE, CNT = Dma::CNT;      // bytes per ring stage; DMA instructions per wave and slab
     constexpr int RPW = 256 / BKB;                 // rows per 256-byte bank wrap
     const int tid = threadIdx.x, lane = tid & 63;
@@ -405,7 +423,7 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
     const int wr = wave / WC, wc = wave % WC;
     const int r16 = lane & 15, q = lane >> 4;
     const int32_t K = a.k;
-    const int nkb = K / BKB, nk = SUM ? nkb * a.nsum : nkb;
+    const int nkb = K / BKB;
     auto swz = [](int r) __attribute__((always_inline)) { return (r / RPW) & (CPR - 1); };
     // fragment offsets of the wave's first block of 16 rows, k-step 0.  Step s reads logical chunk
     // 4s + q: xor (4s << 4) commutes with the swizzle; block i lies 16 rows further on, where the swizzle repeats.
@@ -420,7 +438,7 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
     const uint32_t b = cur_item.b;
     const int32_t j0 = cur_item.j0, i0 = cur_item.i0;
     const bool ahead = dma.ahead;
-    const int LD = dma.LD, ring0 = dma.ring0;
+    const int nk = dma.nk, LD = dma.LD, ring0 = dma.ring0;
     auto dma1 = [&](auto dc, int kt, auto tailc, int stage) __attribute__((always_inline)) {
         dma.template issue<decltype(dc)::value, decltype(tailc)::value>(kt, stage);
     };
@@ -466,7 +484,7 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
         for (int j = 0; j < AC; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[i][j][e] = 0;
-    if constexpr ((LAY & 4) != 0) {
+    if constexpr ((LAY & 4) != 0 && !REST) {
         const int32_t K1 = nkb * BKB, rem = K - K1;
         for (int32_t eb = 0; eb < (SUM ? a.nsum : 1) && rem > 0; ++eb) {
             const int64_t be = SUM ? (int64_t)b * a.nsum + eb : (int64_t)b;
@@ -654,8 +672,7 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
         for (; it < nk; ++it) { slab(it, std::true_type{}); fold(); }
     } else {
         for (; it < nk - LD; ++it) slab(it, std::false_type{});       // slabs LD .. nk-1 of this tile follow
-        dma.retarget();
-        for (; it < nk; ++it) slab(it, std::true_type{});             // then the tail's
+        tail_slabs<REST>(dma, it, slab);                              // then the tail's
     }
     if (!ahead) wait_vmcnt<0>();         // drain the clamped loads before the ring is reused
     ring = cur;                          // (ring0 + nk) % NST: where the next tile's slab 0 is, or will be put
@@ -973,17 +990,7 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
     };
     int it = 0;
     for (; it < nk - LD; ++it) slab(it, std::false_type{});       // slabs LD .. nk-1 of this tile follow
-    if constexpr (REST) {
-        for (; it < nk; ++it) {                                   // then the tail's, slab 0 of the next tile first
-            const int s = it - (nk - LD);
-            if (s == 0 && ahead && dma.rem != 0) dma.retarget_rest();
-            else if (s <= 1) dma.retarget();
-            slab(it, std::true_type{});
-        }
-    } else {
-        dma.retarget();
-        for (; it < nk; ++it) slab(it, std::true_type{});         // then the tail's
-    }
+    tail_slabs<REST>(dma, it, slab);                              // then the tail's
     if (!ahead) wait_vmcnt<0>();         // drain the clamped loads before the ring is reused
     ring = cur;                          // (ring0 + nk) % NST: where the next tile's slab 0 is, or will be put
 

@@ -51,14 +51,20 @@ def checkStatus(status: int) -> None:
         raise RuntimeError("HIP Error: %s" % error_string(status))
 
 
-def _address(obj):
-    """The address a pointer argument that is neither an int nor None stands for (ctypes.c_void_p and what ctypes casts to it)."""
-    return obj.value if isinstance(obj, ctypes.c_void_p) else ctypes.cast(obj, ctypes.c_void_p).value
+def _value(obj, size=None):
+    """What an argument stands for that is no Python number: for a pointer its address (ctypes.c_void_p and what ctypes casts
+    to it), else the value of a ctypes number of the parameter's own type (size 4 or 8: integers, 0: float)."""
+    if size is None:
+        return obj.value if isinstance(obj, ctypes.c_void_p) else ctypes.cast(obj, ctypes.c_void_p).value
+    ctype = {0: ctypes.c_float, 4: ctypes.c_int32, 8: ctypes.c_int64}[size]
+    if isinstance(obj, ctype):
+        return obj.value
+    raise TypeError("expected a number or a %s, got %s" % (ctype.__name__, type(obj).__name__))
 
 
 _native = load_native("_cpmk_call") if lib.loaded else None
 if _native is not None:
-    _native.init(lib.address("cpmk_error_string"), _address)
+    _native.init(lib.address("cpmk_error_string"), _value)
 
 
 def _make(name):

@@ -4,8 +4,8 @@
 //
 // The library itself is loaded by library/base.py (search order, one HIP runtime per process); bind() is given the
 // address of a launcher in it.  Conversions are those of ctypes: integers of any size are taken modulo the parameter's width, pointers
-// are integers, None or ctypes.c_void_p (anything else that ctypes accepts goes through the `address` callable of
-// init()), and the call runs without the interpreter lock.  A non-zero status raises RuntimeError("HIP Error: ...").
+// are integers, None or ctypes.c_void_p (anything else that ctypes accepts goes through the callable of
+// init(), as ctypes numbers do), and the call runs without the interpreter lock.  A non-zero status raises RuntimeError("HIP Error: ...").
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <cstdint>
@@ -18,9 +18,21 @@
 namespace {
 
 const char* (*g_error_string)(int) = nullptr;
-PyObject* g_address = nullptr;          // callable: object -> int, for the pointer arguments that are neither int nor None
+// callable: object -> address, for the pointer arguments that are neither int nor None;
+// (object, bytes of the integer parameter or 0 for a float one) -> number, for what is no Python number
+PyObject* g_value = nullptr;
 
 bool convert(PyObject* o, float& out) {
+    const PyNumberMethods* m = Py_TYPE(o)->tp_as_number;
+    if (m == nullptr || (m->nb_float == nullptr && m->nb_index == nullptr)) {
+        PyObject* f = PyObject_CallFunction(g_value, "Oi", o, 0);
+        if (f == nullptr) return false;
+        const double d = PyFloat_AsDouble(f);
+        Py_DECREF(f);
+        if (d == -1.0 && PyErr_Occurred()) return false;
+        out = (float)d;
+        return true;
+    }
     const double d = PyFloat_AsDouble(o);
     if (d == -1.0 && PyErr_Occurred()) return false;
     out = (float)d;
@@ -30,7 +42,7 @@ bool convert(PyObject* o, float& out) {
 template <class T>
 std::enable_if_t<std::is_integral_v<T>, bool> convert(PyObject* o, T& out) {
     if (!PyLong_Check(o)) {
-        PyObject* i = PyNumber_Index(o);
+        PyObject* i = PyIndex_Check(o) ? PyNumber_Index(o) : PyObject_CallFunction(g_value, "Oi", o, (int)sizeof(T));
         if (i == nullptr) return false;
         const bool ok = convert(i, out);
         Py_DECREF(i);
@@ -49,7 +61,7 @@ bool convert(PyObject* o, T*& out) {
         return true;
     }
     if (!PyLong_Check(o)) {
-        PyObject* i = PyObject_CallOneArg(g_address, o);
+        PyObject* i = PyObject_CallOneArg(g_value, o);
         if (i == nullptr) return false;
         const bool ok = PyLong_Check(i) || i == Py_None ? convert(i, out) : (PyErr_SetString(PyExc_TypeError, "a device address is an integer"), false);
         Py_DECREF(i);
@@ -176,15 +188,15 @@ PyMethodDef g_launchers[] = {
     CPMK_ENTRY(cpmk_selftest_exchange_timeout)
 };
 
-// init(address of cpmk_error_string, callable object -> address)
+// init(address of cpmk_error_string, callable object[, size] -> address or number)
 PyObject* init(PyObject*, PyObject* args) {
     unsigned long long err;
-    PyObject* address;
-    if (!PyArg_ParseTuple(args, "KO", &err, &address)) return nullptr;
+    PyObject* value;
+    if (!PyArg_ParseTuple(args, "KO", &err, &value)) return nullptr;
     g_error_string = reinterpret_cast<const char* (*)(int)>((uintptr_t)err);
-    Py_INCREF(address);
-    Py_XDECREF(g_address);
-    g_address = address;
+    Py_INCREF(value);
+    Py_XDECREF(g_value);
+    g_value = value;
     Py_RETURN_NONE;
 }
 
@@ -207,6 +219,7 @@ PyObject* bind(PyObject*, PyObject* args) {
 
 PyObject* names(PyObject*, PyObject*) {
     PyObject* l = PyList_New(0);
+    if (l == nullptr) return nullptr;
     for (PyMethodDef& d : g_launchers) {
         PyObject* s = PyUnicode_FromString(d.ml_name);
         if (s == nullptr || PyList_Append(l, s) != 0) {
@@ -220,7 +233,7 @@ PyObject* names(PyObject*, PyObject*) {
 }
 
 PyMethodDef g_methods[] = {
-    {"init", init, METH_VARARGS, "init(address of cpmk_error_string, callable object -> address)"},
+    {"init", init, METH_VARARGS, "init(address of cpmk_error_string, callable object[, size] -> address or number)"},
     {"bind", bind, METH_VARARGS, "bind(name, address) -> callable"},
     {"names", names, METH_NOARGS, "names of the launchers"},
     {nullptr, nullptr, 0, nullptr},

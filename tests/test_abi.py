@@ -180,6 +180,24 @@ def test_null_buffers_are_refused_before_any_launch():
             pytest.fail(f"call {i} accepted a null buffer")
 
 
+def test_launchers_take_ctypes_numbers_of_the_parameters_type():
+    """As ctypes function prototypes do: c_int32 for an int32_t parameter (not another width), c_float for a float one, and any
+    object with an index."""
+    import ctypes
+    import numpy as np
+    from cpm_kernels_amd.library import cpmk
+    cpmk.gelu_forward(ctypes.c_int32(0), np.int64(8), None, ctypes.c_void_p(0), None)
+    cpmk.layernorm_forward(0, 4, 8, None, None, ctypes.c_float(1e-5), 1, None)
+    cpmk.layernorm_forward(0, 4, 8, None, None, np.float64(1e-5), True, None)
+    cpmk.arith_global_scale(ctypes.c_int64(0), None, 1, None, None)
+    for bad in (ctypes.c_int64(0), ctypes.c_float(0), 0.0, "0", None):
+        with pytest.raises(TypeError):
+            cpmk.gelu_forward(bad, 8, None, None, None)
+    for bad in (ctypes.c_int32(0), ctypes.c_double(0), "0", None):
+        with pytest.raises(TypeError):
+            cpmk.layernorm_forward(0, 4, 8, None, None, bad, 1, None)
+
+
 def test_missing_library_gives_stubs_not_import_errors():
     """cpm_kernels/library/base.py:67-74 of the reference: an absent library leaves the package
     importable and every bound call raises RuntimeError('Library ... is not initialized')."""

@@ -24,10 +24,10 @@ __device__ inline half8_t affine8(half8_t y, half_t a, half_t b, bool has_beta) 
 }
 
 // Single pass: the whole (n x LPR*8) column tile lives in registers.  Tiles of whole cache lines (LPR == 8) are
-// read and written with the non-temporal hint: every byte is touched once (8 x 4096 x 512 through the team
-// kernel: 17.2 -> 15.2 us).
-// (results are always stored plainly: a product's quantiser reads them next, from the last-level cache where they still are there;
-// a whole layer of 16 x 1024 tokens 5890 -> 5862 us, k_gelu's result alike)
+// read with the non-temporal hint: every byte is touched once.  Results are stored plainly, whatever the kernel alone
+// would gain by the hint (8 x 4096 x 512 through the team kernel, both hints: 17.2 -> 15.2 us): a product's quantiser reads
+// them next, from the last-level cache where they still are there (a whole layer of 16 x 1024 tokens 5890 -> 5862 us,
+// k_gelu's result stored alike).
 // MODE 0: 16-byte accesses, loads non-temporal where a tile's row segments are whole cache lines; 1: 16-byte accesses without
 // the hint (rows that do not start on 128-byte boundaries); 2: any m and alignment, element by element (dim1.h).
 template <int NT, int LPR, int R, bool AFF, int MODE = 0>

@@ -1051,16 +1051,17 @@ int cpmk_arith_ln_sub_div(int32_t batch, int32_t n, int32_t m, const void* inp, 
     if (m % 2) return CPMK_EALIGN;
     return launch_ew<kSubDiv, 2>((int64_t)batch * n, m, n, inp, alpha, beta, out, stream);
 }
-int cpmk_arith_batch_add_backward(int32_t batch, int32_t n, const void* grad_out, void* grad, void* stream) {
+int cpmk_arith_batch_add_backward(int32_t batch, int64_t n, const void* grad_out, void* grad, void* stream) {
     clear_stale_error();
     if (batch < 0 || n < 0) return CPMK_EBADARG;
     if (n == 0) return 0;
     if (grad == nullptr || (batch > 0 && grad_out == nullptr)) return CPMK_EBADARG;
+    if (ceil_div(n, 256 * 8) >= 1 << 24) return CPMK_ETOOBIG;       // (a launch holds fewer than 2^32 threads)
     // enough lanes for the whole chip: with few columns, more row groups per workgroup
     int rgs = 1;
     while (rgs < 64 && ceil_div(n, 8) * rgs < 131072 && rgs * 2 <= batch) rgs *= 2;
     hipLaunchKernelGGL(k_batch_add_backward, dim3((unsigned)ceil_div(n, (256 / rgs) * 8)), dim3(256), 0, (hipStream_t)stream, (int64_t)batch,
-                       (int64_t)n, rgs, (const half_t*)grad_out, (half_t*)grad);
+                       n, rgs, (const half_t*)grad_out, (half_t*)grad);
     return launch_status();
 }
 int cpmk_arith_ln_mul_backward(int32_t batch, int32_t n, int32_t m, const void* inp, const void* grad_out, void* grad, void* stream) {

@@ -331,8 +331,9 @@ int cpmk_arith_global_scale(int64_t n, const void* inp, float scale, void* out, 
 int cpmk_arith_element_mul(int32_t batch, int32_t n, const void* x, const void* y, void* out, void* stream);
 /* out[b,j] = x[b,j] + y[j]; n % 2 == 0.               kernels/arith.py:93-116 / arith.cu:47-58 */
 int cpmk_arith_batch_add_forward(int32_t batch, int32_t n, const void* x, const void* y, void* out, void* stream);
-/* grad[j] = sum_b grad_out[b,j].                      kernels/arith.py:118-133 / arith.cu:61-77 */
-int cpmk_arith_batch_add_backward(int32_t batch, int32_t n, const void* grad_out, void* grad, void* stream);
+/* grad[j] = sum_b grad_out[b,j]; n may pass 2^31 (the weight gradient of a large embedding or projection).
+ *                                                     kernels/arith.py:118-133 / arith.cu:61-77 */
+int cpmk_arith_batch_add_backward(int32_t batch, int64_t n, const void* grad_out, void* grad, void* stream);
 /* out[b,i,j] = x[b,i,j] + beta[i]; m % 2 == 0.        kernels/arith.py:163-188 / arith.cu:80-94 */
 int cpmk_arith_ln_add(int32_t batch, int32_t n, int32_t m, const void* inp, const void* beta, void* out, void* stream);
 /* out[b,i,j] = x * fp16(1 / alpha[i]); m % 2 == 0.    kernels/arith.py:216-240 / arith.cu:131-143 */

@@ -180,6 +180,17 @@ def test_null_buffers_are_refused_before_any_launch():
             pytest.fail(f"call {i} accepted a null buffer")
 
 
+def test_batch_sum_takes_more_than_2_31_columns():
+    """A column count beyond 32 bits reaches the launcher whole (modulo 2^32 it would be an empty problem, which returns
+    without a result)."""
+    from cpm_kernels_amd.library import cpmk
+    for n in (2 ** 31, 2 ** 32, 2 ** 32 + 8):
+        with pytest.raises(RuntimeError, match="invalid argument"):
+            cpmk.arith_batch_add_backward(2, n, None, None, None)
+    with pytest.raises(RuntimeError, match="limit"):
+        cpmk.arith_batch_add_backward(2, 2 ** 36, 8, 8, None)
+
+
 def test_launchers_take_ctypes_numbers_of_the_parameters_type():
     """As ctypes function prototypes do: c_int32 for an int32_t parameter (not another width), c_float for a float one, and any
     object with an index."""

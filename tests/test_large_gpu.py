@@ -307,3 +307,18 @@ def test_general_gemm_with_more_rows_than_a_grid_dimension(gpu):
     refh = (Bh[0].double() @ Ah[0].double().t())
     for sl in (slice(0, 200), slice(65535 * 64 - 100, 65535 * 64 + 100), slice(n - 50, n)):
         assert_close_fp16(to_np(oh[0, sl]), refh[sl].cpu().numpy(), rtol=1e-3, atol=1e-3, what="general fp16 gemm rows %s" % (sl,))
+
+
+def test_batch_sum_beyond_2_32_columns(gpu):
+    """The sum over a batch whose entries have more than 2^32 elements (partial sums of a large weight's gradient)."""
+    n = 2 ** 32 + 12
+    _name("batch sum", 2, n)
+    x = torch.zeros((2, n), dtype=torch.half, device=gpu)
+    spans = ((0, 64), (TWO31 - 8, TWO31 + 8), (2 ** 32 - 8, n))
+    for i, (a, b) in enumerate(spans):
+        x[:, a:b] = torch.arange((b - a) * 2, device=gpu).view(2, -1).half() + i
+    out = torch.full((n,), 77.0, dtype=torch.half, device=gpu)
+    ck.arith_batch_add_backward(2, n, x.data_ptr(), out.data_ptr(), stream())
+    for a, b in spans:
+        assert torch.equal(out[a:b], x[0, a:b] + x[1, a:b]), (a, b)       # (whole numbers below 2048)
+    assert int((out == 77.0).sum()) == 0, "elements left unwritten"

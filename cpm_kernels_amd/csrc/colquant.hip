@@ -393,13 +393,16 @@ int cpmk_gemm_quantize_cols(int32_t batch, int32_t n, int32_t m, const void* mat
 int cpmk_gemm_quantize_cols_ld(int32_t batch, int32_t n, int32_t m, const void* mat, const void* row_scale, int broad_cast_row,
                                void* scale, void* out_t, int32_t ld_t, void* out_n, int32_t ld_n, void* stream) {
     clear_stale_error();
-    if (batch < 0 || n < 1 || m < 0 || (out_t && (ld_t < n || ld_t % 16)) || (out_n && (ld_n < m || (ld_n != m && ld_n % 16)))) return CPMK_EBADARG;
-    if ((out_t == nullptr) == (out_n == nullptr) && (row_scale || out_t == nullptr)) return CPMK_EBADARG;       // (both outputs: without row scales only)
-    if ((int64_t)batch * m == 0) return 0;
-    if (any_null(mat, scale)) return CPMK_EBADARG;
+    if (batch < 0 || n < 0 || m < 0 || (out_t && (ld_t < n || ld_t % 16)) || (out_n && (ld_n < m || (ld_n != m && ld_n % 16)))) return CPMK_EBADARG;
+    if ((int64_t)batch * m == 0) return 0;       // (before the buffers are looked at: those of an empty problem may be null)
+    if (scale == nullptr) return CPMK_EBADARG;
+    if (n > 0) {       // (columns of no elements: scale 0 and whatever lengthens their rows)
+        if ((out_t == nullptr) == (out_n == nullptr) && (row_scale || out_t == nullptr)) return CPMK_EBADARG;       // (both outputs: without row scales only)
+        if (mat == nullptr) return CPMK_EBADARG;
+    }
     const ColQuantArgs p = {n, m, (const half_t*)mat, (const half_t*)row_scale, broad_cast_row, (half_t*)scale, (int8_t*)out_t, (int8_t*)out_n,
                             out_t ? ld_t : 0, out_n ? ld_n : 0};
-    const int rc = row_scale ? col_quantize<true>(batch, p, (hipStream_t)stream) : col_quantize<false>(batch, p, (hipStream_t)stream);
+    const int rc = n == 0 ? -1 : row_scale ? col_quantize<true>(batch, p, (hipStream_t)stream) : col_quantize<false>(batch, p, (hipStream_t)stream);
     if (rc >= 0) return rc;
     for (int64_t b0 = 0; b0 < batch; b0 += 65535) {       // (grid y: at most 65535 batch entries per launch)
         const int64_t nb = batch - b0 < 65535 ? batch - b0 : 65535;

@@ -658,10 +658,14 @@ int cpmk_gemm_quantize_pair(int64_t rows0, const void* mat0, void* scale0, void*
 int cpmk_gemm_quantize_pair_ld(int64_t rows0, const void* mat0, void* scale0, void* out0, int64_t rows1, const void* mat1,
                                void* scale1, void* out1, int32_t m, int32_t ld, void* stream) {
     clear_stale_error();
-    if (rows0 < 0 || rows1 < 0 || m < 1 || rows0 > 0x7fffffff || rows1 > 0x7fffffff || ld < m) return CPMK_EBADARG;
+    if (rows0 < 0 || rows1 < 0 || m < 0 || rows0 > 0x7fffffff || rows1 > 0x7fffffff || ld < m) return CPMK_EBADARG;
     if (ld != m && (ld % 16 || ld > ceil_div(m, 128) * 128)) return CPMK_EBADARG;
     if (m > kRowsMax) return CPMK_ETOOBIG;
     if (rows0 + rows1 == 0) return 0;
+    if (m == 0) {       // rows of no elements, whose buffers may be null: scale 0
+        if (int e = row_absmax(rows0, 0, nullptr, scale0, (hipStream_t)stream)) return e;
+        return row_absmax(rows1, 0, nullptr, scale1, (hipStream_t)stream);
+    }
     if ((rows0 > 0 && any_null(mat0, scale0, out0)) || (rows1 > 0 && any_null(mat1, scale1, out1))) return CPMK_EBADARG;
     return quantize_pair(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, ld, (hipStream_t)stream);
 }

@@ -124,7 +124,7 @@ def _sum_entries(parts: torch.Tensor) -> torch.Tensor:
     if parts.size(0) == 1:
         return parts
     out = torch.empty((1,) + parts.shape[1:], dtype=torch.half, device=parts.device)
-    arith_batch_add_backward(parts.size(0), parts.stride(0), parts.data_ptr(), out.data_ptr(), cur_stream())
+    arith_batch_add_backward(parts.size(0), out.numel(), parts.data_ptr(), out.data_ptr(), cur_stream())
     return out
 
 
@@ -133,7 +133,7 @@ def gemm_and_scale_sum(quantA, scaleA, quantB) -> torch.Tensor:
     batch, M, K = quantA.size()
     N = quantB.size(1)
     groups = gemm_sum_groups(N, M, batch)
-    if groups == batch or quantB.size(0) != batch or K % 128 != 0 or max(M, N) * K >= 2 ** 31 or batch * K >= 2 ** 22:
+    if groups == batch or quantB.size(0) != batch or K == 0 or K % 128 != 0 or max(M, N) * K >= 2 ** 31 or batch * K >= 2 ** 22:
         return _sum_entries(gemm_and_scale(quantA, scaleA, quantB, None, False, True))
     parts = torch.empty((groups, M, N), dtype=torch.half, device=quantA.device)
     gemm_int8_scale_sum(N, quantA.size(2), M, batch, groups, quantB.data_ptr(), quantA.data_ptr(), scaleA.data_ptr(),

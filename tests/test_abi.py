@@ -191,6 +191,26 @@ def test_batch_sum_takes_more_than_2_31_columns():
         cpmk.arith_batch_add_backward(2, 2 ** 36, 8, 8, None)
 
 
+def test_empty_problems_of_the_padded_quantisers_without_a_gpu():
+    """Empty tensors have null buffers: a call that has nothing to do returns, whatever its buffers are."""
+    from cpm_kernels_amd.library import cpmk
+    N = None
+    cpmk.gemm_quantize_cols_ld(2, 64, 0, N, N, 0, N, N, 64, N, 0, N)           # (b, K, 0): no tokens
+    cpmk.gemm_quantize_cols_ld(2, 0, 0, N, N, 0, N, N, 0, N, 0, N)
+    cpmk.gemm_quantize_cols_ld(0, 64, 8, N, N, 0, N, N, 64, N, 8, N)
+    cpmk.gemm_quantize_cols_ld(2, 64, 0, N, 8, 1, N, N, 64, N, 0, N)           # ... scaled by rows
+    cpmk.gemm_quantize_pair_ld(0, N, N, N, 0, N, N, N, 0, 0, N)
+    cpmk.gemm_quantize_pair_ld(0, N, N, N, 0, N, N, N, 64, 128, N)
+    cpmk.gemm_backward_round_scale_ld(2, 0, 64, N, N, N, 128, N, 0, N)
+    cpmk.transpose_i8_ld(2, 0, 64, N, 64, N, 0, N)
+    for call in (lambda: cpmk.gemm_quantize_cols_ld(2, 64, 8, N, N, 0, N, N, 64, N, 8, N),        # null buffers with work to do
+                 lambda: cpmk.gemm_quantize_cols_ld(2, 0, 8, N, N, 0, N, N, 0, N, 8, N),          # ... the scales
+                 lambda: cpmk.gemm_quantize_pair_ld(2, N, N, N, 0, N, N, N, 0, 0, N),
+                 lambda: cpmk.gemm_quantize_pair_ld(2, N, N, N, 0, N, N, N, 64, 128, N)):
+        with pytest.raises(RuntimeError, match="invalid argument"):
+            call()
+
+
 def test_launchers_take_ctypes_numbers_of_the_parameters_type():
     """As ctypes function prototypes do: c_int32 for an int32_t parameter (not another width), c_float for a float one, and any
     object with an index."""

@@ -18,8 +18,12 @@ static int32_t sum_groups(int32_t m, int32_t n, int32_t batch) {
     return batch;
 }
 
+// PART: fp32 out.  A group's sum may pass fp16's range where the sum over all groups does not: sums of more than one group stay
+// fp32 until they are added up (cpmk_gemm_add_parts).
+template <bool PART>
 static int gemm_sum_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                              const void* srow, void* out, hipStream_t st) {
+    constexpr int I8 = PART ? kEpiSumI8Part : kEpiSumI8, F16 = PART ? kEpiSumF16Part : kEpiSumF16;
     if (m < 0 || n < 0 || k <= 0 || batch < 1 || groups < 1 || batch % groups || batch / groups > kSumMax || groups > 65535) return CPMK_EBADARG;
     if (m % 4 || n % 4) return CPMK_EALIGN;
     if (m == 0 || n == 0) return 0;
@@ -47,17 +51,84 @@ static int gemm_sum_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t 
         // the tile is 64 x 64 where the plain product's is 128 x 64: 256x128 tiles of eight waves.  10240 x 4096 outputs over
         // 8 entries of 512: 196 us, against 287 us for the products one by one and 149 us for adding them up; waves of
         // 128 x 64, one per SIMD, 316 us (their accumulators have to be carried between the two register files to be folded).
-        if (ceil_div(n, 256) * ceil_div(m, 128) * groups * 4 >= cus * 3) return launch_dma<4, 2, 2, 2, 128, kEpiSumI8, 2, 0, 16>(a, groups, st);
+        if (ceil_div(n, 256) * ceil_div(m, 128) * groups * 4 >= cus * 3) return launch_dma<4, 2, 2, 2, 128, I8, 2, 0, 16>(a, groups, st);
         // too few of them for most compute units: 128x128 tiles, two workgroups a compute unit when there are more than compute
         // units (1024 x 2560 over 4 x 256: 12.0 us; 15.2 as 256x128), else the deeper ring (2048 x 2048 over 8 x 512: 29.8 us; two stages 31.3)
         const int64_t mid = ceil_div(n, 128) * ceil_div(m, 128) * groups;
-        if (mid > cus) return launch_dma<2, 2, 2, 2, 128, kEpiSumI8, 2, 0, 16>(a, groups, st, 2);
-        return launch_dma<2, 2, 2, 2, 128, kEpiSumI8, kRingSmall, 0, 16>(a, groups, st);
+        if (mid > cus) return launch_dma<2, 2, 2, 2, 128, I8, 2, 0, 16>(a, groups, st, 2);
+        return launch_dma<2, 2, 2, 2, 128, I8, kRingSmall, 0, 16>(a, groups, st);
     }
     const bool large = ceil_div(n, 256) * ceil_div(m, 256) * groups * 4 >= cus * 3;
-    if (kb % 128 == 0) return large ? launch_dma<2, 4, 4, 2, 128, kEpiSumF16, 2, 0, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 128, kEpiSumF16, kRingSmall, 0, 16>(a, groups, st);
-    if (whole) return large ? launch_dma<2, 4, 4, 2, 64, kEpiSumF16, 4, 4, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 64, kEpiSumF16, kRingSmall, 4, 16>(a, groups, st);
-    return large ? launch_dma<2, 4, 4, 2, 64, kEpiSumF16, 4, 12, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 64, kEpiSumF16, kRingSmall, 12, 16>(a, groups, st);
+    if (kb % 128 == 0) return large ? launch_dma<2, 4, 4, 2, 128, F16, 2, 0, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 128, F16, kRingSmall, 0, 16>(a, groups, st);
+    if (whole) return large ? launch_dma<2, 4, 4, 2, 64, F16, 4, 4, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 64, F16, kRingSmall, 4, 16>(a, groups, st);
+    return large ? launch_dma<2, 4, 4, 2, 64, F16, 4, 12, 16>(a, groups, st) : launch_dma<2, 2, 2, 2, 64, F16, kRingSmall, 12, 16>(a, groups, st);
+}
+
+// fp16 products whose operands are both stored (K, rows): the entries of a group lie one behind the other and are one
+// contraction of `k` (all of them together) as they lie.  The tile kernel's part of gemm_f16_dispatch, fp32 out.
+static int gemm_rows_parts(int32_t m, int64_t k, int32_t n, int32_t groups, const void* A, const void* B, void* out, hipStream_t st) {
+    if (m < 0 || n < 0 || k < 0 || groups < 1) return CPMK_EBADARG;
+    if (m % 2 || n % 2 || k % 2) return CPMK_EALIGN;
+    if (m == 0 || n == 0) return 0;
+    if (any_null(A, B, out)) return CPMK_EBADARG;
+    if (n * k * 2 >= (1ll << 32) || m * k * 2 >= (1ll << 32)) return CPMK_ETOOBIG;
+    const bool in_p = n % 8 != 0, in_q = m % 8 != 0;
+    if (k < 64 || (in_p && n < 128) || (in_q && m < 256) || !aligned16(A) || !aligned16(B) || !aligned16(out)) return CPMK_EALIGN;
+    GemmArgs a;
+    a.P = (const int8_t*)B; a.Q = (const int8_t*)A; a.out = out;
+    a.srow = nullptr; a.scol = nullptr;
+    a.strideP = n * k * 2;
+    a.strideQ = m * k * 2;
+    a.n = n; a.m = m; a.k = (int32_t)(k * 2); a.bc_row = 0; a.bc_col = 0;
+    a.tiles_r = a.tiles_c = 0;
+    a.edge_in = (in_p ? 1 : 0) | (in_q ? 2 : 0);
+    a.nsum = 1;
+    a.kmagic = 0;
+    const int64_t big = ceil_div(n, 256) * ceil_div(m, 256), mid = ceil_div(n, 128) * ceil_div(m, 128);
+    const bool large = big * 8 <= mid * 3 && big * groups * 4 >= (int64_t)compute_units() * 3 && n > 128 && m > 128 && (!in_p || n >= 256);
+    const bool rest = k % 64 != 0;
+    if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16Part, 2, 15, 16>(a, groups, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16Part, 2, 3, 16>(a, groups, st);
+    return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16Part, 2, 15, 32>(a, groups, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16Part, kRingSmall, 3, 32>(a, groups, st);
+}
+
+// out[j] = fp16(sum over the groups of parts[g, j]), in the order of the groups.  Bound by reading the parts.  A lane owns four
+// adjacent columns and requests eight groups at a time; with few columns the groups are dealt to `rgs` (a power of two up to 64)
+// sets of 256 / rgs lanes, as in k_batch_add_backward.
+__global__ __launch_bounds__(256) void k_add_parts(int32_t groups, int64_t n, int rgs, const float* __restrict__ parts, half_t* __restrict__ out) {
+    __shared__ float red[1024];                 // [set][column of the workgroup]
+    const int cgs = 256 / rgs, cg = threadIdx.x % cgs, rg = threadIdx.x / cgs;
+    const int64_t col = ((int64_t)blockIdx.x * cgs + cg) * 4;
+    const bool live = col < n;                  // (n % 4 == 0)
+    float4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (live) {
+        for (int32_t g0 = rg; g0 < groups; g0 += 8 * rgs) {
+            float4_t v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int32_t g = g0 + u * rgs;
+                v[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                if (g < groups) v[u] = *reinterpret_cast<const float4_t*>(parts + g * n + col);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] += v[u][e];
+        }
+    }
+    if (rgs > 1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[(rg * cgs + cg) * 4 + e] = s[e];
+        __syncthreads();
+        if (rg != 0) return;
+        for (int g = 1; g < rgs; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += red[(g * cgs + cg) * 4 + e];
+    }
+    if (!live) return;
+    half4_t r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = (half_t)s[e];
+    *reinterpret_cast<half4_t*>(out + col) = r;
 }
 
 }  // namespace cpmk
@@ -73,13 +144,42 @@ int cpmk_gemm_sum_groups(int32_t m, int32_t n, int32_t batch) {
 int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                              const void* scale_row, void* out, void* stream) {
     clear_stale_error();
-    return gemm_sum_dispatch(false, m, k, n, batch, groups, A, B, scale_row, out, (hipStream_t)stream);
+    return gemm_sum_dispatch<false>(false, m, k, n, batch, groups, A, B, scale_row, out, (hipStream_t)stream);
 }
 
 int cpmk_gemm_fp16_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                        void* out, void* stream) {
     clear_stale_error();
-    return gemm_sum_dispatch(true, m, k, n, batch, groups, A, B, nullptr, out, (hipStream_t)stream);
+    return gemm_sum_dispatch<false>(true, m, k, n, batch, groups, A, B, nullptr, out, (hipStream_t)stream);
+}
+
+int cpmk_gemm_int8_scale_parts(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
+                               const void* scale_row, void* parts, void* stream) {
+    clear_stale_error();
+    return gemm_sum_dispatch<true>(false, m, k, n, batch, groups, A, B, scale_row, parts, (hipStream_t)stream);
+}
+
+int cpmk_gemm_fp16_parts(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, int k_first, const void* A, const void* B,
+                         void* parts, void* stream) {
+    clear_stale_error();
+    if (!k_first) return gemm_sum_dispatch<true>(true, m, k, n, batch, groups, A, B, nullptr, parts, (hipStream_t)stream);
+    if (k < 0 || batch < 1 || groups < 1 || batch % groups) return CPMK_EBADARG;
+    return gemm_rows_parts(m, (int64_t)k * (batch / groups), n, groups, A, B, parts, (hipStream_t)stream);
+}
+
+int cpmk_gemm_add_parts(int32_t groups, int64_t n, const void* parts, void* out, void* stream) {
+    clear_stale_error();
+    if (groups < 1 || n < 0) return CPMK_EBADARG;
+    if (n == 0) return 0;
+    if (any_null(parts, out)) return CPMK_EBADARG;
+    if (n % 4 || !aligned16(parts) || (reinterpret_cast<uintptr_t>(out) & 7u)) return CPMK_EALIGN;
+    // enough lanes for the whole chip: with few columns, more sets of groups per workgroup
+    int rgs = 1;
+    while (rgs < 64 && n / 4 * rgs < 131072 && rgs * 2 <= groups) rgs *= 2;
+    const int64_t blocks = ceil_div(n, 256 / rgs * 4);
+    if (blocks >= 1 << 24) return CPMK_ETOOBIG;       // (a launch holds fewer than 2^32 threads)
+    hipLaunchKernelGGL(k_add_parts, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, groups, n, rgs, (const float*)parts, (half_t*)out);
+    return launch_status();
 }
 
 }  // extern "C"

@@ -41,6 +41,13 @@ constexpr int kEpiF16 = 2;       // fp16 product with fp32 accumulation, fp16 ou
 // travel through memory.  Both operands K-major.
 constexpr int kEpiSumI8 = 3;     // int8 products: fp32 sums of f32(acc) * s_row of each entry, fp16 out
 constexpr int kEpiSumF16 = 4;    // fp16 products: one fp32 accumulation over all entries, fp16 out
+// The same, and the fp16 product, with fp32 out: partial sums, which may pass fp16's range although the whole sum does not.
+constexpr int kEpiSumI8Part = 5, kEpiSumF16Part = 6, kEpiF16Part = 7;
+constexpr bool epi_part(int e) { return e == kEpiSumI8Part || e == kEpiSumF16Part || e == kEpiF16Part; }
+constexpr bool epi_fold(int e) { return e == kEpiSumI8 || e == kEpiSumI8Part; }
+constexpr bool epi_f16(int e) { return e == kEpiF16 || e == kEpiF16Part || e == kEpiSumF16 || e == kEpiSumF16Part; }
+constexpr bool epi_sum(int e) { return epi_fold(e) || e == kEpiSumF16 || e == kEpiSumF16Part; }
+constexpr bool epi_out32(int e) { return e == kEpiInt32 || epi_part(e); }      // four bytes per output
 
 struct DmaArgs {
     GemmArgs g;
@@ -343,9 +350,9 @@ __device__ __forceinline__ void tail_slabs(Dma& dma, int it, F&& slab) {
 // (RB = 128 bytes: eight lanes per 128-byte line).
 template <int EPI, int TC>
 struct StripOut {
-    static constexpr int ESZ = EPI == kEpiInt32 ? 4 : 2;
-    static constexpr int CT = EPI == kEpiInt32 ? 1 : TC;       // MFMA tile columns (of 32) side by side in one chunk
-    static constexpr int NCH = EPI == kEpiInt32 ? TC : 1;      // chunks per block of 32 rows
+    static constexpr int ESZ = epi_out32(EPI) ? 4 : 2;
+    static constexpr int CT = epi_out32(EPI) ? 1 : TC;       // MFMA tile columns (of 32) side by side in one chunk
+    static constexpr int NCH = epi_out32(EPI) ? TC : 1;      // chunks per block of 32 rows
     static constexpr int RB = CT * 32 * ESZ, PPR = RB / 16, RPW2 = 256 / RB, PASSES = PPR / 2, RPP = 64 / PPR;
     // 16-byte piece p of strip row r sits at piece slot p ^ ((r / RPW2) % PPR): reads are conflict free
     static __device__ __forceinline__ int slot(int r, int p) { return (p ^ ((r / RPW2) & (PPR - 1))) << 4; }
@@ -402,8 +409,8 @@ struct StripOut {
 template <int WR, int WC, int TR, int TC, int BKB, int EPI, int NST, int LAY = 0>
 __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, int8_t* stg, uint32_t lds_base,
                                               const GemmItem cur_item, const GemmItem nxt_item, const bool have_slabs, int& ring) {
-    constexpr bool FUSED = EPI == kEpiDequant, F16 = EPI == kEpiF16 || EPI == kEpiSumF16;
-    constexpr bool SUM = EPI == kEpiSumI8 || EPI == kEpiSumF16, FOLD = EPI == kEpiSumI8;
+    constexpr bool FUSED = EPI == kEpiDequant, F16 = epi_f16(EPI);
+    constexpr bool SUM = epi_sum(EPI), FOLD = epi_fold(EPI);
     static_assert(!SUM || (LAY & 3) == 0, "sums over the batch: K-major operands");
     constexpr bool PT = (LAY & 1) != 0, QT = (LAY & 2) != 0;
     static_assert((LAY & 3) == 0 || BKB == 128, "transposed operands: 128 bytes of K per slab");
@@ -700,10 +707,14 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int srow = h * 16 + r16;      // row of the strip
-                if constexpr (EPI == kEpiInt32) {
+                if constexpr (epi_out32(EPI)) {
 #pragma unroll
-                    for (int jj = 0; jj < 2; ++jj)
-                        *reinterpret_cast<int4_t*>(stg + srow * RB + slot(srow, jj * 4 + q)) = acc[2 * i + h][2 * c + jj];
+                    for (int jj = 0; jj < 2; ++jj) {
+                        int4_t v;
+                        if constexpr (FOLD) v = __builtin_bit_cast(int4_t, facc[2 * i + h][2 * c + jj]);
+                        else v = __builtin_bit_cast(int4_t, acc[2 * i + h][2 * c + jj]);
+                        *reinterpret_cast<int4_t*>(stg + srow * RB + slot(srow, jj * 4 + q)) = v;
+                    }
                 } else {
                     float sx = 0.0f;
                     if (FUSED) sx = (float)sxr[2 * i + h];
@@ -740,7 +751,8 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
 template <int WR, int WC, int TR, int TC, int BKB, int EPI, int NST, int LAY = 0>
 __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem, int8_t* stg, uint32_t lds_base,
                                               const GemmItem cur_item, const GemmItem nxt_item, const bool have_slabs, int& ring) {
-    constexpr bool FUSED = EPI == kEpiDequant, F16 = EPI == kEpiF16;
+    constexpr bool FUSED = EPI == kEpiDequant, F16 = epi_f16(EPI);
+    static_assert(!epi_sum(EPI), "sums over the batch: the 16x16 form");
     constexpr bool PT = (LAY & 1) != 0, QT = (LAY & 2) != 0;
     static_assert((LAY & 3) == 0 || BKB == 128, "transposed operands: 128 bytes of K per slab");
     constexpr int ESZ_IN = F16 ? 2 : 1;            // bytes per operand element
@@ -1020,11 +1032,15 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
         if (FUSED) sx = (float)sxr[i];
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            if constexpr (EPI == kEpiInt32) {
+            if constexpr (epi_out32(EPI)) {
 #pragma unroll
                 for (int g4 = 0; g4 < 4; ++g4) {
-                    const int4_t v = {(int32_t)acc[i][c][g4 * 4], (int32_t)acc[i][c][g4 * 4 + 1],
-                                      (int32_t)acc[i][c][g4 * 4 + 2], (int32_t)acc[i][c][g4 * 4 + 3]};
+                    int4_t v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const auto x = acc[i][c][g4 * 4 + e];       // (a value of its own: the cast of a vector's element takes the first one)
+                        v[e] = __builtin_bit_cast(int32_t, x);
+                    }
                     *reinterpret_cast<int4_t*>(stg + lrow * RB + slot(lrow, g4 * 2 + lk)) = v;
                 }
             } else {
@@ -1060,7 +1076,7 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
 // (the sums over the batch hold two sets of accumulators: two waves a SIMD, so that the folding of one passes under the
 // products of the other)
 template <int WR, int WC, int TR, int TC, int BKB, int EPI, bool HALVES, int NST, int LAY, int MF>
-__global__ __launch_bounds__(WR* WC * 64, EPI == kEpiSumI8 ? 2 : 1) void k_gemm_dma(DmaArgs da) {
+__global__ __launch_bounds__(WR* WC * 64, epi_fold(EPI) ? 2 : 1) void k_gemm_dma(DmaArgs da) {
     static_assert(!(HALVES && (LAY & 4) != 0), "half tiles only where the depth is whole slabs");
     static_assert(MF == 16 || MF == 32, "MFMA tile");
     constexpr int BR = WR * TR * 32, BC = WC * TC * 32;
@@ -1127,7 +1143,7 @@ static int launch_dma(GemmArgs& a, int batch, hipStream_t st, int per_cu = 1) {
     da.nhalf = 0;
     // (a half tile's slab must split evenly over the waves too, and rows of K of half a tile be whole 128-byte groups;
     // a tile moved inside the matrix has no half of its own)
-    constexpr bool F16 = EPI == kEpiF16 || EPI == kEpiSumF16;
+    constexpr bool F16 = epi_f16(EPI);
     if constexpr (TR % 2 == 0 && (LAY & 4) == 0 && ((BR / 2 + BC) / (1024 / BKB)) % (WR * WC) == 0 && (BR / 2) * (F16 ? 2 : 1) % 128 == 0) {
         if (r > 0 && 2 * r <= grid && (a.edge_in & 1) == 0) {
             da.nfull = (uint32_t)(total - r);

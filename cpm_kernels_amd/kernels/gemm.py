@@ -201,6 +201,34 @@ def gemm_fp16_sum(m: int, k: int, n: int, batch: int, groups: int,
     cpmk.gemm_fp16_sum(m, k, n, batch, groups, A, B, out, stream)
 
 
+def gemm_int8_scale_parts(m: int, k: int, n: int, batch: int, groups: int,
+                          A: DevicePointer, B: DevicePointer, scale_row: DevicePointer,    # as in gemm_int8_scale_sum
+                          parts: DevicePointer,       # (groups, n, m)    fp32
+                          stream: CUDAStream):
+    """gemm_int8_scale_sum with the groups' sums as fp32, for gemm_add_parts."""
+    assert m % 4 == 0 and n % 4 == 0 and k % 128 == 0
+    cpmk.gemm_int8_scale_parts(m, k, n, batch, groups, A, B, scale_row, parts, stream)
+
+
+def gemm_fp16_parts(m: int, k: int, n: int, batch: int, groups: int, k_first: bool,
+                    A: DevicePointer,         # (batch, m, k)     fp16   [(batch, k, m) if k_first]
+                    B: DevicePointer,         # (batch, n, k)     fp16   [(batch, k, n) if k_first]
+                    parts: DevicePointer,     # (groups, n, m)    fp32
+                    stream: CUDAStream):
+    """gemm_fp16_sum with the groups' sums as fp32, for gemm_add_parts."""
+    assert m % 2 == 0 and n % 2 == 0 and k % 2 == 0
+    cpmk.gemm_fp16_parts(m, k, n, batch, groups, 1 if k_first else 0, A, B, parts, stream)
+
+
+def gemm_add_parts(groups: int, n: int,
+                   parts: DevicePointer,      # (groups, n)       fp32
+                   out: DevicePointer,        # (n)               fp16
+                   stream: CUDAStream):
+    """out = sum of the parts, rounded once."""
+    assert n % 4 == 0
+    cpmk.gemm_add_parts(groups, n, parts, out, stream)
+
+
 def gemm_fp16(m: int, k: int, n: int,
               batchA: int, batchB: int,
               aT: bool, bT: bool,

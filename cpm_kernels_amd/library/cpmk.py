@@ -16,6 +16,7 @@ _LAUNCHERS = (
     "gemm_scale_x", "gemm_scale_y", "gemm_int8", "gemm_int8_scale", "gemm_quantize", "gemm_quantize_pair",
     "gemm_quantize_cols", "gemm_fp16", "gemm_quantize_cols_ld", "gemm_quantize_pair_ld",
     "gemm_backward_round_scale_ld", "gemm_int8_scale_one", "transpose_i8_ld", "gemm_int8_scale_sum", "gemm_fp16_sum",
+    "gemm_int8_scale_parts", "gemm_fp16_parts", "gemm_add_parts",
     "gemv_fp16", "gemv_fp16_transpose", "gemv_broadcast_mat_fp16", "embedding_forward", "embedding_step",
     "copy_data_to_kv", "gemv_calc_scale", "gemv_round", "gemv_broadcast_mat_int8", "layernorm_forward",
     "layernorm_forward_noalloc", "layernorm_step", "layernorm_affine_forward", "layernorm_affine_forward_stats",

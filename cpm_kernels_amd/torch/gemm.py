@@ -10,6 +10,7 @@ import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
     gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups, gemm_int8_scale_sum, gemm_fp16_sum, \
+    gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, \
     arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
     transpose_i8, transpose_i8_ld
 from ._common import cur_stream
@@ -128,6 +129,13 @@ def _sum_entries(parts: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _add_parts(parts: torch.Tensor) -> torch.Tensor:
+    """(groups, r, c) fp32 sums -> (1, r, c) fp16"""
+    out = torch.empty((1,) + parts.shape[1:], dtype=torch.half, device=parts.device)
+    gemm_add_parts(parts.size(0), out.numel(), parts.data_ptr(), out.data_ptr(), cur_stream())
+    return out
+
+
 def gemm_and_scale_sum(quantA, scaleA, quantB) -> torch.Tensor:
     """(1, M, N): the sum over the batch of scaleA * (quantA x quantB^T), quantA (b, M, K) and quantB (b, N, K)."""
     batch, M, K = quantA.size()
@@ -135,10 +143,10 @@ def gemm_and_scale_sum(quantA, scaleA, quantB) -> torch.Tensor:
     groups = gemm_sum_groups(N, M, batch)
     if groups == batch or quantB.size(0) != batch or K == 0 or K % 128 != 0 or max(M, N) * K >= 2 ** 31 or batch * K >= 2 ** 22:
         return _sum_entries(gemm_and_scale(quantA, scaleA, quantB, None, False, True))
-    parts = torch.empty((groups, M, N), dtype=torch.half, device=quantA.device)
-    gemm_int8_scale_sum(N, quantA.size(2), M, batch, groups, quantB.data_ptr(), quantA.data_ptr(), scaleA.data_ptr(),
-                        parts.data_ptr(), cur_stream())
-    return _sum_entries(parts)
+    parts = torch.empty((groups, M, N), dtype=torch.half if groups == 1 else torch.float32, device=quantA.device)
+    launch = gemm_int8_scale_sum if groups == 1 else gemm_int8_scale_parts
+    launch(N, K, M, batch, groups, quantB.data_ptr(), quantA.data_ptr(), scaleA.data_ptr(), parts.data_ptr(), cur_stream())
+    return parts if groups == 1 else _add_parts(parts)
 
 
 class GEMMInt8(torch.autograd.Function):
@@ -299,17 +307,26 @@ def gemm_pth_fp16_sum(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> t
     """The same product summed over the batch, (1, M, N)."""
     M, K, N = _dims(A, B, aT, bT)
     batch = A.size(0)
-    if batch == B.size(0) and batch > 1:
-        groups = gemm_sum_groups(N, M, batch)
-        per = batch // groups
-        if groups < batch and aT and not bT:
-            # both operands stored (K, rows): the entries of a group are one longer contraction as they lie
-            return _sum_entries(gemm_pth_fp16(A.view(groups, per * K, M), True, B.view(groups, per * K, N), False))
-        if groups < batch and not aT and bT and M % 4 == 0 and N % 4 == 0 and K > 32 and max(M, N) * K < 2 ** 31 and \
-                batch * K < 2 ** 21 and (A.data_ptr() | B.data_ptr()) % 4 == 0:
-            parts = torch.empty((groups, M, N), dtype=torch.half, device=A.device)
-            gemm_fp16_sum(N, K, M, batch, groups, B.data_ptr(), A.data_ptr(), parts.data_ptr(), cur_stream())
-            return _sum_entries(parts)
+    groups = gemm_sum_groups(N, M, batch) if batch == B.size(0) else batch
+    if groups < batch and aT and not bT:
+        # both operands stored (K, rows): the entries of a group are one longer contraction as they lie
+        depth = batch // groups * K
+        if groups == 1:
+            return gemm_pth_fp16(A.view(1, depth, M), True, B.view(1, depth, N), False)
+        if (M % 8 == 0 or M >= 128) and (N % 8 == 0 or N >= 256) and depth >= 64 and max(M, N) * depth < 2 ** 31 and \
+                (A.data_ptr() | B.data_ptr()) % 16 == 0:
+            parts = torch.empty((groups, M, N), dtype=torch.float32, device=A.device)
+            gemm_fp16_parts(N, K, M, batch, groups, True, B.data_ptr(), A.data_ptr(), parts.data_ptr(), cur_stream())
+            return _add_parts(parts)
+    elif groups < batch and not aT and bT and M % 4 == 0 and N % 4 == 0 and K > 32 and max(M, N) * K < 2 ** 31 and \
+            batch * K < 2 ** 21 and (A.data_ptr() | B.data_ptr()) % 4 == 0:
+        if groups == 1:
+            out = torch.empty((1, M, N), dtype=torch.half, device=A.device)
+            gemm_fp16_sum(N, K, M, batch, 1, B.data_ptr(), A.data_ptr(), out.data_ptr(), cur_stream())
+            return out
+        parts = torch.empty((groups, M, N), dtype=torch.float32, device=A.device)
+        gemm_fp16_parts(N, K, M, batch, groups, False, B.data_ptr(), A.data_ptr(), parts.data_ptr(), cur_stream())
+        return _add_parts(parts)
     return _sum_entries(gemm_pth_fp16(A, aT, B, bT))
 
 

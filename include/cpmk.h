@@ -197,6 +197,15 @@ int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int
                              const void* scale_row, void* out, void* stream);
 int cpmk_gemm_fp16_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                        void* out, void* stream);
+/* The same with the groups' sums as fp32, parts (groups, n, m): a group's sum may pass fp16's range where the whole sum does not.
+ * fp16 with k_first: operands stored A (batch, k, m) and B (batch, k, n), m, n and k even, any number of entries a group; k of a group's
+ * entries together at least 64, m a multiple of 8 or at least 256, n a multiple of 8 or at least 128, buffers on 16-byte boundaries.
+ * cpmk_gemm_add_parts: out[j] = fp16(sum over g of parts[g, j]), in the order of the groups; n a multiple of 4. */
+int cpmk_gemm_int8_scale_parts(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
+                               const void* scale_row, void* parts, void* stream);
+int cpmk_gemm_fp16_parts(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, int k_first, const void* A, const void* B,
+                         void* parts, void* stream);
+int cpmk_gemm_add_parts(int32_t groups, int64_t n, const void* parts, void* out, void* stream);
 /* out[b,o] = sum_k mat[b,o,k] vec[b,k]      kernels/gemv.py:82-149 / cuda/gemv.cu:78-107 */
 int cpmk_gemv_fp16(int32_t batch, int32_t dim_out, int32_t dim_in, const void* mat,
                    const void* vec, void* out, void* stream);

@@ -63,3 +63,81 @@ def test_groups(gpu):
     for m, n, batch in ((4, 4, 1), (512, 512, 8), (4096, 10240, 8), (4096, 4096, 13), (64, 64, 7), (8192, 8192, 64)):
         groups = ck.gemm_sum_groups(m, n, batch)
         assert 1 <= groups <= batch and batch % groups == 0 and (groups == batch or batch // groups <= 16)
+
+
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s[1] > 1])
+def test_int8_parts(gpu, shape):
+    batch, groups, n, m, k = shape
+    print("int8 parts", shape, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n * 7 + m + k)
+    A = torch.randint(-128, 128, (batch, m, k), generator=g, device="cuda", dtype=torch.int8)
+    B = torch.randint(-128, 128, (batch, n, k), generator=g, device="cuda", dtype=torch.int8)
+    s = (torch.rand((batch, n), generator=g, device="cuda") * 1e-1 + 1e-2).half()        # (sums beyond fp16's range among them)
+    parts = torch.full((groups, n, m), float("nan"), device="cuda")
+    ck.gemm_int8_scale_parts(m, k, n, batch, groups, A.data_ptr(), B.data_ptr(), s.data_ptr(), parts.data_ptr(), _st())
+    acc = torch.stack([(B[e].double() @ A[e].double().t()) * s[e].double()[:, None] for e in range(batch)]).view(groups, -1, n, m)
+    bound = acc.abs().sum(1) * (batch + 1) * 2.0 ** -24        # a rounding per entry and one of a 24-bit integer's conversion
+    assert bool(((parts.double() - acc.sum(1)).abs() <= bound).all()), shape
+    _check_add(parts)
+
+
+@pytest.mark.parametrize("k_first,k", [(False, k) for k in (34, 64, 66, 72, 128, 500)] + [(True, k) for k in (32, 34, 64, 128, 250, 500)])
+@pytest.mark.parametrize("shape", [(4, 2, 132, 260), (6, 3, 260, 132), (4, 2, 40, 520), (6, 2, 2564, 2564), (40, 2, 130, 262), (4, 2, 128, 256)])
+def test_fp16_parts(gpu, shape, k_first, k):
+    batch, groups, n, m = shape
+    if not k_first and (n % 4 or m % 4 or batch // groups > 16):
+        n, m, batch = n // 4 * 4, m // 4 * 4, groups * 8
+    if k_first and m == 132:
+        m = 136                  # (rows of 8j + 4 elements: from 256 on)
+    print("fp16 parts", batch, groups, n, m, k_first, k, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n * 7 + m + k)
+    A = torch.randn((batch, k, m) if k_first else (batch, m, k), generator=g, device="cuda").mul_(8).half()
+    B = torch.randn((batch, k, n) if k_first else (batch, n, k), generator=g, device="cuda").mul_(8).half()
+    parts = torch.full((groups, n, m), float("nan"), device="cuda")
+    ck.gemm_fp16_parts(m, k, n, batch, groups, k_first, A.data_ptr(), B.data_ptr(), parts.data_ptr(), _st())
+    p, q = (B.transpose(1, 2), A) if k_first else (B, A.transpose(1, 2))
+    p, q, per = p.double().contiguous(), q.double().contiguous(), batch // groups
+    for i in range(groups):
+        want = sum(p[e] @ q[e] for e in range(i * per, (i + 1) * per))
+        mag = sum(p[e].abs() @ q[e].abs() for e in range(i * per, (i + 1) * per))
+        assert bool(((parts[i].double() - want).abs() <= mag * (per * k) * 2.0 ** -24).all()), (i, k)      # fp32 sums in any order
+    if n * m % 4 == 0:
+        _check_add(parts)
+
+
+def _check_add(parts):
+    groups, total = parts.size(0), parts[0].numel()
+    out = torch.full(parts.shape[1:], float("nan"), device="cuda", dtype=torch.half)
+    ck.gemm_add_parts(groups, total, parts.data_ptr(), out.data_ptr(), _st())
+    want, mag = parts.double().sum(0), parts.double().abs().sum(0)
+    bound = mag * groups * 2.0 ** -24 + want.abs() * 2.0 ** -11 + 2.0 ** -25
+    big = want.abs() > 65504
+    assert bool(((out.double() - want).abs() <= bound)[~big].all()) and bool((out[want.abs() > 65536].isinf()).all())
+
+
+@pytest.mark.parametrize("groups,n", [(1, 4), (2, 4), (3, 1020), (7, 132), (64, 256), (200, 1028), (2, 1 << 21)])
+def test_add_parts(gpu, groups, n):
+    print("add parts", groups, n, flush=True)
+    _check_add(torch.randn((groups, n), generator=torch.Generator(device="cuda").manual_seed(n + groups), device="cuda"))
+
+
+@pytest.mark.parametrize("rows", [True, False])
+@pytest.mark.parametrize("int8", [True, False])
+def test_sums_that_pass_fp16_range_between_groups(gpu, int8, rows):
+    """Entries that are finite each and cancel over the whole batch, while the sum of a group of them passes 65504."""
+    import cpm_kernels_amd.torch as ct
+    batch, tokens, size = 16, 128, 640
+    groups = ck.gemm_sum_groups(size, size, batch)
+    assert 1 < groups < batch
+    print("range between groups", int8, rows, groups, flush=True)
+    x = torch.full((batch, tokens, size) if rows else (batch, size, tokens), 16.0, device="cuda", dtype=torch.half)
+    w = torch.full((1, size, size), 0.001, device="cuda", dtype=torch.half, requires_grad=True)
+    out = ct.bmm(x, False, w, True, int8=int8) if rows else ct.bmm(w, False, x, False, int8=int8)
+    grad = torch.full_like(out, 20.0)                 # 128 products of 16 x 20: 40960 an entry
+    per = batch // groups
+    for e in range(batch):
+        if e // per % 2:
+            grad[e] = -20.0
+    got, = torch.autograd.grad(out, [w], grad)
+    # equal entries of either sign cancel exactly, whatever their rounding, unless a partial sum was lost
+    assert bool((got == 0).all()), got.flatten()[:4]

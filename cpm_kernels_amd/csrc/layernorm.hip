@@ -550,7 +550,7 @@ int cpmk_layernorm_affine_forward(int32_t batch, int32_t n, int32_t m, const voi
 int cpmk_layernorm_affine_forward_stats(int32_t batch, int32_t n, int32_t m, const void* mat, const void* alpha,
                                         const void* beta, void* out, void* stats, float eps, int rd_mean, void* stream) {
     clear_stale_error();
-    if (alpha == nullptr || stats == nullptr) return CPMK_EBADARG;
+    if (alpha == nullptr || (stats == nullptr && (int64_t)batch * n * m > 0)) return CPMK_EBADARG;       // (an empty problem has no statistics)
     return layernorm_dispatch(batch, n, m, mat, out, alpha, beta, eps, rd_mean, (hipStream_t)stream, nullptr, 0, (float*)stats);
 }
 

@@ -211,6 +211,15 @@ def test_empty_problems_of_the_padded_quantisers_without_a_gpu():
             call()
 
 
+def test_empty_layernorm_with_statistics_without_a_gpu():
+    from cpm_kernels_amd.library import cpmk
+    cpmk.layernorm_affine_forward_stats(2, 4, 0, None, 8, 8, None, None, 1e-5, 1, None)        # no tokens: no statistics either
+    cpmk.layernorm_affine_forward_stats(0, 4, 8, None, 8, None, None, None, 1e-5, 0, None)
+    cpmk.layernorm_affine_backward(2, 4, 0, None, None, 8, None, None, 8, 8, None, None)
+    with pytest.raises(RuntimeError, match="invalid argument"):
+        cpmk.layernorm_affine_forward_stats(2, 4, 8, 8, 8, 8, 8, None, 1e-5, 1, None)
+
+
 def test_launchers_take_ctypes_numbers_of_the_parameters_type():
     """As ctypes function prototypes do: c_int32 for an int32_t parameter (not another width), c_float for a float one, and any
     object with an index."""

@@ -52,3 +52,16 @@ def test_layernorm_backward(gpu, shape, mean):
                  rows * (gd.abs() * (xh.abs() + mu.abs() * rstd)).sum((0, 2))).all())
     if mean:
         assert bool(((db.double() - gd.sum((0, 2))).abs() <= gd.sum((0, 2)).abs() * 2.0 ** -11 + 2.0 ** -24 + rows * gd.abs().sum((0, 2))).all())
+
+
+@pytest.mark.parametrize("shape", [(2, 64, 0), (0, 64, 8)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_layernorm_of_no_tokens(gpu, shape, bias):
+    import cpm_kernels_amd.torch as ct
+    print("empty layernorm", shape, bias, flush=True)
+    ln = ct.LayerNorm(shape[1], bias=bias).half().cuda()
+    x = torch.empty(shape, device="cuda", dtype=torch.half, requires_grad=True)
+    out = ln(x)
+    assert out.shape == x.shape
+    grads = torch.autograd.grad(out, [x, ln.weight] + ([ln.bias] if bias else []), torch.empty_like(out))
+    assert grads[0].shape == x.shape and all(bool((g == 0).all()) for g in grads[1:])

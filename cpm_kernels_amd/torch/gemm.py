@@ -303,18 +303,26 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
     return out
 
 
+def _entry_groups(M: int, K: int, N: int, batch: int, joined: bool) -> int:
+    """Groups that an fp16 product summed over the batch is formed in.  `joined`: a group's entries become one contraction, which
+    the tile kernel takes up to operands of 4 GiB; beyond that there are more groups, down to the entries one by one."""
+    groups = gemm_sum_groups(N, M, batch)
+    while joined and groups < batch and max(M, N) * K * (batch // groups) >= 2 ** 31:
+        groups = next(g for g in range(groups + 1, batch + 1) if batch % g == 0)
+    return groups
+
+
 def gemm_pth_fp16_sum(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch.Tensor:
     """The same product summed over the batch, (1, M, N)."""
     M, K, N = _dims(A, B, aT, bT)
     batch = A.size(0)
-    groups = gemm_sum_groups(N, M, batch) if batch == B.size(0) else batch
+    groups = _entry_groups(M, K, N, batch, aT and not bT) if batch == B.size(0) else batch
     if groups < batch and aT and not bT:
         # both operands stored (K, rows): the entries of a group are one longer contraction as they lie
         depth = batch // groups * K
         if groups == 1:
             return gemm_pth_fp16(A.view(1, depth, M), True, B.view(1, depth, N), False)
-        if (M % 8 == 0 or M >= 128) and (N % 8 == 0 or N >= 256) and depth >= 64 and max(M, N) * depth < 2 ** 31 and \
-                (A.data_ptr() | B.data_ptr()) % 16 == 0:
+        if (M % 8 == 0 or M >= 128) and (N % 8 == 0 or N >= 256) and depth >= 64 and (A.data_ptr() | B.data_ptr()) % 16 == 0:
             parts = torch.empty((groups, M, N), dtype=torch.float32, device=A.device)
             gemm_fp16_parts(N, K, M, batch, groups, True, B.data_ptr(), A.data_ptr(), parts.data_ptr(), cur_stream())
             return _add_parts(parts)

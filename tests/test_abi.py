@@ -220,6 +220,18 @@ def test_empty_layernorm_with_statistics_without_a_gpu():
         cpmk.layernorm_affine_forward_stats(2, 4, 8, 8, 8, 8, 8, None, 1e-5, 1, None)
 
 
+def test_joined_entries_stay_within_the_tile_kernels_operands():
+    """Entries of a batch sum that become one contraction: operands below 4 GiB, which the general product kernel would take over from."""
+    from cpm_kernels_amd.torch.gemm import _entry_groups
+    for M, K, N, batch in ((8192, 32768, 8192, 8), (150000, 1024, 4096, 16), (8192, 32768, 512, 8), (4096, 512, 4096, 8), (64, 4, 64, 7),
+                           (8192, 2 ** 18, 8192, 6), (4096, 0, 4096, 4), (8192, 32768, 8192, 9)):
+        groups = _entry_groups(M, K, N, batch, True)
+        assert 1 <= groups <= batch and batch % groups == 0
+        assert groups == batch or 2 * max(M, N) * K * (batch // groups) < 2 ** 32
+        assert _entry_groups(M, K, N, batch, False) <= groups
+    assert _entry_groups(8192, 32768, 8192, 8, True) == 2       # (no more groups than it takes)
+
+
 def test_launchers_take_ctypes_numbers_of_the_parameters_type():
     """As ctypes function prototypes do: c_int32 for an int32_t parameter (not another width), c_float for a float one, and any
     object with an index."""

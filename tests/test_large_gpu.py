@@ -322,3 +322,25 @@ def test_batch_sum_beyond_2_32_columns(gpu):
     for a, b in spans:
         assert torch.equal(out[a:b], x[0, a:b] + x[1, a:b]), (a, b)       # (whole numbers below 2048)
     assert int((out == 77.0).sum()) == 0, "elements left unwritten"
+
+
+def test_weight_gradient_over_more_than_4_gib_of_tokens(gpu):
+    """fp16 training at long sequences: the entries of the batch together pass 2^31 elements."""
+    import cpm_kernels_amd.torch as ct
+    batch, tokens, din, dout = 8, 32768, 8192, 256
+    _name("weight gradient", batch, tokens, din, dout)
+    x = _randn_half((batch, tokens, din), 3, gpu)
+    w = torch.zeros((1, dout, din), dtype=torch.half, device=gpu, requires_grad=True)
+    out = ct.bmm(x, False, w, True, int8=False)
+    g = _randn_half(tuple(out.shape), 4, gpu, 0.01)
+    got, = torch.autograd.grad(out, [w], g)
+    for cols in (slice(0, 16), slice(din - 16, din)):
+        want = torch.zeros((dout, 16), device=gpu, dtype=torch.float64)
+        mag = torch.zeros_like(want)
+        for b in range(batch):
+            gb, xb = g[b].double().t().contiguous(), x[b, :, cols].double()
+            want += gb @ xb
+            mag += gb.abs() @ xb.abs()
+        # fp32 sums in chains of 16-deep products, one rounding to fp16
+        bound = mag * (batch * tokens) * 2.0 ** -24 + want.abs() * 2.0 ** -11
+        assert bool(((got[0, :, cols].double() - want).abs() <= bound).all()), cols

@@ -137,6 +137,7 @@ struct SlabDma {
     int nk;                     // slabs per tile
     int nkb;                    // ... and per batch entry
     int rem;                    // REST: bytes of K in slab 0, or 0: whole slabs only
+    int first;                  // slabs from the bases to the operands' starts
     int32_t oj0, oi0;           // first row / column of the tile
     bool ahead;                 // the next tile is fetched ahead (only if its LDS layout is this one's)
     bool deep;                  // at least as many slabs as stages
@@ -172,8 +173,7 @@ struct SlabDma {
         return (uint32_t)grow * (uint32_t)a.k + c * 16;
     }
 
-    // REST: the same for slab 0, relative to the end of the whole slabs; 16 bytes further on for a K-major operand (kofs takes
-    // them off again), whose last 16 bytes of K may begin before that
+    // REST: the same for slab 0, counted from the operand's start (operands are below 4 GiB)
     __device__ __forceinline__ uint32_t rest_voff(int d, int32_t oj, int32_t oi) const {
         const int dd = wave + d * NW;
         const bool q = dd * RPI >= BR;
@@ -181,23 +181,12 @@ struct SlabDma {
             const int ppr = (q ? BC : BR) / EPP;
             const int kr = (q ? dd - BR / RPI : dd) * (64 / ppr) + lane / ppr;
             const int32_t L = q ? a.m : a.n;
-            return calc_voff(d, oj, oi) - (uint32_t)(kr - min(kr, rem / ESZ_IN - 1)) * (uint32_t)L * (uint32_t)ESZ_IN;
+            return calc_voff(d, oj, oi) + (uint32_t)((nk - 1) * (BKB / ESZ_IN) + min(kr, rem / ESZ_IN - 1) - kr) * (uint32_t)L * (uint32_t)ESZ_IN;
         }
         const int r = dd * RPI + lane / CPR;
         const int c = (lane % CPR) ^ swz(r);
         const int32_t grow = q ? min(oi + (r - BR), a.m - 1) : min(oj + r, a.n - 1);
-        return (uint32_t)grow * (uint32_t)a.k + (uint32_t)(16 + min(c * 16, rem - 16));
-    }
-    // bytes from an operand's start to slab kt
-    __device__ __forceinline__ int64_t kofs(bool q, int kt) const {
-        const int64_t kstep = q ? kstepQ : kstepP;
-        if constexpr (REST) {
-            if (rem != 0) {
-                const bool kmajor = q ? !QT : !PT;
-                return (kt == 0 ? nk - 1 : kt - 1) * kstep - (kt == 0 && kmajor ? 16 : 0);
-            }
-        }
-        return kt * kstep;
+        return (uint32_t)grow * (uint32_t)a.k + (uint32_t)((nk - 1) * BKB + min(c * 16, rem - 16));
     }
 
     __device__ __forceinline__ SlabDma(const GemmArgs& a_, uint32_t lds_base, const GemmItem& cur_item, const GemmItem& nxt_item,
@@ -232,6 +221,17 @@ struct SlabDma {
         }
         kstepP = PT ? (int64_t)BKB * a.n : BKB;
         kstepQ = QT ? (int64_t)BKB * a.m : BKB;
+        // With the rest of the depth as slab 0 slab kt >= 1 is whole slab kt - 1.  The bases move, so that the K loop finds it at kt slabs
+        // all the same: chosen there, slab by slab, the offset cost a fifth of the loop (512 x 140 products of depth 9616 77 -> 92 us).
+        // Slab 0 is at `first` slabs, with the offsets of rest_voff.
+        first = 0;
+        if constexpr (REST) {
+            if (rem != 0) {
+                first = 1;
+                Pb -= kstepP; Pn -= kstepP;
+                Qb -= kstepQ; Qn -= kstepQ;
+            }
+        }
     }
 
     // One DMA instruction of slab kt into ring stage `stage`: of this tile's rows, or (TAIL) of the rows the last LD
@@ -248,7 +248,7 @@ struct SlabDma {
             const uint32_t e = nkb == 1 ? (uint32_t)kt : __umulhi((uint32_t)kt, a.kmagic);       // kt / nkb (exact for kt * nkb < 2^32)
             lds_dma16(v, (q ? qb : pb) + (int64_t)e * (q ? a.strideQ : a.strideP) + (kt - (int)e * nkb) * BKB, ldst[d] + stage * STAGE);
         } else {
-            lds_dma16(v, (q ? qb : pb) + kofs(q, kt), ldst[d] + stage * STAGE);
+            lds_dma16(v, (q ? qb : pb) + kt * (q ? kstepQ : kstepP), ldst[d] + stage * STAGE);
         }
     }
 
@@ -307,7 +307,7 @@ struct SlabDma {
                     constexpr int d = decltype(dc)::value;
                     if constexpr (REST && st == 0) {
                         if (rem != 0) {
-                            lds_dma16(rest_voff(d, oj0, oi0), (isq[d] ? Qb : Pb) + kofs(isq[d], 0), ldst[d] + ring0 * STAGE);
+                            lds_dma16(rest_voff(d, oj0, oi0), (isq[d] ? Qb + kstepQ : Pb + kstepP), ldst[d] + ring0 * STAGE);
                             return;
                         }
                     }
@@ -646,7 +646,7 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
         wait_vmcnt<(NST - 2) * CNT>();       // slab it + 1 has landed (with fewer slabs than stages it had before the loop)
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
-        const int kt2 = TAIL ? it * tmul + tadd : it + LD;
+        const int kt2 = TAIL ? (REST ? max(it * tmul + tadd, dma.first) : it * tmul + tadd) : it + LD;
         const int tgt = cur + LD >= NST ? cur + LD - NST : cur + LD;       // the stage slab it + LD belongs to
         pass(I1{}, nxt, 0, std::true_type{}, nxt, 0,
              [&](auto dc) __attribute__((always_inline)) { dma1(dc, kt2, tailc, tgt); },
@@ -988,7 +988,7 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
         wait_vmcnt<(NST - 2) * CNT>();       // slab it + 1 has landed (with fewer slabs than stages it had before the loop)
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
-        const int kt2 = TAIL ? it * tmul + tadd : it + LD;
+        const int kt2 = TAIL ? (REST ? max(it * tmul + tadd, dma.first) : it * tmul + tadd) : it + LD;
         const int tgt = cur + LD >= NST ? cur + LD - NST : cur + LD;       // the stage slab it + LD belongs to
         kstep(std::integral_constant<int, ((KS - 1) & 1)>{},
               [&](auto xc) __attribute__((always_inline)) {

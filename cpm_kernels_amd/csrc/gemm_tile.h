@@ -145,6 +145,8 @@ struct SlabDma {
     int ring0;                  // stage of this tile's slab 0
     int32_t tj0, ti0;           // rows / columns the tail fetches
     const int8_t *Pb, *Qb, *Pn, *Qn;
+    const int8_t *Pk, *Qk;      // SUM: the slab requested next,
+    int left, step;             // ... slabs up to its entry's end and bytes to the next
     uint32_t voff[CNT], ldst[CNT];
     bool isq[CNT];
     int64_t kstepP, kstepQ;     // bytes from one K slab to the next
@@ -245,11 +247,33 @@ struct SlabDma {
         const uint32_t v = voff[d];            // (rewritten for the tail between the two loops: retarget)
         const bool q = isq[d];
         if constexpr (SUM) {
-            const uint32_t e = nkb == 1 ? (uint32_t)kt : __umulhi((uint32_t)kt, a.kmagic);       // kt / nkb (exact for kt * nkb < 2^32)
-            lds_dma16(v, (q ? qb : pb) + (int64_t)e * (q ? a.strideQ : a.strideP) + (kt - (int)e * nkb) * BKB, ldst[d] + stage * STAGE);
+            lds_dma16(v, q ? Qk : Pk, ldst[d] + stage * STAGE);
         } else {
             lds_dma16(v, (q ? qb : pb) + kt * (q ? kstepQ : kstepP), ldst[d] + stage * STAGE);
         }
+    }
+
+    // SUM: the slab that issue() requests next, followed through the entries by one addition a slab: divided and multiplied out
+    // request by request it held the K loop up (fp16, 1024 x 4096 outputs
+    // over 8 x 1024: 108 -> 95 us; int8 43 -> 36 with its sum in 128x128 tiles, 8192 x 1024 over 7 x 1024 68 -> 62 us).
+    // `tail`: of the next tile, or (not ahead) this tile's last slab again and again.
+    __device__ __forceinline__ void seek(bool tail, int kt) {
+        const uint32_t e = nkb == 1 ? (uint32_t)kt : __umulhi((uint32_t)kt, a.kmagic);       // kt / nkb (exact for kt * nkb < 2^32)
+        left = nkb - (kt - (int)e * nkb);
+        const int32_t in_entry = (nkb - left) * BKB;
+        Pk = (tail ? Pn : Pb) + ((int64_t)e * a.strideP + in_entry);
+        Qk = (tail ? Qn : Qb) + ((int64_t)e * a.strideQ + in_entry);
+        step = BKB;
+        if (tail && !ahead) {
+            step = 0;
+            left = 0;
+        }
+    }
+    __device__ __forceinline__ void advance() {
+        const bool wrap = --left == 0;
+        Pk += step + (wrap ? a.strideP - nkb * BKB : 0);
+        Qk += step + (wrap ? a.strideQ - nkb * BKB : 0);
+        left = wrap ? nkb : left;
     }
 
     // between a tile's main iterations and its tail: the offsets of the rows the tail fetches
@@ -298,7 +322,7 @@ struct SlabDma {
 
     // A tile's start.  Without slabs on their way: request the first NST, wait for slab 0.  Otherwise the first LD
     // slabs were requested during the previous tile; its stores drain too.
-    __device__ __forceinline__ void prime(bool have_slabs) const {
+    __device__ __forceinline__ void prime(bool have_slabs) {
         if (!have_slabs) {
             __syncthreads();                 // every wave is done with the ring of the previous tile
             static_for<0, NST>([&](auto sc) __attribute__((always_inline)) {
@@ -311,6 +335,7 @@ struct SlabDma {
                             return;
                         }
                     }
+                    if constexpr (SUM && d == 0) seek(false, min(st, nk - 1));
                     issue<d, false>(min(st, nk - 1), (ring0 + st) % NST);
                 });
             });
@@ -651,10 +676,12 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
         pass(I1{}, nxt, 0, std::true_type{}, nxt, 0,
              [&](auto dc) __attribute__((always_inline)) { dma1(dc, kt2, tailc, tgt); },
              std::integral_constant<int, CNT>{});
+        if constexpr (SUM) dma.advance();
         __builtin_amdgcn_sched_barrier(0);
         cur = nxt;
     };
     int it = 0;
+    if constexpr (SUM) dma.seek(false, min(LD, nk - 1));
     if constexpr (FOLD) {
         int in_entry = 0, entry = 0;
         auto fold = [&]() __attribute__((always_inline)) {       // the entry's product is complete: into the sums
@@ -676,9 +703,11 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
         };
         for (; it < nk - LD; ++it) { slab(it, std::false_type{}); fold(); }
         dma.retarget();
+        dma.seek(true, ahead ? 0 : nk - 1);
         for (; it < nk; ++it) { slab(it, std::true_type{}); fold(); }
     } else {
         for (; it < nk - LD; ++it) slab(it, std::false_type{});       // slabs LD .. nk-1 of this tile follow
+        if constexpr (SUM) dma.seek(true, ahead ? 0 : nk - 1);
         tail_slabs<REST>(dma, it, slab);                              // then the tail's
     }
     if (!ahead) wait_vmcnt<0>();         // drain the clamped loads before the ring is reused

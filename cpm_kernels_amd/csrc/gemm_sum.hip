@@ -18,6 +18,35 @@ static int32_t sum_groups(int32_t m, int32_t n, int32_t batch) {
     return batch;
 }
 
+// Groups for products of depth k an entry, or `batch` where the products one by one and their sum are the quicker: a product in large
+// tiles makes up for writing and adding its output where the sum over the batch has too few outputs for such tiles and
+// multiplies in small ones.  The sums / entries in us on either side of each line (outputs x batch x k):
+//   int8       one group   8192 x 1024 x 7: k = 2048 111 / 132, 4096 247 / 242; 4096 x 4096 x 8: 3072 359 / 422, 4096 578 / 517
+//              several     1536 x 1536 x 12: 896 49 / 50, 1536 67 / 62
+//   fp16, large tiles      4096 x 4096 x 2: k = 34 ... 4096 all quicker; 4096 x 4096 x 8: 4096 806 / 902
+//   fp16 K-major, one      2560 x 2560 x 5: 384 50 / 50, 448 54 / 48;  k of whole 16-byte pieces 328 52 / 53, 392 62 / 58;  others 66 38 / 42, 140 51 / 45
+//              several     1536 x 1536 x 12: 256 38 / 41, 384 53 / 44;  pieces 72 30 / 38, 136 41 / 40;  others 66 57 / 42
+//   fp16 (K, rows), one    2560 x 2560 x 5: 576 55 / 56, 768 73 / 67
+//              several     1536 x 1536 x 12: 256 36 / 41, 384 47 / 46
+enum SumKind { kSumI8 = 0, kSumF16 = 1, kSumF16KFirst = 2 };
+static int32_t sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t batch) {
+    int32_t g = sum_groups(m, n, batch);
+    // (K, rows): a group's entries become one contraction, which the tile kernel takes up to operands of 4 GiB
+    if (kind == kSumF16KFirst)
+        while (g < batch && (int64_t)(m > n ? m : n) * k >= (1ll << 31) / (batch / g))
+            do ++g; while (batch % g != 0);
+    if (g == batch) return batch;
+    const bool one = g == 1, large = ceil_div(n, 256) * ceil_div(m, 256) * g * 4 >= (int64_t)compute_units() * 3;
+    int32_t limit;
+    if (kind == kSumI8) limit = one ? 2048 : 1024;
+    else if (large) return g;
+    else if (kind == kSumF16KFirst) limit = one ? 576 : 256;
+    else if (k % 32 == 0) limit = one ? 384 : 256;
+    else if (k % 8 == 0) limit = one ? 328 : 96;
+    else limit = one ? 96 : 0;
+    return k <= limit ? g : batch;
+}
+
 // PART: fp32 out.  A group's sum may pass fp16's range where the sum over all groups does not: sums of more than one group stay
 // fp32 until they are added up (cpmk_gemm_add_parts).
 template <bool PART>
@@ -139,6 +168,10 @@ extern "C" {
 
 int cpmk_gemm_sum_groups(int32_t m, int32_t n, int32_t batch) {
     return m < 0 || n < 0 || batch < 1 ? 1 : sum_groups(m, n, batch);
+}
+
+int cpmk_gemm_sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t batch) {
+    return m < 0 || n < 0 || k < 0 || batch < 1 ? 1 : sum_groups_for(kind, m, k, n, batch);
 }
 
 int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,

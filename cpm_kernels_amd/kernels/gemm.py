@@ -179,6 +179,12 @@ def gemm_sum_groups(m: int, n: int, batch: int) -> int:
     return cpmk.gemm_sum_groups(m, n, batch)
 
 
+def gemm_sum_groups_for(kind: int, m: int, k: int, n: int, batch: int) -> int:
+    """The same for a depth of k an entry, or `batch` where one product per entry and the sum of them is the quicker.
+    kind 0: gemm_int8_scale_sum, 1: gemm_fp16_sum, 2: gemm_fp16_parts with k_first."""
+    return cpmk.gemm_sum_groups_for(kind, m, k, n, batch)
+
+
 def gemm_int8_scale_sum(m: int, k: int, n: int, batch: int, groups: int,
                         A: DevicePointer,           # (batch, m, k)     int8
                         B: DevicePointer,           # (batch, n, k)     int8

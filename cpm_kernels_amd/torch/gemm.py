@@ -9,7 +9,7 @@ the six-launch sequence, which ``fused=False`` still runs through the kernel-lev
 import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
-    gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups, gemm_int8_scale_sum, gemm_fp16_sum, \
+    gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_for, gemm_int8_scale_sum, gemm_fp16_sum, \
     gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, \
     arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
     transpose_i8, transpose_i8_ld
@@ -140,7 +140,7 @@ def gemm_and_scale_sum(quantA, scaleA, quantB) -> torch.Tensor:
     """(1, M, N): the sum over the batch of scaleA * (quantA x quantB^T), quantA (b, M, K) and quantB (b, N, K)."""
     batch, M, K = quantA.size()
     N = quantB.size(1)
-    groups = gemm_sum_groups(N, M, batch)
+    groups = gemm_sum_groups_for(0, N, K, M, batch)
     if groups == batch or quantB.size(0) != batch or K == 0 or K % 128 != 0 or max(M, N) * K >= 2 ** 31 or batch * K >= 2 ** 22:
         return _sum_entries(gemm_and_scale(quantA, scaleA, quantB, None, False, True))
     parts = torch.empty((groups, M, N), dtype=torch.half if groups == 1 else torch.float32, device=quantA.device)
@@ -304,12 +304,9 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
 
 
 def _entry_groups(M: int, K: int, N: int, batch: int, joined: bool) -> int:
-    """Groups that an fp16 product summed over the batch is formed in.  `joined`: a group's entries become one contraction, which
-    the tile kernel takes up to operands of 4 GiB; beyond that there are more groups, down to the entries one by one."""
-    groups = gemm_sum_groups(N, M, batch)
-    while joined and groups < batch and max(M, N) * K * (batch // groups) >= 2 ** 31:
-        groups = next(g for g in range(groups + 1, batch + 1) if batch % g == 0)
-    return groups
+    """Groups that an fp16 product summed over the batch is formed in.  `joined`: both operands stored (K, rows), so that a group's
+    entries are one contraction."""
+    return gemm_sum_groups_for(2 if joined else 1, N, K, M, batch)
 
 
 def gemm_pth_fp16_sum(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch.Tensor:

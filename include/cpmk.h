@@ -191,8 +191,11 @@ int cpmk_gemm_fp16(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batc
  * (groups divides batch, at most 16 entries a group), accumulated in fp32 and rounded once.
  * int8: each entry's int32 product is scaled by scale_row (batch, n) first; k a multiple of 128, buffers on 16-byte boundaries.
  * fp16: k > 32, buffers on 4-byte boundaries.  m and n multiples of 4.
- * cpmk_gemm_sum_groups: as few groups as keep the device busy. */
+ * cpmk_gemm_sum_groups: as few groups as keep the device busy.
+ * cpmk_gemm_sum_groups_for: the same for a depth k an entry, or `batch` where one product per entry and the sum of them is the quicker.
+ * kind 0: int8, 1: fp16, 2: fp16 with operands stored (batch, k, m) and (batch, k, n). */
 int cpmk_gemm_sum_groups(int32_t m, int32_t n, int32_t batch);
+int cpmk_gemm_sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t batch);
 int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                              const void* scale_row, void* out, void* stream);
 int cpmk_gemm_fp16_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,

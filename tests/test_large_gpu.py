@@ -327,7 +327,7 @@ def test_batch_sum_beyond_2_32_columns(gpu):
 def test_weight_gradient_over_more_than_4_gib_of_tokens(gpu):
     """fp16 training at long sequences: the entries of the batch together pass 2^31 elements."""
     import cpm_kernels_amd.torch as ct
-    batch, tokens, din, dout = 8, 32768, 8192, 256
+    batch, tokens, din, dout = 8, 32768, 8192, 8192
     _name("weight gradient", batch, tokens, din, dout)
     x = _randn_half((batch, tokens, din), 3, gpu)
     w = torch.zeros((1, dout, din), dtype=torch.half, device=gpu, requires_grad=True)

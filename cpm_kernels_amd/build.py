@@ -6,10 +6,13 @@ The library is built in-tree (cpm_kernels_amd/lib/) so that it travels with the 
 tree; hipcc cross-compiles for gfx950 without a GPU being present.
 """
 import os
+import shlex
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
+from .library.base import native_path
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -84,17 +87,34 @@ def build_library(verbose=True, jobs=None):
     return library_path()
 
 
+def find_cxx():
+    """A host C++ compiler, None if there is none (hipcc's own clang++ counts)."""
+    rocm = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "clang++")
+    for cand in (os.environ.get("CXX"), "g++", "c++", "clang++", rocm):
+        if cand and shutil.which(shlex.split(cand)[0]):
+            return shlex.split(cand)
+    return None
+
+
 def build_native(verbose=True):
-    """The extension modules that call the library from Python (host code only)."""
-    import sysconfig
-    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    """The extension module that calls the library from Python (host code only), for the running Python.  Without a C++ compiler
+    or the Python headers there is none, and the calls go through ctypes.  Returns its path, or None."""
+    include = sysconfig.get_paths()["include"]
+    out = native_path("_cpmk_call")
+    cxx = find_cxx()
+    if cxx is None or not os.path.exists(os.path.join(include, "Python.h")):
+        if os.path.exists(out):         # (made for the library as it was)
+            os.remove(out)
+        if verbose:
+            print("[cpmk build] no C++ compiler or no Python headers: launchers are called through ctypes", flush=True)
+        return None
     os.makedirs(LIBDIR, exist_ok=True)
-    base = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-I" + sysconfig.get_paths()["include"]]
-    out = os.path.join(LIBDIR, "_cpmk_call.so")
-    _run(base + [os.path.join(NATIVE_SRC, "call.cpp"), "-o", out + ".tmp"])
+    _run(cxx + ["-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-I" + include,
+                os.path.join(NATIVE_SRC, "call.cpp"), "-o", out + ".tmp"])
     os.replace(out + ".tmp", out)
     if verbose:
         print("[cpmk build] linked %s" % out, flush=True)
+    return out
 
 
 def build_bench_library(verbose=True):

@@ -69,13 +69,19 @@ def find_lib(name: str):
     return ctypes.util.find_library(name)
 
 
+def native_path(name: str) -> str:
+    """Where the extension module `name` for the running Python lies (the suffix names its version and ABI)."""
+    import sysconfig
+    return os.path.join(_PKG_DIR, "lib", name + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
 def load_native(name: str):
-    """The in-tree extension module lib/<name>.so (cpm_kernels_amd/build.py), None if it is not there."""
+    """The in-tree extension module of that name for this Python (cpm_kernels_amd/build.py), None if it is not there."""
     import importlib.machinery
     import importlib.util
-    path = os.path.join(_PKG_DIR, "lib", name + ".so")
+    path = native_path(name)
     if not os.path.exists(path):
-        logger.warning("%s is not built", path)
+        logger.info("%s is not built", path)
         return None
     try:
         loader = importlib.machinery.ExtensionFileLoader(name, path)
@@ -111,13 +117,8 @@ class Lib:
 
     def address(self, name):
         """The address of a symbol, None if the library or the symbol is missing."""
-        if self._lib is None:
-            return None
-        try:
-            return ctypes.cast(getattr(self._lib, name), ctypes.c_void_p).value
-        except AttributeError:
-            logger.warning("Symbol %s not found in %s", name, self._path)
-            return None
+        func = getattr(self._lib, name, None) if self._lib is not None else None
+        return None if func is None else ctypes.cast(func, ctypes.c_void_p).value
 
     def bind(self, name, arg_types, ret_type) -> Callable[[LibCall], LibCall]:
         if self._lib is None:

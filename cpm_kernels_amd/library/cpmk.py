@@ -1,4 +1,4 @@
-"""Binding of libcpmk_hip.so (include/cpmk.h): the launchers through native/call.cpp, the rest through ctypes.
+"""Binding of libcpmk_hip.so (include/cpmk.h): the launchers through native/call.cpp where it is built, all else through ctypes.
 
 Replaces cpm_kernels/library/{cuda,cudart,cublaslt}.py of the reference: instead of a CUDA
 driver launch (library/cuda.py:249-267) or a cuBLASLt call (library/cublaslt.py:113-150)
@@ -10,26 +10,39 @@ from .base import Lib, load_native
 
 lib = Lib("cpmk_hip")
 
-# the launchers (all return an int status), without their prefix; native/call.cpp takes their argument types from include/cpmk.h
-_LAUNCHERS = (
-    "gemm_calc_scale", "gemm_calc_scale_transpose", "gemm_round", "gemm_round_transpose", "gemm_scale",
-    "gemm_scale_x", "gemm_scale_y", "gemm_int8", "gemm_int8_scale", "gemm_quantize", "gemm_quantize_pair",
-    "gemm_quantize_cols", "gemm_fp16", "gemm_quantize_cols_ld", "gemm_quantize_pair_ld",
-    "gemm_backward_round_scale_ld", "gemm_int8_scale_one", "transpose_i8_ld", "gemm_int8_scale_sum", "gemm_fp16_sum",
-    "gemm_int8_scale_parts", "gemm_fp16_parts", "gemm_add_parts",
-    "gemv_fp16", "gemv_fp16_transpose", "gemv_broadcast_mat_fp16", "embedding_forward", "embedding_step",
-    "copy_data_to_kv", "gemv_calc_scale", "gemv_round", "gemv_broadcast_mat_int8", "layernorm_forward",
-    "layernorm_forward_noalloc", "layernorm_step", "layernorm_affine_forward", "layernorm_affine_forward_stats",
-    "layernorm_affine_backward", "softmax_forward", "softmax_step_inplace", "gelu_forward", "position_embedding_init",
-    "position_embedding_forward", "position_embedding_step", "arith_ln_mul_add", "arith_ln_mul", "arith_element_add",
-    "mask", "arith_global_scale", "arith_element_mul", "arith_batch_add_forward", "arith_batch_add_backward",
-    "arith_ln_add", "arith_ln_div", "arith_ln_sub_div", "arith_ln_mul_backward", "arith_ln_add_backward",
-    "arith_batch_mul_add", "arith_batch_mul", "gelu_backward", "softmax_backward", "layernorm_forward_v",
-    "layernorm_forward_mv", "layernorm_backward_v", "layernorm_backward_mv", "gemm_backward_round_scale",
-    "gemm_backward_scale_round", "position_embedding_backward", "embedding_backward_stage1",
-    "embedding_backward_stage2", "embedding_order_ids", "embedding_backward_rows", "transpose", "transpose_i8", "array_add",
-    "adjustify_logits", "copy_extend_buffer", "has_nan_inf", "copy_pos_hidden", "async_status", "selftest_exchange_timeout",
-)
+# the launchers (all return an int status), without their prefix, with their parameters: i int32_t or int, l int64_t, f float,
+# p pointer
+_LAUNCHERS = {
+    "gemm_calc_scale": "iiippp", "gemm_calc_scale_transpose": "iiippp", "gemm_round": "iiipppp",
+    "gemm_round_transpose": "iiipppp", "gemm_scale": "iiippppiip", "gemm_scale_x": "iiipppp",
+    "gemm_scale_y": "iiipppp", "gemm_int8": "iiiiiiipppp", "gemm_int8_scale": "iiiiiiippppiipp",
+    "gemm_quantize": "iiipppip", "gemm_quantize_pair": "lppplpppip", "gemm_quantize_cols": "iiipppip",
+    "gemm_fp16": "iiiiiiipppp", "gemm_quantize_cols_ld": "iiippippipip", "gemm_quantize_pair_ld": "lppplpppiip",
+    "gemm_backward_round_scale_ld": "iiipppipip", "gemm_int8_scale_one": "iiiiiiippppiipp",
+    "transpose_i8_ld": "iiipipip", "gemm_int8_scale_sum": "iiiiippppp", "gemm_fp16_sum": "iiiiipppp",
+    "gemm_int8_scale_parts": "iiiiippppp", "gemm_fp16_parts": "iiiiiipppp", "gemm_add_parts": "ilppp",
+    "gemv_fp16": "iiipppp", "gemv_fp16_transpose": "iiipppp", "gemv_broadcast_mat_fp16": "iiipppp",
+    "embedding_forward": "iiipppp", "embedding_step": "iipppp", "copy_data_to_kv": "iiippip",
+    "gemv_calc_scale": "iippp", "gemv_round": "iipppp", "gemv_broadcast_mat_int8": "iiipppppp",
+    "layernorm_forward": "iiippfip", "layernorm_forward_noalloc": "iiippfip", "layernorm_step": "iippfip",
+    "layernorm_affine_forward": "iiippppfip", "layernorm_affine_forward_stats": "iiipppppfip",
+    "layernorm_affine_backward": "iiippppppppp", "softmax_forward": "iiippp", "softmax_step_inplace": "iipp",
+    "gelu_forward": "iippp", "position_embedding_init": "iipip", "position_embedding_forward": "iiiiipppip",
+    "position_embedding_step": "iiiiipppip", "arith_ln_mul_add": "iiippppp", "arith_ln_mul": "iiipppp",
+    "arith_element_add": "iipppp", "mask": "iiippfpp", "arith_global_scale": "lpfpp", "arith_element_mul": "iipppp",
+    "arith_batch_add_forward": "iipppp", "arith_batch_add_backward": "ilppp", "arith_ln_add": "iiipppp",
+    "arith_ln_div": "iiipppp", "arith_ln_sub_div": "iiippppp", "arith_ln_mul_backward": "iiipppp",
+    "arith_ln_add_backward": "iiippp", "arith_batch_mul_add": "iippppp", "arith_batch_mul": "iipppp",
+    "gelu_backward": "iipppp", "softmax_backward": "iiipppp", "layernorm_forward_v": "iiipppfp",
+    "layernorm_forward_mv": "iiippppfp", "layernorm_backward_v": "iiippppp", "layernorm_backward_mv": "iiipppppp",
+    "gemm_backward_round_scale": "iiippppip", "gemm_backward_scale_round": "iiippppip",
+    "position_embedding_backward": "iiiiipppip", "embedding_backward_stage1": "iiippppppp",
+    "embedding_backward_stage2": "iipppp", "embedding_order_ids": "ipppp", "embedding_backward_rows": "iipppppp",
+    "transpose": "iiippp", "transpose_i8": "iiippp", "array_add": "piip", "adjustify_logits": "iipfffpp",
+    "copy_extend_buffer": "iiippp", "has_nan_inf": "lppp", "copy_pos_hidden": "iiiippp", "async_status": "",
+    "selftest_exchange_timeout": "ip",
+}
+_CTYPES = {"i": ctypes.c_int32, "l": ctypes.c_int64, "f": ctypes.c_float, "p": ctypes.c_void_p}
 
 EXPORTED_SYMBOLS = sorted(["cpmk_" + n for n in _LAUNCHERS] + [
     "cpmk_version", "cpmk_error_string", "cpmk_device_count", "cpmk_get_device",
@@ -63,26 +76,28 @@ def _value(obj, size=None):
     raise TypeError("expected a number or a %s, got %s" % (ctype.__name__, type(obj).__name__))
 
 
+# Beside the library there may be an extension module for this Python that calls the launchers at a third of ctypes' cost
+# (native/call.cpp); without it (a library from elsewhere, another Python, a build without a C++ compiler) ctypes does it.
 _native = load_native("_cpmk_call") if lib.loaded else None
+_native_names = ()
 if _native is not None:
     _native.init(lib.address("cpmk_error_string"), _value)
+    _native_names = _native.names()
 
 
-def _make(name):
-    address = lib.address(name)
-    if address is not None and _native is not None:
-        return _native.bind(name, address)
-
+def _make(name, parameters):
+    @lib.bind(name, [_CTYPES[c] for c in parameters], ctypes.c_int)
     def call(*args):
-        if lib.loaded and _native is not None:
-            raise AttributeError("%s: undefined symbol: %s" % (lib.path, name))
-        raise RuntimeError("Library %s is not initialized" % ("_cpmk_call" if lib.loaded else "cpmk_hip"))
+        checkStatus(getattr(lib, name)(*args))
     call.__name__ = name[len("cpmk_"):]
+    call.__doc__ = "Launch %s (see include/cpmk.h)." % name
+    if name in _native_names and hasattr(lib, name):
+        return _native.bind(name, lib.address(name))
     return call
 
 
-for _name in _LAUNCHERS:
-    globals()[_name] = _make("cpmk_" + _name)
+for _name, _parameters in _LAUNCHERS.items():
+    globals()[_name] = _make("cpmk_" + _name, _parameters)
 
 
 def check() -> None:

@@ -231,6 +231,49 @@ def test_joined_entries_stay_within_the_tile_kernels_operands():
     assert _entry_groups(8192, 32768, 8192, 8, True) == 2       # (no more groups than it takes)
 
 
+def test_binding_agrees_with_the_header():
+    """The parameter codes that ctypes binds the launchers by, against the prototypes."""
+    from cpm_kernels_amd.library import cpmk
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "cpmk.h")).read(), flags=re.S)
+    protos = dict(re.findall(r"\bint\s+(cpmk_[a-z0-9_]+)\s*\(([^)]*)\)", text))
+    for name, codes in cpmk._LAUNCHERS.items():
+        params = [p.strip() for p in protos["cpmk_" + name].split(",") if p.strip() != "void"]
+        assert codes == "".join("p" if "*" in p else {"int": "i", "int32_t": "i", "int64_t": "l", "float": "f"}[p.split()[0]] for p in params), name
+
+
+def test_launchers_without_the_extension_module():
+    """A library without the extension module beside it is called through ctypes, with the same results and errors."""
+    code = """
+import importlib, cpm_kernels_amd.library.base as base
+from cpm_kernels_amd.library import cpmk
+native = type(cpmk.gelu_forward)
+base.load_native = lambda name: None
+importlib.reload(cpmk)
+assert type(cpmk.gelu_forward) is type(lambda: 0), native
+import cpm_kernels_amd.kernels as ck
+ck.gelu_forward(0, 8, None, None, None)
+cpmk.arith_global_scale(0, None, 1.5, None, None)
+for call in (lambda: cpmk.gelu_forward(1, 8, None, None, None), lambda: cpmk.arith_batch_add_backward(2, 2 ** 32, None, None, None)):
+    try:
+        call()
+    except RuntimeError as e:
+        assert "invalid argument" in str(e)
+    else:
+        raise AssertionError("accepted null buffers")
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=ROOT)
+
+
+def test_build_without_a_cxx_compiler(monkeypatch, tmp_path):
+    from cpm_kernels_amd import build
+    old = tmp_path / "_cpmk_call.so"
+    old.write_bytes(b"")
+    monkeypatch.setattr(build, "native_path", lambda name: str(old))
+    monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    assert build.find_cxx() is None and build.build_native(verbose=False) is None
+    assert not old.exists()         # (it was made for another library)
+
+
 def test_launchers_take_ctypes_numbers_of_the_parameters_type():
     """As ctypes function prototypes do: c_int32 for an int32_t parameter (not another width), c_float for a float one, and any
     object with an index."""

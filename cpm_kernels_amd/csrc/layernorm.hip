@@ -24,11 +24,9 @@ __device__ inline half8_t affine8(half8_t y, half_t a, half_t b, bool has_beta) 
 }
 
 // Single pass: the whole (n x LPR*8) column tile lives in registers.  Tiles of whole cache lines (LPR == 8) are
-// read with the non-temporal hint: every byte is touched once.  Results are stored plainly, whatever the kernel alone
-// would gain by the hint (8 x 4096 x 512 through the team kernel, both hints: 17.2 -> 15.2 us): a product's quantiser reads
-// them next, from the last-level cache where they still are there (a whole layer of 16 x 1024 tokens 5890 -> 5862 us,
-// k_gelu's result stored alike).
-// MODE 0: 16-byte accesses, loads non-temporal where a tile's row segments are whole cache lines; 1: 16-byte accesses without
+// read and written with the non-temporal hint: every byte is touched once (8 x 4096 x 512 through the team
+// kernel: 17.2 -> 15.2 us).
+// MODE 0: 16-byte accesses, non-temporal where a tile's row segments are whole cache lines; 1: 16-byte accesses without
 // the hint (rows that do not start on 128-byte boundaries); 2: any m and alignment, element by element (dim1.h).
 template <int NT, int LPR, int R, bool AFF, int MODE = 0>
 __global__ __launch_bounds__(NT) void k_layernorm_tile(int32_t n, int32_t m, int32_t tiles_per_batch,
@@ -114,7 +112,7 @@ __global__ __launch_bounds__(NT) void k_layernorm_tile(int32_t n, int32_t m, int
         if constexpr (AFF) y = affine8(y, coef[0][p * T::RPP + rg], coef[1][p * T::RPP + rg], beta != nullptr);
         v[p] = y;
     }
-    coltile_store<NT, LPR, R, false, MODE == 2>(v, out + boff, n, m, col0);
+    coltile_store<NT, LPR, R, LPR == 8 && MODE == 0, MODE == 2>(v, out + boff, n, m, col0);
 }
 
 // Tall columns.  A register tile holds T::ROWS rows of 64 columns (128-byte row segments, whole
@@ -231,7 +229,7 @@ __global__ __launch_bounds__(NT) void k_layernorm_team(int32_t n, int32_t m, int
         if constexpr (AFF) y = affine8(y, coef[0][p * T::RPP + rg], coef[1][p * T::RPP + rg], beta != nullptr);
         v[p] = y;
     }
-    coltile_store<NT, LPR, R, false, MODE == 2>(v, out + boff, own_n, m, col0);
+    coltile_store<NT, LPR, R, MODE == 0, MODE == 2>(v, out + boff, own_n, m, col0);
     if (tid < 64) xch_retire(xl, team, parts);     // after the barrier above: this workgroup holds all it needs
 }
 

@@ -356,12 +356,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA && NV > 
 // loads pass under another's rounding.  A wave per row held such rows in 64 to 128 registers, and those past 8192
 // columns went through memory twice (scales, then rounding): [4096, 10240] 41 us; 24 us here.
 template <int NV, bool QUANT, bool UA>
-__global__ __launch_bounds__(256) void k_rows_wg(RowsArgs a) {
+__global__ __launch_bounds__(256) void k_rows_wg(RowsArgs a, int64_t row0) {
     __shared__ uint32_t red[4];
     __shared__ float redf[4];
     const int tid = threadIdx.x;
     const int32_t m = a.m;
-    const int64_t row = blockIdx.x;
+    const int64_t row = row0 + blockIdx.x;
     const bool second = row >= a.rows0;
     const int64_t lrow = second ? row - a.rows0 : row;
     const half_t* mat = (second ? a.mat1 : a.mat0) + lrow * m;
@@ -442,15 +442,17 @@ template <bool QUANT, bool UA = false>
 static int launch_rows(const RowsArgs& ra, hipStream_t st) {
     const int64_t rows = ra.rows0 + ra.rows1;
     const int32_t len = ra.ld > ra.m ? ra.ld : ra.m;
-    if (ra.m > kRowsWave) {
-        if (!grid_fits(rows)) return CPMK_ETOOBIG;
-        const dim3 g((unsigned)rows);
+    if (ra.m > kRowsWave) {       // (more rows than a launch holds workgroups: several launches)
         const int nv = (int)ceil_div(len, 2048);
-        if (nv <= 3) hipLaunchKernelGGL((k_rows_wg<3, QUANT, UA>), g, dim3(256), 0, st, ra);
-        else if (nv <= 4) hipLaunchKernelGGL((k_rows_wg<4, QUANT, UA>), g, dim3(256), 0, st, ra);
-        else if (nv <= 5) hipLaunchKernelGGL((k_rows_wg<5, QUANT, UA>), g, dim3(256), 0, st, ra);
-        else hipLaunchKernelGGL((k_rows_wg<8, QUANT, UA>), g, dim3(256), 0, st, ra);
-        return launch_status();
+        for (int64_t r0 = 0; r0 < rows; r0 += kRowsGrid) {
+            const dim3 g((unsigned)(rows - r0 < kRowsGrid ? rows - r0 : kRowsGrid));
+            if (nv <= 3) hipLaunchKernelGGL((k_rows_wg<3, QUANT, UA>), g, dim3(256), 0, st, ra, r0);
+            else if (nv <= 4) hipLaunchKernelGGL((k_rows_wg<4, QUANT, UA>), g, dim3(256), 0, st, ra, r0);
+            else if (nv <= 5) hipLaunchKernelGGL((k_rows_wg<5, QUANT, UA>), g, dim3(256), 0, st, ra, r0);
+            else hipLaunchKernelGGL((k_rows_wg<8, QUANT, UA>), g, dim3(256), 0, st, ra, r0);
+            if (int e = launch_status()) return e;
+        }
+        return 0;
     }
     const int nv = (int)ceil_div(len, 512);
     const dim3 g(rows_grid(rows));

@@ -344,3 +344,22 @@ def test_weight_gradient_over_more_than_4_gib_of_tokens(gpu):
         # fp32 sums in chains of 16-deep products, one rounding to fp16
         bound = mag * (batch * tokens) * 2.0 ** -24 + want.abs() * 2.0 ** -11
         assert bool(((got[0, :, cols].double() - want).abs() <= bound).all()), cols
+
+
+@pytest.mark.parametrize("m,rows", [(4104, 2 ** 24 + 3), (8, 2 ** 25 + 5)])
+def test_row_scales_of_more_rows_than_a_launch_holds(gpu, m, rows):
+    """2^24 rows of a workgroup each are 2^32 threads, more than one launch holds; 2^25 rows of a wave each make the grid loop."""
+    need = rows * (m + 1) * 2
+    if torch.cuda.mem_get_info()[0] < need + (4 << 30):
+        pytest.skip("needs %d GB" % (need >> 30))
+    _name("row scales", rows, m)
+    x = torch.zeros((rows, m), dtype=torch.half, device=gpu)
+    scale = torch.full((rows,), 77.0, dtype=torch.half, device=gpu)
+    picked = sorted({0, 1, 2 ** 23 - 1, 2 ** 23, 2 ** 24 - 1, 2 ** 24, 2 ** 24 + 2, rows - 1})
+    for i, r in enumerate(picked):
+        x[r, m - 1 - i] = -127.0 * (i + 1)
+    ck.gemm_calc_scale(1, rows, m, x.data_ptr(), scale.data_ptr(), stream())
+    assert [float(scale[r]) for r in picked] == [i + 1.0 for i in range(len(picked))]
+    assert int((scale != 0).sum()) == len(picked), "rows written wrongly or not at all"
+    del x, scale
+    torch.cuda.empty_cache()

@@ -27,7 +27,14 @@ __device__ inline half_t gelu1(half_t h) {
     return (half_t)(x * __builtin_amdgcn_rcpf(1.0f + e));
 }
 
-__global__ __launch_bounds__(256) void k_gelu(int64_t total, const half_t* mat, half_t* out, int vec) {
+// Bound by memory.  Results of 17 to 92 MB are stored without the non-temporal hint: the quantiser that reads them next finds
+// them in the last-level cache (256 MB, which holds the input too).  gelu alone, and with the quantiser of its result, hint /
+// plain: 34 MB 12.8 / 12.3 and 32.8 / 31.4 us, 67 MB 22.9 / 22.0 and 56.0 / 53.9, 84 MB 28.1 / 28.3 and 71.8 / 68.5.  Smaller
+// ones lose as much alone as the two gain together (4 MB 3.1 / 3.5 and 16.4 / 15.9), larger ones more and more (101 MB 33.1 /
+// 35.3 and 86.1 / 83.1, 268 MB 84.1 / 88.0 and 196.2 / 195.9, 671 MB 209 / 218 and 500 / 507).
+static bool gelu_keeps(int64_t total) { return total >= 8 << 20 && total <= 44 << 20; }
+
+__global__ __launch_bounds__(256) void k_gelu(int64_t total, const half_t* mat, half_t* out, int vec, int keep) {
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (vec) {
         const int64_t e0 = gid * 8;
@@ -35,7 +42,7 @@ __global__ __launch_bounds__(256) void k_gelu(int64_t total, const half_t* mat, 
             half8_t v = flat_load8(mat + e0, vec);
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = gelu1(v[e]);
-            flat_store8(out + e0, v, vec);
+            flat_store8(out + e0, v, keep ? 2 : vec);
         } else {
             for (int64_t i = e0; i < total; ++i) out[i] = gelu1(mat[i]);
         }
@@ -172,7 +179,7 @@ int cpmk_gelu_forward(int32_t batch, int32_t n, const void* mat, void* out, void
     const int vec = aligned16(mat) && aligned16(out) ? 1 : 2;       // (2: buffers off 16-byte boundaries)
     const int64_t g = ceil_div(ceil_div(total, 8), 256);
     hipLaunchKernelGGL(k_gelu, dim3((unsigned)g), dim3(256), 0, (hipStream_t)stream, total, (const half_t*)mat,
-                       (half_t*)out, vec);
+                       (half_t*)out, vec, gelu_keeps(total) ? 1 : 0);
     return launch_status();
 }
 

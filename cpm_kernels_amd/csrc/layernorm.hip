@@ -27,7 +27,8 @@ __device__ inline half8_t affine8(half8_t y, half_t a, half_t b, bool has_beta) 
 // read and written with the non-temporal hint: every byte is touched once (8 x 4096 x 512 through the team
 // kernel: 17.2 -> 15.2 us).
 // MODE 0: 16-byte accesses, non-temporal where a tile's row segments are whole cache lines; 1: 16-byte accesses without
-// the hint (rows that do not start on 128-byte boundaries); 2: any m and alignment, element by element (dim1.h).
+// the hint (rows that do not start on 128-byte boundaries); 2: any m and alignment, element by element (dim1.h); 3: as 0 with
+// plain stores, for results that the next kernel finds in the last-level cache (keeps()); affine form only.
 template <int NT, int LPR, int R, bool AFF, int MODE = 0>
 __global__ __launch_bounds__(NT) void k_layernorm_tile(int32_t n, int32_t m, int32_t tiles_per_batch,
                                                        const half_t* mat, half_t* out,
@@ -56,7 +57,7 @@ __global__ __launch_bounds__(NT) void k_layernorm_tile(int32_t n, int32_t m, int
         }
     }
     half8_t v[R];
-    coltile_load<NT, LPR, R, LPR == 8 && MODE == 0, MODE == 2>(v, mat + boff, n, m, col0, (half_t)0.0f);
+    coltile_load<NT, LPR, R, LPR == 8 && (MODE == 0 || MODE == 3), MODE == 2>(v, mat + boff, n, m, col0, (half_t)0.0f);
     if constexpr (AFF) {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(NT) void k_layernorm_team(int32_t n, int32_t m, int
         if (beta != nullptr) cb = beta[row];
     }
     half8_t v[R];
-    coltile_load<NT, LPR, R, MODE == 0, MODE == 2>(v, mat + boff, own_n, m, col0, (half_t)0.0f);
+    coltile_load<NT, LPR, R, MODE == 0 || MODE == 3, MODE == 2>(v, mat + boff, own_n, m, col0, (half_t)0.0f);
     if constexpr (AFF) {
         coef[0][tid] = ca;
         coef[1][tid] = cb;
@@ -371,7 +372,7 @@ static void launch_tile(int32_t batch, int32_t n, int32_t m, const half_t* mat, 
     if (alpha != nullptr)
         hipLaunchKernelGGL((k_layernorm_tile<NT, LPR, R, true, MODE>), dim3((unsigned)((int64_t)tiles * batch)), dim3(NT), 0, st, n,
                            m, tiles, mat, out, alpha, beta, eps, rd_mean, stats);
-    else
+    else if constexpr (MODE != 3)
         hipLaunchKernelGGL((k_layernorm_tile<NT, LPR, R, false, MODE>), dim3((unsigned)((int64_t)tiles * batch)), dim3(NT), 0, st, n,
                            m, tiles, mat, out, alpha, beta, eps, rd_mean, stats);
 }
@@ -386,6 +387,15 @@ static bool launch_tile_r(int r, int32_t batch, int32_t n, int32_t m, const half
     else return false;
     return true;
 }
+
+// Affine results (a product's input: a quantiser reads them next) of 64 to 160 MB are stored without the non-temporal hint and
+// found in the last-level cache (256 MB).  The layernorm alone, and with the quantiser of its result, hint / plain:
+// 8 x 4096 x 1024 (67 MB) 36.0 / 36.3 and 68.3 / 65.4 us, 12 x 4096 x 1024 51.8 / 51.3 and 96.6 / 90.9, 16 x 4096 x 1024
+// 66.6 / 66.3 and 123.4 / 113.6, 64 x 1024 x 1024 58.8 / 57.7 and 113.4 / 104.3, 18 x 4096 x 1024 (151 MB) 73.7 / 75.6 and
+// 136.9 / 124.4.  Smaller ones are slower (4 x 4096 x 512 13.6 / 15.0 and 28.4 / 29.4, 16 x 1024 x 1024 13.4 / 15.2 and
+// 31.9 / 33.8; 8 x 4096 x 512 17.7 / 18.4 and 37.7 / 37.1), larger ones lose more alone than they gain (24 x 4096 x 1024
+// 94.4 / 100.0 and 176.3 / 171.2, 64 x 4096 x 512 121.7 / 131.2 and 229.3 / 227.2).
+static bool keeps(int64_t elements) { return elements >= 32 << 20 && elements <= 80 << 20; }
 
 // `fixed` == nullptr: team launches take their packet slots from the library's pool (exchange.hip).
 // Otherwise the one team launch a call may need uses the slots, counters and status word `fixed`
@@ -408,6 +418,7 @@ static int layernorm_dispatch(int32_t batch, int32_t n, int32_t m, const void* m
     const bool wide = m % 8 == 0 && aligned16(mat) && aligned16(out);
     // the 128-byte row segments of the 64-column tiles are whole cache lines: the non-temporal hint pays there only
     const bool lines = m % 64 == 0 && (reinterpret_cast<uintptr_t>(mat) & 127u) == 0 && (reinterpret_cast<uintptr_t>(out) & 127u) == 0;
+    const bool keep = lines && alpha != nullptr && keeps((int64_t)batch * n * m);
     if ((int64_t)n * m < (1ll << 31) && (wide || m > 1)) {
         // widest row segment whose tile still fits the register budget (at most 8 pieces per lane)
         bool ok = false;
@@ -448,15 +459,16 @@ static int layernorm_dispatch(int32_t batch, int32_t n, int32_t m, const void* m
                     };
                     auto pick = [&](auto modec) {
                         constexpr int MODE = decltype(modec)::value;
-                        if (big) {
-                            if (al != nullptr) go(k_layernorm_team<1024, 8, true, MODE>, 1024);
-                            else go(k_layernorm_team<1024, 8, false, MODE>, 1024);
-                        } else {
-                            if (al != nullptr) go(k_layernorm_team<512, 8, true, MODE>, 512);
+                        if (al != nullptr) {
+                            if (big) go(k_layernorm_team<1024, 8, true, MODE>, 1024);
+                            else go(k_layernorm_team<512, 8, true, MODE>, 512);
+                        } else if constexpr (MODE != 3) {
+                            if (big) go(k_layernorm_team<1024, 8, false, MODE>, 1024);
                             else go(k_layernorm_team<512, 8, false, MODE>, 512);
                         }
                     };
                     if (!wide) pick(std::integral_constant<int, 2>{});
+                    else if (keep) pick(std::integral_constant<int, 3>{});
                     else if (lines) pick(std::integral_constant<int, 0>{});
                     else pick(std::integral_constant<int, 1>{});
                     const int e = launch_status();
@@ -468,6 +480,7 @@ static int layernorm_dispatch(int32_t batch, int32_t n, int32_t m, const void* m
         }
         if (!wide) ok = n <= 128 * 8 && launch_tile_r<8, 2>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
         else if (n <= 128 * 8 && m >= 64 && !lines) ok = launch_tile_r<8, 1>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
+        else if (n <= 128 * 8 && m >= 64 && keep) ok = launch_tile_r<8, 3>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
         else if (n <= 128 * 8 && m >= 64) ok = launch_tile_r<8>((int)ceil_div(n, 128), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
         else if (n <= 256 * 8 && m >= 32) ok = launch_tile_r<4>((int)ceil_div(n, 256), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);
         else ok = launch_tile_r<2>((int)ceil_div(n, 512), batch, n, m, x, y, al, be, eps, rd_mean, stats, st);

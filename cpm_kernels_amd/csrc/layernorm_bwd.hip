@@ -5,8 +5,8 @@
 // The reference recomputes the normalised tensor and its statistics and walks the tensors five times
 // (cpm_kernels/torch/layernorm.py:31-86, 113-156; cuda/layernorm.cu:142-339, cuda/arith.cu:213-330).
 //
-// Bound by memory: x and grad in, grad_x out, once each.  The column tile of dim1.h (64 columns x 512 rows of both
-// inputs in registers, taller columns in teams), whose rows' sums over its 64 columns leave as fp32 partials that a second small
+// Bound by memory: x and grad in, grad_x out, once each.  The column tile of dim1.h (64 columns x 256 rows of both
+// inputs in registers, 512 rows beyond 8192; taller columns in teams), whose rows' sums over its 64 columns leave as fp32 partials that a second small
 // kernel adds up in a fixed order.  8 x 4096 x 512: 82 us in five kernels and ten passes before, now 31 + 5 us
 // (3.2 TB/s; with 512 rows a part and one workgroup a compute unit 33; 16 x 4096 x 1024: 114, 119).
 #include "dim1.h"

@@ -222,10 +222,10 @@ __global__ __launch_bounds__(256) void k_dequant(int64_t total, int32_t n, int32
 // ---------------------------------------------------------------------------------------
 // Contiguous rows of up to 64 lanes x NV x 8 halves, one wave per row, the row in registers:
 // absmax -> scale (QUANT false: cu_gemm_calc_scale) and, fused, the rounding of the same
-// registers (QUANT true: calc_scale + round in one pass over HBM).  Waves stride over the rows;
-// the launcher picks the wave count so that every wave gets the same number of rows when the
-// row count allows.  Many resident waves, each with one row in flight, hide the memory latency
-// better here than fewer waves that prefetch their next row (measured).
+// registers (QUANT true: calc_scale + round in one pass over HBM).  A wave takes one row (rows_grid);
+// waves stride over the rows only in grids too large for a launch.  Many resident waves, each with
+// one row in flight, hide the memory latency better here than fewer waves that prefetch their next
+// row (measured).
 // ---------------------------------------------------------------------------------------
 // One or two tensors with rows of the same length per launch (the two operands of a product):
 // virtual row r < rows0 is row r of the first, otherwise row r - rows0 of the second.
@@ -236,7 +236,7 @@ struct RowsArgs {
     int32_t ld;       // bytes from one output row to the next: m, or a multiple of 16 beyond it whose surplus is zeros
 };
 
-// (the launcher counts on 8 resident workgroups per compute unit up to NV = 8, 4 beyond)
+// (eight workgroups share a compute unit, four where pieces of any address need more registers)
 // UA: rows that are not whole 16-byte pieces, or buffers off 16-byte boundaries: a piece inside its row still comes in one
 // 16-byte load and leaves in one 8-byte store (global accesses need no alignment), the piece across a row's end in at
 // most three narrower accesses each way.
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA && NV > 
 // The same for rows of more than 4096 columns: a workgroup per row, NV 16-byte pieces a thread (up to 16384 columns), the
 // maxima of its four waves exchanged through LDS.  Bound by memory: several workgroups share a compute unit and one's
 // loads pass under another's rounding.  A wave per row held such rows in 64 to 128 registers, and those past 8192
-// columns went through memory twice (scales, then rounding): [4096, 10240] 41 us; 24 us here.
+// columns went through memory twice (scales, then rounding): [4096, 10240] 41 us; 22 us here.
 template <int NV, bool QUANT, bool UA>
 __global__ __launch_bounds__(256) void k_rows_wg(RowsArgs a, int64_t row0) {
     __shared__ uint32_t red[4];

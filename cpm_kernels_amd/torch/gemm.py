@@ -12,7 +12,7 @@ from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, ge
     gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_for, gemm_int8_scale_sum, gemm_fp16_sum, \
     gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, \
     arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
-    transpose_i8, transpose_i8_ld
+    transpose_i8_ld
 from ._common import cur_stream
 
 

@@ -1170,10 +1170,11 @@ static int launch_dma(GemmArgs& a, int batch, hipStream_t st, int per_cu = 1) {
     const int64_t r = total % grid;
     da.nfull = (uint32_t)total;
     da.nhalf = 0;
-    // (a half tile's slab must split evenly over the waves too, and rows of K of half a tile be whole 128-byte groups;
-    // a tile moved inside the matrix has no half of its own)
+    // (a half tile's slab must split evenly over the waves too, and beside operands stored (K, rows) rows of K be whole 128-byte groups
+    // in half a tile; a tile moved inside the matrix has no half of its own)
     constexpr bool F16 = epi_f16(EPI);
-    if constexpr (TR % 2 == 0 && (LAY & 4) == 0 && ((BR / 2 + BC) / (1024 / BKB)) % (WR * WC) == 0 && (BR / 2) * (F16 ? 2 : 1) % 128 == 0) {
+    if constexpr (TR % 2 == 0 && (LAY & 4) == 0 && ((BR / 2 + BC) / (1024 / BKB)) % (WR * WC) == 0 &&
+                  ((LAY & 3) == 0 || (BR / 2) * (F16 ? 2 : 1) % 128 == 0)) {
         if (r > 0 && 2 * r <= grid && (a.edge_in & 1) == 0) {
             da.nfull = (uint32_t)(total - r);
             da.nhalf = (uint32_t)(2 * r);

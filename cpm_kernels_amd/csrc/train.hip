@@ -528,7 +528,9 @@ __global__ __launch_bounds__(256) void k_round_scale_rows(int32_t n, int32_t m, 
     mx = block_max<4>(mx, red);
     const float s = (float)((double)mx / 127.0);
     if (threadIdx.x == 0) scale_x[row] = (half_t)s;
-    for (int32_t j = threadIdx.x; j < ld; j += 256) out[row * ld + j] = j < m ? (int8_t)quant_i8((float)x[j] * (float)sy[j], s) : 0;
+    // (the surplus apart: a choice inside the loop keeps its loads from running ahead, 11 rows of 9749 15.3 us instead of 10.8)
+    for (int32_t j = threadIdx.x; j < m; j += 256) out[row * ld + j] = (int8_t)quant_i8((float)x[j] * (float)sy[j], s);
+    for (int32_t j = m + threadIdx.x; j < ld; j += 256) out[row * ld + j] = 0;
 }
 
 // The same with a wave per row and 16-byte accesses (m % 8 == 0, aligned pointers); the second pass

@@ -360,9 +360,8 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     const uint32_t tag = xl.tag;
     constexpr int NT = 512, LPR = 8, R = 8;
     using T = ColTile<NT, LPR, R>;
-    static_assert(KIND != kScaleRound, "colquant.hip");
-    constexpr bool TWO = KIND != kLnFwdV && KIND != kLnFwdMV && KIND != kColAbsmax;     // reads grad_in too
-    constexpr bool IS_MAX = KIND == kColAbsmax;
+    constexpr bool TWO = KIND != kLnFwdV && KIND != kLnFwdMV && KIND != kScaleRound && KIND != kColAbsmax;     // reads grad_in too
+    constexpr bool IS_MAX = KIND == kScaleRound || KIND == kColAbsmax;
     constexpr int NV = (KIND == kLnFwdMV || KIND == kLnBwdMV) ? 2 : 1;      // statistics per column
     __shared__ float lds[(T::NW + 1) * T::COLS * NV];
     __shared__ float tot[T::COLS * 2];
@@ -380,6 +379,14 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     // The per-column and per-row operands of the sums are requested ahead of the tiles: loads return in
     // order, and behind the tiles they would hold the sums back until the last piece had arrived.
     half8_t hv = {0, 0, 0, 0, 0, 0, 0, 0}, hm = {0, 0, 0, 0, 0, 0, 0, 0};
+    half_t sxh[KIND == kScaleRound ? R : 1];
+    if constexpr (KIND == kScaleRound) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int32_t row = own0 + q * T::RPP + rg;
+            sxh[q] = row < p.n ? p.sx[(p.bc ? 0 : (int64_t)b * p.n) + row] : (half_t)0.0f;
+        }
+    }
     constexpr bool NTH = MODE == 0, UA = MODE == 2;
     auto load8 = [&](const half_t* src) __attribute__((always_inline)) {       // eight per-column values of this lane's columns
         half8_t r = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -429,7 +436,8 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
             else if constexpr (KIND == kLnBwdV) s[e] += gi * c3[e] * x;
             else if constexpr (KIND == kLnBwdMV) { s[e] += gi * c3[e] * (x - mean[e]); s[8 + e] += -gi * var[e]; }
             else if constexpr (KIND == kSoftmaxBwd) s[e] += x * gi;
-            else s[e] = fmaxf(s[e], fabsf(x));
+            else if constexpr (KIND == kColAbsmax) s[e] = fmaxf(s[e], fabsf(x));
+            else s[e] = fmaxf(s[e], fabsf(x * (float)sxh[q]));
         }
     if (parts == 1) {
         coltile_reduce<NT, LPR, NV, IS_MAX>(s, lds);      // every lane: the statistics of its 8 columns
@@ -465,6 +473,7 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
         if constexpr (KIND == kLnFwdV) k1[e] = rsqrtf(s[e] / fn + p.eps);
         else if constexpr (KIND == kLnFwdMV) { k0[e] = s[e] / fn; k1[e] = rsqrtf(s[8 + e] / fn - k0[e] * k0[e] + p.eps); }
         else if constexpr (KIND == kLnBwdMV) s[8 + e] -= 2.0f * s[e] * mean[e];        // local_grad_mean -= 2 * local_grad_var * local_mean
+        else if constexpr (KIND == kScaleRound) k0[e] = (float)((double)s[e] / 127.0);     // float / double constant, as the reference writes it
     }
     if (live && part == 0 && rg == 0) {
         half8_t h0, h1;
@@ -472,6 +481,7 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
         for (int e = 0; e < 8; ++e) { h0[e] = (half_t)k0[e]; h1[e] = (half_t)k1[e]; }
         if (KIND == kLnFwdV || KIND == kLnFwdMV) store8(p.out_var + (int64_t)b * p.m + col0, h1);
         if (KIND == kLnFwdMV) store8(p.out_mean + (int64_t)b * p.m + col0, h0);
+        if (KIND == kScaleRound) store8(p.out_var + (int64_t)b * p.m + col0, h0);
         if constexpr (KIND == kColAbsmax) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) h0[e] = scale_from_absmax(s[e]);
@@ -480,6 +490,22 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     }
     if constexpr (KIND == kColAbsmax) {
         // the scales are all there is to write
+    } else if constexpr (KIND == kScaleRound) {
+        if (live) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int32_t lrow = q * T::RPP + rg;
+                if (lrow >= own_n) continue;
+                int32_t t[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) t[e] = quant_i8((float)va[q][e] * (float)sxh[q], k0[e]);
+                const uint32_t lo = pack4_i8(t[0], t[1], t[2], t[3]), hi = pack4_i8(t[4], t[5], t[6], t[7]);
+                int8_t* dst = p.out_i8 + boff + ((uint32_t)lrow * (uint32_t)p.m + (uint32_t)col0);
+                if constexpr (!UA) *reinterpret_cast<uint2_t*>(dst) = uint2_t{lo, hi};
+                else if (col0 + 8 <= p.m) store_byte8_any(dst, lo, hi);
+                else store_byte8_head_any(dst, p.m & 7, lo, hi);
+            }
+        }
     } else {
 #pragma unroll
         for (int q = 0; q < R; ++q)
@@ -946,7 +972,7 @@ static int launch_col(int32_t batch, const ColArgs& p, void* stream, bool missin
     const bool wide = (int64_t)p.n * p.m < (1ll << 31) && parts <= kColTeamMaxParts && tiles * parts <= kXchSlots;
     auto on_line = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 127u) == 0; };
     const bool lines = p.m % 64 == 0 && on_line(p.a) && on_line(p.g) && on_line(p.out);      // (a null pointer counts as aligned)
-    if constexpr (KIND != kScaleRound) if (wide) {
+    if (wide) {
         // teams use one packet slot per (team, part): batches beyond the pool go out in several launches
         const int64_t per_launch = parts > 1 ? kXchSlots / (tiles * parts) : ((1ll << 31) - 8) / (tiles * parts);
         bool no_slots = false;
@@ -1138,7 +1164,10 @@ int cpmk_gemm_backward_scale_round(int32_t batch, int32_t n, int32_t m, const vo
     ColArgs p = {n, m, (const half_t*)mat, nullptr, nullptr, nullptr, (const half_t*)scale_x, nullptr, (int8_t*)out, nullptr,
                  (half_t*)scale_y, 0.0f, broad_cast_x};
     const bool missing = any_null(mat, scale_x, out, scale_y);
-    if (batch > 0 && n > 0 && m > 0 && !missing) {
+    // The column quantiser's lanes take eight rows each, whether they are there or not: it is as fast or faster from 256 rows on, from
+    // 384 where rows are not whole 16-byte pieces (8 x 512 x 1024 9.4 -> 7.4 us, 8 x 4096 x 500 29.7 -> 25.6, 8 x 256 x 1024 6.6 / 6.5), below it
+    // slower than the tile whose lanes skip what is not there (32 x 359 8.9 us, 4.6 here; 300 x 359 10.1 and 8.8).
+    if (batch > 0 && n >= (m % 8 == 0 ? 256 : 384) && m > 0 && !missing) {
         const int rc = col_scale_round_team(batch, n, m, mat, scale_x, broad_cast_x, scale_y, out, stream);
         if (rc >= 0) return rc;
     }

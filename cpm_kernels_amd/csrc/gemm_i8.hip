@@ -565,25 +565,37 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         // saves: 300 x 300 over 400 heads, K = 512 152 us with large tiles, 125 us with small ones, K = 80 both stored (K, rows) 66 and 48 us;
         // 580 x 580 (1.44 times the area) alike; with one operand K-major and K = 80 70 us with large tiles, 74 us with small ones.
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256), mid = ceil_div(n, 128) * ceil_div(m, 128);
-        const bool waste = big * 8 > mid * 3 && (lay == 3 || k >= 256);
-        const bool large = !waste && big * batch * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!(in_q || odd) || m >= 256);
+        // (not where the large tiles are one round of the device: 384 x 384 over 50 heads, K = 1024 28 us with large tiles, 38 us with small ones)
+        const int64_t cus = compute_units();
+        const bool waste = big * 8 > mid * 3 && (lay == 3 || k >= 256) && big * batch > cus;
+        // At depths that are not whole slabs no last round is split into half tiles, and whole rounds of the device count: a large tile takes
+        // as long as two to two and a half small ones (3592 x 384 over 4 entries, K = 8576 and the rest 8: two rounds of large tiles 226 us,
+        // four of small ones 181; 1792 x 384 x 24, K = 3592: 257 and 219).
+        const bool rest = k % 64 != 0;       // (see below)
+        const bool idle = rest && k >= 256 && ceil_div(big * batch, cus) * 9 > ceil_div(mid * batch, cus) * 4;
+        const bool large = !waste && !idle && big * batch * 4 >= cus * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!(in_q || odd) || m >= 256);
         a.edge_in = (in_p ? 1 : 0) | (in_q || odd ? 2 : 0);
         // a depth that is not whole slabs (probabilities x values over 500 keys, scores over heads of 80): its rest is a slab
         // filled up with zeros
-        const bool rest = k % 64 != 0;
+        // more 128x128 tiles than compute units but at most two each: two workgroups a compute unit, as for K-major operands (2460 x 384 over
+        // 7 entries, K = 6144, 420 tiles: 144 -> 120 us; 300 tiles of 640 x 640, K = 2048: 50 -> 37 us)
+        const bool two = mid * batch > cus && mid * batch <= 2 * cus;
         switch (lay) {
             case 1:
                 if (low) return rest ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 13, 32>(a, batch, st) : launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 1, 32>(a, batch, st);
                 if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 13, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 1, 16>(a, batch, st);
-                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 13, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 1, 32>(a, batch, st);
+                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 13, 32>(a, batch, st)
+                     : two ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 1, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 1, 32>(a, batch, st);
             case 2:
                 if (low) return rest ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 14, 32>(a, batch, st) : launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 2, 32>(a, batch, st);
                 if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 14, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 2, 16>(a, batch, st);
-                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 14, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 2, 32>(a, batch, st);
+                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 14, 32>(a, batch, st)
+                     : two ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 2, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 2, 32>(a, batch, st);
             default:
                 if (low && !rest) return launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 3, 32>(a, batch, st);
                 if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 15, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 3, 16>(a, batch, st);
-                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 15, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 3, 32>(a, batch, st);
+                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 15, 32>(a, batch, st, 2)
+                     : two ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 3, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 3, 32>(a, batch, st);
         }
     }
     for (int64_t r0 = 0; r0 < n; r0 += 65535ll * 64) {        // (rows beyond the grid's y dimension: several launches)

@@ -65,6 +65,20 @@ def test_groups(gpu):
         assert 1 <= groups <= batch and batch % groups == 0 and (groups == batch or batch // groups <= 16)
 
 
+def test_groups_fill_the_device(gpu):
+    """No sum over the batch whose last round of tiles leaves the device mostly idle."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for m, n, batch in ((896, 5376, 16), (5376, 3328, 12), (4096, 4352, 8), (4096, 4096, 8), (2560, 2560, 5), (1536, 1536, 12)):
+        for kind in (1, 2):
+            for k in (68, 128, 512):
+                groups = ck.gemm_sum_groups_for(kind, m, k, n, batch)
+                assert 1 <= groups <= batch and batch % groups == 0
+                if groups < batch:
+                    fit = [-(-n // t) * -(-m // t) * groups for t in (128, 256)]
+                    fill = [t / cus / (t // cus + (0 if t % cus == 0 else 0.5 if 2 * (t % cus) <= cus else 1)) for t in fit]
+                    assert max(fill) >= 0.75, (m, n, batch, kind, k, groups)
+
+
 @pytest.mark.parametrize("shape", [s for s in SHAPES if s[1] > 1])
 def test_int8_parts(gpu, shape):
     batch, groups, n, m, k = shape

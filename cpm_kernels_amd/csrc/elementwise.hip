@@ -27,12 +27,13 @@ __device__ inline half_t gelu1(half_t h) {
     return (half_t)(x * __builtin_amdgcn_rcpf(1.0f + e));
 }
 
-// Bound by memory.  Results of 17 to 92 MB are stored without the non-temporal hint: the quantiser that reads them next finds
+// Bound by memory.  Results of 50 to 92 MB are stored without the non-temporal hint: the quantiser that reads them next finds
 // them in the last-level cache (256 MB, which holds the input too).  gelu alone, and with the quantiser of its result, hint /
-// plain: 34 MB 12.8 / 12.3 and 32.8 / 31.4 us, 67 MB 22.9 / 22.0 and 56.0 / 53.9, 84 MB 28.1 / 28.3 and 71.8 / 68.5.  Smaller
-// ones lose as much alone as the two gain together (4 MB 3.1 / 3.5 and 16.4 / 15.9), larger ones more and more (101 MB 33.1 /
-// 35.3 and 86.1 / 83.1, 268 MB 84.1 / 88.0 and 196.2 / 195.9, 671 MB 209 / 218 and 500 / 507).
-static bool gelu_keeps(int64_t total) { return total >= 8 << 20 && total <= 44 << 20; }
+// plain, the input from memory and in the cache: 67 MB 22.9 / 22.0, 56.0 / 53.9 and 19.9 / 19.8, 51.8 / 49.3 us; 84 MB 28.1 /
+// 28.3, 71.8 / 68.5 and 24.6 / 24.3, 67.3 / 63.4.  Smaller ones are slower from the cache (25 MB 10.0 / 10.0, 28.6 / 27.1 and 5.7 /
+// 8.3, 25.6 / 25.5; 34 MB 12.8 / 12.3, 31.6 / 30.6 and 10.5 / 10.9, 29.2 / 30.1), larger ones in either way (101 MB 33.1 / 35.3,
+// 86.1 / 83.1 and 28.9 / 29.0, 73.4 / 73.8; 151 MB 48.4 / 51.6, 112.2 / 110.0 and 42.3 / 50.7, 104.8 / 110.0).
+static bool gelu_keeps(int64_t total) { return total >= 24 << 20 && total <= 44 << 20; }
 
 __global__ __launch_bounds__(256) void k_gelu(int64_t total, const half_t* mat, half_t* out, int vec, int keep) {
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;

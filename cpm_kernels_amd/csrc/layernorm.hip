@@ -388,14 +388,14 @@ static bool launch_tile_r(int r, int32_t batch, int32_t n, int32_t m, const half
     return true;
 }
 
-// Affine results (a product's input: a quantiser reads them next) of 64 to 160 MB are stored without the non-temporal hint and
-// found in the last-level cache (256 MB).  The layernorm alone, and with the quantiser of its result, hint / plain:
-// 8 x 4096 x 1024 (67 MB) 36.0 / 36.3 and 68.3 / 65.4 us, 12 x 4096 x 1024 51.8 / 51.3 and 96.6 / 90.9, 16 x 4096 x 1024
-// 66.6 / 66.3 and 123.4 / 113.6, 64 x 1024 x 1024 58.8 / 57.7 and 113.4 / 104.3, 18 x 4096 x 1024 (151 MB) 73.7 / 75.6 and
-// 136.9 / 124.4.  Smaller ones are slower (4 x 4096 x 512 13.6 / 15.0 and 28.4 / 29.4, 16 x 1024 x 1024 13.4 / 15.2 and
-// 31.9 / 33.8; 8 x 4096 x 512 17.7 / 18.4 and 37.7 / 37.1), larger ones lose more alone than they gain (24 x 4096 x 1024
-// 94.4 / 100.0 and 176.3 / 171.2, 64 x 4096 x 512 121.7 / 131.2 and 229.3 / 227.2).
-static bool keeps(int64_t elements) { return elements >= 32 << 20 && elements <= 80 << 20; }
+// Affine results (a product's input: a quantiser reads them next) of 80 to 160 MB are stored without the non-temporal hint and
+// found in the last-level cache (256 MB).  The layernorm alone, and with the quantiser of its result, hint / plain, the input from
+// memory and in the cache: 12 x 4096 x 1024 (101 MB) 51.8 / 51.3, 96.6 / 90.9 and 48.8 / 51.1, 96.1 / 90.0 us; 16 x 4096 x 1024
+// 66.6 / 66.3, 123.4 / 113.6 and 63.6 / 65.5, 122.6 / 112.2; 18 x 4096 x 1024 (151 MB) 73.7 / 75.6, 136.9 / 124.4 and 71.6 /
+// 75.0, 136.2 / 123.8.  Smaller ones lose more alone than the two gain (8 x 4096 x 1024 36.0 / 36.3, 68.3 / 65.4 and 32.9 / 35.9,
+// 68.2 / 65.2; 16 x 1024 x 1024 13.4 / 15.2, 31.9 / 33.8 and 11.6 / 15.0, 31.0 / 34.2), larger ones too (24 x 4096 x 1024 94.4 /
+// 100.0, 176.3 / 171.2; 64 x 4096 x 512 121.7 / 131.2, 229.3 / 227.2).
+static bool keeps(int64_t elements) { return elements >= 40 << 20 && elements <= 80 << 20; }
 
 // `fixed` == nullptr: team launches take their packet slots from the library's pool (exchange.hip).
 // Otherwise the one team launch a call may need uses the slots, counters and status word `fixed`

@@ -8,7 +8,7 @@ from util import stream
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("shape", [(8, 4096, 1024), (7, 4096, 1024), (64, 1024, 512), (32, 1000, 1088), (20, 4096, 1024), (21, 4096, 1024)])
+@pytest.mark.parametrize("shape", [(10, 4096, 1024), (9, 4096, 1024), (80, 1024, 512), (40, 1000, 1088), (20, 4096, 1024), (21, 4096, 1024)])
 @pytest.mark.parametrize("bias", [True, False])
 def test_layernorm(gpu, shape, bias):
     """The fused form against the norm (which never keeps its result) followed by the affine kernel, bit for bit."""
@@ -27,7 +27,7 @@ def test_layernorm(gpu, shape, bias):
     assert torch.equal(one, two)
 
 
-@pytest.mark.parametrize("total", [(8 << 20) - 8, 8 << 20, (8 << 20) + 5, 44 << 20, (44 << 20) + 3])
+@pytest.mark.parametrize("total", [(24 << 20) - 8, 24 << 20, (24 << 20) + 5, 44 << 20, (44 << 20) + 3])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_gelu(gpu, total, shift):
     """One call against pieces too small to be kept, bit for bit; off 16-byte boundaries too."""

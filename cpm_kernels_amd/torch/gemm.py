@@ -363,6 +363,7 @@ class GEMMFloat(torch.autograd.Function):
 def bmm(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool, int8: bool = False, fused: bool = True) -> torch.Tensor:
     assert A.ndim == 3
     assert B.ndim == 3
+    assert A.size(1 if aT else 2) == B.size(2 if bT else 1), "operands of different contraction lengths"      # (B would be read past its end)
     if int8:
         return GEMMInt8.apply(A, aT, B, bT, fused, torch.is_grad_enabled())
     return GEMMFloat.apply(A, aT, B, bT)

@@ -274,6 +274,17 @@ def test_build_without_a_cxx_compiler(monkeypatch, tmp_path):
     assert not old.exists()         # (it was made for another library)
 
 
+def test_products_of_different_contraction_lengths_are_refused():
+    """Before anything is launched: the second operand would be read past its end."""
+    import torch
+    import cpm_kernels_amd.torch as ct
+    A = torch.zeros((1, 64, 128), dtype=torch.half)
+    for B, aT, bT in (((1, 64, 32), False, False), ((1, 32, 64), False, True), ((2, 128, 32), True, False), ((1, 32, 128), True, True)):
+        for int8 in (False, True):
+            with pytest.raises(AssertionError, match="contraction"):
+                ct.bmm(A, aT, torch.zeros(B, dtype=torch.half), bT, int8=int8)
+
+
 def test_launchers_take_ctypes_numbers_of_the_parameters_type():
     """As ctypes function prototypes do: c_int32 for an int32_t parameter (not another width), c_float for a float one, and any
     object with an index."""

@@ -290,13 +290,17 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
     (M, N) result comes out row-major.  The MFMA tile kernel reads an operand stored (K, rows) as it lies, at 2-8 % more time
     than K-major ones: a transposed copy pays only for products very large next to the operand.  Measured (direct / with a copy):
     8 x 4096 x 4096 x 512, B transposed 108 / 121 us, A 109 / 118; 4 x 1024 x 4096 x 512 34 / 40-44; 8192 x 4096 x 4096 204 / 208;
-    8 x 10240 x 4096 x 512, B transposed 298 / 279; 4096 x 4096 x 10240, A transposed 298 / 275.  Rows of A that are
-    not whole 16-byte pieces are copied always."""
+    8 x 10240 x 4096 x 512, B transposed 298 / 279; 4096 x 4096 x 10240, A transposed 298 / 275.  Or for results beyond the
+    last-level cache of few slabs, where the two compete for memory: 2032 x 4096 over 32 entries of A, K = 256 223 / 203 us, 2048 x 8064
+    x 32 434 / 398 (512 MB and more; 2048 x 2048 x 32 and K = 1024 about even).  Rows of A that are not whole 16-byte pieces are
+    copied always."""
     M, K, N = _dims(A, B, aT, bT)
     if K % 64 == 0 and N % 8 == 0 and M * K < 2 ** 31 and N * K < 2 ** 31:
-        if aT and ((N * (B.size(0) // A.size(0)) > 8192 and K > 128) or M % 8 != 0):     # (short K: the product is bound by writing its output)
+        large = K > 128 and K <= 512 and M * N * max(A.size(0), B.size(0)) > 2 ** 27
+        # (short K: the product is bound by writing its output)
+        if aT and ((N * max(B.size(0) // A.size(0), 1) > 8192 and K > 128) or large and N > 512 or M % 8 != 0):
             A, aT = _transposed_copy(A), False
-        if not bT and M > 8192 and K > 128:
+        if not bT and (M > 8192 and K > 128 or large and M > 2048):
             B, bT = _transposed_copy(B), True
     out = torch.empty((max(A.size(0), B.size(0)), M, N), dtype=torch.half, device=A.device)
     gemm_fp16(N, K, M, B.size(0), A.size(0), bT, aT, B.data_ptr(), A.data_ptr(), out.data_ptr(), cur_stream())

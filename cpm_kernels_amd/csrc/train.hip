@@ -597,9 +597,9 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_wide(int64_t rows, int
 // UA: rows that are not whole 16-byte pieces or buffers off 16-byte boundaries -- a piece inside its row still comes in
 // one 16-byte load and leaves in one 8-byte store (global accesses need no alignment), the piece across a row's end
 // in at most three narrower accesses each way.
-// DIV: the rounding by the IEEE division alone, for short rows, of which a lane has few elements: the second sequence costs them more in
-// code than its shorter form saves (780 rows of 24 6.9 us, 5.9 so).
-template <int P, int U, bool UA, bool DIV>
+// The two rounding sequences are chosen once for the wave's rows: a choice per row kept their chains from running side by side (780 rows
+// of 24 6.9 us, 4.7 so; 20000 of 512 11.1 -> 8.1; 81920 of 512 30 -> 23.5, 5.3 TB/s).
+template <int P, int U, bool UA>
 __global__ __launch_bounds__(256) void k_round_scale_rows_reg(int64_t rows, int32_t n, int32_t m, const half_t* __restrict__ mat,
                                                               const half_t* __restrict__ scale_y, int8_t* __restrict__ out,
                                                               half_t* __restrict__ scale_x, int bc, int32_t ld) {
@@ -633,6 +633,8 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_reg(int64_t rows, int3
             }
         }
     }
+    float s[U];
+    bool own = true;        // (the same for the whole wave)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         float mx = 0.0f;
@@ -641,17 +643,21 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_reg(int64_t rows, int3
 #pragma unroll
             for (int e = 0; e < 8; ++e) mx = fmaxf(fabsf((float)xv[u][p][e] * (float)sv[u][p][e]), mx);
         mx = __builtin_bit_cast(float, wave_max_u32_uniform(__builtin_bit_cast(uint32_t, mx)));      // (non-negative floats order as their bits)
-        const float s = (float)((double)mx / 127.0);
-        const int64_t row = row0 + u;
-        if (row < rows) {
-            const float y = 1.0f / s;
-            const bool own = !DIV && own_scale_in_range(s);       // (the same for the whole wave)
-            if (lane == 0) scale_x[row] = (half_t)s;
+        s[u] = (float)((double)mx / 127.0);
+        own = own && own_scale_in_range(s[u]);
+        if (lane == 0 && row0 + u < rows) scale_x[row0 + u] = (half_t)s[u];
+    }
+    auto finish = [&](auto ownc) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t row = row0 + u;
+            if (row >= rows) break;
+            const float y = 1.0f / s[u];
 #pragma unroll
             for (int p = 0; p < P; ++p) {
                 const int32_t j = lane * 8 + p * 512;
                 if (j < ld) {        // (past the end of the row: zeros)
-                    const uint2_t w = round8_own_scale(xv[u][p], sv[u][p], s, y, own);
+                    const uint2_t w = round8_own_scale(xv[u][p], sv[u][p], s[u], y, decltype(ownc)::value);
                     int8_t* dst = out + row * ld + j;
                     if constexpr (!UA) {
                         *reinterpret_cast<uint2_t*>(dst) = w;
@@ -663,7 +669,9 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_reg(int64_t rows, int3
                 }
             }
         }
-    }
+    };
+    if (own) finish(std::true_type{});
+    else finish(std::false_type{});
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1196,15 +1204,8 @@ int cpmk_gemm_backward_round_scale_ld(int32_t batch, int32_t n, int32_t m, const
                 hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(rows, 4 * U)), dim3(256), 0, (hipStream_t)stream, rows, n, m, (const half_t*)mat,
                                    (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, broad_cast_y, ld);
             };
-            if constexpr (P == 1) {
-                if (vec16 ? m <= 64 : m <= 512) {
-                    if (vec16) run(k_round_scale_rows_reg<P, U, false, true>);
-                    else run(k_round_scale_rows_reg<P, U, true, true>);
-                    return;
-                }
-            }
-            if (vec16) run(k_round_scale_rows_reg<P, U, false, false>);
-            else if constexpr (P > 1) run(k_round_scale_rows_reg<P, U, true, false>);
+            if (vec16) run(k_round_scale_rows_reg<P, U, false>);
+            else run(k_round_scale_rows_reg<P, U, true>);
         };
         if (m <= 512) go(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
         else if (m <= 1024) go(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});

@@ -86,9 +86,10 @@ def _quantize_cols(x, both: bool, row_scale=None):
 
 
 def _dims(quantA, quantB, aT, bT):
-    M = quantA.size(2) if aT else quantA.size(1)
-    K = quantA.size(1) if aT else quantA.size(2)
-    N = quantB.size(1) if bT else quantB.size(2)
+    _, M, K = quantA.shape
+    if aT:
+        M, K = K, M
+    N = quantB.shape[1 if bT else 2]
     return M, K, N
 
 
@@ -295,15 +296,16 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
     x 32 434 / 398 (512 MB and more; 2048 x 2048 x 32 and K = 1024 about even).  Rows of A that are not whole 16-byte pieces are
     copied always."""
     M, K, N = _dims(A, B, aT, bT)
+    bA, bB = A.shape[0], B.shape[0]
     if K % 64 == 0 and N % 8 == 0 and M * K < 2 ** 31 and N * K < 2 ** 31:
-        large = K > 128 and K <= 512 and M * N * max(A.size(0), B.size(0)) > 2 ** 27
+        large = 128 < K <= 512 and M * N * max(bA, bB) > 2 ** 27
         # (short K: the product is bound by writing its output)
-        if aT and ((N * max(B.size(0) // A.size(0), 1) > 8192 and K > 128) or large and N > 512 or M % 8 != 0):
+        if aT and ((N * max(bB // bA, 1) > 8192 and K > 128) or large and N > 512 or M % 8 != 0):
             A, aT = _transposed_copy(A), False
         if not bT and (M > 8192 and K > 128 or large and M > 2048):
             B, bT = _transposed_copy(B), True
-    out = torch.empty((max(A.size(0), B.size(0)), M, N), dtype=torch.half, device=A.device)
-    gemm_fp16(N, K, M, B.size(0), A.size(0), bT, aT, B.data_ptr(), A.data_ptr(), out.data_ptr(), cur_stream())
+    out = torch.empty((max(bA, bB), M, N), dtype=torch.half, device=A.device)
+    gemm_fp16(N, K, M, bB, bA, bT, aT, B.data_ptr(), A.data_ptr(), out.data_ptr(), cur_stream())
     return out
 
 
@@ -365,9 +367,10 @@ class GEMMFloat(torch.autograd.Function):
 
 
 def bmm(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool, int8: bool = False, fused: bool = True) -> torch.Tensor:
-    assert A.ndim == 3
-    assert B.ndim == 3
-    assert A.size(1 if aT else 2) == B.size(2 if bT else 1), "operands of different contraction lengths"      # (B would be read past its end)
+    size_A, size_B = A.shape, B.shape
+    assert len(size_A) == 3
+    assert len(size_B) == 3
+    assert size_A[1 if aT else 2] == size_B[2 if bT else 1], "operands of different contraction lengths"      # (B would be read past its end)
     if int8:
         return GEMMInt8.apply(A, aT, B, bT, fused, torch.is_grad_enabled())
     return GEMMFloat.apply(A, aT, B, bT)

@@ -27,13 +27,14 @@ __device__ inline half_t gelu1(half_t h) {
     return (half_t)(x * __builtin_amdgcn_rcpf(1.0f + e));
 }
 
-// Bound by memory.  Results of 50 to 92 MB are stored without the non-temporal hint: the quantiser that reads them next finds
-// them in the last-level cache (256 MB, which holds the input too).  gelu alone, and with the quantiser of its result, hint /
-// plain, the input from memory and in the cache: 67 MB 22.9 / 22.0, 56.0 / 53.9 and 19.9 / 19.8, 51.8 / 49.3 us; 84 MB 28.1 /
-// 28.3, 71.8 / 68.5 and 24.6 / 24.3, 67.3 / 63.4.  Smaller ones are slower from the cache (25 MB 10.0 / 10.0, 28.6 / 27.1 and 5.7 /
-// 8.3, 25.6 / 25.5; 34 MB 12.8 / 12.3, 31.6 / 30.6 and 10.5 / 10.9, 29.2 / 30.1), larger ones in either way (101 MB 33.1 / 35.3,
-// 86.1 / 83.1 and 28.9 / 29.0, 73.4 / 73.8; 151 MB 48.4 / 51.6, 112.2 / 110.0 and 42.3 / 50.7, 104.8 / 110.0).
-static bool gelu_keeps(int64_t total) { return total >= 24 << 20 && total <= 44 << 20; }
+// Bound by memory.  Results of up to 6 MB and of 50 to 92 MB are stored without the non-temporal hint: the quantiser that reads them
+// next finds them in L2 or in the last-level cache (256 MB, which holds the input too).  gelu alone, and with the quantiser of its
+// result, hint / plain, the input from memory and in the cache: 4 MB 3.7 / 3.7, 16.3 / 15.6 and 3.8 / 3.8, 16.5 / 15.6 us; 67 MB 22.9 /
+// 22.0, 56.0 / 53.9 and 19.9 / 19.8, 51.8 / 49.3; 84 MB 28.1 / 28.3, 71.8 / 68.5 and 24.6 / 24.3, 67.3 / 63.4.  Those between are slower
+// from the cache (8 MB 3.8 / 4.3, 16.9 / 18.4 and 3.8 / 4.2, 18.3 / 18.1; 25 MB 10.0 / 10.0, 28.6 / 27.1 and 5.7 / 8.3, 25.6 / 25.5;
+// 34 MB 12.8 / 12.3, 31.6 / 30.6 and 10.5 / 10.9, 29.2 / 30.1), larger ones in either way (101 MB 33.1 / 35.3, 86.1 / 83.1 and 28.9 /
+// 29.0, 73.4 / 73.8; 151 MB 48.4 / 51.6, 112.2 / 110.0 and 42.3 / 50.7, 104.8 / 110.0).
+static bool gelu_keeps(int64_t total) { return total <= 3 << 20 || (total >= 24 << 20 && total <= 44 << 20); }
 
 __global__ __launch_bounds__(256) void k_gelu(int64_t total, const half_t* mat, half_t* out, int vec, int keep) {
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;

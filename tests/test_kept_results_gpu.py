@@ -27,16 +27,16 @@ def test_layernorm(gpu, shape, bias):
     assert torch.equal(one, two)
 
 
-@pytest.mark.parametrize("total", [(24 << 20) - 8, 24 << 20, (24 << 20) + 5, 44 << 20, (44 << 20) + 3])
+@pytest.mark.parametrize("total", [3 << 20, (3 << 20) + 8, (24 << 20) - 8, 24 << 20, (24 << 20) + 5, 44 << 20, (44 << 20) + 3])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_gelu(gpu, total, shift):
-    """One call against pieces too small to be kept, bit for bit; off 16-byte boundaries too."""
+    """One call against pieces of another choice, bit for bit; off 16-byte boundaries too."""
     print("kept gelu", total, shift, flush=True)
     g = torch.Generator(device=gpu).manual_seed(total)
     x = torch.randn(total + 8, generator=g, device=gpu).half()[shift:shift + total]
     out, pieces = torch.full((total + 16,), 77.0, dtype=torch.half, device=gpu), torch.empty(total, dtype=torch.half, device=gpu)
     ck.gelu_forward(1, total, x.data_ptr(), out[shift:].data_ptr(), stream())
-    step = 1 << 22
+    step = 1 << (22 if total > 1 << 24 else 20)
     for i in range(0, total, step):
         ck.gelu_forward(1, min(step, total - i), x[i:].data_ptr(), pieces[i:].data_ptr(), stream())
     assert torch.equal(out[shift:shift + total], pieces)

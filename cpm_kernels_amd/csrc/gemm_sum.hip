@@ -87,9 +87,12 @@ static int gemm_sum_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t 
     const int64_t cus = compute_units();
     if (!f16) {
         // Bound by the LDS reads of the K loop.  Beside the int32 accumulators a wave holds as many fp32 sums, so its share of
-        // the tile is 64 x 64 where the plain product's is 128 x 64: 256x128 tiles of eight waves.  10240 x 4096 outputs over
-        // 8 entries of 512: 196 us, against 287 us for the products one by one and 149 us for adding them up; waves of
-        // 128 x 64, one per SIMD, 316 us (their accumulators have to be carried between the two register files to be folded).
+        // Bound by the LDS traffic of the K loop.  Beside the int32 accumulators a wave holds as many fp32 sums, so its share of
+        // the tile is 64 x 64 where the plain product's is 128 x 64: 256x128 tiles of eight waves, whose fragment reads alone take as
+        // long as their products (the DMA's writes come on top).  10240 x 4096 outputs over 8 entries of 512: 194 us (202 with an entry's
+        // product folded between two slabs instead of under the next entry's first products), against 287 us for the products one by
+        // one and 149 us for adding them up; waves of 128 x 64, one per SIMD, 316 us (their accumulators have to be carried
+        // between the two register files to be folded).
         if (ceil_div(n, 256) * ceil_div(m, 128) * groups * 4 >= cus * 3) return launch_dma<4, 2, 2, 2, 128, I8, 2, 0, 16>(a, groups, st);
         // too few of them for most compute units: 128x128 tiles, two workgroups a compute unit when there are more than compute
         // units (1024 x 2560 over 4 x 256: 12.0 us; 15.2 as 256x128), else the deeper ring (2048 x 2048 over 8 x 512: 29.8 us; two stages 31.3)

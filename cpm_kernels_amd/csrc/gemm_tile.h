@@ -614,13 +614,25 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
     // One pass: the AR x HC MFMAs of column half `jh`, order pinned.  Between them the other set of column
     // fragments is read from k-step `qks` of stage `qs`; with REFILL the row fragments are refilled from
     // k-step `nks` of stage `ns`; and ND further memory operations (`memop`) are spread over the pass.
+    // FIRST (kEpiSumI8): the pass starts the next entry's products; a tile's finished product goes into the sums right before its
+    // accumulators start again from zero, eight vector operations under each MFMA of the wave beside it on the SIMD.
     constexpr int NMP = AR * HC;
-    auto pass = [&](auto jhc, int qs, int qks, auto refillc, int ns, int nks, auto&& memop, auto nd_c) __attribute__((always_inline)) {
+    float fsx[FOLD ? AR : 1];            // FOLD: the scales of this lane's rows for the entry whose products are in the accumulators
+    auto fold = [&](int i, int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) facc[i][j][e] = __builtin_fmaf((float)acc[i][j][e], fsx[i], facc[i][j][e]);
+        asm volatile("" : "+v"(facc[i][j]));
+    };
+    auto pass = [&](auto jhc, int qs, int qks, auto refillc, int ns, int nks, auto&& memop, auto nd_c, auto firstc) __attribute__((always_inline)) {
         constexpr int jh = decltype(jhc)::value, ND = decltype(nd_c)::value;
-        constexpr bool REFILL = decltype(refillc)::value;
+        constexpr bool REFILL = decltype(refillc)::value, FIRST = decltype(firstc)::value;
         static_for<0, NMP>([&](auto xc) __attribute__((always_inline)) {
             constexpr int x = decltype(xc)::value;
             constexpr int i = x / HC, jj = x % HC;
+            if constexpr (FIRST) {
+                fold(i, jh * HC + jj);
+                acc[i][jh * HC + jj] = acc_t{0, 0, 0, 0};
+            }
             // MFMA "A" = column-operand rows, "B" = row-operand rows: lane l, register e of the
             // result is output row l%16, column (l/16)*4 + e of the 16x16 tile
             if constexpr (F16)      // 64 bytes of K are 32 halves: same lane -> byte assignment as the int8 MFMA
@@ -658,15 +670,16 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
     int cur = ring0;
     // tail slab index: it + LD - nk of the next tile, or nk - 1 of this one
     const int tmul = ahead ? 1 : 0, tadd = ahead ? LD - nk : nk - 1;
-    auto slab = [&](int it, auto tailc) __attribute__((always_inline)) {
+    auto slab = [&](int it, auto tailc, auto firstc) __attribute__((always_inline)) {
         constexpr bool TAIL = decltype(tailc)::value;
         const int nxt = cur + 1 == NST ? 0 : cur + 1;
         static_for<0, KS - 1>([&](auto ksc) __attribute__((always_inline)) {
             constexpr int ks = decltype(ksc)::value;
-            pass(I0{}, cur, ks, std::false_type{}, 0, 0, no_memop, I0{});
-            pass(I1{}, cur, ks + 1, std::true_type{}, cur, ks + 1, no_memop, I0{});
+            constexpr std::integral_constant<bool, decltype(firstc)::value && ks == 0> start{};
+            pass(I0{}, cur, ks, std::false_type{}, 0, 0, no_memop, I0{}, start);
+            pass(I1{}, cur, ks + 1, std::true_type{}, cur, ks + 1, no_memop, I0{}, start);
         });
-        pass(I0{}, cur, KS - 1, std::false_type{}, 0, 0, no_memop, I0{});       // the last reads of stage cur
+        pass(I0{}, cur, KS - 1, std::false_type{}, 0, 0, no_memop, I0{}, std::false_type{});       // the last reads of stage cur
         __builtin_amdgcn_sched_barrier(0);
         wait_vmcnt<(NST - 2) * CNT>();       // slab it + 1 has landed (with fewer slabs than stages it had before the loop)
         __syncthreads();
@@ -675,7 +688,7 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
         const int tgt = cur + LD >= NST ? cur + LD - NST : cur + LD;       // the stage slab it + LD belongs to
         pass(I1{}, nxt, 0, std::true_type{}, nxt, 0,
              [&](auto dc) __attribute__((always_inline)) { dma1(dc, kt2, tailc, tgt); },
-             std::integral_constant<int, CNT>{});
+             std::integral_constant<int, CNT>{}, std::false_type{});
         if constexpr (SUM) dma.advance();
         __builtin_amdgcn_sched_barrier(0);
         cur = nxt;
@@ -683,32 +696,34 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
     int it = 0;
     if constexpr (SUM) dma.seek(false, min(LD, nk - 1));
     if constexpr (FOLD) {
-        int in_entry = 0, entry = 0;
-        auto fold = [&]() __attribute__((always_inline)) {       // the entry's product is complete: into the sums
-            if (++in_entry == nkb) {
-                in_entry = 0;
-#pragma unroll
-                for (int i = 0; i < AR; ++i) {
-                    const float sx = (float)*reinterpret_cast<const half_t*>(stg + (entry * TR * 32 + i * 16 + r16) * 2);
-#pragma unroll
-                    for (int j = 0; j < AC; ++j)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            facc[i][j][e] = __builtin_fmaf((float)acc[i][j][e], sx, facc[i][j][e]);
-                            acc[i][j][e] = 0;
-                        }
-                }
-                ++entry;
+        // One loop for the slabs before the tail and the tail's (what they request follows Pk / Qk), two bodies: an entry's first slab
+        // and its others.
+        static_assert(KS > 1, "an entry starts in a k-step of its own");
+        auto next_slab = [&](auto firstc) __attribute__((always_inline)) {
+            if (it == nk - LD) {
+                dma.retarget();
+                dma.seek(true, ahead ? 0 : nk - 1);
             }
+            slab(it, std::false_type{}, firstc);
+            ++it;
         };
-        for (; it < nk - LD; ++it) { slab(it, std::false_type{}); fold(); }
-        dma.retarget();
-        dma.seek(true, ahead ? 0 : nk - 1);
-        for (; it < nk; ++it) { slab(it, std::true_type{}); fold(); }
+#pragma unroll
+        for (int i = 0; i < AR; ++i) fsx[i] = 0.0f;
+        for (int entry = 0; entry < a.nsum; ++entry) {
+            next_slab(std::true_type{});
+#pragma unroll
+            for (int i = 0; i < AR; ++i) fsx[i] = (float)*reinterpret_cast<const half_t*>(stg + (entry * TR * 32 + i * 16 + r16) * 2);
+            for (int s = 1; s < nkb; ++s) next_slab(std::false_type{});
+        }
+#pragma unroll
+        for (int i = 0; i < AR; ++i)
+#pragma unroll
+            for (int j = 0; j < AC; ++j) fold(i, j);
     } else {
-        for (; it < nk - LD; ++it) slab(it, std::false_type{});       // slabs LD .. nk-1 of this tile follow
+        auto plain = [&](int t, auto tailc) __attribute__((always_inline)) { slab(t, tailc, std::false_type{}); };
+        for (; it < nk - LD; ++it) plain(it, std::false_type{});       // slabs LD .. nk-1 of this tile follow
         if constexpr (SUM) dma.seek(true, ahead ? 0 : nk - 1);
-        tail_slabs<REST>(dma, it, slab);                              // then the tail's
+        tail_slabs<REST>(dma, it, plain);                              // then the tail's
     }
     if (!ahead) wait_vmcnt<0>();         // drain the clamped loads before the ring is reused
     ring = cur;                          // (ring0 + nk) % NST: where the next tile's slab 0 is, or will be put

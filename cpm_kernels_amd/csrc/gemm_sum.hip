@@ -86,7 +86,6 @@ static int gemm_sum_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t 
     a.kmagic = (uint32_t)(((1ull << 32) + nkb - 1) / nkb);
     const int64_t cus = compute_units();
     if (!f16) {
-        // Bound by the LDS reads of the K loop.  Beside the int32 accumulators a wave holds as many fp32 sums, so its share of
         // Bound by the LDS traffic of the K loop.  Beside the int32 accumulators a wave holds as many fp32 sums, so its share of
         // the tile is 64 x 64 where the plain product's is 128 x 64: 256x128 tiles of eight waves, whose fragment reads alone take as
         // long as their products (the DMA's writes come on top).  10240 x 4096 outputs over 8 entries of 512: 194 us (202 with an entry's

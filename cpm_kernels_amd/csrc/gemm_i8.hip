@@ -25,7 +25,6 @@
 // The tile kernel also serves the fp16 product of kernels/gemm.py:188-256 (cpmk_gemm_fp16): the
 // same bytes of K per lane feed v_mfma_f32_16x16x32_f16 / v_mfma_f32_32x32x16_f16, with fp32 accumulators.
 #include "gemm_tile.h"
-#include "gemm_short.h"
 
 namespace cpmk {
 
@@ -495,10 +494,6 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     if (m == 0 || n == 0) return 0;
     if (out == nullptr || (k > 0 && any_null(A, B))) return CPMK_EBADARG;
     if (k > (1 << 30)) return CPMK_ETOOBIG;
-    if (aT == 0 && bT != 0 && k <= 128) {       // both stored (K, rows), a short contraction
-        const int rc = gemm_short(m, k, n, batch, batchA == 1 ? 0 : (int64_t)m * k, batchB == 1 ? 0 : (int64_t)n * k, A, B, out, st);
-        if (rc >= 0) return rc;
-    }
     if (batch > 65535) {      // (grid z: at most 65535 batch entries per call)
         for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
             const int32_t nb = (int32_t)(batch - b0 < 65535 ? batch - b0 : 65535);

@@ -20,7 +20,10 @@ namespace cpmk {
 // exchanges the per-column maxima.  Lane (cg = tid % 8, rg = tid / 8) holds 8 columns of the 8
 // consecutive rows rg*8 .. rg*8+7, so that its int8 results are 8 contiguous bytes in either
 // output layout.
-// (two 512-thread workgroups share a compute unit: at most 128 registers per lane)
+// Bound by the two memory phases of a workgroup -- all of its reads, then all of its writes -- around the wait for its team: without one
+// (128 x 512 x 1024) it runs at 5.3 TB/s, with one at 4.0.  Three workgroups a compute unit (at most 80 registers per lane) while some
+// wait: 8 x 10240 x 512 transposed 43.4 -> 37.1 us, with both outputs 48.4 -> 45.2, with row scales 51.5 -> 44.7; 16 x 4096 x 1024 57 -> 49.8;
+// 8 x 4096 x 512, one round of the device, 19.2 -> 17.6.  Two a compute unit: 39.4, 46.8, 47.3, 52.7, 17.7; four (64 registers): 39.3, 50.3, 44.1, 50.9, 18.2.
 // NTH: the tile's 128-byte row segments are whole cache lines (m % 64 == 0, the matrix on a 128-byte boundary): the input is
 // read with the non-temporal hint.  Elsewhere a line is shared with the neighbouring tile and has to stay in L2 for it.
 // UA: any m and alignment: a piece inside its row still moves whole, at whatever address it lies (global accesses need
@@ -40,7 +43,7 @@ struct ColQuantArgs {
 constexpr int kOutT = 1, kOutN = 2;
 
 template <int NT, int OUT, bool NTH, bool UA, bool SCALED>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_col_quantize_team(ColQuantArgs a, int32_t tiles_per_batch, int32_t parts,
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_col_quantize_team(ColQuantArgs a, int32_t tiles_per_batch, int32_t parts,
                                                           uint32_t nteams, XchLaunch xl) {
     constexpr bool TRANSPOSED = (OUT & kOutT) != 0, NATURAL = (OUT & kOutN) != 0;
     const int32_t n = a.n, m = a.m;
@@ -49,8 +52,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     constexpr int LPR = 8, R = 8, COLS = 64, ROWS = NT / LPR * R;
     uint64_t* const xch = xl.region;
     const uint32_t tag = xl.tag;
-    __shared__ float lds[(NT / 64 + 1) * COLS];
-    __shared__ float tot[COLS];
+    __shared__ __attribute__((aligned(16))) union { float f[NT / 64 * COLS]; uint16_t h[NT / 64 * COLS]; } wmax;       // column maxima of each wave
+    __shared__ float xmax[NT];                                    // the team's column maxima, [wave][column]
+    __shared__ __attribute__((aligned(16))) float colscale[COLS], colrcp[COLS];
+    __shared__ bool all_normal;
     __shared__ __attribute__((aligned(16))) int8_t tbuf[TRANSPOSED ? COLS * ROWS : 16];       // the transposed int8 tile on its way out
     const int tid = threadIdx.x, cg = tid % LPR, rg = tid / LPR;
     XchMember me;
@@ -67,14 +72,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 #pragma unroll
         for (int p = 0; p < R; ++p) sx[p] = row0 + p < n ? (float)rs[row0 + p] : 0.0f;
     }
+    // one lane offset beside a scalar address per row of the lane (n * m < 2^31: the offset in bytes of a row within the matrix fits)
+    const half_t* const tbase = mat + boff + (int64_t)part * ROWS * m;
+    const uint32_t loff = ((uint32_t)(rg * 8) * (uint32_t)m + (uint32_t)col0) * 2u;
     half8_t v[R];
 #pragma unroll
     for (int p = 0; p < R; ++p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[p][e] = (half_t)0.0f;
+        const half_t* const src = reinterpret_cast<const half_t*>(reinterpret_cast<const char*>(tbase + (int64_t)p * m) + loff);
         if constexpr (UA) {
             if (row0 + p < n) {
-                const half_t* src = mat + boff + ((uint32_t)(row0 + p) * (uint32_t)m + (uint32_t)col0);
                 if (col0 + 8 <= m) {
                     v[p] = load_half8_any(src);
                 } else if (col0 < m) {
@@ -82,94 +90,93 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
                 }
             }
         } else if (row0 + p < n && col0 < m) {
-            const half8_t* src = reinterpret_cast<const half8_t*>(mat + boff + ((uint32_t)(row0 + p) * (uint32_t)m + (uint32_t)col0));
-            v[p] = NTH ? __builtin_nontemporal_load(src) : *src;        // read once; the int8 output below is what the next kernel wants in cache
+            const half8_t* src8 = reinterpret_cast<const half8_t*>(src);
+            v[p] = NTH ? __builtin_nontemporal_load(src8) : *src8;        // read once; the int8 output below is what the next kernel wants in cache
         }
     }
-    float mx[8];
+    // The maxima over the rows of a wave, then over the workgroup's waves: thread i < COLS ends up with that of column i.
+    float M = 0.0f;
     if constexpr (SCALED) {
+        float mx[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) mx[e] = 0.0f;
 #pragma unroll
         for (int p = 0; p < R; ++p)
 #pragma unroll
             for (int e = 0; e < 8; ++e) mx[e] = fmaxf(mx[e], fabsf((float)v[p][e] * sx[p]));       // (skips NaN products, as the reference's fmaxf does)
+        coltile_reduce_to<NT, LPR, 1, true>(mx, wmax.f, [&](int, float r) { M = r; });
     } else {
-        // |x| maxima of the lane's 8 columns as integers; a NaN among them (rare) repeats the maximum in
+        // |x| of the lane's 8 columns as integers, two to a register all the way through; a NaN among them (rare) repeats the maximum in
         // floating point, which skips NaN elements
         ushort8_t um = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int p = 0; p < R; ++p) um = absbits_max(um, v[p]);
-        half8_t hm = __builtin_bit_cast(half8_t, um);
         if (absbits_max_of(um) > 0x7c00u) {
-            hm = __builtin_elementwise_abs(v[0]);
+            half8_t hm = __builtin_elementwise_abs(v[0]);
 #pragma unroll
             for (int p = 1; p < R; ++p) hm = __builtin_elementwise_max(hm, __builtin_elementwise_abs(v[p]));
-        }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) mx[e] = (float)hm[e];
-    }
-    if (parts == 1) {
-        coltile_reduce<NT, LPR, 1, true>(mx, lds);       // every lane: the maxima of its 8 columns
-    } else {
-        uint64_t* team_slots = xch + (size_t)team * parts * kXchVals;
-        // this part's maxima go straight from the reduction to its slot
-        coltile_reduce_to<NT, LPR, 1, true>(mx, lds, [&](int i, float r) { xch_post(team_slots + (size_t)part * kXchVals, i, r, tag); });
-        if (tid < COLS) {
-            const uint64_t deadline = wall_clock64() + kXchTimeoutTicks;
-            float M = 0.0f;
-            bool ok = true;
-            for (int32_t q0 = 0; q0 < parts; q0 += 8) {
-                float x[8];
-                ok &= xch_gather<8>(team_slots, parts, q0, tid, tag, deadline, x);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) M = fmaxf(M, x[j]);       // maxima are >= 0: absent parts (zeros) do not matter
-            }
-            tot[tid] = ok ? M : __builtin_nanf("");
-            if (!ok) xch_flag(xl, kXchStatusTimeout);
+            for (int e = 0; e < 8; ++e) hm[e] = hm[e] != hm[e] ? (half_t)0.0f : hm[e];       // (nothing but NaN)
+            um = __builtin_bit_cast(ushort8_t, hm);
         }
+        um = lanes_mod8_max(um);
+        if ((tid & 63) < LPR) *reinterpret_cast<ushort8_t*>(wmax.h + (tid >> 6) * COLS + cg * 8) = um;
         __syncthreads();
+        if (tid < COLS) {
+            uint16_t r = wmax.h[tid];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) mx[e] = tot[cg * 8 + e];
-    }
-
-    half8_t sh;
-    float s[8], y[8];
-    // (columns past the matrix's edge get a scale of 1: theirs of 0 would send the whole wave through the long rounding sequence,
-    // 32 x 359 with row scales 10.8 us, 8.9 so; 8 x 4096 x 500 25.9 -> 23.6)
-    if (col0 + 8 > m) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            if (col0 + e >= m) mx[e] = 127.0f;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        if constexpr (SCALED) {
-            s[e] = (float)((double)mx[e] / 127.0);       // float / double constant, as the reference writes it
-            sh[e] = (half_t)s[e];
-        } else {
-            sh[e] = scale_from_absmax(mx[e]);
-            s[e] = (float)sh[e];
+            for (int w = 1; w < NT / 64; ++w) r = max(r, wmax.h[w * COLS + tid]);
+            M = (float)__builtin_bit_cast(half_t, r);
         }
-        y[e] = 1.0f / s[e];
     }
-    if (part == 0 && rg == 0) {
-        if constexpr (UA) {
-            if (col0 + 8 <= m) {
-                store_half8_any(scale + (int64_t)b * m + col0, sh);
-            } else if (col0 < m) {
-                store_half8_head_any(scale + (int64_t)b * m + col0, m & 7, sh);
+    if (parts > 1) {
+        // The packets of the team's parts are dealt to the waves, four to a thread, which all wait at the same time: one wave asking for
+        // eight at a time held 40 registers and went through them in turn.
+        uint64_t* team_slots = xch + (size_t)team * parts * kXchVals;
+        if (tid < COLS) xch_post(team_slots + (size_t)part * kXchVals, tid, M, tag);
+        const int w = tid >> 6;
+        float x[4];
+        const bool ok = xch_gather<4>(team_slots, parts, w * 4, tid & 63, tag, wall_clock64() + kXchTimeoutTicks, x);
+        const float m4 = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));       // maxima are >= 0: absent parts (zeros) do not matter
+        xmax[tid] = ok ? m4 : __builtin_nanf("");
+        if (!ok) xch_flag(xl, kXchStatusTimeout);
+        __syncthreads();
+    }
+    // One wave: the maximum of each column, its scale and the reciprocal, for all lanes of the column (a lane's 16 divisions, if
+    // each made its own eight columns', were a quarter of the kernel's instructions).
+    if (tid < COLS) {
+        if (parts > 1) {
+            M = xmax[tid];
+#pragma unroll
+            for (int w = 1; w < NT / 64; ++w) {
+                const float x = xmax[w * COLS + tid];
+                M = x > M || x != x ? x : M;       // (a NaN, where a packet did not arrive, stays)
             }
-        } else if (col0 < m) {
-            *reinterpret_cast<half8_t*>(scale + (int64_t)b * m + col0) = sh;
         }
+        // (columns past the matrix's edge get a scale of 1: theirs of 0 would send the whole tile through the long rounding sequence,
+        // 32 x 359 with row scales 10.8 us, 8.9 so; 8 x 4096 x 500 25.9 -> 23.6)
+        const int32_t col = ct * COLS + tid;
+        if (col >= m) M = 127.0f;
+        const float s1 = SCALED ? (float)((double)M / 127.0) : 0.0f;       // float / double constant, as the reference writes it
+        const half_t sh = SCALED ? (half_t)s1 : scale_from_absmax(M);
+        const float s = SCALED ? s1 : (float)sh;
+        colscale[tid] = s;
+        colrcp[tid] = 1.0f / s;
+        const bool normal = SCALED ? own_scale_in_range(s) : scale_is_normal(sh);
+        const bool every = __builtin_amdgcn_ballot_w64(!normal) == 0;
+        if (tid == 0) all_normal = every;
+        if (part == 0 && col < m) scale[(int64_t)b * m + col] = sh;
     }
+    __syncthreads();
 
     uint32_t q[R][2];       // [row p][columns 0-3 | 4-7], one byte each
-    bool normal = true;
+    if (all_normal) {    // every scale of the tile's columns is a normal number: the short rounding sequence
+        float s[8], y[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) normal = normal && (SCALED ? own_scale_in_range(s[e]) : scale_is_normal(sh[e]));
-    if (__builtin_amdgcn_ballot_w64(!normal) == 0) {    // every scale of the wave's columns is a normal number: the short rounding sequence
+        for (int e = 0; e < 8; ++e) {
+            y[e] = colrcp[cg * 8 + e];
+            s[e] = SCALED ? colscale[cg * 8 + e] : 0.0f;
+        }
 #pragma unroll
         for (int p = 0; p < R; ++p) {
             uint32_t t[8];
@@ -178,7 +185,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
             const half8_t vh = __builtin_bit_cast(half8_t, vp);
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                t[e] = SCALED ? quant_i8_own_fp32_scale_bits((float)vh[e] * sx[p], s[e], y[e]) : quant_i8_own_scale_bits((float)vh[e], s[e], y[e]);
+                t[e] = SCALED ? quant_i8_own_fp32_scale_bits((float)vh[e] * sx[p], s[e], y[e]) : quant_i8_own_scale_bits((float)vh[e], y[e]);
             q[p][0] = pack4_i8((int32_t)t[0], (int32_t)t[1], (int32_t)t[2], (int32_t)t[3]);
             q[p][1] = pack4_i8((int32_t)t[4], (int32_t)t[5], (int32_t)t[6], (int32_t)t[7]);
             __builtin_amdgcn_sched_barrier(0);      // one row at a time: interleaving all 64 elements costs registers
@@ -188,22 +195,26 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         for (int p = 0; p < R; ++p) {
             int32_t t[8];
             int4_t vp = __builtin_bit_cast(int4_t, v[p]);
-            if constexpr (SCALED) asm volatile("" : "+v"(vp));             // (the products of the maxima are not to be kept for here)
+            asm volatile("" : "+v"(vp));             // (what was computed for the maxima is not to be kept for here)
             const half8_t vh = __builtin_bit_cast(half8_t, vp);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) t[e] = SCALED ? quant_i8((float)vh[e] * sx[p], s[e]) : quant_i8_rcp((float)vh[e], s[e], y[e]);
+            for (int e = 0; e < 8; ++e) {
+                t[e] = quant_i8(SCALED ? (float)vh[e] * sx[p] : (float)vh[e], colscale[cg * 8 + e]);
+                __builtin_amdgcn_sched_barrier(0);      // one division at a time: this rare path is not to set the register count
+            }
             q[p][0] = pack4_i8(t[0], t[1], t[2], t[3]);
             q[p][1] = pack4_i8(t[4], t[5], t[6], t[7]);
-            if constexpr (SCALED) __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     if constexpr (NATURAL) {
         if (col0 < a.ld_n) {
-            int8_t* const obase = a.out_n + (int64_t)b * n * a.ld_n;
+            int8_t* const obase = a.out_n + (int64_t)b * n * a.ld_n + (int64_t)part * ROWS * a.ld_n;
+            const uint32_t ooff = (uint32_t)(rg * 8) * (uint32_t)a.ld_n + (uint32_t)col0;
 #pragma unroll
             for (int p = 0; p < R; ++p)
                 if (row0 + p < n) {
-                    int8_t* dst = obase + ((uint32_t)(row0 + p) * (uint32_t)a.ld_n + (uint32_t)col0);
+                    int8_t* dst = obase + (int64_t)p * a.ld_n + ooff;
                     if constexpr (UA) {       // (ld_n is m, or a multiple of 16 beyond it: the piece across the matrix's edge ends in zeros then)
                         if (col0 + 8 <= a.ld_n) store_byte8_any(dst, q[p][0], q[p][1]);
                         else store_byte8_head_any(dst, a.ld_n & 7, q[p][0], q[p][1]);
@@ -355,7 +366,7 @@ static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st) {
     // a team here only exchanges one maximum per column and gathers it in a loop over the parts, so
     // it may be larger than the teams of the kernels that keep per-part values in registers
     // (16384 rows; far fewer workgroups than are resident at once, which is what progress needs)
-    constexpr int64_t kColMaxParts = 32;
+    constexpr int64_t kColMaxParts = 32;       // four for each of a workgroup's eight waves
     const int64_t tiles = ceil_div(p.out_n ? p.ld_n : m, 64), parts = ceil_div(n, 512);
     // rows of whole 16-byte pieces in aligned buffers: 16-byte accesses; any other width or alignment: the same kernel moving
     // its columns one by one (the transposed output runs along n either way)

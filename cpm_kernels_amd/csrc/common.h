@@ -178,7 +178,13 @@ __device__ inline float block_sum(float v, float* red) {
 // like the reference's fmaxf (cuda/gemm.cu:68-72).
 typedef uint16_t ushort8_t __attribute__((ext_vector_type(8)));
 __device__ inline ushort8_t absbits_max(ushort8_t m, half8_t x) {
-    const uint4_t b = __builtin_bit_cast(uint4_t, x) & 0x7fff7fffu;
+    uint4_t b = __builtin_bit_cast(uint4_t, x);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t t = b[i] & 0x7fff7fffu;
+        asm("" : "+v"(t));          // (else the compiler takes the AND apart by halves and puts them together again: four operations for two)
+        b[i] = t;
+    }
     return __builtin_elementwise_max(m, __builtin_bit_cast(ushort8_t, b));
 }
 __device__ inline uint32_t absbits_max_of(ushort8_t m) {
@@ -228,21 +234,21 @@ __device__ inline int32_t quant_i8_rcp(float x, float s, float y) {
 
 // The short form for a scale that comes from the data it divides and is a normal fp16 number:
 //     s = fp16(absmax / 127),  |x| <= absmax   =>   |x / s| <= 127 * (1 + 2^-11),
-// so nothing saturates and the residual is always finite.  q + 1.5 * 2^23 lands in [2^23, 2^24),
-// where the fp32 grid is the integers: the one round-to-nearest-even of that addition is rint(q), and
-// the low byte of the sum's bit pattern is the two's-complement int8.  A NaN element (which the
+// so nothing saturates.  With X and S the 11-bit integers of the two, x / s is either exactly k + 1/2 or at least 1 / (2 S) >= 2^-12
+// away from it, and the fp32 division the reference rounds keeps it there (its grid is 2^-17 at 127).  x * y is within 2^-16 of the quotient: the
+// one rounding of the fma below, to the grid of 2^-12 that [2^11, 2^12) has, makes an exact tie of a tie and leaves everything else on
+// its side.  q + 1.5 * 2^23 lands in [2^23, 2^24), where the fp32 grid is the integers: the one round-to-nearest-even of that addition
+// is rint(q), and the low byte of the sum's bit pattern is the two's-complement int8.  A NaN element (which the
 // absmax ignores) propagates as a quiet NaN whose low byte is 0, the value the long form gives it.
 // Equality with quant_i8 for every such (absmax, x) pair is proven by enumeration in
-// tests/native/fused_round_check.c.  Returns the fp32 bit pattern; its low byte is the result.
+// tests/native/grid_round_check.c.  Returns the fp32 bit pattern; its low byte is the result.
 __device__ inline bool scale_is_normal(half_t sh) {
     const uint16_t b = __builtin_bit_cast(uint16_t, sh);
     return b >= 0x0400u && b <= 0x7bffu;
 }
-__device__ inline uint32_t quant_i8_own_scale_bits(float x, float s, float y) {
-    const float q0 = __builtin_fmaf(x, y, 0.0f);     // x * y (the sign of a zero does not matter below); as an fma the fp16 -> fp32 conversion of x folds into the instruction
-    const float r = __builtin_fmaf(-s, q0, x);
-    const float q1 = __builtin_fmaf(r, y, q0);
-    float t = q1 + 12582912.0f;
+__device__ inline uint32_t quant_i8_own_scale_bits(float x, float y) {
+    const float q = __builtin_fmaf(x, y, 3072.0f);      // 1.5 * 2^11; as an fma the fp16 -> fp32 conversion of x folds into the instruction
+    float t = q + 12579840.0f;                          // to 1.5 * 2^23, exactly
     asm("" : "+v"(t));          // the sum must exist as a rounded fp32 number
     return __builtin_bit_cast(uint32_t, t);
 }

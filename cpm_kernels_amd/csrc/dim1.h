@@ -122,6 +122,25 @@ __device__ __forceinline__ float lanes_mod8_combine(float v) {
     return op(__builtin_bit_cast(float, (uint32_t)q[0]), __builtin_bit_cast(float, (uint32_t)q[1]));
 }
 
+// The same for maxima of eight unsigned 16-bit numbers, two to a register.
+__device__ __forceinline__ ushort8_t lanes_mod8_max(ushort8_t v) {
+    uint4_t b = __builtin_bit_cast(uint4_t, v);
+    typedef uint16_t ushort2_t __attribute__((ext_vector_type(2)));
+    auto op = [](uint32_t x, uint32_t y) __attribute__((always_inline)) {
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(ushort2_t, x), __builtin_bit_cast(ushort2_t, y)));
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t x = b[i];
+        x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, true));      // row_ror:8
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        x = op(r[0], r[1]);
+        const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        b[i] = op(q[0], q[1]);
+    }
+    return __builtin_bit_cast(ushort8_t, b);
+}
+
 // Reduce NV groups of 8 per-lane column partials over all rows of the tile.  On return every
 // lane holds the totals of its own 8 columns.  `lds` must hold (NT/64 + 1) * LPR*8 * NV floats.
 template <int NT, int LPR, int NV, bool IS_MAX>

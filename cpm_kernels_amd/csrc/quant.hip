@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA && NV > 
                     asm volatile("" : "+v"(ci));     // keeps the fp32 conversions of the two paths apart (hoisted above the branch they hold NV * 8 registers)
                     const half8_t ch = __builtin_bit_cast(half8_t, ci);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) q[e] = quant_i8_own_scale_bits((float)ch[e], s, y);
+                    for (int e = 0; e < 8; ++e) q[e] = quant_i8_own_scale_bits((float)ch[e], y);
                     uint2_t w;
                     w.x = pack4_i8((int32_t)q[0], (int32_t)q[1], (int32_t)q[2], (int32_t)q[3]);
                     w.y = pack4_i8((int32_t)q[4], (int32_t)q[5], (int32_t)q[6], (int32_t)q[7]);
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(256) void k_rows_wg(RowsArgs a, int64_t row0) {
             int32_t q[8];
             if (normal) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) q[e] = (int32_t)quant_i8_own_scale_bits((float)h[e], s, y);
+                for (int e = 0; e < 8; ++e) q[e] = (int32_t)quant_i8_own_scale_bits((float)h[e], y);
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) q[e] = quant_i8_rcp((float)h[e], s, y);

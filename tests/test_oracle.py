@@ -401,6 +401,20 @@ def test_short_rounding_of_the_fused_quantisers_exhaustively(tmp_path):
     assert r.stdout.startswith("23568 rows, 989078256 pairs, 0 mismatches"), r.stdout
 
 
+def test_rounding_on_the_grid_exhaustively(tmp_path):
+    """Two operations give the integers of the divide-then-round of cuda/gemm.cu:16 for every fp16 value a row (column) of a normal
+    scale can hold: tests/native/grid_round_check.c enumerates them with the same IEEE operations on the host."""
+    import os, shutil, subprocess
+    if shutil.which("gcc") is None:
+        pytest.skip("no gcc")
+    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "grid_round_check.c")
+    exe = str(tmp_path / "grid_round_check")
+    subprocess.run(["gcc", "-O2", "-ffp-contract=off", "-mfma", "-mf16c", "-msse4.1", "-fopenmp", src, "-o", exe, "-lm"], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.startswith("23377 scales, 981085934 pairs, 0 mismatches"), r.stdout
+
+
 def test_calc_scale_skips_nan_elements_of_either_kind():
     """cuda/gemm.cu:68-72 takes the maximum with the device's fmaxf, which drops any NaN operand:
     the scale is that of the row with its NaN elements, quiet or signalling, replaced by zeros."""

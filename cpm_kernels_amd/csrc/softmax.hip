@@ -18,9 +18,99 @@ constexpr float kLog2e = 1.4426950408889634f;
 // exp(x - M) as one fma and one v_exp_f32: exp2(x*log2e - M*log2e).
 __device__ inline float exp_shift(float x, float mlog2e) { return __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, -mlog2e)); }
 
-// The softmax of the columns of one register-resident tile, in place in v (rows past n hold -inf).
+// LDS floats of softmax_cols: maxima of each wave (packed halves) and of the tile, sums of each wave and reciprocals of the tile's
+template <int NT, int LPR>
+constexpr int softmax_lds() { return (NT / 64 + 1) * LPR * 8 + NT / 64 * LPR * 4 + LPR * 8; }
+
+// max of two pairs of halves.  Written out because the compiler puts a canonicalisation of both operands in front of its own; what that
+// would change are signalling NaN, and a column with any NaN is NaN whatever its maximum.
+__device__ __forceinline__ uint32_t pk_max_f16(uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_pk_max_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// The softmax of the columns of one register-resident tile, in place in v (rows past n hold -inf).  `lds`: softmax_lds floats, whose
+// parts are each written once, so that no barrier is needed before they are written again but one between two calls.
+// Bound by the vector instructions as much as by memory, so what is the same for all rows of a column -- maximum times log2(e), reciprocal of the sum --
+// is made once for the tile, and maxima stay pairs of halves through the wave (1024 x 512 x 512 198 -> 179 us, 256 of them 59.4 -> 53.4;
+// 64 x 500 x 500 15.7 -> 14.4; 1024 x 1024 x 1024, at the rate of a copy, 746 -> 742).
 template <int NT, int LPR, int R>
 __device__ __forceinline__ void softmax_cols(half8_t (&v)[R], float* lds) {
+    constexpr int NW = NT / 64, COLS = LPR * 8;
+    float* const wsum = lds;                                               // [wave][column]
+    float* const tot = lds + NW * COLS;                                    // reciprocals
+    uint16_t* const wmax = reinterpret_cast<uint16_t*>(tot + COLS);        // [wave][column]
+    float* const tmax = tot + COLS + NW * COLS / 2;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, cg = tid % LPR;
+    uint4_t um = __builtin_bit_cast(uint4_t, v[0]);
+#pragma unroll
+    for (int p = 1; p < R; ++p) {
+        const uint4_t x = __builtin_bit_cast(uint4_t, v[p]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) um[i] = pk_max_f16(um[i], x[i]);
+    }
+    if constexpr (LPR == 8) {       // lanes l, l ^ 8, l ^ 16, l ^ 32, as in lanes_mod8_combine
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t x = um[i];
+            x = pk_max_f16(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, true));
+            const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+            x = pk_max_f16(r[0], r[1]);
+            const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+            um[i] = pk_max_f16(q[0], q[1]);
+        }
+    } else {
+#pragma unroll
+        for (int o = LPR; o < 64; o <<= 1)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) um[i] = pk_max_f16(um[i], (uint32_t)__shfl_xor((int)um[i], o, kWave));
+    }
+    if (lane < LPR) *reinterpret_cast<uint4_t*>(wmax + w * COLS + lane * 8) = um;
+    __syncthreads();
+    if (tid < COLS) {
+        float M = -1e6f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) M = fmaxf(M, (float)__builtin_bit_cast(half_t, wmax[i * COLS + tid]));
+        tmax[tid] = M * kLog2e;
+    }
+    __syncthreads();
+    float mx[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx[e] = tmax[cg * 8 + e];
+
+    float ex[R][8], s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = 0.0f;
+#pragma unroll
+    for (int p = 0; p < R; ++p) {
+        const uint4_t raw = __builtin_bit_cast(uint4_t, v[p]);
+        const bool all_ninf = (raw.x == 0xfc00fc00u) & (raw.y == 0xfc00fc00u) & (raw.z == 0xfc00fc00u) & (raw.w == 0xfc00fc00u);
+        if (__builtin_amdgcn_ballot_w64(!all_ninf) == 0) {      // wave-uniform: nothing but -inf here
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ex[p][e] = 0.0f;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                ex[p][e] = exp_shift((float)v[p][e], mx[e]);   // rows >= n hold -inf -> 0
+                s[e] += ex[p][e];
+            }
+        }
+    }
+    coltile_reduce_to<NT, LPR, 1, false>(s, wsum, [&](int i, float r) { tot[i] = 1.0f / (r + 1e-10f); });
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = tot[cg * 8 + e];
+#pragma unroll
+    for (int p = 0; p < R; ++p)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[p][e] = round_f16(ex[p][e] * s[e]);
+}
+
+// The same with every lane working out its own eight columns' maxima and reciprocals: more instructions, of which tiles that share their cache
+// lines in 16-byte pieces get quicker where there are many (softmax_dispatch).  `lds`: (NT / 64 + 1) * LPR * 8 floats.
+template <int NT, int LPR, int R>
+__device__ __forceinline__ void softmax_cols_by_lane(half8_t (&v)[R], float* lds) {
     half8_t hm = v[0];
 #pragma unroll
     for (int p = 1; p < R; ++p) hm = __builtin_elementwise_max(hm, v[p]);
@@ -67,11 +157,11 @@ __device__ __forceinline__ void softmax_cols(half8_t (&v)[R], float* lds) {
 // exponentials are exactly 0.
 // MODE 0: 16-byte accesses, non-temporal where a tile's row segments are whole cache lines; 1: 16-byte accesses without
 // the hint (rows that do not start on 128-byte boundaries); 2: any m and alignment, element by element (dim1.h).
-template <int NT, int LPR, int R, int MODE = 0>
+template <int NT, int LPR, int R, int MODE = 0, bool BY_LANE = false>
 __global__ __launch_bounds__(NT) void k_softmax_tile(int32_t n, int32_t m, int32_t tiles_per_batch,
                                                      const half_t* inp, half_t* out) {
     using T = ColTile<NT, LPR, R>;
-    __shared__ float lds[(T::NW + 1) * T::COLS];
+    __shared__ __attribute__((aligned(16))) float lds[softmax_lds<NT, LPR>()];
     const uint32_t t = xcd_remap(blockIdx.x, gridDim.x);
     const uint32_t b = t / tiles_per_batch, ct = t - b * tiles_per_batch;
     const int32_t col0 = ct * T::COLS + (threadIdx.x % LPR) * 8;
@@ -80,8 +170,17 @@ __global__ __launch_bounds__(NT) void k_softmax_tile(int32_t n, int32_t m, int32
     half8_t v[R];
     coltile_load<NT, LPR, R, LPR == 8 && MODE == 0, MODE == 2>(v, inp + boff, n, m, col0, (half_t)(-__builtin_inff()));
 
-    softmax_cols<NT, LPR, R>(v, lds);
+    if constexpr (BY_LANE) softmax_cols_by_lane<NT, LPR, R>(v, lds);
+    else softmax_cols<NT, LPR, R>(v, lds);
     coltile_store<NT, LPR, R, LPR == 8 && MODE == 0, MODE == 2>(v, out + boff, n, m, col0);
+}
+
+// The next tile from a counter.  The address goes through a vector register: of one that is the same for all lanes the compiler makes
+// a single atomic whose result it reads at once, and that wait covers the loads of the next tile too.
+__device__ __forceinline__ uint32_t take_tile(unsigned int* counter) {
+    uint32_t zero = 0;
+    asm volatile("" : "+v"(zero));
+    return __hip_atomic_fetch_add(counter + zero, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The same for many tiles per compute unit: persistent workgroups, each wave fetching its share
@@ -107,7 +206,7 @@ __global__ __launch_bounds__(NT) void k_softmax_stream(int32_t n, int32_t m, int
     constexpr int RPP = NT / LPR;
     extern __shared__ __attribute__((aligned(16))) int8_t dyn[];        // NT*R*16 bytes of staging, the reduction scratch, one word for the next tile
     float* lds = reinterpret_cast<float*>(dyn + NT * R * 16);
-    uint32_t* s_next = reinterpret_cast<uint32_t*>(lds + (T::NW + 1) * T::COLS);
+    uint32_t* s_next = reinterpret_cast<uint32_t*>(lds + softmax_lds<NT, LPR>());
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int8_t* stage = dyn + wave * (R * 1024) + lane * 16;
@@ -152,12 +251,12 @@ __global__ __launch_bounds__(NT) void k_softmax_stream(int32_t n, int32_t m, int
         __builtin_amdgcn_sched_barrier(0);
         if (tn < ntiles) issue(tn);
         uint32_t after = 0;
-        if (tid == 0) after = G + atomicAdd(ctr, 1u);                   // the tile after the next; used only after the arithmetic
+        if (tid == 0) after = take_tile(ctr);                   // the tile after the next; used only after the arithmetic
         __builtin_amdgcn_sched_barrier(0);
         softmax_cols<NT, LPR, R>(v, lds);
         __builtin_amdgcn_sched_barrier(0);
         wait_vmcnt<0>();            // the next tile has landed; the previous tile's stores finished long ago
-        if (tid == 0) *s_next = after;
+        if (tid == 0) *s_next = G + after;
         __syncthreads();
         const uint32_t tnn = __builtin_amdgcn_readfirstlane(*s_next);
         __builtin_amdgcn_sched_barrier(0);
@@ -384,10 +483,10 @@ static int launch_rows(int32_t rows, int32_t n, const half_t* x, half_t* y, hipS
     return launch_status();
 }
 
-template <int NT, int LPR, int R, int MODE>
+template <int NT, int LPR, int R, int MODE, bool BY_LANE = false>
 static void launch_tile(int32_t batch, int32_t n, int32_t m, const half_t* inp, half_t* out, hipStream_t st) {
     const int32_t tiles = (int32_t)ceil_div(m, LPR * 8);
-    hipLaunchKernelGGL((k_softmax_tile<NT, LPR, R, MODE>), dim3((unsigned)((int64_t)tiles * batch)), dim3(NT), 0, st, n, m,
+    hipLaunchKernelGGL((k_softmax_tile<NT, LPR, R, MODE, BY_LANE>), dim3((unsigned)((int64_t)tiles * batch)), dim3(NT), 0, st, n, m,
                        tiles, inp, out);
 }
 
@@ -396,8 +495,7 @@ static void launch_tile(int32_t batch, int32_t n, int32_t m, const half_t* inp, 
 // for the launch's counters: the caller then records a kernel that needs none.
 template <int NT, int LPR, int R>
 static int launch_stream(int32_t batch, int32_t n, int32_t m, const half_t* inp, half_t* out, hipStream_t st) {
-    using T = ColTile<NT, LPR, R>;
-    constexpr int smem = NT * R * 16 + (T::NW + 1) * T::COLS * (int)sizeof(float) + 16;
+    constexpr int smem = NT * R * 16 + softmax_lds<NT, LPR>() * (int)sizeof(float) + 16;
     static_assert(smem <= 160 * 1024, "LDS of one compute unit");
     auto kern = k_softmax_stream<NT, LPR, R>;
     static std::atomic<bool> lds_enabled[64];
@@ -421,8 +519,8 @@ static bool launch_tile_r(int r, int32_t batch, int32_t n, int32_t m, const half
     if (r <= 1) launch_tile<NT, LPR, 1, MODE>(batch, n, m, inp, out, st);
     else if (r <= 2) launch_tile<NT, LPR, 2, MODE>(batch, n, m, inp, out, st);
     else if (r <= 4) launch_tile<NT, LPR, 4, MODE>(batch, n, m, inp, out, st);
-    else if (r <= 8) launch_tile<NT, LPR, 8, MODE>(batch, n, m, inp, out, st);
-    else return false;
+    else if (r > 8) return false;
+    else if constexpr (NT != 512 || MODE != 2) launch_tile<NT, LPR, 8, MODE>(batch, n, m, inp, out, st);
     return true;
 }
 
@@ -489,7 +587,15 @@ static int softmax_dispatch(int32_t batch, int32_t n, int32_t m, const void* inp
         }
         ok = with_mode([&](auto mc) {
             constexpr int MODE = decltype(mc)::value;
-            if (n <= 64 * 8 && m >= 64) return launch_tile_r<512, 8, MODE>((int)ceil_div(n, 64), batch, n, m, x, y, st);
+            // 257 to 512 rows.  Rows off 16-byte boundaries: 1024 threads of four rows (1024 x 500 x 500 243 us, 261 as 512 of eight; 128 x 333 x
+            // 1001 38 and 40).  Rows that start on 16-byte boundaries but not on cache lines, more tiles than are resident at once: each lane for
+            // itself (1024 x 504 x 504 192 us, else 208 and with 1024 threads 198; 256 x 480 x 480 40.7, 43.0 and 42.8; with 512 tiles, 64 x 480 x
+            // 480, 13.0, 11.8 and 12.1).
+            if (MODE == 1 && n > 256 && n <= 512 && m >= 64 && ceil_div(m, 64) * batch > 2 * (int64_t)compute_units()) {
+                launch_tile<512, 8, 8, 1, true>(batch, n, m, x, y, st);
+                return true;
+            }
+            if (n <= (MODE == 2 ? 256 : 512) && m >= 64) return launch_tile_r<512, 8, MODE>((int)ceil_div(n, 64), batch, n, m, x, y, st);
             if (n <= 128 * 8 && m >= 64) return launch_tile_r<1024, 8, MODE>((int)ceil_div(n, 128), batch, n, m, x, y, st);
             if (n <= 256 * 8 && m >= 32) return launch_tile_r<1024, 4, MODE>((int)ceil_div(n, 256), batch, n, m, x, y, st);
             if (n <= 512 * 8) return launch_tile_r<1024, 2, MODE>((int)ceil_div(n, 512), batch, n, m, x, y, st);

@@ -520,6 +520,15 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     // (Tiles of the general kernel waste less of narrow ones: 80 heads of 150 x 150 6.7 us there, 9.0 here; 228 of 402 x 402, 58 and 33.)
     const bool wide = (reinterpret_cast<uintptr_t>(out) & 3u) == 0 && (!odd || m >= 192);
     const bool p_kmajor = !bT, q_kmajor = aT != 0;
+    // A depth up to 128: a kernel of its own -- but where the output's rows are not whole cache lines and it exceeds half of the last-level
+    // cache, the tile kernel, whose large tiles share fewer of the lines (1024 of 500 x 500, K = 64 149 us, 162 there; 100 of 1000 x 1000 52.6 and
+    // 56.4; 250 of 500 x 500 32.7 and 25.1), unless those cover much more than the matrix (1500 of 300 x 300 179 and 113).
+    if (!p_kmajor && !q_kmajor && k > 0 && k <= 128) {
+        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256), mid = ceil_div(n, 128) * ceil_div(m, 128), outs = (int64_t)batch * n * m;
+        const bool large = big * 8 <= mid * 3 && big * batch * 4 >= (int64_t)compute_units() * 3;
+        if (m % 64 == 0 || outs <= 1 << 26 || !large)
+            if (const int rc = gemm_f16_short(m, k, n, batchA, batchB, A, B, out, st); rc >= 0) return rc;
+    }
     if (p_kmajor && q_kmajor && wide && k > 0 && (k % 32 == 0) && aligned16(A) && aligned16(B) &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;

@@ -3,7 +3,7 @@
 //
 // Bound by reading Q once.  A workgroup is one tile of 64 rows x 128 columns; it brings the next 64 rows of K into registers while
 // the slab in LDS is multiplied, so pieces need no alignment, and four workgroups a compute unit have 96 KB in flight between them.
-// Batch x depth x columns for 64 rows: 256 x 512 x 512 30.4 -> 28.0 us (6.0 TB/s), 512 of them 65.5 -> 58.2, 64 10.6 -> 8.9, 100 x 700 x 700 33.7 -> 27.7,
+// Batch x depth x columns for 64 rows: 256 x 512 x 512 30.4 -> 29.8 us (5.6 TB/s), 512 of them 65.5 -> 58.2, 64 10.6 -> 8.9, 100 x 700 x 700 33.7 -> 27.7,
 // 300 x 130 x 130 20.8 -> 7.4 (on the general kernel before), 128 x 400 x 400 13.5 -> 10.9.
 #include "common.h"
 
@@ -145,8 +145,9 @@ int gemm_f16_low(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB
     const int64_t tc = ceil_div(m, 128);
     if (tc * batch >= 1 << 24 || (int64_t)n * k >= (1ll << 31) || (int64_t)m * (k + 64) >= (1ll << 31)) return -1;       // (a launch holds fewer than 2^32 threads)
     a.tiles_c = (uint32_t)tc; a.tiles = (uint32_t)(tc * batch);
-    // (the hint from 64 MB on: 64 of 64 x 1024 x 1024 23.9 us, 26.4 without; 16 of them 15.0 and 12.9)
-    if (lines && q >= 1 << 25) hipLaunchKernelGGL(k_gemm_low<true>, dim3(a.tiles), dim3(256), 0, st, a);
+    // (the hint where Q exceeds what the last-level cache keeps for its next reader: 512 of 64 x 512 x 512 58.1 us, 69 without; 256 of them
+    // 28.4 and 29.8 by themselves, but the training step that reads Q again 528 and 524)
+    if (lines && q >= 3ll << 25) hipLaunchKernelGGL(k_gemm_low<true>, dim3(a.tiles), dim3(256), 0, st, a);
     else hipLaunchKernelGGL(k_gemm_low<false>, dim3(a.tiles), dim3(256), 0, st, a);
     return launch_status();
 }

@@ -50,7 +50,7 @@ def test_unaligned_buffers(shift):
     assert (po[:shift] == 0).all() and (po[shift + batch * m * n:] == 0).all()
 
 
-@pytest.mark.parametrize("batch,k,m", [(127, 512, 512), (129, 512, 512), (770, 512, 512), (400, 500, 500), (1000, 300, 300)])
+@pytest.mark.parametrize("batch,k,m", [(383, 512, 512), (385, 512, 512), (770, 512, 512), (400, 500, 500), (1000, 300, 300)])
 def test_large_operands(batch, k, m):
     a, b = _operands(batch, batch, 64, k, m, batch)
     out = ct.bmm(a, False, b, False, int8=False)

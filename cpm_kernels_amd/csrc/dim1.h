@@ -146,7 +146,7 @@ __device__ __forceinline__ ushort8_t lanes_mod8_max(ushort8_t v) {
 template <int NT, int LPR, int NV, bool IS_MAX>
 __device__ inline void coltile_reduce(float (&v)[NV * 8], float* lds) {
     constexpr int NW = NT / 64, COLS = LPR * 8, W = COLS * NV;
-    if constexpr (LPR == 8 && !IS_MAX) {        // (for the maxima of the column quantiser the lane-swap form measured 4 % slower than the shuffles)
+    if constexpr (LPR == 8 && !IS_MAX) {        // (for fp32 maxima the lane-swap form measured 4 % slower than the shuffles; those of halves go two to a register, lanes_mod8_max)
 #pragma unroll
         for (int e = 0; e < NV * 8; ++e) v[e] = lanes_mod8_combine<IS_MAX>(v[e]);
     } else {
@@ -190,7 +190,7 @@ template <int NT, int LPR, int NV, bool IS_MAX, class F>
 __device__ inline void coltile_reduce_to(float (&v)[NV * 8], float* lds, F&& sink) {
     constexpr int NW = NT / 64, COLS = LPR * 8, W = COLS * NV;
     static_assert(NW > 1, "one wave has nothing to combine");
-    if constexpr (LPR == 8 && !IS_MAX) {        // (for the maxima of the column quantiser the lane-swap form measured 4 % slower than the shuffles)
+    if constexpr (LPR == 8 && !IS_MAX) {        // (for fp32 maxima the lane-swap form measured 4 % slower than the shuffles; those of halves go two to a register, lanes_mod8_max)
 #pragma unroll
         for (int e = 0; e < NV * 8; ++e) v[e] = lanes_mod8_combine<IS_MAX>(v[e]);
     } else {

@@ -194,20 +194,29 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 6))) void
             __builtin_amdgcn_sched_barrier(0);      // one row at a time: interleaving all 64 elements costs registers
         }
     } else {
+        // A scale below the normal numbers, or not finite.  Four columns at a time, so that scales and reciprocals are eight registers
+        // (8 x 4096 x 512 with one such column a tile @@ us; one IEEE division an element, one element at a time, 25.7).
 #pragma unroll
-        for (int p = 0; p < R; ++p) {
-            int32_t t[8];
-            int4_t vp = __builtin_bit_cast(int4_t, v[p]);
-            asm volatile("" : "+v"(vp));             // (what was computed for the maxima is not to be kept for here)
-            const half8_t vh = __builtin_bit_cast(half8_t, vp);
+        for (int h = 0; h < 2; ++h) {
+            const float4_t s = *reinterpret_cast<const float4_t*>(colscale + cg * 8 + h * 4), y = *reinterpret_cast<const float4_t*>(colrcp + cg * 8 + h * 4);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                t[e] = quant_i8(SCALED ? (float)vh[e] * sx[p] : (float)vh[e], colscale[cg * 8 + e]);
-                __builtin_amdgcn_sched_barrier(0);      // one division at a time: this rare path is not to set the register count
+            for (int p = 0; p < R; ++p) {
+                int32_t t[4];
+                int4_t vp = __builtin_bit_cast(int4_t, v[p]);
+                asm volatile("" : "+v"(vp));             // (what was computed for the maxima is not to be kept for here)
+                const half8_t vh = __builtin_bit_cast(half8_t, vp);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (SCALED) {
+                        t[e] = quant_i8((float)vh[h * 4 + e] * sx[p], s[e]);
+                        __builtin_amdgcn_sched_barrier(0);      // one division at a time: infinite products only, which are not to set the register count
+                    } else {
+                        t[e] = quant_i8_rcp((float)vh[h * 4 + e], s[e], y[e]);
+                    }
+                }
+                q[p][h] = pack4_i8(t[0], t[1], t[2], t[3]);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            q[p][0] = pack4_i8(t[0], t[1], t[2], t[3]);
-            q[p][1] = pack4_i8(t[4], t[5], t[6], t[7]);
-            __builtin_amdgcn_sched_barrier(0);
         }
     }
     if constexpr (NATURAL) {

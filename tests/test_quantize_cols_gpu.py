@@ -1,8 +1,11 @@
 """The column quantiser's two ways of rounding: what sends a tile of 64 columns to the longer one, and what that may cost."""
+import numpy as np
 import pytest
 import torch
 
 import cpm_kernels_amd.kernels as ck
+import oracle
+from util import assert_bits_equal, to_gpu, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -71,3 +74,35 @@ def test_empty_columns_cost_nothing(gpu, scaled):
     t = _quickest([_quantise(x, rs)[0], _quantise(y, rs)[0]])
     print("ordinary %.1f us, with empty columns %.1f us" % tuple(t), flush=True)
     assert t[1] <= 1.15 * t[0], t
+
+
+@pytest.mark.parametrize("n", [40, 1030])
+def test_every_scale_below_the_normal_numbers(gpu, n):
+    """One column for each largest magnitude whose scale is subnormal or 0, one with an infinity among them: the oracle's divisions."""
+    rng = np.random.default_rng(n)
+    top = np.arange(1, 8192, dtype=np.uint16)          # up to 127 * 2^-14 and a little more
+    x = (rng.integers(0, 65536, (1, n, top.size)) % (top.astype(np.int64) + 1)).astype(np.uint16)
+    x[0, 0] = top
+    x |= (rng.integers(0, 2, x.shape) << 15).astype(np.uint16)
+    x = x.view(np.float16)
+    x[0, n // 2, 77] = np.inf
+    d = to_gpu(x)
+    want = oracle.gemm_calc_scale_transpose(x)
+    q_want = oracle.gemm_round_transpose(x, want)
+    for tr in (False, True):
+        s2 = torch.full((1, top.size), -1.0, dtype=torch.half, device=gpu)
+        q2 = torch.full((1, top.size, n) if tr else x.shape, 77, dtype=torch.int8, device=gpu)
+        ck.gemm_quantize_cols(1, n, top.size, d.data_ptr(), s2.data_ptr(), q2.data_ptr(), tr, torch.cuda.current_stream().cuda_stream)
+        assert_bits_equal(to_np(s2), want, "scales")
+        assert_bits_equal(to_np(q2), np.ascontiguousarray(q_want.transpose(0, 2, 1)) if tr else q_want, "int8 (transposed=%s)" % tr)
+
+
+def test_scales_below_the_normal_numbers_cost_little(gpu):
+    """One such column in every tile: 23.9 us against 15.7 when the longer rounding divided element by element, 18.7 through the reciprocal."""
+    b, n, m = 8, 4096, 512
+    x = torch.randn((b, n, m), device=gpu).half()
+    y = x.clone()
+    y[:, :, ::64] *= 1e-4
+    t = _quickest([_quantise(x)[0], _quantise(y)[0]])
+    print("ordinary %.1f us, with columns of a subnormal scale %.1f us" % tuple(t), flush=True)
+    assert t[1] <= 1.3 * t[0], t

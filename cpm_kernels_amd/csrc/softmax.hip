@@ -513,14 +513,18 @@ static int launch_stream(int32_t batch, int32_t n, int32_t m, const half_t* inp,
     return e ? e : rc2;
 }
 
+// false, and nothing launched: more rows than this form of the tile is made for
 template <int NT, int LPR, int MODE>
 static bool launch_tile_r(int r, int32_t batch, int32_t n, int32_t m, const half_t* inp, half_t* out,
                           hipStream_t st) {
+    // off 16-byte boundaries 257 to 512 rows are quicker as four rows of 1024 threads (1024 x 500 x 500 243 us, 261 as eight of 512; 128 x 333 x
+    // 1001 38 and 40)
+    constexpr int most = NT == 512 && MODE == 2 ? 4 : 8;
+    if (r > most) return false;
     if (r <= 1) launch_tile<NT, LPR, 1, MODE>(batch, n, m, inp, out, st);
     else if (r <= 2) launch_tile<NT, LPR, 2, MODE>(batch, n, m, inp, out, st);
     else if (r <= 4) launch_tile<NT, LPR, 4, MODE>(batch, n, m, inp, out, st);
-    else if (r > 8) return false;
-    else if constexpr (NT != 512 || MODE != 2) launch_tile<NT, LPR, 8, MODE>(batch, n, m, inp, out, st);
+    else if constexpr (most > 4) launch_tile<NT, LPR, 8, MODE>(batch, n, m, inp, out, st);
     return true;
 }
 
@@ -587,15 +591,14 @@ static int softmax_dispatch(int32_t batch, int32_t n, int32_t m, const void* inp
         }
         ok = with_mode([&](auto mc) {
             constexpr int MODE = decltype(mc)::value;
-            // 257 to 512 rows.  Rows off 16-byte boundaries: 1024 threads of four rows (1024 x 500 x 500 243 us, 261 as 512 of eight; 128 x 333 x
-            // 1001 38 and 40).  Rows that start on 16-byte boundaries but not on cache lines, more tiles than are resident at once: each lane for
+            // 257 to 512 rows that start on 16-byte boundaries but not on cache lines, more tiles than are resident at once: each lane for
             // itself (1024 x 504 x 504 192 us, else 208 and with 1024 threads 198; 256 x 480 x 480 40.7, 43.0 and 42.8; with 512 tiles, 64 x 480 x
             // 480, 13.0, 11.8 and 12.1).
             if (MODE == 1 && n > 256 && n <= 512 && m >= 64 && ceil_div(m, 64) * batch > 2 * (int64_t)compute_units()) {
                 launch_tile<512, 8, 8, 1, true>(batch, n, m, x, y, st);
                 return true;
             }
-            if (n <= (MODE == 2 ? 256 : 512) && m >= 64) return launch_tile_r<512, 8, MODE>((int)ceil_div(n, 64), batch, n, m, x, y, st);
+            if (n <= 512 && m >= 64 && launch_tile_r<512, 8, MODE>((int)ceil_div(n, 64), batch, n, m, x, y, st)) return true;
             if (n <= 128 * 8 && m >= 64) return launch_tile_r<1024, 8, MODE>((int)ceil_div(n, 128), batch, n, m, x, y, st);
             if (n <= 256 * 8 && m >= 32) return launch_tile_r<1024, 4, MODE>((int)ceil_div(n, 256), batch, n, m, x, y, st);
             if (n <= 512 * 8) return launch_tile_r<1024, 2, MODE>((int)ceil_div(n, 512), batch, n, m, x, y, st);

@@ -591,12 +591,22 @@ static int softmax_dispatch(int32_t batch, int32_t n, int32_t m, const void* inp
         }
         ok = with_mode([&](auto mc) {
             constexpr int MODE = decltype(mc)::value;
-            // 257 to 512 rows that start on 16-byte boundaries but not on cache lines, more tiles than are resident at once: each lane for
-            // itself (1024 x 504 x 504 192 us, else 208 and with 1024 threads 198; 256 x 480 x 480 40.7, 43.0 and 42.8; with 512 tiles, 64 x 480 x
-            // 480, 13.0, 11.8 and 12.1).
-            if (MODE == 1 && n > 256 && n <= 512 && m >= 64 && ceil_div(m, 64) * batch > 2 * (int64_t)compute_units()) {
-                launch_tile<512, 8, 8, 1, true>(batch, n, m, x, y, st);
-                return true;
+            // Each lane for itself where tiles share their cache lines and are many.  Rows on 16-byte boundaries: 257 to 512 rows with more
+            // tiles than are resident at once (1024 x 504 x 504 192 us, else 208 and with 1024 threads 198; 256 x 480 x 480 40.7, 43.0 and 42.8; with
+            // 512 tiles, 64 x 480 x 480, 13.0, 11.8 and 12.1), and 161 to 256 rows beyond the last-level cache (2250 x 200 x 504 180 us, else 195; 4500 x 192 x
+            // 200 147 and 174; 1125 x 256 x 504 128.6 and 131.4; within it, 2250 x 192 x 200, 75.8 and 73.3; 160 rows the same within 2 %, 562 x 136 x 2008
+            // 128 and 121.5).  Rows off them: from 1500 columns on, 225 to 320 rows beyond that cache (382 x
+            // 256 x 3003 271 us, else 282; 187 x 257 x 2002 84.9 and 88.5; 2250 x 240 x 505 256 and 252; 187 x 384 x 2002 124 and 125).
+            if constexpr (MODE != 0) {
+                const bool beyond = (int64_t)batch * n * m > 11ll << 23, wide_rows = m >= 1500;
+                if (m >= 64 && n > 256 && (MODE == 1 ? n <= 512 && ceil_div(m, 64) * batch > 2 * (int64_t)compute_units() : n <= 320 && beyond && wide_rows)) {
+                    launch_tile<512, 8, 8, MODE, true>(batch, n, m, x, y, st);
+                    return true;
+                }
+                if (m >= 64 && n <= 256 && beyond && (MODE == 1 ? n > 160 : n > 224 && wide_rows)) {
+                    launch_tile<512, 8, 4, MODE, true>(batch, n, m, x, y, st);
+                    return true;
+                }
             }
             if (n <= 512 && m >= 64 && launch_tile_r<512, 8, MODE>((int)ceil_div(n, 64), batch, n, m, x, y, st)) return true;
             if (n <= 128 * 8 && m >= 64) return launch_tile_r<1024, 8, MODE>((int)ceil_div(n, 128), batch, n, m, x, y, st);

@@ -12,6 +12,8 @@ pytestmark = pytest.mark.gpu
     (2, 256, 100), (2, 257, 100), (3, 512, 65), (2, 513, 66), (130, 300, 500), (2, 1, 70),
     (2, 257, 72), (64, 300, 504), (65, 300, 504), (65, 512, 504), (520, 257, 72), (65, 256, 504),
     (2, 300, 128), (3, 512, 192), (300, 257, 128),
+    # both sides of the last-level cache's line, where lanes work for themselves beyond it
+    (915, 200, 504), (916, 200, 504), (1135, 161, 505), (205, 225, 2001), (180, 257, 2002), (144, 320, 2001), (716, 256, 504),
 ])
 def test_softmax_tiles(batch, n, m):
     g = torch.Generator(device="cuda").manual_seed(batch * 7 + n + m)

@@ -5,7 +5,7 @@ import torch
 
 import cpm_kernels_amd.kernels as ck
 import oracle
-from util import assert_bits_equal, to_gpu, to_np
+from util import assert_bits_equal, quickest, to_gpu, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -46,22 +46,6 @@ def test_empty_columns(gpu, n, scaled):
     assert (q[:, 70, 5] == 0).all()
 
 
-def _quickest(calls, rounds=9, reps=20):
-    """Microseconds a call, the quickest of `rounds` runs of each, taken in turn."""
-    best = [float("inf")] * len(calls)
-    for _ in range(rounds):
-        for i, call in enumerate(calls):
-            call()
-            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            start.record()
-            for _ in range(reps):
-                call()
-            end.record()
-            end.synchronize()
-            best[i] = min(best[i], start.elapsed_time(end) * 1e3 / reps)
-    return best
-
-
 @pytest.mark.parametrize("scaled", [False, True])
 def test_empty_columns_cost_nothing(gpu, scaled):
     """A padded token in every tile: 23.7 us against 15.7 (25.0 against 18.7 with row scales) when such a column sent its tile through
@@ -71,7 +55,7 @@ def test_empty_columns_cost_nothing(gpu, scaled):
     y = x.clone()
     y[:, :, ::64] = 0
     rs = (torch.rand((b, n), device=gpu) + 0.5).half() if scaled else None
-    t = _quickest([_quantise(x, rs)[0], _quantise(y, rs)[0]])
+    t = quickest([_quantise(x, rs)[0], _quantise(y, rs)[0]])
     print("ordinary %.1f us, with empty columns %.1f us" % tuple(t), flush=True)
     assert t[1] <= 1.15 * t[0], t
 
@@ -103,6 +87,6 @@ def test_scales_below_the_normal_numbers_cost_little(gpu):
     x = torch.randn((b, n, m), device=gpu).half()
     y = x.clone()
     y[:, :, ::64] *= 1e-4
-    t = _quickest([_quantise(x)[0], _quantise(y)[0]])
+    t = quickest([_quantise(x)[0], _quantise(y)[0]])
     print("ordinary %.1f us, with columns of a subnormal scale %.1f us" % tuple(t), flush=True)
     assert t[1] <= 1.3 * t[0], t

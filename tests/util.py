@@ -57,3 +57,19 @@ def assert_close_fp16(actual, expected, rtol=1e-3, atol=0.0, max_ulp=None, what=
 
 def rand_half(rng, shape, std=1.0):
     return (rng.standard_normal(shape) * std).astype(np.float16)
+
+
+def quickest(calls, rounds=9, reps=20):
+    """Microseconds a call, the quickest of `rounds` runs of each, taken in turn."""
+    best = [float("inf")] * len(calls)
+    for _ in range(rounds):
+        for i, call in enumerate(calls):
+            call()
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(reps):
+                call()
+            end.record()
+            end.synchronize()
+            best[i] = min(best[i], start.elapsed_time(end) * 1e3 / reps)
+    return best

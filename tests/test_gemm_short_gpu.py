@@ -79,3 +79,20 @@ def test_overlapping_tiles_store_once():
     t = quickest([product(3051, 256, 256), product(6510, 160, 192)], reps=10)
     print("whole tiles %.1f us, overlapping ones %.1f us" % tuple(t), flush=True)
     assert t[1] <= 2.05 * t[0], t
+
+
+@pytest.mark.parametrize("batch_a,batch_b,m,n,k", [
+    # both sides of a quarter of the last-level cache, where overlapping tiles give way to the large ones: two slabs, a shared operand
+    (1285, 1285, 192, 136, 128), (1286, 1286, 192, 136, 128), (1286, 1286, 192, 136, 112),
+    (1285, 1, 192, 136, 64), (1286, 1, 192, 136, 64), (1, 1286, 192, 136, 64), (1, 1286, 192, 136, 120), (340, 1, 512, 200, 64), (1, 340, 512, 200, 64),
+    # rows that are not whole pieces, in and beyond a tile
+    (190, 1, 400, 450, 128), (600, 1, 400, 250, 128), (1, 1300, 198, 136, 64),
+])
+def test_overlap_and_depth_choose_the_kernel(batch_a, batch_b, m, n, k):
+    a, b = _operands(batch_a, batch_b, k, m, n, m + n)
+    batch = max(batch_a, batch_b)
+    out = torch.full((batch, n, m), float("nan"), dtype=torch.half, device="cuda")
+    ck.gemm_fp16(m, k, n, batch_a, batch_b, False, True, a.data_ptr(), b.data_ptr(), out.data_ptr(), stream())
+    assert torch.isfinite(out).all()
+    for i in (0, batch // 2, batch - 1):
+        _check(b[i % batch_b:][:1], a[i % batch_a:][:1], out[i:i + 1])

@@ -3,7 +3,7 @@
 //
 // Bound by reading Q once.  A workgroup is one tile of 64 rows x 128 columns; it brings the next 64 rows of K into registers while
 // the slab in LDS is multiplied, so pieces need no alignment, and four workgroups a compute unit have 96 KB in flight between them.
-// Batch x depth x columns for 64 rows: 256 x 512 x 512 30.4 -> 29.8 us (5.6 TB/s), 512 of them 65.5 -> 58.2, 64 10.6 -> 8.9, 100 x 700 x 700 33.7 -> 27.7,
+// Batch x depth x columns for 64 rows: 256 x 512 x 512 31.3 -> 30.8 us (5.4 TB/s), 512 of them 63.2 -> 58.7, 64 10.6 -> 8.8, 64 x 1024 x 1024 29 -> 27.3, 100 x 700 x 700 33.5 -> 28.1,
 // 300 x 130 x 130 20.8 -> 7.4 (on the general kernel before), 128 x 400 x 400 13.5 -> 10.9.
 #include "common.h"
 
@@ -130,13 +130,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 int gemm_f16_low(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, const void* A, const void* B, void* out, hipStream_t st) {
     const int32_t batch = batchA > batchB ? batchA : batchB;
     // The tile kernel's workgroups of 256 columns and three slabs in flight are the better ones for deep products, which leave few workgroups (one of 64 x 1024 x
-    // 1024 12.4 us, 11.3 here; 8 of 64 x 1500 x 1500 20.7 and 21.2; one of 64 x 8192 x 512 65 and 80), and where Q exceeds the last-level cache by far
-    // (1024 of 64 x 1024 x 1024 443 and 457) or, in rows off cache lines, at all (1024 of 64 x 500 x 500 127.5 and 134; 300 of them 42.9 and 41.8),
-    // unless its columns cover much more than the matrix (1024 of 64 x 300 x 300 69 and 58).
+    // 1024 12.1 us, 11.1 here; 8 of 64 x 1500 x 1500 20.4 and 21.2; one of 64 x 8192 x 512 65 and 80), and where Q exceeds the last-level cache by far
+    // (402 MB: 1024 of 64 x 1024 x 1024 443 and 457) or, in rows off cache lines, two thirds of it (168 MB: 1024 of 64 x 500 x 500 128.6 and 134; 300 of
+    // them 43.3 and 42.8), unless its columns cover much more than the matrix (1024 of 64 x 300 x 300 67 and 58).
     if (n < 1 || n > 64 || m < 128 || k < 1 || k > 1024) return -1;
-    const int64_t q = (int64_t)batchA * k * m;
-    const bool lines = m % 64 == 0 && (reinterpret_cast<uintptr_t>(A) & 127u) == 0;
-    if (q > (lines ? 3ll << 26 : 5ll << 24) && ceil_div(m, 256) * 256 * 4 <= ceil_div(m, 128) * 128 * 5) return -1;
+    const int64_t q = (int64_t)batchA * k * m, cover = ceil_div(m, 256) * 256;
+    const bool lines = m % 64 == 0 && (reinterpret_cast<uintptr_t>(A) & 127u) == 0, wasteful = cover * 4 > ceil_div(m, 128) * 128 * 5;
+    if (q > (lines ? 3ll << 26 : 5ll << 24) && !wasteful) return -1;
+    // Off cache lines also beyond a depth of 512 where its tiles fill their rounds of the device (400 of 64 x 1000 x 200 47.3 and 54.2 us, 126 of 64 x 700 x
+    // 900 37.5 and 40.5, 25 of 64 x 700 x 4454 37.3 and 40.0; 234 of 64 x 700 x 500, nearly two rounds, 39.5 and 42.5, 171 of them, a round and a third, 36.4 and 32.1), and
+    // where it takes one of them for what are two tiles here, beyond a depth of 896 (150 of 64 x 1000 x 200 17.3 and 19, of 64 x 600 x 200 13.3 and 13.0).
+    if (!lines && !wasteful && k > 512 && (m % 8 == 0 || m >= 256) && aligned16(A) && aligned16(B) && (reinterpret_cast<uintptr_t>(out) & 3u) == 0) {
+        const int64_t cus = compute_units(), tiles = cover / 256 * batch, rounds = ceil_div(tiles, cus);
+        if (rounds > 1 && tiles * 4 >= rounds * cus * 3) return -1;
+        if (m < 256 && k > 896 && rounds == 1 && tiles * 5 >= cus * 2) return -1;
+    }
     LowArgs a;
     a.P = (const half_t*)B; a.Q = (const half_t*)A; a.out = (half_t*)out;
     a.strideP = batchB == 1 ? 0 : (int64_t)n * k;

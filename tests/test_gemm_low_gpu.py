@@ -56,3 +56,15 @@ def test_large_operands(batch, k, m):
     out = ct.bmm(a, False, b, False, int8=False)
     for i in (0, batch // 2, batch - 1):
         _check(a[i:i + 1], b[i:i + 1], out[i:i + 1])
+
+
+# off cache lines, around the depth and the rounds of the device where the tile kernel takes over (256 tiles of 64 x 256 at a time)
+@pytest.mark.parametrize("batch,n,k,m", [(400, 64, 1000, 200), (150, 64, 1000, 200), (80, 64, 1000, 200), (400, 30, 600, 200), (300, 64, 600, 200),
+                                         (400, 64, 510, 200), (234, 64, 700, 500), (171, 64, 700, 500), (400, 64, 700, 198), (58, 2, 700, 2002)])
+def test_deep_products_choose_the_kernel(batch, n, k, m):
+    a, b = _operands(batch, batch, n, k, m, batch + k)
+    out = torch.full((batch, n, m), float("nan"), dtype=torch.half, device="cuda")
+    ck.gemm_fp16(m, k, n, batch, batch, False, False, b.data_ptr(), a.data_ptr(), out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert torch.isfinite(out).all()
+    for i in (0, batch // 2, batch - 1):
+        _check(a[i:i + 1], b[i:i + 1], out[i:i + 1])

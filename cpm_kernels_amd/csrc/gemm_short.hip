@@ -20,7 +20,9 @@ struct ShortArgs {
 };
 
 // NTS: the output is stored with the non-temporal hint.
-template <bool NTS>
+// WHOLE: the tiles do not overlap.  Elsewhere the last ones leave out the rows, and the whole pieces of them, that the tiles before store (6510 of
+// 160 x 192, K = 64 203 us with them written again, 145 so; with the choice also where nothing overlaps 1024 of 1024 x 1024 527 us, 513 so).
+template <bool NTS, bool WHOLE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_gemm_short(ShortArgs a) {
     constexpr int T = 128, SLAB = 64, ROW = T * 2;            // tile edge, rows of K at a time, bytes per row in LDS
     __shared__ __attribute__((aligned(16))) int8_t lds[2 * SLAB * ROW];
@@ -109,13 +111,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         }
     __syncthreads();
     half_t* const ob = a.out + ((int64_t)b * a.n + j0) * a.m + i0;
-    // (rows and whole pieces of them that the tiles before store: 6510 of 160 x 192, K = 64 203 us with them written again, 145 so)
-    const int32_t skip_r = (int32_t)tr * T - j0;
-    if (lc * 8 + 8 <= (int32_t)tc * T - i0) return;
 #pragma unroll
     for (int p = 0; p < 8; ++p) {
         const int r = lr + 16 * p;
-        if (r < skip_r) continue;
+        if constexpr (!WHOLE)
+            if (r < (int32_t)tr * T - j0 || lc * 8 + 8 <= (int32_t)tc * T - i0) continue;
         const half8_t h = *reinterpret_cast<const half8_t*>(lds + r * ROW + ((lc ^ (r & 15)) << 4));
         half_t* const dst = ob + (int64_t)r * a.m + lc * 8;
         if constexpr (NTS) __builtin_nontemporal_store(h, reinterpret_cast<half8_t*>(dst));
@@ -138,8 +138,10 @@ int gemm_f16_short(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batc
     // Whole cache lines and more of them than the last-level cache holds beside what is read: 512 of 512 x 512 52 us with the hint, 70 without,
     // 400 of them 41 and 47, 1024 of 1024 x 1024 485 and 516; 256 of 512 x 512, which the next kernel finds in the cache, 26.6 either way.
     const bool lines = m % 64 == 0 && (reinterpret_cast<uintptr_t>(out) & 127u) == 0, large = (int64_t)batch * n * m >= 3ll << 25;
-    if (lines && large) hipLaunchKernelGGL(k_gemm_short<true>, dim3(a.tiles), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(k_gemm_short<false>, dim3(a.tiles), dim3(256), 0, st, a);
+    const bool whole = n % 128 == 0 && m % 128 == 0;
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(a.tiles), dim3(256), 0, st, a); };
+    if (lines && large) go(whole ? k_gemm_short<true, true> : k_gemm_short<true, false>);
+    else go(whole ? k_gemm_short<false, true> : k_gemm_short<false, false>);
     return launch_status();
 }
 

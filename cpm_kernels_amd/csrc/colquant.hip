@@ -41,6 +41,9 @@ struct ColQuantArgs {
     int32_t ld_t, ld_n;
 };
 constexpr int kOutT = 1, kOutN = 2;
+// Parts of a team: the packets of all of them are dealt to the waves of a workgroup once, kColPackets to a wave.
+constexpr int kColThreads = 512, kColPackets = 4;
+constexpr int64_t kColMaxParts = kColThreads / 64 * kColPackets;
 
 template <int NT, int OUT, bool NTH, bool UA, bool SCALED>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_col_quantize_team(ColQuantArgs a, int32_t tiles_per_batch, int32_t parts,
@@ -132,11 +135,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 6))) void
     if (parts > 1) {
         // The packets of the team's parts are dealt to the waves, four to a thread, which all wait at the same time: one wave asking for
         // eight at a time held 40 registers and went through them in turn.
+        static_assert(NT / 64 * kColPackets >= kColMaxParts, "a part beyond these would be left out of the maxima");
         uint64_t* team_slots = xch + (size_t)team * parts * kXchVals;
         if (tid < COLS) xch_post(team_slots + (size_t)part * kXchVals, tid, M, tag);
         const int w = tid >> 6;
-        float x[4];
-        const bool ok = xch_gather<4>(team_slots, parts, w * 4, tid & 63, tag, wall_clock64() + kXchTimeoutTicks, x);
+        static_assert(kColPackets == 4, "the maximum below");
+        float x[kColPackets];
+        const bool ok = xch_gather<kColPackets>(team_slots, parts, w * kColPackets, tid & 63, tag, wall_clock64() + kXchTimeoutTicks, x);
         const float m4 = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));       // maxima are >= 0: absent parts (zeros) do not matter
         xmax[tid] = ok ? m4 : __builtin_nanf("");
         if (!ok) xch_flag(xl, kXchStatusTimeout);
@@ -375,10 +380,9 @@ int cpmk_gemm_round_transpose(int32_t, int32_t, int32_t, const void*, const void
 template <bool SCALED>
 static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st) {
     const int32_t n = p.n, m = p.m;
-    // a team here only exchanges one maximum per column and gathers it in a loop over the parts, so
-    // it may be larger than the teams of the kernels that keep per-part values in registers
-    // (16384 rows; far fewer workgroups than are resident at once, which is what progress needs)
-    constexpr int64_t kColMaxParts = 32;       // four for each of a workgroup's eight waves
+    // a team here exchanges one maximum per column, dealt to all waves, so it may be larger than the teams of the kernels that keep
+    // per-part values in registers (kColMaxParts of 512 rows: 16384; far fewer workgroups than are resident at once, which is what progress
+    // needs)
     const int64_t tiles = ceil_div(p.out_n ? p.ld_n : m, 64), parts = ceil_div(n, 512);
     // rows of whole 16-byte pieces in aligned buffers: 16-byte accesses; any other width or alignment: the same kernel moving
     // its columns one by one (the transposed output runs along n either way)
@@ -405,14 +409,14 @@ static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st) {
         if (p.out_t) q.out_t += b0 * m * p.ld_t;
         if (p.out_n) q.out_n += b0 * n * p.ld_n;
         auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3((unsigned)xch_team_grid(tiles * nb, parts)), dim3(512), 0, st, q, (int32_t)tiles, (int32_t)parts,
+            hipLaunchKernelGGL(kern, dim3((unsigned)xch_team_grid(tiles * nb, parts)), dim3(kColThreads), 0, st, q, (int32_t)tiles, (int32_t)parts,
                                (uint32_t)(tiles * nb), xs.xl);
         };
         auto pick = [&](auto oc) {
             constexpr int OUT = decltype(oc)::value;
-            if (!wide) go(k_col_quantize_team<512, OUT, false, true, SCALED>);
-            else if (lines) go(k_col_quantize_team<512, OUT, true, false, SCALED>);
-            else go(k_col_quantize_team<512, OUT, false, false, SCALED>);
+            if (!wide) go(k_col_quantize_team<kColThreads, OUT, false, true, SCALED>);
+            else if (lines) go(k_col_quantize_team<kColThreads, OUT, true, false, SCALED>);
+            else go(k_col_quantize_team<kColThreads, OUT, false, false, SCALED>);
         };
         if (p.out_t && p.out_n) {
             if constexpr (!SCALED) pick(std::integral_constant<int, kOutT | kOutN>{});

@@ -5,6 +5,7 @@ import torch
 
 import cpm_kernels_amd.kernels as ck
 import oracle
+from oracle import training as ot
 from util import assert_bits_equal, quickest, to_gpu, to_np
 
 pytestmark = pytest.mark.gpu
@@ -90,3 +91,45 @@ def test_scales_below_the_normal_numbers_cost_little(gpu):
     t = quickest([_quantise(x)[0], _quantise(y)[0]])
     print("ordinary %.1f us, with columns of a subnormal scale %.1f us" % tuple(t), flush=True)
     assert t[1] <= 1.3 * t[0], t
+
+
+@pytest.mark.parametrize("n", [40, 512, 1030, 16384])
+@pytest.mark.parametrize("scaled", [False, True])
+@pytest.mark.parametrize("m", [128, 100])
+def test_short_rounding_of_whole_tiles(gpu, n, scaled, m):
+    """Tiles in which every column has a normal scale, so that all of them take the shorter rounding: exact ties between all neighbouring
+    integers, the largest magnitudes of either sign, quiet and signalling NaN.  One part of a team and several, both output layouts."""
+    rng = np.random.default_rng(n + m)
+    x = rng.standard_normal((1, n, m)).astype(np.float16)
+    for c in range(0, m, 3):       # scale 2^e exactly: k + 1/2 of it is a tie
+        e = np.float16(2.0 ** rng.integers(-4, 6))
+        x[0, :, c] = ((np.arange(n) * 7 % 252 - 126) + 0.5).astype(np.float16) * e
+        x[0, rng.integers(n), c] = np.float16(127) * e * (-1) ** c
+    for c in range(1, m, 3):
+        x[0, rng.integers(n), c] = np.float16(-60000 if c % 2 else 60000)
+    bits = x.view(np.uint16)
+    for c in range(2, m, 3):
+        bits[0, rng.integers(n), c] = (0x7e00, 0x7c01, 0xfe01, 0xfdff)[c % 4]
+    rs = np.ones((1, n), np.float16) * np.float16(0.5) if scaled else None
+    clean = np.where(np.isnan(x.astype(np.float32)), np.float16(0), x)         # a NaN element takes no part in the maximum and rounds to 0
+    if scaled:
+        want_q, want = ot.gemm_backward_scale_round(clean, rs, False)
+    else:
+        want = oracle.gemm_calc_scale_transpose(clean)
+        want_q = oracle.gemm_round_transpose(clean, want)
+    assert (want >= np.float16(2.0 ** -14)).all()
+    d = to_gpu(x)
+    drs = to_gpu(rs) if scaled else None
+    ld = (n + 15) // 16 * 16
+    s = torch.full((1, m), -1.0, dtype=torch.half, device=gpu)
+    qt = torch.full((1, m, ld), 77, dtype=torch.int8, device=gpu)
+    qn = torch.full((1, n, m), 77, dtype=torch.int8, device=gpu)
+    for t, nat in ((True, False), (False, True)) if scaled else ((True, True), (True, False), (False, True)):
+        s.fill_(-1); qt.fill_(77); qn.fill_(77)
+        ck.gemm_quantize_cols_ld(1, n, m, d.data_ptr(), drs.data_ptr() if scaled else None, False, s.data_ptr(), qt.data_ptr() if t else None,
+                                 ld if t else 0, qn.data_ptr() if nat else None, m if nat else 0, torch.cuda.current_stream().cuda_stream)
+        assert_bits_equal(to_np(s), want, "scales")
+        if t:
+            assert_bits_equal(to_np(qt)[:, :, :n], np.ascontiguousarray(want_q.transpose(0, 2, 1)), "transposed")
+        if nat:
+            assert_bits_equal(to_np(qn), want_q, "in place")

@@ -240,7 +240,7 @@ __device__ inline int32_t quant_i8_rcp(float x, float s, float y) {
 // its side.  q + 1.5 * 2^23 lands in [2^23, 2^24), where the fp32 grid is the integers: the one round-to-nearest-even of that addition
 // is rint(q), and the low byte of the sum's bit pattern is the two's-complement int8.  A NaN element (which the
 // absmax ignores) propagates as a quiet NaN whose low byte is 0, the value the long form gives it.
-// Equality with quant_i8 for every such (absmax, x) pair is proven by enumeration in
+// Equality with quant_i8 for every (scale, x) pair such data can hold is proven by enumeration in
 // tests/native/grid_round_check.c.  Returns the fp32 bit pattern; its low byte is the result.
 __device__ inline bool scale_is_normal(half_t sh) {
     const uint16_t b = __builtin_bit_cast(uint16_t, sh);
@@ -258,7 +258,8 @@ __device__ inline uint32_t quant_i8_own_scale_bits(float x, float y) {
 // last place of x / s and one residual step q1 within one; a residual step from such a q1 with such a y gives the correctly
 // rounded quotient (Markstein, IBM J. Res. Dev. 34, 1990, theorem on the division by fused multiply-adds), so the rint() below
 // sees what the IEEE division gives.  The residuals are exact: with s in [2^-60, 2^60] and |x / s| <= 127.1 no product of
-// the steps comes near the subnormal range except for quotients far below one half, which round to 0 either way.
+// the steps comes near the subnormal range except for quotients far below one half, which round to 0 either way
+// (tests/native/fused_round_check.c: every significand of an absmax, the numbers around every boundary between two integers).
 // Two operations more than the fp16 form, half of the division's.
 __device__ inline bool own_scale_in_range(float s) { return s >= 0x1p-60f && s <= 0x1p60f; }
 __device__ inline uint32_t quant_i8_own_fp32_scale_bits(float x, float s, float y) {

@@ -386,10 +386,10 @@ def test_reciprocal_rounding_equals_divide_rounding_exhaustively(tmp_path):
 
 
 def test_short_rounding_of_the_fused_quantisers_exhaustively(tmp_path):
-    """The fused quantisers round a row (column) whose scale is a normal fp16 number through
-    y = 1/s, one residual step and the low byte of q + 1.5 * 2^23; tests/native/fused_round_check.c
-    enumerates every (absmax, x) pair such a row can hold -- about 10^9 -- against the
-    divide-then-round of cuda/gemm.cu:16 with the same IEEE operations on the host."""
+    """The backward quantisers divide products of two fp16 numbers by an fp32 scale of their own through y = 1/s, two residual steps and
+    the low byte of q + 1.5 * 2^23; tests/native/fused_round_check.c takes every significand of a largest magnitude and the numbers around
+    every boundary between two integers through it, against the divide-then-round of cuda/gemm.cu:139-172 with the same IEEE
+    operations on the host."""
     import os, shutil, subprocess
     if shutil.which("gcc") is None:
         pytest.skip("no gcc")
@@ -398,7 +398,7 @@ def test_short_rounding_of_the_fused_quantisers_exhaustively(tmp_path):
     subprocess.run(["gcc", "-O2", "-ffp-contract=off", "-mfma", "-msse4.1", "-fopenmp", src, "-o", exe, "-lm"], check=True)
     r = subprocess.run([exe], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
-    assert r.stdout.startswith("23568 rows, 989078256 pairs, 0 mismatches"), r.stdout
+    assert r.stdout.startswith("419629 scales, 373889439 pairs, 0 mismatches"), r.stdout
 
 
 def test_rounding_on_the_grid_exhaustively(tmp_path):

@@ -517,7 +517,9 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     // The tile kernel stores 16-byte pieces of output rows that start on dwords, and 8-byte halves at a row's end.  Rows of 4j + 2
     // elements end in neither: their last column tile lies inside the matrix (edge_in), which takes a matrix of at least one tile.
     const bool odd = m % 4 != 0;
-    // (Tiles of the general kernel waste less of narrow ones: 80 heads of 150 x 150 6.7 us there, 9.0 here; 228 of 402 x 402, 58 and 33.)
+    // (The line at 192 columns was drawn for depths up to 128 with both operands stored (K, rows), which have a kernel of their own now; what it still keeps on
+    // the general kernel is deeper or stored otherwise and would mostly be quicker on the tiles from 128 columns on: 80 of 150 x 150, both stored (K, rows),
+    // K = 256 22.6 us and 8.6, K = 512 42.6 and 12.2; both K-major, K = 512 15.8 and 11.4, 300 of 130 x 130, K = 1000 84 and 103.)
     const bool wide = (reinterpret_cast<uintptr_t>(out) & 3u) == 0 && (!odd || m >= 192);
     const bool p_kmajor = !bT, q_kmajor = aT != 0;
     // A depth up to 128: a kernel of its own -- but where the output's rows are not whole cache lines and it exceeds half of the last-level
@@ -580,7 +582,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         const int lay = (p_kmajor ? 0 : 1) | (q_kmajor ? 0 : 2);
         // 256x256 tiles when they give most compute units a tile, else 128x128 (as for K-major operands) -- and when the
         // larger ones cover over half as much again as the smaller ones do, where that costs more than their better ratio of products to reads
-        // saves: 300 x 300 over 400 heads, K = 512 152 us with large tiles, 125 us with small ones, K = 80 both stored (K, rows) 66 and 48 us;
+        // saves: 300 x 300 over 400 heads, both stored (K, rows), K = 512 140 us with large tiles, 120 us with small ones, K = 160 70 and 46 us;
         // 580 x 580 (1.44 times the area) alike; with one operand K-major and K = 80 70 us with large tiles, 74 us with small ones.
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256), mid = ceil_div(n, 128) * ceil_div(m, 128);
         // (not where the large tiles are one round of the device: 384 x 384 over 50 heads, K = 1024 28 us with large tiles, 38 us with small ones)

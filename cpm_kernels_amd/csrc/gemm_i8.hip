@@ -276,9 +276,22 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
     if (m < 0 || n < 0 || k < 0 || batchA < 1 || batchB < 1) return CPMK_EBADARG;
     if ((m % 4) || (n % 4) || (k % 4)) return CPMK_EALIGN;      // kernels/gemm.py:139
     if (!(batchA == batchB || batchA == 1 || batchB == 1)) return CPMK_EBADARG;   // :140
-    const int batch = batchA > batchB ? batchA : batchB;
+    int batch = batchA > batchB ? batchA : batchB;
     if (m == 0 || n == 0) return 0;
     if (out == nullptr || (k > 0 && any_null(A, B)) || (FUSED && srow == nullptr && scol == nullptr)) return CPMK_EBADARG;
+    if (batchA == 1 && !bT && (srow == nullptr || !bcr) && (scol == nullptr || bcc) && rows_join(batch, n, k)) {
+        n *= batch;
+        batch = batchB = 1;
+    }
+    // (columns: where whole entries of them leave tiles half empty)
+    int32_t seg = 0;
+    if (FUSED && batchB == 1 && aT && (srow == nullptr || bcr) && (scol == nullptr || !bcc) && cols_join(batch, m, k) && aligned16(A) && aligned16(B) && aligned16(out) &&
+        k > 0 && (bT ? k % 128 == 0 && n % 16 == 0 : k % 64 == 0) &&
+        (ceil_div((int64_t)m * batch, 128) < ceil_div(m, 128) * batch || ceil_div((int64_t)m * batch, 256) < ceil_div(m, 256) * batch)) {
+        seg = m;
+        m *= batch;
+        batch = batchA = 1;
+    }
     if (batch > 65535) {      // some kernels index the batch with the grid's z dimension: at most 65535 entries per call
         constexpr int64_t ESZ_OUT = FUSED ? 2 : 4;
         for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
@@ -302,6 +315,8 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
     a.edge_in = 0;
     a.nsum = 1;
     a.kmagic = 0;
+    a.seg = seg;
+    a.segmagic = seg ? (uint32_t)(((1ull << 32) + seg - 1) / seg) : 0;
     // the tile kernel stores 16-byte pieces of output rows (8-byte halves where fp16 rows are not whole pieces: m % 8 == 4)
     const bool wide = aligned16(out);
     const bool p_kmajor = !bT, q_kmajor = aT != 0;
@@ -310,28 +325,34 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
         // 256x256 tiles when they give most compute units a tile, else 128x128
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
         constexpr int EPI = FUSED ? kEpiDequant : kEpiInt32;
-        if (k % 128 != 0) {
-            // a depth of whole 64-byte but not whole 128-byte slabs (1600, 4544 ...): the same kernels on 64-byte slabs and
-            // a ring of four stages -- twice the barriers per byte of K, 5-10 % behind the 128-byte form
-            if (big * 4 >= compute_units() * 3 && n > 128 && m > 128) return launch_dma<2, 4, 4, 2, 64, EPI, 4, 0, 16>(a, batch, st);
-            return launch_dma<2, 2, 2, 2, 64, EPI, kRingSmall, 0, 32>(a, batch, st);
+        auto kmajor = [&](auto lay) __attribute__((always_inline)) {
+            constexpr int LAY = decltype(lay)::value;
+            if (k % 128 != 0) {
+                // a depth of whole 64-byte but not whole 128-byte slabs (1600, 4544 ...): the same kernels on 64-byte slabs and
+                // a ring of four stages -- twice the barriers per byte of K, 5-10 % behind the 128-byte form
+                if (big * 4 >= compute_units() * 3 && n > 128 && m > 128) return launch_dma<2, 4, 4, 2, 64, EPI, 4, LAY, 16>(a, batch, st);
+                return launch_dma<2, 2, 2, 2, 64, EPI, kRingSmall, LAY, 32>(a, batch, st);
+            }
+            // (a dimension of at most 128 would leave half or more of every 256-wide tile empty)
+            if (big * 4 >= compute_units() * 3 && n > 128 && m > 128) return launch_dma<2, 4, 4, 2, 128, EPI, kRingBig, LAY, 16>(a, batch, st);
+            // 128x128 tiles, or 128x64 when even those leave a quarter of the compute units idle and twice as many of half their size are one round
+            // (two workgroups a compute unit of the latter: 500 x 5000, 160 tiles or 320, K = 4096 23.5 us, 18.5 so; K = 12160 58 and 43; K = 512 8.1 and 8.0)
+            const int64_t mid = ceil_div(n, 128) * ceil_div(m, 128) * batch;
+            // the smaller tiles finish a slab before a load from L2 returns: four ring stages keep them fed.  More
+            // tiles than compute units but at most two each: a ring of two stages instead, which lets two
+            // workgroups share a compute unit (2 x 80 KB of LDS) and all tiles run in one round, each
+            // workgroup's waits covered by the other's MFMAs (6-11 % over 1.25-2 rounds of single workgroups)
+            const int64_t cus = compute_units(), small = ceil_div(n, 128) * ceil_div(m, 64) * batch;
+            if (mid * 4 >= cus * 3 || small > cus) {
+                if (mid > cus && mid <= 2 * cus) return launch_dma<2, 2, 2, 2, 128, EPI, 2, LAY, 32>(a, batch, st, 2);
+                return launch_dma<2, 2, 2, 2, 128, EPI, kRingSmall, LAY, 32>(a, batch, st);
+            }
+            return launch_dma<2, 2, 2, 1, 128, EPI, kRingSmall, LAY, 32>(a, batch, st);
+        };
+        if constexpr (FUSED) {
+            if (seg) return kmajor(std::integral_constant<int, 16>{});
         }
-        // (a dimension of at most 128 would leave half or more of every 256-wide tile empty)
-        if (big * 4 >= compute_units() * 3 && n > 128 && m > 128) return launch_dma<2, 4, 4, 2, 128, EPI, kRingBig, 0, 16>(a, batch, st);
-        // 128x128 tiles, or 128x64 when even those leave a quarter of the compute units idle
-        const int64_t mid = ceil_div(n, 128) * ceil_div(m, 128) * batch;
-        // the smaller tiles finish a slab before a load from L2 returns: four ring stages keep them fed.  More
-        // tiles than compute units but at most two each: a ring of two stages instead, which lets two
-        // workgroups share a compute unit (2 x 80 KB of LDS) and all tiles run in one round, each
-        // workgroup's waits covered by the other's MFMAs (6-11 % over 1.25-2 rounds of single workgroups)
-        const int64_t cus = compute_units();
-        if (mid * 4 >= cus * 3) {
-            if (mid > cus && mid <= 2 * cus) return launch_dma<2, 2, 2, 2, 128, EPI, 2, 0, 32>(a, batch, st, 2);
-            return launch_dma<2, 2, 2, 2, 128, EPI, kRingSmall, 0, 32>(a, batch, st);
-        }
-        const int64_t small = ceil_div(n, 128) * ceil_div(m, 64) * batch;
-        if (small > cus && small <= 2 * cus) return launch_dma<2, 2, 2, 1, 128, EPI, 2, 0, 32>(a, batch, st, 2);
-        return launch_dma<2, 2, 2, 1, 128, EPI, kRingSmall, 0, 32>(a, batch, st);
+        return kmajor(std::integral_constant<int, 0>{});
     }
     // a depth that is not whole 64-byte slabs (4000, 4048, 4100 ...): the tile kernels on 64-byte slabs, the rest of the
     // depth straight from memory into the fragments (k % 4 == 0 is the reference's precondition: rows of whole dwords)
@@ -354,6 +375,9 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
         const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!in_q || m >= 256);
         a.edge_in = (in_p ? 1 : 0) | (in_q ? 2 : 0);
+        if constexpr (FUSED) {
+            if (seg) return large ? launch_dma<2, 4, 4, 2, 128, EPI, 2, 17, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, EPI, kRingSmall, 17, 32>(a, batch, st);
+        }
         switch ((p_kmajor ? 0 : 1) | (q_kmajor ? 0 : 2)) {
             case 1: return large ? launch_dma<2, 4, 4, 2, 128, EPI, 2, 1, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, EPI, kRingSmall, 1, 32>(a, batch, st);
             case 2: return large ? launch_dma<2, 4, 4, 2, 128, EPI, 2, 2, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, EPI, kRingSmall, 2, 32>(a, batch, st);
@@ -490,10 +514,14 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     if (m < 0 || n < 0 || k < 0 || batchA < 1 || batchB < 1) return CPMK_EBADARG;
     if ((m % 2) || (n % 2) || (k % 2)) return CPMK_EALIGN;      // kernels/gemm.py:200
     if (!(batchA == batchB || batchA == 1 || batchB == 1)) return CPMK_EBADARG;   // :201
-    const int batch = batchA > batchB ? batchA : batchB;
+    int batch = batchA > batchB ? batchA : batchB;
     if (m == 0 || n == 0) return 0;
     if (out == nullptr || (k > 0 && any_null(A, B))) return CPMK_EBADARG;
     if (k > (1 << 30)) return CPMK_ETOOBIG;
+    if (batchA == 1 && !bT && rows_join(batch, n, (int64_t)k * 2)) {
+        n *= batch;
+        batch = batchB = 1;
+    }
     if (batch > 65535) {      // (grid z: at most 65535 batch entries per call)
         for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
             const int32_t nb = (int32_t)(batch - b0 < 65535 ? batch - b0 : 65535);
@@ -514,6 +542,8 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     a.edge_in = 0;
     a.nsum = 1;
     a.kmagic = 0;
+    a.seg = 0;
+    a.segmagic = 0;
     // The tile kernel stores 16-byte pieces of output rows that start on dwords, and 8-byte halves at a row's end.  Rows of 4j + 2
     // elements end in neither: their last column tile lies inside the matrix (edge_in), which takes a matrix of at least one tile.
     const bool odd = m % 4 != 0;

@@ -72,7 +72,7 @@ static int gemm_sum_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t 
     if (!aligned16(out) || (f16 ? (kb <= 64 || kb % 4 != 0) : kb % 128 != 0)) return CPMK_EALIGN;
     const bool whole = kb % 16 == 0 && aligned16(A) && aligned16(B);
     if (!whole && (!f16 || ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 3u))) return CPMK_EALIGN;
-    GemmArgs a;
+    GemmArgs a = {};
     a.P = (const int8_t*)B; a.Q = (const int8_t*)A; a.out = out;
     a.srow = (const half_t*)srow; a.scol = nullptr;
     a.strideP = (int64_t)n * kb;
@@ -115,7 +115,7 @@ static int gemm_rows_parts(int32_t m, int64_t k, int32_t n, int32_t groups, cons
     if (n * k * 2 >= (1ll << 32) || m * k * 2 >= (1ll << 32)) return CPMK_ETOOBIG;
     const bool in_p = n % 8 != 0, in_q = m % 8 != 0;
     if (k < 64 || (in_p && n < 128) || (in_q && m < 256) || !aligned16(A) || !aligned16(B) || !aligned16(out)) return CPMK_EALIGN;
-    GemmArgs a;
+    GemmArgs a = {};
     a.P = (const int8_t*)B; a.Q = (const int8_t*)A; a.out = out;
     a.srow = nullptr; a.scol = nullptr;
     a.strideP = n * k * 2;

@@ -19,6 +19,11 @@ struct GemmArgs {
     int32_t edge_in;      // bit 0 / 1: the last row / column tile starts at n - BR / m - BC instead of reaching past the end
     int32_t nsum;         // kEpiSum*: consecutive batch entries that one output is the sum of
     uint32_t kmagic;      // kEpiSum*: ceil(2^32 / slabs of one entry)
+    int32_t seg;          // LAY bit 4: columns of one entry (the m columns are those of several entries side by side)
+    uint32_t segmagic;    // ... ceil(2^32 / seg)
+    int32_t entries;      // LAY bit 5: batch entries (work entry s * entries + e is part s of the depth of entry e),
+    int32_t part_slabs;   // ... slabs of a part (the last one may have fewer)
+    int64_t partP, partQ; // ... and bytes from one part's operands to the next's
 };
 
 // ---------------------------------------------------------------------------------------
@@ -120,6 +125,8 @@ __device__ __forceinline__ void store_piece(int8_t* dst, int4_t v, int32_t left)
 template <int BR, int BC, int BKB, int NW, int NST, int LAY, bool F16, bool TSW = false, bool SUM = false, bool REST = false>
 struct SlabDma {
     static_assert(!(REST && SUM), "sums over the batch take the rest of the depth from memory");
+    static constexpr bool PARTS = (LAY & 32) != 0;        // the work entry is one part of the depth of its batch entry
+    static_assert(!(PARTS && (REST || SUM)), "parts of the depth are whole slabs");
     static constexpr bool PT = (LAY & 1) != 0, QT = (LAY & 2) != 0;
     static constexpr int ESZ_IN = F16 ? 2 : 1;            // bytes per operand element
     static constexpr int EPP = 16 / ESZ_IN;               // elements per 16-byte piece
@@ -199,10 +206,16 @@ struct SlabDma {
         nk = SUM ? nkb * a.nsum : REST && rem != 0 ? nkb + 1 : nkb;
         oj0 = cur_item.j0;
         oi0 = cur_item.i0;
-        const uint32_t b = SUM ? cur_item.b * (uint32_t)a.nsum : cur_item.b;
-        Pb = a.P + (int64_t)b * a.strideP;
-        Qb = a.Q + (int64_t)b * a.strideQ;
-        ahead = nxt_item.valid && nxt_item.half == cur_item.half;
+        uint32_t b = SUM ? cur_item.b * (uint32_t)a.nsum : cur_item.b;
+        uint32_t part = 0;
+        if constexpr (PARTS) {
+            part = b / (uint32_t)a.entries;
+            b -= part * (uint32_t)a.entries;
+            nk = nkb = min(a.part_slabs, nkb - (int)part * a.part_slabs);
+        }
+        Pb = a.P + (int64_t)b * a.strideP + (PARTS ? part * a.partP : 0);
+        Qb = a.Q + (int64_t)b * a.strideQ + (PARTS ? part * a.partQ : 0);
+        ahead = !PARTS && nxt_item.valid && nxt_item.half == cur_item.half;       // (parts differ in their slabs; a launch of them has a tile a workgroup)
         // slab s of this tile lives in stage (ring + s) % NST.  With fewer slabs than stages (!deep) all of a
         // tile's slabs are requested one tile ahead and every wait is a full one.
         deep = nk >= NST;
@@ -212,8 +225,8 @@ struct SlabDma {
         const uint32_t tb = !ahead ? b : SUM ? nxt_item.b * (uint32_t)a.nsum : nxt_item.b;
         tj0 = ahead ? nxt_item.j0 : cur_item.j0;
         ti0 = ahead ? nxt_item.i0 : cur_item.i0;
-        Pn = a.P + (int64_t)tb * a.strideP;
-        Qn = a.Q + (int64_t)tb * a.strideQ;
+        Pn = PARTS ? Pb : a.P + (int64_t)tb * a.strideP;
+        Qn = PARTS ? Qb : a.Q + (int64_t)tb * a.strideQ;
 #pragma unroll
         for (int d = 0; d < CNT; ++d) {
             const int dd = wave + d * NW;
@@ -373,7 +386,8 @@ __device__ __forceinline__ void tail_slabs(Dma& dma, int it, F&& slab) {
 // would touch 32 different rows with 8 or 16 bytes each per instruction.  Written to the strip as 32 rows x RB
 // bytes and read back 16 bytes per lane, every store instruction covers whole contiguous rows of the chunk
 // (RB = 128 bytes: eight lanes per 128-byte line).
-template <int EPI, int TC>
+// SEG: the columns are those of several entries side by side, `a.seg` (a multiple of 4) each, and go out to one (n, seg) matrix an entry.
+template <int EPI, int TC, bool SEG = false>
 struct StripOut {
     static constexpr int ESZ = epi_out32(EPI) ? 4 : 2;
     static constexpr int CT = epi_out32(EPI) ? 1 : TC;       // MFMA tile columns (of 32) side by side in one chunk
@@ -389,7 +403,17 @@ struct StripOut {
             const int4_t v = *reinterpret_cast<const int4_t*>(stg + R * RB + slot(R, pc));
             const int32_t row = row0 + R;
             const int32_t col = col0 + pc * (16 / ESZ);
-            if (row < a.n && col < a.m)
+            if constexpr (SEG) {
+                static_assert(ESZ == 2, "fp16 results");
+                if (row < a.n && col < a.m) {
+                    const uint32_t e = __umulhi((uint32_t)col, a.segmagic);          // col / seg (exact for m * seg < 2^32)
+                    const int32_t c = col - (int32_t)e * a.seg;
+                    half_t* dst = reinterpret_cast<half_t*>(a.out) + ((int64_t)e * a.n + row) * a.seg + c;
+                    store_piece<ESZ>(reinterpret_cast<int8_t*>(dst), v, a.seg - c);
+                    if (a.seg - c < 8 && col + 4 < a.m)      // the piece's second half is the next entry's
+                        *reinterpret_cast<int2_t*>(reinterpret_cast<half_t*>(a.out) + ((int64_t)(e + 1) * a.n + row) * a.seg) = int2_t{v.z, v.w};
+                }
+            } else if (row < a.n && col < a.m)
                 store_piece<ESZ>(reinterpret_cast<int8_t*>(a.out) + (obase + (int64_t)row * a.m + col) * ESZ, v, a.m - col);
         }
     }
@@ -426,6 +450,8 @@ struct StripOut {
 // operand stored (K, rows) the rest is a slab of the ring: SlabDma's REST.)
 // LAY bit 3, with bit 2: the rest of a row may start off a 16-byte boundary and end inside a piece (depths and rows of
 // whole dwords only); without it every piece of the rest is whole and aligned.
+// LAY bit 4: the columns of several batch entries side by side (StripOut's SEG).  LAY bit 5: an entry's depth in parts, each a
+// work entry with an output of its own (SlabDma's PARTS).
 // LAY marks operands whose rows are K instead: bit 0 = the row operand is stored (K, n), bit 1 =
 // the column operand is stored (K, m).  Such an operand's part of a stage holds the slab's rows
 // of K (64 for fp16, 128 for int8) with the tile's BR (BC) elements each, DMA'd as they lie in
@@ -729,7 +755,7 @@ __device__ __forceinline__ bool gemm_dma_tile(const GemmArgs& a, int8_t* smem, i
     ring = cur;                          // (ring0 + nk) % NST: where the next tile's slab 0 is, or will be put
 
     const int64_t obase = (int64_t)b * a.n * a.m;
-    using Out = StripOut<EPI, TC>;       // the results leave through this wave's strip of LDS
+    using Out = StripOut<EPI, TC, (LAY & 16) != 0>;       // the results leave through this wave's strip of LDS
     constexpr int NCH = Out::NCH, RB = Out::RB;
     auto slot = [](int r, int p) __attribute__((always_inline)) { return Out::slot(r, p); };
     half_t sxr[AR];
@@ -1051,7 +1077,7 @@ __device__ __forceinline__ bool gemm_dma_tile32(const GemmArgs& a, int8_t* smem,
     ring = cur;                          // (ring0 + nk) % NST: where the next tile's slab 0 is, or will be put
 
     const int64_t obase = (int64_t)b * a.n * a.m;
-    using Out = StripOut<EPI, TC>;       // the results leave through this wave's strip of LDS
+    using Out = StripOut<EPI, TC, (LAY & 16) != 0>;       // the results leave through this wave's strip of LDS
     constexpr int NCH = Out::NCH, RB = Out::RB;
     auto slot = [](int r, int p) __attribute__((always_inline)) { return Out::slot(r, p); };
     half_t sxr[TR];
@@ -1188,7 +1214,7 @@ static int launch_dma(GemmArgs& a, int batch, hipStream_t st, int per_cu = 1) {
     // (a half tile's slab must split evenly over the waves too, and beside operands stored (K, rows) rows of K be whole 128-byte groups
     // in half a tile; a tile moved inside the matrix has no half of its own)
     constexpr bool F16 = epi_f16(EPI);
-    if constexpr (TR % 2 == 0 && (LAY & 4) == 0 && ((BR / 2 + BC) / (1024 / BKB)) % (WR * WC) == 0 &&
+    if constexpr (TR % 2 == 0 && (LAY & (4 | 32)) == 0 && ((BR / 2 + BC) / (1024 / BKB)) % (WR * WC) == 0 &&
                   ((LAY & 3) == 0 || (BR / 2) * (F16 ? 2 : 1) % 128 == 0)) {
         if (r > 0 && 2 * r <= grid && (a.edge_in & 1) == 0) {
             da.nfull = (uint32_t)(total - r);
@@ -1197,6 +1223,21 @@ static int launch_dma(GemmArgs& a, int batch, hipStream_t st, int per_cu = 1) {
         }
     }
     return launch_dma_kernel<WR, WC, TR, TC, BKB, EPI, false, NST, LAY, MF>(da, (unsigned)grid, st);
+}
+
+// A row operand stored (batch, n, k) beside a column operand that the batch shares: its entries, and the outputs', lie one behind the other
+// and are one product of batch x n rows, whose tiles reach across the entries.  Entry by entry the last row tile of each was filled up to
+// 128 rows, and the shared operand read for every entry: fp16, 16 entries of 32 x 8192 beside 4096 rows 127 -> 59 us, 7 of 300 x 1540 beside
+// 7000 123 -> 67, the gradient of the 300 x 1540 117 -> 67; int8, 4 of 436 x 3712 beside 2304 29 -> 24.  (Operands stay below 4 GiB, what the tile kernels address.)
+static bool rows_join(int batch, int32_t n, int64_t row_bytes) {
+    return batch > 1 && (int64_t)batch * n < (1ll << 31) && batch * n * row_bytes < (1ll << 32);
+}
+
+// The same for a column operand stored (batch, m, k) beside a row operand that the batch shares: one product of batch x m columns, whose
+// results go out to one matrix an entry (StripOut's SEG): 3 entries of 40 columns, 3904 x 12096, 34 -> 34 us and 12096 x 3904 28 -> 20; 5 of 136, the
+// training step of a 3200 x 6848 ffn block 415 -> 369.
+static bool cols_join(int batch, int32_t m, int64_t row_bytes) {
+    return batch > 1 && (int64_t)batch * m < (1ll << 31) && batch * m * row_bytes < (1ll << 32) && (int64_t)batch * m * m < (1ll << 32);
 }
 
 }  // namespace cpmk

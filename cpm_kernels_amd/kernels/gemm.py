@@ -235,6 +235,33 @@ def gemm_add_parts(groups: int, n: int,
     cpmk.gemm_add_parts(groups, n, parts, out, stream)
 
 
+def gemm_depth_parts(f16: bool, m: int, k: int, n: int, batchA: int, batchB: int, aT: bool, bT: bool) -> int:
+    """Parts that the depth of a product is worth dividing into (gemm_int8_scale_split, gemm_fp16_split), 1 if none."""
+    return cpmk.gemm_depth_parts(1 if f16 else 0, m, k, n, batchA, batchB, 1 if aT else 0, 1 if bT else 0)
+
+
+def gemm_int8_scale_split(m: int, k: int, n: int, batchA: int, batchB: int, aT: bool, bT: bool,
+                          A: DevicePointer, B: DevicePointer, scale_row: DevicePointer, scale_col: DevicePointer,
+                          broad_cast_row: bool, broad_cast_col: bool,
+                          out: DevicePointer,         # (batch, n, m)  fp16
+                          parts: int,
+                          workspace: DevicePointer,   # (parts, batch, n, m)  int32
+                          stream: CUDAStream):
+    """gemm_int8_scale_one with the depth divided into parts that are formed side by side."""
+    cpmk.gemm_int8_scale_split(m, k, n, batchA, batchB, 1 if aT else 0, 1 if bT else 0, A, B, scale_row, scale_col,
+                               1 if broad_cast_row else 0, 1 if broad_cast_col else 0, out, parts, workspace, stream)
+
+
+def gemm_fp16_split(m: int, k: int, n: int, batchA: int, batchB: int, aT: bool, bT: bool,
+                    A: DevicePointer, B: DevicePointer,
+                    out: DevicePointer,         # (batch, n, m)         fp16
+                    parts: int,
+                    workspace: DevicePointer,   # (parts, batch, n, m)  fp32
+                    stream: CUDAStream):
+    """gemm_fp16 with the depth divided into parts that are formed side by side, their fp32 sums added and rounded once."""
+    cpmk.gemm_fp16_split(m, k, n, batchA, batchB, 1 if aT else 0, 1 if bT else 0, A, B, out, parts, workspace, stream)
+
+
 def gemm_fp16(m: int, k: int, n: int,
               batchA: int, batchB: int,
               aT: bool, bT: bool,

@@ -21,6 +21,7 @@ _LAUNCHERS = {
     "gemm_backward_round_scale_ld": "iiipppipip", "gemm_int8_scale_one": "iiiiiiippppiipp",
     "transpose_i8_ld": "iiipipip", "gemm_int8_scale_sum": "iiiiippppp", "gemm_fp16_sum": "iiiiipppp",
     "gemm_int8_scale_parts": "iiiiippppp", "gemm_fp16_parts": "iiiiiipppp", "gemm_add_parts": "ilppp",
+    "gemm_int8_scale_split": "iiiiiiippppiipipp", "gemm_fp16_split": "iiiiiiipppipp",
     "gemv_fp16": "iiipppp", "gemv_fp16_transpose": "iiipppp", "gemv_broadcast_mat_fp16": "iiipppp",
     "embedding_forward": "iiipppp", "embedding_step": "iipppp", "copy_data_to_kv": "iiippip",
     "gemv_calc_scale": "iippp", "gemv_round": "iipppp", "gemv_broadcast_mat_int8": "iiipppppp",
@@ -47,6 +48,7 @@ _CTYPES = {"i": ctypes.c_int32, "l": ctypes.c_int64, "f": ctypes.c_float, "p": c
 EXPORTED_SYMBOLS = sorted(["cpmk_" + n for n in _LAUNCHERS] + [
     "cpmk_version", "cpmk_error_string", "cpmk_device_count", "cpmk_get_device",
     "cpmk_set_device", "cpmk_device_props", "cpmk_exchange_capture_slots_left", "cpmk_gemm_sum_groups", "cpmk_gemm_sum_groups_for",
+    "cpmk_gemm_depth_parts",
 ])
 
 
@@ -125,6 +127,11 @@ def gemm_sum_groups(m: int, n: int, batch: int) -> int:
 @lib.bind("cpmk_gemm_sum_groups_for", [ctypes.c_int] + [ctypes.c_int32] * 4, ctypes.c_int32)
 def gemm_sum_groups_for(kind: int, m: int, k: int, n: int, batch: int) -> int:
     return lib.cpmk_gemm_sum_groups_for(kind, m, k, n, batch)
+
+
+@lib.bind("cpmk_gemm_depth_parts", [ctypes.c_int] + [ctypes.c_int32] * 5 + [ctypes.c_int] * 2, ctypes.c_int32)
+def gemm_depth_parts(f16: int, m: int, k: int, n: int, batchA: int, batchB: int, aT: int, bT: int) -> int:
+    return lib.cpmk_gemm_depth_parts(f16, m, k, n, batchA, batchB, aT, bT)
 
 
 @lib.bind("cpmk_device_count", [ctypes.POINTER(ctypes.c_int)], ctypes.c_int)

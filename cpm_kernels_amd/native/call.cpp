@@ -128,6 +128,8 @@ PyMethodDef g_launchers[] = {
     CPMK_ENTRY(cpmk_transpose_i8_ld)
     CPMK_ENTRY(cpmk_gemm_int8_scale_sum)
     CPMK_ENTRY(cpmk_gemm_fp16_sum)
+    CPMK_ENTRY(cpmk_gemm_int8_scale_split)
+    CPMK_ENTRY(cpmk_gemm_fp16_split)
     CPMK_ENTRY(cpmk_gemm_int8_scale_parts)
     CPMK_ENTRY(cpmk_gemm_fp16_parts)
     CPMK_ENTRY(cpmk_gemm_add_parts)

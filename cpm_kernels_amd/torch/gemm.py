@@ -10,7 +10,7 @@ import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
     gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_for, gemm_int8_scale_sum, gemm_fp16_sum, \
-    gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, \
+    gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, gemm_depth_parts, gemm_int8_scale_split, gemm_fp16_split, \
     arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
     transpose_i8_ld
 from ._common import cur_stream
@@ -85,6 +85,10 @@ def _quantize_cols(x, both: bool, row_scale=None):
     return scale, out_t, out_n
 
 
+# Outputs of a product that may be worth dividing along its depth (gemm_depth_parts): a larger one has a tile for every compute unit.
+_PARTS_MOST = 1 << 22
+
+
 def _dims(quantA, quantB, aT, bT):
     _, M, K = quantA.shape
     if aT:
@@ -101,6 +105,14 @@ def gemm_and_scale(quantA, scaleA, quantB, scaleB, aT, bT, fused=True) -> torch.
     batch = max(quantA.size(0), quantB.size(0))
     result_fp = torch.empty((batch, M, N), dtype=torch.float16, device=quantA.device)
     if fused:
+        parts = gemm_depth_parts(False, N, K, M, quantB.size(0), quantA.size(0), bT, aT) if K >= 2048 and result_fp.numel() < _PARTS_MOST else 1
+        if parts > 1:
+            workspace = torch.empty((parts, result_fp.numel()), dtype=torch.int32, device=quantA.device)
+            gemm_int8_scale_split(N, K, M, quantB.size(0), quantA.size(0), bT, aT, quantB.data_ptr(), quantA.data_ptr(),
+                                  None if scaleA is None else scaleA.data_ptr(), None if scaleB is None else scaleB.data_ptr(),
+                                  scaleA is None or scaleA.size(0) == 1, scaleB is None or scaleB.size(0) == 1,
+                                  result_fp.data_ptr(), parts, workspace.data_ptr(), cur_stream())
+            return result_fp
         gemm_int8_scale_one(N, K, M, quantB.size(0), quantA.size(0), bT, aT,
                             quantB.data_ptr(), quantA.data_ptr(),
                             None if scaleA is None else scaleA.data_ptr(), None if scaleB is None else scaleB.data_ptr(),
@@ -305,6 +317,11 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
         if not bT and (M > 8192 and K > 128 or large and M > 2048):
             B, bT = _transposed_copy(B), True
     out = torch.empty((max(bA, bB), M, N), dtype=torch.half, device=A.device)
+    parts = gemm_depth_parts(True, N, K, M, bB, bA, bT, aT) if K >= 1024 and out.numel() < _PARTS_MOST and (A.data_ptr() | B.data_ptr()) % 16 == 0 else 1
+    if parts > 1:
+        workspace = torch.empty((parts, out.numel()), dtype=torch.float32, device=A.device)
+        gemm_fp16_split(N, K, M, bB, bA, bT, aT, B.data_ptr(), A.data_ptr(), out.data_ptr(), parts, workspace.data_ptr(), cur_stream())
+        return out
     gemm_fp16(N, K, M, bB, bA, bT, aT, B.data_ptr(), A.data_ptr(), out.data_ptr(), cur_stream())
     return out
 

@@ -209,6 +209,17 @@ int cpmk_gemm_int8_scale_parts(int32_t m, int32_t k, int32_t n, int32_t batch, i
 int cpmk_gemm_fp16_parts(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, int k_first, const void* A, const void* B,
                          void* parts, void* stream);
 int cpmk_gemm_add_parts(int32_t groups, int64_t n, const void* parts, void* out, void* stream);
+/* cpmk_gemm_int8_scale_one / cpmk_gemm_fp16 with the depth divided into `parts` that are formed side by side and added up, for products
+ * of few outputs and a long contraction; workspace: parts * batch * n * m * 4 bytes on a 16-byte boundary.  The same results (int8: the same
+ * bits).  cpmk_gemm_depth_parts: the parts that are worth it, 1 where cpmk_gemm_int8_scale_one (f16 = 0) or cpmk_gemm_fp16 is the quicker
+ * or the product has no such form: these take depths of whole 128-byte slabs, at least two, n and m multiples of 4 (of whole 16-byte pieces for an
+ * operand stored (K, rows)), A (batchA, m, k) in the int8 form, buffers on 16-byte boundaries. */
+int cpmk_gemm_depth_parts(int f16, int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT);
+int cpmk_gemm_int8_scale_split(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, const void* A, const void* B,
+                               const void* scale_row, const void* scale_col, int broad_cast_row, int broad_cast_col, void* out, int32_t parts,
+                               void* workspace, void* stream);
+int cpmk_gemm_fp16_split(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, const void* A, const void* B, void* out,
+                         int32_t parts, void* workspace, void* stream);
 /* out[b,o] = sum_k mat[b,o,k] vec[b,k]      kernels/gemv.py:82-149 / cuda/gemv.cu:78-107 */
 int cpmk_gemv_fp16(int32_t batch, int32_t dim_out, int32_t dim_in, const void* mat,
                    const void* vec, void* out, void* stream);

@@ -1,0 +1,96 @@
+"""Products of a batch and an operand that it shares, as one product over the joined rows or columns, and products whose depth is divided."""
+import pytest
+import torch
+
+import cpm_kernels_amd.kernels as ck
+from util import stream
+
+pytestmark = pytest.mark.gpu
+
+
+def _int8(batch_a, batch_b, m, k, n, bT, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def ints(*shape):
+        return torch.randint(-127, 128, shape, generator=g, device="cuda", dtype=torch.int8)
+
+    def scales(*shape):
+        return (torch.rand(shape, generator=g, device="cuda") * 0.01 + 0.001).half()
+    return ints(batch_a, m, k), ints(*((batch_b, k, n) if bT else (batch_b, n, k))), scales(batch_b, n), scales(batch_a, m)
+
+
+def _reference(A, B, bT, s_row, s_col):
+    """(batch, n, m): exact sums, scaled as the epilogue does it"""
+    out = []
+    for i in range(max(A.size(0), B.size(0))):
+        ia, ib = i % A.size(0), i % B.size(0)
+        b = B[ib].double()
+        acc = (b.t() if bT else b).contiguous() @ A[ia].double().t().contiguous()
+        out.append(((acc.float() * s_row[ib].float()[:, None]) * s_col[ia].float()[None, :]).half())
+    return torch.stack(out)
+
+
+def _whole(A, B, bT, s_row, s_col, k, parts=0):
+    batch, m, n = max(A.size(0), B.size(0)), A.size(1), s_row.size(1)
+    out = torch.full((batch, n, m), float("nan"), dtype=torch.half, device="cuda")
+    args = (m, k, n, A.size(0), B.size(0), True, bT, A.data_ptr(), B.data_ptr(), s_row.data_ptr(), s_col.data_ptr(), B.size(0) == 1, A.size(0) == 1, out.data_ptr())
+    if parts:
+        ws = torch.full((parts, batch, n, m), -1, dtype=torch.int32, device="cuda")
+        ck.gemm_int8_scale_split(*args, parts, ws.data_ptr(), stream())
+    else:
+        ck.gemm_int8_scale_one(*args, stream())
+    return out
+
+
+# (depths of 64-byte and 128-byte slabs; entries of whole pieces, of half pieces, shorter than a piece, and around a tile; few and many tiles)
+@pytest.mark.parametrize("m,batch,n", [(4, 33, 132), (36, 7, 300), (100, 5, 128), (132, 3, 260), (64, 7, 272), (252, 16, 4112)])
+@pytest.mark.parametrize("k,bT", [(64, False), (192, False), (128, False), (1152, False), (128, True), (640, True)])
+def test_shared_row_operand(m, batch, n, k, bT):
+    if bT:
+        n = (n + 15) // 16 * 16
+    A, B, s_row, s_col = _int8(batch, 1, m, k, n, bT, m + k)
+    assert torch.equal(_whole(A, B, bT, s_row, s_col, k), _reference(A, B, bT, s_row, s_col))
+
+
+@pytest.mark.parametrize("n,batch,m", [(4, 33, 132), (36, 7, 300), (132, 3, 260), (252, 16, 4112)])
+@pytest.mark.parametrize("k", [4, 68, 128, 640])
+def test_shared_column_operand(n, batch, m, k):
+    A, B, s_row, s_col = _int8(1, batch, m, k, n, False, n + k)
+    assert torch.equal(_whole(A, B, False, s_row, s_col, k), _reference(A, B, False, s_row, s_col))
+
+
+# (parts of one slab, of several, a shorter last part, more parts than slabs)
+@pytest.mark.parametrize("batch_a,batch_b,m,n,bT", [(1, 1, 64, 128, False), (3, 1, 44, 260, False), (1, 5, 132, 60, False), (2, 2, 132, 132, False),
+                                                    (3, 1, 100, 272, True), (3, 1, 20, 16, True)])
+@pytest.mark.parametrize("slabs,parts", [(2, 2), (7, 3), (33, 16), (5, 9)])
+def test_int8_in_parts(batch_a, batch_b, m, n, bT, slabs, parts):
+    k = slabs * 128
+    A, B, s_row, s_col = _int8(batch_a, batch_b, m, k, n, bT, slabs)
+    assert torch.equal(_whole(A, B, bT, s_row, s_col, k, parts), _reference(A, B, bT, s_row, s_col))
+
+
+@pytest.mark.parametrize("aT,bT", [(True, False), (False, False), (True, True), (False, True)])
+@pytest.mark.parametrize("batch_a,batch_b,m,n", [(1, 1, 56, 136), (3, 1, 40, 264), (1, 5, 136, 64), (2, 2, 136, 136)])
+@pytest.mark.parametrize("slabs,parts", [(2, 2), (7, 3), (33, 16)])
+def test_fp16_in_parts(aT, bT, batch_a, batch_b, m, n, slabs, parts):
+    k = slabs * 64
+    g = torch.Generator(device="cuda").manual_seed(slabs)
+    A = torch.randn((batch_a, m, k) if aT else (batch_a, k, m), generator=g, device="cuda").half()
+    B = torch.randn((batch_b, k, n) if bT else (batch_b, n, k), generator=g, device="cuda").half()
+    batch = max(batch_a, batch_b)
+    out = torch.full((batch, n, m), float("nan"), dtype=torch.half, device="cuda")
+    ws = torch.full((parts, batch, n, m), float("nan"), dtype=torch.float32, device="cuda")
+    ck.gemm_fp16_split(m, k, n, batch_a, batch_b, aT, bT, A.data_ptr(), B.data_ptr(), out.data_ptr(), parts, ws.data_ptr(), stream())
+    for i in range(batch):
+        a, b = A[i % batch_a].double(), B[i % batch_b].double()
+        a, b = (a.t() if aT else a).contiguous(), (b.t() if bT else b).contiguous()        # (k, m), (n, k)
+        ref, size = b @ a, b.abs() @ a.abs()
+        # k additions in fp32, one rounding to fp16 (or half a subnormal step)
+        assert ((out[i].double() - ref).abs() <= size * k * 2.0 ** -24 + ref.abs() * 2.0 ** -10.9 + 2.0 ** -25).all()
+
+
+def test_parts_are_refused_elsewhere():
+    A, B, s_row, s_col = _int8(1, 1, 64, 320, 128, False, 0)       # (a depth of whole 64-byte slabs only)
+    assert ck.gemm_depth_parts(False, 64, 320, 128, 1, 1, True, False) == 1
+    with pytest.raises(RuntimeError):
+        _whole(A, B, False, s_row, s_col, 320, 2)

@@ -46,8 +46,7 @@ constexpr int kColThreads = 512, kColPackets = 4;
 constexpr int64_t kColMaxParts = kColThreads / 64 * kColPackets;
 
 template <int NT, int OUT, bool NTH, bool UA, bool SCALED>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_col_quantize_team(ColQuantArgs a, int32_t tiles_per_batch, int32_t parts,
-                                                          uint32_t nteams, XchLaunch xl) {
+__device__ __forceinline__ void col_quantize_team(const ColQuantArgs& a, int32_t tiles_per_batch, int32_t parts, uint32_t nteams, const XchLaunch& xl) {
     constexpr bool TRANSPOSED = (OUT & kOutT) != 0, NATURAL = (OUT & kOutN) != 0;
     const int32_t n = a.n, m = a.m;
     const half_t* const mat = a.mat;
@@ -284,6 +283,107 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 6))) void
     if (parts > 1 && tid < 64) xch_retire(xl, team, parts);
 }
 
+template <int NT, int OUT, bool NTH, bool UA, bool SCALED>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_col_quantize_team(ColQuantArgs a, int32_t tiles_per_batch, int32_t parts,
+                                                          uint32_t nteams, XchLaunch xl) {
+    col_quantize_team<NT, OUT, NTH, UA, SCALED>(a, tiles_per_batch, parts, nteams, xl);
+}
+
+// The other operand of the same product, quantised along its rows, in the same launch (k_col_quantize_rows): its workgroups follow the
+// teams', and stream while those wait for their members and for their phases to pass.  Bound by memory: an 8 x 4096 x 512 and an 8 x 10240 x 512
+// operand beside their 10240 x 4096 weights, 428 MB, 82 us (5.2 TB/s) where a launch for each takes 90; 4 x 2944 x 296 beside 2944 rows 15 and 18,
+// 2 x 1024 x 72 beside 824 9 and 12.  Six waves a SIMD for the rows too, as for the teams; a wave a row up to 4096 columns, a workgroup beyond.
+struct RowQuantArgs {
+    const half_t* mat;            // (rows, m), m % 8 == 0, 16-byte aligned
+    half_t* scale;
+    int8_t* out;                  // (rows, ld), 8-byte aligned, ld % 8 == 0: the surplus is zeros
+    int32_t m, ld;
+    int64_t rows;
+    uint32_t first;               // number of the first workgroup of the rows
+};
+
+// A row's pieces of eight, NV of them a lane, `step` pieces apart; ROW_WG: the row is the whole workgroup's, else a wave's.
+template <int NV, bool ROW_WG>
+__device__ __forceinline__ void quantize_row(const RowQuantArgs& a, uint32_t block) {
+    __shared__ uint32_t red[kColThreads / 64];
+    __shared__ float redf[kColThreads / 64];
+    constexpr int STEP = ROW_WG ? kColThreads : 64;
+    const int tid = threadIdx.x, lane = ROW_WG ? tid : tid & 63;
+    const int64_t row = ROW_WG ? (int64_t)block : (int64_t)block * (kColThreads / 64) + (tid >> 6);
+    if (row >= a.rows) return;                        // (the same for the whole workgroup where it meets at barriers)
+    const half8_t* p8 = reinterpret_cast<const half8_t*>(a.mat + row * a.m);
+    const int m8 = a.m >> 3, l8 = a.ld >> 3;
+    half8_t v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        v[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        if (lane + i * STEP < m8) v[i] = __builtin_nontemporal_load(p8 + lane + i * STEP);
+    }
+    ushort8_t um = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < NV; ++i) um = absbits_max(um, v[i]);
+    uint32_t ub = wave_max_u32_uniform(absbits_max_of(um));
+    if constexpr (ROW_WG) {
+        if ((tid & 63) == 0) red[tid >> 6] = ub;
+        __syncthreads();
+        ub = red[0];
+#pragma unroll
+        for (int w = 1; w < kColThreads / 64; ++w) ub = max(ub, red[w]);
+    }
+    float mx = (float)__builtin_bit_cast(half_t, (uint16_t)ub);
+    if (ub > 0x7c00u) {      // (the same for the whole row) a NaN: the maximum that skips NaN elements
+        mx = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            int4_t ci = __builtin_bit_cast(int4_t, v[i]);
+            asm volatile("" : "+v"(ci));         // nothing of this rare path is to be computed ahead of the branch
+            const half8_t h = __builtin_bit_cast(half8_t, ci);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mx = fmaxf(fabsf((float)h[e]), mx);
+        }
+        if constexpr (ROW_WG) mx = block_max<kColThreads / 64>(mx, redf);
+        else mx = wave_max(mx);
+    }
+    const half_t sh = scale_from_absmax(mx);
+    if (lane == 0) a.scale[row] = sh;
+    const float s = (float)sh, y = 1.0f / s;
+    uint2_t* const orow = reinterpret_cast<uint2_t*>(a.out + row * a.ld);
+    const bool normal = scale_is_normal(sh);       // (the same for the whole row) the short rounding sequence
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int j = lane + i * STEP;
+        int4_t ci = __builtin_bit_cast(int4_t, v[i]);
+        asm volatile("" : "+v"(ci));             // (a piece's fp32 conversions are made where they are used)
+        const half8_t h = __builtin_bit_cast(half8_t, ci);
+        int32_t q[8];
+        if (normal) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q[e] = (int32_t)quant_i8_own_scale_bits((float)h[e], y);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q[e] = quant_i8_rcp((float)h[e], s, y);
+        }
+        if (j < l8) orow[j] = uint2_t{pack4_i8(q[0], q[1], q[2], q[3]), pack4_i8(q[4], q[5], q[6], q[7])};
+    }
+}
+
+template <int OUT, bool NTH, bool UA>
+__global__ __launch_bounds__(kColThreads) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_col_quantize_rows(ColQuantArgs a, int32_t tiles_per_batch, int32_t parts,
+                                                                                                            uint32_t nteams, XchLaunch xl, RowQuantArgs r) {
+    if (blockIdx.x < r.first) {
+        col_quantize_team<kColThreads, OUT, NTH, UA, false>(a, tiles_per_batch, parts, nteams, xl);
+        return;
+    }
+    const uint32_t block = blockIdx.x - r.first;
+    const int32_t len = r.ld;                    // (ld >= m)
+    if (len <= 1024) quantize_row<2, false>(r, block);
+    else if (len <= 2048) quantize_row<4, false>(r, block);
+    else if (len <= 4096) quantize_row<8, false>(r, block);
+    else if (len <= 8192) quantize_row<2, true>(r, block);
+    else if (len <= 12288) quantize_row<3, true>(r, block);
+    else quantize_row<4, true>(r, block);
+}
+
 // Rows r0 .. r0 + 63 of a tile of 64 columns, rounded with the scale of the lane's column, into the wanted outputs (256 threads;
 // the transposed one through `tile`, so that a wave stores 64 bytes of one column and not one of 64).  The surplus of longer
 // rows becomes zeros: rows from n on in the transposed output, columns from m on in the other.
@@ -376,9 +476,10 @@ int cpmk_gemm_round_transpose(int32_t, int32_t, int32_t, const void*, const void
 
 }  // extern "C"
 
-// The team kernel on (batch, n, m): 0, an error code, or -1 when the shape is not one it takes.
+// The team kernel on (batch, n, m): 0, an error code, or -1 when the shape is not one it takes.  rq: rows to quantise beside the (first)
+// launch of the teams; -1 also where they are not of the form that takes.
 template <bool SCALED>
-static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st) {
+static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st, const RowQuantArgs* rq = nullptr) {
     const int32_t n = p.n, m = p.m;
     // a team here exchanges one maximum per column, dealt to all waves, so it may be larger than the teams of the kernels that keep
     // per-part values in registers (kColMaxParts of 512 rows: 16384; far fewer workgroups than are resident at once, which is what progress
@@ -391,6 +492,11 @@ static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st) {
                          (int64_t)n * (p.out_n ? p.ld_n : m) < (1ll << 31) && (int64_t)m * p.ld_t < (1ll << 31) && p.ld_t <= parts * 512 &&
                          parts <= kColMaxParts && tiles * parts <= kXchSlots;
     if (!team_ok) return -1;
+    int64_t row_blocks = 0;
+    if (rq) {
+        row_blocks = rq->ld > 4096 ? rq->rows : ceil_div(rq->rows, kColThreads / 64);
+        if (SCALED || rq->m % 8 || rq->ld % 8 || rq->ld > 16384 || !aligned16(rq->mat) || (reinterpret_cast<uintptr_t>(rq->out) & 7u) || row_blocks > 1 << 21) return -1;
+    }
     // teams use one packet slot per (team, part): batches beyond the pool go out in several launches
     const int64_t per_launch = parts > 1 ? kXchSlots / (tiles * parts) : ((1ll << 31) - 8) / (tiles * parts);
     for (int64_t b0 = 0; b0 < batch; b0 += per_launch) {
@@ -408,12 +514,27 @@ static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st) {
         q.scale += b0 * m;
         if (p.out_t) q.out_t += b0 * m * p.ld_t;
         if (p.out_n) q.out_n += b0 * n * p.ld_n;
+        const int64_t team_blocks = xch_team_grid(tiles * nb, parts);
+        auto go_rows = [&](auto kern) {
+            RowQuantArgs r = *rq;
+            r.first = (uint32_t)team_blocks;
+            hipLaunchKernelGGL(kern, dim3((unsigned)(team_blocks + row_blocks)), dim3(kColThreads), 0, st, q, (int32_t)tiles, (int32_t)parts, (uint32_t)(tiles * nb),
+                               xs.xl, r);
+        };
         auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3((unsigned)xch_team_grid(tiles * nb, parts)), dim3(kColThreads), 0, st, q, (int32_t)tiles, (int32_t)parts,
+            hipLaunchKernelGGL(kern, dim3((unsigned)team_blocks), dim3(kColThreads), 0, st, q, (int32_t)tiles, (int32_t)parts,
                                (uint32_t)(tiles * nb), xs.xl);
         };
         auto pick = [&](auto oc) {
             constexpr int OUT = decltype(oc)::value;
+            if constexpr (!SCALED && (OUT & kOutT) != 0) {
+                if (rq && b0 == 0) {
+                    if (!wide) go_rows(k_col_quantize_rows<OUT, false, true>);
+                    else if (lines) go_rows(k_col_quantize_rows<OUT, true, false>);
+                    else go_rows(k_col_quantize_rows<OUT, false, false>);
+                    return;
+                }
+            }
             if (!wide) go(k_col_quantize_team<kColThreads, OUT, false, true, SCALED>);
             else if (lines) go(k_col_quantize_team<kColThreads, OUT, true, false, SCALED>);
             else go(k_col_quantize_team<kColThreads, OUT, false, false, SCALED>);
@@ -503,6 +624,23 @@ int cpmk_gemm_quantize_cols_ld(int32_t batch, int32_t n, int32_t m, const void* 
         }
     }
     return 0;
+}
+
+int cpmk_gemm_quantize_pair_ld(int64_t, const void*, void*, void*, int64_t, const void*, void*, void*, int32_t, int32_t, void*);   // quant.hip
+
+int cpmk_gemm_quantize_cols_rows(int32_t batch, int32_t n, int32_t m, const void* mat, void* scale, void* out_t, int32_t ld_t, void* out_n, int32_t ld_n,
+                                 int64_t rows, const void* row_mat, void* row_scale, void* row_out, void* stream) {
+    clear_stale_error();
+    if (rows < 0) return CPMK_EBADARG;
+    if (n > 0 && batch > 0 && m > 0 && rows > 0 && scale && mat && out_t && ld_t >= n && ld_t % 16 == 0 && (!out_n || (ld_n >= m && (ld_n == m || ld_n % 16 == 0))) &&
+        !any_null(row_mat, row_scale, row_out)) {
+        const ColQuantArgs p = {n, m, (const half_t*)mat, nullptr, 0, (half_t*)scale, (int8_t*)out_t, (int8_t*)out_n, ld_t, out_n ? ld_n : 0};
+        const RowQuantArgs r = {(const half_t*)row_mat, (half_t*)row_scale, (int8_t*)row_out, n, ld_t, rows, 0};
+        const int rc = col_quantize<false>(batch, p, (hipStream_t)stream, &r);
+        if (rc >= 0) return rc;
+    }
+    if (const int rc = cpmk_gemm_quantize_cols_ld(batch, n, m, mat, nullptr, 0, scale, out_t, ld_t, out_n, ld_n, stream)) return rc;
+    return cpmk_gemm_quantize_pair_ld(rows, row_mat, row_scale, row_out, 0, nullptr, nullptr, nullptr, n, ld_t, stream);
 }
 
 }  // extern "C"

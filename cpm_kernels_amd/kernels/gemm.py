@@ -164,6 +164,17 @@ def gemm_quantize_pair_ld(rows0: int, mat0: DevicePointer, scale0: DevicePointer
     cpmk.gemm_quantize_pair_ld(rows0, mat0, scale0, out0, rows1, mat1, scale1, out1, m, ld, stream)
 
 
+def gemm_quantize_cols_rows(batch: int, n: int, m: int, mat: DevicePointer, scale: DevicePointer,
+                            out_t: DevicePointer, ld_t: int, out_n: DevicePointer, ld_n: int,      # as in gemm_quantize_cols_ld
+                            rows: int,
+                            row_mat: DevicePointer,     # (rows, n)     fp16
+                            row_scale: DevicePointer,   # (rows)        fp16
+                            row_out: DevicePointer,     # (rows, ld_t)  int8
+                            stream: CUDAStream):
+    """The two operands of a product, one quantised along its columns and the other along its rows, in one launch; n <= 16384."""
+    cpmk.gemm_quantize_cols_rows(batch, n, m, mat, scale, out_t, ld_t, out_n, ld_n, rows, row_mat, row_scale, row_out, stream)
+
+
 def gemm_backward_round_scale_ld(batch: int, n: int, m: int, mat: DevicePointer, scale_y: DevicePointer,
                                  out: DevicePointer,        # (batch, n, ld)  int8
                                  ld: int,

@@ -9,7 +9,7 @@ the six-launch sequence, which ``fused=False`` still runs through the kernel-lev
 import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
-    gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_for, gemm_int8_scale_sum, gemm_fp16_sum, \
+    gemm_quantize_cols_ld, gemm_quantize_cols_rows, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_for, gemm_int8_scale_sum, gemm_fp16_sum, \
     gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, gemm_depth_parts, gemm_int8_scale_split, gemm_fp16_split, \
     arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
     transpose_i8_ld
@@ -87,6 +87,23 @@ def _quantize_cols(x, both: bool, row_scale=None):
 
 # Outputs of a product that may be worth dividing along its depth (gemm_depth_parts): a larger one has a tile for every compute unit.
 _PARTS_MOST = 1 << 22
+
+
+def _quantize_cols_rows(x, both: bool, w):
+    """_quantize_cols of x (b, K, m) and _quantize_rows of w (b', rows, K) in one launch, whose streaming of the rows fills the
+    waits of the columns' workgroups."""
+    b, n, m = x.size()
+    if n > 16384:
+        return _quantize_cols(x, both), _quantize_rows(w)[0]
+    ld, ld_n = _row_bytes(n), _row_bytes(m) if both else 0
+    scale = torch.empty((b, m), dtype=torch.half, device=x.device)
+    out_t = torch.empty((b, m, ld), dtype=torch.int8, device=x.device)
+    out_n = torch.empty((b, n, ld_n), dtype=torch.int8, device=x.device) if both else None
+    row_scale = torch.empty(w.shape[:2], dtype=torch.half, device=x.device)
+    row_out = torch.empty((w.size(0), w.size(1), ld), dtype=torch.int8, device=x.device)
+    gemm_quantize_cols_rows(b, n, m, x.data_ptr(), scale.data_ptr(), out_t.data_ptr(), ld, out_n.data_ptr() if both else None, ld_n,
+                            w.size(0) * w.size(1), w.data_ptr(), row_scale.data_ptr(), row_out.data_ptr(), cur_stream())
+    return (scale, out_t, out_n), (row_scale, row_out)
 
 
 def _dims(quantA, quantB, aT, bT):
@@ -188,15 +205,13 @@ class GEMMInt8(torch.autograd.Function):
         own_A = own_B = None
         if not aT and bT:
             (scale_A, quant_A), (scale_B, quant_B) = _quantize_rows(A, B)
+        elif aT and bT:
+            (scale_A, quant_A, own_A), (scale_B, quant_B) = _quantize_cols_rows(A, want_B, B)
+        elif not aT:
+            (scale_B, quant_B, own_B), (scale_A, quant_A) = _quantize_cols_rows(B, want_A, A)
         else:
-            if aT:
-                scale_A, quant_A, own_A = _quantize_cols(A, want_B)
-            else:
-                (scale_A, quant_A), = _quantize_rows(A)
-            if bT:
-                (scale_B, quant_B), = _quantize_rows(B)
-            else:
-                scale_B, quant_B, own_B = _quantize_cols(B, want_A)
+            scale_A, quant_A, own_A = _quantize_cols(A, want_B)
+            scale_B, quant_B, own_B = _quantize_cols(B, want_A)
         if quant_A.size(2) != quant_B.size(2):      # (contractions beyond what the row quantiser holds in registers)
             quant_A, quant_B = (x[:, :, :K].contiguous() for x in (quant_A, quant_B))
         if train:

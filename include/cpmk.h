@@ -177,6 +177,10 @@ int cpmk_gemm_quantize_cols(int32_t batch, int32_t n, int32_t m, const void* mat
  * (a multiple of 16; ld_n may be m). */
 int cpmk_gemm_quantize_cols_ld(int32_t batch, int32_t n, int32_t m, const void* mat, const void* row_scale, int broad_cast_row,
                                void* scale, void* out_t, int32_t ld_t, void* out_n, int32_t ld_n, void* stream);
+/* cpmk_gemm_quantize_cols_ld (without row scales; out_t is wanted) of one operand of a product and cpmk_gemm_quantize_pair_ld of the other,
+ * row_mat (rows, n), row_out (rows, ld_t), in one launch: both contracted over n <= 16384. */
+int cpmk_gemm_quantize_cols_rows(int32_t batch, int32_t n, int32_t m, const void* mat, void* scale, void* out_t, int32_t ld_t, void* out_n, int32_t ld_n,
+                                 int64_t rows, const void* row_mat, void* row_scale, void* row_out, void* stream);
 
 /* ---- fp16 products next to the path (attention scores, fp16 decode) ---------------- */
 /* Same operand convention as cpmk_gemm_int8 with fp16 operands and fp16 output, fp32

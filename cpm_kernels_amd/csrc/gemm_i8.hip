@@ -279,6 +279,7 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
     int batch = batchA > batchB ? batchA : batchB;
     if (m == 0 || n == 0) return 0;
     if (out == nullptr || (k > 0 && any_null(A, B)) || (FUSED && srow == nullptr && scol == nullptr)) return CPMK_EBADARG;
+    const int64_t big_apart = n > 128 && m > 128 ? ceil_div(n, 256) * ceil_div(m, 256) * batch : 0;       // (big_tiles)
     if (batchA == 1 && !bT && (srow == nullptr || !bcr) && (scol == nullptr || bcc) && rows_join(batch, n, k)) {
         n *= batch;
         batch = batchB = 1;
@@ -323,7 +324,7 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
     const bool fast = p_kmajor && q_kmajor && k > 0 && (k % 16 == 0) && aligned16(A) && aligned16(B);
     if (fast && wide && (k % 64 == 0) && (int64_t)n * k < (1ll << 32) && (int64_t)m * k < (1ll << 32)) {
         // 256x256 tiles when they give most compute units a tile, else 128x128
-        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
+        const int64_t big = big_tiles(n, m, batch, big_apart);
         constexpr int EPI = FUSED ? kEpiDequant : kEpiInt32;
         auto kmajor = [&](auto lay) __attribute__((always_inline)) {
             constexpr int LAY = decltype(lay)::value;
@@ -359,7 +360,7 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
     if (p_kmajor && q_kmajor && wide && k > 64 && (k % 4 == 0) && (reinterpret_cast<uintptr_t>(A) & 3u) == 0 &&
         (reinterpret_cast<uintptr_t>(B) & 3u) == 0 && (int64_t)n * k < (1ll << 32) && (int64_t)m * k < (1ll << 32)) {
         constexpr int EPI = FUSED ? kEpiDequant : kEpiInt32;
-        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
+        const int64_t big = big_tiles(n, m, batch, big_apart);
         const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128;
         if (fast) return large ? launch_dma<2, 4, 4, 2, 64, EPI, 4, 4, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 64, EPI, kRingSmall, 4, 32>(a, batch, st);
         return large ? launch_dma<2, 4, 4, 2, 64, EPI, 4, 12, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 64, EPI, kRingSmall, 12, 32>(a, batch, st);
@@ -372,7 +373,7 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
         (!in_q || m >= 128) && (int64_t)n * k < (1ll << 32) && (int64_t)m * k < (1ll << 32)) {
         constexpr int EPI = FUSED ? kEpiDequant : kEpiInt32;
         // 256x256 tiles when they give most compute units a tile, else 128x128 (as for K-major operands)
-        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
+        const int64_t big = big_tiles(n, m, batch, big_apart);
         const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!in_q || m >= 256);
         a.edge_in = (in_p ? 1 : 0) | (in_q ? 2 : 0);
         if constexpr (FUSED) {
@@ -518,6 +519,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     if (m == 0 || n == 0) return 0;
     if (out == nullptr || (k > 0 && any_null(A, B))) return CPMK_EBADARG;
     if (k > (1 << 30)) return CPMK_ETOOBIG;
+    const int64_t big_apart = n > 128 && m > 128 ? ceil_div(n, 256) * ceil_div(m, 256) * batch : 0;       // (big_tiles)
     if (batchA == 1 && !bT && rows_join(batch, n, (int64_t)k * 2)) {
         n *= batch;
         batch = batchB = 1;
@@ -572,7 +574,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         if (const int rc = gemm_f16_low(m, k, n, batchA, batchB, A, B, out, st); rc >= 0) return rc;
     if (p_kmajor && q_kmajor && wide && k > 0 && (k % 32 == 0) && aligned16(A) && aligned16(B) &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
-        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
+        const int64_t big = big_tiles(n, m, batch, big_apart);
         const bool whole128 = k % 64 == 0;       // the depth is whole 128-byte slabs (else whole 64-byte ones: 96, 160 ...)
         a.edge_in = odd ? 2 : 0;
         if (big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!odd || m >= 256)) {
@@ -593,7 +595,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     // from memory into the fragments (large tiles) or as a slab filled up with zeros
     if (p_kmajor && q_kmajor && wide && k > 32 && (reinterpret_cast<uintptr_t>(A) & 3u) == 0 && (reinterpret_cast<uintptr_t>(B) & 3u) == 0 &&
         (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
-        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
+        const int64_t big = big_tiles(n, m, batch, big_apart);
         const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!odd || m >= 256);
         a.edge_in = odd ? 2 : 0;
         if (k % 8 == 0 && aligned16(A) && aligned16(B))       // whole, aligned 16-byte pieces
@@ -623,7 +625,8 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         // four of small ones 181; 1792 x 384 x 24, K = 3592: 257 and 219).
         const bool rest = k % 64 != 0;       // (see below)
         const bool idle = rest && k >= 256 && ceil_div(big * batch, cus) * 9 > ceil_div(mid * batch, cus) * 4;
-        const bool large = !waste && !idle && big * batch * 4 >= cus * 3 && n > 128 && m > 128 && (!in_p || n >= 256) && (!(in_q || odd) || m >= 256);
+        const bool large = !waste && !idle && big_tiles(n, m, batch, big_apart) * 4 >= cus * 3 && n > 128 && m > 128 && (!in_p || n >= 256) &&
+                           (!(in_q || odd) || m >= 256);
         a.edge_in = (in_p ? 1 : 0) | (in_q || odd ? 2 : 0);
         // a depth that is not whole slabs (probabilities x values over 500 keys, scores over heads of 80): its rest is a slab
         // filled up with zeros

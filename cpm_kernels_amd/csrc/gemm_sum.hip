@@ -57,6 +57,47 @@ static int32_t sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t
     return k <= limit ? g : batch;
 }
 
+// The quickest number of groups, whether it fills the device or not.  Up to 512 tiles of 128 x 128 the least of these estimates, in us, over the numbers of groups (int8, fp16 K-major; within 15 % of 130 sizes of
+// 16 to 432 tiles, 2 to 16 entries and depths of 40 to 1024).  A group: 4.5, and for each of its entries 0.40 and 0.45 a slab of 128 bytes (int8: folding,
+// products), or 0.65 a slab (fp16; depths that are not whole ones 0.7 and 0.26 a 64-byte slab, 2.0 and 0.30 where rows are not whole 16-byte
+// pieces), half as much again where int8 tiles share compute units, a round of the device after the other for fp16; several groups 3 and their
+// fp32 sums at 4.7 TB/s.  One by one: 12 (9), results written and read at 5.2 TB/s and products at 4.4 (2.0) PFLOP/s, which large tiles reach half under the writes.
+// Groups / one by one: int8 512 x 512 x 2, k = 128 7 / 16; x 13, 128 15 / 22; 832 x 1856 x 7, 128 11 / 23; x 16, 512 30 (two groups) / 39;
+// fp16 1280 x 3328 x 14, k = 48 28 / 54; 512 x 512 x 6, 512 36 / 14 (one by one).
+static int32_t sum_groups_few(bool i8, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch) {
+    const int64_t cus = compute_units();
+    const float area = (float)n * (float)m * 1e-6f, kb = (float)(i8 ? k : 2 * k);
+    const bool slabs = i8 || k % 64 == 0;
+    const float entry = i8 ? 0.40f + 0.45f * ceilf(kb / 128.0f) : slabs ? 0.65f * kb / 128.0f : k % 8 == 0 ? 0.7f + 0.26f * floorf(kb / 64.0f) : 2.0f + 0.30f * floorf(kb / 64.0f);
+    int32_t best = batch;
+    float best_t = (i8 ? 12.0f : 9.0f) + (float)batch * area * (4.0f / 5.2f + 2.0f * (float)k / (i8 ? 4400.0f : 2000.0f));
+    for (int32_t g = 1; g < batch && g * tiles <= 4 * cus; ++g) {
+        if (batch % g != 0 || batch / g > kSumMax) continue;
+        const int64_t work = tiles * g, last = work % cus;
+        float rounds;
+        if (i8) rounds = work <= cus ? 1.0f : 1.5f * (float)ceil_div(work, 2 * cus);
+        else rounds = (float)(work / cus) + (last == 0 ? 0.0f : 2 * last <= cus && work > cus && slabs ? 0.5f : 1.0f);
+        const float t = 4.5f + rounds * (float)(batch / g) * entry + (g > 1 ? 3.0f + (float)g * area * 8.0f / 4.7f : 0.0f);
+        if (t < best_t) {
+            best_t = t;
+            best = g;
+        }
+    }
+    return best;
+}
+
+// (K, rows): one contraction of all entries where it fits, whose depth is divided among workgroups again where it has few tiles
+// (cpmk_gemm_depth_parts).  Joined / one by one: 1280 x 3328 x 7, k = 100 14 / 32, 1024 86 / 78; 832 x 1856 x 14, 48 10.7 / 26; x 2, 1024 20.6 / 19.3;
+// 512 x 512 x 16, 512 19.3 / 18.4, x 3, 40 8.2 / 13.0.
+static int32_t sum_groups_timed(int kind, int32_t m, int32_t k, int32_t n, int32_t batch) {
+    const int64_t cus = compute_units(), tiles = ceil_div(n, 128) * ceil_div(m, 128);
+    if (kind == kSumI8 ? tiles <= 2 * cus : ceil_div(n, 256) * ceil_div(m, 256) * 4 < cus * 3 && tiles <= 2 * cus) {
+        if (kind != kSumF16KFirst) return sum_groups_few(kind == kSumI8, tiles, m, k, n, batch);
+        if ((int64_t)(m > n ? m : n) * k < (1ll << 31) / batch && k <= (tiles > cus ? 640 : 1023)) return 1;
+    }
+    return sum_groups_for(kind, m, k, n, batch);
+}
+
 // PART: fp32 out.  A group's sum may pass fp16's range where the sum over all groups does not: sums of more than one group stay
 // fp32 until they are added up (cpmk_gemm_add_parts).
 template <bool PART>
@@ -184,6 +225,10 @@ int cpmk_gemm_sum_groups(int32_t m, int32_t n, int32_t batch) {
 
 int cpmk_gemm_sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t batch) {
     return m < 0 || n < 0 || k < 0 || batch < 1 ? 1 : sum_groups_for(kind, m, k, n, batch);
+}
+
+int cpmk_gemm_sum_groups_timed(int kind, int32_t m, int32_t k, int32_t n, int32_t batch) {
+    return m <= 0 || n <= 0 || k <= 0 || batch < 1 ? 1 : sum_groups_timed(kind, m, k, n, batch);
 }
 
 int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,

@@ -196,6 +196,11 @@ def gemm_sum_groups_for(kind: int, m: int, k: int, n: int, batch: int) -> int:
     return cpmk.gemm_sum_groups_for(kind, m, k, n, batch)
 
 
+def gemm_sum_groups_timed(kind: int, m: int, k: int, n: int, batch: int) -> int:
+    """The quickest number of groups, also where it leaves part of the device idle."""
+    return cpmk.gemm_sum_groups_timed(kind, m, k, n, batch)
+
+
 def gemm_int8_scale_sum(m: int, k: int, n: int, batch: int, groups: int,
                         A: DevicePointer,           # (batch, m, k)     int8
                         B: DevicePointer,           # (batch, n, k)     int8

@@ -48,6 +48,7 @@ _CTYPES = {"i": ctypes.c_int32, "l": ctypes.c_int64, "f": ctypes.c_float, "p": c
 EXPORTED_SYMBOLS = sorted(["cpmk_" + n for n in _LAUNCHERS] + [
     "cpmk_version", "cpmk_error_string", "cpmk_device_count", "cpmk_get_device",
     "cpmk_set_device", "cpmk_device_props", "cpmk_exchange_capture_slots_left", "cpmk_gemm_sum_groups", "cpmk_gemm_sum_groups_for",
+    "cpmk_gemm_sum_groups_timed",
     "cpmk_gemm_depth_parts",
 ])
 
@@ -127,6 +128,11 @@ def gemm_sum_groups(m: int, n: int, batch: int) -> int:
 @lib.bind("cpmk_gemm_sum_groups_for", [ctypes.c_int] + [ctypes.c_int32] * 4, ctypes.c_int32)
 def gemm_sum_groups_for(kind: int, m: int, k: int, n: int, batch: int) -> int:
     return lib.cpmk_gemm_sum_groups_for(kind, m, k, n, batch)
+
+
+@lib.bind("cpmk_gemm_sum_groups_timed", [ctypes.c_int] + [ctypes.c_int32] * 4, ctypes.c_int32)
+def gemm_sum_groups_timed(kind: int, m: int, k: int, n: int, batch: int) -> int:
+    return lib.cpmk_gemm_sum_groups_timed(kind, m, k, n, batch)
 
 
 @lib.bind("cpmk_gemm_depth_parts", [ctypes.c_int] + [ctypes.c_int32] * 5 + [ctypes.c_int] * 2, ctypes.c_int32)

@@ -9,7 +9,7 @@ the six-launch sequence, which ``fused=False`` still runs through the kernel-lev
 import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
-    gemm_quantize_cols_ld, gemm_quantize_cols_rows, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_for, gemm_int8_scale_sum, gemm_fp16_sum, \
+    gemm_quantize_cols_ld, gemm_quantize_cols_rows, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_timed, gemm_int8_scale_sum, gemm_fp16_sum, \
     gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, gemm_depth_parts, gemm_int8_scale_split, gemm_fp16_split, \
     arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
     transpose_i8_ld
@@ -54,6 +54,11 @@ def _row_bytes(k: int) -> int:
     return k if k % 128 == 0 or k > 16384 or (k % 64 == 0 and k < 1024) else (k + 127) // 128 * 128
 
 
+def _sum_row_bytes(k: int) -> int:
+    """The same where the product is summed over the batch (gemm_and_scale_sum): whole slabs always."""
+    return _row_bytes(k) if k > 16384 else (k + 127) // 128 * 128
+
+
 def _quantize_rows(*mats):
     """One or two (b, rows, K) operands quantised along K in one launch: [(scale (b, rows), int8 (b, rows, _row_bytes(K)))]"""
     K = mats[0].size(2)
@@ -71,12 +76,14 @@ def _quantize_rows(*mats):
     return out
 
 
-def _quantize_cols(x, both: bool, row_scale=None):
-    """A (b, n, m) operand quantised along n: scale (b, m), int8 (b, m, _row_bytes(n)) and, with `both`, the same values
-    where they were, (b, n, _row_bytes(m)) (else None).  row_scale: of the values multiplied by it, see gemm_backward_scale_round."""
+def _quantize_cols(x, both: bool, row_scale=None, summed: bool = False):
+    """A (b, n, m) operand quantised along n: scale (b, m), int8 (b, m, _row_bytes(n)) -- _sum_row_bytes(n) if `summed` -- and, with
+    `both`, the same values where they were, (b, n, _sum_row_bytes(m)) (else None).  row_scale: of the values multiplied by it, see
+    gemm_backward_scale_round."""
     b, n, m = x.size()
     scale = torch.empty((b, m), dtype=torch.half, device=x.device)
-    ld_t, ld_n = (n + 15) // 16 * 16 if n > 16384 else _row_bytes(n), _row_bytes(m) if both else 0
+    ld_t = (n + 15) // 16 * 16 if n > 16384 else _sum_row_bytes(n) if summed else _row_bytes(n)
+    ld_n = _sum_row_bytes(m) if both else 0
     out_t = torch.empty((b, m, ld_t), dtype=torch.int8, device=x.device)
     out_n = torch.empty((b, n, ld_n), dtype=torch.int8, device=x.device) if both else None
     gemm_quantize_cols_ld(b, n, m, x.data_ptr(), None if row_scale is None else row_scale.data_ptr(),
@@ -95,7 +102,7 @@ def _quantize_cols_rows(x, both: bool, w):
     b, n, m = x.size()
     if n > 16384:
         return _quantize_cols(x, both), _quantize_rows(w)[0]
-    ld, ld_n = _row_bytes(n), _row_bytes(m) if both else 0
+    ld, ld_n = _row_bytes(n), _sum_row_bytes(m) if both else 0
     scale = torch.empty((b, m), dtype=torch.half, device=x.device)
     out_t = torch.empty((b, m, ld), dtype=torch.int8, device=x.device)
     out_n = torch.empty((b, n, ld_n), dtype=torch.int8, device=x.device) if both else None
@@ -170,7 +177,7 @@ def gemm_and_scale_sum(quantA, scaleA, quantB) -> torch.Tensor:
     """(1, M, N): the sum over the batch of scaleA * (quantA x quantB^T), quantA (b, M, K) and quantB (b, N, K)."""
     batch, M, K = quantA.size()
     N = quantB.size(1)
-    groups = gemm_sum_groups_for(0, N, K, M, batch)
+    groups = gemm_sum_groups_timed(0, N, K, M, batch)
     if groups == batch or quantB.size(0) != batch or K == 0 or K % 128 != 0 or max(M, N) * K >= 2 ** 31 or batch * K >= 2 ** 22:
         return _sum_entries(gemm_and_scale(quantA, scaleA, quantB, None, False, True))
     parts = torch.empty((groups, M, N), dtype=torch.half if groups == 1 else torch.float32, device=quantA.device)
@@ -237,12 +244,12 @@ class GEMMInt8(torch.autograd.Function):
             own_A, own_B = ctx.own
             grad_A = grad_B = None
             if ctx.needs_input_grad[0]:                                     # contracted over N
-                ld = _row_bytes(N)
+                summed = scale_A.size(0) == 1 and batch > 1 and not aT
+                ld = quantized_B.size(2) if own_B else _sum_row_bytes(N) if summed else _row_bytes(N)
                 scale_G = torch.empty((batch, M), dtype=torch.half, device=grad_f.device)
                 quant_G = torch.empty((batch, M, ld), dtype=torch.int8, device=grad_f.device)
                 gemm_backward_round_scale_ld(batch, M, N, grad_f.data_ptr(), scale_B.data_ptr(), quant_G.data_ptr(), ld,
                                              scale_G.data_ptr(), scale_B.size(0) == 1, st)
-                summed = scale_A.size(0) == 1 and batch > 1 and not aT
                 other, lies = _contracted(quantized_B, K, N, ld, own_B, summed)
                 if aT:              # grad_A (b, K, M), scaled per column m
                     grad_A = gemm_and_scale(other, None, quant_G, scale_G, lies, True)
@@ -254,8 +261,8 @@ class GEMMInt8(torch.autograd.Function):
                 if scale_A.size(0) == 1 and grad_A.size(0) > 1:
                     grad_A = grad_A.sum(dim=0, keepdim=True)
             if ctx.needs_input_grad[2]:                                     # contracted over M
-                scale_G, quant_G, _ = _quantize_cols(grad_f, False, scale_A)
                 summed = scale_B.size(0) == 1 and batch > 1 and bT
+                scale_G, quant_G, _ = _quantize_cols(grad_f, False, scale_A, summed or own_A)
                 other, lies = _contracted(quantized_A, K, M, quant_G.size(2), own_A, summed)
                 if summed:
                     grad_B = gemm_and_scale_sum(quant_G, scale_G, other)
@@ -344,7 +351,7 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
 def _entry_groups(M: int, K: int, N: int, batch: int, joined: bool) -> int:
     """Groups that an fp16 product summed over the batch is formed in.  `joined`: both operands stored (K, rows), so that a group's
     entries are one contraction."""
-    return gemm_sum_groups_for(2 if joined else 1, N, K, M, batch)
+    return gemm_sum_groups_timed(2 if joined else 1, N, K, M, batch)
 
 
 def gemm_pth_fp16_sum(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch.Tensor:

@@ -199,6 +199,8 @@ int cpmk_gemm_fp16(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batc
  * cpmk_gemm_sum_groups_for: the same for a depth k an entry, or `batch` where one product per entry and the sum of them is the quicker.
  * kind 0: int8, 1: fp16, 2: fp16 with operands stored (batch, k, m) and (batch, k, n). */
 int cpmk_gemm_sum_groups(int32_t m, int32_t n, int32_t batch);
+/* cpmk_gemm_sum_groups_timed: the quickest number of groups, whether they fill the device or not. */
+int cpmk_gemm_sum_groups_timed(int kind, int32_t m, int32_t k, int32_t n, int32_t batch);
 int cpmk_gemm_sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t batch);
 int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                              const void* scale_row, void* out, void* stream);

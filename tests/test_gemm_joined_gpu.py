@@ -3,6 +3,7 @@ import pytest
 import torch
 
 import cpm_kernels_amd.kernels as ck
+import cpm_kernels_amd.torch as ct
 from util import stream
 
 pytestmark = pytest.mark.gpu
@@ -94,3 +95,28 @@ def test_parts_are_refused_elsewhere():
     assert ck.gemm_depth_parts(False, 64, 320, 128, 1, 1, True, False) == 1
     with pytest.raises(RuntimeError):
         _whole(A, B, False, s_row, s_col, 320, 2)
+
+
+@pytest.mark.parametrize("rows", [True, False])
+@pytest.mark.parametrize("batch,tokens,din,dout", [(2, 4, 128, 132), (13, 64, 832, 260), (5, 192, 132, 1024), (16, 68, 640, 640), (3, 512, 512, 2304)])
+def test_weight_gradient_of_few_tiles(rows, batch, tokens, din, dout):
+    """int8: against the separate launches, whose entries are rounded to fp16 before they are added (and once more behind that); fp16: in 64 bits"""
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    x = torch.randn((batch, tokens, din) if rows else (batch, din, tokens), generator=g, device="cuda").half()
+    w = (torch.randn((1, dout, din), generator=g, device="cuda") * 0.02).half().requires_grad_()
+    grad = (torch.randn((batch, tokens, dout) if rows else (batch, dout, tokens), generator=g, device="cuda") * 0.05).half()
+
+    def product(w, x, grad, **how):
+        out = ct.bmm(x, False, w, True, **how) if rows else ct.bmm(w, False, x, False, **how)
+        return torch.autograd.grad(out, w, grad)[0]
+    ours = product(w, x, grad, int8=True).double()
+    apart = [product(w, x[i:i + 1].contiguous(), grad[i:i + 1].contiguous(), int8=True, fused=False).double() for i in range(batch)]
+    bound = sum(a.abs() * 2.0 ** -11 + 2.0 ** -25 for a in apart) * (1 + batch * 2.0 ** -12)
+    want = sum(apart)
+    assert ((ours - want).abs() <= bound + want.abs() * 2.0 ** -11 + 2.0 ** -25).all()
+    xd, gd = (t.double() if rows else t.double().transpose(1, 2).contiguous() for t in (x, grad))
+    want = sum(gd[i].t().contiguous() @ xd[i] for i in range(batch))
+    size = sum(gd[i].abs().t().contiguous() @ xd[i].abs() for i in range(batch))
+    ours = product(w, x, grad, int8=False).double()[0]
+    rounded = sum((gd[i].t().contiguous() @ xd[i]).abs() for i in range(batch)) * 2.0 ** -11        # (where entries are formed one by one)
+    assert ((ours - want).abs() <= rounded + size * (batch * tokens) * 2.0 ** -24 + want.abs() * 2.0 ** -10.9 + batch * 2.0 ** -25).all()

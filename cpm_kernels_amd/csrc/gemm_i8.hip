@@ -22,7 +22,7 @@
 //                  (rows of whole 16-byte pieces), gathering the MFMA fragments element by element.
 //   k_gemm_kmajor  both operands K-major, k % 16 == 0 (16-byte loads) or any k % 4 == 0 (4-byte loads): register-staged 64-byte K slabs.
 //   k_gemm_generic any layout and size: LDS tiles + v_dot4_i32_i8.
-// The tile kernel also serves the fp16 product of kernels/gemm.py:188-256 (cpmk_gemm_fp16): the
+// The tile kernel also serves the fp16 products (gemm_f16.hip): the
 // same bytes of K per lane feed v_mfma_f32_16x16x32_f16 / v_mfma_f32_32x32x16_f16, with fp32 accumulators.
 #include "gemm_tile.h"
 
@@ -416,258 +416,6 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
     return 0;
 }
 
-// ---------------------------------------------------------------------------------------
-// fp16 product (fp32 accumulation), any layout, size and alignment: 64x64 output tile, 64 halves of K per
-// stage, four waves of one 32x32 MFMA tile each.  Shapes that are whole slabs and pieces run on the tile
-// kernel above instead.
-// ---------------------------------------------------------------------------------------
-// V: halves per global access (4, 2 or 1: what the contiguous dimension of both operands and the alignment of the buffers allow).
-template <int V>
-__global__ __launch_bounds__(256) void k_gemm_f16_generic(GemmArgs a, int p_kmajor, int q_kmajor, int32_t row_base) {
-    // Guarded loads bring a 64 x 64 piece of each operand into LDS with K contiguous (zeros past the edges,
-    // so any size, layout and alignment works); each of the four waves then owns a 32 x 32 quarter of the tile and
-    // multiplies with v_mfma_f32_32x32x16_f16.
-    constexpr int T = 64, GK = 64, LD = GK + 4;        // rows of 136 bytes: 8-byte aligned fragment reads, spread over the banks
-    __shared__ __attribute__((aligned(16))) half_t sP[T * LD];
-    __shared__ __attribute__((aligned(16))) half_t sQ[T * LD];
-    const int b = blockIdx.z;
-    const int32_t k = a.k >> 1;                        // a.k is the row length in bytes
-    const half_t* P = reinterpret_cast<const half_t*>(a.P + (int64_t)b * a.strideP);
-    const half_t* Q = reinterpret_cast<const half_t*>(a.Q + (int64_t)b * a.strideQ);
-    const int32_t j0 = row_base + blockIdx.y * T, i0 = blockIdx.x * T;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const int lrow = lane & 31, lk = lane >> 5;
-    float16_tv acc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-    typedef _Float16 halfV_t __attribute__((ext_vector_type(V > 1 ? V : 2)));
-    // V halves of one operand's piece: along K for a K-major operand (one row), along the rows for one stored (K, rows).
-    // A stage's pieces are requested one stage ahead into registers, so that their latency passes under the products.
-    constexpr int S = T * GK / V / 256;       // accesses per thread, operand and stage
-    auto place = [&](int kmajor, int q, int& r, int& kk) __attribute__((always_inline)) {
-        if (kmajor) { r = q / (GK / V); kk = (q % (GK / V)) * V; } else { r = (q % (T / V)) * V; kk = q / (T / V); }
-    };
-    auto fetch = [&](half_t (&v)[V], const half_t* G, int kmajor, int32_t r0, int32_t L, int32_t k0, int q) __attribute__((always_inline)) {
-        int r, kk;
-        place(kmajor, q, r, kk);
-        const int32_t row = r0 + r, kg = k0 + kk;
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[e] = (half_t)0.0f;
-        if (row < L && kg < k) {            // (L and k are multiples of V where the access runs along them)
-            const half_t* src = kmajor ? G + ((int64_t)row * k + kg) : G + ((int64_t)kg * L + row);
-            if constexpr (V > 1) {
-                const halfV_t t = *reinterpret_cast<const halfV_t*>(src);
-#pragma unroll
-                for (int e = 0; e < V; ++e) v[e] = t[e];
-            } else {
-                v[0] = *src;
-            }
-        }
-    };
-    auto put = [&](half_t* sm, const half_t (&v)[V], int kmajor, int q) __attribute__((always_inline)) {
-        int r, kk;
-        place(kmajor, q, r, kk);
-#pragma unroll
-        for (int e = 0; e < V; ++e) sm[kmajor ? r * LD + kk + e : (r + e) * LD + kk] = v[e];
-    };
-    half_t rp[S][V], rq[S][V];
-    auto fetch_all = [&](int32_t k0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            fetch(rp[s], P, p_kmajor, j0, a.n, k0, tid + s * 256);
-            fetch(rq[s], Q, q_kmajor, i0, a.m, k0, tid + s * 256);
-        }
-    };
-    fetch_all(0);
-    for (int32_t k0 = 0; k0 < k; k0 += GK) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            put(sP, rp[s], p_kmajor, tid + s * 256);
-            put(sQ, rq[s], q_kmajor, tid + s * 256);
-        }
-        __syncthreads();
-        if (k0 + GK < k) fetch_all(k0 + GK);
-#pragma unroll
-        for (int ks = 0; ks < GK / 16; ++ks) {
-            // lane (lrow, lk): the 8 halves k = 16 ks + 8 lk .. + 7 of its row / column, as two 8-byte reads
-            const half_t* pp = sP + (wr * 32 + lrow) * LD + ks * 16 + lk * 8;
-            const half_t* qp = sQ + (wc * 32 + lrow) * LD + ks * 16 + lk * 8;
-            const half4_t p0 = *reinterpret_cast<const half4_t*>(pp), p1 = *reinterpret_cast<const half4_t*>(pp + 4);
-            const half4_t q0 = *reinterpret_cast<const half4_t*>(qp), q1 = *reinterpret_cast<const half4_t*>(qp + 4);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_shufflevector(p0, p1, 0, 1, 2, 3, 4, 5, 6, 7),
-                                                         __builtin_shufflevector(q0, q1, 0, 1, 2, 3, 4, 5, 6, 7), acc, 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    // accumulator register e of lane l: output row (e / 4) * 8 + (l / 32) * 4 + e % 4, column l % 32 of the wave's quarter
-    const int64_t obase = (int64_t)b * a.n * a.m;
-    const int32_t col = i0 + wc * 32 + lrow;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int32_t row = j0 + wr * 32 + (e >> 2) * 8 + lk * 4 + (e & 3);
-        if (row < a.n && col < a.m) reinterpret_cast<half_t*>(a.out)[obase + (int64_t)row * a.m + col] = (half_t)acc[e];
-    }
-}
-
-static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT,
-                             const void* A, const void* B, void* out, hipStream_t st) {
-    if (m < 0 || n < 0 || k < 0 || batchA < 1 || batchB < 1) return CPMK_EBADARG;
-    if ((m % 2) || (n % 2) || (k % 2)) return CPMK_EALIGN;      // kernels/gemm.py:200
-    if (!(batchA == batchB || batchA == 1 || batchB == 1)) return CPMK_EBADARG;   // :201
-    int batch = batchA > batchB ? batchA : batchB;
-    if (m == 0 || n == 0) return 0;
-    if (out == nullptr || (k > 0 && any_null(A, B))) return CPMK_EBADARG;
-    if (k > (1 << 30)) return CPMK_ETOOBIG;
-    const int64_t big_apart = n > 128 && m > 128 ? ceil_div(n, 256) * ceil_div(m, 256) * batch : 0;       // (big_tiles)
-    if (batchA == 1 && !bT && rows_join(batch, n, (int64_t)k * 2)) {
-        n *= batch;
-        batch = batchB = 1;
-    }
-    if (batch > 65535) {      // (grid z: at most 65535 batch entries per call)
-        for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
-            const int32_t nb = (int32_t)(batch - b0 < 65535 ? batch - b0 : 65535);
-            const int rc = gemm_f16_dispatch(m, k, n, batchA == 1 ? 1 : nb, batchB == 1 ? 1 : nb, aT, bT,
-                                             (const half_t*)A + (batchA == 1 ? 0 : b0 * m * k), (const half_t*)B + (batchB == 1 ? 0 : b0 * n * k),
-                                             (half_t*)out + b0 * n * m, st);
-            if (rc != 0) return rc;
-        }
-        return 0;
-    }
-    GemmArgs a;
-    a.P = (const int8_t*)B; a.Q = (const int8_t*)A; a.out = out;
-    a.srow = nullptr; a.scol = nullptr;
-    a.strideP = batchB == 1 ? 0 : (int64_t)n * k * 2;          // bytes
-    a.strideQ = batchA == 1 ? 0 : (int64_t)m * k * 2;
-    a.n = n; a.m = m; a.k = k * 2; a.bc_row = 0; a.bc_col = 0;
-    a.tiles_r = a.tiles_c = 0;
-    a.edge_in = 0;
-    a.nsum = 1;
-    a.kmagic = 0;
-    a.seg = 0;
-    a.segmagic = 0;
-    // The tile kernel stores 16-byte pieces of output rows that start on dwords, and 8-byte halves at a row's end.  Rows of 4j + 2
-    // elements end in neither: their last column tile lies inside the matrix (edge_in), which takes a matrix of at least one tile.
-    const bool odd = m % 4 != 0;
-    // (The line at 192 columns was drawn for depths up to 128 with both operands stored (K, rows), which have a kernel of their own now; what it still keeps on
-    // the general kernel is deeper or stored otherwise and would mostly be quicker on the tiles from 128 columns on: 80 of 150 x 150, both stored (K, rows),
-    // K = 256 22.6 us and 8.6, K = 512 42.6 and 12.2; both K-major, K = 512 15.8 and 11.4, 300 of 130 x 130, K = 1000 84 and 103.)
-    const bool wide = (reinterpret_cast<uintptr_t>(out) & 3u) == 0 && (!odd || m >= 192);
-    const bool p_kmajor = !bT, q_kmajor = aT != 0;
-    // A depth up to 128: a kernel of its own -- but where the output's rows are not whole cache lines and it exceeds half of the last-level
-    // cache, the tile kernel, whose large tiles share fewer of the lines (1024 of 500 x 500, K = 64 149 us, 162 there; 100 of 1000 x 1000 52.6 and
-    // 56.4; 250 of 500 x 500 32.7 and 25.1), unless those cover much more than the matrix (1500 of 300 x 300 179 and 113).  And the tile kernel
-    // too, beyond a quarter of that cache, where its large tiles cover no more than the small ones do, of which the last overlap the ones before
-    // them: for depths of two slabs (7659 of 136 x 192, K = 128 217 us, 245 there; 976 of 200 x 1024 145 and 161; 5425 of 192 x 192 187 and 199), and
-    // for an operand shared by the batch that is one large tile, of one whole slab or of two (2034 of 192 x 512 with the 192 shared, K = 64 104 and
-    // 119; with the 512 shared 111 and 68; 976 of 400 x 512, the 400 shared, 106 and 71), or of two if it is the row operand (the same, K = 128, 134 and 146).
-    if (!p_kmajor && !q_kmajor && k > 0 && k <= 128) {
-        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256), mid = ceil_div(n, 128) * ceil_div(m, 128), area = (int64_t)n * m, outs = batch * area;
-        const bool large = big * 8 <= mid * 3 && big * batch * 4 >= (int64_t)compute_units() * 3;
-        const bool exact = big * 4 == mid && (n % 8 == 0 || n >= 256) && (m % 8 == 0 || m >= 256) && wide && aligned16(A) && aligned16(B);
-        const bool overlap = batchA == batchB ? k > 112 && mid * 65536 > 5 * area
-                                              : mid * 131072 > 9 * area && (batchB == 1 ? k > 112 || (k == 64 && n <= 256) : m <= 256 && (k == 64 || k > 112));
-        if (!large || ((m % 64 == 0 || outs <= 1 << 26) && !(exact && overlap && outs > 1 << 25)))
-            if (const int rc = gemm_f16_short(m, k, n, batchA, batchB, A, B, out, st); rc >= 0) return rc;
-    }
-    if (p_kmajor && !q_kmajor && n <= 64 && k > 0)       // probabilities x values
-        if (const int rc = gemm_f16_low(m, k, n, batchA, batchB, A, B, out, st); rc >= 0) return rc;
-    if (p_kmajor && q_kmajor && wide && k > 0 && (k % 32 == 0) && aligned16(A) && aligned16(B) &&
-        (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
-        const int64_t big = big_tiles(n, m, batch, big_apart);
-        const bool whole128 = k % 64 == 0;       // the depth is whole 128-byte slabs (else whole 64-byte ones: 96, 160 ...)
-        a.edge_in = odd ? 2 : 0;
-        if (big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!odd || m >= 256)) {
-            if (whole128 && k >= 256) return launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 0, 16>(a, batch, st);
-            // Products of a few slabs -- attention scores, K = 64 -- are all prologue and epilogue, bound by the stores (and
-            // depths of whole 64-byte slabs only need this form anyway):
-            // the 32x32 form is quicker there, and waves of 64 rows x 128 columns, whose row segments are 256 bytes,
-            // store 5-15 % faster than waves of 128 x 64 (slabs of 64 bytes make room for their wider output strips)
-            return launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, 0, 32>(a, batch, st);
-        }
-        if (!whole128) return launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, 0, 32>(a, batch, st);
-        // (as for int8: more 128x128 tiles than compute units but at most two each -> two workgroups per compute unit)
-        const int64_t mid = ceil_div(n, 128) * ceil_div(m, 128) * batch, cus = compute_units();
-        if (mid > cus && mid <= 2 * cus) return launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 0, 32>(a, batch, st, 2);
-        return launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 0, 32>(a, batch, st);
-    }
-    // a depth that is not whole 64-byte slabs (K = 40, 72, 500, 1000 ...): the same kernels, the rest of the depth straight
-    // from memory into the fragments (large tiles) or as a slab filled up with zeros
-    if (p_kmajor && q_kmajor && wide && k > 32 && (reinterpret_cast<uintptr_t>(A) & 3u) == 0 && (reinterpret_cast<uintptr_t>(B) & 3u) == 0 &&
-        (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
-        const int64_t big = big_tiles(n, m, batch, big_apart);
-        const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!odd || m >= 256);
-        a.edge_in = odd ? 2 : 0;
-        if (k % 8 == 0 && aligned16(A) && aligned16(B))       // whole, aligned 16-byte pieces
-            return large ? launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, 4, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, 4, 32>(a, batch, st);
-        return large ? launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, 12, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, 12, 32>(a, batch, st);
-    }
-    // an operand stored (K, rows): the tile kernel reads it as it lies, with transposing LDS reads for the fragments
-    // (rows of such an operand that are not whole 16-byte pieces: tiles that stay inside the matrix, which takes a matrix of at
-    // least one tile)
-    const bool in_p = !p_kmajor && n % 8 != 0, in_q = !q_kmajor && m % 8 != 0;
-    // 64 x 256 tiles for few output rows (attention: probabilities x values)
-    const bool low = n <= 64 && !((in_q || odd) && m < 256);
-    if (!(p_kmajor && q_kmajor) && wide && k >= 64 && aligned16(A) && aligned16(B) &&
-        (!in_p || n >= 128) && (!in_q || m >= (low ? 256 : 128)) &&
-        (int64_t)n * k * 2 < (1ll << 32) && (int64_t)m * k * 2 < (1ll << 32)) {
-        const int lay = (p_kmajor ? 0 : 1) | (q_kmajor ? 0 : 2);
-        // 256x256 tiles when they give most compute units a tile, else 128x128 (as for K-major operands) -- and when the
-        // larger ones cover over half as much again as the smaller ones do, where that costs more than their better ratio of products to reads
-        // saves: 300 x 300 over 400 heads, both stored (K, rows), K = 512 140 us with large tiles, 120 us with small ones, K = 160 70 and 46 us;
-        // 580 x 580 (1.44 times the area) alike; with one operand K-major and K = 80 70 us with large tiles, 74 us with small ones.
-        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256), mid = ceil_div(n, 128) * ceil_div(m, 128);
-        // (not where the large tiles are one round of the device: 384 x 384 over 50 heads, K = 1024 28 us with large tiles, 38 us with small ones)
-        const int64_t cus = compute_units();
-        const bool waste = big * 8 > mid * 3 && (lay == 3 || k >= 256) && big * batch > cus;
-        // At depths that are not whole slabs no last round is split into half tiles, and whole rounds of the device count: a large tile takes
-        // as long as two to two and a half small ones (3592 x 384 over 4 entries, K = 8576 and the rest 8: two rounds of large tiles 226 us,
-        // four of small ones 181; 1792 x 384 x 24, K = 3592: 257 and 219).
-        const bool rest = k % 64 != 0;       // (see below)
-        const bool idle = rest && k >= 256 && ceil_div(big * batch, cus) * 9 > ceil_div(mid * batch, cus) * 4;
-        const bool large = !waste && !idle && big_tiles(n, m, batch, big_apart) * 4 >= cus * 3 && n > 128 && m > 128 && (!in_p || n >= 256) &&
-                           (!(in_q || odd) || m >= 256);
-        a.edge_in = (in_p ? 1 : 0) | (in_q || odd ? 2 : 0);
-        // a depth that is not whole slabs (probabilities x values over 500 keys, scores over heads of 80): its rest is a slab
-        // filled up with zeros
-        // more 128x128 tiles than compute units but at most two each: two workgroups a compute unit, as for K-major operands (2460 x 384 over
-        // 7 entries, K = 6144, 420 tiles: 144 -> 120 us; 300 tiles of 640 x 640, K = 2048: 50 -> 37 us)
-        const bool two = mid * batch > cus && mid * batch <= 2 * cus;
-        switch (lay) {
-            case 1:
-                if (low) return rest ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 13, 32>(a, batch, st) : launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 1, 32>(a, batch, st);
-                if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 13, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 1, 16>(a, batch, st);
-                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 13, 32>(a, batch, st)
-                     : two ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 1, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 1, 32>(a, batch, st);
-            case 2:
-                if (low) return rest ? launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 14, 32>(a, batch, st) : launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 2, 32>(a, batch, st);
-                if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 14, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 2, 16>(a, batch, st);
-                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 14, 32>(a, batch, st)
-                     : two ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 2, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 2, 32>(a, batch, st);
-            default:
-                if (low && !rest) return launch_dma<1, 4, 2, 2, 128, kEpiF16, 3, 3, 32>(a, batch, st);
-                if (large) return rest ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 15, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, 3, 16>(a, batch, st);
-                return rest ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 15, 32>(a, batch, st, 2)
-                     : two ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 3, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 3, 32>(a, batch, st);
-        }
-    }
-    for (int64_t r0 = 0; r0 < n; r0 += 65535ll * 64) {        // (rows beyond the grid's y dimension: several launches)
-        const int64_t nr = n - r0 < 65535ll * 64 ? n - r0 : 65535ll * 64;
-        dim3 grid((unsigned)ceil_div(m, 64), (unsigned)ceil_div(nr, 64), (unsigned)batch);
-        // the widest access both operands allow: their contiguous dimension a multiple of it, their buffers aligned to it
-        const int32_t cp = p_kmajor ? k : n, cq = q_kmajor ? k : m;
-        const uintptr_t al = reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B);
-        if (cp % 4 == 0 && cq % 4 == 0 && (al & 7u) == 0)
-            hipLaunchKernelGGL(k_gemm_f16_generic<4>, grid, dim3(256), 0, st, a, (int)p_kmajor, (int)q_kmajor, (int32_t)r0);
-        else if (cp % 2 == 0 && cq % 2 == 0 && (al & 3u) == 0)
-            hipLaunchKernelGGL(k_gemm_f16_generic<2>, grid, dim3(256), 0, st, a, (int)p_kmajor, (int)q_kmajor, (int32_t)r0);
-        else
-            hipLaunchKernelGGL(k_gemm_f16_generic<1>, grid, dim3(256), 0, st, a, (int)p_kmajor, (int)q_kmajor, (int32_t)r0);
-        if (int e = launch_status()) return e;
-    }
-    return 0;
-}
-
 }  // namespace cpmk
 
 using namespace cpmk;
@@ -696,12 +444,6 @@ int cpmk_gemm_int8_scale_one(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     clear_stale_error();
     return gemm_dispatch<true>(m, k, n, batchA, batchB, aT, bT, A, B, scale_row, scale_col, broad_cast_row,
                                broad_cast_col, out, (hipStream_t)stream);
-}
-
-int cpmk_gemm_fp16(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT,
-                   const void* A, const void* B, void* out, void* stream) {
-    clear_stale_error();
-    return gemm_f16_dispatch(m, k, n, batchA, batchB, aT, bT, A, B, out, (hipStream_t)stream);
 }
 
 }  // extern "C"

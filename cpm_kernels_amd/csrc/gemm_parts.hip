@@ -145,7 +145,7 @@ static int parts_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t bat
 // outputs 0.31 (0.34), start and end of the product 4.5, the second kernel 3 and the time to write and read the parts at 4.7 TB/s.  Whole / divided:
 // int8 120 x 3904, K = 4096 15.3 / 14.0 (3 parts, left whole), 8192 25.0 / 16.0 (6), 12160 34.3 / 18.3 (8); 136 x 3200 over 5 entries, K = 8192 39.5 / 33.2 (3);
 // 512 x 4096, K = 12160 38.2 / 36.0 (2, left whole); fp16 56 x 4608, K = 1024 12.0 / 10.1 (left whole), 2048 19.1 / 11.6 (4), 9664 69 / 20.6 (6).
-static int32_t depth_parts(bool f16, int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT) {
+static int32_t depth_parts(bool f16, int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, float* time = nullptr) {
     PartsForm f;
     if (!parts_form(f16, m, k, n, batchA, batchB, aT, bT, true, true, f)) return 1;
     const int64_t cus = compute_units();
@@ -164,7 +164,34 @@ static int32_t depth_parts(bool f16, int32_t m, int32_t k, int32_t n, int32_t ba
             best = s;
         }
     }
+    if (best > 1 && time) *time = best_t;
     return best;
+}
+
+// fp16, a weight A (1, n, k) [(1, k, n) if aT] beside entries B (batch, k, m) of few columns: whether a copy of the entries as (batch, m, k) pays.  Then
+// they are joined to one product and its depth may be divided, where entries stored (K, rows) of less than a tile, or of rows that are not whole
+// 16-byte pieces, are a tile or more each, on the kernel for any size or on the tile kernel.  Estimates in us as above, within 20 % at
+// columns x entries x k beside rows (direct / with the copy, us): 36 x 1 x 4096 beside 1024 65 / 18, 40 x 1 13 / 19; 100 x 16 x 1024 beside 4608 49 / 29, 104 x 16
+// 38 / 28, 240 x 16 51 / 54; 40 x 5 x 9664 beside 4608 59 / 40; 188 x 1 x 4096 beside 1024 33 / 20, 36 x 5 x 512 beside 2048 10.7 / 14.2.
+static bool copy_pays(int32_t n, int32_t k, int32_t m, int32_t batch, int aT) {
+    if (m >= 512 || k < 256 || n < 128) return false;
+    const int64_t cus = compute_units(), cols = (int64_t)m * batch;
+    if (cols * k >= 1ll << 30) return false;
+    const float slabs = (float)k / 64.0f;
+    auto tiled = [&](int64_t rt, int64_t width, int64_t entries, float one) {
+        const int64_t t = rt * ceil_div(width, 128) * entries, big = ceil_div(n, 256) * ceil_div(width, 256) * entries;
+        if (big * 4 >= cus * 3 && n > 128 && width > 128) return (float)ceil_div(big, cus) * (slabs * 1.25f + 8.0f);
+        if (t <= cus) return 4.5f + slabs * one;
+        if (t <= 2 * cus) return 5.0f + slabs * one * 1.8f;
+        return (float)ceil_div(t, cus) * (slabs * one + 3.5f);
+    };
+    const int64_t rt = ceil_div(n, 128);
+    const bool whole = k % 64 == 0, join = m % 4 == 0 && (!aT || n % 8 == 0);
+    float direct = m % 8 != 0 && m < 128 ? 3.0f + slabs * (m <= 64 ? 1.4f : 2.4f) : tiled(rt, m, batch, whole ? 0.44f : 0.5f);
+    depth_parts(true, m, k, n, batch, 1, 0, aT, &direct);
+    float joined = tiled(rt, join ? cols : m, join ? 1 : batch, whole ? 0.44f : aT ? 0.5f : 0.85f);
+    depth_parts(true, m, k, n, batch, 1, 1, aT, &joined);
+    return joined + 7.0f + 1e-6f * (float)cols * (float)k < 0.93f * direct;
 }
 
 }  // namespace cpmk
@@ -175,6 +202,10 @@ extern "C" {
 
 int cpmk_gemm_depth_parts(int f16, int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT) {
     return m <= 0 || n <= 0 || k <= 0 || batchA < 1 || batchB < 1 ? 1 : depth_parts(f16 != 0, m, k, n, batchA, batchB, aT, bT);
+}
+
+int cpmk_gemm_fp16_copy_pays(int32_t m, int32_t k, int32_t n, int32_t batch, int bT) {
+    return m > 0 && n > 0 && k > 0 && batch > 0 && copy_pays(n, k, m, batch, bT) ? 1 : 0;
 }
 
 int cpmk_gemm_int8_scale_split(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, const void* A, const void* B,

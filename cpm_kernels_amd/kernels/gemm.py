@@ -256,6 +256,11 @@ def gemm_depth_parts(f16: bool, m: int, k: int, n: int, batchA: int, batchB: int
     return cpmk.gemm_depth_parts(1 if f16 else 0, m, k, n, batchA, batchB, 1 if aT else 0, 1 if bT else 0)
 
 
+def gemm_fp16_copy_pays(m: int, k: int, n: int, batch: int, bT: bool) -> bool:
+    """Whether gemm_fp16 of A (batch, k, m) beside one B for all of them is quicker with a copy of A as (batch, m, k)."""
+    return cpmk.gemm_fp16_copy_pays(m, k, n, batch, 1 if bT else 0) != 0
+
+
 def gemm_int8_scale_split(m: int, k: int, n: int, batchA: int, batchB: int, aT: bool, bT: bool,
                           A: DevicePointer, B: DevicePointer, scale_row: DevicePointer, scale_col: DevicePointer,
                           broad_cast_row: bool, broad_cast_col: bool,

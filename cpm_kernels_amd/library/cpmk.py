@@ -49,7 +49,7 @@ EXPORTED_SYMBOLS = sorted(["cpmk_" + n for n in _LAUNCHERS] + [
     "cpmk_version", "cpmk_error_string", "cpmk_device_count", "cpmk_get_device",
     "cpmk_set_device", "cpmk_device_props", "cpmk_exchange_capture_slots_left", "cpmk_gemm_sum_groups", "cpmk_gemm_sum_groups_for",
     "cpmk_gemm_sum_groups_timed",
-    "cpmk_gemm_depth_parts",
+    "cpmk_gemm_depth_parts", "cpmk_gemm_fp16_copy_pays",
 ])
 
 
@@ -138,6 +138,11 @@ def gemm_sum_groups_timed(kind: int, m: int, k: int, n: int, batch: int) -> int:
 @lib.bind("cpmk_gemm_depth_parts", [ctypes.c_int] + [ctypes.c_int32] * 5 + [ctypes.c_int] * 2, ctypes.c_int32)
 def gemm_depth_parts(f16: int, m: int, k: int, n: int, batchA: int, batchB: int, aT: int, bT: int) -> int:
     return lib.cpmk_gemm_depth_parts(f16, m, k, n, batchA, batchB, aT, bT)
+
+
+@lib.bind("cpmk_gemm_fp16_copy_pays", [ctypes.c_int32] * 4 + [ctypes.c_int], ctypes.c_int)
+def gemm_fp16_copy_pays(m: int, k: int, n: int, batch: int, bT: int) -> int:
+    return lib.cpmk_gemm_fp16_copy_pays(m, k, n, batch, bT)
 
 
 @lib.bind("cpmk_device_count", [ctypes.POINTER(ctypes.c_int)], ctypes.c_int)

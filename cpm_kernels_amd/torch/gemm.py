@@ -10,7 +10,7 @@ import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
     gemm_quantize_cols_ld, gemm_quantize_cols_rows, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_timed, gemm_int8_scale_sum, gemm_fp16_sum, \
-    gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, gemm_depth_parts, gemm_int8_scale_split, gemm_fp16_split, \
+    gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, gemm_depth_parts, gemm_fp16_copy_pays, gemm_int8_scale_split, gemm_fp16_split, \
     arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
     transpose_i8_ld
 from ._common import cur_stream
@@ -327,7 +327,7 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
     8 x 4096 x 4096 x 512, B transposed 108 / 121 us, A 109 / 118; 4 x 1024 x 4096 x 512 34 / 40-44; 8192 x 4096 x 4096 204 / 208;
     8 x 10240 x 4096 x 512, B transposed 298 / 279; 4096 x 4096 x 10240, A transposed 298 / 275.  Or for results beyond the
     last-level cache of few slabs, where the two compete for memory: 2032 x 4096 over 32 entries of A, K = 256 223 / 203 us, 2048 x 8064
-    x 32 434 / 398 (512 MB and more; 2048 x 2048 x 32 and K = 1024 about even).  Rows of A that are not whole 16-byte pieces are
+    x 32 434 / 398 (512 MB and more; 2048 x 2048 x 32 and K = 1024 about even); or for few columns an entry (gemm_fp16_copy_pays).  Rows of A that are not whole 16-byte pieces are
     copied always."""
     M, K, N = _dims(A, B, aT, bT)
     bA, bB = A.shape[0], B.shape[0]
@@ -338,6 +338,8 @@ def gemm_pth_fp16(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> torch
             A, aT = _transposed_copy(A), False
         if not bT and (M > 8192 and K > 128 or large and M > 2048):
             B, bT = _transposed_copy(B), True
+    if bA == 1 and not bT and N < 512 and K >= 256 and gemm_fp16_copy_pays(N, K, M, bB, aT):
+        B, bT = _transposed_copy(B), True
     out = torch.empty((max(bA, bB), M, N), dtype=torch.half, device=A.device)
     parts = gemm_depth_parts(True, N, K, M, bB, bA, bT, aT) if K >= 1024 and out.numel() < _PARTS_MOST and (A.data_ptr() | B.data_ptr()) % 16 == 0 else 1
     if parts > 1:

@@ -221,6 +221,9 @@ int cpmk_gemm_add_parts(int32_t groups, int64_t n, const void* parts, void* out,
  * or the product has no such form: these take depths of whole 128-byte slabs, at least two, n and m multiples of 4 (of whole 16-byte pieces for an
  * operand stored (K, rows)), A (batchA, m, k) in the int8 form, buffers on 16-byte boundaries. */
 int cpmk_gemm_depth_parts(int f16, int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT);
+/* cpmk_gemm_fp16_copy_pays: 1 where cpmk_gemm_fp16 of A (batch, k, m) beside B (1, n, k) [(1, k, n) if bT] takes longer than with a copy of A
+ * as (batch, m, k). */
+int cpmk_gemm_fp16_copy_pays(int32_t m, int32_t k, int32_t n, int32_t batch, int bT);
 int cpmk_gemm_int8_scale_split(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, const void* A, const void* B,
                                const void* scale_row, const void* scale_col, int broad_cast_row, int broad_cast_col, void* out, int32_t parts,
                                void* workspace, void* stream);

@@ -1,0 +1,73 @@
+"""fp16 products of few rows or columns or of rows that are not whole pieces: edges of tiles and slabs, pieces across the end of a row, odd addresses."""
+import pytest
+import torch
+
+import cpm_kernels_amd.kernels as ck
+import cpm_kernels_amd.torch as ct
+from util import stream
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(A, aT, B, bT, out):
+    """out (batch, n, m) of A (., k, m) [(., m, k) if aT] and B (., n, k) [(., k, n) if bT]"""
+    k = A.size(2 if aT else 1)
+    for i in range(out.size(0)):
+        a, b = A[i % A.size(0)].double(), B[i % B.size(0)].double()
+        a, b = (a.t() if aT else a).contiguous(), (b.t() if bT else b).contiguous()
+        ref, size = b @ a, b.abs() @ a.abs()
+        # k additions in fp32, one rounding to fp16 (or half a subnormal step)
+        assert ((out[i].double() - ref).abs() <= size * k * 2.0 ** -24 + ref.abs() * 2.0 ** -10.9 + 2.0 ** -25).all()
+
+
+def _product(batch_a, batch_b, m, k, n, aT, bT, shift=0):
+    g = torch.Generator(device="cuda").manual_seed(m * 3 + n + k)
+    A = torch.randn((batch_a, m, k) if aT else (batch_a, k, m), generator=g, device="cuda").half()
+    B = torch.randn((batch_b, k, n) if bT else (batch_b, n, k), generator=g, device="cuda").half()
+    batch = max(batch_a, batch_b)
+    sizes = (A.numel(), B.numel(), batch * n * m)
+    pa, pb, po = (torch.full((t + 16,), float("nan"), dtype=torch.half, device="cuda") for t in sizes)
+    ua, ub, uo = (p[shift:shift + t] for p, t in zip((pa, pb, po), sizes))
+    ua.copy_(A.view(-1))
+    ub.copy_(B.view(-1))
+    ck.gemm_fp16(m, k, n, batch_a, batch_b, aT, bT, ua.data_ptr(), ub.data_ptr(), uo.data_ptr(), stream())
+    _check(A, aT, B, bT, uo.view(batch, n, m))
+    assert po[:shift].isnan().all() and po[shift + sizes[2]:].isnan().all()
+
+
+@pytest.mark.parametrize("aT,bT", [(True, False), (False, False), (True, True), (False, True)])
+@pytest.mark.parametrize("m,n", [(2, 2), (6, 64), (62, 66), (64, 128), (66, 126), (126, 80), (128, 34), (130, 100), (200, 128), (258, 66)])
+@pytest.mark.parametrize("k", [2, 30, 64, 66, 100, 192])
+def test_edges(aT, bT, m, n, k):
+    _product(3, 3, m, k, n, aT, bT)
+
+
+@pytest.mark.parametrize("aT,bT", [(True, False), (False, False), (True, True), (False, True)])
+@pytest.mark.parametrize("shift", [1, 2, 7])
+def test_any_address(aT, bT, shift):
+    _product(2, 2, 190, 70, 100, aT, bT, shift)
+    _product(1, 4, 60, 250, 130, aT, bT, shift)
+    _product(4, 1, 130, 250, 60, aT, bT, shift)
+
+
+@pytest.mark.parametrize("aT", [True, False])
+@pytest.mark.parametrize("m,n,k,batch", [(500, 64, 500, 130), (512, 128, 512, 120), (700, 80, 700, 80), (400, 96, 400, 4)])
+def test_many_small_tiles(aT, m, n, k, batch):
+    _product(batch, batch, m, k, n, aT, False)
+
+
+# the columns of several entries side by side: depths of 64- and 128-byte slabs and with a rest, P K-major and stored (K, rows), few and many tiles
+@pytest.mark.parametrize("m,batch,n", [(4, 33, 136), (36, 7, 304), (100, 5, 128), (132, 3, 264), (252, 16, 4112)])
+@pytest.mark.parametrize("k", [34, 64, 96, 130, 136, 512, 1000])
+@pytest.mark.parametrize("bT", [False, True])
+def test_joined_columns(m, batch, n, k, bT):
+    _product(batch, 1, m, k, n, True, bT)
+
+
+@pytest.mark.parametrize("aT", [False, True])
+@pytest.mark.parametrize("tokens,batch,din,dout", [(36, 1, 4096, 1024), (100, 16, 1024, 4608), (52, 3, 1500, 640), (188, 1, 4096, 1024), (44, 5, 600, 600)])
+def test_copied_operand(aT, tokens, batch, din, dout):
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    w = torch.randn((1, din, dout) if aT else (1, dout, din), generator=g, device="cuda").half()
+    x = torch.randn((batch, din, tokens), generator=g, device="cuda").half()
+    _check(x, False, w, aT, ct.bmm(w, aT, x, False, int8=False))

@@ -100,27 +100,37 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         const int64_t big = big_tiles(n, m, batch, big_apart);
         const bool large = big * 4 >= compute_units() * 3 && n > 128 && m > 128 && (!odd || m >= 256), pieces = operands % 16 == 0;
         a.edge_in = odd ? 2 : 0;
-        if (k % 32 == 0 && pieces) {
-            const bool whole128 = k % 64 == 0;       // the depth is whole 128-byte slabs (else whole 64-byte ones: 96, 160 ...)
-            if (large) {
-                if (whole128 && k >= 256) return launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, SEG, 16>(a, batch, st);
-                // Products of a few slabs -- attention scores, K = 64 -- are all prologue and epilogue, bound by the stores (and
-                // depths of whole 64-byte slabs only need this form anyway):
-                // the 32x32 form is quicker there, and waves of 64 rows x 128 columns, whose row segments are 256 bytes,
-                // store 5-15 % faster than waves of 128 x 64 (slabs of 64 bytes make room for their wider output strips)
-                return launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, SEG, 32>(a, batch, st);
-            }
-            if (!whole128) return launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, SEG, 32>(a, batch, st);
-            // (as for int8: more 128x128 tiles than compute units but at most two each -> two workgroups per compute unit)
-            const int64_t mid = ceil_div(n, 128) * ceil_div(m, 128) * batch, cus = compute_units();
-            if (mid > cus && mid <= 2 * cus) return launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, SEG, 32>(a, batch, st, 2);
-            return launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, SEG, 32>(a, batch, st);
+        // A depth that is whole 128-byte slabs, whole 64-byte ones (96, 160 ...) or neither: then the rest of it comes straight from memory into the fragments
+        // (large tiles) or as a slab filled up with zeros, as whole pieces (LAY bit 2) or as dwords (bit 3 too).
+        const bool whole64 = k % 32 == 0 && pieces, whole128 = whole64 && k % 64 == 0, rest16 = k % 8 == 0 && pieces;
+        if (large) {
+            if (whole128 && k >= 256) return launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, SEG, 16>(a, batch, st);
+            // Rows off cache lines: a 64-byte piece of a row lies in two lines nearly as often as a 128-byte one, so the longer slabs ask for a third
+            // fewer (2700 x 8000, k = 1000 79.6 -> 65.3 us, 1500 121.9 -> 95.3, 9196 652 -> 487; 500 52.2 and 54.3).
+            if (!whole128 && k >= 704)
+                return rest16 ? launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, SEG | 4, 16>(a, batch, st) : launch_dma<2, 4, 4, 2, 128, kEpiF16, 2, SEG | 12, 16>(a, batch, st);
+            // Products of a few slabs -- attention scores, K = 64 -- are all prologue and epilogue, bound by the stores:
+            // the 32x32 form is quicker there, and waves of 64 rows x 128 columns, whose row segments are 256 bytes,
+            // store 5-15 % faster than waves of 128 x 64 (slabs of 64 bytes make room for their wider output strips)
+            if (whole64) return launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, SEG, 32>(a, batch, st);
+            return rest16 ? launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, SEG | 4, 32>(a, batch, st) : launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, SEG | 12, 32>(a, batch, st);
         }
-        // a depth that is not whole 64-byte slabs (K = 40, 72, 500, 1000 ...): the same kernels, the rest of the depth straight
-        // from memory into the fragments (large tiles) or as a slab filled up with zeros
-        if (k % 8 == 0 && pieces)       // whole, aligned 16-byte pieces
-            return large ? launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, SEG | 4, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, SEG | 4, 32>(a, batch, st);
-        return large ? launch_dma<4, 2, 2, 4, 64, kEpiF16, 2, SEG | 12, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, SEG | 12, 32>(a, batch, st);
+        // (as for int8: more 128x128 tiles than compute units but at most two each -> two workgroups per compute unit)
+        const int64_t mid = ceil_div(n, 128) * ceil_div(m, 128) * batch, cus = compute_units();
+        const bool two = mid > cus && mid <= 2 * cus;
+        if (whole128)
+            return two ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, SEG, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, SEG, 32>(a, batch, st);
+        // The same choice of slabs where rows are off cache lines: 1200 x 4004, 320 tiles, k = 200 11.6 us on 64-byte slabs, one workgroup a compute unit, 10.6 so with two and 11.0 on 128-byte ones,
+        // 500 18.4, 16.2 and 16.1, 1500 42.5, 38.0 and 31.5; 640 x 640, k = 1000 11.0 and 13.0, 2056 17.1 and 20.2, 1200 x 1500, 1500 22.0 and 19.8, 9196 120 and 88; 3000 x 3000, 500
+        // 27.3 and 27.0, 1500 62.1 and 55.8.  (Rows of whole 64-byte slabs: 3000 x 3000, 1504 41.7 and 47.5.)
+        if (!whole64 && two && k >= 320)
+            return rest16 ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, SEG | 4, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, SEG | 12, 32>(a, batch, st, 2);
+        if (!whole64 && !two && k >= (mid > cus ? 448 : rest16 ? 2816 : 1280))
+            return rest16 ? launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, SEG | 4, 32>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, SEG | 12, 32>(a, batch, st);
+        const int per_cu = two && k < 704 ? 2 : 1;
+        if (whole64) return launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, SEG, 32>(a, batch, st, per_cu);
+        return rest16 ? launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, SEG | 4, 32>(a, batch, st, per_cu)
+                      : launch_dma<2, 2, 2, 2, 64, kEpiF16, kRingSmall, SEG | 12, 32>(a, batch, st, per_cu);
     };
     if (p_kmajor && q_kmajor && wide && k > 0 && (k > 32 ? operands % 4 == 0 : k == 32 && operands % 16 == 0) && (int64_t)n * k * 2 < (1ll << 32) &&
         (int64_t)m * k * 2 < (1ll << 32))

@@ -71,3 +71,10 @@ def test_copied_operand(aT, tokens, batch, din, dout):
     w = torch.randn((1, din, dout) if aT else (1, dout, din), generator=g, device="cuda").half()
     x = torch.randn((batch, din, tokens), generator=g, device="cuda").half()
     _check(x, False, w, aT, ct.bmm(w, aT, x, False, int8=False))
+
+
+# depths that are not whole slabs beyond a few of them: large tiles, one and two small ones a compute unit and several, whole pieces and dwords
+@pytest.mark.parametrize("m,n,batch,k", [(4100, 4112, 1, 708), (4100, 4112, 1, 1000), (4100, 4112, 1, 1504), (1500, 1200, 1, 1286), (640, 640, 1, 2824), (4004, 1200, 1, 324),
+                                         (4004, 1200, 1, 1000), (300, 300, 70, 450), (300, 300, 70, 1000), (130, 1300, 9, 1500)])
+def test_long_ragged_depths(m, n, batch, k):
+    _product(batch, 1 if m == 130 else batch, m, k, n, True, False)

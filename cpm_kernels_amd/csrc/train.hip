@@ -345,7 +345,7 @@ __global__ __launch_bounds__(256) void k_col(ColArgs p) {
     }
 }
 
-// The same reductions with the tile in registers: 64 columns x 512 rows per workgroup (16-byte
+// The same reductions with the tile in registers: 64 columns x 512 rows per workgroup (128 to 1024 for the softmax gradient; 16-byte
 // loads, each input read once), taller columns shared by a team of up to 32 workgroups that
 // exchange their partial column statistics (exchange.h).  Used when the shape allows 16-byte
 // accesses; k_col above serves everything else.
@@ -354,11 +354,12 @@ constexpr int kColTeamMaxParts = 32;
 // MODE 0: 16-byte accesses with the non-temporal hint (the tile's row segments are whole cache lines: m % 64 == 0, buffers on
 // 128-byte boundaries); 1: 16-byte accesses without it; 2: any m and alignment (pieces inside a row still whole, at whatever
 // address they lie; the piece across a row's end in at most three narrower accesses).
-template <int KIND, int MODE>
-__global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_batch, int32_t parts, uint32_t nteams, XchLaunch xl) {
+// NT, R: threads, rows a lane: tiles of NT / 8 * R rows.
+template <int KIND, int MODE, int NT = 512, int R = 8>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KIND == kSoftmaxBwd ? 4 : 1))) void k_col_team(ColArgs p, int32_t tiles_per_batch, int32_t parts, uint32_t nteams, XchLaunch xl) {
     uint64_t* const xch = xl.region;
     const uint32_t tag = xl.tag;
-    constexpr int NT = 512, LPR = 8, R = 8;
+    constexpr int LPR = 8;
     using T = ColTile<NT, LPR, R>;
     constexpr bool TWO = KIND != kLnFwdV && KIND != kLnFwdMV && KIND != kScaleRound && KIND != kColAbsmax;     // reads grad_in too
     constexpr bool IS_MAX = KIND == kScaleRound || KIND == kColAbsmax;
@@ -367,7 +368,8 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
     __shared__ float tot[T::COLS * 2];
     const int tid = threadIdx.x, cg = tid % LPR, rg = tid / LPR;
     XchMember me;
-    if (!xch_member(blockIdx.x, parts, nteams, me)) return;
+    if (parts == 1) me = {xcd_remap(blockIdx.x, nteams), 0};        // (neighbouring tiles on one XCD: they share cache lines where rows are not whole ones)
+    else if (!xch_member(blockIdx.x, parts, nteams, me)) return;
     const uint32_t part = me.part, team = me.team;
     const uint32_t b = team / tiles_per_batch, ct = team - b * tiles_per_batch;
     const int32_t col0 = ct * T::COLS + cg * 8;
@@ -508,7 +510,14 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
         }
     } else {
 #pragma unroll
-        for (int q = 0; q < R; ++q)
+        for (int q = 0; q < R; ++q) {
+            if constexpr (KIND == kSoftmaxBwd) {       // a row at a time, converted again: kept from the sums on, the tile in fp32 takes the registers of a second workgroup
+                __builtin_amdgcn_sched_barrier(0);
+                int4_t a4 = __builtin_bit_cast(int4_t, va[q]), g4 = __builtin_bit_cast(int4_t, vg[TWO ? q : 0]);
+                asm volatile("" : "+v"(a4), "+v"(g4));
+                va[q] = __builtin_bit_cast(half8_t, a4);
+                vg[TWO ? q : 0] = __builtin_bit_cast(half8_t, g4);
+            }
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const float x = (float)va[q][e];
@@ -521,6 +530,7 @@ __global__ __launch_bounds__(512) void k_col_team(ColArgs p, int32_t tiles_per_b
                 else o = x * (gi - s[e]);
                 va[q][e] = round_f16(o);
             }
+        }
         coltile_store<NT, LPR, R, NTS, UA>(va, p.out + boff, own_n, p.m, col0);
     }
     if (parts > 1 && tid < 64) xch_retire(xl, team, parts);
@@ -772,7 +782,7 @@ __global__ __launch_bounds__(256) void k_position_backward_team(int32_t query_le
     if (tid < 64) xch_retire(xl, h, parts);
 }
 
-// The same team layout for query rows of whole 16-byte pieces: the bias depends on q - k only, so the sum over
+// The same team layout by diagonals (UA: query rows that are not whole 16-byte pieces, or buffers off them): the bias depends on q - k only, so the sum over
 // a bucket is a sum over diagonals of grad_out.  A thread takes pieces of eight key rows x eight queries (eight
 // 16-byte non-temporal loads in flight, pieces dealt query-fastest so that a wave reads whole rows), adds the 64
 // values into the 15 diagonals that cross the piece -- element (row kk, query e) belongs to diagonal e - kk, a
@@ -780,6 +790,7 @@ __global__ __launch_bounds__(256) void k_position_backward_team(int32_t query_le
 // diagonal adds the pieces' contributions to it (two pieces per block of eight rows) in a fixed order: no
 // atomics up to here.  At the end the diagonals' sums go into the bucket histogram, and the parts' histograms
 // to part 0 as above.
+template <bool UA>
 __global__ __launch_bounds__(256) void k_position_backward_diag(int32_t query_len, int32_t key_len, int32_t num_buckets,
                                                                 int32_t max_distance, const int32_t* __restrict__ mapping,
                                                                 const half_t* __restrict__ grad_out, half_t* __restrict__ grad,
@@ -798,15 +809,20 @@ __global__ __launch_bounds__(256) void k_position_backward_diag(int32_t query_le
     const int32_t rel_min = -(k1 - 1), nd = query_len + (k1 - k0) - 1;      // rel = q - k of the part's rows: rel_min + [0, nd)
     for (int i = tid; i < num_buckets; i += 256) hist[i] = 0.0f;
     const half_t* g = grad_out + (int64_t)h * key_len * query_len;
-    const int32_t ncp = query_len >> 3, nrb = (k1 - k0 + 7) >> 3;
+    const int32_t ncp = UA ? (query_len + 7) >> 3 : query_len >> 3, nrb = (k1 - k0 + 7) >> 3;
     for (int32_t pi = tid; pi < ncp * nrb; pi += 256) {
         const int32_t rb = pi / ncp, cp = pi - rb * ncp;
         const int32_t kr = k0 + rb * 8;
         half8_t v[8];
+        auto at = [&](int kk) __attribute__((always_inline)) {       // (rows past the part's last repeat it and are left out below)
+            return g + (int64_t)min(kr + kk, k1 - 1) * query_len + cp * 8;
+        };
+        if (!UA || cp * 8 + 8 <= query_len) {        // (one condition for all eight: each under its own would be waited for before the next)
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-            const int32_t row = min(kr + kk, k1 - 1);      // (rows past the part's last repeat it and are left out below)
-            v[kk] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(g + (int64_t)row * query_len) + cp);
+            for (int kk = 0; kk < 8; ++kk) v[kk] = UA ? load_half8_any(at(kk)) : __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(at(kk)));
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) v[kk] = load_half8_head_any(at(kk), query_len & 7, half8_t{0, 0, 0, 0, 0, 0, 0, 0});
         }
         float d[15];
 #pragma unroll
@@ -973,12 +989,16 @@ static int launch_col(int32_t batch, const ColArgs& p, void* stream, bool missin
     if (batch < 0 || p.n < 0 || p.m < 0) return CPMK_EBADARG;
     if ((int64_t)batch * p.n * p.m == 0) return 0;
     if (missing) return CPMK_EBADARG;       // (a null buffer, found by the caller, in a call that has work to do)
-    const int64_t tiles = ceil_div(p.m, 64), parts = ceil_div(p.n, 512);
+    const int64_t tiles = ceil_div(p.m, 64);
     // 16-byte accesses when every row and buffer allows them, else the same kernel moving its columns one by one
     const bool vec16 = p.m % 8 == 0 && aligned16(p.a) && (p.g == nullptr || aligned16(p.g)) && (p.out == nullptr || aligned16(p.out)) &&
                        (p.mean == nullptr || aligned16(p.mean)) && (p.var == nullptr || aligned16(p.var)) &&
                        (p.out_mean == nullptr || aligned16(p.out_mean)) && (p.out_var == nullptr || aligned16(p.out_var)) &&
                        (p.out_i8 == nullptr || (reinterpret_cast<uintptr_t>(p.out_i8) & 7u) == 0);
+    // The softmax gradient, whose columns are a sequence: tiles no taller than they take, so that more workgroups share a compute unit (1024 of 100 x 100
+    // 42.6 -> 15.5 us, 528 of 236 x 236 74 -> 35), and up to 1024 rows in one workgroup, which waits for no other one (66 of 902 x 902 114 -> 64,
+    // 128 of 1024 x 1024 162 -> 130; with two of them a compute unit, 128 registers a lane, 256 of 512 x 512 74 -> 63).
+    const int64_t parts = KIND == kSoftmaxBwd && p.n <= 1024 ? 1 : ceil_div(p.n, 512);
     const bool wide = (int64_t)p.n * p.m < (1ll << 31) && parts <= kColTeamMaxParts && tiles * parts <= kXchSlots;
     auto on_line = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 127u) == 0; };
     const bool lines = p.m % 64 == 0 && on_line(p.a) && on_line(p.g) && on_line(p.out);      // (a null pointer counts as aligned)
@@ -998,13 +1018,22 @@ static int launch_col(int32_t batch, const ColArgs& p, void* stream, bool missin
                 }
                 if (rc != 0) return rc == kXchFull ? CPMK_ETOOBIG : rc;
             }
-            auto go = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3((unsigned)xch_team_grid(tiles * nb, parts)), dim3(512), 0, (hipStream_t)stream, q, (int32_t)tiles,
-                                   (int32_t)parts, (uint32_t)(tiles * nb), xs.xl);
+            auto go = [&](auto kern, int nt = 512) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)(parts == 1 ? tiles * nb : xch_team_grid(tiles * nb, parts))), dim3(nt), 0, (hipStream_t)stream, q,
+                                   (int32_t)tiles, (int32_t)parts, (uint32_t)(tiles * nb), xs.xl);
             };
-            if (!vec16) go(k_col_team<KIND, 2>);
-            else if (lines) go(k_col_team<KIND, 0>);
-            else go(k_col_team<KIND, 1>);
+            auto pick = [&](auto mode) {
+                constexpr int MODE = decltype(mode)::value;
+                if constexpr (KIND == kSoftmaxBwd) {
+                    if (p.n <= 128) return go(k_col_team<KIND, MODE, 512, 2>);
+                    if (p.n <= 256) return go(k_col_team<KIND, MODE, 512, 4>);
+                    if (p.n > 512 && parts == 1) return go(k_col_team<KIND, MODE, 1024, 8>, 1024);
+                }
+                go(k_col_team<KIND, MODE>);
+            };
+            if (!vec16) pick(std::integral_constant<int, 2>{});
+            else if (lines) pick(std::integral_constant<int, 0>{});
+            else pick(std::integral_constant<int, 1>{});
             const int e = launch_status();
             const int rc2 = xs.end();
             if (e != 0 || rc2 != 0) return e ? e : rc2;
@@ -1229,28 +1258,35 @@ int cpmk_position_embedding_backward(int32_t query_len, int32_t key_len, int32_t
     if (num_heads == 0) return 0;
     if (num_buckets > 8192) return CPMK_ETOOBIG;
     if (grad == nullptr || ((int64_t)query_len * key_len > 0 && any_null(position_mapping, grad_out))) return CPMK_EBADARG;
-    if (num_buckets <= kXchVals && max_distance <= 8192 && key_len > 64) {
+    if (num_buckets <= kXchVals && max_distance <= 8192 && key_len > 0 && query_len > 0) {
         // key rows of a head over a team: 64 rows a part, more when that would make more than 32 parts
         int64_t rpp = 64;
         while (ceil_div(key_len, rpp) > kColTeamMaxParts) rpp *= 2;
         const int64_t parts = ceil_div(key_len, rpp);
-        if ((int64_t)num_heads * parts <= kXchSlots) {
+        const int64_t pieces = ceil_div(query_len, 8) * ceil_div(rpp, 8);          // of eight key rows x eight queries, 15 floats each
+        const int64_t smem = (num_buckets + pieces * 15) * (int64_t)sizeof(float);
+        const bool diag = smem <= 128 * 1024;
+        if ((diag || key_len > 64) && (int64_t)num_heads * parts <= kXchSlots) {
             XchScope xs;
-            const int rc = xs.begin((int64_t)num_heads * parts, (hipStream_t)stream);
+            const int rc = parts > 1 ? xs.begin((int64_t)num_heads * parts, (hipStream_t)stream) : 0;
             if (rc != 0 && rc != kXchFull) return rc;
-            const int64_t pieces = (query_len / 8) * ceil_div(rpp, 8);          // of eight key rows x eight queries, 15 floats each
-            const size_t smem = (size_t)(num_buckets + pieces * 15) * sizeof(float);
-            if (rc == 0 && query_len % 8 == 0 && smem <= 64 * 1024 && aligned16(grad_out)) {
-                hipLaunchKernelGGL(k_position_backward_diag, dim3((unsigned)xch_team_grid(num_heads, parts)), dim3(256), smem,
-                                   (hipStream_t)stream, query_len, key_len, num_buckets, max_distance, (const int32_t*)position_mapping,
-                                   (const half_t*)grad_out, (half_t*)grad, bidirectional, (int32_t)parts, (int32_t)rpp,
+            const dim3 grid((unsigned)xch_team_grid(num_heads, parts));
+            if (rc == 0 && diag) {
+                // (1022 x 1022, 15 heads 68 -> 22 us, 902 x 902, 33 heads 98 -> 35, off 16-byte pieces, where a thread walked down each column with a load and a look-up an element)
+                const bool ua = query_len % 8 != 0 || !aligned16(grad_out);
+                auto kern = ua ? k_position_backward_diag<true> : k_position_backward_diag<false>;
+                static std::atomic<bool> lds_enabled[2][64];
+                if (smem > 48 * 1024)
+                    if (int e = enable_dynamic_lds(reinterpret_cast<const void*>(kern), 128 * 1024, lds_enabled[ua])) return e;
+                hipLaunchKernelGGL(kern, grid, dim3(256), (unsigned)smem, (hipStream_t)stream, query_len, key_len, num_buckets, max_distance,
+                                   (const int32_t*)position_mapping, (const half_t*)grad_out, (half_t*)grad, bidirectional, (int32_t)parts, (int32_t)rpp,
                                    (uint32_t)num_heads, xs.xl);
                 const int e = launch_status();
                 const int rc2 = xs.end();
                 return e ? e : rc2;
             }
             if (rc == 0) {      // (kXchFull: recorded into a graph and the capture reserve is used up: the kernel without packets below)
-                hipLaunchKernelGGL(k_position_backward_team, dim3((unsigned)xch_team_grid(num_heads, parts)), dim3(256),
+                hipLaunchKernelGGL(k_position_backward_team, grid, dim3(256),
                                    num_buckets * sizeof(float) + max_distance * sizeof(int32_t), (hipStream_t)stream, query_len, key_len,
                                    num_buckets, max_distance, (const int32_t*)position_mapping, (const half_t*)grad_out, (half_t*)grad,
                                    bidirectional, (int32_t)parts, (int32_t)rpp, (uint32_t)num_heads, xs.xl);

@@ -13,12 +13,12 @@ namespace cpmk {
 // lane, and its 16 waves a sixteenth of the ids each, which reach a wave as scalars (two vector operations per id and 64
 // tokens).  One launch and no scratch where a radix sort takes several of each.
 constexpr int kRankWaves = 16;
-__global__ __launch_bounds__(64 * kRankWaves) void k_rank_ids(int32_t tokens, const int32_t* __restrict__ ids, int32_t* __restrict__ order,
-                                                              int32_t* __restrict__ sorted) {
+__device__ __forceinline__ void rank_ids(uint32_t block, int32_t tokens, const int32_t* __restrict__ ids, int32_t* __restrict__ order,
+                                         int32_t* __restrict__ sorted) {
     __shared__ int32_t part[kRankWaves][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int32_t p0 = blockIdx.x * 64, p = p0 + lane;
+    const int32_t p0 = block * 64, p = p0 + lane;
     const int32_t id = ids[min(p, tokens - 1)];
     const int32_t share = (tokens + kRankWaves - 1) / kRankWaves;
     const int32_t q0 = min(wave * share, tokens), q1 = min(q0 + share, tokens);
@@ -39,6 +39,111 @@ __global__ __launch_bounds__(64 * kRankWaves) void k_rank_ids(int32_t tokens, co
         order[rank] = p;
         sorted[rank] = id;
     }
+}
+
+__global__ __launch_bounds__(64 * kRankWaves) void k_rank_ids(int32_t tokens, const int32_t* __restrict__ ids, int32_t* __restrict__ order,
+                                                              int32_t* __restrict__ sorted) {
+    rank_ids(blockIdx.x, tokens, ids, order, sorted);
+}
+
+// What has to be done before the rows are summed, in one launch: the order of the ids, the gradient (batch, hidden, seq) as rows (tokens, hidden),
+// and zeros in the table.  Bound by memory: the counting, 64 workgroups that hardly use it, and the transposition, which waits at barriers, pass under
+// the zeros: 4096 tokens x 4096 beside 30000 rows 63 us in three launches, 50 so; 310 x 1216 beside 11794 14.6 and 7.9; 16384 x 2048 beside 50000, where the
+// counting takes 28, 85 and 73 (tiles and zeros in turn 84).
+struct PrepareArgs {
+    int32_t tokens, hidden, seq;
+    const int32_t* ids;
+    int32_t *order, *sorted;      // null: ordered already
+    const half_t* grad;
+    half_t *rows, *table;
+    int64_t total;                // elements of the table
+    uint32_t rank_blocks, tile_blocks, tiles_c, tiles_r, tiles;
+};
+constexpr int kPrepareThreads = 64 * kRankWaves;
+constexpr int64_t kFillBytes = 8 * 16 * kPrepareThreads;      // zeros a workgroup writes
+
+// PIECES: rows of grad and of the transposed rows are whole aligned 16-byte pieces: a wave transposes a tile of 64 x 64 in registers, each
+// lane a block of 8 x 8, with 128-byte segments on both sides; else through LDS.
+template <bool PIECES>
+__global__ __launch_bounds__(kPrepareThreads) void k_embedding_prepare(PrepareArgs a) {
+    if (blockIdx.x < a.rank_blocks) {
+        rank_ids(blockIdx.x, a.tokens, a.ids, a.order, a.sorted);
+        return;
+    }
+    const uint32_t at = blockIdx.x - a.rank_blocks;
+    const bool is_tile = at < a.tile_blocks;
+    const uint32_t block = is_tile ? at : at - a.tile_blocks;
+    if (is_tile) {
+        const int32_t n = a.hidden, m = a.seq;
+        const uint32_t per = a.tiles_c * a.tiles_r;
+        if constexpr (PIECES) {
+            const uint32_t t = block * kRankWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+            if (t >= a.tiles) return;
+            const uint32_t b = t / per, in = t - b * per, tr = in / a.tiles_c, tc = in - tr * a.tiles_c;
+            const int64_t boff = (int64_t)b * n * m;
+            const int lane = threadIdx.x & 63;
+            half8_t v[8];
+            {
+                const int32_t r = tr * 64 + (lane >> 3) * 8, c = tc * 64 + (lane & 7) * 8;
+#pragma unroll
+                for (int p = 0; p < 8; ++p) {
+                    v[p] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+                    if (r < n && c < m) v[p] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(a.grad + boff + (int64_t)(r + p) * m + c));
+                }
+            }
+            transpose_half8x8(v);
+            // (lane l has block (l / 8, l % 8): what it stores lies beside what the lanes eight apart do)
+            const int32_t r = tr * 64 + (lane >> 3) * 8, c = tc * 64 + (lane & 7) * 8;
+            if (r < n && c < m)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) *reinterpret_cast<half8_t*>(a.rows + boff + (int64_t)(c + e) * n + r) = v[e];
+        } else {
+            // four tiles of 64 x 64, 256 lanes each; pieces of eight on both sides, wherever they start
+            __shared__ __attribute__((aligned(16))) half_t tile4[4][64][72];       // (pitch 144 bytes: an odd multiple of 16)
+            const int sub = threadIdx.x >> 8, tid = threadIdx.x & 255, pc = tid & 7, rr = tid >> 3;
+            half_t(&tile)[64][72] = tile4[sub];
+            const uint32_t t = block * 4 + sub;
+            const bool live = t < a.tiles;
+            const uint32_t b = t / per, in = t - b * per, tr = in / a.tiles_c, tc = in - tr * a.tiles_c;
+            const int32_t r0 = tr * 64, c0 = tc * 64;
+            const int64_t boff = (int64_t)b * n * m;
+#pragma unroll
+            for (int ps = 0; ps < 2; ++ps) {
+                const int r = ps * 32 + rr;
+                const int32_t c = c0 + pc * 8;
+                if (live && r0 + r < n && c < m) {
+                    const half_t* src = a.grad + boff + (int64_t)(r0 + r) * m + c;
+                    half8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
+                    if (c + 8 <= m) v = load_half8_any(src);
+                    else v = load_half8_head_any(src, m - c, v);
+                    *reinterpret_cast<half8_t*>(&tile[r][pc * 8]) = v;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int ps = 0; ps < 2; ++ps) {
+                const int c = ps * 32 + rr;                     // row of the transposed tile
+                const int32_t r = r0 + pc * 8;
+                if (live && c0 + c < m && r < n) {
+                    half8_t v;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = tile[pc * 8 + e][c];
+                    half_t* dst = a.rows + boff + (int64_t)(c0 + c) * n + r;
+                    if (r + 8 <= n) store_half8_any(dst, v);
+                    else store_half8_head_any(dst, n - r, v);
+                }
+            }
+        }
+        return;
+    }
+    const int64_t pieces = a.total >> 3, p0 = (int64_t)block * (kFillBytes / 16) + threadIdx.x;
+    half8_t* const table = reinterpret_cast<half8_t*>(a.table);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int64_t p = p0 + u * kPrepareThreads;
+        if (p < pieces) table[p] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+    if (block == 0 && threadIdx.x < (a.total & 7)) a.table[(pieces << 3) + threadIdx.x] = (half_t)0.0f;
 }
 
 // Sorted tokens a workgroup sums up.  Thirty-two rows hide the latency of the gather (all are requested before the first is
@@ -188,6 +293,30 @@ int cpmk_embedding_backward_rows(int32_t tokens, int32_t hidden_size, const void
     if (ceil_div(hidden_size, 256) > 65535) return CPMK_ETOOBIG;
     if (hidden_size % 8 == 0 && aligned16(grad_rows) && aligned16(grad)) return go(std::integral_constant<int, 8>{});
     return go(std::integral_constant<int, 1>{});
+}
+
+int cpmk_embedding_backward_prepare(int32_t batch, int32_t hidden_size, int32_t seq_len, int32_t vocab_size, const void* ids, void* order, void* sorted_ids,
+                                    const void* grad_out, void* grad_rows, void* grad, void* stream) {
+    clear_stale_error();
+    if (batch < 0 || hidden_size < 0 || seq_len < 0 || vocab_size < 0) return CPMK_EBADARG;
+    const int64_t tokens = (int64_t)batch * seq_len, total = (int64_t)vocab_size * hidden_size;
+    if (tokens >= 1ll << 31) return CPMK_ETOOBIG;
+    if ((total > 0 && grad == nullptr) || (tokens * hidden_size > 0 && any_null(grad_out, grad_rows)) || (tokens > 0 && ids && any_null(order, sorted_ids))) return CPMK_EBADARG;
+    if (total > 0 && !aligned16(grad)) return CPMK_EALIGN;
+    PrepareArgs a;
+    a.tokens = (int32_t)tokens; a.hidden = hidden_size; a.seq = seq_len;
+    a.ids = (const int32_t*)ids; a.order = (int32_t*)order; a.sorted = (int32_t*)sorted_ids;
+    a.grad = (const half_t*)grad_out; a.rows = (half_t*)grad_rows; a.table = (half_t*)grad; a.total = total;
+    const bool pieces = hidden_size % 8 == 0 && seq_len % 8 == 0 && aligned16(grad_out) && aligned16(grad_rows);
+    const int64_t tc = ceil_div(seq_len, 64), tr = ceil_div(hidden_size, 64), tiles = tc * tr * batch;
+    const int64_t rank = ids ? ceil_div(tokens, 64) : 0, tile_blocks = ceil_div(tiles, pieces ? kRankWaves : 4), fill = ceil_div(total * 2, kFillBytes);
+    if (rank + tile_blocks + fill == 0) return 0;
+    if (tiles >= 1ll << 32 || rank + tile_blocks + fill >= 1ll << 22) return CPMK_ETOOBIG;       // (a launch holds fewer than 2^32 threads)
+    a.rank_blocks = (uint32_t)rank; a.tile_blocks = (uint32_t)tile_blocks; a.tiles_c = (uint32_t)tc; a.tiles_r = (uint32_t)tr; a.tiles = (uint32_t)tiles;
+    const dim3 grid((unsigned)(rank + tile_blocks + fill));
+    if (pieces) hipLaunchKernelGGL(k_embedding_prepare<true>, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL(k_embedding_prepare<false>, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a);
+    return launch_status();
 }
 
 }  // extern "C"

@@ -2,9 +2,10 @@
 launchers this build adds (gemm_int8_scale, gemm_quantize, gemm_quantize_cols, gemm_quantize_pair,
 their `_ld` forms with padded rows, gemm_int8_scale_one, gemm_int8_scale_sum, gemm_fp16_sum, gemm_int8_scale_parts, gemm_fp16_parts,
 gemm_add_parts, gemm_int8_scale_split, gemm_fp16_split, gemm_quantize_cols_rows, layernorm_affine_forward,
-layernorm_affine_forward_stats, layernorm_affine_backward, embedding_order_ids, embedding_backward_rows)."""
+layernorm_affine_forward_stats, layernorm_affine_backward, embedding_order_ids, embedding_backward_rows,
+embedding_backward_prepare)."""
 from .embedding import embedding_forward, embedding_backward_stage1, embedding_backward_stage2, embedding_step, \
-    embedding_order_ids, embedding_backward_rows
+    embedding_order_ids, embedding_backward_rows, embedding_backward_prepare
 from .gelu import gelu_forward, gelu_backward, gelu_inplace_forward
 from .gemm import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, gemm_scale, \
     gemm_fp16, gemm_int8, gemm_backward_round_scale, gemm_backward_scale_round, gemm_scale_x, gemm_scale_y, \

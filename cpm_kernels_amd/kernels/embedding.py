@@ -63,3 +63,14 @@ def embedding_backward_rows(tokens: int, hidden_size: int,
                             stream: CUDAStream):
     """What embedding_backward_stage1 and _stage2 compute together, summed in fp32 and rounded once."""
     cpmk.embedding_backward_rows(tokens, hidden_size, grad_rows, order, sorted_ids, grad, partials, stream)
+
+
+def embedding_backward_prepare(batch: int, hidden_size: int, seq_len: int, vocab_size: int,
+                               ids: DevicePointer,          # (batch * seq_len) int32, or None: order and sorted_ids are there already
+                               order: DevicePointer, sorted_ids: DevicePointer,     # as in embedding_order_ids
+                               grad_out: DevicePointer,     # (batch, hidden_size, seq_len) fp16
+                               grad_rows: DevicePointer,    # (batch * seq_len, hidden_size) fp16
+                               grad: DevicePointer,         # (vocab_size, hidden_size) fp16: cleared
+                               stream: CUDAStream):
+    """What embedding_backward_rows needs, in one launch: the order of the ids, grad_out as rows, zeros in the table."""
+    cpmk.embedding_backward_prepare(batch, hidden_size, seq_len, vocab_size, ids, order, sorted_ids, grad_out, grad_rows, grad, stream)

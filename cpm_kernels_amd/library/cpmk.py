@@ -38,7 +38,7 @@ _LAUNCHERS = {
     "layernorm_forward_mv": "iiippppfp", "layernorm_backward_v": "iiippppp", "layernorm_backward_mv": "iiipppppp",
     "gemm_backward_round_scale": "iiippppip", "gemm_backward_scale_round": "iiippppip",
     "position_embedding_backward": "iiiiipppip", "embedding_backward_stage1": "iiippppppp",
-    "embedding_backward_stage2": "iipppp", "embedding_order_ids": "ipppp", "embedding_backward_rows": "iipppppp",
+    "embedding_backward_stage2": "iipppp", "embedding_order_ids": "ipppp", "embedding_backward_rows": "iipppppp", "embedding_backward_prepare": "iiiippppppp",
     "transpose": "iiippp", "transpose_i8": "iiippp", "array_add": "piip", "adjustify_logits": "iipfffpp",
     "copy_extend_buffer": "iiippp", "has_nan_inf": "lppp", "copy_pos_hidden": "iiiippp", "async_status": "",
     "selftest_exchange_timeout": "ip",

@@ -183,6 +183,7 @@ PyMethodDef g_launchers[] = {
     CPMK_ENTRY(cpmk_embedding_backward_stage2)
     CPMK_ENTRY(cpmk_embedding_order_ids)
     CPMK_ENTRY(cpmk_embedding_backward_rows)
+    CPMK_ENTRY(cpmk_embedding_backward_prepare)
     CPMK_ENTRY(cpmk_transpose)
     CPMK_ENTRY(cpmk_transpose_i8)
     CPMK_ENTRY(cpmk_array_add)

@@ -2,7 +2,7 @@
 (batch, embedding_size, seq); the gradient sums the rows of equal ids, as the two-stage sorted scatter-add of the
 reference does."""
 import torch
-from ..kernels import embedding_forward, embedding_order_ids, embedding_backward_rows, transpose
+from ..kernels import embedding_forward, embedding_backward_prepare, embedding_backward_rows
 from ._common import cur_stream, check_half
 
 # More tokens than this are put in order by a radix sort: counting ranks is quadratic in their number (4096 tokens: 10 us
@@ -43,14 +43,13 @@ class OpEmbedding(torch.autograd.Function):
         partials = rows + rows_bytes
         order = partials + partial_bytes
         sorted_ids = order + 4 * tokens
-        if tokens <= MAX_RANKED:
-            embedding_order_ids(tokens, ids.data_ptr(), order, sorted_ids, st)
-        else:
+        unordered = ids.data_ptr()
+        if tokens > MAX_RANKED:
             sort_result = ids.view(-1).sort()
             indices = sort_result.indices.to(torch.int32)
-            order, sorted_ids = indices.data_ptr(), sort_result.values.data_ptr()
-        transpose(batch, n, m, grad_output.data_ptr(), rows, st)
-        ret = torch.zeros((weight.size(0), n), device=grad_output.device, dtype=torch.half)
+            order, sorted_ids, unordered = indices.data_ptr(), sort_result.values.data_ptr(), None
+        ret = torch.empty((weight.size(0), n), device=grad_output.device, dtype=torch.half)
+        embedding_backward_prepare(batch, n, m, weight.size(0), unordered, order, sorted_ids, grad_output.data_ptr(), rows, ret.data_ptr(), st)
         embedding_backward_rows(tokens, n, rows, order, sorted_ids, ret.data_ptr(), partials, st)
         return None, ret
 

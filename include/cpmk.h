@@ -437,6 +437,10 @@ int cpmk_embedding_backward_stage2(int32_t batch, int32_t hidden_size, const voi
 /* The tokens in the order of their ids (equal ids in the order of the tokens): order[r] = token, sorted_ids[r] = its id.
  * Quadratic in the number of tokens: meant for up to some tens of thousands. */
 int cpmk_embedding_order_ids(int32_t tokens, const void* ids, void* order, void* sorted_ids, void* stream);
+/* What cpmk_embedding_backward_rows needs, in one launch: cpmk_embedding_order_ids of ids (batch * seq) -- null: the caller has the order --,
+ * grad_rows (batch * seq, hidden) = grad_out (batch, hidden, seq) transposed, and zeros in grad (vocab, hidden), which starts on a 16-byte boundary. */
+int cpmk_embedding_backward_prepare(int32_t batch, int32_t hidden_size, int32_t seq_len, int32_t vocab_size, const void* ids, void* order, void* sorted_ids,
+                                    const void* grad_out, void* grad_rows, void* grad, void* stream);
 /* The whole gradient of a table from gradient rows (tokens, hidden) and the order of the ids: the fp32 sum of the rows of
  * every id that occurs, rounded once; other rows of grad are left alone.  partials: 2 * ceil(tokens / 32) * hidden fp32. */
 int cpmk_embedding_backward_rows(int32_t tokens, int32_t hidden_size, const void* grad_rows, const void* order,

@@ -1,5 +1,5 @@
 // fp16 products with fp32 accumulation (cpm_kernels/kernels/gemm.py:188-256, cuBLASLt): which kernel takes which.  Operands P and Q as in
-// gemm_i8.hip; the tile kernel of gemm_tile.h, kernels of their own for short depths (gemm_short.hip), few rows (gemm_low.hip) and
+// gemm_i8.hip; the tile kernel of gemm_tile.h, kernels of their own for short depths (gemm_short.hip, gemm_rows.hip), few rows (gemm_low.hip) and
 // everything else (gemm_any.hip).
 #include "gemm_tile.h"
 
@@ -59,10 +59,9 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     // K = 256 22.6 us and 8.6, K = 512 42.6 and 12.2; both K-major, K = 512 15.8 and 11.4, 300 of 130 x 130, K = 1000 84 and 103.)
     const bool wide = (reinterpret_cast<uintptr_t>(out) & 3u) == 0 && (!odd || m >= 192);
     const bool p_kmajor = !bT, q_kmajor = aT != 0;
-    // A depth up to 128: a kernel of its own -- but where the output's rows are not whole cache lines and it exceeds half of the last-level
-    // cache, the tile kernel, whose large tiles share fewer of the lines (1024 of 500 x 500, K = 64 149 us, 162 there; 100 of 1000 x 1000 52.6 and
-    // 56.4; 250 of 500 x 500 32.7 and 25.1), unless those cover much more than the matrix (1500 of 300 x 300 179 and 113).  And the tile kernel
-    // too, beyond a quarter of that cache, where its large tiles cover no more than the small ones do, of which the last overlap the ones before
+    // A depth up to 128: kernels of their own, one for rows off cache lines where those are many (gemm_f16_rows), one of small tiles -- but where the output's
+    // rows are not whole cache lines and it exceeds half of the last-level cache, the tile kernel, whose large tiles share fewer of the lines, unless those cover
+    // much more than the matrix.  And the tile kernel too, beyond a quarter of that cache, where its large tiles cover no more than the small ones do, of which the last overlap the ones before
     // them: for depths of two slabs (7659 of 136 x 192, K = 128 217 us, 245 there; 976 of 200 x 1024 145 and 161; 5425 of 192 x 192 187 and 199), and
     // for an operand shared by the batch that is one large tile, of one whole slab or of two (2034 of 192 x 512 with the 192 shared, K = 64 104 and
     // 119; with the 512 shared 111 and 68; 976 of 400 x 512, the 400 shared, 106 and 71), or of two if it is the row operand (the same, K = 128, 134 and 146).
@@ -72,6 +71,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         const bool exact = big * 4 == mid && (n % 8 == 0 || n >= 256) && (m % 8 == 0 || m >= 256) && wide && aligned16(A) && aligned16(B);
         const bool overlap = batchA == batchB ? k > 112 && mid * 65536 > 5 * area
                                               : mid * 131072 > 9 * area && (batchB == 1 ? k > 112 || (k == 64 && n <= 256) : m <= 256 && (k == 64 || k > 112));
+        if (const int rc = gemm_f16_rows(m, k, n, batchA, batchB, A, B, out, st); rc >= 0) return rc;
         if (!large || ((m % 64 == 0 || outs <= 1 << 26) && !(exact && overlap && outs > 1 << 25)))
             if (const int rc = gemm_f16_short(m, k, n, batchA, batchB, A, B, out, st); rc >= 0) return rc;
     }

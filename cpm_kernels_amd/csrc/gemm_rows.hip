@@ -3,11 +3,11 @@
 // (cpm_kernels/torch/gemm.py:189-203).
 //
 // Bound by writing the output.  Tiles of part of a row write segments that begin and end inside cache lines, which their neighbours complete at
-// another time.  Here a workgroup has whole rows, 64 to 256 of them: 16 at a time are put together in LDS as they lie in memory and leave as whole aligned
+// another time.  Here a workgroup has whole rows, 64 to 560 of them: 16 at a time are put together in LDS as they lie in memory and leave as whole aligned
 // lines.  A wave has 128 columns, whose operand it keeps in registers, transposed there, for all rows of the workgroup.
 // Heads of seq x seq, K = 64, with operands that are not in the caches and a pass over the output behind (of 186 us for 1024 of 500, 63 for 300, which is in both figures):
-// 1024 of 500 338 -> 294 us, 256 of 500 84 -> 72, 128 of 500 45 -> 40, 1024 of 300 131 -> 114, 100 of 902 114 -> 89; 1024 of 110 38 -> 29, 16 of 100 13.2 -> 11.1; K = 80 250 of 350
-// 52 -> 44, 900 of 70 33 -> 21.  Stores with the non-temporal hint are quicker by themselves (1024 of 500 161 -> 94 us over operands in the cache), but leave the next
+// 1024 of 500 330 -> 290 us, 512 158 -> 133, 128 45 -> 40, 1024 of 300 131 -> 115, 100 of 902 114 -> 86; 1024 of 110 38 -> 28, 32 14.8 -> 9.7; K = 80 66 of 902 81 -> 72,
+// 900 of 70 33 -> 21.  Stores with the non-temporal hint are quicker by themselves (1024 of 500 161 -> 94 us over operands in the cache), but leave the next
 // kernel nothing there (334 us with the pass behind for 64 rows a workgroup, 320 with the hint; 256 rows 292 and 298; 512 of 500 139 and 156).
 #include "common.h"
 #include <type_traits>
@@ -130,40 +130,50 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KS == 3 ? 3
     }
 }
 
-// Rows of a workgroup: up to 256, which load the columns' operand that seldom, but 512 workgroups where that leaves them 64 rows each (1024 of 500 x 500 in one, two and
-// four parts 289, 293 and 309 us, 256 of them 81, 72 and 73, 128 58, 45 and 40).
-static int32_t rows_tall(int32_t n, int64_t batch) {
-    const int64_t deal = ceil_div(512, batch), most = ceil_div(n, 64), least = ceil_div(n, 256);
-    const int64_t parts = deal < least ? least : deal > most ? most : deal;
-    return (int32_t)ceil_div(ceil_div(n, parts), 16) * 16;
+// Rows of a workgroup, 32 at least: the fewest rounds of the device, of eight waves a compute unit at least (twelve of short rows), times the time of one, its start as long as 200
+// rows; two of them fit the LDS (1024 of 500 x 500 in one, two and four parts 289, 293 and 309 us, 128 of them 58, 45 and 40, 256 81, 72 and 73; 186 of 572 x 572
+// in two, three and four 71, 79 and 74, 150 of 570 x 570 62, 58 and 64).
+static int32_t rows_tall(int32_t n, int32_t m, int ks, int64_t batch) {
+    const int64_t cus = compute_units(), waves = ceil_div(m, 128), floor = waves >= 4 ? 2 : 12 / waves, cap = (80 * 1024 - 128 - 32ll * m) / (ks * 64) / 16 * 16;
+    const int64_t least = ceil_div(n, cap);
+    int64_t best = 0, best_t = 0;
+    for (int64_t parts = least; parts == least || (parts <= ceil_div(n, 32) && parts < least + 32); ++parts) {
+        const int64_t tall = ceil_div(ceil_div(n, parts), 16) * 16, each = ceil_div(ceil_div(n, tall) * batch, cus), t = (each > floor ? each : floor) * (tall + 200);
+        if (best == 0 || t < best_t) {
+            best = tall;
+            best_t = t;
+        }
+    }
+    return (int32_t)best;
 }
 
 // 0, an error code, or -1: not a product for this kernel.  A (batchA, k, m), B (batchB, k, n), out (batch, n, m).
 int gemm_f16_rows(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, const void* A, const void* B, void* out, hipStream_t st) {
     const int64_t batch = batchA > batchB ? batchA : batchB;
     if (m <= 64 || m > 1024 || m % 64 == 0 || n < 8 || k < 1 || k > 80 || m % 2 || n % 2 || !aligned16(out)) return -1;
-    // Outputs of 50 MB and more, from where the workgroups' start is hidden (the other kernels and this one, timed as above: 128 of 500 x 500 45 / 40 us, 64 of them 24.3 / 26.5; 200 of
-    // 300 x 300 33 / 32, 64 of them 15 / 17; 48 of 700 x 700 36 / 39, 60 of 900 x 900 67 / 61), with three k-steps not of two waves that are nearly full (1024 of 154 x 154, K = 80 56 / 45,
-    // 900 of 240 x 240 81 / 88); and any number where the matrix is smaller than the other kernels' tiles (100 of 100 x 100 13.8 / 12.5, 32 of 110 x 110 14.8 / 11.2; 400 of
-    // 120 x 120 17.9 / 18.9).  Whole lines stay where they are (512 of 256 x 256 45 / 52, 128 of 512 x 512 43 / 46).
-    const bool large = batch * n * m >= 3ll << 23 && (k <= 64 || m > 256 || m <= 180), little = n > 64 && n <= 112 && m <= 112;
+    // Outputs of 38 MB and more, with three k-steps 50 unless the rows are short, from where the workgroups' start is hidden (the other kernels and this one, timed as above:
+    // 128 of 500 x 500 45 / 40 us, 64 of them 24.4 / 26.6; 200 of 300 x 300 33 / 30, 64 of them 15 / 17; 48 of 700 x 700 36 / 34; 800 of 150 x 150 38 / 34, 64 of them
+    // 9.6 / 11.3; K = 80 50 of 600 x 600 32 / 35, 528 of 154 x 154 34 / 30), and any number where the matrix is smaller than the other kernels' tiles (100 of 100 x 100 13.6 / 11.1,
+    // 32 of 110 x 110 14.8 / 9.7, 400 of 120 x 120 17.6 / 17.1).  Whole lines stay where they are (512 of 256 x 256 45 / 52, 128 of 512 x 512 43 / 46), and tall matrices of
+    // less than a wave's columns (512 of 500 x 80 42 / 47).
+    const bool large = m > 128 && batch * n * m >= (k <= 64 ? 9ll << 21 : m <= 256 ? 3ll << 22 : 3ll << 23), little = n > 64 && n < 128 && m < 128;
     if (!large && !little) return -1;
     RowsArgs a;
     a.P = (const half_t*)B; a.Q = (const half_t*)A; a.out = (half_t*)out;
     a.strideP = batchB == 1 ? 0 : (int64_t)n * k;
     a.strideQ = batchA == 1 ? 0 : (int64_t)m * k;
     a.n = n; a.m = m; a.k = k;
-    a.tall = rows_tall(n, batch);
+    const int ks = (int)ceil_div(k, 32);
+    a.tall = rows_tall(n, m, ks, batch);
     const int64_t chunks = ceil_div(n, a.tall), nt = ceil_div(m, 128) * 64;
     if (chunks * batch * nt >= 1ll << 32) return -1;       // (a launch holds fewer than 2^32 threads)
     a.chunks = (uint32_t)chunks; a.items = (uint32_t)(chunks * batch);
-    const int ks = (int)ceil_div(k, 32);
-    const int lds = a.tall * ks * 64 + 128 + 16 * m * 2;       // (at most 80 KB + 128)
+    const int lds = a.tall * ks * 64 + 128 + 16 * m * 2;
     int rc = 0;
     auto go = [&](auto ksc, auto alc) {
         auto kern = k_gemm_rows<decltype(ksc)::value, decltype(alc)::value>;
         static std::atomic<bool> lds_enabled[64];
-        rc = enable_dynamic_lds(reinterpret_cast<const void*>(kern), 81 * 1024, lds_enabled);
+        rc = enable_dynamic_lds(reinterpret_cast<const void*>(kern), 80 * 1024, lds_enabled);
         if (rc == 0) hipLaunchKernelGGL(kern, dim3(a.items), dim3((unsigned)nt), (unsigned)lds, st, a);
     };
     auto steps = [&](auto alc) {

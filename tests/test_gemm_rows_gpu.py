@@ -28,9 +28,9 @@ def _product(batch, n, m, k, shared=""):
         assert ((out[i].double() - ref).abs() <= size * k * 2.0 ** -24 + ref.abs() * 2.0 ** -10.9 + 2.0 ** -25).all()
 
 
-# rows that start on 16, 8 and 4 bytes; one wave of columns to eight; blocks of 16 rows and parts of them, workgroups of 16 rows to 256 and shorter last ones
-@pytest.mark.parametrize("n,m,k", [(8, 66, 64), (10, 74, 64), (66, 130, 64), (64, 254, 2), (500, 500, 64), (500, 500, 80), (62, 136, 32), (72, 362, 34), (130, 502, 66),
-                                   (300, 300, 48), (18, 1022, 78), (1000, 1000, 64), (80, 900, 62), (200, 260, 30), (8, 1000, 64), (1030, 120, 62), (256, 72, 64), (254, 154, 80)])
+# rows that start on 16, 8 and 4 bytes; one wave of columns to eight; blocks of 16 rows and parts of them, workgroups of 16 rows to 560 and shorter last ones
+@pytest.mark.parametrize("n,m,k", [(8, 130, 64), (10, 134, 64), (66, 130, 64), (64, 254, 2), (500, 500, 64), (500, 500, 80), (62, 136, 32), (72, 362, 34), (130, 502, 66),
+                                   (300, 300, 48), (18, 1022, 78), (1000, 1000, 64), (80, 900, 62), (200, 260, 30), (8, 1000, 64), (1030, 140, 62), (254, 154, 80), (560, 162, 28)])
 def test_large(n, m, k):
     _product(LARGE // (n * m) + 1, n, m, k)
 
@@ -40,7 +40,7 @@ def test_few_entries(batch, n, m, k):
     _product(batch, n, m, k)
 
 
-@pytest.mark.parametrize("n,m", [(66, 66), (66, 112), (112, 68), (100, 100), (98, 74)])
+@pytest.mark.parametrize("n,m", [(66, 66), (66, 126), (112, 68), (100, 100), (98, 74)])
 @pytest.mark.parametrize("batch", [1, 5, 600])
 @pytest.mark.parametrize("k", [2, 64, 80])
 def test_little(n, m, batch, k):

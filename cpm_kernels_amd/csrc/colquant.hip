@@ -13,6 +13,7 @@
 // whole slabs then, whatever the number of rows or columns is.
 #include "dim1.h"
 #include "exchange.h"
+#include "round_scale.h"
 
 namespace cpmk {
 
@@ -384,6 +385,22 @@ __global__ __launch_bounds__(kColThreads) __attribute__((amdgpu_waves_per_eu(6, 
     else quantize_row<4, true>(r, block);
 }
 
+// The gradient on its way to both products of a backward pass: its columns and its rows in one launch, as above, bound the same way; rows that a wave holds in
+// registers (75 of them beside the teams' 80, no LDS).  A launch for each / one, operands outside the caches, us: 8 x 10240 x 512 84 / 79, 8 x 4096 x 512 41.4 / 35.7, 4 x 10240 x 500
+// 66 / 50, 15 x 2048 x 736 52 / 46, 4 x 896 x 172 27 / 19.5, 16 x 4096 x 1024 112 / 112.
+template <bool NTH, bool UA>
+__global__ __launch_bounds__(kColThreads) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_col_scale_round_rows(ColQuantArgs a, int32_t tiles_per_batch, int32_t parts,
+                                                                                                               uint32_t nteams, XchLaunch xl, RoundScaleArgs r) {
+    if (blockIdx.x < r.first) {
+        col_quantize_team<kColThreads, kOutT, NTH, UA, true>(a, tiles_per_batch, parts, nteams, xl);
+        return;
+    }
+    const int64_t wave = (int64_t)(blockIdx.x - r.first) * (kColThreads / 64) + (threadIdx.x >> 6);
+    if (r.m <= 512) round_scale_rows_reg<1, 4, UA>(r, wave);
+    else if (r.m <= 1024) round_scale_rows_reg<2, 2, UA>(r, wave);
+    else round_scale_rows_reg<4, 1, UA>(r, wave);
+}
+
 // Rows r0 .. r0 + 63 of a tile of 64 columns, rounded with the scale of the lane's column, into the wanted outputs (256 threads;
 // the transposed one through `tile`, so that a wave stores 64 bytes of one column and not one of 64).  The surplus of longer
 // rows becomes zeros: rows from n on in the transposed output, columns from m on in the other.
@@ -479,7 +496,7 @@ int cpmk_gemm_round_transpose(int32_t, int32_t, int32_t, const void*, const void
 // The team kernel on (batch, n, m): 0, an error code, or -1 when the shape is not one it takes.  rq: rows to quantise beside the (first)
 // launch of the teams; -1 also where they are not of the form that takes.
 template <bool SCALED>
-static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st, const RowQuantArgs* rq = nullptr) {
+static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st, const std::conditional_t<SCALED, RoundScaleArgs, RowQuantArgs>* rq = nullptr) {
     const int32_t n = p.n, m = p.m;
     // a team here exchanges one maximum per column, dealt to all waves, so it may be larger than the teams of the kernels that keep
     // per-part values in registers (kColMaxParts of 512 rows: 16384; far fewer workgroups than are resident at once, which is what progress
@@ -494,8 +511,14 @@ static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st, co
     if (!team_ok) return -1;
     int64_t row_blocks = 0;
     if (rq) {
-        row_blocks = rq->ld > 4096 ? rq->rows : ceil_div(rq->rows, kColThreads / 64);
-        if (SCALED || rq->m % 8 || rq->ld % 8 || rq->ld > 16384 || !aligned16(rq->mat) || (reinterpret_cast<uintptr_t>(rq->out) & 7u) || row_blocks > 1 << 21) return -1;
+        if constexpr (SCALED) {
+            row_blocks = ceil_div(rq->rows, kColThreads / 64 * (rq->m <= 512 ? 4 : rq->m <= 1024 ? 2 : 1));
+            if (rq->m > 2048 || (wide && (!aligned16(rq->scale_y) || (reinterpret_cast<uintptr_t>(rq->out) & 7u)))) return -1;
+        } else {
+            row_blocks = rq->ld > 4096 ? rq->rows : ceil_div(rq->rows, kColThreads / 64);
+            if (rq->m % 8 || rq->ld % 8 || rq->ld > 16384 || !aligned16(rq->mat) || (reinterpret_cast<uintptr_t>(rq->out) & 7u)) return -1;
+        }
+        if (row_blocks > 1 << 21) return -1;
     }
     // teams use one packet slot per (team, part): batches beyond the pool go out in several launches
     const int64_t per_launch = parts > 1 ? kXchSlots / (tiles * parts) : ((1ll << 31) - 8) / (tiles * parts);
@@ -516,7 +539,7 @@ static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st, co
         if (p.out_n) q.out_n += b0 * n * p.ld_n;
         const int64_t team_blocks = xch_team_grid(tiles * nb, parts);
         auto go_rows = [&](auto kern) {
-            RowQuantArgs r = *rq;
+            auto r = *rq;
             r.first = (uint32_t)team_blocks;
             hipLaunchKernelGGL(kern, dim3((unsigned)(team_blocks + row_blocks)), dim3(kColThreads), 0, st, q, (int32_t)tiles, (int32_t)parts, (uint32_t)(tiles * nb),
                                xs.xl, r);
@@ -532,6 +555,14 @@ static int col_quantize(int32_t batch, const ColQuantArgs& p, hipStream_t st, co
                     if (!wide) go_rows(k_col_quantize_rows<OUT, false, true>);
                     else if (lines) go_rows(k_col_quantize_rows<OUT, true, false>);
                     else go_rows(k_col_quantize_rows<OUT, false, false>);
+                    return;
+                }
+            }
+            if constexpr (SCALED) {
+                if (rq && b0 == 0) {        // (rows beside columns: the transposed output only)
+                    if (!wide) go_rows(k_col_scale_round_rows<false, true>);
+                    else if (lines) go_rows(k_col_scale_round_rows<true, false>);
+                    else go_rows(k_col_scale_round_rows<false, false>);
                     return;
                 }
             }
@@ -641,6 +672,24 @@ int cpmk_gemm_quantize_cols_rows(int32_t batch, int32_t n, int32_t m, const void
     }
     if (const int rc = cpmk_gemm_quantize_cols_ld(batch, n, m, mat, nullptr, 0, scale, out_t, ld_t, out_n, ld_n, stream)) return rc;
     return cpmk_gemm_quantize_pair_ld(rows, row_mat, row_scale, row_out, 0, nullptr, nullptr, nullptr, n, ld_t, stream);
+}
+
+int cpmk_gemm_backward_round_scale_ld(int32_t, int32_t, int32_t, const void*, const void*, void*, int32_t, void*, int, void*);       // train.hip
+
+int cpmk_gemm_backward_quantize_both(int32_t batch, int32_t n, int32_t m, const void* mat, const void* row_scale, int broad_cast_row, void* scale, void* out_t, int32_t ld_t,
+                                     const void* scale_y, int broad_cast_y, void* out, int32_t ld, void* scale_x, void* stream) {
+    clear_stale_error();
+    const int64_t rows = (int64_t)batch * n;
+    if (n > 0 && batch > 0 && m > 0 && rows <= 0x7fffffff && ld_t >= n && ld_t % 16 == 0 && ld >= m && (ld == m || (ld % 16 == 0 && ld <= (m + 127) / 128 * 128)) &&
+        !any_null(mat, row_scale, scale, out_t) && !any_null(scale_y, out, scale_x)) {
+        const ColQuantArgs p = {n, m, (const half_t*)mat, (const half_t*)row_scale, broad_cast_row, (half_t*)scale, (int8_t*)out_t, nullptr, ld_t, 0};
+        const RoundScaleArgs r = {(const half_t*)mat, (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, rows, n, m, broad_cast_y, ld, 0};
+        const int rc = col_quantize<true>(batch, p, (hipStream_t)stream, &r);
+        if (rc >= 0) return rc;
+    }
+    if (const int rc = cpmk_gemm_backward_round_scale_ld(batch, n, m, mat, scale_y, out, ld, scale_x, broad_cast_y, stream)) return rc;
+    if (row_scale == nullptr && (int64_t)batch * m > 0) return CPMK_EBADARG;
+    return cpmk_gemm_quantize_cols_ld(batch, n, m, mat, row_scale, broad_cast_row, scale, out_t, ld_t, nullptr, 0, stream);
 }
 
 }  // extern "C"

@@ -6,6 +6,7 @@
 // forward layernorm.
 #include "dim1.h"
 #include "exchange.h"
+#include "round_scale.h"
 
 namespace cpmk {
 
@@ -536,19 +537,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KIND == kSof
     if (parts > 1 && tid < 64) xch_retire(xl, team, parts);
 }
 
-// eight products x * sy rounded to multiples of s (own: s is the data's own and in the range of the short sequence)
-__device__ __forceinline__ uint2_t round8_own_scale(half8_t x, half8_t sy, float s, float y, bool own) {
-    int32_t t[8];
-    if (own) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) t[e] = (int32_t)quant_i8_own_fp32_scale_bits((float)x[e] * (float)sy[e], s, y);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) t[e] = quant_i8((float)x[e] * (float)sy[e], s);
-    }
-    return uint2_t{pack4_i8(t[0], t[1], t[2], t[3]), pack4_i8(t[4], t[5], t[6], t[7])};
-}
-
 // cu_gemm_backward_round_scale: per-row absmax of mat * scale_y[col] -> scale_x, then rounding.
 // (ld: bytes from one row of the output to the next; past the matrix's columns they are zeros)
 __global__ __launch_bounds__(256) void k_round_scale_rows(int32_t n, int32_t m, const half_t* __restrict__ mat,
@@ -601,87 +589,10 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_wide(int64_t rows, int
     }
 }
 
-// The same for rows of at most 2048 columns, kept in registers: a wave takes U consecutive rows of P 16-byte pieces
-// per lane (P * U = 4 loads in flight per lane, the matrix read once and with the non-temporal hint), finds each
-// row's maximum over the wave with data-parallel-primitive operands and rounds from the registers.
-// UA: rows that are not whole 16-byte pieces or buffers off 16-byte boundaries -- a piece inside its row still comes in
-// one 16-byte load and leaves in one 8-byte store (global accesses need no alignment), the piece across a row's end
-// in at most three narrower accesses each way.
-// The two rounding sequences are chosen once for the wave's rows: a choice per row kept their chains from running side by side (780 rows
-// of 24 6.9 us, 4.7 so; 20000 of 512 11.1 -> 8.1; 81920 of 512 30 -> 23.5, 5.3 TB/s).
+// The same for rows of at most 2048 columns, kept in registers (round_scale.h).
 template <int P, int U, bool UA>
-__global__ __launch_bounds__(256) void k_round_scale_rows_reg(int64_t rows, int32_t n, int32_t m, const half_t* __restrict__ mat,
-                                                              const half_t* __restrict__ scale_y, int8_t* __restrict__ out,
-                                                              half_t* __restrict__ scale_x, int bc, int32_t ld) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * U;
-    if (row0 >= rows) return;
-    auto load8 = [&](const half_t* src, int32_t j, bool nt) __attribute__((always_inline)) {
-        half8_t r = {0, 0, 0, 0, 0, 0, 0, 0};
-        if constexpr (!UA) {
-            r = nt ? __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(src + j)) : *reinterpret_cast<const half8_t*>(src + j);
-        } else if (j + 8 <= m) {
-            r = load_half8_any(src + j);
-        } else {
-            r = load_half8_head_any(src + j, m & 7, r);       // (callers pass j < m)
-        }
-        return r;
-    };
-    half8_t xv[U][P], sv[U][P];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int64_t row = row0 + u < rows ? row0 + u : rows - 1;
-        const half_t* x = mat + row * m;
-        const half_t* sy = scale_y + (bc ? 0 : (row / n) * m);
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const int32_t j = lane * 8 + p * 512;
-            xv[u][p] = sv[u][p] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-            if (j < m) {
-                xv[u][p] = load8(x, j, true);
-                sv[u][p] = load8(sy, j, false);
-            }
-        }
-    }
-    float s[U];
-    bool own = true;        // (the same for the whole wave)
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        float mx = 0.0f;
-#pragma unroll
-        for (int p = 0; p < P; ++p)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) mx = fmaxf(fabsf((float)xv[u][p][e] * (float)sv[u][p][e]), mx);
-        mx = __builtin_bit_cast(float, wave_max_u32_uniform(__builtin_bit_cast(uint32_t, mx)));      // (non-negative floats order as their bits)
-        s[u] = (float)((double)mx / 127.0);
-        own = own && own_scale_in_range(s[u]);
-        if (lane == 0 && row0 + u < rows) scale_x[row0 + u] = (half_t)s[u];
-    }
-    auto finish = [&](auto ownc) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t row = row0 + u;
-            if (row >= rows) break;
-            const float y = 1.0f / s[u];
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const int32_t j = lane * 8 + p * 512;
-                if (j < ld) {        // (past the end of the row: zeros)
-                    const uint2_t w = round8_own_scale(xv[u][p], sv[u][p], s[u], y, decltype(ownc)::value);
-                    int8_t* dst = out + row * ld + j;
-                    if constexpr (!UA) {
-                        *reinterpret_cast<uint2_t*>(dst) = w;
-                    } else if (j + 8 <= ld) {
-                        store_byte8_any(dst, w.x, w.y);
-                    } else {
-                        store_byte8_head_any(dst, ld & 7, w.x, w.y);
-                    }
-                }
-            }
-        }
-    };
-    if (own) finish(std::true_type{});
-    else finish(std::false_type{});
+__global__ __launch_bounds__(256) void k_round_scale_rows_reg(RoundScaleArgs a) {
+    round_scale_rows_reg<P, U, UA>(a, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1230,8 +1141,8 @@ int cpmk_gemm_backward_round_scale_ld(int32_t batch, int32_t n, int32_t m, const
         auto go = [&](auto pc, auto uc) {
             constexpr int P = decltype(pc)::value, U = decltype(uc)::value;
             auto run = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(rows, 4 * U)), dim3(256), 0, (hipStream_t)stream, rows, n, m, (const half_t*)mat,
-                                   (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, broad_cast_y, ld);
+                const RoundScaleArgs a = {(const half_t*)mat, (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, rows, n, m, broad_cast_y, ld, 0};
+                hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(rows, 4 * U)), dim3(256), 0, (hipStream_t)stream, a);
             };
             if (vec16) run(k_round_scale_rows_reg<P, U, false>);
             else run(k_round_scale_rows_reg<P, U, true>);

@@ -1,7 +1,7 @@
 """Same export list as cpm_kernels/kernels/__init__.py:1-14 of the reference, plus the fused
 launchers this build adds (gemm_int8_scale, gemm_quantize, gemm_quantize_cols, gemm_quantize_pair,
 their `_ld` forms with padded rows, gemm_int8_scale_one, gemm_int8_scale_sum, gemm_fp16_sum, gemm_int8_scale_parts, gemm_fp16_parts,
-gemm_add_parts, gemm_int8_scale_split, gemm_fp16_split, gemm_quantize_cols_rows, layernorm_affine_forward,
+gemm_add_parts, gemm_int8_scale_split, gemm_fp16_split, gemm_quantize_cols_rows, gemm_backward_quantize_both, layernorm_affine_forward,
 layernorm_affine_forward_stats, layernorm_affine_backward, embedding_order_ids, embedding_backward_rows,
 embedding_backward_prepare)."""
 from .embedding import embedding_forward, embedding_backward_stage1, embedding_backward_stage2, embedding_step, \
@@ -12,7 +12,7 @@ from .gemm import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_r
     gemm_int8_scale, gemm_quantize, gemm_quantize_cols, gemm_quantize_pair, \
     gemm_int8_scale_one, gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_backward_round_scale_ld, gemm_sum_groups, gemm_sum_groups_for, gemm_sum_groups_timed, \
     gemm_int8_scale_sum, gemm_fp16_sum, gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, \
-    gemm_depth_parts, gemm_fp16_copy_pays, gemm_int8_scale_split, gemm_fp16_split, gemm_quantize_cols_rows
+    gemm_depth_parts, gemm_fp16_copy_pays, gemm_int8_scale_split, gemm_fp16_split, gemm_quantize_cols_rows, gemm_backward_quantize_both
 from .gemv import gemv_fp16, gemv_broadcast_mat_int8, gemv_fp16_transpose, gemv_broadcast_mat_fp16, \
     gemv_calc_scale, gemv_round, gemv_broadcast_mat_fp16_light, gemv_fp16_light, gemv_fp16_transpose_light
 from .mask import mask

@@ -184,6 +184,23 @@ def gemm_backward_round_scale_ld(batch: int, n: int, m: int, mat: DevicePointer,
     cpmk.gemm_backward_round_scale_ld(batch, n, m, mat, scale_y, out, ld, scale_x, 1 if broad_cast_y else 0, stream)
 
 
+def gemm_backward_quantize_both(batch: int, n: int, m: int,
+                                mat: DevicePointer,        # (batch, n, m)     fp16
+                                row_scale: DevicePointer, broad_cast_row: bool,        # (batch, n) or (n)
+                                scale: DevicePointer,      # (batch, m)        fp16
+                                out_t: DevicePointer,      # (batch, m, ld_t)  int8
+                                ld_t: int,
+                                scale_y: DevicePointer, broad_cast_y: bool,            # (batch, m) or (m)
+                                out: DevicePointer,        # (batch, n, ld)    int8
+                                ld: int,
+                                scale_x: DevicePointer,    # (batch, n)        fp16
+                                stream: CUDAStream):
+    """gemm_quantize_cols_ld of mat with row scales (transposed) and gemm_backward_round_scale_ld of it in one launch: a gradient on its way
+    to both products of a backward pass."""
+    cpmk.gemm_backward_quantize_both(batch, n, m, mat, row_scale, 1 if broad_cast_row else 0, scale, out_t, ld_t, scale_y, 1 if broad_cast_y else 0, out, ld,
+                                     scale_x, stream)
+
+
 def gemm_sum_groups(m: int, n: int, batch: int) -> int:
     """Partial sums that gemm_int8_scale_sum / gemm_fp16_sum form for (n, m) outputs over `batch` entries: as few as
     keep the device busy (a divisor of the batch)."""

@@ -21,7 +21,7 @@ _LAUNCHERS = {
     "gemm_backward_round_scale_ld": "iiipppipip", "gemm_int8_scale_one": "iiiiiiippppiipp",
     "transpose_i8_ld": "iiipipip", "gemm_int8_scale_sum": "iiiiippppp", "gemm_fp16_sum": "iiiiipppp",
     "gemm_int8_scale_parts": "iiiiippppp", "gemm_fp16_parts": "iiiiiipppp", "gemm_add_parts": "ilppp",
-    "gemm_quantize_cols_rows": "iiipppipilpppp", "gemm_int8_scale_split": "iiiiiiippppiipipp", "gemm_fp16_split": "iiiiiiipppipp",
+    "gemm_quantize_cols_rows": "iiipppipilpppp", "gemm_backward_quantize_both": "iiippippipipipp", "gemm_int8_scale_split": "iiiiiiippppiipipp", "gemm_fp16_split": "iiiiiiipppipp",
     "gemv_fp16": "iiipppp", "gemv_fp16_transpose": "iiipppp", "gemv_broadcast_mat_fp16": "iiipppp",
     "embedding_forward": "iiipppp", "embedding_step": "iipppp", "copy_data_to_kv": "iiippip",
     "gemv_calc_scale": "iippp", "gemv_round": "iipppp", "gemv_broadcast_mat_int8": "iiipppppp",

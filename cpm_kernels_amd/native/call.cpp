@@ -129,6 +129,7 @@ PyMethodDef g_launchers[] = {
     CPMK_ENTRY(cpmk_gemm_int8_scale_sum)
     CPMK_ENTRY(cpmk_gemm_fp16_sum)
     CPMK_ENTRY(cpmk_gemm_quantize_cols_rows)
+    CPMK_ENTRY(cpmk_gemm_backward_quantize_both)
     CPMK_ENTRY(cpmk_gemm_int8_scale_split)
     CPMK_ENTRY(cpmk_gemm_fp16_split)
     CPMK_ENTRY(cpmk_gemm_int8_scale_parts)

@@ -11,7 +11,7 @@ from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, ge
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
     gemm_quantize_cols_ld, gemm_quantize_cols_rows, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_timed, gemm_int8_scale_sum, gemm_fp16_sum, \
     gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, gemm_depth_parts, gemm_fp16_copy_pays, gemm_int8_scale_split, gemm_fp16_split, \
-    arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_scale_round, transpose, \
+    arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_quantize_both, gemm_backward_scale_round, transpose, \
     transpose_i8_ld
 from ._common import cur_stream
 
@@ -76,13 +76,17 @@ def _quantize_rows(*mats):
     return out
 
 
+def _cols_row_bytes(n: int, summed: bool) -> int:
+    return (n + 15) // 16 * 16 if n > 16384 else _sum_row_bytes(n) if summed else _row_bytes(n)
+
+
 def _quantize_cols(x, both: bool, row_scale=None, summed: bool = False):
     """A (b, n, m) operand quantised along n: scale (b, m), int8 (b, m, _row_bytes(n)) -- _sum_row_bytes(n) if `summed` -- and, with
     `both`, the same values where they were, (b, n, _sum_row_bytes(m)) (else None).  row_scale: of the values multiplied by it, see
     gemm_backward_scale_round."""
     b, n, m = x.size()
     scale = torch.empty((b, m), dtype=torch.half, device=x.device)
-    ld_t = (n + 15) // 16 * 16 if n > 16384 else _sum_row_bytes(n) if summed else _row_bytes(n)
+    ld_t = _cols_row_bytes(n, summed)
     ld_n = _sum_row_bytes(m) if both else 0
     out_t = torch.empty((b, m, ld_t), dtype=torch.int8, device=x.device)
     out_n = torch.empty((b, n, ld_n), dtype=torch.int8, device=x.device) if both else None
@@ -243,13 +247,25 @@ class GEMMInt8(torch.autograd.Function):
             M, K, N = ctx.dims
             own_A, own_B = ctx.own
             grad_A = grad_B = None
-            if ctx.needs_input_grad[0]:                                     # contracted over N
+            want_A, want_B = ctx.needs_input_grad[0], ctx.needs_input_grad[2]
+            quant_B_side = None
+            if want_A:                                                      # contracted over N
                 summed = scale_A.size(0) == 1 and batch > 1 and not aT
                 ld = quantized_B.size(2) if own_B else _sum_row_bytes(N) if summed else _row_bytes(N)
                 scale_G = torch.empty((batch, M), dtype=torch.half, device=grad_f.device)
                 quant_G = torch.empty((batch, M, ld), dtype=torch.int8, device=grad_f.device)
-                gemm_backward_round_scale_ld(batch, M, N, grad_f.data_ptr(), scale_B.data_ptr(), quant_G.data_ptr(), ld,
-                                             scale_G.data_ptr(), scale_B.size(0) == 1, st)
+                if want_B:
+                    # (both operands made from the gradient in one launch)
+                    summed_B = scale_B.size(0) == 1 and batch > 1 and bT
+                    ld_t = _cols_row_bytes(M, summed_B or own_A)
+                    quant_B_side = (torch.empty((batch, N), dtype=torch.half, device=grad_f.device),
+                                    torch.empty((batch, N, ld_t), dtype=torch.int8, device=grad_f.device))
+                    gemm_backward_quantize_both(batch, M, N, grad_f.data_ptr(), scale_A.data_ptr(), scale_A.size(0) == 1, quant_B_side[0].data_ptr(),
+                                                quant_B_side[1].data_ptr(), ld_t, scale_B.data_ptr(), scale_B.size(0) == 1, quant_G.data_ptr(), ld,
+                                                scale_G.data_ptr(), st)
+                else:
+                    gemm_backward_round_scale_ld(batch, M, N, grad_f.data_ptr(), scale_B.data_ptr(), quant_G.data_ptr(), ld,
+                                                 scale_G.data_ptr(), scale_B.size(0) == 1, st)
                 other, lies = _contracted(quantized_B, K, N, ld, own_B, summed)
                 if aT:              # grad_A (b, K, M), scaled per column m
                     grad_A = gemm_and_scale(other, None, quant_G, scale_G, lies, True)
@@ -260,9 +276,9 @@ class GEMMInt8(torch.autograd.Function):
                 del quant_G, other
                 if scale_A.size(0) == 1 and grad_A.size(0) > 1:
                     grad_A = grad_A.sum(dim=0, keepdim=True)
-            if ctx.needs_input_grad[2]:                                     # contracted over M
+            if want_B:                                                      # contracted over M
                 summed = scale_B.size(0) == 1 and batch > 1 and bT
-                scale_G, quant_G, _ = _quantize_cols(grad_f, False, scale_A, summed or own_A)
+                scale_G, quant_G = quant_B_side if quant_B_side is not None else _quantize_cols(grad_f, False, scale_A, summed or own_A)[:2]
                 other, lies = _contracted(quantized_A, K, M, quant_G.size(2), own_A, summed)
                 if summed:
                     grad_B = gemm_and_scale_sum(quant_G, scale_G, other)

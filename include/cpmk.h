@@ -182,6 +182,11 @@ int cpmk_gemm_quantize_cols_ld(int32_t batch, int32_t n, int32_t m, const void* 
 int cpmk_gemm_quantize_cols_rows(int32_t batch, int32_t n, int32_t m, const void* mat, void* scale, void* out_t, int32_t ld_t, void* out_n, int32_t ld_n,
                                  int64_t rows, const void* row_mat, void* row_scale, void* row_out, void* stream);
 
+/* cpmk_gemm_quantize_cols_ld (with row scales, transposed) and cpmk_gemm_backward_round_scale_ld of one matrix in one launch: a gradient
+ * on its way to both products of a backward pass. */
+int cpmk_gemm_backward_quantize_both(int32_t batch, int32_t n, int32_t m, const void* mat, const void* row_scale, int broad_cast_row, void* scale,
+                                     void* out_t, int32_t ld_t, const void* scale_y, int broad_cast_y, void* out, int32_t ld, void* scale_x, void* stream);
+
 /* ---- fp16 products next to the path (attention scores, fp16 decode) ---------------- */
 /* Same operand convention as cpmk_gemm_int8 with fp16 operands and fp16 output, fp32
  * accumulation (the reference asks cuBLASLt for fp16 accumulation where the device has it).

@@ -41,3 +41,32 @@ def test_one_launch_equals_two(k, batch, m, rows, both):
         outs.append((scale.view(torch.int16), out_t, out_n, row_scale.view(torch.int16), row_out))
     for one, two in zip(*outs):
         assert torch.equal(one, two)
+
+
+# (rows of one to four pieces a lane and beyond them, of whole pieces or not; columns of one part and of several; scales shared by the batch or not)
+@pytest.mark.parametrize("m", [4, 72, 500, 512, 516, 1024, 1500, 2048, 2052, 2056])
+@pytest.mark.parametrize("batch,n,bc_row,bc_col", [(1, 4, True, True), (3, 70, True, False), (2, 516, False, True), (2, 1200, False, False)])
+def test_gradient_in_one_launch_equals_two(m, batch, n, bc_row, bc_col):
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    x = torch.randn((batch, n, m), generator=g, device="cuda").half()
+    rs = (torch.rand((1 if bc_row else batch, n), generator=g, device="cuda") * 0.1).half()
+    cs = (torch.rand((1 if bc_col else batch, m), generator=g, device="cuda") * 0.1).half()
+    x[0, 1], x[-1, :, 2] = 0.0, 0.0
+    x[0, 0, 1] = float("nan")
+    x[-1, 3] *= 1e-4
+    ld, ld_t = _ld(m), _ld(n)
+    outs = []
+    for joint in (False, True):
+        scale = torch.full((batch, m), 7.0, dtype=torch.half, device="cuda")
+        out_t = torch.full((batch, m, ld_t), 77, dtype=torch.int8, device="cuda")
+        row_scale = torch.full((batch, n), 7.0, dtype=torch.half, device="cuda")
+        out = torch.full((batch, n, ld), 77, dtype=torch.int8, device="cuda")
+        if joint:
+            ck.gemm_backward_quantize_both(batch, n, m, x.data_ptr(), rs.data_ptr(), bc_row, scale.data_ptr(), out_t.data_ptr(), ld_t,
+                                           cs.data_ptr(), bc_col, out.data_ptr(), ld, row_scale.data_ptr(), stream())
+        else:
+            ck.gemm_quantize_cols_ld(batch, n, m, x.data_ptr(), rs.data_ptr(), bc_row, scale.data_ptr(), out_t.data_ptr(), ld_t, None, 0, stream())
+            ck.gemm_backward_round_scale_ld(batch, n, m, x.data_ptr(), cs.data_ptr(), out.data_ptr(), ld, row_scale.data_ptr(), bc_col, stream())
+        outs.append((scale.view(torch.int16), out_t, row_scale.view(torch.int16), out))
+    for one, two in zip(*outs):
+        assert torch.equal(one, two)

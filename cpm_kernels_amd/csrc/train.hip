@@ -168,34 +168,38 @@ __global__ __launch_bounds__(256) void k_gelu_backward(int64_t total, const half
 // Sums over everything but one index (fp32 accumulation, one workgroup per output).
 // ---------------------------------------------------------------------------------------
 // grad[j] = sum_b grad_out[b, j]                                            cu_arith_batch_add_backward
-// A lane owns eight adjacent columns: one 16-byte load per row at whatever address the piece starts (global loads need
-// no alignment), eight rows requested at a time, the sums in fp32; the piece across the end of the row in narrower
-// accesses.  With few columns the rows are dealt to `rgs` (a power of two up to 64) groups of 256 / rgs lanes, whose
-// sums are added in group order.
+// Bound by reading grad_out.  A lane owns eight adjacent columns, of the last ones those that end the row (they repeat some of the lane's before): one 16-byte load per row at
+// whatever address the piece starts (global loads need no alignment), NB rows requested at a time, rows past the last as the last one once more, so that no load is under a
+// condition; the sums in fp32.  With few columns the rows are dealt to `rgs` (a power of two up to 64) groups of 256 / rgs lanes, whose sums are added in group order.
+// 4 rows of 16.8 million 34 -> 27 us (6.3 TB/s), 3 of 24.4 million 42 -> 30, 8 of 16 million 57 -> 45, each load under conditions of its own before.
+// WHOLE: at least eight columns.  NTH: with the non-temporal hint.
+template <int NB, bool WHOLE, bool NTH>
 __global__ __launch_bounds__(256) void k_batch_add_backward(int64_t batch, int64_t n, int rgs, const half_t* __restrict__ grad_out,
                                                             half_t* __restrict__ grad) {
     __shared__ float red[2048];                 // [row group][column of the workgroup]
     const int cgs = 256 / rgs, cg = threadIdx.x % cgs, rg = threadIdx.x / cgs;
-    const int64_t col = ((int64_t)blockIdx.x * cgs + cg) * 8;
-    const int t = col >= n ? 0 : n - col >= 8 ? 8 : (int)(n - col);
+    const int64_t first = ((int64_t)blockIdx.x * cgs + cg) * 8;
+    const bool live = first < n;
+    const int64_t col = WHOLE ? min(first, n - 8) : 0;
+    const int t = WHOLE ? 8 : (int)n;           // columns of a lane
     const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
     float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    if (t > 0) {
-        for (int64_t i0 = rg; i0 < batch; i0 += 8 * rgs) {
-            half8_t v[8];
+    if (live) {
+        for (int64_t i0 = rg; i0 < batch; i0 += NB * rgs) {
+            half8_t v[NB];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                v[u] = zero;
-                const int64_t i = i0 + (int64_t)u * rgs;
-                if (i < batch) {
-                    const half_t* src = grad_out + i * n + col;
-                    v[u] = t == 8 ? load_half8_any(src) : load_half8_head_any(src, t, zero);
-                }
+            for (int u = 0; u < NB; ++u) {
+                const half_t* const src = grad_out + min(i0 + (int64_t)u * rgs, batch - 1) * n + col;
+                if constexpr (!WHOLE) v[u] = i0 + (int64_t)u * rgs < batch ? load_half8_head_any(src, t, zero) : zero;
+                else if constexpr (NTH) v[u] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(src));
+                else v[u] = load_half8_any(src);
             }
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
+            for (int u = 0; u < NB; ++u) {
+                const bool in = i0 + (int64_t)u * rgs < batch;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) s[e] += (float)v[u][e];
+                for (int e = 0; e < 8; ++e) s[e] = in ? s[e] + (float)v[u][e] : s[e];
+            }
         }
     }
     if (rgs > 1) {
@@ -210,11 +214,11 @@ __global__ __launch_bounds__(256) void k_batch_add_backward(int64_t batch, int64
             s[e] = a;
         }
     }
-    if (t == 0) return;
+    if (!live) return;
     half8_t r;
 #pragma unroll
     for (int e = 0; e < 8; ++e) r[e] = round_f16(s[e]);
-    if (t == 8) store_half8_any(grad + col, r);
+    if constexpr (WHOLE) store_half8_any(grad + col, r);
     else store_half8_head_any(grad + col, t, r);
 }
 
@@ -1038,8 +1042,16 @@ int cpmk_arith_batch_add_backward(int32_t batch, int64_t n, const void* grad_out
     // enough lanes for the whole chip: with few columns, more row groups per workgroup
     int rgs = 1;
     while (rgs < 64 && ceil_div(n, 8) * rgs < 131072 && rgs * 2 <= batch) rgs *= 2;
-    hipLaunchKernelGGL(k_batch_add_backward, dim3((unsigned)ceil_div(n, (256 / rgs) * 8)), dim3(256), 0, (hipStream_t)stream, (int64_t)batch,
-                       n, rgs, (const half_t*)grad_out, (half_t*)grad);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(n, (256 / rgs) * 8)), dim3(256), 0, (hipStream_t)stream, (int64_t)batch, n, rgs, (const half_t*)grad_out,
+                           (half_t*)grad);
+    };
+    // (the hint for what is twice the last-level cache and more: 16 rows of 67 million 404 us, 491 without; 16 of 5.8 million 39 and 31)
+    const bool nth = n % 8 == 0 && aligned16(grad_out) && (int64_t)batch * n >= 1ll << 28;
+    if (n < 8) go(k_batch_add_backward<8, false, false>);
+    else if (rgs > 1) go(k_batch_add_backward<8, true, false>);
+    else if (nth) go(k_batch_add_backward<4, true, true>);
+    else go(k_batch_add_backward<4, true, false>);
     return launch_status();
 }
 int cpmk_arith_ln_mul_backward(int32_t batch, int32_t n, int32_t m, const void* inp, const void* grad_out, void* grad, void* stream) {

@@ -688,7 +688,7 @@ int cpmk_gemm_backward_quantize_both(int32_t batch, int32_t n, int32_t m, const 
         if (rc >= 0) return rc;
     }
     if (const int rc = cpmk_gemm_backward_round_scale_ld(batch, n, m, mat, scale_y, out, ld, scale_x, broad_cast_y, stream)) return rc;
-    if (row_scale == nullptr && (int64_t)batch * m > 0) return CPMK_EBADARG;
+    if (row_scale == nullptr && rows > 0 && m > 0) return CPMK_EBADARG;       // (without rows there are no scales of theirs)
     return cpmk_gemm_quantize_cols_ld(batch, n, m, mat, row_scale, broad_cast_row, scale, out_t, ld_t, nullptr, 0, stream);
 }
 

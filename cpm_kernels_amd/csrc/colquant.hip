@@ -28,7 +28,7 @@ namespace cpmk {
 // NTH: the tile's 128-byte row segments are whole cache lines (m % 64 == 0, the matrix on a 128-byte boundary): the input is
 // read with the non-temporal hint.  Elsewhere a line is shared with the neighbouring tile and has to stay in L2 for it.
 // UA: any m and alignment: a piece inside its row still moves whole, at whatever address it lies (global accesses need
-// no alignment); the piece across a row's end is read (and its scales and, not transposed, its int8 values are
+// no alignment); the piece across a row's end is read with what lies behind it (and its scales and, not transposed, its int8 values are
 // written) in at most three narrower accesses.
 // OUT: bit 0 the transposed output, bit 1 the one in place.
 struct ColQuantArgs {
@@ -69,33 +69,50 @@ __device__ __forceinline__ void col_quantize_team(const ColQuantArgs& a, int32_t
     const int32_t row0 = part * ROWS + rg * 8;           // this lane's first row
     const int64_t boff = (int64_t)b * n * m;
 
-    float sx[R];        // SCALED: the lane's rows' scales, requested ahead of the tile
+    half_t sxh[SCALED ? R : 1];        // the lane's rows' scales, requested ahead of the tile (each under a condition they waited for one another)
     if constexpr (SCALED) {
         const half_t* rs = a.row_scale + (a.bc ? 0 : (int64_t)b * n);
 #pragma unroll
-        for (int p = 0; p < R; ++p) sx[p] = row0 + p < n ? (float)rs[row0 + p] : 0.0f;
+        for (int p = 0; p < R; ++p) sxh[p] = rs[min(row0 + p, n - 1)];
     }
     // one lane offset beside a scalar address per row of the lane (n * m < 2^31: the offset in bytes of a row within the matrix fits)
     const half_t* const tbase = mat + boff + (int64_t)part * ROWS * m;
     const uint32_t loff = ((uint32_t)(rg * 8) * (uint32_t)m + (uint32_t)col0) * 2u;
     half8_t v[R];
+    const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    const bool narrow = UA && (int64_t)n * m < 8;        // (a matrix of less than a piece)
+    if (UA && !narrow) {
+        // every load is made, rows past the last as the last one, and put right behind them all
+        const half_t* const mb = mat + boff;
+        const uint32_t last = (uint32_t)n * (uint32_t)m - 8u, col = (uint32_t)min(col0, m - 1);
 #pragma unroll
-    for (int p = 0; p < R; ++p) {
+        for (int p = 0; p < R; ++p) v[p] = load_half8_any(mb + min((uint32_t)min(row0 + p, n - 1) * (uint32_t)m + col, last));
+        if (row0 + R > n || col0 + 8 > m) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[p][e] = (half_t)0.0f;
-        const half_t* const src = reinterpret_cast<const half_t*>(reinterpret_cast<const char*>(tbase + (int64_t)p * m) + loff);
-        if constexpr (UA) {
-            if (row0 + p < n) {
-                if (col0 + 8 <= m) {
-                    v[p] = load_half8_any(src);
-                } else if (col0 < m) {
-                    v[p] = load_half8_head_any(src, m & 7, v[p]);
+            for (int p = 0; p < R; ++p) {
+                const uint32_t at = (uint32_t)min(row0 + p, n - 1) * (uint32_t)m + col;
+                v[p] = half8_head(v[p], at > last ? (int)(at - last) : 0, row0 + p < n ? m - col0 : 0, (half_t)0.0f);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int p = 0; p < R; ++p) {
+            v[p] = zero8;
+            const half_t* const src = reinterpret_cast<const half_t*>(reinterpret_cast<const char*>(tbase + (int64_t)p * m) + loff);
+            if (row0 + p < n && col0 < m) {
+                if constexpr (UA) {
+                    v[p] = load_half8_head_any(src, m & 7, zero8);
+                } else {
+                    const half8_t* src8 = reinterpret_cast<const half8_t*>(src);
+                    v[p] = NTH ? __builtin_nontemporal_load(src8) : *src8;        // read once; the int8 output below is what the next kernel wants in cache
                 }
             }
-        } else if (row0 + p < n && col0 < m) {
-            const half8_t* src8 = reinterpret_cast<const half8_t*>(src);
-            v[p] = NTH ? __builtin_nontemporal_load(src8) : *src8;        // read once; the int8 output below is what the next kernel wants in cache
         }
+    }
+    float sx[SCALED ? R : 1];
+    if constexpr (SCALED) {
+#pragma unroll
+        for (int p = 0; p < R; ++p) sx[p] = row0 + p < n ? (float)sxh[p] : 0.0f;
     }
     // The maxima over the rows of a wave, then over the workgroup's waves: thread i < COLS ends up with that of column i.
     float M = 0.0f;

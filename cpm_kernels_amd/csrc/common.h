@@ -75,6 +75,24 @@ __device__ __forceinline__ void store_half8_head_any(half_t* p, int t, half8_t v
     }
     if (t & 1) p[t & 6] = (t & 6) == 0 ? v[0] : (t & 6) == 2 ? v[2] : (t & 6) == 4 ? v[4] : v[6];
 }
+// Pieces that may end behind a row's end, for loads that are not under conditions (which the compiler lets wait for one another, with copies behind each): read
+// where the piece lies, or the buffer's last eight halves if it would end behind those (`over` halves later), and put right afterwards: moved down by `over`, halves from `keep` on
+// replaced by `fill`.
+__device__ __forceinline__ half8_t half8_head(half8_t v, int over, int keep, half_t fill) {
+    typedef uint64_t ulong2_t __attribute__((ext_vector_type(2)));
+    ulong2_t w = __builtin_bit_cast(ulong2_t, v);
+    if (over >= 4) {
+        w[0] = w[1];
+        w[1] = 0;
+    }
+    const int bits = (over & 3) * 16;
+    w[0] = (w[0] >> bits) | ((w[1] << 1) << (63 - bits));
+    w[1] >>= bits;
+    v = __builtin_bit_cast(half8_t, w);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = e < keep ? v[e] : fill;
+    return v;
+}
 // the first t (1..7) of the eight bytes lo | hi << 32 to p, at any address
 struct __attribute__((packed, aligned(1))) Byte4Any { uint32_t x; };
 struct __attribute__((packed, aligned(1))) Byte2Any { uint16_t x; };

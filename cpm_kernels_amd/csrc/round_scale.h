@@ -35,7 +35,7 @@ __device__ __forceinline__ uint2_t round8_own_scale(half8_t x, half8_t sy, float
 // row's maximum over the wave with data-parallel-primitive operands and rounds from the registers.
 // UA: rows that are not whole 16-byte pieces or buffers off 16-byte boundaries -- a piece inside its row still comes in
 // one 16-byte load and leaves in one 8-byte store (global accesses need no alignment), the piece across a row's end
-// in at most three narrower accesses each way.
+// is read with what lies behind it and leaves in at most three narrower accesses.
 // The two rounding sequences are chosen once for the wave's rows: a choice per row kept their chains from running side by side (780 rows
 // of 24 6.9 us, 4.7 so; 20000 of 512 11.1 -> 8.1; 81920 of 512 30 -> 23.5, 5.3 TB/s).
 template <int P, int U, bool UA>
@@ -45,30 +45,51 @@ __device__ __forceinline__ void round_scale_rows_reg(const RoundScaleArgs& a, in
     const int lane = threadIdx.x & 63;
     const int64_t row0 = wave * U;
     if (row0 >= rows) return;
-    auto load8 = [&](const half_t* src, int32_t j, bool nt) __attribute__((always_inline)) {
-        half8_t r = {0, 0, 0, 0, 0, 0, 0, 0};
-        if constexpr (!UA) {
-            r = nt ? __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(src + j)) : *reinterpret_cast<const half8_t*>(src + j);
-        } else if (j + 8 <= m) {
-            r = load_half8_any(src + j);
-        } else {
-            r = load_half8_head_any(src + j, m & 7, r);       // (callers pass j < m)
-        }
-        return r;
-    };
     half8_t xv[U][P], sv[U][P];
+    const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    // UA: every load is made (pieces past a row's end as its first one) and put right behind them all: a row's end lies in every wave, and under conditions of their own the loads
+    // waited for one another (4 x 10240 rows of 500 33 -> 26 us, 4 x 896 of 172 9.6 -> 8.0).  Rows of less than a piece take the conditions.
+    const int64_t last_x = rows * m - 8, last_s = (a.bc ? 1 : rows / n) * (int64_t)m - 8;
+    const bool pieces = !UA || m >= 8;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int64_t row = row0 + u < rows ? row0 + u : rows - 1;
-        const half_t* x = a.mat + row * m;
-        const half_t* sy = a.scale_y + (a.bc ? 0 : (row / n) * m);
+        const int64_t x0 = row * m, s0 = a.bc ? 0 : (row / n) * m;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             const int32_t j = lane * 8 + p * 512;
-            xv[u][p] = sv[u][p] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-            if (j < m) {
-                xv[u][p] = load8(x, j, true);
-                sv[u][p] = load8(sy, j, false);
+            if constexpr (UA) {
+                if (pieces) {
+                    const int32_t jc = j < m ? j : 0;
+                    xv[u][p] = load_half8_any(a.mat + min(x0 + jc, last_x));
+                    sv[u][p] = load_half8_any(a.scale_y + min(s0 + jc, last_s));
+                } else {
+                    xv[u][p] = j < m ? load_half8_head_any(a.mat + x0, m, zero) : zero;
+                    sv[u][p] = j < m ? load_half8_head_any(a.scale_y + s0, m, zero) : zero;
+                }
+            } else {
+                xv[u][p] = sv[u][p] = zero;
+                if (j < m) {
+                    xv[u][p] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(a.mat + x0 + j));
+                    sv[u][p] = *reinterpret_cast<const half8_t*>(a.scale_y + s0 + j);
+                }
+            }
+        }
+    }
+    if (UA && pieces) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t row = row0 + u < rows ? row0 + u : rows - 1;
+            const int64_t x0 = row * m, s0 = a.bc ? 0 : (row / n) * m;
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int32_t j = lane * 8 + p * 512;
+                if (j + 8 > m) {
+                    const int32_t keep = m - j;
+                    const int64_t ox = x0 + j - last_x, os = s0 + j - last_s;
+                    xv[u][p] = half8_head(xv[u][p], keep > 0 && ox > 0 ? (int)ox : 0, keep, (half_t)0.0f);
+                    sv[u][p] = half8_head(sv[u][p], keep > 0 && os > 0 ? (int)os : 0, keep, (half_t)0.0f);
+                }
             }
         }
     }

@@ -390,8 +390,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KIND == kSof
     if constexpr (KIND == kScaleRound) {
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-            const int32_t row = own0 + q * T::RPP + rg;
-            sxh[q] = row < p.n ? p.sx[(p.bc ? 0 : (int64_t)b * p.n) + row] : (half_t)0.0f;
+            sxh[q] = p.sx[(p.bc ? 0 : (int64_t)b * p.n) + min(own0 + q * T::RPP + rg, p.n - 1)];       // (the tile's rows past the last are zeros)
         }
     }
     constexpr bool NTH = MODE == 0, UA = MODE == 2;

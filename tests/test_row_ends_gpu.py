@@ -1,0 +1,74 @@
+"""Pieces across the end of a row are read with what lies behind it: columns of NaN next to it, in the following row, stay out of the others, also in the last row and in
+matrices of less than a piece."""
+import pytest
+import torch
+
+import cpm_kernels_amd.kernels as ck
+from util import stream
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 2), (1, 6), (2, 2), (3, 4), (1, 10), (2, 12), (50, 70), (100, 100), (130, 66), (300, 30), (240, 236), (500, 500), (520, 20), (1000, 134)]
+
+
+def _pair(batch, n, m, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn((batch, n, m), generator=g, device="cuda").half()
+    y = x.clone()
+    y[:, :, 0] = float("nan")
+    return x, y
+
+
+def _same(outs, axis):
+    for one, two in zip(*outs):
+        keep = torch.arange(1, one.size(axis), device="cuda")
+        a, b = one.index_select(axis, keep), two.index_select(axis, keep)
+        assert torch.equal(a.view(torch.int16) if a.dtype == torch.half else a, b.view(torch.int16) if b.dtype == torch.half else b)
+        if one.dtype == torch.half:
+            assert not a.isnan().any()
+
+
+@pytest.mark.parametrize("n,m", SIZES)
+def test_softmax_columns(n, m):
+    x, y = _pair(3, n, m, n + m)
+    grad = _pair(3, n, m, n)[0]
+    outs = []
+    for v in (x, y):
+        out, back = torch.empty_like(v), torch.empty_like(v)
+        ck.softmax_forward(3, n, m, v.data_ptr(), out.data_ptr(), stream())
+        probs = out.clone()
+        probs[:, :, 0] = v[:, :, 0]
+        ck.softmax_backward(3, n, m, probs.data_ptr(), grad.data_ptr(), back.data_ptr(), stream())
+        outs.append((out, back))
+    _same(outs, 2)
+    ref = torch.softmax(x.double(), 1)
+    assert ((outs[0][0].double() - ref).abs() <= ref * 2.0 ** -10 + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("n,m", SIZES)
+@pytest.mark.parametrize("scaled", [False, True])
+def test_quantised_columns(n, m, scaled):
+    rows = torch.rand((3, n), device="cuda").half()
+    ld = (n + 127) // 128 * 128
+    outs = []
+    for v in _pair(3, n, m, n * 3 + m):
+        scale, out = torch.empty((3, m), dtype=torch.half, device="cuda"), torch.empty((3, m, ld), dtype=torch.int8, device="cuda")
+        ck.gemm_quantize_cols_ld(3, n, m, v.data_ptr(), rows.data_ptr() if scaled else None, False, scale.data_ptr(), out.data_ptr(), ld, None, 0, stream())
+        outs.append((scale, out))
+    _same(outs, 1)
+    assert (outs[0][1][:, :, n:] == 0).all()
+
+
+# (the maximum of a row skips NaN, so it has a row of values of its own in front: what a row's end must not take from the next row)
+@pytest.mark.parametrize("m", [2, 6, 10, 70, 172, 500, 516, 1030, 2044])
+def test_scaled_rows(m):
+    n, ld = 70, (m + 127) // 128 * 128
+    x = _pair(2, n, m, m)[0]
+    x[:, 1::2] *= 1000.0
+    cols = torch.rand((2, m), device="cuda").half() + 0.5
+    scale, out = torch.empty((2, n), dtype=torch.half, device="cuda"), torch.empty((2, n, ld), dtype=torch.int8, device="cuda")
+    ck.gemm_backward_round_scale_ld(2, n, m, x.data_ptr(), cols.data_ptr(), out.data_ptr(), ld, scale.data_ptr(), False, stream())
+    p = x.float() * cols.float()[:, None, :]
+    s = (p.abs().amax(2).double() / 127.0).float()
+    assert torch.equal(scale, s.half())
+    assert torch.equal(out[:, :, :m].float(), torch.round(p / s[:, :, None])) and (out[:, :, m:] == 0).all()

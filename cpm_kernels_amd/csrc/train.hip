@@ -910,7 +910,7 @@ static int launch_col(int32_t batch, const ColArgs& p, void* stream, bool missin
                        (p.out_mean == nullptr || aligned16(p.out_mean)) && (p.out_var == nullptr || aligned16(p.out_var)) &&
                        (p.out_i8 == nullptr || (reinterpret_cast<uintptr_t>(p.out_i8) & 7u) == 0);
     // The softmax gradient, whose columns are a sequence: tiles no taller than they take, so that more workgroups share a compute unit (1024 of 100 x 100
-    // 42.6 -> 15.5 us, 528 of 236 x 236 74 -> 35), and up to 1024 rows in one workgroup, which waits for no other one (66 of 902 x 902 114 -> 64,
+    // 42.6 -> 15.5 us, 528 of 236 x 236 74 -> 35, both quicker still with loads that do not wait for one another), and up to 1024 rows in one workgroup, which waits for no other one (66 of 902 x 902 114 -> 64,
     // 128 of 1024 x 1024 162 -> 130; with two of them a compute unit, 128 registers a lane, 256 of 512 x 512 74 -> 63).
     const int64_t parts = KIND == kSoftmaxBwd && p.n <= 1024 ? 1 : ceil_div(p.n, 512);
     const bool wide = (int64_t)p.n * p.m < (1ll << 31) && parts <= kColTeamMaxParts && tiles * parts <= kXchSlots;

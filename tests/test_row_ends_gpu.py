@@ -72,3 +72,14 @@ def test_scaled_rows(m):
     s = (p.abs().amax(2).double() / 127.0).float()
     assert torch.equal(scale, s.half())
     assert torch.equal(out[:, :, :m].float(), torch.round(p / s[:, :, None])) and (out[:, :, m:] == 0).all()
+
+
+# many ragged sequences: lanes that work for themselves
+@pytest.mark.parametrize("batch,n,m", [(1024, 386, 266), (420, 512, 470), (400, 500, 502), (1540, 450, 146)])
+def test_softmax_of_many_sequences(batch, n, m):
+    x = _pair(batch, n, m, batch)[0]
+    out = torch.empty_like(x)
+    ck.softmax_forward(batch, n, m, x.data_ptr(), out.data_ptr(), stream())
+    for i in (0, 1, batch // 2, batch - 1):
+        ref = torch.softmax(x[i].double(), 0)
+        assert ((out[i].double() - ref).abs() <= ref * 2.0 ** -10 + 2.0 ** -24).all()

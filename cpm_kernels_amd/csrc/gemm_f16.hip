@@ -189,6 +189,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
                      : two ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, 3, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, kRingSmall, 3, 32>(a, batch, st);
         }
     }
+    if (seg) return CPMK_EBADARG;       // (never: joined products are the tile kernel's; here they would be written as one matrix)
     return gemm_f16_any(m, k, n, batchA, batchB, aT, bT, A, B, out, st);
 }
 

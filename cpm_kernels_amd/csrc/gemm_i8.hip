@@ -284,10 +284,10 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
         n *= batch;
         batch = batchB = 1;
     }
-    // (columns: where whole entries of them leave tiles half empty)
+    // (columns: where whole entries of them leave tiles half empty, and operands that the tile kernel takes: it alone knows of `seg`)
     int32_t seg = 0;
-    if (FUSED && batchB == 1 && aT && (srow == nullptr || bcr) && (scol == nullptr || !bcc) && cols_join(batch, m, k) && aligned16(A) && aligned16(B) && aligned16(out) &&
-        k > 0 && (bT ? k % 128 == 0 && n % 16 == 0 : k % 64 == 0) &&
+    if (FUSED && batchB == 1 && aT && (srow == nullptr || bcr) && (scol == nullptr || !bcc) && cols_join(batch, m, k) && (int64_t)n * k < (1ll << 32) && aligned16(A) &&
+        aligned16(B) && aligned16(out) && k > 0 && (bT ? k % 128 == 0 && n % 16 == 0 : k % 64 == 0) &&
         (ceil_div((int64_t)m * batch, 128) < ceil_div(m, 128) * batch || ceil_div((int64_t)m * batch, 256) < ceil_div(m, 256) * batch)) {
         seg = m;
         m *= batch;
@@ -385,6 +385,7 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
             default: return large ? launch_dma<2, 4, 4, 2, 128, EPI, 2, 3, 16>(a, batch, st) : launch_dma<2, 2, 2, 2, 128, EPI, kRingSmall, 3, 32>(a, batch, st);
         }
     }
+    if (seg) return CPMK_EBADARG;       // (never: joined products are the tile kernel's; below they would be written as one matrix)
     // one operand stored (K, rows) and a depth beyond one slab that is not whole slabs: the 32x32 form of the tile kernel,
     // the rest of the depth as a slab filled up with zeros
     if (p_kmajor != q_kmajor && wide && k > 128 && (k % 4 == 0) && aligned16(A) && aligned16(B) && (!in_p || n >= 128) &&

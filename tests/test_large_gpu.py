@@ -179,6 +179,31 @@ def test_gemm_int8_operand_beyond_2_gib_and_output_beyond_2_31(gpu):
         assert_bits_equal(to_np(o16[:, rows]), ref, "fused rows %d.." % r0)
 
 
+@pytest.mark.parametrize("n", [262128, 262144])
+@pytest.mark.parametrize("bT", [False, True])
+def test_gemm_int8_row_operand_of_4_gib_shared_by_the_batch(gpu, n, bT):
+    """Four entries of 64 columns beside a row operand of just under and of exactly 2^32 bytes: the columns are one product up to there"""
+    k, m, batch = 16384, 64, 4
+    _name("gemm_int8_scale, shared row operand", (n, k, m, batch), bT)
+    g = torch.Generator(device=gpu).manual_seed(16)
+    P = torch.empty((k, n) if bT else (n, k), dtype=torch.int8, device=gpu)
+    P.view(torch.int64).random_(generator=g)
+    P.clamp_(min=-127)
+    Q = torch.randint(-127, 128, (batch, m, k), generator=g, dtype=torch.int8, device=gpu)
+    srow = (torch.rand(n, generator=g, device=gpu) * 0.01 + 1e-4).half()
+    scol = (torch.rand((batch, m), generator=g, device=gpu) * 0.01 + 1e-4).half()
+    out = torch.full((batch, n, m), float("nan"), dtype=torch.half, device=gpu)
+    ck.gemm_int8_scale(m, k, n, batch, 1, True, bT, Q.data_ptr(), P.data_ptr(), srow.data_ptr(), scol.data_ptr(), True, False, out.data_ptr(), stream())
+    Qn = to_np(Q)
+    for r0 in (0, n // 2 - 8, n - 16):
+        rows = slice(r0, r0 + 16)
+        Pn = to_np(P[:, rows].t().contiguous() if bT else P[rows])
+        for i in range(batch):
+            ref = oracle.gemm_scale(_rows_ref(Pn, Qn[i], slice(None))[None], to_np(srow[rows]), to_np(scol[i]), True, True)
+            assert_bits_equal(to_np(out[i:i + 1, rows]), ref, "entry %d, rows %d.." % (i, r0))
+    assert not out.isnan().any()
+
+
 def test_batches_beyond_the_grid_limit(gpu):
     """70000 batch entries: more than a grid's y or z dimension holds (65535).  The reference indexes
     the batch with the grid's x dimension and has no such limit (kernels/softmax.py:20,

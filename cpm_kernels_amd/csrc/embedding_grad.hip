@@ -58,6 +58,7 @@ struct PrepareArgs {
     half_t *rows, *table;
     int64_t total;                // elements of the table
     uint32_t rank_blocks, tile_blocks, tiles_c, tiles_r, tiles;
+    uint32_t first;               // number of the launch's first workgroup
 };
 constexpr int kPrepareThreads = 64 * kRankWaves;
 constexpr int64_t kFillBytes = 8 * 16 * kPrepareThreads;      // zeros a workgroup writes
@@ -66,11 +67,12 @@ constexpr int64_t kFillBytes = 8 * 16 * kPrepareThreads;      // zeros a workgro
 // lane a block of 8 x 8, with 128-byte segments on both sides; else through LDS.
 template <bool PIECES>
 __global__ __launch_bounds__(kPrepareThreads) void k_embedding_prepare(PrepareArgs a) {
-    if (blockIdx.x < a.rank_blocks) {
-        rank_ids(blockIdx.x, a.tokens, a.ids, a.order, a.sorted);
+    const uint32_t wg = a.first + blockIdx.x;
+    if (wg < a.rank_blocks) {
+        rank_ids(wg, a.tokens, a.ids, a.order, a.sorted);
         return;
     }
-    const uint32_t at = blockIdx.x - a.rank_blocks;
+    const uint32_t at = wg - a.rank_blocks;
     const bool is_tile = at < a.tile_blocks;
     const uint32_t block = is_tile ? at : at - a.tile_blocks;
     if (is_tile) {
@@ -310,13 +312,19 @@ int cpmk_embedding_backward_prepare(int32_t batch, int32_t hidden_size, int32_t 
     const bool pieces = hidden_size % 8 == 0 && seq_len % 8 == 0 && aligned16(grad_out) && aligned16(grad_rows);
     const int64_t tc = ceil_div(seq_len, 64), tr = ceil_div(hidden_size, 64), tiles = tc * tr * batch;
     const int64_t rank = ids ? ceil_div(tokens, 64) : 0, tile_blocks = ceil_div(tiles, pieces ? kRankWaves : 4), fill = ceil_div(total * 2, kFillBytes);
-    if (rank + tile_blocks + fill == 0) return 0;
-    if (tiles >= 1ll << 32 || rank + tile_blocks + fill >= 1ll << 22) return CPMK_ETOOBIG;       // (a launch holds fewer than 2^32 threads)
+    const int64_t total_blocks = rank + tile_blocks + fill;
+    if (tiles >= 1ll << 32 || total_blocks >= 1ll << 32) return CPMK_ETOOBIG;       // (more than the device's memory holds)
     a.rank_blocks = (uint32_t)rank; a.tile_blocks = (uint32_t)tile_blocks; a.tiles_c = (uint32_t)tc; a.tiles_r = (uint32_t)tr; a.tiles = (uint32_t)tiles;
-    const dim3 grid((unsigned)(rank + tile_blocks + fill));
-    if (pieces) hipLaunchKernelGGL(k_embedding_prepare<true>, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a);
-    else hipLaunchKernelGGL(k_embedding_prepare<false>, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a);
-    return launch_status();
+    // a launch holds fewer than 2^32 threads: many short sequences, each a tile and more, go out in several
+    constexpr int64_t most = (1ll << 32) / kPrepareThreads - 1;
+    for (int64_t b0 = 0; b0 < total_blocks; b0 += most) {
+        a.first = (uint32_t)b0;
+        const dim3 grid((unsigned)(total_blocks - b0 < most ? total_blocks - b0 : most));
+        if (pieces) hipLaunchKernelGGL(k_embedding_prepare<true>, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL(k_embedding_prepare<false>, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a);
+        if (const int e = launch_status()) return e;
+    }
+    return 0;
 }
 
 }  // extern "C"

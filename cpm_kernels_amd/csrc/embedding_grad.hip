@@ -48,12 +48,10 @@ __global__ __launch_bounds__(64 * kRankWaves) void k_rank_ids(int32_t tokens, co
 
 // What has to be done before the rows are summed, in one launch: the order of the ids, the gradient (batch, hidden, seq) as rows (tokens, hidden),
 // and zeros in the table.  Bound by memory: the counting, 64 workgroups that hardly use it, and the transposition, which waits at barriers, pass under
-// the zeros: 4096 tokens x 4096 beside 30000 rows 63 us in three launches, 50 so; 310 x 1216 beside 11794 14.6 and 7.9; 16384 x 2048 beside 50000, where the
-// counting takes 28, 85 and 73 (tiles and zeros in turn 84).
+// the zeros: 4096 tokens x 4096 beside 30000 rows 64 us in three launches, 42 so; 310 x 1216 beside 11794 12.1 and 7.3; 16384 x 2048 beside 50000, where the
+// counting takes 24, 92 and 48.
 struct PrepareArgs {
     int32_t tokens, hidden, seq;
-    const int32_t* ids;
-    int32_t *order, *sorted;      // null: ordered already
     const half_t* grad;
     half_t *rows, *table;
     int64_t total;                // elements of the table
@@ -65,11 +63,14 @@ constexpr int64_t kFillBytes = 8 * 16 * kPrepareThreads;      // zeros a workgro
 
 // PIECES: rows of grad and of the transposed rows are whole aligned 16-byte pieces: a wave transposes a tile of 64 x 64 in registers, each
 // lane a block of 8 x 8, with 128-byte segments on both sides; else through LDS.
+// (the ids are an argument of their own, which no other pointer reaches: as a member of `a` the compiler took their loads for ones that the stores here
+// could change and left them to the vector unit, sixteen ids four vector loads instead of one scalar one: 250 x 64 tokens of 70 beside 500 rows 38.1 us, 24.2 so)
 template <bool PIECES>
-__global__ __launch_bounds__(kPrepareThreads) void k_embedding_prepare(PrepareArgs a) {
+__global__ __launch_bounds__(kPrepareThreads) void k_embedding_prepare(PrepareArgs a, const int32_t* __restrict__ ids, int32_t* __restrict__ order,
+                                                                       int32_t* __restrict__ sorted) {
     const uint32_t wg = a.first + blockIdx.x;
     if (wg < a.rank_blocks) {
-        rank_ids(wg, a.tokens, a.ids, a.order, a.sorted);
+        rank_ids(wg, a.tokens, ids, order, sorted);
         return;
     }
     const uint32_t at = wg - a.rank_blocks;
@@ -307,7 +308,6 @@ int cpmk_embedding_backward_prepare(int32_t batch, int32_t hidden_size, int32_t 
     if (total > 0 && !aligned16(grad)) return CPMK_EALIGN;
     PrepareArgs a;
     a.tokens = (int32_t)tokens; a.hidden = hidden_size; a.seq = seq_len;
-    a.ids = (const int32_t*)ids; a.order = (int32_t*)order; a.sorted = (int32_t*)sorted_ids;
     a.grad = (const half_t*)grad_out; a.rows = (half_t*)grad_rows; a.table = (half_t*)grad; a.total = total;
     const bool pieces = hidden_size % 8 == 0 && seq_len % 8 == 0 && aligned16(grad_out) && aligned16(grad_rows);
     const int64_t tc = ceil_div(seq_len, 64), tr = ceil_div(hidden_size, 64), tiles = tc * tr * batch;
@@ -320,8 +320,11 @@ int cpmk_embedding_backward_prepare(int32_t batch, int32_t hidden_size, int32_t 
     for (int64_t b0 = 0; b0 < total_blocks; b0 += most) {
         a.first = (uint32_t)b0;
         const dim3 grid((unsigned)(total_blocks - b0 < most ? total_blocks - b0 : most));
-        if (pieces) hipLaunchKernelGGL(k_embedding_prepare<true>, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL(k_embedding_prepare<false>, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(kPrepareThreads), 0, (hipStream_t)stream, a, (const int32_t*)ids, (int32_t*)order, (int32_t*)sorted_ids);
+        };
+        if (pieces) go(k_embedding_prepare<true>);
+        else go(k_embedding_prepare<false>);
         if (const int e = launch_status()) return e;
     }
     return 0;

@@ -82,16 +82,29 @@ __device__ __forceinline__ void col_quantize_team(const ColQuantArgs& a, int32_t
     const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
     const bool narrow = UA && (int64_t)n * m < 8;        // (a matrix of less than a piece)
     if (UA && !narrow) {
-        // every load is made, rows past the last as the last one, and put right behind them all
+        // Every load is made, rows past the last as the last one, and put right behind them all; waves that have no rows leave them out
         const half_t* const mb = mat + boff;
         const uint32_t last = (uint32_t)n * (uint32_t)m - 8u, col = (uint32_t)min(col0, m - 1);
+        if (!SCALED && __builtin_amdgcn_readfirstlane(row0) >= n) {        // (80 registers do not hold that choice beside the scales)
 #pragma unroll
-        for (int p = 0; p < R; ++p) v[p] = load_half8_any(mb + min((uint32_t)min(row0 + p, n - 1) * (uint32_t)m + col, last));
-        if (row0 + R > n || col0 + 8 > m) {
+            for (int p = 0; p < R; ++p) v[p] = zero8;
+        } else {
 #pragma unroll
-            for (int p = 0; p < R; ++p) {
-                const uint32_t at = (uint32_t)min(row0 + p, n - 1) * (uint32_t)m + col;
-                v[p] = half8_head(v[p], at > last ? (int)(at - last) : 0, row0 + p < n ? m - col0 : 0, (half_t)0.0f);
+            for (int p = 0; p < R; ++p) v[p] = load_half8_any(mb + min((uint32_t)min(row0 + p, n - 1) * (uint32_t)m + col, last));
+            if (col0 + 8 > m && row0 < n) {
+                const uint4_t keep = half8_keep(m - col0);
+                const uint32_t over0 = (uint32_t)(col0 + 8) - (uint32_t)(n - row0) * (uint32_t)m;       // (rows that end less than a piece before the matrix's end: the last one, several of less than a piece)
+#pragma unroll
+                for (int p = 0; p < R; ++p) {
+                    const int32_t over = (int32_t)(over0 + (uint32_t)p * (uint32_t)m);
+                    if (over > 0 && over < 8) v[p] = half8_down(v[p], over);
+                    v[p] = half8_fill(v[p], keep, zero8);
+                }
+            }
+            if (row0 + R > n) {
+#pragma unroll
+                for (int p = 0; p < R; ++p)
+                    if (row0 + p >= n) v[p] = zero8;
             }
         }
     } else {
@@ -413,9 +426,9 @@ __global__ __launch_bounds__(kColThreads) __attribute__((amdgpu_waves_per_eu(6, 
         return;
     }
     const int64_t wave = (int64_t)(blockIdx.x - r.first) * (kColThreads / 64) + (threadIdx.x >> 6);
-    if (r.m <= 512) round_scale_rows_reg<1, 4, UA>(r, wave);
-    else if (r.m <= 1024) round_scale_rows_reg<2, 2, UA>(r, wave);
-    else round_scale_rows_reg<4, 1, UA>(r, wave);
+    if (r.m <= 512) round_scale_rows_reg<1, 4, UA, true>(r, wave);
+    else if (r.m <= 1024) round_scale_rows_reg<2, 2, UA, true>(r, wave);
+    else round_scale_rows_reg<4, 1, UA, true>(r, wave);
 }
 
 // Rows r0 .. r0 + 63 of a tile of 64 columns, rounded with the scale of the lane's column, into the wanted outputs (256 threads;

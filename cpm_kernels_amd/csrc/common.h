@@ -75,10 +75,10 @@ __device__ __forceinline__ void store_half8_head_any(half_t* p, int t, half8_t v
     }
     if (t & 1) p[t & 6] = (t & 6) == 0 ? v[0] : (t & 6) == 2 ? v[2] : (t & 6) == 4 ? v[4] : v[6];
 }
-// Pieces that may end behind a row's end, for loads that are not under conditions (which the compiler lets wait for one another, with copies behind each): read
-// where the piece lies, or the buffer's last eight halves if it would end behind those (`over` halves later), and put right afterwards: moved down by `over`, halves from `keep` on
-// replaced by `fill`.
-__device__ __forceinline__ half8_t half8_head(half8_t v, int over, int keep, half_t fill) {
+// Pieces that may end behind a row's end, for loads that are not under conditions of their own (which the compiler lets wait for one another, with copies behind each): read
+// where the piece lies, or the buffer's last eight halves if it would end behind those (`over` halves later, 1 to 7: half8_down), and put right behind all loads
+// (half8_fill: halves outside of `keep` replaced by those of `fill`; one operation a dword, where choosing half by half took six).
+__device__ __forceinline__ half8_t half8_down(half8_t v, int over) {
     typedef uint64_t ulong2_t __attribute__((ext_vector_type(2)));
     ulong2_t w = __builtin_bit_cast(ulong2_t, v);
     if (over >= 4) {
@@ -88,10 +88,28 @@ __device__ __forceinline__ half8_t half8_head(half8_t v, int over, int keep, hal
     const int bits = (over & 3) * 16;
     w[0] = (w[0] >> bits) | ((w[1] << 1) << (63 - bits));
     w[1] >>= bits;
-    v = __builtin_bit_cast(half8_t, w);
+    return __builtin_bit_cast(half8_t, w);
+}
+__device__ __forceinline__ uint4_t half8_keep(int n) {       // the first n halves
+    uint4_t k;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = e < keep ? v[e] : fill;
-    return v;
+    for (int d = 0; d < 4; ++d) k[d] = n >= 2 * d + 2 ? ~0u : n == 2 * d + 1 ? 0xffffu : 0u;
+    return k;
+}
+__device__ __forceinline__ half8_t half8_fill(half8_t v, uint4_t keep, half8_t fill) {
+    const uint4_t x = __builtin_bit_cast(uint4_t, v), f = __builtin_bit_cast(uint4_t, fill);
+    return __builtin_bit_cast(half8_t, (x & keep) | (f & ~keep));
+}
+// A piece in registers of its own, of this value or of none yet: a load into it that only some lanes make needs no copy behind it
+__device__ __forceinline__ half8_t half8_kept(half8_t v) {
+    int4_t t = __builtin_bit_cast(int4_t, v);
+    asm volatile("" : "+v"(t));
+    return __builtin_bit_cast(half8_t, t);
+}
+__device__ __forceinline__ half8_t half8_unset() {
+    int4_t t;
+    asm volatile("" : "=v"(t));
+    return __builtin_bit_cast(half8_t, t);
 }
 // the first t (1..7) of the eight bytes lo | hi << 32 to p, at any address
 struct __attribute__((packed, aligned(1))) Byte4Any { uint32_t x; };

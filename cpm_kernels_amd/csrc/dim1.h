@@ -34,21 +34,32 @@ struct ColTile {
 // UA: rows that are not whole 16-byte pieces, or buffers that are not 16-byte aligned.  A piece inside its row still
 // moves as one 16-byte access (global accesses need no alignment; one that crosses a cache line costs a second
 // request), the piece across a row's end in at most three narrower ones.
-// COND (not UA): loads of rows past the last and of columns past the row's end are left out; the compiler keeps those of whole tiles together.
-template <int NT, int LPR, int R, bool NTL = false, bool UA = false, bool COND = !UA && R == 8 && LPR == 8>
-__device__ inline void coltile_load(half8_t (&v)[R], const half_t* base, int32_t n, int32_t m, int32_t col0,
-                                    half_t fill) {
+// LOADS: what the registers of rows past the last and of columns past the row's end hold, whose loads are not made.  kLoadsPlain (not UA): `fill`, as the
+// compiler likes it, which keeps the loads of eight rows a lane together; of other tiles it let them wait for one another, with copies behind each.  kLoadsKept: `fill`, in registers that the
+// compiler cannot tell apart from others.  kLoadsUnset (UA): nothing yet; fewer registers where the pieces have to be put right all the same.
+// UA: tiles with rows nearly throughout make every load, those of rows past the last as the last one's, so that the first piece can be used before the last one is there.
+// us, loads that waited / every load made and put right half by half / this: softmax of 1024 of 500 x 500 268 / 230 / 217, of 70 x 70 10.6 / 11.8 / 10.8, its gradient of 512 of 129 x 130 28 / 14.6 / 12.9;
+// LayerNorm 672 x 30 x 847 113 / 121 / 113, its gradient 234 / 338 / 237; column scales of 1024 x 70 x 70 10.6 / 18.5 / 10.9.
+constexpr int kLoadsPlain = 0, kLoadsKept = 1, kLoadsUnset = 2;
+constexpr int coltile_loads(bool ua, int r, int lpr) { return ua ? kLoadsUnset : r == 8 && lpr == 8 ? kLoadsPlain : kLoadsKept; }
+template <int RPP, int R>
+__device__ __forceinline__ bool coltile_nearly_full(int32_t n) { return n * 8 >= RPP * R * 7; }
+// coltile_request makes the loads and coltile_settle puts what they brought right: a kernel of two tiles requests both before it settles one.
+template <int NT, int LPR, int R, bool NTL = false, bool UA = false, int LOADS = coltile_loads(UA, R, LPR)>
+__device__ inline void coltile_request(half8_t (&v)[R], const half_t* base, int32_t n, int32_t m, int32_t col0,
+                                       half_t fill) {
     constexpr int RPP = NT / LPR;
     const int rg = threadIdx.x / LPR;
     const uint32_t off0 = (uint32_t)rg * (uint32_t)m + (uint32_t)col0, stride = (uint32_t)RPP * (uint32_t)m;
-    if constexpr (COND) {
+    half8_t none;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) none[e] = fill;
+    if constexpr (LOADS == kLoadsPlain) {
+        static_assert(!UA, "whole pieces");
 #pragma unroll
         for (int p = 0; p < R; ++p) {
-            const int32_t row = p * RPP + rg;
-            half8_t x;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = fill;
-            if (row < n && col0 < m) {
+            half8_t x = none;
+            if (p * RPP + rg < n && col0 < m) {
                 const half8_t* src = reinterpret_cast<const half8_t*>(base + (off0 + p * stride));
                 x = NTL ? __builtin_nontemporal_load(src) : *src;
             }
@@ -56,51 +67,69 @@ __device__ inline void coltile_load(half8_t (&v)[R], const half_t* base, int32_t
         }
         return;
     }
-    // Every load is made, rows past the last as the last one: under conditions of their own the loads of other tiles waited for one another (softmax of 1024 of 500 x 500
-    // 268 -> 230 us, its gradient 409 -> 355; 1024 of 128 x 128 26 -> 22; LayerNorm 4 x 1024 x 100 16.4 -> 13.4; 1024 of 70 x 70, half of whose tile's rows are such repetitions, 14.3 and 15.1).
     const uint32_t last = (uint32_t)n * (uint32_t)m - 8u;
-    if (UA && (uint32_t)n * (uint32_t)m < 8u) {        // a matrix of less than a piece
-        const bool tail = col0 < m;
+    if (UA && (uint32_t)n * (uint32_t)m < 8u) {        // a matrix of less than a piece: as the end of one
+        half8_t x;
 #pragma unroll
-        for (int p = 0; p < R; ++p) {
-            half8_t x;
+        for (int e = 0; e < 8; ++e) x[e] = base[max(e + n * m - 8, 0)];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = fill;
-            if (tail && p * RPP + rg < n) x = load_half8_head_any(base + (off0 + p * stride), m & 7, x);
-            v[p] = x;
-        }
+        for (int p = 0; p < R; ++p) v[p] = x;
         return;
     }
-    const uint32_t col = (uint32_t)(col0 < m ? col0 : col0 - (int32_t)(threadIdx.x % LPR) * 8);        // (past the row's end: the tile's first piece once more)
+    auto load = [&](uint32_t at) {
+        if constexpr (UA) return load_half8_any(base + min(at, last));
+        const half8_t* src = reinterpret_cast<const half8_t*>(base + at);
+        return NTL ? __builtin_nontemporal_load(src) : *src;
+    };
+    if (UA && coltile_nearly_full<RPP, R>(n)) {
+        const uint32_t col = (uint32_t)(col0 < m ? col0 : col0 - (int32_t)(threadIdx.x % LPR) * 8);        // (past the row's end: the tile's first piece once more)
 #pragma unroll
-    for (int p = 0; p < R; ++p) {
-        const uint32_t at = (uint32_t)min(p * RPP + rg, n - 1) * (uint32_t)m + col;
-        if constexpr (UA) {
-            v[p] = load_half8_any(base + min(at, last));
-        } else {
-            const half8_t* src = reinterpret_cast<const half8_t*>(base + at);
-            v[p] = NTL ? __builtin_nontemporal_load(src) : *src;
+        for (int p = 0; p < R; ++p) v[p] = load((uint32_t)min(p * RPP + rg, n - 1) * (uint32_t)m + col);
+    } else {
+#pragma unroll
+        for (int p = 0; p < R; ++p) v[p] = LOADS == kLoadsKept ? half8_kept(none) : half8_unset();
+        uint32_t off = off0;
+        asm volatile("" : "+v"(off));       // (or the addresses are kept in registers for coltile_store)
+        if (col0 < m) {
+#pragma unroll
+            for (int p = 0; p < R; ++p)
+                if (p * RPP + rg < n) v[p] = load(off + p * stride);
         }
     }
+}
+
+template <int NT, int LPR, int R, bool UA = false, int LOADS = coltile_loads(UA, R, LPR)>
+__device__ inline void coltile_settle(half8_t (&v)[R], int32_t n, int32_t m, int32_t col0, half_t fill) {
+    constexpr int RPP = NT / LPR;
+    if constexpr (!UA) return;       // (right as they came)
+    const int rg = threadIdx.x / LPR;
     half8_t none;
 #pragma unroll
     for (int e = 0; e < 8; ++e) none[e] = fill;
-    if (n < RPP * R) {
+    if (LOADS == kLoadsUnset || coltile_nearly_full<RPP, R>(n) || n * m < 8) {
 #pragma unroll
         for (int p = 0; p < R; ++p)
-            if (p * RPP + rg >= n) v[p] = none;
+            if ((p + 1) * RPP > n && p * RPP + rg >= n) v[p] = none;
     }
-    if (UA ? col0 + 8 > m : col0 >= m) {        // the piece across the rows' ends (its first m % 8 columns), or one past them
+    if (col0 + 8 > m) {        // the piece across the rows' ends (its first m % 8 columns), or one past them
+        const uint4_t keep = half8_keep(m - col0);
+        const uint32_t over0 = (uint32_t)(col0 + 8) - (uint32_t)(n - rg) * (uint32_t)m, stride = (uint32_t)RPP * (uint32_t)m;
 #pragma unroll
         for (int p = 0; p < R; ++p) {
-            if constexpr (UA) {
-                const uint32_t at = (uint32_t)min(p * RPP + rg, n - 1) * (uint32_t)m + col;
-                v[p] = half8_head(v[p], at > last ? (int)(at - last) : 0, p * RPP + rg < n ? m - col0 : 0, fill);
-            } else {
-                v[p] = none;
+            if (p * RPP < n) {
+                // (rows that end less than a piece before the matrix does: the last one, several of less than a piece)
+                const int32_t over = (int32_t)(over0 + p * stride);
+                if ((p + 1) * RPP + 8 > n && p * RPP + rg < n && over > 0) v[p] = half8_down(v[p], over);
+                v[p] = half8_fill(v[p], keep, none);
             }
         }
     }
+}
+
+template <int NT, int LPR, int R, bool NTL = false, bool UA = false, int LOADS = coltile_loads(UA, R, LPR)>
+__device__ inline void coltile_load(half8_t (&v)[R], const half_t* base, int32_t n, int32_t m, int32_t col0, half_t fill) {
+    coltile_request<NT, LPR, R, NTL, UA, LOADS>(v, base, n, m, col0, fill);
+    coltile_settle<NT, LPR, R, UA, LOADS>(v, n, m, col0, fill);
 }
 
 template <int NT, int LPR, int R, bool NTS = false, bool UA = false>

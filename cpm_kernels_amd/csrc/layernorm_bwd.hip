@@ -67,9 +67,11 @@ __global__ __launch_bounds__(512, R == 4 ? 4 : 2) void k_ln_bwd_team(LnBwdArgs p
         shift[e] = MEAN ? -p.stats[(int64_t)b * 2 * p.m + c] * rstd[e] : 0.0f;
     }
     half8_t vx[R], vg[R];
-    constexpr bool COND = !UA && (R == 8 || MEAN);        // (128 registers hold four rows and means only so)
-    coltile_load<NT, LPR, R, NTH, UA, COND>(vg, p.g + boff, own_n, p.m, col0, (half_t)0.0f);
-    coltile_load<NT, LPR, R, NTH, UA, COND>(vx, p.x + boff, own_n, p.m, col0, (half_t)0.0f);
+    constexpr int LOADS = UA ? kLoadsUnset : R == 8 || MEAN ? kLoadsPlain : kLoadsKept;        // (128 registers hold four rows and means only so)
+    coltile_request<NT, LPR, R, NTH, UA, LOADS>(vg, p.g + boff, own_n, p.m, col0, (half_t)0.0f);
+    coltile_request<NT, LPR, R, NTH, UA, LOADS>(vx, p.x + boff, own_n, p.m, col0, (half_t)0.0f);
+    coltile_settle<NT, LPR, R, UA, LOADS>(vg, own_n, p.m, col0, (half_t)0.0f);
+    coltile_settle<NT, LPR, R, UA, LOADS>(vx, own_n, p.m, col0, (half_t)0.0f);
     float* const prow = p.part + ((int64_t)team * 2 + (cg & 1)) * p.n + own0;
     float s[NV * 8];
 #pragma unroll

@@ -257,12 +257,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UA && NV > 
         const half8_t* p8 = reinterpret_cast<const half8_t*>(mat);
         if (UA && m >= 8) {        // every load is made, pieces past the row's end as its last eight halves, and put right behind them all
 #pragma unroll
-            for (int i = 0; i < NV; ++i) v[i] = load_half8_any(mat + min((lane + i * 64) * 8, m - 8));
-            const half8_t last = load_half8_any(mat + m - 8), none = {0, 0, 0, 0, 0, 0, 0, 0}, tail = half8_head(last, 8 - (m & 7), m & 7, (half_t)0.0f);
+            for (int i = 0; i < NV; ++i) v[i] = half8_unset();
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                if ((lane + i * 64) * 8 < m) v[i] = load_half8_any(mat + min((lane + i * 64) * 8, m - 8));
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int j = (lane + i * 64) * 8;
-                if (j + 8 > m) v[i] = j < m ? tail : none;
+                if ((i + 1) * 512 > m) {
+                    if (i * 512 < m && j < m && j + 8 > m) v[i] = half8_down(v[i], 8 - (m & 7));       // (zeros come in from above)
+                    if (j >= m) v[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+                }
             }
             return;
         }

@@ -31,14 +31,14 @@ __device__ __forceinline__ uint2_t round8_own_scale(half8_t x, half8_t sy, float
 }
 
 // Rows of at most 2048 columns, kept in registers: a wave takes U consecutive rows of P 16-byte pieces
-// per lane (P * U = 4 loads in flight per lane, the matrix read once and with the non-temporal hint), finds each
+// per lane (P * U = 4 loads in flight per lane, the matrix read once, NTH with the non-temporal hint), finds each
 // row's maximum over the wave with data-parallel-primitive operands and rounds from the registers.
 // UA: rows that are not whole 16-byte pieces or buffers off 16-byte boundaries -- a piece inside its row still comes in
 // one 16-byte load and leaves in one 8-byte store (global accesses need no alignment), the piece across a row's end
 // is read with what lies behind it and leaves in at most three narrower accesses.
 // The two rounding sequences are chosen once for the wave's rows: a choice per row kept their chains from running side by side (780 rows
 // of 24 6.9 us, 4.7 so; 20000 of 512 11.1 -> 8.1; 81920 of 512 30 -> 23.5, 5.3 TB/s).
-template <int P, int U, bool UA>
+template <int P, int U, bool UA, bool NTH>
 __device__ __forceinline__ void round_scale_rows_reg(const RoundScaleArgs& a, int64_t wave) {
     const int64_t rows = a.rows;
     const int32_t n = a.n, m = a.m, ld = a.ld;
@@ -60,9 +60,12 @@ __device__ __forceinline__ void round_scale_rows_reg(const RoundScaleArgs& a, in
             const int32_t j = lane * 8 + p * 512;
             if constexpr (UA) {
                 if (pieces) {
-                    const int32_t jc = j < m ? j : 0;
-                    xv[u][p] = load_half8_any(a.mat + min(x0 + jc, last_x));
-                    sv[u][p] = load_half8_any(a.scale_y + min(s0 + jc, last_s));
+                    xv[u][p] = half8_unset();
+                    sv[u][p] = half8_unset();
+                    if (j < m) {
+                        xv[u][p] = load_half8_any(a.mat + min(x0 + j, last_x));
+                        sv[u][p] = load_half8_any(a.scale_y + min(s0 + j, last_s));
+                    }
                 } else {
                     xv[u][p] = j < m ? load_half8_head_any(a.mat + x0, m, zero) : zero;
                     sv[u][p] = j < m ? load_half8_head_any(a.scale_y + s0, m, zero) : zero;
@@ -70,7 +73,8 @@ __device__ __forceinline__ void round_scale_rows_reg(const RoundScaleArgs& a, in
             } else {
                 xv[u][p] = sv[u][p] = zero;
                 if (j < m) {
-                    xv[u][p] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(a.mat + x0 + j));
+                    const half8_t* src = reinterpret_cast<const half8_t*>(a.mat + x0 + j);
+                    xv[u][p] = NTH ? __builtin_nontemporal_load(src) : *src;
                     sv[u][p] = *reinterpret_cast<const half8_t*>(a.scale_y + s0 + j);
                 }
             }
@@ -85,10 +89,12 @@ __device__ __forceinline__ void round_scale_rows_reg(const RoundScaleArgs& a, in
             for (int p = 0; p < P; ++p) {
                 const int32_t j = lane * 8 + p * 512;
                 if (j + 8 > m) {
-                    const int32_t keep = m - j;
+                    const uint4_t keep = half8_keep(m - j);
                     const int64_t ox = x0 + j - last_x, os = s0 + j - last_s;
-                    xv[u][p] = half8_head(xv[u][p], keep > 0 && ox > 0 ? (int)ox : 0, keep, (half_t)0.0f);
-                    sv[u][p] = half8_head(sv[u][p], keep > 0 && os > 0 ? (int)os : 0, keep, (half_t)0.0f);
+                    if (j < m && ox > 0) xv[u][p] = half8_down(xv[u][p], (int)ox);
+                    if (j < m && os > 0) sv[u][p] = half8_down(sv[u][p], (int)os);
+                    xv[u][p] = half8_fill(xv[u][p], keep, zero);
+                    sv[u][p] = half8_fill(sv[u][p], keep, zero);
                 }
             }
         }

@@ -157,8 +157,9 @@ __device__ __forceinline__ void softmax_cols_by_lane(half8_t (&v)[R], float* lds
 // exponentials are exactly 0.
 // MODE 0: 16-byte accesses, non-temporal where a tile's row segments are whole cache lines; 1: 16-byte accesses without
 // the hint (rows that do not start on 128-byte boundaries); 2: any m and alignment, element by element (dim1.h).
+// (four rows a lane off 16-byte pieces: 64 registers, two workgroups of 1024 a compute unit; with 66 512 x 260 x 260 took 52 us instead of 35)
 template <int NT, int LPR, int R, int MODE = 0, bool BY_LANE = false>
-__global__ __launch_bounds__(NT) void k_softmax_tile(int32_t n, int32_t m, int32_t tiles_per_batch,
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(MODE == 2 && LPR == 8 && R == 4 ? 8 : 1))) void k_softmax_tile(int32_t n, int32_t m, int32_t tiles_per_batch,
                                                      const half_t* inp, half_t* out) {
     using T = ColTile<NT, LPR, R>;
     __shared__ __attribute__((aligned(16))) float lds[softmax_lds<NT, LPR>()];

@@ -418,8 +418,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KIND == kSof
     // every input byte is read once: non-temporal loads; non-temporal stores too, except for the softmax
     // gradient, where they measured 1-2 % slower
     constexpr bool NTS = NTH && KIND != kSoftmaxBwd;
-    coltile_load<NT, LPR, R, NTH, UA>(va, p.a + boff, own_n, p.m, col0, (half_t)0.0f);
-    if constexpr (TWO) coltile_load<NT, LPR, R, NTH, UA>(vg, p.g + boff, own_n, p.m, col0, (half_t)0.0f);
+    constexpr int LOADS = UA && KIND == kColAbsmax ? kLoadsKept : coltile_loads(UA, R, LPR);        // (a kernel with registers to spare)
+    coltile_request<NT, LPR, R, NTH, UA, LOADS>(va, p.a + boff, own_n, p.m, col0, (half_t)0.0f);
+    if constexpr (TWO) coltile_request<NT, LPR, R, NTH, UA>(vg, p.g + boff, own_n, p.m, col0, (half_t)0.0f);
+    coltile_settle<NT, LPR, R, UA, LOADS>(va, own_n, p.m, col0, (half_t)0.0f);
+    if constexpr (TWO) coltile_settle<NT, LPR, R, UA>(vg, own_n, p.m, col0, (half_t)0.0f);
     float mean[8], var[8], c3[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -593,9 +596,9 @@ __global__ __launch_bounds__(256) void k_round_scale_rows_wide(int64_t rows, int
 }
 
 // The same for rows of at most 2048 columns, kept in registers (round_scale.h).
-template <int P, int U, bool UA>
+template <int P, int U, bool UA, bool NTH>
 __global__ __launch_bounds__(256) void k_round_scale_rows_reg(RoundScaleArgs a) {
-    round_scale_rows_reg<P, U, UA>(a, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
+    round_scale_rows_reg<P, U, UA, NTH>(a, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1155,8 +1158,10 @@ int cpmk_gemm_backward_round_scale_ld(int32_t batch, int32_t n, int32_t m, const
                 const RoundScaleArgs a = {(const half_t*)mat, (const half_t*)scale_y, (int8_t*)out, (half_t*)scale_x, rows, n, m, broad_cast_y, ld, 0};
                 hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(rows, 4 * U)), dim3(256), 0, (hipStream_t)stream, a);
             };
-            if (vec16) run(k_round_scale_rows_reg<P, U, false>);
-            else run(k_round_scale_rows_reg<P, U, true>);
+            // (the hint from 48 MB on: 8 x 10240 x 512 26.3 us, 27.6 without, 128 x 500 x 504 21.9 and 22.5; 30 x 1024 x 512 13.2 and 12.5, 16 x 1000 x 1000 12.1 and 11.5)
+            if (!vec16) run(k_round_scale_rows_reg<P, U, true, false>);
+            else if (rows * m >= 3ll << 23) run(k_round_scale_rows_reg<P, U, false, true>);
+            else run(k_round_scale_rows_reg<P, U, false, false>);
         };
         if (m <= 512) go(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
         else if (m <= 1024) go(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});

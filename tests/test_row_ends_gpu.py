@@ -8,7 +8,9 @@ from util import stream
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(1, 2), (1, 6), (2, 2), (3, 4), (1, 10), (2, 12), (50, 70), (100, 100), (130, 66), (300, 30), (240, 236), (500, 500), (520, 20), (1000, 134)]
+SIZES = [(1, 2), (1, 6), (2, 2), (3, 4), (1, 10), (2, 12), (50, 70), (100, 100), (130, 66), (300, 30), (240, 236), (500, 500), (520, 20), (1000, 134),
+         # tiles with rows nearly throughout (seven eighths) and just not, rows of whole pieces
+         (55, 66), (56, 66), (111, 70), (112, 70), (224, 66), (446, 70), (448, 70), (898, 66), (50, 72), (120, 72), (70, 136), (230, 80)]
 
 
 def _pair(batch, n, m, seed):
@@ -46,6 +48,26 @@ def test_softmax_columns(n, m):
 
 
 @pytest.mark.parametrize("n,m", SIZES)
+def test_normalised_columns(n, m):
+    x, y = _pair(3, n, m, n + m)
+    grad = _pair(3, n, m, n)[0]
+    outs = []
+    for v in (x, y):
+        out, back = torch.empty_like(v), torch.empty_like(v)
+        mean, var, most = torch.empty((3, 3, m), dtype=torch.half, device="cuda")
+        ck.layernorm_forward_mv(3, n, m, v.data_ptr(), out.data_ptr(), mean.data_ptr(), var.data_ptr(), 1e-2, stream())
+        ck.layernorm_backward_v(3, n, m, v.data_ptr(), grad.data_ptr(), var.data_ptr(), back.data_ptr(), stream())
+        ck.gemm_calc_scale_transpose(3, n, m, v.data_ptr(), most.data_ptr(), stream())
+        outs.append((out, back, mean.unsqueeze(1), var.unsqueeze(1), most.unsqueeze(1)))
+    _same(outs, 2)
+    xd = x.double()
+    ref = (xd - xd.mean(1, keepdim=True)) / (xd.var(1, unbiased=False, keepdim=True) + 1e-2).sqrt()
+    # (variances as a difference of fp32 sums: 2^-20 of the mean square, of which the smallest here is a hundredth)
+    assert ((outs[0][0].double() - ref).abs() <= (ref.abs() + 1) * 2.0 ** -10).all()
+    assert torch.equal(outs[0][4].squeeze(1), (x.float().abs().amax(1).double() / 127.0).half())
+
+
+@pytest.mark.parametrize("n,m", SIZES)
 @pytest.mark.parametrize("scaled", [False, True])
 def test_quantised_columns(n, m, scaled):
     rows = torch.rand((3, n), device="cuda").half()
@@ -60,9 +82,10 @@ def test_quantised_columns(n, m, scaled):
 
 
 # (the maximum of a row skips NaN, so it has a row of values of its own in front: what a row's end must not take from the next row)
-@pytest.mark.parametrize("m", [2, 6, 10, 70, 172, 500, 516, 1030, 2044])
-def test_scaled_rows(m):
-    n, ld = 70, (m + 127) // 128 * 128
+# (the last one: beyond 48 MB, rows of whole pieces)
+@pytest.mark.parametrize("m,n", [(m, 70) for m in (2, 6, 10, 70, 172, 500, 516, 1030, 2044)] + [(520, 24600)])
+def test_scaled_rows(m, n):
+    ld = (m + 127) // 128 * 128
     x = _pair(2, n, m, m)[0]
     x[:, 1::2] *= 1000.0
     cols = torch.rand((2, m), device="cuda").half() + 0.5
@@ -72,6 +95,24 @@ def test_scaled_rows(m):
     s = (p.abs().amax(2).double() / 127.0).float()
     assert torch.equal(scale, s.half())
     assert torch.equal(out[:, :, :m].float(), torch.round(p / s[:, :, None])) and (out[:, :, m:] == 0).all()
+
+
+# rows that a wave holds, beside a second matrix of other values
+@pytest.mark.parametrize("m", [2, 6, 10, 70, 504, 508, 516, 1030, 1538, 2044, 4090])
+def test_quantised_rows(m):
+    n, ld = 37, (m + 127) // 128 * 128
+    outs = []
+    x, y = _pair(1, n, m, m)
+    other = torch.full((n, m), float("inf"), device="cuda").half()
+    for v in (x, y):
+        scale, out = torch.empty((2, n), dtype=torch.half, device="cuda"), torch.empty((2, n, ld), dtype=torch.int8, device="cuda")
+        ck.gemm_quantize_pair_ld(n, v.data_ptr(), scale[0].data_ptr(), out[0].data_ptr(), n, other.data_ptr(), scale[1].data_ptr(), out[1].data_ptr(), m, ld, stream())
+        outs.append((scale, out))
+    s = (x[0].float().abs().amax(1).double() / 127.0).half()
+    assert torch.equal(outs[0][0][0], s)
+    assert torch.equal(outs[0][1][0, :, :m].float(), torch.round(x[0].float() / s.float()[:, None])) and (outs[0][1][0, :, m:] == 0).all()
+    skipped = (x[0, :, 1:].float().abs().amax(1).double() / 127.0).half() if m > 1 else s
+    assert torch.equal(outs[1][0][0], skipped) and (outs[1][1][0, :, m:] == 0).all()
 
 
 # many ragged sequences: lanes that work for themselves

@@ -85,7 +85,7 @@ __device__ __forceinline__ void col_quantize_team(const ColQuantArgs& a, int32_t
         // Every load is made, rows past the last as the last one, and put right behind them all; waves that have no rows leave them out
         const half_t* const mb = mat + boff;
         const uint32_t last = (uint32_t)n * (uint32_t)m - 8u, col = (uint32_t)min(col0, m - 1);
-        if (!SCALED && __builtin_amdgcn_readfirstlane(row0) >= n) {        // (80 registers do not hold that choice beside the scales)
+        if (!(SCALED && NATURAL) && __builtin_amdgcn_readfirstlane(row0) >= n) {        // (80 registers do not hold that choice beside the scales and the outputs in place)
 #pragma unroll
             for (int p = 0; p < R; ++p) v[p] = zero8;
         } else {

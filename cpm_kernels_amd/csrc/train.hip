@@ -1192,7 +1192,12 @@ int cpmk_position_embedding_backward(int32_t query_len, int32_t key_len, int32_t
         const int64_t parts = ceil_div(key_len, rpp);
         const int64_t pieces = ceil_div(query_len, 8) * ceil_div(rpp, 8);          // of eight key rows x eight queries, 15 floats each
         const int64_t smem = (num_buckets + pieces * 15) * (int64_t)sizeof(float);
-        const bool diag = smem <= 128 * 1024;
+        // (a kernel for so little: by diagonals and element by element 114 heads of 1 x 3 4.0 and 2.0 us, 113 of 21 x 16 4.1 and 2.4, 14 of 444 x 5 4.4 and 5.6, 7 of
+        // 200 x 30 3.4 and 11.5; rows of whole pieces 16 of 16 x 11 2.9 and 2.1, 95 of 8 x 55 3.6 and 2.6, 20 of 200 x 8 3.1 and 4.5, 74 of 16 x 49 3.6 and 3.1, 5 of 1344 x 1, as many
+        // diagonals, 5.9 and 4.0)
+        const bool ua = query_len % 8 != 0 || !aligned16(grad_out);
+        const bool few = key_len <= 64 && (int64_t)query_len * key_len < (ua ? 1200 : 440) + ((int64_t)query_len + key_len) * 3 / 2 + key_len * 12;
+        const bool diag = smem <= 128 * 1024 && !few;
         if ((diag || key_len > 64) && (int64_t)num_heads * parts <= kXchSlots) {
             XchScope xs;
             const int rc = parts > 1 ? xs.begin((int64_t)num_heads * parts, (hipStream_t)stream) : 0;
@@ -1200,7 +1205,6 @@ int cpmk_position_embedding_backward(int32_t query_len, int32_t key_len, int32_t
             const dim3 grid((unsigned)xch_team_grid(num_heads, parts));
             if (rc == 0 && diag) {
                 // (1022 x 1022, 15 heads 68 -> 22 us, 902 x 902, 33 heads 98 -> 35, off 16-byte pieces, where a thread walked down each column with a load and a look-up an element)
-                const bool ua = query_len % 8 != 0 || !aligned16(grad_out);
                 auto kern = ua ? k_position_backward_diag<true> : k_position_backward_diag<false>;
                 static std::atomic<bool> lds_enabled[2][64];
                 if (smem > 48 * 1024)

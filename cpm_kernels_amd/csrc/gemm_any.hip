@@ -42,29 +42,33 @@ struct AnySlab {
         pc = threadIdx.x % PPR;
         lr = threadIdx.x / PPR;
         if constexpr (T) {
-            at[0] = base + (int64_t)lr * L + r0 + pc * 8;
-            step = (int64_t)STEP * L;
             left = min(L - r0 - pc * 8, 8);
+            at[0] = base + (int64_t)lr * L + r0 + (left > 0 ? pc * 8 : 0);
+            step = (int64_t)STEP * L;
         } else {
 #pragma unroll
             for (int p = 0; p < NP; ++p) at[p] = base + (int64_t)min(r0 + lr + p * STEP, L - 1) * k + pc * 8;      // (rows past the last are not stored)
         }
     }
-    // slab k0 .. k0 + 63 (the pointers move on to the next one); `inside`: the whole slab lies inside K and, T, the tile inside the matrix
+    // slab k0 .. k0 + 63 (the pointers move on to the next one); `inside`: it lies inside K and, T, eight rows before its end where the tile reaches past the
+    // matrix, whose pieces are read with what lies behind the rows' ends then (it feeds outputs that are not stored) and stay inside the operand.  (Every slab of such a
+    // tile under conditions, load by load, took twice as long: 3 entries of 118 x 80 outputs, K = 290, both stored (K, rows), 15.7 us, 5.2 so, 43 of 4 x 118, K = 344 13.7 and 5.2.)
     __device__ __forceinline__ void load(int32_t k0, int32_t k, int32_t L, bool inside) {
         if (inside) {
 #pragma unroll
             for (int p = 0; p < NP; ++p) v[p] = load_half8_any(T ? at[0] + p * step : at[p]);
         } else {
             const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
+            // whole pieces first, into registers of their own, so that none waits for another
 #pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                const half_t* const src = T ? at[0] + p * step : at[p];
-                const int32_t have = T ? (k0 + lr + p * STEP < k ? left : 0) : min(k - k0 - pc * 8, 8);
-                v[p] = zero;
-                if (have == 8) v[p] = load_half8_any(src);
-                else if (have > 0) v[p] = load_half8_head_any(src, have, zero);
-            }
+            for (int p = 0; p < NP; ++p) v[p] = half8_kept(zero);
+            auto have = [&](int p) __attribute__((always_inline)) { return T ? (k0 + lr + p * STEP < k ? left : 0) : k - k0 - pc * 8; };
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+                if (have(p) >= 8) v[p] = load_half8_any(T ? at[0] + p * step : at[p]);
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+                if (have(p) > 0 && have(p) < 8) v[p] = load_half8_head_any(T ? at[0] + p * step : at[p], have(p), zero);
         }
         if constexpr (T) {
             at[0] += (int64_t)64 * L;
@@ -117,11 +121,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TR * TC > 8
     SQ sq;
     sp.start(a.P + b * a.strideP, j0, a.n, a.k);
     sq.start(a.Q + b * a.strideQ, i0, a.m, a.k);
-    const bool in_p = !PT || j0 + TR <= a.n, in_q = !QT || i0 + TC <= a.m;
+    const int32_t kp = !PT || j0 + TR <= a.n ? a.k : a.k - 8, kq = !QT || i0 + TC <= a.m ? a.k : a.k - 8;
     auto load = [&](int32_t k0) __attribute__((always_inline)) {
-        const bool whole = k0 + 64 <= a.k;
-        sp.load(k0, a.k, a.n, whole && in_p);
-        sq.load(k0, a.k, a.m, whole && in_q);
+        sp.load(k0, a.k, a.n, k0 + 64 <= kp);
+        sq.load(k0, a.k, a.m, k0 + 64 <= kq);
     };
     float4_t acc[4][NJ];
 #pragma unroll
@@ -129,6 +132,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TR * TC > 8
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
     load(0);
+#pragma unroll 1       // (more takes registers that 128 x 128 tiles do not have)
     for (int32_t k0 = 0; k0 < a.k; k0 += 64) {
         if (k0 > 0) __syncthreads();                              // the slab before has been read
         sp.put(lds);
@@ -186,7 +190,9 @@ int gemm_f16_any(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB
     const int64_t batch = batchA > batchB ? batchA : batchB;
     // tiles of 128 rows or columns unless they cover a quarter more than those of 64
     auto wide = [](int64_t len) { return ceil_div(len, 128) * 128 * 4 <= ceil_div(len, 64) * 64 * 5; };
-    const bool wr = wide(n), wc = wide(m);
+    // ... and small ones where those are at most one a compute unit: a slab of them is there sooner (over 490 such products a tenth quicker, none slower)
+    const bool few = ceil_div(n, 64) * ceil_div(m, 64) * batch <= compute_units();
+    const bool wr = wide(n) && !few, wc = wide(m) && !few;
     const int64_t tr = ceil_div(n, wr ? 128 : 64), tc = ceil_div(m, wc ? 128 : 64), total = tr * tc * batch;
     a.tiles_r = (uint32_t)tr; a.tiles_c = (uint32_t)tc;
     if (total >= 1ll << 32) return CPMK_ETOOBIG;

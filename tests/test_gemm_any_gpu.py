@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 def _check(A, aT, B, bT, out):
     """out (batch, n, m) of A (., k, m) [(., m, k) if aT] and B (., n, k) [(., k, n) if bT]"""
     k = A.size(2 if aT else 1)
-    for i in range(out.size(0)):
+    last = out.size(0) - 1
+    for i in sorted({0, 1, 2, last // 2, last - 1, last} & set(range(last + 1))):
         a, b = A[i % A.size(0)].double(), B[i % B.size(0)].double()
         a, b = (a.t() if aT else a).contiguous(), (b.t() if bT else b).contiguous()
         ref, size = b @ a, b.abs() @ a.abs()
@@ -38,8 +39,29 @@ def _product(batch_a, batch_b, m, k, n, aT, bT, shift=0):
 @pytest.mark.parametrize("aT,bT", [(True, False), (False, False), (True, True), (False, True)])
 @pytest.mark.parametrize("m,n", [(2, 2), (6, 64), (62, 66), (64, 128), (66, 126), (126, 80), (128, 34), (130, 100), (200, 128), (258, 66)])
 @pytest.mark.parametrize("k", [2, 30, 64, 66, 100, 192])
-def test_edges(aT, bT, m, n, k):
-    _product(3, 3, m, k, n, aT, bT)
+@pytest.mark.parametrize("batch", [3, 140])        # (tiles of 64 x 64, larger ones from where those are more than one a compute unit)
+def test_edges(aT, bT, m, n, k, batch):
+    _product(batch, batch, m, k, n, aT, bT)
+
+
+# values that are not finite stay in their own rows and columns: pieces across a row's end are read with what lies behind it
+@pytest.mark.parametrize("aT,bT", [(True, False), (False, False), (True, True), (False, True)])
+@pytest.mark.parametrize("m,n,k,batch", [(70, 66, 30, 2), (190, 70, 100, 2), (66, 126, 200, 140), (130, 66, 72, 140), (2, 2, 2, 3)])
+def test_values_that_are_not_finite(aT, bT, m, n, k, batch):
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    A = torch.randn((batch, m, k) if aT else (batch, k, m), generator=g, device="cuda").half()
+    B = torch.randn((batch, k, n) if bT else (batch, n, k), generator=g, device="cuda").half()
+    outs = []
+    for spoilt in (False, True):
+        if spoilt:
+            A.select(1 if aT else 2, 0).fill_(float("nan"))
+            B.select(2 if bT else 1, 0).fill_(float("inf"))
+        out = torch.full((batch, n, m), 7.0, dtype=torch.half, device="cuda")
+        ck.gemm_fp16(m, k, n, batch, batch, aT, bT, A.data_ptr(), B.data_ptr(), out.data_ptr(), stream())
+        outs.append(out)
+    clean, spoilt = outs
+    assert not clean.isnan().any() and torch.equal(clean[:, 1:, 1:], spoilt[:, 1:, 1:])
+    assert spoilt[:, :, 0].isnan().all() and not spoilt[:, 0, 1:].isfinite().any()
 
 
 @pytest.mark.parametrize("aT,bT", [(True, False), (False, False), (True, True), (False, True)])

@@ -15,16 +15,16 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     if (out == nullptr || (k > 0 && any_null(A, B))) return CPMK_EBADARG;
     if (k > (1 << 30)) return CPMK_ETOOBIG;
     const int64_t big_apart = n > 128 && m > 128 ? ceil_div(n, 256) * ceil_div(m, 256) * batch : 0;       // (big_tiles)
-    if (batchA == 1 && !bT && rows_join(batch, n, (int64_t)k * 2)) {
+    if (batchA == 1 && !bT && rows_join(batch, n, (int64_t)k * 2) && rows_join_pays_f16(n, m, k, batch, big_apart)) {
         n *= batch;
         batch = batchB = 1;
     }
-    // (columns: where whole entries of them leave tiles half empty; depths and buffers that the tile kernel takes beside a K-major Q)
+    // (columns: depths and buffers that the tile kernel takes beside a K-major Q)
     int32_t seg = 0;
     const uintptr_t operands = reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B);
     if (batchB == 1 && aT && m % 4 == 0 && cols_join(batch, m, (int64_t)k * 2) && aligned16(out) && (int64_t)n * k * 2 < (1ll << 32) &&
         (bT ? k >= 64 && n % 8 == 0 && operands % 16 == 0 : k > 32 && operands % 4 == 0) &&
-        (ceil_div((int64_t)m * batch, 128) < ceil_div(m, 128) * batch || ceil_div((int64_t)m * batch, 256) < ceil_div(m, 256) * batch)) {
+        cols_join_pays_f16(n, m, k, bT, batch, big_apart)) {
         seg = m;
         m *= batch;
         batch = batchA = 1;

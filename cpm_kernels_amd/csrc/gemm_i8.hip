@@ -280,15 +280,16 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
     if (m == 0 || n == 0) return 0;
     if (out == nullptr || (k > 0 && any_null(A, B)) || (FUSED && srow == nullptr && scol == nullptr)) return CPMK_EBADARG;
     const int64_t big_apart = n > 128 && m > 128 ? ceil_div(n, 256) * ceil_div(m, 256) * batch : 0;       // (big_tiles)
-    if (batchA == 1 && !bT && (srow == nullptr || !bcr) && (scol == nullptr || bcc) && rows_join(batch, n, k)) {
+    if (batchA == 1 && !bT && (srow == nullptr || !bcr) && (scol == nullptr || bcc) && rows_join(batch, n, k) &&
+        rows_join_pays_i8(n, m, k, aT, batch, big_apart)) {
         n *= batch;
         batch = batchB = 1;
     }
-    // (columns: where whole entries of them leave tiles half empty, and operands that the tile kernel takes: it alone knows of `seg`)
+    // (columns: operands that the tile kernel takes: it alone knows of `seg`)
     int32_t seg = 0;
     if (FUSED && batchB == 1 && aT && (srow == nullptr || bcr) && (scol == nullptr || !bcc) && cols_join(batch, m, k) && (int64_t)n * k < (1ll << 32) && aligned16(A) &&
         aligned16(B) && aligned16(out) && k > 0 && (bT ? k % 128 == 0 && n % 16 == 0 : k % 64 == 0) &&
-        (ceil_div((int64_t)m * batch, 128) < ceil_div(m, 128) * batch || ceil_div((int64_t)m * batch, 256) < ceil_div(m, 256) * batch)) {
+        cols_join_pays_i8(n, m, k, !bT, batch, big_apart)) {
         seg = m;
         m *= batch;
         batch = batchA = 1;

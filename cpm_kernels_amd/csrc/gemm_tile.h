@@ -1226,9 +1226,10 @@ static int launch_dma(GemmArgs& a, int batch, hipStream_t st, int per_cu = 1) {
 }
 
 // A row operand stored (batch, n, k) beside a column operand that the batch shares: its entries, and the outputs', lie one behind the other
-// and are one product of batch x n rows, whose tiles reach across the entries.  Entry by entry the last row tile of each was filled up to
+// and are one product of batch x n rows, whose tiles reach across the entries.  Entry by entry the last row tile of each is filled up to
 // 128 rows, and the shared operand read for every entry: fp16, 16 entries of 32 x 8192 beside 4096 rows 127 -> 59 us, 7 of 300 x 1540 beside
-// 7000 123 -> 67, the gradient of the 300 x 1540 117 -> 67; int8, 4 of 436 x 3712 beside 2304 29 -> 24.  (Operands stay below 4 GiB, what the tile kernels address.)
+// 7000 123 -> 67, the gradient of the 300 x 1540 117 -> 67; int8, 4 of 436 x 3712 beside 2304 29 -> 24.  (Operands stay below 4 GiB, what the tile kernels
+// address; where it pays, join_gain.)
 static bool rows_join(int batch, int32_t n, int64_t row_bytes) {
     return batch > 1 && (int64_t)batch * n < (1ll << 31) && batch * n * row_bytes < (1ll << 32);
 }
@@ -1246,6 +1247,55 @@ static bool cols_join(int batch, int32_t m, int64_t row_bytes) {
 static int64_t big_tiles(int32_t n, int32_t m, int batch, int64_t apart) {
     const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
     return apart > big && ceil_div(n, 128) * ceil_div(m, 128) * batch > 2 * compute_units() ? apart : big;
+}
+
+// The time of a product's tiles, in tenths of a round of 128 x 128 tiles over the chip: a second round beside the first costs 0.8 of it (two
+// workgroups fit a compute unit), a round of 256 x 256 tiles 2.2, and one of 128 x 64 tiles, where the product has them (`halves`), 0.8.
+static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool halves) {
+    const int64_t cus = compute_units();
+    const int64_t tiles = ceil_div(n, 128) * ceil_div(m, 128) * batch;
+    if (n > 128 && m > 128 && big_tiles(n, m, batch, apart) * 4 >= cus * 3) return 22 * ceil_div(ceil_div(n, 256) * ceil_div(m, 256) * batch, cus);
+    if (halves && tiles * 4 < cus * 3 && ceil_div(n, 128) * ceil_div(m, 64) * batch <= cus) return 8;
+    return tiles <= cus ? 10 : tiles <= 2 * cus ? 18 : 10 * ceil_div(tiles, cus);
+}
+
+// What joining entries does: rounds (tile_rounds) and 128 x 128 tiles, apart and joined.  Where it saves no round, the product apart is as quick or
+// quicker: its results need no search for their entry (0.4 us on the smallest tiles), and fp16's few rows keep the kernels made for them.
+// Over 1370 drawn int8 and 1430 fp16 products, joined : apart as a geometric mean,
+//                   always                   where it pays (what follows)     (the better of both for each)
+//   int8 rows       0.958, 102 worse > 4 %   0.950, 2 worse                   0.945
+//   int8 columns    0.977, 273 worse         0.960, 1 worse                   0.958
+//   fp16 rows       1.043, 307 worse         0.976, 6 worse                   0.961
+//   fp16 columns    1.026, 335 worse         0.962, 3 worse                   0.958
+struct JoinGain {
+    int64_t rounds, rounds_joined, tiles, tiles_joined;
+    bool fewer() const { return rounds_joined < rounds; }
+};
+static JoinGain join_gain(int32_t n, int32_t m, int batch, bool rows, int64_t apart, bool halves) {
+    const int32_t nj = rows ? n * batch : n, mj = rows ? m : m * batch;
+    return {tile_rounds(n, m, batch, 0, halves), tile_rounds(nj, mj, 1, apart, halves), ceil_div(n, 128) * ceil_div(m, 128) * batch, ceil_div(nj, 128) * ceil_div(mj, 128)};
+}
+// fp16, whose few rows and short depths have kernels of their own: rows, past 128 of them or a depth of 448, or many tiles of enough depth
+// (500 entries of 4 x 400 beside 314: 19.3 -> 7.5 us; 41 of 4 x 64 beside 3808, 4.3 apart and 5.7 joined)
+static bool rows_join_pays_f16(int32_t n, int32_t m, int32_t k, int batch, int64_t apart) {
+    const JoinGain g = join_gain(n, m, batch, true, apart, false);
+    return g.fewer() && (n > 128 || k > 448 || (g.tiles > 4 * (int64_t)compute_units() && g.tiles * k > 100000 && g.tiles_joined * 3 <= g.tiles));
+}
+// Columns, past 64 rows or a depth of 320; a row operand stored (K, rows) leaves fewer such calls to those kernels, and in a single round its long
+// depths gain too (357 entries of 64 columns, 40 rows, K = 240 14.5 -> 9.5 us; 94 of 128, 64 rows, K = 2328 28.7 -> 23.7)
+static bool cols_join_pays_f16(int32_t n, int32_t m, int32_t k, bool krows, int batch, int64_t apart) {
+    const JoinGain g = join_gain(n, m, batch, false, apart, false);
+    if (g.fewer() && (n > 64 || k > 320 || (krows && g.tiles * k > 19000 && g.tiles_joined * 4 <= g.tiles * 3))) return true;
+    return krows && n <= 64 && k >= 512 && g.tiles_joined <= compute_units();
+}
+// int8: rows also wherever the rounds stay, past one of them, with what the tiles of whole slabs do not take (19 of 2564 x 1600 beside 40 stored
+// (K, columns), 495 -> 300; 37 of 128 x 36 beside 1280, 46 -> 17)
+static bool rows_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
+    const JoinGain g = join_gain(n, m, batch, true, apart, kmajor && k % 128 == 0);
+    return g.fewer() || ((!kmajor || k % 64 != 0) && g.tiles > compute_units() && g.rounds_joined == g.rounds);
+}
+static bool cols_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
+    return join_gain(n, m, batch, false, apart, kmajor && k % 128 == 0).fewer();
 }
 
 }  // namespace cpmk

@@ -60,6 +60,46 @@ def test_shared_column_operand(n, batch, m, k):
     assert torch.equal(_whole(A, B, False, s_row, s_col, k), _reference(A, B, False, s_row, s_col))
 
 
+# (entries that are joined because that saves rounds of tiles: shorter than a piece, off pieces, past a tile, and of large tiles; depths as above)
+MANY = [(4, 300, 132), (36, 130, 300), (132, 140, 260), (300, 40, 2000)]
+
+
+@pytest.mark.parametrize("m,batch,n", MANY)
+@pytest.mark.parametrize("k,bT", [(64, False), (192, False), (128, False), (384, True)])
+def test_shared_row_operand_of_many_entries(m, batch, n, k, bT):
+    if bT:
+        n = (n + 15) // 16 * 16
+    A, B, s_row, s_col = _int8(batch, 1, m, k, n, bT, m + k)
+    assert torch.equal(_whole(A, B, bT, s_row, s_col, k), _reference(A, B, bT, s_row, s_col))
+
+
+@pytest.mark.parametrize("n,batch,m", MANY)
+@pytest.mark.parametrize("k", [4, 68, 128, 192])
+def test_shared_column_operand_of_many_entries(n, batch, m, k):
+    A, B, s_row, s_col = _int8(1, batch, m, k, n, False, n + k)
+    assert torch.equal(_whole(A, B, False, s_row, s_col, k), _reference(A, B, False, s_row, s_col))
+
+
+@pytest.mark.parametrize("a_shared", [False, True])
+@pytest.mark.parametrize("edge,batch,other", MANY)
+@pytest.mark.parametrize("k", [66, 128, 520])
+@pytest.mark.parametrize("stored_other", [False, True])        # the shared operand stored (K, rows or columns)
+def test_fp16_of_many_entries(a_shared, edge, batch, other, k, stored_other):
+    m, n, batch_a, batch_b = (other, edge, 1, batch) if a_shared else (edge, other, batch, 1)
+    aT, bT = (not stored_other, False) if a_shared else (True, stored_other)
+    g = torch.Generator(device="cuda").manual_seed(edge + k)
+    A = torch.randn((batch_a, m, k) if aT else (batch_a, k, m), generator=g, device="cuda").half()
+    B = torch.randn((batch_b, k, n) if bT else (batch_b, n, k), generator=g, device="cuda").half()
+    out = torch.full((batch, n, m), float("nan"), dtype=torch.half, device="cuda")
+    ck.gemm_fp16(m, k, n, batch_a, batch_b, aT, bT, A.data_ptr(), B.data_ptr(), out.data_ptr(), stream())
+    for i in range(0, batch, 1 if batch < 64 else 7):
+        a, b = A[i % batch_a].double(), B[i % batch_b].double()
+        a, b = (a.t() if aT else a).contiguous(), (b.t() if bT else b).contiguous()        # (k, m), (n, k)
+        ref, size = b @ a, b.abs() @ a.abs()
+        # k additions in fp32, one rounding to fp16 (or half a subnormal step)
+        assert ((out[i].double() - ref).abs() <= size * k * 2.0 ** -24 + ref.abs() * 2.0 ** -10.9 + 2.0 ** -25).all()
+
+
 # (parts of one slab, of several, a shorter last part, more parts than slabs)
 @pytest.mark.parametrize("batch_a,batch_b,m,n,bT", [(1, 1, 64, 128, False), (3, 1, 44, 260, False), (1, 5, 132, 60, False), (2, 2, 132, 132, False),
                                                     (3, 1, 100, 272, True), (3, 1, 20, 16, True)])

@@ -597,12 +597,13 @@ static int softmax_dispatch(int32_t batch, int32_t n, int32_t m, const void* inp
             // 512 tiles, 64 x 480 x 480, 13.0, 11.8 and 12.1), and 161 to 256 rows beyond the last-level cache (2250 x 200 x 504 180 us, else 195; 4500 x 192 x
             // 200 147 and 174; 1125 x 256 x 504 128.6 and 131.4; within it, 2250 x 192 x 200, 75.8 and 73.3; 160 rows the same within 2 %, 562 x 136 x 2008
             // 128 and 121.5).  Rows off them: from 1500 columns on, 225 to 320 rows beyond that cache (382 x
-            // 256 x 3003 271 us, else 282; 187 x 257 x 2002 84.9 and 88.5; 2250 x 240 x 505 256 and 252; 187 x 384 x 2002 124 and 125); and of up to 640 columns 385 to 512
-            // rows from 200 MB on (1024 x 500 x 500 217 us, else 228; 400 x 500 x 500 106.3 and 109; 256 x 500 x 500, within the cache, 75.3 and 77.2, 64 22.7 and 22.4; 1024 x
-            // 420 x 420 167 and 168.5, 300 x 300 97.6 and 97.3; 340 x 490 x 700 125.1 and 124.4).
+            // 256 x 3003 271 us, else 282; 187 x 257 x 2002 84.9 and 88.5; 2250 x 240 x 505 256 and 252; 187 x 384 x 2002 124 and 125); and, of at least 300
+            // columns and 200 MB, 257 to 384 rows (250 million elements: 333 x 467 203 us, else 213; 300 x 500 190 and 202, 300 x 1300 201 and 209; 290 x 255 218 and 217)
+            // and 385 to 512 of whole 8-byte pieces, past 448 of them up to 640 columns (386 x 500 187 and 199, 420 x 700 196 and 200, 500 x 500 190 and 197, 480 x 620 200
+            // both; 480 x 644 209 and 204, 447 x 633 202 and 203, 401 x 777 206 and 205).  At half of that size 330 x 500 57.1 and 54.4, but 447 x 507 58.7 and 59.3.
             if constexpr (MODE != 0) {
                 const bool beyond = (int64_t)batch * n * m > 11ll << 23, wide_rows = m >= 1500;
-                const bool sequences = n > 384 && n <= 512 && m <= 640 && (int64_t)batch * n * m >= 3ll << 25;
+                const bool sequences = n <= 512 && m >= 300 && (int64_t)batch * n * m >= 3ll << 25 && (n <= 384 || (m % 4 == 0 && (n <= 448 || m <= 640)));
                 if (m >= 64 && n > 256 && (MODE == 1 ? n <= 512 && ceil_div(m, 64) * batch > 2 * (int64_t)compute_units() : (n <= 320 && beyond && wide_rows) || sequences)) {
                     launch_tile<512, 8, 8, MODE, true>(batch, n, m, x, y, st);
                     return true;

@@ -47,6 +47,20 @@ def test_softmax_columns(n, m):
     assert ((outs[0][0].double() - ref).abs() <= ref * 2.0 ** -10 + 2.0 ** -24).all()
 
 
+# (from 100 million elements on: the form of lanes for themselves, its rows and columns at the edges of where it is taken)
+@pytest.mark.parametrize("n,m", [(257, 300), (330, 501), (384, 310), (386, 500), (448, 700), (450, 640), (512, 388)])
+def test_softmax_columns_of_large_batches(n, m):
+    batch = -(-(3 << 25) // (n * m)) + 1
+    x, y = _pair(batch, n, m, n + m)
+    out, out_nan = torch.empty_like(x), torch.empty_like(x)
+    for v, o in ((x, out), (y, out_nan)):
+        ck.softmax_forward(batch, n, m, v.data_ptr(), o.data_ptr(), stream())
+    assert torch.equal(out[:, :, 1:].contiguous().view(torch.int16), out_nan[:, :, 1:].contiguous().view(torch.int16))
+    for i in (0, batch // 2, batch - 1):
+        ref = torch.softmax(x[i].double(), 0)
+        assert ((out[i].double() - ref).abs() <= ref * 2.0 ** -10 + 2.0 ** -24).all()
+
+
 @pytest.mark.parametrize("n,m", SIZES)
 def test_normalised_columns(n, m):
     x, y = _pair(3, n, m, n + m)

@@ -431,3 +431,19 @@ def test_yardstick_library_is_separate_from_the_product():
     assert "ceil_" not in out
     # the async status and the allocation-free entry point are part of the product ABI
     assert "gave up waiting" in __import__("cpm_kernels_amd.library.cpmk", fromlist=["x"]).error_string(10004)
+
+
+def test_current_stream_of_other_builds_of_torch(monkeypatch):
+    """The stream's number comes from calls that a build of torch may lack: the stream object then has it."""
+    import types
+    import torch
+    from cpm_kernels_amd.torch import _common
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=7))
+    monkeypatch.setattr(_common, "_raw_stream", lambda device: 100 + device)
+    monkeypatch.setattr(_common, "_device", lambda: 3)
+    assert _common.cur_stream() == 103
+    for name in ("_raw_stream", "_device"):
+        with monkeypatch.context() as m:
+            m.setattr(_common, name, None)
+            assert _common.cur_stream() == 7

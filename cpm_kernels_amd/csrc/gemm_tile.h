@@ -215,7 +215,9 @@ struct SlabDma {
         }
         Pb = a.P + (int64_t)b * a.strideP + (PARTS ? part * a.partP : 0);
         Qb = a.Q + (int64_t)b * a.strideQ + (PARTS ? part * a.partQ : 0);
-        ahead = !PARTS && nxt_item.valid && nxt_item.half == cur_item.half;       // (parts differ in their slabs; a launch of them has a tile a workgroup)
+        // (parts differ in their slabs: each is begun anew, as half tiles are.  The number of parts that the host picks leaves at most a tile a workgroup;
+        // a caller's own may leave several.)
+        ahead = !PARTS && nxt_item.valid && nxt_item.half == cur_item.half;
         // slab s of this tile lives in stage (ring + s) % NST.  With fewer slabs than stages (!deep) all of a
         // tile's slabs are requested one tile ahead and every wait is a full one.
         deep = nk >= NST;

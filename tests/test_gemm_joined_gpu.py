@@ -130,6 +130,15 @@ def test_fp16_in_parts(aT, bT, batch_a, batch_b, m, n, slabs, parts):
         assert ((out[i].double() - ref).abs() <= size * k * 2.0 ** -24 + ref.abs() * 2.0 ** -10.9 + 2.0 ** -25).all()
 
 
+# (more parts of tiles than workgroups that are resident at once, two a compute unit, of 128 x 64 outputs and of 128 x 128; sixteen even parts, eleven of which the last is shorter)
+@pytest.mark.parametrize("m,n", [(64, 16256), (1280, 1664)])
+def test_more_parts_than_workgroups(m, n):
+    A, B, s_row, s_col = _int8(1, 1, m, 32 * 128, n, False, m)
+    assert torch.equal(_whole(A, B, False, s_row, s_col, 32 * 128, 16), _reference(A, B, False, s_row, s_col))
+    test_fp16_in_parts(True, False, 1, 1, m, n, 32, 11)
+    test_fp16_in_parts(False, True, 1, 1, m, n, 32, 11)
+
+
 def test_parts_are_refused_elsewhere():
     A, B, s_row, s_col = _int8(1, 1, 64, 320, 128, False, 0)       # (a depth of whole 64-byte slabs only)
     assert ck.gemm_depth_parts(False, 64, 320, 128, 1, 1, True, False) == 1

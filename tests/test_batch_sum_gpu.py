@@ -79,6 +79,21 @@ def test_groups_fill_the_device(gpu):
                     assert max(fill) >= 0.75, (m, n, batch, kind, k, groups)
 
 
+@pytest.mark.parametrize("kind", [0, 1, 2])       # int8, fp16 K-major, fp16 (K, rows)
+@pytest.mark.parametrize("batch", [1, 2, 7, 12, 16, 17, 32, 34, 48, 1009])
+def test_quickest_groups(gpu, kind, batch):
+    """A divisor of the batch whose groups the sums take (16 entries; (K, rows), one contraction, operands below 4 GiB), or the batch: one by one."""
+    for m, n in ((4, 4), (512, 512), (832, 1856), (1280, 3328), (2560, 2560), (8192, 8192)):
+        for k in (40, 66, 128, 1000, 4096):
+            groups = ck.gemm_sum_groups_timed(kind, m, k, n, batch)
+            assert 1 <= groups <= batch and batch % groups == 0, (m, n, k, groups)
+            if groups < batch:
+                if kind == 2:
+                    assert max(m, n) * k * (batch // groups) * 2 < 1 << 32, (m, n, k, groups)
+                else:
+                    assert batch // groups <= 16, (m, n, k, groups)
+
+
 @pytest.mark.parametrize("shape", [s for s in SHAPES if s[1] > 1])
 def test_int8_parts(gpu, shape):
     batch, groups, n, m, k = shape

@@ -123,6 +123,8 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
         // The same choice of slabs where rows are off cache lines: 1200 x 4004, 320 tiles, k = 200 11.6 us on 64-byte slabs, one workgroup a compute unit, 10.6 so with two and 11.0 on 128-byte ones,
         // 500 18.4, 16.2 and 16.1, 1500 42.5, 38.0 and 31.5; 640 x 640, k = 1000 11.0 and 13.0, 2056 17.1 and 20.2, 1200 x 1500, 1500 22.0 and 19.8, 9196 120 and 88; 3000 x 3000, 500
         // 27.3 and 27.0, 1500 62.1 and 55.8.  (Rows of whole 64-byte slabs: 3000 x 3000, 1504 41.7 and 47.5.)
+        // (Those are operands in reach of L2, where the shorter slabs stay ahead at any depth: 64 x 64, 1452 12.9 and 15.5.  Out of memory the longer ones are ahead from
+        // 500 on, 640 x 640, 1540 34.6 and 28.5.  One line serves both.)
         if (!whole64 && two && k >= 320)
             return rest16 ? launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, SEG | 4, 32>(a, batch, st, 2) : launch_dma<2, 2, 2, 2, 128, kEpiF16, 2, SEG | 12, 32>(a, batch, st, 2);
         if (!whole64 && !two && k >= (mid > cus ? 448 : rest16 ? 2816 : 1280))

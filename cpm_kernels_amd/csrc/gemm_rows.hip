@@ -3,7 +3,7 @@
 // (cpm_kernels/torch/gemm.py:189-203).
 //
 // Bound by writing the output.  Tiles of part of a row write segments that begin and end inside cache lines, which their neighbours complete at
-// another time.  Here a workgroup has whole rows, 64 to 560 of them: 16 at a time are put together in LDS as they lie in memory and leave as whole aligned
+// another time.  Here a workgroup has whole rows, a multiple of 16 and as many as LDS holds at most (about 1200 at K <= 32, 400 at K = 80): 16 at a time are put together in LDS as they lie in memory and leave as whole aligned
 // lines.  A wave has 128 columns, whose operand it keeps in registers, transposed there, for all rows of the workgroup.
 // Heads of seq x seq, K = 64, with operands that are not in the caches and a pass over the output behind (of 186 us for 1024 of 500, 63 for 300, which is in both figures):
 // 1024 of 500 330 -> 290 us, 512 158 -> 133, 128 45 -> 40, 1024 of 300 131 -> 115, 100 of 902 114 -> 86; 1024 of 110 38 -> 28, 32 14.8 -> 9.7; K = 80 66 of 902 81 -> 72,
@@ -130,8 +130,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KS == 3 ? 3
     }
 }
 
-// Rows of a workgroup, 32 at least: the fewest rounds of the device, of eight waves a compute unit at least (twelve of short rows), times the time of one, its start as long as 200
-// rows; two of them fit the LDS (1024 of 500 x 500 in one, two and four parts 289, 293 and 309 us, 128 of them 58, 45 and 40, 256 81, 72 and 73; 186 of 572 x 572
+// Rows of a workgroup, a multiple of 16, at most the 80 KB of LDS that two workgroups a compute unit leave each: the fewest rounds of the device, of eight waves a compute unit at least (twelve of short rows), times the time of one, its start as long as 200
+// rows (1024 of 500 x 500 in one, two and four parts 289, 293 and 309 us, 128 of them 58, 45 and 40, 256 81, 72 and 73; 186 of 572 x 572
 // in two, three and four 71, 79 and 74, 150 of 570 x 570 62, 58 and 64).
 static int32_t rows_tall(int32_t n, int32_t m, int ks, int64_t batch) {
     const int64_t cus = compute_units(), waves = ceil_div(m, 128), floor = waves >= 4 ? 2 : 12 / waves, cap = (80 * 1024 - 128 - 32ll * m) / (ks * 64) / 16 * 16;

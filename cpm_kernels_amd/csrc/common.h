@@ -422,4 +422,41 @@ inline int enable_dynamic_lds(const void* kern, int bytes, std::atomic<bool>* do
     return 0;
 }
 
+// A 64 x 64 tile from (r0, c0) on of an (n, m) matrix, through LDS to the transposed one, by 256 lanes: pieces of eight on both sides, wherever they start
+// (a barrier lies between the two).  Rows of 144 bytes, an odd multiple of 16.
+using TransposeTile = half_t[64][72];
+
+__device__ __forceinline__ void transpose_tile_in(TransposeTile& tile, const half_t* in, int32_t n, int32_t m, int32_t r0, int32_t c0, int tid) {
+    const int pc = tid & 7, rr = tid >> 3;          // 8 pieces x 32 rows per pass
+#pragma unroll
+    for (int ps = 0; ps < 2; ++ps) {
+        const int r = ps * 32 + rr;
+        const int32_t c = c0 + pc * 8;
+        if (r0 + r < n && c < m) {
+            const half_t* src = in + (int64_t)(r0 + r) * m + c;
+            half8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
+            if (c + 8 <= m) v = load_half8_any(src);
+            else v = load_half8_head_any(src, m - c, v);
+            *reinterpret_cast<half8_t*>(&tile[r][pc * 8]) = v;
+        }
+    }
+}
+
+__device__ __forceinline__ void transpose_tile_out(const TransposeTile& tile, half_t* out, int32_t n, int32_t m, int32_t r0, int32_t c0, int tid) {
+    const int pc = tid & 7, rr = tid >> 3;
+#pragma unroll
+    for (int ps = 0; ps < 2; ++ps) {
+        const int c = ps * 32 + rr;                     // row of the transposed tile
+        const int32_t r = r0 + pc * 8;
+        if (c0 + c < m && r < n) {
+            half8_t v;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = tile[pc * 8 + e][c];
+            half_t* dst = out + (int64_t)(c0 + c) * n + r;
+            if (r + 8 <= n) store_half8_any(dst, v);
+            else store_half8_head_any(dst, n - r, v);
+        }
+    }
+}
+
 }  // namespace cpmk

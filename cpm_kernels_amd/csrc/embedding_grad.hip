@@ -101,41 +101,16 @@ __global__ __launch_bounds__(kPrepareThreads) void k_embedding_prepare(PrepareAr
 #pragma unroll
                 for (int e = 0; e < 8; ++e) *reinterpret_cast<half8_t*>(a.rows + boff + (int64_t)(c + e) * n + r) = v[e];
         } else {
-            // four tiles of 64 x 64, 256 lanes each; pieces of eight on both sides, wherever they start
-            __shared__ __attribute__((aligned(16))) half_t tile4[4][64][72];       // (pitch 144 bytes: an odd multiple of 16)
-            const int sub = threadIdx.x >> 8, tid = threadIdx.x & 255, pc = tid & 7, rr = tid >> 3;
-            half_t(&tile)[64][72] = tile4[sub];
+            // four tiles of 64 x 64, 256 lanes each
+            __shared__ __attribute__((aligned(16))) TransposeTile tile[4];
+            const int sub = threadIdx.x >> 8, tid = threadIdx.x & 255;
             const uint32_t t = block * 4 + sub;
-            const bool live = t < a.tiles;
             const uint32_t b = t / per, in = t - b * per, tr = in / a.tiles_c, tc = in - tr * a.tiles_c;
-            const int32_t r0 = tr * 64, c0 = tc * 64;
+            const int32_t r0 = tr * 64, c0 = tc * 64, rows = t < a.tiles ? n : 0;
             const int64_t boff = (int64_t)b * n * m;
-#pragma unroll
-            for (int ps = 0; ps < 2; ++ps) {
-                const int r = ps * 32 + rr;
-                const int32_t c = c0 + pc * 8;
-                if (live && r0 + r < n && c < m) {
-                    const half_t* src = a.grad + boff + (int64_t)(r0 + r) * m + c;
-                    half8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
-                    if (c + 8 <= m) v = load_half8_any(src);
-                    else v = load_half8_head_any(src, m - c, v);
-                    *reinterpret_cast<half8_t*>(&tile[r][pc * 8]) = v;
-                }
-            }
+            transpose_tile_in(tile[sub], a.grad + boff, rows, m, r0, c0, tid);
             __syncthreads();
-#pragma unroll
-            for (int ps = 0; ps < 2; ++ps) {
-                const int c = ps * 32 + rr;                     // row of the transposed tile
-                const int32_t r = r0 + pc * 8;
-                if (live && c0 + c < m && r < n) {
-                    half8_t v;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[e] = tile[pc * 8 + e][c];
-                    half_t* dst = a.rows + boff + (int64_t)(c0 + c) * n + r;
-                    if (r + 8 <= n) store_half8_any(dst, v);
-                    else store_half8_head_any(dst, n - r, v);
-                }
-            }
+            if (rows) transpose_tile_out(tile[sub], a.rows + boff, n, m, r0, c0, tid);
         }
         return;
     }

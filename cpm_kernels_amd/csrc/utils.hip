@@ -11,43 +11,19 @@ namespace cpmk {
 // alignment), single halves for the piece across a row's end; the scalar form (IN = OUT = false) for rows under eight.
 template <bool IN, bool OUT>
 __global__ __launch_bounds__(256) void k_transpose(int32_t n, int32_t m, const half_t* __restrict__ in, half_t* __restrict__ out) {
-    __shared__ __attribute__((aligned(16))) half_t tile[64][72];    // pitch 144 bytes: 16-byte aligned rows, odd multiple of 16 bytes
+    __shared__ __attribute__((aligned(16))) TransposeTile tile;
     const int64_t boff = (int64_t)blockIdx.z * n * m;
     const int32_t r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-    const int pc = threadIdx.x & 7, rr = threadIdx.x >> 3;          // 8 pieces x 32 rows per pass
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     if constexpr (IN) {
-#pragma unroll
-        for (int ps = 0; ps < 2; ++ps) {
-            const int r = ps * 32 + rr;
-            const int32_t c = c0 + pc * 8;
-            if (r0 + r < n && c < m) {
-                const half_t* src = in + boff + (int64_t)(r0 + r) * m + c;
-                half8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
-                if (c + 8 <= m) v = load_half8_any(src);
-                else v = load_half8_head_any(src, m - c, v);
-                *reinterpret_cast<half8_t*>(&tile[r][pc * 8]) = v;
-            }
-        }
+        transpose_tile_in(tile, in + boff, n, m, r0, c0, threadIdx.x);
     } else {
         for (int r = ty; r < 64; r += 4)
             if (r0 + r < n && c0 + tx < m) tile[r][tx] = in[boff + (int64_t)(r0 + r) * m + c0 + tx];
     }
     __syncthreads();
     if constexpr (OUT) {
-#pragma unroll
-        for (int ps = 0; ps < 2; ++ps) {
-            const int c = ps * 32 + rr;                     // row of the transposed tile
-            const int32_t r = r0 + pc * 8;
-            if (c0 + c < m && r < n) {
-                half8_t v;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = tile[pc * 8 + e][c];
-                half_t* dst = out + boff + (int64_t)(c0 + c) * n + r;
-                if (r + 8 <= n) store_half8_any(dst, v);
-                else store_half8_head_any(dst, n - r, v);
-            }
-        }
+        transpose_tile_out(tile, out + boff, n, m, r0, c0, threadIdx.x);
     } else {
         for (int c = ty; c < 64; c += 4)
             if (c0 + c < m && r0 + tx < n) out[boff + (int64_t)(c0 + c) * n + r0 + tx] = tile[tx][c];

@@ -1252,11 +1252,15 @@ static int64_t big_tiles(int32_t n, int32_t m, int batch, int64_t apart) {
 }
 
 // The time of a product's tiles, in tenths of a round of 128 x 128 tiles over the chip: a second round beside the first costs 0.8 of it (two
-// workgroups fit a compute unit), a round of 256 x 256 tiles 2.2, and one of 128 x 64 tiles, where the product has them (`halves`), 0.8.
-static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool halves) {
+// workgroups fit a compute unit), a round of 256 x 256 tiles 2.2.  int8, K-major: `halves`, whether there are tiles of 128 x 64, a round of which is 0.8,
+// and `whole`, whether a last round of large tiles is one of half tiles (fp16 products are drawn without: no better for it).
+static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool whole, bool halves) {
     const int64_t cus = compute_units();
     const int64_t tiles = ceil_div(n, 128) * ceil_div(m, 128) * batch;
-    if (n > 128 && m > 128 && big_tiles(n, m, batch, apart) * 4 >= cus * 3) return 22 * ceil_div(ceil_div(n, 256) * ceil_div(m, 256) * batch, cus);
+    if (n > 128 && m > 128 && big_tiles(n, m, batch, apart) * 4 >= cus * 3) {
+        const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch, r = big % cus;
+        return whole && big > cus && r != 0 && 2 * r <= cus ? 22 * (big / cus) + 13 : 22 * ceil_div(big, cus);
+    }
     if (halves && tiles * 4 < cus * 3 && ceil_div(n, 128) * ceil_div(m, 64) * batch <= cus) return 8;
     return tiles <= cus ? 10 : tiles <= 2 * cus ? 18 : 10 * ceil_div(tiles, cus);
 }
@@ -1265,39 +1269,39 @@ static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool 
 // quicker: its results need no search for their entry (0.4 us on the smallest tiles), and fp16's few rows keep the kernels made for them.
 // Over 1370 drawn int8 and 1430 fp16 products, joined : apart as a geometric mean,
 //                   always                   where it pays (what follows)     (the better of both for each)
-//   int8 rows       0.958, 102 worse > 4 %   0.950, 2 worse                   0.945
-//   int8 columns    0.977, 273 worse         0.960, 1 worse                   0.958
+//   int8 rows       0.958, 102 worse > 4 %   0.949, 2 worse                   0.945
+//   int8 columns    0.977, 273 worse         0.960, 4 worse                   0.958
 //   fp16 rows       1.043, 307 worse         0.976, 6 worse                   0.961
-//   fp16 columns    1.026, 335 worse         0.962, 3 worse                   0.958
+//   fp16 columns    1.026, 335 worse         0.960, 3 worse                   0.958
 struct JoinGain {
     int64_t rounds, rounds_joined, tiles, tiles_joined;
     bool fewer() const { return rounds_joined < rounds; }
 };
-static JoinGain join_gain(int32_t n, int32_t m, int batch, bool rows, int64_t apart, bool halves) {
+static JoinGain join_gain(int32_t n, int32_t m, int batch, bool rows, int64_t apart, bool whole, bool halves) {
     const int32_t nj = rows ? n * batch : n, mj = rows ? m : m * batch;
-    return {tile_rounds(n, m, batch, 0, halves), tile_rounds(nj, mj, 1, apart, halves), ceil_div(n, 128) * ceil_div(m, 128) * batch, ceil_div(nj, 128) * ceil_div(mj, 128)};
+    return {tile_rounds(n, m, batch, 0, whole, halves), tile_rounds(nj, mj, 1, apart, whole, halves), ceil_div(n, 128) * ceil_div(m, 128) * batch, ceil_div(nj, 128) * ceil_div(mj, 128)};
 }
 // fp16, whose few rows and short depths have kernels of their own: rows, past 128 of them or a depth of 448, or many tiles of enough depth
 // (500 entries of 4 x 400 beside 314: 19.3 -> 7.5 us; 41 of 4 x 64 beside 3808, 4.3 apart and 5.7 joined)
 static bool rows_join_pays_f16(int32_t n, int32_t m, int32_t k, int batch, int64_t apart) {
-    const JoinGain g = join_gain(n, m, batch, true, apart, false);
+    const JoinGain g = join_gain(n, m, batch, true, apart, false, false);
     return g.fewer() && (n > 128 || k > 448 || (g.tiles > 4 * (int64_t)compute_units() && g.tiles * k > 100000 && g.tiles_joined * 3 <= g.tiles));
 }
 // Columns, past 64 rows or a depth of 320; a row operand stored (K, rows) leaves fewer such calls to those kernels, and in a single round its long
 // depths gain too (357 entries of 64 columns, 40 rows, K = 240 14.5 -> 9.5 us; 94 of 128, 64 rows, K = 2328 28.7 -> 23.7)
 static bool cols_join_pays_f16(int32_t n, int32_t m, int32_t k, bool krows, int batch, int64_t apart) {
-    const JoinGain g = join_gain(n, m, batch, false, apart, false);
+    const JoinGain g = join_gain(n, m, batch, false, apart, false, false);
     if (g.fewer() && (n > 64 || k > 320 || (krows && g.tiles * k > 19000 && g.tiles_joined * 4 <= g.tiles * 3))) return true;
     return krows && n <= 64 && k >= 512 && g.tiles_joined <= compute_units();
 }
 // int8: rows also wherever the rounds stay, past one of them, with what the tiles of whole slabs do not take (19 of 2564 x 1600 beside 40 stored
 // (K, columns), 495 -> 300; 37 of 128 x 36 beside 1280, 46 -> 17)
 static bool rows_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
-    const JoinGain g = join_gain(n, m, batch, true, apart, kmajor && k % 128 == 0);
+    const JoinGain g = join_gain(n, m, batch, true, apart, k % 64 == 0, kmajor && k % 128 == 0);
     return g.fewer() || ((!kmajor || k % 64 != 0) && g.tiles > compute_units() && g.rounds_joined == g.rounds);
 }
 static bool cols_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
-    return join_gain(n, m, batch, false, apart, kmajor && k % 128 == 0).fewer();
+    return join_gain(n, m, batch, false, apart, k % 64 == 0, kmajor && k % 128 == 0).fewer();
 }
 
 }  // namespace cpmk

@@ -337,18 +337,20 @@ static int gemm_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_
             }
             // (a dimension of at most 128 would leave half or more of every 256-wide tile empty)
             if (big * 4 >= compute_units() * 3 && n > 128 && m > 128) return launch_dma<2, 4, 4, 2, 128, EPI, kRingBig, LAY, 16>(a, batch, st);
-            // 128x128 tiles, or 128x64 when even those leave a quarter of the compute units idle and twice as many of half their size are one round
-            // (two workgroups a compute unit of the latter: 500 x 5000, 160 tiles or 320, K = 4096 23.5 us, 18.5 so; K = 12160 58 and 43; K = 512 8.1 and 8.0)
+            // 128x128 tiles, or 128x64 when even those leave a quarter of the compute units idle, where these are one round, or two of them a compute unit and a
+            // depth up to 768: 1208 x 2296, 180 tiles or 360, K = 128 7.3 us and 6.7, 512 8.5 and 8.0, 768 9.3 and 8.8, 4096 21.4 and 23.3 (operands out of memory
+            // 8.0 and 7.2, 10.2 and 9.1, 11.3 and 10.7, 25.4 and 30.9); 500 x 5000, 160 or 316, K = 768 9.1 and 8.9 (11.5 and 11.6), 4096 20.6 and 27.4
             const int64_t mid = ceil_div(n, 128) * ceil_div(m, 128) * batch;
             // the smaller tiles finish a slab before a load from L2 returns: four ring stages keep them fed.  More
             // tiles than compute units but at most two each: a ring of two stages instead, which lets two
             // workgroups share a compute unit (2 x 80 KB of LDS) and all tiles run in one round, each
             // workgroup's waits covered by the other's MFMAs (6-11 % over 1.25-2 rounds of single workgroups)
             const int64_t cus = compute_units(), small = ceil_div(n, 128) * ceil_div(m, 64) * batch;
-            if (mid * 4 >= cus * 3 || small > cus) {
+            if (mid * 4 >= cus * 3 || (small > cus && k > 768)) {
                 if (mid > cus && mid <= 2 * cus) return launch_dma<2, 2, 2, 2, 128, EPI, 2, LAY, 32>(a, batch, st, 2);
                 return launch_dma<2, 2, 2, 2, 128, EPI, kRingSmall, LAY, 32>(a, batch, st);
             }
+            if (small > cus) return launch_dma<2, 2, 2, 1, 128, EPI, 2, LAY, 32>(a, batch, st, 2);
             return launch_dma<2, 2, 2, 1, 128, EPI, kRingSmall, LAY, 32>(a, batch, st);
         };
         if constexpr (FUSED) {

@@ -100,6 +100,14 @@ def test_fp16_of_many_entries(a_shared, edge, batch, other, k, stored_other):
         assert ((out[i].double() - ref).abs() <= size * k * 2.0 ** -24 + ref.abs() * 2.0 ** -10.9 + 2.0 ** -25).all()
 
 
+# (tiles of 128 x 64, two a compute unit, up to a depth of 768, of 128 x 128 beyond; whole and over the joined columns of many entries)
+@pytest.mark.parametrize("m,batch,n", [(5000, 1, 500), (1100, 1, 2164), (36, 500, 128), (68, 130, 252)])
+@pytest.mark.parametrize("k", [128, 768, 896])
+def test_narrow_tiles(m, batch, n, k):
+    A, B, s_row, s_col = _int8(batch, 1, m, k, n, False, m + k)
+    assert torch.equal(_whole(A, B, False, s_row, s_col, k), _reference(A, B, False, s_row, s_col))
+
+
 # (parts of one slab, of several, a shorter last part, more parts than slabs)
 @pytest.mark.parametrize("batch_a,batch_b,m,n,bT", [(1, 1, 64, 128, False), (3, 1, 44, 260, False), (1, 5, 132, 60, False), (2, 2, 132, 132, False),
                                                     (3, 1, 100, 272, True), (3, 1, 20, 16, True)])

@@ -133,7 +133,10 @@ def gemm_and_scale(quantA, scaleA, quantB, scaleB, aT, bT, fused=True) -> torch.
     batch = max(quantA.size(0), quantB.size(0))
     result_fp = torch.empty((batch, M, N), dtype=torch.float16, device=quantA.device)
     if fused:
-        parts = gemm_depth_parts(False, N, K, M, quantB.size(0), quantA.size(0), bT, aT) if K >= 2048 and result_fp.numel() < _PARTS_MOST else 1
+        parts = 1
+        # (whole 16-byte pieces: a caller's operands may lie anywhere)
+        if K >= 2048 and result_fp.numel() < _PARTS_MOST and (quantA.data_ptr() | quantB.data_ptr()) % 16 == 0 and (scaleB is None or scaleB.data_ptr() % 8 == 0):
+            parts = gemm_depth_parts(False, N, K, M, quantB.size(0), quantA.size(0), bT, aT)
         if parts > 1:
             workspace = torch.empty((parts, result_fp.numel()), dtype=torch.int32, device=quantA.device)
             gemm_int8_scale_split(N, K, M, quantB.size(0), quantA.size(0), bT, aT, quantB.data_ptr(), quantA.data_ptr(),

@@ -147,6 +147,21 @@ def test_more_parts_than_workgroups(m, n):
     test_fp16_in_parts(False, True, 1, 1, m, n, 32, 11)
 
 
+@pytest.mark.parametrize("at_a,at_b,at_scale", [(4, 0, 0), (0, 1, 0), (0, 0, 2), (0, 0, 0)])
+def test_operands_off_whole_pieces(at_a, at_b, at_scale):
+    """A product whose depth would be divided, from operands and scales at any address"""
+    from cpm_kernels_amd.torch.gemm import gemm_and_scale
+    M, K, N = 120, 8192, 512
+    assert ck.gemm_depth_parts(False, N, K, M, 1, 1, True, False) > 1
+    B, A, s_row, s_col = _int8(1, 1, N, K, M, False, 3)
+
+    def moved(t, at):
+        flat = torch.empty(t.numel() + at, dtype=t.dtype, device="cuda")
+        return flat[at:].view(t.shape).copy_(t)
+    out = gemm_and_scale(moved(A, at_a), s_row, moved(B, at_b), moved(s_col, at_scale), False, True)
+    assert torch.equal(out, _reference(B, A, False, s_row, s_col))
+
+
 def test_parts_are_refused_elsewhere():
     A, B, s_row, s_col = _int8(1, 1, 64, 320, 128, False, 0)       # (a depth of whole 64-byte slabs only)
     assert ck.gemm_depth_parts(False, 64, 320, 128, 1, 1, True, False) == 1

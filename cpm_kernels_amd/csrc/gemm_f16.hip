@@ -15,7 +15,7 @@ static int gemm_f16_dispatch(int32_t m, int32_t k, int32_t n, int32_t batchA, in
     if (out == nullptr || (k > 0 && any_null(A, B))) return CPMK_EBADARG;
     if (k > (1 << 30)) return CPMK_ETOOBIG;
     const int64_t big_apart = n > 128 && m > 128 ? ceil_div(n, 256) * ceil_div(m, 256) * batch : 0;       // (big_tiles)
-    if (batchA == 1 && !bT && rows_join(batch, n, (int64_t)k * 2) && rows_join_pays_f16(n, m, k, batch, big_apart)) {
+    if (batchA == 1 && !bT && rows_join(batch, n, (int64_t)k * 2) && rows_join_pays_f16(n, m, k, aT, batch, big_apart)) {
         n *= batch;
         batch = batchB = 1;
     }

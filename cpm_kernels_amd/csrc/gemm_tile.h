@@ -1265,17 +1265,20 @@ static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool 
     return tiles <= cus ? 10 : tiles <= 2 * cus ? 18 : 10 * ceil_div(tiles, cus);
 }
 
-// What joining entries does: rounds (tile_rounds) and 128 x 128 tiles, apart and joined.  Where it saves no round, the product apart is as quick or
+// What joining entries does: rounds (tile_rounds) and 128 x 128 tiles, apart and joined.  Where it saves neither, the product apart is as quick or
 // quicker: its results need no search for their entry (0.4 us on the smallest tiles), and fp16's few rows keep the kernels made for them.
 // Over 1370 drawn int8 and 1430 fp16 products, joined : apart as a geometric mean,
-//                   always                   where it pays (what follows)     (the better of both for each)
+//                   always                   where it saves rounds            (the better of both for each)
 //   int8 rows       0.958, 102 worse > 4 %   0.949, 2 worse                   0.945
 //   int8 columns    0.977, 273 worse         0.960, 4 worse                   0.958
 //   fp16 rows       1.043, 307 worse         0.976, 6 worse                   0.961
 //   fp16 columns    1.026, 335 worse         0.960, 3 worse                   0.958
+// Where the rounds stay and tiles are saved it pays too for K-major operands of enough whole slabs (the same figures over those that the rules below take):
+//   int8 rows 0.980, none of 103; fp16 rows 0.973, 1 of 66; int8 columns 0.964, 1 of 135; fp16 columns 0.948, none of 68
 struct JoinGain {
     int64_t rounds, rounds_joined, tiles, tiles_joined;
     bool fewer() const { return rounds_joined < rounds; }
+    bool even(int64_t num, int64_t den) const { return rounds_joined == rounds && tiles_joined < tiles && tiles_joined * den <= tiles * num; }      // .. at most num / den of the tiles
 };
 static JoinGain join_gain(int32_t n, int32_t m, int batch, bool rows, int64_t apart, bool whole, bool halves) {
     const int32_t nj = rows ? n * batch : n, mj = rows ? m : m * batch;
@@ -1283,8 +1286,9 @@ static JoinGain join_gain(int32_t n, int32_t m, int batch, bool rows, int64_t ap
 }
 // fp16, whose few rows and short depths have kernels of their own: rows, past 128 of them or a depth of 448, or many tiles of enough depth
 // (500 entries of 4 x 400 beside 314: 19.3 -> 7.5 us; 41 of 4 x 64 beside 3808, 4.3 apart and 5.7 joined)
-static bool rows_join_pays_f16(int32_t n, int32_t m, int32_t k, int batch, int64_t apart) {
+static bool rows_join_pays_f16(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, true, apart, false, false);
+    if (kmajor && k % 64 == 0 && k >= 704 && g.even(1, 1)) return true;
     return g.fewer() && (n > 128 || k > 448 || (g.tiles > 4 * (int64_t)compute_units() && g.tiles * k > 100000 && g.tiles_joined * 3 <= g.tiles));
 }
 // Columns, past 64 rows or a depth of 320; a row operand stored (K, rows) leaves fewer such calls to those kernels, and in a single round its long
@@ -1292,16 +1296,20 @@ static bool rows_join_pays_f16(int32_t n, int32_t m, int32_t k, int batch, int64
 static bool cols_join_pays_f16(int32_t n, int32_t m, int32_t k, bool krows, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, false, apart, false, false);
     if (g.fewer() && (n > 64 || k > 320 || (krows && g.tiles * k > 19000 && g.tiles_joined * 4 <= g.tiles * 3))) return true;
+    if (!krows && k % 64 == 0 && k >= 1536 && g.rounds >= 22 && g.even(1, 1)) return true;
     return krows && n <= 64 && k >= 512 && g.tiles_joined <= compute_units();
 }
 // int8: rows also wherever the rounds stay, past one of them, with what the tiles of whole slabs do not take (19 of 2564 x 1600 beside 40 stored
 // (K, columns), 495 -> 300; 37 of 128 x 36 beside 1280, 46 -> 17)
 static bool rows_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, true, apart, k % 64 == 0, kmajor && k % 128 == 0);
+    if (kmajor && k % 128 == 0 && k >= 384 && g.even(1, 1)) return true;
     return g.fewer() || ((!kmajor || k % 64 != 0) && g.tiles > compute_units() && g.rounds_joined == g.rounds);
 }
 static bool cols_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
-    return join_gain(n, m, batch, false, apart, k % 64 == 0, kmajor && k % 128 == 0).fewer();
+    const JoinGain g = join_gain(n, m, batch, false, apart, k % 64 == 0, kmajor && k % 128 == 0);
+    if (kmajor && k % 128 == 0 && k >= 1536 && g.rounds >= 18 && (g.rounds > 18 || n >= 2048 ? g.even(19, 20) : g.even(17, 20))) return true;
+    return g.fewer();
 }
 
 }  // namespace cpmk

@@ -100,6 +100,18 @@ def test_fp16_of_many_entries(a_shared, edge, batch, other, k, stored_other):
         assert ((out[i].double() - ref).abs() <= size * k * 2.0 ** -24 + ref.abs() * 2.0 ** -10.9 + 2.0 ** -25).all()
 
 
+# (as many rounds of fewer tiles: 128 x 64, 128 x 128 in two rounds, 256 x 256)
+@pytest.mark.parametrize("shared,edge,batch", [(432, 164, 7), (2176, 196, 12), (2048, 192, 24)])
+@pytest.mark.parametrize("k", [384, 704, 1536])
+def test_fewer_tiles(shared, edge, batch, k):
+    A, B, s_row, s_col = _int8(batch, 1, edge, k, shared, False, edge + k)
+    assert torch.equal(_whole(A, B, False, s_row, s_col, k), _reference(A, B, False, s_row, s_col))
+    A, B, s_row, s_col = _int8(1, batch, shared, k, edge, False, edge + k)
+    assert torch.equal(_whole(A, B, False, s_row, s_col, k), _reference(A, B, False, s_row, s_col))
+    for a_shared in (False, True):
+        test_fp16_of_many_entries(a_shared, edge, batch, shared, k, False)
+
+
 # (tiles of 128 x 64, two a compute unit, up to a depth of 768, of 128 x 128 beyond; whole and over the joined columns of many entries)
 @pytest.mark.parametrize("m,batch,n", [(5000, 1, 500), (1100, 1, 2164), (36, 500, 128), (68, 130, 252)])
 @pytest.mark.parametrize("k", [128, 768, 896])

@@ -1273,8 +1273,9 @@ static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool 
 //   int8 columns    0.977, 273 worse         0.960, 4 worse                   0.958
 //   fp16 rows       1.043, 307 worse         0.976, 6 worse                   0.961
 //   fp16 columns    1.026, 335 worse         0.960, 3 worse                   0.958
-// Where the rounds stay and tiles are saved it pays too for K-major operands of enough whole slabs (the same figures over those that the rules below take):
-//   int8 rows 0.980, none of 103; fp16 rows 0.973, 1 of 66; int8 columns 0.964, 1 of 135; fp16 columns 0.948, none of 68
+// Where the rounds stay and tiles are saved it pays too for K-major operands of enough whole slabs, fp16 rows of any depth from 1024 on (the same figures over those that the
+// rules below take): int8 rows 0.980, none of 103; fp16 rows 0.973, 2 of 120; int8 columns 0.964, 1 of 135; fp16 columns 0.948, none of 68; rows
+// from 1024 on where the tiles stay too, 0.985, none of 19 (47 entries of 128 x 1280 beside 832 26.2 -> 22.8 us)
 struct JoinGain {
     int64_t rounds, rounds_joined, tiles, tiles_joined;
     bool fewer() const { return rounds_joined < rounds; }
@@ -1288,7 +1289,7 @@ static JoinGain join_gain(int32_t n, int32_t m, int batch, bool rows, int64_t ap
 // (500 entries of 4 x 400 beside 314: 19.3 -> 7.5 us; 41 of 4 x 64 beside 3808, 4.3 apart and 5.7 joined)
 static bool rows_join_pays_f16(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, true, apart, false, false);
-    if (kmajor && k % 64 == 0 && k >= 704 && g.even(1, 1)) return true;
+    if (k >= 1024 ? g.rounds_joined == g.rounds : kmajor && k % 64 == 0 && k >= 512 && g.even(1, 1)) return true;
     return g.fewer() && (n > 128 || k > 448 || (g.tiles > 4 * (int64_t)compute_units() && g.tiles * k > 100000 && g.tiles_joined * 3 <= g.tiles));
 }
 // Columns, past 64 rows or a depth of 320; a row operand stored (K, rows) leaves fewer such calls to those kernels, and in a single round its long
@@ -1303,7 +1304,7 @@ static bool cols_join_pays_f16(int32_t n, int32_t m, int32_t k, bool krows, int 
 // (K, columns), 495 -> 300; 37 of 128 x 36 beside 1280, 46 -> 17)
 static bool rows_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, true, apart, k % 64 == 0, kmajor && k % 128 == 0);
-    if (kmajor && k % 128 == 0 && k >= 384 && g.even(1, 1)) return true;
+    if (kmajor && k % 128 == 0 && (k >= 1024 ? g.rounds_joined == g.rounds : k >= 384 && g.even(1, 1))) return true;
     return g.fewer() || ((!kmajor || k % 64 != 0) && g.tiles > compute_units() && g.rounds_joined == g.rounds);
 }
 static bool cols_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {

@@ -145,7 +145,7 @@ static int parts_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t bat
 // outputs 0.31 (0.34), start and end of the product 4.5, the second kernel 3 and the time to write and read the parts at 4.7 TB/s.  Whole / divided:
 // int8 120 x 3904, K = 4096 15.3 / 14.0 (3 parts, left whole), 8192 25.0 / 16.0 (6), 12160 34.3 / 18.3 (8); 136 x 3200 over 5 entries, K = 8192 39.5 / 33.2 (3);
 // 512 x 4096, K = 12160 38.2 / 36.0 (2, left whole); fp16 56 x 4608, K = 1024 12.0 / 10.1 (left whole), 2048 19.1 / 11.6 (4), 9664 69 / 20.6 (6).
-static int32_t depth_parts(bool f16, int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, float* time = nullptr) {
+int32_t depth_parts(bool f16, int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, float* time) {
     PartsForm f;
     if (!parts_form(f16, m, k, n, batchA, batchB, aT, bT, true, true, f)) return 1;
     const int64_t cus = compute_units();
@@ -168,30 +168,54 @@ static int32_t depth_parts(bool f16, int32_t m, int32_t k, int32_t n, int32_t ba
     return best;
 }
 
-// fp16, a weight A (1, n, k) [(1, k, n) if aT] beside entries B (batch, k, m) of few columns: whether a copy of the entries as (batch, m, k) pays.  Then
-// they are joined to one product and its depth may be divided, where entries stored (K, rows) of less than a tile, or of rows that are not whole
-// 16-byte pieces, are a tile or more each, on the kernel for any size or on the tile kernel.  Estimates in us as above, within 20 % at
-// columns x entries x k beside rows (direct / with the copy, us): 36 x 1 x 4096 beside 1024 65 / 18, 40 x 1 13 / 19; 100 x 16 x 1024 beside 4608 49 / 29, 104 x 16
-// 38 / 28, 240 x 16 51 / 54; 40 x 5 x 9664 beside 4608 59 / 40; 188 x 1 x 4096 beside 1024 33 / 20, 36 x 5 x 512 beside 2048 10.7 / 14.2.
-static bool copy_pays(int32_t n, int32_t k, int32_t m, int32_t batch, int aT) {
-    if (m >= 512 || k < 256 || n < 128) return false;
-    const int64_t cus = compute_units(), cols = (int64_t)m * batch;
-    if (cols * k >= 1ll << 30) return false;
-    const float slabs = (float)k / 64.0f;
-    auto tiled = [&](int64_t rt, int64_t width, int64_t entries, float one) {
-        const int64_t t = rt * ceil_div(width, 128) * entries, big = ceil_div(n, 256) * ceil_div(width, 256) * entries;
-        if (big * 4 >= cus * 3 && n > 128 && width > 128) return (float)ceil_div(big, cus) * (slabs * 1.25f + 8.0f);
-        if (t <= cus) return 4.5f + slabs * one;
-        if (t <= 2 * cus) return 5.0f + slabs * one * 1.8f;
-        return (float)ceil_div(t, cus) * (slabs * one + 3.5f);
+// fp16, a weight A (1, n, k) [(1, k, n) if aT] beside entries B (batch, k, m): estimates in us as above, of the product as it lies and with a copy of the
+// entries as (batch, m, k), which are joined to one product then and whose depth may be divided, where entries stored (K, rows) of less than a
+// tile, or of rows that are not whole 16-byte pieces, are a tile or more each, on the kernel for any size or on the tile kernel.  Fitted to 700 products of 4
+// to 508 columns, 1 to 24 entries and depths of 256 to 24000 beside 128 to 10240 rows, the most within 15 %.
+struct CopyTimes {
+    float direct, copied;
+};
+static CopyTimes copy_times(int32_t n, int32_t k, int32_t m, int32_t batch, int aT) {
+    const float cus = (float)compute_units(), slabs = (float)k / 64.0f, mb = 1e-6f * (float)k * (float)m * (float)batch;
+    auto tiled = [&](int64_t width, int64_t entries, float base, float one, float two, float many) {        // (tiles of up to a round, two, more of them)
+        const float rounds = (float)(ceil_div(n, 128) * ceil_div(width, 128) * entries) / cus;
+        return base + slabs * (rounds <= 1.0f ? one : rounds <= 2.0f ? two : many * rounds);
     };
-    const int64_t rt = ceil_div(n, 128);
-    const bool whole = k % 64 == 0, join = m % 4 == 0 && (!aT || n % 8 == 0);
-    float direct = m % 8 != 0 && m < 128 ? 3.0f + slabs * (m <= 64 ? 1.4f : 2.4f) : tiled(rt, m, batch, whole ? 0.44f : 0.5f);
-    depth_parts(true, m, k, n, batch, 1, 0, aT, &direct);
-    float joined = tiled(rt, join ? cols : m, join ? 1 : batch, whole ? 0.44f : aT ? 0.5f : 0.85f);
-    depth_parts(true, m, k, n, batch, 1, 1, aT, &joined);
-    return joined + 7.0f + 1e-6f * (float)cols * (float)k < 0.93f * direct;
+    const bool whole = k % 64 == 0;
+    CopyTimes t;
+    if (depth_parts(true, m, k, n, batch, 1, 0, aT, &t.direct) == 1) {
+        if (m % 8 != 0 && m < 128) {
+            const float rounds = (float)(ceil_div(n, 64) * ceil_div(m, 64) * batch) / cus;
+            t.direct = 2.6f + slabs * (rounds <= 1.0f ? 0.58f : rounds <= 4.0f ? 1.1f : 0.29f * rounds);
+        } else {
+            t.direct = aT ? tiled(m, batch, 4.8f, whole ? 0.49f : 0.58f, 0.8f, 0.86f) : whole ? tiled(m, batch, 5.0f, 0.48f, 0.87f, 0.82f) : tiled(m, batch, 7.7f, 0.46f, 1.24f, 0.92f);
+        }
+    }
+    if (depth_parts(true, m, k, n, batch, 1, 1, aT, &t.copied) > 1) {
+        t.copied += 3.0f + mb;
+    } else {
+        const int64_t apart = n > 128 && m > 128 ? ceil_div(n, 256) * ceil_div(m, 256) * batch : 0;
+        const bool join = batch > 1 && (!aT || n % 8 == 0) && cols_join(batch, m, (int64_t)k * 2) && cols_join_pays_f16(n, m, k, aT, batch, apart);
+        const int64_t width = join ? (int64_t)m * batch : m, entries = join ? 1 : batch;
+        t.copied = 2.0f * mb + (aT ? tiled(width, entries, 10.1f, 0.44f, 0.8f, 0.84f) : whole ? tiled(width, entries, 7.0f, 0.5f, 0.81f, 0.65f)
+                                                                                       : tiled(width, entries, 7.8f, 0.46f, 1.08f, 1.03f));
+    }
+    return t;
+}
+
+// Whether the copy pays (columns x entries x k beside rows, direct / with the copy, us: 24 x 1 x 4480 beside 1028 18.3 / 20.0; 12 x 5 x 1920 beside 3496 21 / 13;
+// 108 x 1 x 640 beside 1452 7.8 / 12.2; 124 x 4 x 1152 beside 4224 26 / 19).  Over the 700 products the choice is 0.8 % behind the better
+// form of each, always copying 18 %, never 16 %.  Rows of 4j + 2 columns stay as they are: they are not joined (81 products, 0.6 % behind).
+static bool copy_pays(int32_t n, int32_t k, int32_t m, int32_t batch, int aT) {
+    if (m >= 512 || m % 4 != 0 || k < 256 || n < 128 || (int64_t)m * batch * k >= 1ll << 30) return false;
+    const CopyTimes t = copy_times(n, k, m, batch, aT);
+    return t.copied < 0.95f * t.direct;
+}
+
+// The time of one product of two operands stored (K, rows), by the form that copy_pays and depth_parts choose
+float krows_time(int32_t m, int32_t k, int32_t n) {
+    const CopyTimes t = copy_times(n, k, m, 1, 1);
+    return copy_pays(n, k, m, 1, 1) ? t.copied : t.direct;
 }
 
 }  // namespace cpmk

@@ -1313,4 +1313,9 @@ static bool cols_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int 
     return g.fewer();
 }
 
+// gemm_parts.hip: parts that the depth of a product is divided into, 1 if it runs whole, else the time by its estimate in us as well; and that of one fp16 product of
+// two operands stored (K, rows)
+int32_t depth_parts(bool f16, int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, float* time = nullptr);
+float krows_time(int32_t m, int32_t k, int32_t n);
+
 }  // namespace cpmk

@@ -384,8 +384,8 @@ int gemv_f16_mfma(int32_t batch, int32_t dim_out, int32_t dim_in, const void* ma
 int gemm_f16_short(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, const void* A, const void* B, void* out, hipStream_t st);
 // ... of a depth up to 80 in rows off cache lines (gemm_rows.hip): 0, an error code, or -1 (shape not taken)
 int gemm_f16_rows(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, const void* A, const void* B, void* out, hipStream_t st);
-// ... of any size, layout and alignment (gemm_any.hip): 0 or an error code
-int gemm_f16_any(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, const void* A, const void* B, void* out, hipStream_t st);
+// ... of any size, layout and alignment (gemm_any.hip), fp32 out with f32: 0 or an error code
+int gemm_f16_any(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, const void* A, const void* B, void* out, hipStream_t st, bool f32 = false);
 // ... of up to 64 rows beside an operand stored (K, rows) (gemm_low.hip): 0, an error code, or -1 (shape not taken)
 int gemm_f16_low(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, const void* A, const void* B, void* out, hipStream_t st);
 

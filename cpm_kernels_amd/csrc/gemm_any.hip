@@ -15,7 +15,7 @@ namespace cpmk {
 
 struct AnyArgs {
     const half_t *P, *Q;           // a stride of 0 for one entry shared by the batch
-    half_t* out;                   // (batch, n, m)
+    void* out;                     // (batch, n, m), fp16 or fp32
     int64_t strideP, strideQ;      // elements
     int32_t n, m, k;
     uint32_t tiles_r, tiles_c, tiles, first;      // tiles of a launch, number of its first one
@@ -100,7 +100,8 @@ struct AnySlab {
     }
 };
 
-template <bool PT, bool QT, int TR, int TC>
+// F32: the sums as they are, straight from the registers (parts of a sum that is not rounded yet, gemm_sum.hip).
+template <bool PT, bool QT, int TR, int TC, bool F32 = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TR * TC > 8192 ? 3 : 4))) void k_gemm_any(AnyArgs a) {
     constexpr int WC = TR == 128 ? 2 : 4;                         // waves side by side; each has 64 rows x TC / WC columns
     constexpr int NJ = TC / WC / 16;
@@ -152,6 +153,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TR * TC > 8
                 for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fq[j], fp[i], acc[i][j], 0, 0, 0);
         }
     }
+    if constexpr (F32) {
+        struct __attribute__((packed, aligned(8))) Float4Pairs { float4_t v; };      // (m is even)
+        struct __attribute__((packed, aligned(8))) Float2 { float x, y; };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int32_t row = j0 + wr * 64 + i * 16 + r16;
+            if (row >= a.n) continue;
+            float* const dst = static_cast<float*>(a.out) + ((int64_t)b * a.n + row) * a.m;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int32_t col = i0 + (wc * NJ + j) * 16 + q * 4;
+                if (col + 4 <= a.m) reinterpret_cast<Float4Pairs*>(dst + col)->v = acc[i][j];
+                else if (col < a.m) *reinterpret_cast<Float2*>(dst + col) = Float2{acc[i][j][0], acc[i][j][1]};
+            }
+        }
+        return;
+    }
     __syncthreads();
     // Lane l, register e of a 16 x 16 result: output row l % 16, column (l / 16) * 4 + e.  The tile is put together in LDS, piece p of
     // row r at p ^ (r % 8), and leaves in whole rows.
@@ -169,7 +187,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TR * TC > 8
     __syncthreads();
     const int oc = tid % PPO;
     const int32_t left = a.m - i0 - oc * 8;
-    half_t* const ob = a.out + ((int64_t)b * a.n + j0) * a.m + i0 + oc * 8;
+    half_t* const ob = static_cast<half_t*>(a.out) + ((int64_t)b * a.n + j0) * a.m + i0 + oc * 8;
 #pragma unroll
     for (int r = tid / PPO; r < TR; r += 256 / PPO) {
         if (j0 + r >= a.n || left <= 0) continue;
@@ -180,10 +198,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TR * TC > 8
     }
 }
 
-// 0 or an error code.  A (batchA, k, m) [(batchA, m, k) if aT], B (batchB, n, k) [(batchB, k, n) if bT], out (batch, n, m).
-int gemm_f16_any(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, const void* A, const void* B, void* out, hipStream_t st) {
+// 0 or an error code.  A (batchA, k, m) [(batchA, m, k) if aT], B (batchB, n, k) [(batchB, k, n) if bT], out (batch, n, m); f32 (operands stored (K, rows)): fp32 out.
+int gemm_f16_any(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB, int aT, int bT, const void* A, const void* B, void* out, hipStream_t st, bool f32) {
     AnyArgs a;
-    a.P = (const half_t*)B; a.Q = (const half_t*)A; a.out = (half_t*)out;
+    a.P = (const half_t*)B; a.Q = (const half_t*)A; a.out = out;
     a.strideP = batchB == 1 ? 0 : (int64_t)n * k;
     a.strideQ = batchA == 1 ? 0 : (int64_t)m * k;
     a.n = n; a.m = m; a.k = k;
@@ -200,13 +218,14 @@ int gemm_f16_any(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batchB
         a.first = (uint32_t)t0;
         a.tiles = (uint32_t)(total - t0 < 1 << 23 ? total - t0 : 1 << 23);
         auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(a.tiles), dim3(256), 0, st, a); };
-        auto pick = [&](auto pt, auto qt) {
-            constexpr bool PT = decltype(pt)::value, QT = decltype(qt)::value;
-            if (wr) wc ? go(k_gemm_any<PT, QT, 128, 128>) : go(k_gemm_any<PT, QT, 128, 64>);
-            else wc ? go(k_gemm_any<PT, QT, 64, 128>) : go(k_gemm_any<PT, QT, 64, 64>);
+        auto pick = [&](auto pt, auto qt, auto fc) {
+            constexpr bool PT = decltype(pt)::value, QT = decltype(qt)::value, F = decltype(fc)::value;
+            if (wr) wc ? go(k_gemm_any<PT, QT, 128, 128, F>) : go(k_gemm_any<PT, QT, 128, 64, F>);
+            else wc ? go(k_gemm_any<PT, QT, 64, 128, F>) : go(k_gemm_any<PT, QT, 64, 64, F>);
         };
-        if (!bT) aT ? pick(std::false_type{}, std::false_type{}) : pick(std::false_type{}, std::true_type{});
-        else aT ? pick(std::true_type{}, std::false_type{}) : pick(std::true_type{}, std::true_type{});
+        if (f32) pick(std::true_type{}, std::true_type{}, std::true_type{});
+        else if (!bT) aT ? pick(std::false_type{}, std::false_type{}, std::false_type{}) : pick(std::false_type{}, std::true_type{}, std::false_type{});
+        else aT ? pick(std::true_type{}, std::false_type{}, std::false_type{}) : pick(std::true_type{}, std::true_type{}, std::false_type{});
         if (const int e = launch_status()) return e;
     }
     return 0;

@@ -57,27 +57,69 @@ static int32_t sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t
     return k <= limit ? g : batch;
 }
 
-// The quickest number of groups, whether it fills the device or not.  Up to 512 tiles of 128 x 128 the least of these estimates, in us, over the numbers of groups (int8, fp16 K-major; within 15 % of 130 sizes of
-// 16 to 432 tiles, 2 to 16 entries and depths of 40 to 1024).  A group: 4.5, and for each of its entries 0.40 and 0.45 a slab of 128 bytes (int8: folding,
-// products), or 0.65 a slab (fp16; depths that are not whole ones 0.7 and 0.26 a 64-byte slab, 2.0 and 0.30 where rows are not whole 16-byte
-// pieces), half as much again where int8 tiles share compute units, a round of the device after the other for fp16; several groups 3 and their
-// fp32 sums at 4.7 TB/s.  One by one: 12 (9), results written and read at 5.2 TB/s and products at 4.4 (2.0) PFLOP/s, which large tiles reach half under the writes.
-// Groups / one by one: int8 512 x 512 x 2, k = 128 7 / 16; x 13, 128 15 / 22; 832 x 1856 x 7, 128 11 / 23; x 16, 512 30 (two groups) / 39;
+// Products of up to 512 tiles of 128 x 128 (fp16: of too few large ones): the number of groups of the least of these estimates, in us, whether it fills the device or
+// not.  Fitted to 900 sizes of 4 to 4096 a side, 2 to 64 entries and depths of 32 to 2048; the choice over the best number for each as a geometric mean, int8
+// 1.017, fp16 K-major 1.012 (23 of 271 and 15 of 317 more than a tenth slower than the best; the lines above, which ask for a tile a compute unit, 1.05 and 1.06).
+// Groups / one by one: int8 512 x 512 x 2, k = 128 7 / 16; x 13, 128 15 / 22; 832 x 1856 x 7, 128 11 / 23; x 16, 512 30 (two groups) / 39; 384 x 64 x 5, 256 11.7 / 9.5 (the
+// second launch costs the host more);
 // fp16 1280 x 3328 x 14, k = 48 28 / 54; 512 x 512 x 6, 512 36 / 14 (one by one).
-static int32_t sum_groups_few(bool i8, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch) {
-    const int64_t cus = compute_units();
+// One by one: entries of at least half a round of the device's two tiles a compute unit, and no less than results written and read at 5.2 TB/s and products at
+// 4.4 (2.0) PFLOP/s take.
+static float sum_apart_time(bool i8, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch) {
+    const float rounds = (float)(tiles * batch) / (float)(2 * compute_units()), slabs = (float)ceil_div((int64_t)k * (i8 ? 1 : 2), 128), out = (float)batch * (float)n * (float)m * 1e-6f;
+    const float part = rounds > 1.0f ? (i8 ? 0.69f : 0.91f) * rounds : (i8 ? 0.67f : 0.73f) * (rounds > 0.5f ? rounds : 0.5f);
+    const float t = (i8 ? 9.1f : 9.4f) + slabs * part + (i8 ? 0.16f : 0.35f) * out + (i8 ? 7.8f : 5.4f) * rounds;
+    const float least = (i8 ? 12.0f : 9.0f) + out * (4.0f / 5.2f + 2.0f * (float)k / (i8 ? 4400.0f : 2000.0f));
+    return t > least ? t : least;
+}
+// A group: 4.5, and for each of its entries 0.40 and 0.45 a slab of 128 bytes (int8: folding, products), or 0.65 a slab (fp16; depths that are not whole
+// ones 0.7 and 0.26 a 64-byte slab, 2.0 and 0.30 where rows are not whole 16-byte pieces), half as much again where int8 tiles share compute units, a round of the
+// device after the other for fp16; several groups 3 and their fp32 sums at 4.7 TB/s.
+static float sum_group_time(bool i8, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch, int32_t g) {
+    const int64_t cus = compute_units(), work = tiles * g, last = work % cus;
     const float area = (float)n * (float)m * 1e-6f, kb = (float)(i8 ? k : 2 * k);
     const bool slabs = i8 || k % 64 == 0;
     const float entry = i8 ? 0.40f + 0.45f * ceilf(kb / 128.0f) : slabs ? 0.65f * kb / 128.0f : k % 8 == 0 ? 0.7f + 0.26f * floorf(kb / 64.0f) : 2.0f + 0.30f * floorf(kb / 64.0f);
-    int32_t best = batch;
-    float best_t = (i8 ? 12.0f : 9.0f) + (float)batch * area * (4.0f / 5.2f + 2.0f * (float)k / (i8 ? 4400.0f : 2000.0f));
-    for (int32_t g = 1; g < batch && g * tiles <= 4 * cus; ++g) {
-        if (batch % g != 0 || batch / g > kSumMax) continue;
-        const int64_t work = tiles * g, last = work % cus;
-        float rounds;
-        if (i8) rounds = work <= cus ? 1.0f : 1.5f * (float)ceil_div(work, 2 * cus);
-        else rounds = (float)(work / cus) + (last == 0 ? 0.0f : 2 * last <= cus && work > cus && slabs ? 0.5f : 1.0f);
-        const float t = 4.5f + rounds * (float)(batch / g) * entry + (g > 1 ? 3.0f + (float)g * area * 8.0f / 4.7f : 0.0f);
+    float rounds;
+    if (i8) rounds = work <= cus ? 1.0f : 1.5f * (float)ceil_div(work, 2 * cus);
+    else rounds = (float)(work / cus) + (last == 0 ? 0.0f : 2 * last <= cus && work > cus && slabs ? 0.5f : 1.0f);
+    return 4.5f + rounds * (float)(batch / g) * entry + (g > 1 ? 3.0f + (float)g * area * 8.0f / 4.7f : 0.0f);
+}
+
+// (K, rows): whether the tile kernel takes the groups (gemm_rows_parts), else the kernel for any size does
+static bool krows_tiles(int32_t m, int64_t depth, int32_t n) { return depth >= 64 && (n % 8 == 0 || n >= 128) && (m % 8 == 0 || m >= 256); }
+// The entries of a group are one contraction of operands below 4 GiB; one group's is a product like any other (krows_time), whose depth may be divided.
+static float sum_krows_time(int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch, int32_t g) {
+    const int64_t depth = (int64_t)k * (batch / g), cus = compute_units();
+    if ((m > n ? m : n) * depth >= 1ll << 31) return 1e30f;
+    if (g == 1) return krows_time(m, (int32_t)depth, n);
+    const float slabs = (float)ceil_div(depth, 64), add = 3.0f + (float)g * (float)n * (float)m * 8e-6f / 4.7f;
+    if (krows_tiles(m, depth, n)) {
+        const float rounds = (float)(tiles * g) / (float)cus;
+        return 4.5f + add + slabs * (depth % 64 == 0 ? 0.47f : 0.55f) * (rounds <= 1.0f ? 1.0f : rounds <= 2.0f ? 2.05f : 1.15f * rounds);
+    }
+    const float rounds = (float)(ceil_div(n, 64) * ceil_div(m, 64) * g) / (float)cus;
+    return 2.6f + add + slabs * (rounds <= 1.0f ? 0.58f : rounds <= 4.0f ? 1.1f : 0.29f * rounds);
+}
+static bool sum_few_tiles(int kind, int32_t m, int32_t n) {
+    const int64_t cus = compute_units();
+    return ceil_div(n, 128) * ceil_div(m, 128) <= 2 * cus && (kind == kSumI8 || ceil_div(n, 256) * ceil_div(m, 256) * 4 < cus * 3);
+}
+
+// (K, rows): groups, the batch's entries one by one among them, whose sums stay fp32; 0: one by one, rounded, from the depths on where that is the quicker.  One contraction
+// of all entries whatever its depth had left a few tiles with one slab after another: 8 x 44 outputs, 26 entries of k = 128 30.8 us, 28 x 8 x 24, 980 200 us; as the 26 and the 24
+// groups of one entry 6.5 and 13.8 (one by one 9.9 and 17.1); 136 x 890 x 49, 128 50 us, seven groups 17.0 (20.7); 1644 x 2132 x 10, 512 in one 54 (75)
+static int32_t sum_krows_groups(int32_t m, int32_t k, int32_t n, int32_t batch) {
+    const int64_t cus = compute_units(), tiles = ceil_div(n, 128) * ceil_div(m, 128);
+    if (!sum_few_tiles(kSumF16KFirst, m, n) || k > (tiles > cus ? 640 : 1023)) {
+        const int32_t g = sum_groups_for(kSumF16KFirst, m, k, n, batch);
+        return g == batch && batch > 1 ? 0 : g;
+    }
+    int32_t best = 0;
+    float best_t = 1e30f;
+    for (int32_t g = 1; g <= batch && (g == 1 || g * tiles <= 4 * cus); ++g) {
+        if (batch % g != 0) continue;
+        const float t = sum_krows_time(tiles, m, k, n, batch, g);
         if (t < best_t) {
             best_t = t;
             best = g;
@@ -86,16 +128,24 @@ static int32_t sum_groups_few(bool i8, int64_t tiles, int32_t m, int32_t k, int3
     return best;
 }
 
-// (K, rows): one contraction of all entries where it fits, whose depth is divided among workgroups again where it has few tiles
-// (cpmk_gemm_depth_parts).  Joined / one by one: 1280 x 3328 x 7, k = 100 14 / 32, 1024 86 / 78; 832 x 1856 x 14, 48 10.7 / 26; x 2, 1024 20.6 / 19.3;
-// 512 x 512 x 16, 512 19.3 / 18.4, x 3, 40 8.2 / 13.0.
 static int32_t sum_groups_timed(int kind, int32_t m, int32_t k, int32_t n, int32_t batch) {
     const int64_t cus = compute_units(), tiles = ceil_div(n, 128) * ceil_div(m, 128);
-    if (kind == kSumI8 ? tiles <= 2 * cus : ceil_div(n, 256) * ceil_div(m, 256) * 4 < cus * 3 && tiles <= 2 * cus) {
-        if (kind != kSumF16KFirst) return sum_groups_few(kind == kSumI8, tiles, m, k, n, batch);
-        if ((int64_t)(m > n ? m : n) * k < (1ll << 31) / batch && k <= (tiles > cus ? 640 : 1023)) return 1;
+    if (kind == kSumF16KFirst) {
+        const int32_t g = sum_krows_groups(m, k, n, batch);
+        return g == 0 ? batch : g;
     }
-    return sum_groups_for(kind, m, k, n, batch);
+    if (!sum_few_tiles(kind, m, n)) return sum_groups_for(kind, m, k, n, batch);
+    int32_t best = batch;
+    float best_t = sum_apart_time(kind == kSumI8, tiles, m, k, n, batch);
+    for (int32_t g = 1; g < batch && g * tiles <= 4 * cus; ++g) {
+        if (batch % g != 0 || batch / g > kSumMax) continue;
+        const float t = sum_group_time(kind == kSumI8, tiles, m, k, n, batch, g);
+        if (t < best_t) {
+            best_t = t;
+            best = g;
+        }
+    }
+    return best;
 }
 
 // PART: fp32 out.  A group's sum may pass fp16's range where the sum over all groups does not: sums of more than one group stay
@@ -147,15 +197,17 @@ static int gemm_sum_dispatch(bool f16, int32_t m, int32_t k, int32_t n, int32_t 
 }
 
 // fp16 products whose operands are both stored (K, rows): the entries of a group lie one behind the other and are one
-// contraction of `k` (all of them together) as they lie.  The tile kernel's part of gemm_f16_dispatch, fp32 out.
-static int gemm_rows_parts(int32_t m, int64_t k, int32_t n, int32_t groups, const void* A, const void* B, void* out, hipStream_t st) {
+// contraction of `k` (all of them together) as they lie.  The tile kernel's part of gemm_f16_dispatch, fp32 out; `any`: what it does not take on the kernel for any size.
+static int gemm_rows_parts(int32_t m, int64_t k, int32_t n, int32_t groups, const void* A, const void* B, void* out, bool any, hipStream_t st) {
     if (m < 0 || n < 0 || k < 0 || groups < 1) return CPMK_EBADARG;
     if (m % 2 || n % 2 || k % 2) return CPMK_EALIGN;
     if (m == 0 || n == 0) return 0;
     if (any_null(A, B, out)) return CPMK_EBADARG;
     if (n * k * 2 >= (1ll << 32) || m * k * 2 >= (1ll << 32)) return CPMK_ETOOBIG;
     const bool in_p = n % 8 != 0, in_q = m % 8 != 0;
-    if (k < 64 || (in_p && n < 128) || (in_q && m < 256) || !aligned16(A) || !aligned16(B) || !aligned16(out)) return CPMK_EALIGN;
+    if (!aligned16(out)) return CPMK_EALIGN;
+    if (!krows_tiles(m, k, n) || !aligned16(A) || !aligned16(B))
+        return any ? gemm_f16_any(m, (int32_t)k, n, groups, groups, 0, 1, A, B, out, st, true) : CPMK_EALIGN;
     GemmArgs a = {};
     a.P = (const int8_t*)B; a.Q = (const int8_t*)A; a.out = out;
     a.srow = nullptr; a.scol = nullptr;
@@ -231,6 +283,10 @@ int cpmk_gemm_sum_groups_timed(int kind, int32_t m, int32_t k, int32_t n, int32_
     return m <= 0 || n <= 0 || k <= 0 || batch < 1 ? 1 : sum_groups_timed(kind, m, k, n, batch);
 }
 
+int cpmk_gemm_sum_krows_groups(int32_t m, int32_t k, int32_t n, int32_t batch) {
+    return m <= 0 || n <= 0 || k <= 0 || batch < 1 ? 0 : sum_krows_groups(m, k, n, batch);
+}
+
 int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                              const void* scale_row, void* out, void* stream) {
     clear_stale_error();
@@ -254,7 +310,7 @@ int cpmk_gemm_fp16_parts(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t
     clear_stale_error();
     if (!k_first) return gemm_sum_dispatch<true>(true, m, k, n, batch, groups, A, B, nullptr, parts, (hipStream_t)stream);
     if (k < 0 || batch < 1 || groups < 1 || batch % groups) return CPMK_EBADARG;
-    return gemm_rows_parts(m, (int64_t)k * (batch / groups), n, groups, A, B, parts, (hipStream_t)stream);
+    return gemm_rows_parts(m, (int64_t)k * (batch / groups), n, groups, A, B, parts, k_first == 2, (hipStream_t)stream);
 }
 
 int cpmk_gemm_add_parts(int32_t groups, int64_t n, const void* parts, void* out, void* stream) {

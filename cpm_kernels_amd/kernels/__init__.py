@@ -10,7 +10,7 @@ from .gelu import gelu_forward, gelu_backward, gelu_inplace_forward
 from .gemm import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, gemm_scale, \
     gemm_fp16, gemm_int8, gemm_backward_round_scale, gemm_backward_scale_round, gemm_scale_x, gemm_scale_y, \
     gemm_int8_scale, gemm_quantize, gemm_quantize_cols, gemm_quantize_pair, \
-    gemm_int8_scale_one, gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_backward_round_scale_ld, gemm_sum_groups, gemm_sum_groups_for, gemm_sum_groups_timed, \
+    gemm_int8_scale_one, gemm_quantize_cols_ld, gemm_quantize_pair_ld, gemm_backward_round_scale_ld, gemm_sum_groups, gemm_sum_groups_for, gemm_sum_groups_timed, gemm_sum_krows_groups, \
     gemm_int8_scale_sum, gemm_fp16_sum, gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, \
     gemm_depth_parts, gemm_fp16_copy_pays, gemm_int8_scale_split, gemm_fp16_split, gemm_quantize_cols_rows, gemm_backward_quantize_both
 from .gemv import gemv_fp16, gemv_broadcast_mat_int8, gemv_fp16_transpose, gemv_broadcast_mat_fp16, \

@@ -207,6 +207,11 @@ def gemm_sum_groups(m: int, n: int, batch: int) -> int:
     return cpmk.gemm_sum_groups(m, n, batch)
 
 
+def gemm_sum_krows_groups(m: int, k: int, n: int, batch: int) -> int:
+    """Groups (up to the batch) for gemm_fp16_parts with k_first, 0 where one product per entry and the sum of them is the quicker."""
+    return cpmk.gemm_sum_krows_groups(m, k, n, batch)
+
+
 def gemm_sum_groups_for(kind: int, m: int, k: int, n: int, batch: int) -> int:
     """The same for a depth of k an entry, or `batch` where one product per entry and the sum of them is the quicker.
     kind 0: gemm_int8_scale_sum, 1: gemm_fp16_sum, 2: gemm_fp16_parts with k_first."""
@@ -249,14 +254,14 @@ def gemm_int8_scale_parts(m: int, k: int, n: int, batch: int, groups: int,
     cpmk.gemm_int8_scale_parts(m, k, n, batch, groups, A, B, scale_row, parts, stream)
 
 
-def gemm_fp16_parts(m: int, k: int, n: int, batch: int, groups: int, k_first: bool,
+def gemm_fp16_parts(m: int, k: int, n: int, batch: int, groups: int, k_first: int,
                     A: DevicePointer,         # (batch, m, k)     fp16   [(batch, k, m) if k_first]
                     B: DevicePointer,         # (batch, n, k)     fp16   [(batch, k, n) if k_first]
                     parts: DevicePointer,     # (groups, n, m)    fp32
                     stream: CUDAStream):
-    """gemm_fp16_sum with the groups' sums as fp32, for gemm_add_parts."""
+    """gemm_fp16_sum with the groups' sums as fp32, for gemm_add_parts.  k_first 2: any sizes and addresses."""
     assert m % 2 == 0 and n % 2 == 0 and k % 2 == 0
-    cpmk.gemm_fp16_parts(m, k, n, batch, groups, 1 if k_first else 0, A, B, parts, stream)
+    cpmk.gemm_fp16_parts(m, k, n, batch, groups, int(k_first), A, B, parts, stream)
 
 
 def gemm_add_parts(groups: int, n: int,

@@ -47,7 +47,7 @@ _CTYPES = {"i": ctypes.c_int32, "l": ctypes.c_int64, "f": ctypes.c_float, "p": c
 
 EXPORTED_SYMBOLS = sorted(["cpmk_" + n for n in _LAUNCHERS] + [
     "cpmk_version", "cpmk_error_string", "cpmk_device_count", "cpmk_get_device",
-    "cpmk_set_device", "cpmk_device_props", "cpmk_exchange_capture_slots_left", "cpmk_gemm_sum_groups", "cpmk_gemm_sum_groups_for",
+    "cpmk_set_device", "cpmk_device_props", "cpmk_exchange_capture_slots_left", "cpmk_gemm_sum_groups", "cpmk_gemm_sum_groups_for", "cpmk_gemm_sum_krows_groups",
     "cpmk_gemm_sum_groups_timed",
     "cpmk_gemm_depth_parts", "cpmk_gemm_fp16_copy_pays",
 ])
@@ -123,6 +123,11 @@ def exchange_capture_slots_left() -> int:
 @lib.bind("cpmk_gemm_sum_groups", [ctypes.c_int32] * 3, ctypes.c_int32)
 def gemm_sum_groups(m: int, n: int, batch: int) -> int:
     return lib.cpmk_gemm_sum_groups(m, n, batch)
+
+
+@lib.bind("cpmk_gemm_sum_krows_groups", [ctypes.c_int32] * 4, ctypes.c_int32)
+def gemm_sum_krows_groups(m: int, k: int, n: int, batch: int) -> int:
+    return lib.cpmk_gemm_sum_krows_groups(m, k, n, batch)
 
 
 @lib.bind("cpmk_gemm_sum_groups_for", [ctypes.c_int] + [ctypes.c_int32] * 4, ctypes.c_int32)

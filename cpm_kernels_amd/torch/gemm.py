@@ -9,7 +9,7 @@ the six-launch sequence, which ``fused=False`` still runs through the kernel-lev
 import torch
 from ..kernels import gemm_calc_scale, gemm_calc_scale_transpose, gemm_round, gemm_round_transpose, \
     gemm_scale, gemm_scale_x, gemm_scale_y, gemm_int8, gemm_int8_scale_one, gemm_quantize, \
-    gemm_quantize_cols_ld, gemm_quantize_cols_rows, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_timed, gemm_int8_scale_sum, gemm_fp16_sum, \
+    gemm_quantize_cols_ld, gemm_quantize_cols_rows, gemm_quantize_pair_ld, gemm_fp16, gemm_sum_groups_timed, gemm_sum_krows_groups, gemm_int8_scale_sum, gemm_fp16_sum, \
     gemm_int8_scale_parts, gemm_fp16_parts, gemm_add_parts, gemm_depth_parts, gemm_fp16_copy_pays, gemm_int8_scale_split, gemm_fp16_split, \
     arith_batch_add_backward, gemm_backward_round_scale, gemm_backward_round_scale_ld, gemm_backward_quantize_both, gemm_backward_scale_round, transpose, \
     transpose_i8_ld
@@ -379,17 +379,16 @@ def gemm_pth_fp16_sum(A: torch.Tensor, aT: bool, B: torch.Tensor, bT: bool) -> t
     """The same product summed over the batch, (1, M, N)."""
     M, K, N = _dims(A, B, aT, bT)
     batch = A.size(0)
-    groups = _entry_groups(M, K, N, batch, aT and not bT) if batch == B.size(0) else batch
-    if groups < batch and aT and not bT:
+    joined = aT and not bT
+    groups = batch if batch != B.size(0) else gemm_sum_krows_groups(N, K, M, batch) if joined else _entry_groups(M, K, N, batch, False)
+    if joined and groups and batch == B.size(0):
         # both operands stored (K, rows): the entries of a group are one longer contraction as they lie
-        depth = batch // groups * K
         if groups == 1:
-            return gemm_pth_fp16(A.view(1, depth, M), True, B.view(1, depth, N), False)
-        if (M % 8 == 0 or M >= 128) and (N % 8 == 0 or N >= 256) and depth >= 64 and (A.data_ptr() | B.data_ptr()) % 16 == 0:
-            parts = torch.empty((groups, M, N), dtype=torch.float32, device=A.device)
-            gemm_fp16_parts(N, K, M, batch, groups, True, B.data_ptr(), A.data_ptr(), parts.data_ptr(), cur_stream())
-            return _add_parts(parts)
-    elif groups < batch and not aT and bT and M % 4 == 0 and N % 4 == 0 and K > 32 and max(M, N) * K < 2 ** 31 and \
+            return gemm_pth_fp16(A.view(1, batch * K, M), True, B.view(1, batch * K, N), False)
+        parts = torch.empty((groups, M, N), dtype=torch.float32, device=A.device)
+        gemm_fp16_parts(N, K, M, batch, groups, 2, B.data_ptr(), A.data_ptr(), parts.data_ptr(), cur_stream())
+        return _add_parts(parts)
+    if groups < batch and not aT and bT and M % 4 == 0 and N % 4 == 0 and K > 32 and max(M, N) * K < 2 ** 31 and \
             batch * K < 2 ** 21 and (A.data_ptr() | B.data_ptr()) % 4 == 0:
         if groups == 1:
             out = torch.empty((1, M, N), dtype=torch.half, device=A.device)

@@ -206,6 +206,8 @@ int cpmk_gemm_fp16(int32_t m, int32_t k, int32_t n, int32_t batchA, int32_t batc
 int cpmk_gemm_sum_groups(int32_t m, int32_t n, int32_t batch);
 /* cpmk_gemm_sum_groups_timed: the quickest number of groups, whether they fill the device or not. */
 int cpmk_gemm_sum_groups_timed(int kind, int32_t m, int32_t k, int32_t n, int32_t batch);
+/* cpmk_gemm_sum_krows_groups: kind 2, groups (up to the batch) for cpmk_gemm_fp16_parts, 0 where one product per entry and the sum of them is the quicker. */
+int cpmk_gemm_sum_krows_groups(int32_t m, int32_t k, int32_t n, int32_t batch);
 int cpmk_gemm_sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t batch);
 int cpmk_gemm_int8_scale_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                              const void* scale_row, void* out, void* stream);
@@ -213,7 +215,8 @@ int cpmk_gemm_fp16_sum(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t g
                        void* out, void* stream);
 /* The same with the groups' sums as fp32, parts (groups, n, m): a group's sum may pass fp16's range where the whole sum does not.
  * fp16 with k_first: operands stored A (batch, k, m) and B (batch, k, n), m, n and k even, any number of entries a group; k of a group's
- * entries together at least 64, m a multiple of 8 or at least 256, n a multiple of 8 or at least 128, buffers on 16-byte boundaries.
+ * entries together at least 64, m a multiple of 8 or at least 256, n a multiple of 8 or at least 128, buffers on 16-byte boundaries;
+ * k_first 2: any such sizes and operands at any address.
  * cpmk_gemm_add_parts: out[j] = fp16(sum over g of parts[g, j]), in the order of the groups; n a multiple of 4. */
 int cpmk_gemm_int8_scale_parts(int32_t m, int32_t k, int32_t n, int32_t batch, int32_t groups, const void* A, const void* B,
                                const void* scale_row, void* parts, void* stream);

@@ -134,6 +134,42 @@ def test_fp16_parts(gpu, shape, k_first, k):
         _check_add(parts)
 
 
+# (edges of the kernel for any size: rows of half pieces and of 4j + 2 elements, less than a tile, past one, several tiles of each width, operands off
+# 16-byte boundaries; depths of a slab and less, a rest, many slabs; as many groups as entries)
+@pytest.mark.parametrize("k", [2, 62, 64, 250])
+@pytest.mark.parametrize("shape", [(6, 6, 8, 44), (4, 2, 6, 2), (9, 3, 66, 130), (20, 20, 126, 1030), (6, 2, 1002, 62), (300, 150, 4, 132), (6, 3, 260, 252)])
+@pytest.mark.parametrize("at", [0, 1])
+def test_fp16_parts_of_any_size(gpu, shape, k, at):
+    batch, groups, n, m = shape
+    print("fp16 parts of any size", shape, k, at, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n * 7 + m + k)
+
+    def operand(rows):
+        flat = torch.randn(batch * k * rows + at, generator=g, device="cuda").mul_(8).half()
+        return flat[at:].view(batch, k, rows)
+    A, B = operand(m), operand(n)
+    parts = torch.full((groups, n, m), float("nan"), device="cuda")
+    ck.gemm_fp16_parts(m, k, n, batch, groups, 2, A.data_ptr(), B.data_ptr(), parts.data_ptr(), _st())
+    p, q, per = B.double().transpose(1, 2).contiguous(), A.double(), batch // groups
+    want, mag = (torch.stack([x[i] @ y[i] for i in range(batch)]).view(groups, per, n, m).sum(1) for x, y in ((p, q), (p.abs(), q.abs())))
+    assert bool(((parts.double() - want).abs() <= mag * (per * k) * 2.0 ** -24).all())      # fp32 sums in any order
+    _check_add(parts)
+
+
+@pytest.mark.parametrize("batch,k,m,n", [(26, 128, 44, 8), (49, 128, 890, 136), (24, 980, 8, 28), (33, 836, 768, 128), (7, 66, 132, 260), (16, 64, 1024, 512), (5, 1024, 12, 48)])
+def test_sum_of_krows_entries(gpu, batch, k, m, n):
+    """Weight gradients of operands stored (K, rows): groups of any number of entries, none that leaves one workgroup a depth of thousands; sums in fp32, rounded once"""
+    from cpm_kernels_amd.torch.gemm import gemm_pth_fp16_sum
+    print("sum of (K, rows) entries", batch, k, m, n, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n + m + k)
+    A, B = (torch.randn((batch, k, r), generator=g, device="cuda").half() for r in (n, m))
+    out = gemm_pth_fp16_sum(A, True, B, False).double()[0]
+    p, q = A.double().transpose(1, 2).contiguous(), B.double()
+    want, mag = (sum(x[i] @ y[i] for i in range(batch)) for x, y in ((p, q), (p.abs(), q.abs())))
+    each = sum((p[i] @ q[i]).abs() for i in range(batch)) * 2.0 ** -11 if ck.gemm_sum_krows_groups(m, k, n, batch) == 0 else 0      # (one by one: each entry's rounding)
+    assert bool(((out - want).abs() <= mag * (batch * k) * 2.0 ** -24 + each + want.abs() * 2.0 ** -10.9 + 2.0 ** -25).all())
+
+
 def _check_add(parts):
     groups, total = parts.size(0), parts[0].numel()
     out = torch.full(parts.shape[1:], float("nan"), device="cuda", dtype=torch.half)

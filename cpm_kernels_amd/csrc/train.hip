@@ -1194,9 +1194,10 @@ int cpmk_position_embedding_backward(int32_t query_len, int32_t key_len, int32_t
         const int64_t smem = (num_buckets + pieces * 15) * (int64_t)sizeof(float);
         // (a kernel for so little: by diagonals and element by element 114 heads of 1 x 3 4.0 and 2.0 us, 113 of 21 x 16 4.1 and 2.4, 14 of 444 x 5 4.4 and 5.6, 7 of
         // 200 x 30 3.4 and 11.5; rows of whole pieces 16 of 16 x 11 2.9 and 2.1, 95 of 8 x 55 3.6 and 2.6, 20 of 200 x 8 3.1 and 4.5, 74 of 16 x 49 3.6 and 3.1, 5 of 1344 x 1, as many
-        // diagonals, 5.9 and 4.0)
+        // diagonals, 5.9 and 4.0; of heads that share compute units 770 of 36 x 27 4.3 and 7.3, 1590 of 44 x 23 5.1 and 12.3, 304 of 8 x 13 3.8 both)
         const bool ua = query_len % 8 != 0 || !aligned16(grad_out);
-        const bool few = key_len <= 64 && (int64_t)query_len * key_len < (ua ? 1200 : 440) + ((int64_t)query_len + key_len) * 3 / 2 + key_len * 12;
+        const bool few = key_len <= 64 && (int64_t)query_len * key_len < (ua ? 1200 : 440) + ((int64_t)query_len + key_len) * 3 / 2 + key_len * 12 &&
+                         (num_heads <= compute_units() || (int64_t)num_heads * query_len * key_len <= 300000);
         const bool diag = smem <= 128 * 1024 && !few;
         if ((diag || key_len > 64) && (int64_t)num_heads * parts <= kXchSlots) {
             XchScope xs;

@@ -44,7 +44,7 @@ def test_softmax_backward_teams_in_several_launches():
 
 
 @pytest.mark.parametrize("bidirectional", [True, False])
-@pytest.mark.parametrize("ql,kl,heads", [(1, 1, 3), (7, 5, 4), (1344, 1, 5), (102, 10, 3), (102, 20, 3), (96, 6, 4), (96, 8, 4), (50, 64, 32), (64, 64, 2), (100, 65, 12), (333, 130, 5), (250, 250, 40), (1022, 1022, 15), (2050, 40, 3), (2050, 2050, 2)])
+@pytest.mark.parametrize("ql,kl,heads", [(1, 1, 3), (7, 5, 4), (1344, 1, 5), (102, 10, 3), (102, 20, 3), (96, 6, 4), (96, 8, 4), (50, 64, 32), (64, 64, 2), (36, 27, 770), (8, 13, 304), (100, 65, 12), (333, 130, 5), (250, 250, 40), (1022, 1022, 15), (2050, 40, 3), (2050, 2050, 2)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_position_bias_gradient(bidirectional, ql, kl, heads, shift):
     buckets, far = 32, 128

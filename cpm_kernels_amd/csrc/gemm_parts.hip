@@ -170,14 +170,17 @@ int32_t depth_parts(bool f16, int32_t m, int32_t k, int32_t n, int32_t batchA, i
 
 // fp16, a weight A (1, n, k) [(1, k, n) if aT] beside entries B (batch, k, m): estimates in us as above, of the product as it lies and with a copy of the
 // entries as (batch, m, k), which are joined to one product then and whose depth may be divided, where entries stored (K, rows) of less than a
-// tile, or of rows that are not whole 16-byte pieces, are a tile or more each, on the kernel for any size or on the tile kernel.  Fitted to 700 products of 4
+// tile, or of rows that are not whole 16-byte pieces, are a tile or more each, on the kernel for any size or on the tile kernel.  Fitted to 860 products of 4
 // to 508 columns, 1 to 24 entries and depths of 256 to 24000 beside 128 to 10240 rows, the most within 15 %.
 struct CopyTimes {
     float direct, copied;
 };
 static CopyTimes copy_times(int32_t n, int32_t k, int32_t m, int32_t batch, int aT) {
     const float cus = (float)compute_units(), slabs = (float)k / 64.0f, mb = 1e-6f * (float)k * (float)m * (float)batch;
-    auto tiled = [&](int64_t width, int64_t entries, float base, float one, float two, float many) {        // (tiles of up to a round, two, more of them)
+    // (a round of large tiles, or tiles of 128 x 128 of up to a round, two, more of them; `apart`: of joined entries, big_tiles)
+    auto tiled = [&](int64_t width, int64_t entries, int64_t apart, float base, float one, float two, float many, float large) {
+        if (large > 0.0f && n > 128 && width > 128 && big_tiles(n, (int32_t)width, (int)entries, apart) * 4 >= compute_units() * 3ll)
+            return (float)ceil_div(ceil_div(n, 256) * ceil_div(width, 256) * entries, compute_units()) * (slabs * large + 8.0f);
         const float rounds = (float)(ceil_div(n, 128) * ceil_div(width, 128) * entries) / cus;
         return base + slabs * (rounds <= 1.0f ? one : rounds <= 2.0f ? two : many * rounds);
     };
@@ -188,7 +191,9 @@ static CopyTimes copy_times(int32_t n, int32_t k, int32_t m, int32_t batch, int 
             const float rounds = (float)(ceil_div(n, 64) * ceil_div(m, 64) * batch) / cus;
             t.direct = 2.6f + slabs * (rounds <= 1.0f ? 0.58f : rounds <= 4.0f ? 1.1f : 0.29f * rounds);
         } else {
-            t.direct = aT ? tiled(m, batch, 4.8f, whole ? 0.49f : 0.58f, 0.8f, 0.86f) : whole ? tiled(m, batch, 5.0f, 0.48f, 0.87f, 0.82f) : tiled(m, batch, 7.7f, 0.46f, 1.24f, 0.92f);
+            const float large = m % 8 == 0 || m >= 256 ? 1.4f : 0.0f;
+            t.direct = aT ? tiled(m, batch, 0, 4.8f, whole ? 0.49f : 0.58f, 0.8f, 0.86f, large) : whole ? tiled(m, batch, 0, 5.0f, 0.48f, 0.87f, 0.82f, large)
+                                                                                                       : tiled(m, batch, 0, 7.7f, 0.46f, 1.24f, 0.92f, large);
         }
     }
     if (depth_parts(true, m, k, n, batch, 1, 1, aT, &t.copied) > 1) {
@@ -196,16 +201,16 @@ static CopyTimes copy_times(int32_t n, int32_t k, int32_t m, int32_t batch, int 
     } else {
         const int64_t apart = n > 128 && m > 128 ? ceil_div(n, 256) * ceil_div(m, 256) * batch : 0;
         const bool join = batch > 1 && (!aT || n % 8 == 0) && cols_join(batch, m, (int64_t)k * 2) && cols_join_pays_f16(n, m, k, aT, batch, apart);
-        const int64_t width = join ? (int64_t)m * batch : m, entries = join ? 1 : batch;
-        t.copied = 2.0f * mb + (aT ? tiled(width, entries, 10.1f, 0.44f, 0.8f, 0.84f) : whole ? tiled(width, entries, 7.0f, 0.5f, 0.81f, 0.65f)
-                                                                                       : tiled(width, entries, 7.8f, 0.46f, 1.08f, 1.03f));
+        const int64_t width = join ? (int64_t)m * batch : m, entries = join ? 1 : batch, big = join ? apart : 0;
+        t.copied = 2.0f * mb + (aT ? tiled(width, entries, big, 10.1f, 0.44f, 0.8f, 0.84f, 1.25f) : whole ? tiled(width, entries, big, 7.0f, 0.5f, 0.81f, 0.65f, 1.25f)
+                                                                                                        : tiled(width, entries, big, 7.8f, 0.46f, 1.08f, 1.03f, 1.25f));
     }
     return t;
 }
 
 // Whether the copy pays (columns x entries x k beside rows, direct / with the copy, us: 24 x 1 x 4480 beside 1028 18.3 / 20.0; 12 x 5 x 1920 beside 3496 21 / 13;
-// 108 x 1 x 640 beside 1452 7.8 / 12.2; 124 x 4 x 1152 beside 4224 26 / 19).  Over the 700 products the choice is 0.8 % behind the better
-// form of each, always copying 18 %, never 16 %.  Rows of 4j + 2 columns stay as they are: they are not joined (81 products, 0.6 % behind).
+// 108 x 1 x 640 beside 1452 7.8 / 12.2; 124 x 4 x 1152 beside 4224 26 / 19; 164 x 22 x 9344 beside 3072 392 / 225; 500 x 8 x 4096 beside 7996 220 / 223).  Over the 860 products the choice is 0.8 % behind
+// the better form of each, always copying 16 %, never 16 %.  Rows of 4j + 2 columns stay as they are: they are not joined (81 products, 0.6 % behind).
 static bool copy_pays(int32_t n, int32_t k, int32_t m, int32_t batch, int aT) {
     if (m >= 512 || m % 4 != 0 || k < 256 || n < 128 || (int64_t)m * batch * k >= 1ll << 30) return false;
     const CopyTimes t = copy_times(n, k, m, batch, aT);

@@ -70,7 +70,7 @@ static float sum_apart_time(bool i8, int64_t tiles, int32_t m, int32_t k, int32_
     const float part = rounds > 1.0f ? (i8 ? 0.69f : 0.91f) * rounds : (i8 ? 0.67f : 0.73f) * (rounds > 0.5f ? rounds : 0.5f);
     const float t = (i8 ? 9.1f : 9.4f) + slabs * part + (i8 ? 0.16f : 0.35f) * out + (i8 ? 7.8f : 5.4f) * rounds;
     const float least = (i8 ? 12.0f : 9.0f) + out * (4.0f / 5.2f + 2.0f * (float)k / (i8 ? 4400.0f : 2000.0f));
-    return t > least ? t : least;
+    return t > least && out * (float)k <= 75000.0f ? t : least;        // (the first is not fitted to more than 1.5e11 operations, where large tiles are quicker than it says)
 }
 // A group: 4.5, and for each of its entries 0.40 and 0.45 a slab of 128 bytes (int8: folding, products), or 0.65 a slab (fp16; depths that are not whole
 // ones 0.7 and 0.26 a 64-byte slab, 2.0 and 0.30 where rows are not whole 16-byte pieces), half as much again where int8 tiles share compute units, a round of the

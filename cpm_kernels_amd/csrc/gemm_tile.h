@@ -1273,9 +1273,9 @@ static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool 
 //   int8 columns    0.977, 273 worse         0.960, 4 worse                   0.958
 //   fp16 rows       1.043, 307 worse         0.976, 6 worse                   0.961
 //   fp16 columns    1.026, 335 worse         0.960, 3 worse                   0.958
-// Where the rounds stay and tiles are saved it pays too for K-major operands of enough whole slabs, fp16 rows of any depth from 1024 on (the same figures over those that the
-// rules below take): int8 rows 0.980, none of 103; fp16 rows 0.973, 2 of 120; int8 columns 0.964, 1 of 135; fp16 columns 0.948, none of 68; rows
-// from 1024 on where the tiles stay too, 0.985, none of 19 (47 entries of 128 x 1280 beside 832 26.2 -> 22.8 us)
+// Where the rounds stay and tiles are saved it pays too at enough depth of whole slabs (fp16 rows: any from 1024 on); the same figures over those that the rules below take:
+//   int8 rows 0.980, none of 103; fp16 rows 0.973, 2 of 120; int8 columns 0.964, 1 of 135; fp16 columns 0.948, none of 68, beside rows stored (K, rows) 0.944,
+//   none of 26; rows from 1024 on where the tiles stay too 0.985, none of 19 (47 entries of 128 x 1280 beside 832 26.2 -> 22.8 us)
 struct JoinGain {
     int64_t rounds, rounds_joined, tiles, tiles_joined;
     bool fewer() const { return rounds_joined < rounds; }
@@ -1297,7 +1297,7 @@ static bool rows_join_pays_f16(int32_t n, int32_t m, int32_t k, bool kmajor, int
 static bool cols_join_pays_f16(int32_t n, int32_t m, int32_t k, bool krows, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, false, apart, false, false);
     if (g.fewer() && (n > 64 || k > 320 || (krows && g.tiles * k > 19000 && g.tiles_joined * 4 <= g.tiles * 3))) return true;
-    if (!krows && k % 64 == 0 && k >= 1536 && g.rounds >= 22 && g.even(1, 1)) return true;
+    if (k % 64 == 0 && g.rounds >= 22 && (krows ? k >= 1024 && g.even(19, 20) : k >= 1536 && g.even(1, 1))) return true;
     return krows && n <= 64 && k >= 512 && g.tiles_joined <= compute_units();
 }
 // int8: rows also wherever the rounds stay, past one of them, with what the tiles of whole slabs do not take (19 of 2564 x 1600 beside 40 stored

@@ -110,6 +110,7 @@ def test_fewer_tiles(shared, edge, batch, k):
     assert torch.equal(_whole(A, B, False, s_row, s_col, k), _reference(A, B, False, s_row, s_col))
     for a_shared in (False, True):
         test_fp16_of_many_entries(a_shared, edge, batch, shared, k, False)
+    test_fp16_of_many_entries(False, edge, batch, shared, k, True)
 
 
 # (tiles of 128 x 64, two a compute unit, up to a depth of 768, of 128 x 128 beyond; whole and over the joined columns of many entries)

@@ -176,11 +176,12 @@ struct CopyTimes {
     float direct, copied;
 };
 static CopyTimes copy_times(int32_t n, int32_t k, int32_t m, int32_t batch, int aT) {
-    const float cus = (float)compute_units(), slabs = (float)k / 64.0f, mb = 1e-6f * (float)k * (float)m * (float)batch;
+    const int64_t units = compute_units();
+    const float cus = (float)units, slabs = (float)k / 64.0f, mb = 1e-6f * (float)k * (float)m * (float)batch;
     // (a round of large tiles, or tiles of 128 x 128 of up to a round, two, more of them; `apart`: of joined entries, big_tiles)
     auto tiled = [&](int64_t width, int64_t entries, int64_t apart, float base, float one, float two, float many, float large) {
-        if (large > 0.0f && n > 128 && width > 128 && big_tiles(n, (int32_t)width, (int)entries, apart) * 4 >= compute_units() * 3ll)
-            return (float)ceil_div(ceil_div(n, 256) * ceil_div(width, 256) * entries, compute_units()) * (slabs * large + 8.0f);
+        if (large > 0.0f && n > 128 && width > 128 && big_tiles(n, (int32_t)width, (int)entries, apart, units) * 4 >= units * 3)
+            return (float)ceil_div(ceil_div(n, 256) * ceil_div(width, 256) * entries, units) * (slabs * large + 8.0f);
         const float rounds = (float)(ceil_div(n, 128) * ceil_div(width, 128) * entries) / cus;
         return base + slabs * (rounds <= 1.0f ? one : rounds <= 2.0f ? two : many * rounds);
     };

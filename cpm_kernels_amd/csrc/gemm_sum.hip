@@ -65,8 +65,8 @@ static int32_t sum_groups_for(int kind, int32_t m, int32_t k, int32_t n, int32_t
 // fp16 1280 x 3328 x 14, k = 48 28 / 54; 512 x 512 x 6, 512 36 / 14 (one by one).
 // One by one: entries of at least half a round of the device's two tiles a compute unit, and no less than results written and read at 5.2 TB/s and products at
 // 4.4 (2.0) PFLOP/s take.
-static float sum_apart_time(bool i8, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch) {
-    const float rounds = (float)(tiles * batch) / (float)(2 * compute_units()), slabs = (float)ceil_div((int64_t)k * (i8 ? 1 : 2), 128), out = (float)batch * (float)n * (float)m * 1e-6f;
+static float sum_apart_time(bool i8, int64_t cus, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch) {
+    const float rounds = (float)(tiles * batch) / (float)(2 * cus), slabs = (float)ceil_div((int64_t)k * (i8 ? 1 : 2), 128), out = (float)batch * (float)n * (float)m * 1e-6f;
     const float part = rounds > 1.0f ? (i8 ? 0.69f : 0.91f) * rounds : (i8 ? 0.67f : 0.73f) * (rounds > 0.5f ? rounds : 0.5f);
     const float t = (i8 ? 9.1f : 9.4f) + slabs * part + (i8 ? 0.16f : 0.35f) * out + (i8 ? 7.8f : 5.4f) * rounds;
     const float least = (i8 ? 12.0f : 9.0f) + out * (4.0f / 5.2f + 2.0f * (float)k / (i8 ? 4400.0f : 2000.0f));
@@ -75,8 +75,8 @@ static float sum_apart_time(bool i8, int64_t tiles, int32_t m, int32_t k, int32_
 // A group: 4.5, and for each of its entries 0.40 and 0.45 a slab of 128 bytes (int8: folding, products), or 0.65 a slab (fp16; depths that are not whole
 // ones 0.7 and 0.26 a 64-byte slab, 2.0 and 0.30 where rows are not whole 16-byte pieces), half as much again where int8 tiles share compute units, a round of the
 // device after the other for fp16; several groups 3 and their fp32 sums at 4.7 TB/s.
-static float sum_group_time(bool i8, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch, int32_t g) {
-    const int64_t cus = compute_units(), work = tiles * g, last = work % cus;
+static float sum_group_time(bool i8, int64_t cus, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch, int32_t g) {
+    const int64_t work = tiles * g, last = work % cus;
     const float area = (float)n * (float)m * 1e-6f, kb = (float)(i8 ? k : 2 * k);
     const bool slabs = i8 || k % 64 == 0;
     const float entry = i8 ? 0.40f + 0.45f * ceilf(kb / 128.0f) : slabs ? 0.65f * kb / 128.0f : k % 8 == 0 ? 0.7f + 0.26f * floorf(kb / 64.0f) : 2.0f + 0.30f * floorf(kb / 64.0f);
@@ -89,8 +89,8 @@ static float sum_group_time(bool i8, int64_t tiles, int32_t m, int32_t k, int32_
 // (K, rows): whether the tile kernel takes the groups (gemm_rows_parts), else the kernel for any size does
 static bool krows_tiles(int32_t m, int64_t depth, int32_t n) { return depth >= 64 && (n % 8 == 0 || n >= 128) && (m % 8 == 0 || m >= 256); }
 // The entries of a group are one contraction of operands below 4 GiB; one group's is a product like any other (krows_time), whose depth may be divided.
-static float sum_krows_time(int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch, int32_t g) {
-    const int64_t depth = (int64_t)k * (batch / g), cus = compute_units();
+static float sum_krows_time(int64_t cus, int64_t tiles, int32_t m, int32_t k, int32_t n, int32_t batch, int32_t g) {
+    const int64_t depth = (int64_t)k * (batch / g);
     if ((m > n ? m : n) * depth >= 1ll << 31) return 1e30f;
     if (g == 1) return krows_time(m, (int32_t)depth, n);
     const float slabs = (float)ceil_div(depth, 64), add = 3.0f + (float)g * (float)n * (float)m * 8e-6f / 4.7f;
@@ -101,8 +101,7 @@ static float sum_krows_time(int64_t tiles, int32_t m, int32_t k, int32_t n, int3
     const float rounds = (float)(ceil_div(n, 64) * ceil_div(m, 64) * g) / (float)cus;
     return 2.6f + add + slabs * (rounds <= 1.0f ? 0.58f : rounds <= 4.0f ? 1.1f : 0.29f * rounds);
 }
-static bool sum_few_tiles(int kind, int32_t m, int32_t n) {
-    const int64_t cus = compute_units();
+static bool sum_few_tiles(int kind, int64_t cus, int32_t m, int32_t n) {
     return ceil_div(n, 128) * ceil_div(m, 128) <= 2 * cus && (kind == kSumI8 || ceil_div(n, 256) * ceil_div(m, 256) * 4 < cus * 3);
 }
 
@@ -111,7 +110,7 @@ static bool sum_few_tiles(int kind, int32_t m, int32_t n) {
 // groups of one entry 6.5 and 13.8 (one by one 9.9 and 17.1); 136 x 890 x 49, 128 50 us, seven groups 17.0 (20.7); 1644 x 2132 x 10, 512 in one 54 (75)
 static int32_t sum_krows_groups(int32_t m, int32_t k, int32_t n, int32_t batch) {
     const int64_t cus = compute_units(), tiles = ceil_div(n, 128) * ceil_div(m, 128);
-    if (!sum_few_tiles(kSumF16KFirst, m, n) || k > (tiles > cus ? 640 : 1023)) {
+    if (!sum_few_tiles(kSumF16KFirst, cus, m, n) || k > (tiles > cus ? 640 : 1023)) {
         const int32_t g = sum_groups_for(kSumF16KFirst, m, k, n, batch);
         return g == batch && batch > 1 ? 0 : g;
     }
@@ -119,7 +118,7 @@ static int32_t sum_krows_groups(int32_t m, int32_t k, int32_t n, int32_t batch) 
     float best_t = 1e30f;
     for (int32_t g = 1; g <= batch && (g == 1 || g * tiles <= 4 * cus); ++g) {
         if (batch % g != 0) continue;
-        const float t = sum_krows_time(tiles, m, k, n, batch, g);
+        const float t = sum_krows_time(cus, tiles, m, k, n, batch, g);
         if (t < best_t) {
             best_t = t;
             best = g;
@@ -129,17 +128,17 @@ static int32_t sum_krows_groups(int32_t m, int32_t k, int32_t n, int32_t batch) 
 }
 
 static int32_t sum_groups_timed(int kind, int32_t m, int32_t k, int32_t n, int32_t batch) {
-    const int64_t cus = compute_units(), tiles = ceil_div(n, 128) * ceil_div(m, 128);
     if (kind == kSumF16KFirst) {
         const int32_t g = sum_krows_groups(m, k, n, batch);
         return g == 0 ? batch : g;
     }
-    if (!sum_few_tiles(kind, m, n)) return sum_groups_for(kind, m, k, n, batch);
+    const int64_t cus = compute_units(), tiles = ceil_div(n, 128) * ceil_div(m, 128);
+    if (!sum_few_tiles(kind, cus, m, n)) return sum_groups_for(kind, m, k, n, batch);
     int32_t best = batch;
-    float best_t = sum_apart_time(kind == kSumI8, tiles, m, k, n, batch);
+    float best_t = sum_apart_time(kind == kSumI8, cus, tiles, m, k, n, batch);
     for (int32_t g = 1; g < batch && g * tiles <= 4 * cus; ++g) {
         if (batch % g != 0 || batch / g > kSumMax) continue;
-        const float t = sum_group_time(kind == kSumI8, tiles, m, k, n, batch, g);
+        const float t = sum_group_time(kind == kSumI8, cus, tiles, m, k, n, batch, g);
         if (t < best_t) {
             best_t = t;
             best = g;

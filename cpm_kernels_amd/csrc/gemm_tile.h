@@ -1246,18 +1246,17 @@ static bool cols_join(int batch, int32_t m, int64_t row_bytes) {
 // Tiles of 256 x 256, or those of the entries before they were joined (`apart`) where the joined product has more than two smaller ones a
 // compute unit: fewer and fuller tiles are no reason to take those (16 entries of 960 columns, 640 x 2304, 192 large tiles apart, 180 joined
 // or 600 small ones: 39, 37 and 45 us).
-static int64_t big_tiles(int32_t n, int32_t m, int batch, int64_t apart) {
+static int64_t big_tiles(int32_t n, int32_t m, int batch, int64_t apart, int64_t cus = compute_units()) {
     const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch;
-    return apart > big && ceil_div(n, 128) * ceil_div(m, 128) * batch > 2 * compute_units() ? apart : big;
+    return apart > big && ceil_div(n, 128) * ceil_div(m, 128) * batch > 2 * cus ? apart : big;
 }
 
 // The time of a product's tiles, in tenths of a round of 128 x 128 tiles over the chip: a second round beside the first costs 0.8 of it (two
 // workgroups fit a compute unit), a round of 256 x 256 tiles 2.2.  int8, K-major: `halves`, whether there are tiles of 128 x 64, a round of which is 0.8,
 // and `whole`, whether a last round of large tiles is one of half tiles (fp16 products are drawn without: no better for it).
-static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool whole, bool halves) {
-    const int64_t cus = compute_units();
+static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool whole, bool halves, int64_t cus) {
     const int64_t tiles = ceil_div(n, 128) * ceil_div(m, 128) * batch;
-    if (n > 128 && m > 128 && big_tiles(n, m, batch, apart) * 4 >= cus * 3) {
+    if (n > 128 && m > 128 && big_tiles(n, m, batch, apart, cus) * 4 >= cus * 3) {
         const int64_t big = ceil_div(n, 256) * ceil_div(m, 256) * batch, r = big % cus;
         return whole && big > cus && r != 0 && 2 * r <= cus ? 22 * (big / cus) + 13 : 22 * ceil_div(big, cus);
     }
@@ -1277,20 +1276,21 @@ static int64_t tile_rounds(int32_t n, int32_t m, int batch, int64_t apart, bool 
 //   int8 rows 0.980, none of 103; fp16 rows 0.973, 2 of 120; int8 columns 0.964, 1 of 135; fp16 columns 0.948, none of 68, beside rows stored (K, rows) 0.944,
 //   none of 26; rows from 1024 on where the tiles stay too 0.985, none of 19 (47 entries of 128 x 1280 beside 832 26.2 -> 22.8 us)
 struct JoinGain {
-    int64_t rounds, rounds_joined, tiles, tiles_joined;
+    int64_t rounds, rounds_joined, tiles, tiles_joined, cus;
     bool fewer() const { return rounds_joined < rounds; }
     bool even(int64_t num, int64_t den) const { return rounds_joined == rounds && tiles_joined < tiles && tiles_joined * den <= tiles * num; }      // .. at most num / den of the tiles
 };
 static JoinGain join_gain(int32_t n, int32_t m, int batch, bool rows, int64_t apart, bool whole, bool halves) {
     const int32_t nj = rows ? n * batch : n, mj = rows ? m : m * batch;
-    return {tile_rounds(n, m, batch, 0, whole, halves), tile_rounds(nj, mj, 1, apart, whole, halves), ceil_div(n, 128) * ceil_div(m, 128) * batch, ceil_div(nj, 128) * ceil_div(mj, 128)};
+    const int64_t cus = compute_units();       // (asked once: it is a call into the runtime)
+    return {tile_rounds(n, m, batch, 0, whole, halves, cus), tile_rounds(nj, mj, 1, apart, whole, halves, cus), ceil_div(n, 128) * ceil_div(m, 128) * batch, ceil_div(nj, 128) * ceil_div(mj, 128), cus};
 }
 // fp16, whose few rows and short depths have kernels of their own: rows, past 128 of them or a depth of 448, or many tiles of enough depth
 // (500 entries of 4 x 400 beside 314: 19.3 -> 7.5 us; 41 of 4 x 64 beside 3808, 4.3 apart and 5.7 joined)
 static bool rows_join_pays_f16(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, true, apart, false, false);
     if (k >= 1024 ? g.rounds_joined == g.rounds : kmajor && k % 64 == 0 && k >= 512 && g.even(1, 1)) return true;
-    return g.fewer() && (n > 128 || k > 448 || (g.tiles > 4 * (int64_t)compute_units() && g.tiles * k > 100000 && g.tiles_joined * 3 <= g.tiles));
+    return g.fewer() && (n > 128 || k > 448 || (g.tiles > 4 * g.cus && g.tiles * k > 100000 && g.tiles_joined * 3 <= g.tiles));
 }
 // Columns, past 64 rows or a depth of 320; a row operand stored (K, rows) leaves fewer such calls to those kernels, and in a single round its long
 // depths gain too (357 entries of 64 columns, 40 rows, K = 240 14.5 -> 9.5 us; 94 of 128, 64 rows, K = 2328 28.7 -> 23.7)
@@ -1298,14 +1298,14 @@ static bool cols_join_pays_f16(int32_t n, int32_t m, int32_t k, bool krows, int 
     const JoinGain g = join_gain(n, m, batch, false, apart, false, false);
     if (g.fewer() && (n > 64 || k > 320 || (krows && g.tiles * k > 19000 && g.tiles_joined * 4 <= g.tiles * 3))) return true;
     if (k % 64 == 0 && g.rounds >= 22 && (krows ? k >= 1024 && g.even(19, 20) : k >= 1536 && g.even(1, 1))) return true;
-    return krows && n <= 64 && k >= 512 && g.tiles_joined <= compute_units();
+    return krows && n <= 64 && k >= 512 && g.tiles_joined <= g.cus;
 }
 // int8: rows also wherever the rounds stay, past one of them, with what the tiles of whole slabs do not take (19 of 2564 x 1600 beside 40 stored
 // (K, columns), 495 -> 300; 37 of 128 x 36 beside 1280, 46 -> 17)
 static bool rows_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, true, apart, k % 64 == 0, kmajor && k % 128 == 0);
     if (kmajor && k % 128 == 0 && (k >= 1024 ? g.rounds_joined == g.rounds : k >= 384 && g.even(1, 1))) return true;
-    return g.fewer() || ((!kmajor || k % 64 != 0) && g.tiles > compute_units() && g.rounds_joined == g.rounds);
+    return g.fewer() || ((!kmajor || k % 64 != 0) && g.tiles > g.cus && g.rounds_joined == g.rounds);
 }
 static bool cols_join_pays_i8(int32_t n, int32_t m, int32_t k, bool kmajor, int batch, int64_t apart) {
     const JoinGain g = join_gain(n, m, batch, false, apart, k % 64 == 0, kmajor && k % 128 == 0);
